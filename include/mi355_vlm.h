@@ -447,6 +447,10 @@ int mi355_decode_advance(int B, const int64_t* next_ids, int64_t* tok, int32_t* 
  * step can be replayed): cache[b, *pos, :] = rows[b, :] for keys and values; width = kv_heads * head_dim. */
 int mi355_kv_append(int B, int width, const void* k_rows, int64_t ldk, const void* v_rows, int64_t ldv, void* k_cache, void* v_cache,
                     int64_t batch_stride, int64_t ld, int capacity, const int32_t* pos, void* stream);
+/* KVCache append with the position known on the host (utils.py:496-531): cache[b, start + s, :] = rows[b * S + s, :] for keys and values, one launch for every
+ * sequence; any element type (widths, pitches and addresses are multiples of 16 bytes). */
+int mi355_kv_append_rows(int B, int S, int64_t width_bytes, const void* k_rows, int64_t ldk_bytes, const void* v_rows, int64_t ldv_bytes, void* k_cache, void* v_cache,
+                         int64_t batch_stride_bytes, int64_t ld_bytes, int start, int capacity, void* stream);
 /* Greedy sampling (generate.py:472-476, temp == 0): out[r] = index of the row maximum of bf16 logits [rows, V] (first on ties).
  * workspace: rows * 64 * 12 bytes (+8), 8-byte aligned: 64 column ranges per row are scanned in parallel, then merged. */
 int mi355_argmax_rows(int64_t rows, int64_t V, const void* logits, int64_t ld, int64_t* out, void* workspace, void* stream);

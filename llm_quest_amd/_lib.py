@@ -98,6 +98,7 @@ SIGNATURES = {
     "mi355_attn_decode_qkv": [_I, _I, _I, _I, _P, _L, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _P, _P, _P, _L, _P, _F, _F, _I, _P, _P],
     "mi355_decode_advance": [_I, _P, _P, _P, _P, _P, _P],
     "mi355_attn_decode": [_I, _I, _I, _I, _P, _P, _P, _L, _L, _I, _P, _P, _L, _P, _F, _I, _P, _P],
+    "mi355_kv_append_rows": [_I, _I, _L, _P, _L, _P, _L, _P, _P, _L, _L, _I, _I, _P],
     "mi355_kv_append": [_I, _I, _P, _L, _P, _L, _P, _P, _L, _L, _I, _P, _P],
     "mi355_argmax_rows": [_L, _L, _P, _L, _P, _P, _P],
     "mi355_argmax_rows_f32": [_L, _L, _P, _L, _P, _P, _P],

@@ -65,6 +65,19 @@ class KVCache:
                 self._grow_kv_capacity(layer_idx)
         self.end_pos = saved_end
 
+    def claim_rows(self, layer_idx, new_seq_len):
+        """Room for ``new_seq_len`` more rows of a layer whose buffers exist: (k_cache, v_cache, end_pos), the counters as after ``append_rows`` -- the caller's
+        launch writes rows [end_pos - new_seq_len, end_pos)."""
+        self.end_pos = self.start_pos + new_seq_len
+        if self.end_pos > self.context_len:
+            raise ValueError(f"KVCache: sequence length {self.end_pos} exceeds context_len {self.context_len}")
+        if self.end_pos > self.keys_cache[layer_idx].shape[1]:
+            self._grow_kv_capacity(layer_idx)
+        end = self.end_pos
+        if layer_idx == self.num_layers - 1:
+            self.start_pos += new_seq_len
+        return self.keys_cache[layer_idx], self.values_cache[layer_idx], end
+
     def append_rows(self, k_rows, v_rows, layer_idx, batch_size, new_seq_len):
         """k_rows / v_rows: token-major [batch*new_seq_len, kv_heads*head_dim] (row-strided views allowed).  Returns
         (k_cache [batch, capacity, width], v_cache, end_pos) with the new rows in place at [start_pos, end_pos)."""
@@ -73,18 +86,17 @@ class KVCache:
         if not self.keys_cache:
             self.batch_size, self.device, self.dtype = batch_size, k_rows.device, k_rows.dtype
             self._initialize(batch_size, width, k_rows.device, k_rows.dtype)
-        self.end_pos = self.start_pos + new_seq_len
-        if self.end_pos > self.context_len:
-            raise ValueError(f"KVCache: sequence length {self.end_pos} exceeds context_len {self.context_len}")
-        if self.end_pos > self.keys_cache[layer_idx].shape[1]:
-            self._grow_kv_capacity(layer_idx)
-        kc, vc = self.keys_cache[layer_idx], self.values_cache[layer_idx]
-        for b in range(batch_size):
-            K.copy2d(k_rows[b * new_seq_len : (b + 1) * new_seq_len], kc[b, self.start_pos : self.end_pos])
-            K.copy2d(v_rows[b * new_seq_len : (b + 1) * new_seq_len], vc[b, self.start_pos : self.end_pos])
-        end = self.end_pos
-        if layer_idx == self.num_layers - 1:
-            self.start_pos += new_seq_len
+        kc, vc, end = self.claim_rows(layer_idx, new_seq_len)
+        start, es = end - new_seq_len, kc.element_size()
+        if (k_rows.dtype == v_rows.dtype == kc.dtype and k_rows.shape == v_rows.shape == (batch_size * new_seq_len, kc.shape[2]) and k_rows.stride(1) == v_rows.stride(1) == 1
+                and kc.shape[0] >= batch_size and kc.stride() == vc.stride() and kc.stride(2) == 1 and new_seq_len > 0 and k_rows.device == kc.device
+                and not (width * es | k_rows.stride(0) * es | v_rows.stride(0) * es | kc.stride(0) * es | kc.stride(1) * es | k_rows.data_ptr() | v_rows.data_ptr()) & 15):
+            L.call("mi355_kv_append_rows", batch_size, new_seq_len, width * es, L.ptr(k_rows), k_rows.stride(0) * es, L.ptr(v_rows), v_rows.stride(0) * es, L.ptr(kc), L.ptr(vc),
+                   kc.stride(0) * es, kc.stride(1) * es, start, kc.shape[1])
+        else:  # rows that are not whole 16-byte words
+            for b in range(batch_size):
+                K.copy2d(k_rows[b * new_seq_len : (b + 1) * new_seq_len], kc[b, start:end])
+                K.copy2d(v_rows[b * new_seq_len : (b + 1) * new_seq_len], vc[b, start:end])
         return kc, vc, end
 
     # ------------------------------------------------------------------ reference signature
