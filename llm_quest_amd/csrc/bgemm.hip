@@ -9,13 +9,15 @@
 // Uses: the per-head products of latent attention with the key / value up-projections folded onto the query and the output side;
 // the experts of a mixture (batch = expert, a batch's rows given by device-side offsets, A rows gathered through a dispatch list,
 // C rows scattered back and scaled by the routing weight); and every linear layer of the true-fp32 mode (fp32 activations,
-// weights kept in bf16 -- exactly representable -- and widened on load, fp32 FMA accumulation in a fixed k order, so a row's result does not depend
-// on which other rows share its tile).
+// weights kept in bf16, exact products, fp32 accumulation in a fixed k order, so a row's result does not depend on which other rows share its tile).
 //
 // Compute paths:
-//   * FMA: 64 x 64 tile, 256 threads, 4 x 4 outputs per thread, k in steps of 16 through LDS (any operand type);
+//   * FMA: 64 x 64 tile, 256 threads, 4 x 4 outputs per thread, k in steps of 16 through LDS (any operand type and stride);
+//   * fp32 A, bf16 B stored [out, in] in 16-byte words: an fp32 number as three bf16 numbers, v_mfma_f32_32x32x16_bf16, tile or weight stream;
 //   * MFMA (bf16 A and B): the same tile, four waves of 32 x 32 on v_mfma_f32_32x32x8_bf16_1k, k in steps of 32; a 128 x 128 tile on v_mfma_f32_32x32x16_bf16 for
 //     weights stored [out, in]; and, for few rows in all groups together, a stream of the weights that deals k to the waves of a workgroup.
+#include <type_traits>
+
 #include "common.h"
 
 #define ST(s) ((hipStream_t)(s))
@@ -361,37 +363,212 @@ __global__ __launch_bounds__(256) void bgemm_mfma128_kernel(BgemmArgs p) {
             }
 }
 
+// ---- fp32 A times bf16 B on the matrix pipe, with the fp32 product's accuracy.  An fp32 number is the sum of three bf16 numbers exactly (its 24 significant bits cut into three
+// runs of 8 by truncation: no rounding, no overflow; what is lost lies below 2^-133), a product of two bf16 numbers is exact in fp32, and the accumulator is fp32 -- so three
+// products (lo, mid, hi) stand for one fp32 product, and what rounds is the sum, as in an FMA chain.  K is cut into SW runs of 16-steps that are summed one by one and
+// then joined in order, in EVERY kernel of this path: a row's bits depend neither on the rows beside it nor on which of the kernels its row count takes.
+// Against the FMA kernel (64 x 64 tile, scalar fp32: VALU-bound, and at few rows a chain of uncached 2-byte loads): a fp32 replay of three 150-token prompts and four
+// single tokens through four layers with experts 19.9 -> 6.0 ms, its logits' error against 64 bits 4.9e-6 -> 2.1e-6
+// (fewer roundings per sum).  Weights are finite: an infinite one would meet a zero part (NaN).
+#define SW 8
+struct Split8 { u32x4 hi, mid, lo; };
+struct FragF32 { f32x4 a, b; };  // eight consecutive k of a row
+__device__ __forceinline__ void split_pair(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {
+    const unsigned u0 = __float_as_uint(x0), u1 = __float_as_uint(x1), h0 = u0 & 0xffff0000u, h1 = u1 & 0xffff0000u;
+    const bool f0 = (u0 & 0x7f800000u) != 0x7f800000u, f1 = (u1 & 0x7f800000u) != 0x7f800000u;  // infinities and NaN stay whole in `hi` (a NaN keeps a set top bit below)
+    const float r0 = f0 ? x0 - __uint_as_float(h0) : 0.f, r1 = f1 ? x1 - __uint_as_float(h1) : 0.f;
+    const unsigned m0 = __float_as_uint(r0) & 0xffff0000u, m1 = __float_as_uint(r1) & 0xffff0000u;
+    const float s0 = r0 - __uint_as_float(m0), s1 = r1 - __uint_as_float(m1);
+    const unsigned n0 = !f0 && (u0 & 0x007fffffu) ? h0 | 0x00400000u : h0, n1 = !f1 && (u1 & 0x007fffffu) ? h1 | 0x00400000u : h1;
+    hi = (n0 >> 16) | n1;
+    mid = (m0 >> 16) | m1;
+    lo = (__float_as_uint(s0) >> 16) | (__float_as_uint(s1) & 0xffff0000u);
+}
+__device__ __forceinline__ Split8 split8(const f32x4 a, const f32x4 b) {
+    Split8 r;
+    unsigned h, m, l;
+    split_pair(a[0], a[1], h, m, l); r.hi[0] = h; r.mid[0] = m; r.lo[0] = l;
+    split_pair(a[2], a[3], h, m, l); r.hi[1] = h; r.mid[1] = m; r.lo[1] = l;
+    split_pair(b[0], b[1], h, m, l); r.hi[2] = h; r.mid[2] = m; r.lo[2] = l;
+    split_pair(b[2], b[3], h, m, l); r.hi[3] = h; r.mid[3] = m; r.lo[3] = l;
+    return r;
+}
+
+// Tile of 64 WM rows x 128 columns, four waves of 32 WM x 64 (2 x 2): k in steps of 32 through one LDS stage (A as three bf16 planes, split once per tile), the next
+// step's operands on their way in registers.  VALU (the split) and matrix pipe are level at WM = 1; WM = 2 halves the split's and B's share where there are rows for it.
+#define FK 32
+template <int WM>
+__global__ __launch_bounds__(256) void bgemm_f32_tile_kernel(BgemmArgs p) {
+    constexpr int R = 64 * WM, AP = R / 32;  // A: 8 threads per row of 32 fp32, 32 rows per pass; B: 4 threads per row of 32 bf16, 64 rows per pass
+    __shared__ __attribute__((aligned(16))) bf16_t As[3][R][FK + MPAD];
+    __shared__ __attribute__((aligned(16))) bf16_t Bs[128][FK + MPAD];
+    const int b = blockIdx.z;
+    int row0 = 0, rows = p.M;
+    if (p.grp_offs) {
+        row0 = p.grp_offs[b];
+        rows = p.grp_offs[b + 1] - row0;
+    }
+    const int m0 = blockIdx.y * R, n0 = blockIdx.x * 128;
+    if (m0 >= rows) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
+    const float* a_row[AP];
+    const int ar = tid >> 3, ak = (tid & 7) * 4, br = tid >> 2, bk = (tid & 3) * 8;
+#pragma unroll
+    for (int i = 0; i < AP; ++i) {
+        a_row[i] = nullptr;
+        if (m0 + ar + 32 * i < rows) {
+            const int r = row0 + m0 + ar + 32 * i;
+            a_row[i] = (const float*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
+        }
+    }
+    const bf16_t* b_row[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) b_row[i] = n0 + br + 64 * i < p.N ? (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)(n0 + br + 64 * i) * p.sbn : nullptr;
+    f32x4 ra[AP];
+    u32x4 rb[2];
+    auto fetch = [&](int k0) {  // K is a multiple of 8: a 16-byte word lies inside or outside as a whole
+#pragma unroll
+        for (int i = 0; i < AP; ++i) ra[i] = a_row[i] && k0 + ak < p.K ? *(const f32x4*)(a_row[i] + k0 + ak) : (f32x4){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 2; ++i) rb[i] = b_row[i] && k0 + bk < p.K ? *(const u32x4*)(b_row[i] + k0 + bk) : (u32x4){0u, 0u, 0u, 0u};
+    };
+    f32x16 acc[WM][2], tot[WM][2];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[i][j][e] = tot[i][j][e] = 0.f;
+    const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW;
+    int left = per;
+    const int wm = (wave >> 1) * 32 * WM, wn = (wave & 1) * 64;
+    fetch(0);
+    for (int k0 = 0; k0 < p.K; k0 += FK) {
+        __syncthreads();  // the previous step's fragments are read
+#pragma unroll
+        for (int i = 0; i < AP; ++i) {
+            u32x2 h, m, l;
+            unsigned x, y, z;
+            split_pair(ra[i][0], ra[i][1], x, y, z); h[0] = x; m[0] = y; l[0] = z;
+            split_pair(ra[i][2], ra[i][3], x, y, z); h[1] = x; m[1] = y; l[1] = z;
+            *(u32x2*)&As[0][ar + 32 * i][ak] = h;
+            *(u32x2*)&As[1][ar + 32 * i][ak] = m;
+            *(u32x2*)&As[2][ar + 32 * i][ak] = l;
+        }
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *(u32x4*)&Bs[br + 64 * i][bk] = rb[i];
+        __syncthreads();
+        if (k0 + FK < p.K) fetch(k0 + FK);
+#pragma unroll
+        for (int kk = 0; kk < FK; kk += 16) {
+            if (k0 + kk >= p.K) break;
+            bf16x8 bf[2];
+#pragma unroll
+            for (int j = 0; j < 2; ++j) bf[j] = *(const bf16x8*)&Bs[wn + 32 * j + ln][kk + 8 * hf];
+#pragma unroll
+            for (int s = 2; s >= 0; --s)
+#pragma unroll
+                for (int i = 0; i < WM; ++i) {
+                    const bf16x8 af = *(const bf16x8*)&As[s][wm + 32 * i + ln][kk + 8 * hf];
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf[j], acc[i][j], 0, 0, 0);
+                }
+            if (--left == 0) {
+                left = per;
+#pragma unroll
+                for (int i = 0; i < WM; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) {
+                            tot[i][j][e] += acc[i][j][e];
+                            acc[i][j][e] = 0.f;
+                        }
+            }
+        }
+    }
+    if (left != per) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) tot[i][j][e] += acc[i][j][e];
+    }
+#pragma unroll
+    for (int bi = 0; bi < WM; ++bi)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int m = m0 + wm + 32 * bi + 8 * g + 4 * hf + i;
+                if (m >= rows) continue;
+                const int r = row0 + m;
+                const int64_t crow = p.c_rows ? p.c_rows[r] : r;
+                const float sc = p.row_scale ? p.row_scale[crow] : 1.0f;
+                const int64_t cb = (int64_t)b * p.c_bs + crow * p.ldc;
+                if (p.epi >= 2) {  // this wave's 64 columns are one [32 gates | 32 ups] block
+                    const int n = ((n0 + wn) >> 1) + ln;
+                    if (n < p.n_out) {
+                        const float v = gated_act(p.epi, tot[bi][0][4 * g + i], tot[bi][1][4 * g + i], p.limit) * sc;
+                        if (p.c_dt == MI355_DT_F32) ((float*)p.C)[cb + n] = v;
+                        else ((bf16_t*)p.C)[cb + n] = f2bf(v);
+                    }
+                    continue;
+                }
+#pragma unroll
+                for (int bj = 0; bj < 2; ++bj) {
+                    const int n = n0 + wn + 32 * bj + ln;
+                    if (n >= p.N) continue;
+                    float v = tot[bi][bj][4 * g + i] + (p.bias ? p.bias[n] : 0.f);
+                    if (p.epi == 1) v = v > 0.f ? v * v : 0.f;
+                    v *= sc;
+                    if (p.c_dt == MI355_DT_F32) ((float*)p.C)[cb + n] = v;
+                    else ((bf16_t*)p.C)[cb + n] = f2bf(v);
+                }
+            }
+}
+
 // ---- MFMA path for few rows per group (one-token steps through a mixture's experts): bound by the stream of the weights.  A workgroup is eight waves on 32 rows x 32
 // columns (GLU: the 32 gate and the 32 up columns of one block); the waves deal the k range among themselves, read both operands straight from memory in
 // fragment form -- 16 bytes per lane, SU steps of 16 in flight while the previous SU multiply -- and their partial sums meet in LDS.
-#define SW 8
 #define SU 4
+#define F32_STREAM_ROWS 128  // fp32 A: beyond this many rows the tile kernel's one split per 128 columns beats the stream's one per 32 (450 rows: a third of the time)
 #define STREAM_ROWS 256  // up to this many sorted rows in all groups together
-template <bool GLU>
+// F32: A is fp32, split into three bf16 fragments in registers (see above: the waves' k runs are that path's runs).
+template <bool GLU, bool F32>
 __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
     constexpr int NB = GLU ? 2 : 1;
+    using elem_t = std::conditional_t<F32, float, bf16_t>;
+    using frag_t = std::conditional_t<F32, FragF32, u32x4>;
     __shared__ float red[SW][NB][16][64];
-    const int b = blockIdx.z, row0 = p.grp_offs[b], rows = p.grp_offs[b + 1] - row0;
+    const int b = blockIdx.z, row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? p.grp_offs[b + 1] - row0 : p.M;
     const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32 * NB;
     if (m0 >= rows) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
-    const bf16_t* a_row = nullptr;
+    const elem_t* a_row = nullptr;
     if (m0 + ln < rows) {
         const int r = row0 + m0 + ln;
-        a_row = (const bf16_t*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
+        a_row = (const elem_t*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
     }
     const bf16_t* b_row[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j) b_row[j] = n0 + 32 * j + ln < p.N ? (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)(n0 + 32 * j + ln) * p.sbn : nullptr;
     const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
     const u32x4 zero = {0u, 0u, 0u, 0u};
-    u32x4 fa[SU], fb[SU][NB];
+    frag_t fa[SU];
+    u32x4 fb[SU][NB];
     auto fetch = [&](int st) {
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
             const int k = (st + u) * 16 + 8 * hf;  // K is a multiple of 8
             const bool in = st + u < s1 && k < p.K;
-            fa[u] = in && a_row ? *(const u32x4*)(a_row + k) : zero;
+            if constexpr (F32) {
+                fa[u].a = in && a_row ? *(const f32x4*)(a_row + k) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                fa[u].b = in && a_row ? *(const f32x4*)(a_row + k + 4) : (f32x4){0.f, 0.f, 0.f, 0.f};
+            } else {
+                fa[u] = in && a_row ? *(const u32x4*)(a_row + k) : zero;
+            }
 #pragma unroll
             for (int j = 0; j < NB; ++j) fb[u][j] = in && b_row[j] ? *(const u32x4*)(b_row[j] + k) : zero;
         }
@@ -403,7 +580,8 @@ __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
     fetch(s0);
     for (int st = s0; st < s1; st += SU) {
-        u32x4 ca[SU], cb[SU][NB];
+        frag_t ca[SU];
+        u32x4 cb[SU][NB];
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
             ca[u] = fa[u];
@@ -412,9 +590,21 @@ __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
         }
         if (st + SU < s1) fetch(st + SU);
 #pragma unroll
-        for (int u = 0; u < SU; ++u)
+        for (int u = 0; u < SU; ++u) {
+            if constexpr (F32) {
+                const Split8 t = split8(ca[u].a, ca[u].b);
 #pragma unroll
-            for (int j = 0; j < NB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ca[u]), __builtin_bit_cast(bf16x8, cb[u][j]), acc[j], 0, 0, 0);
+                for (int j = 0; j < NB; ++j) {
+                    const bf16x8 w = __builtin_bit_cast(bf16x8, cb[u][j]);
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.lo), w, acc[j], 0, 0, 0);
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.mid), w, acc[j], 0, 0, 0);
+                    acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.hi), w, acc[j], 0, 0, 0);
+                }
+            } else {
+#pragma unroll
+                for (int j = 0; j < NB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ca[u]), __builtin_bit_cast(bf16x8, cb[u][j]), acc[j], 0, 0, 0);
+            }
+        }
     }
 #pragma unroll
     for (int j = 0; j < NB; ++j)
@@ -471,8 +661,8 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
     const bool vec = sbk == 1 && K % 8 == 0 && lda % 8 == 0 && a_bs % 8 == 0 && sbn % 8 == 0 && b_bs % 8 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0;
     if (use_mfma && grp_offs && M <= STREAM_ROWS && K >= 256 && vec) {
         const dim3 grid((N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
-        if (epi >= 2) bgemm_stream_kernel<true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
-        else bgemm_stream_kernel<false><<<grid, 64 * SW, 0, ST(stream)>>>(p);
+        if (epi >= 2) bgemm_stream_kernel<true, false><<<grid, 64 * SW, 0, ST(stream)>>>(p);
+        else bgemm_stream_kernel<false, false><<<grid, 64 * SW, 0, ST(stream)>>>(p);
         MI355_LAUNCH_CHECK("bgemm(stream)");
         return 0;
     }
@@ -483,6 +673,25 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
         if (vec) bgemm_mfma128_kernel<true><<<grid, 256, 0, ST(stream)>>>(p);
         else bgemm_mfma128_kernel<false><<<grid, 256, 0, ST(stream)>>>(p);
         MI355_LAUNCH_CHECK("bgemm");
+        return 0;
+    }
+    // fp32 rows times bf16 weights stored [out, in], in 16-byte words: three bf16 products for one.  The choice looks at types, strides and K only, never at M: a row's
+    // bits do not depend on the batch.  Among the kernels: few rows stream the weights, more take the tile; 128-row tiles once they fill the chip.
+    const bool f32_split = !use_mfma && a_dt == MI355_DT_F32 && b_dt == MI355_DT_BF16 && sbk == 1 && K % 8 == 0 && lda % 4 == 0 && a_bs % 4 == 0 && sbn % 8 == 0 && b_bs % 8 == 0 &&
+                           ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0;
+    if (f32_split) {
+        const int64_t ty = ((int64_t)M + 63) / 64;
+        MI355_REQUIRE(ty <= 65535, "bgemm: too many row tiles");
+        if (M <= F32_STREAM_ROWS) {
+            const dim3 grid((N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
+            if (epi >= 2) bgemm_stream_kernel<true, true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
+            else bgemm_stream_kernel<false, true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
+        } else {
+            const int64_t tn = (N + 127) / 128, tiles = (grp_offs ? 1 : batch) * tn * ((M + 127) / 128);
+            if (tiles >= 512) bgemm_f32_tile_kernel<2><<<dim3((unsigned)tn, (unsigned)((M + 127) / 128), batch), 256, 0, ST(stream)>>>(p);
+            else bgemm_f32_tile_kernel<1><<<dim3((unsigned)tn, (unsigned)ty, batch), 256, 0, ST(stream)>>>(p);
+        }
+        MI355_LAUNCH_CHECK("bgemm(f32)");
         return 0;
     }
     const int64_t my = ((int64_t)M + BM - 1) / BM;

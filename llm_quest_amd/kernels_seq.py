@@ -234,7 +234,7 @@ def bgemm(a, b, c, M, N, Kd, batch=1, lda=None, a_bs=0, sbn=None, sbk=1, b_bs=0,
 
 def linear(x, w, out_dtype=None, bias=None):
     """x [M, K] (bf16 or fp32) times w[N, K]^T (bf16) (+ bias fp32 [N]).  bf16 rows go through the MFMA GEMMs (weight stream for <= 8 rows), fp32 rows through
-    the fp32 FMA product."""
+    the fp32 product (``bgemm``: exact products, fp32 sums in an order that does not depend on M)."""
     _rows(x, "linear(x)")
     M, Kd = x.shape
     N = w.shape[0]

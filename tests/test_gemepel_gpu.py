@@ -450,3 +450,56 @@ def test_post_sum_layernorm_and_head_norm():
     got = S.gated_headnorm(o.to(DEV), wn.to(DEV), gate.to(DEV), 3, 70, 1e-5, F32)
     want = (G.rms_unit(o.view(11, 3, 70).double(), 1e-5) * wn.double()).view(11, -1) * torch.nn.functional.silu(gate.double())
     assert (got.cpu() - want).abs().max() < 1e-5
+
+
+# ----------------------------------------------------------------------------------------------- the fp32 product on split operands
+@pytest.mark.parametrize("M,N,K", [(1, 32, 8), (3, 33, 24), (31, 1000, 136), (32, 64, 1024), (33, 200, 264), (128, 96, 2048), (129, 130, 2056), (450, 256, 520), (700, 16640, 72)])
+def test_fp32_product_on_split_operands(M, N, K):
+    """fp32 rows times bf16 weights: edges of the stream's and both tiles' rows, columns and k runs, strided rows, against fp64 -- per output the error of n fp32 roundings of
+    the partial sums, n = the 16-steps (three products each) plus the eight runs -- and a row's bits with and without other rows."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(M + N + K)
+    wide = (torch.randn(M, K + 12, generator=g) * torch.exp(3 * torch.randn(M, K + 12, generator=g))).cuda()
+    x, w = wide[:, 4 : 4 + K], (torch.randn(N, K, generator=g) / K ** 0.5).to(BF16).cuda()
+    got = S.linear(x, w)
+    want = x.double() @ w.double().T
+    bound = (3 * ((K + 15) // 16) + 8 + 16) * 2.0 ** -23 * (x.double().abs() @ w.double().abs().T)
+    assert bool(((got.double() - want).abs() <= bound).all())
+    for rows in ([M - 1], list(range(0, M, 3)), list(range(M // 2, M))):
+        if rows:
+            assert torch.equal(S.linear(x[rows].contiguous(), w), got[rows])
+    if M > 2:  # infinities and NaN stay what they are, in their rows alone; the largest numbers do not overflow in the split
+        y = x.clone()
+        y[0, 0], y[1, K - 1], y[2] = float("inf"), float("nan"), 0.0
+        y[2, 0] = 3.4028234e38
+        out = S.linear(y, w)
+        assert torch.equal(out[0].sign(), w[:, 0].float().sign()) and bool(out[0][w[:, 0] != 0].isinf().all()) and bool(out[1].isnan().all())
+        big = 3.4028234663852886e38 * w[:, 0].double()
+        assert float((out[2].double() - big).abs().max()) <= 2.0 ** -22 * float(big.abs().max()) and torch.equal(out[3:], got[3:])
+
+
+@pytest.mark.parametrize("T,top,epi", [(5, 2, 1), (70, 3, 0), (90, 2, 4), (400, 2, 4)])
+def test_fp32_grouped_product_on_split_operands(T, top, epi):
+    """Experts (rows gathered, scaled and scattered; one expert without rows; gated blocks): stream and tile against fp64."""
+    from llm_quest_amd import kernels_seq as S
+
+    E, K, ff = 5, 200, 96
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, K, generator=g).cuda()
+    ids = torch.stack([torch.randperm(E - 1, generator=g)[:top] for _ in range(T)])
+    offs, perm = S.moe_dispatch(ids.reshape(-1).to(torch.int32).cuda(), E)
+    n_out = ff // 2 if epi == 4 else ff
+    n = 64 * -(-n_out // 32) if epi == 4 else ff
+    w = (torch.randn(E, n, K, generator=g) / K ** 0.5).to(BF16).cuda()
+    sc = torch.rand(T * top, generator=g).cuda()
+    out = torch.zeros((T * top, n_out), device="cuda")
+    S.bgemm(x, w, out, T * top, n, K, batch=E, sbn=K, b_bs=n * K, grp_offs=offs, a_rows=perm, a_div=top, c_rows=perm, row_scale=sc, epi=epi, n_out=n_out if epi == 4 else 0)
+    y = torch.einsum("tk,tnk->tn", x.double().repeat_interleave(top, 0), w.double()[ids.reshape(-1).cuda()])
+    if epi == 4:
+        b = y.view(T * top, -1, 2, 32)
+        y = (torch.nn.functional.silu(b[:, :, 0]) * b[:, :, 1]).flatten(1)[:, :n_out]
+    elif epi == 1:
+        y = torch.relu(y) ** 2
+    want = y * sc.double()[:, None]
+    assert float((out.double() - want).norm() / want.norm()) < 2e-6  # fp32 sums of 200 products and the epilogue's few roundings
