@@ -379,6 +379,17 @@ int mi355_gated_delta_rule_bwd(int B, int S, int Hqk, int Hv, int Dk, int Dv, co
  * (the state gradient's starting value) and where d(loss) / d(initial_state) is left -- training through a carried recurrent state
  * (gated_delta_rule(..., prev_state), qwen3_next_attention.py:103-159).  The forward must have run with that initial_state and checkpoints. */
 
+/* The same rule in chunks of 64 tokens on the fp32 matrix pipe, for heads of 128 | 128 and the operands a layer makes (unit keys, 0 <= alpha <= 1; alpha below
+ * 1e-30 counts as 1e-30).  saved: mi355_gdr_chunked_saved_bytes, 16-byte aligned: the forward's scratch, and (keep != 0) what the backward reads; v's row pitch a
+ * multiple of 8; states as above.  The backward's workspace: mi355_gdr_chunked_bwd_workspace_bytes. */
+int64_t mi355_gdr_chunked_saved_bytes(int B, int S, int Hv);
+int64_t mi355_gdr_chunked_bwd_workspace_bytes(int B, int S, int Hqk, int Hv);
+int mi355_gdr_chunked_fwd(int B, int S, int Hqk, int Hv, const void* q, const void* k, const void* v, int64_t ldv, const float* beta, const float* alpha, void* o,
+                          float* saved, int64_t saved_bytes, int keep, const float* initial_state, float* final_state, void* stream);
+int mi355_gdr_chunked_bwd(int B, int S, int Hqk, int Hv, const void* q, const void* k, const void* v, int64_t ldv, const float* beta, const float* alpha, const float* saved,
+                          int64_t saved_bytes, const void* d_o, void* dq, void* dk, void* dv, int64_t lddv, float* dbeta, float* dalpha, void* workspace, int64_t workspace_bytes,
+                          const float* d_final_state, float* d_initial_state, void* stream);
+
 /* out = bf16(silu(float(gate)) * RMSNorm_fp32(float(o)))  (post_norm + output gate, qwen3_5_text_model.py:181-187): o bf16
  * [tokens, H*D], w fp32 [D], gate bf16 at gate[t*ldg + h*D]. */
 int mi355_gated_rmsnorm_fwd(int64_t tokens, int H, int D, const void* o, const float* w, const void* gate, int64_t ldg, void* out, float* rstd,

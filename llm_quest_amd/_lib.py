@@ -85,6 +85,8 @@ SIGNATURES = {
     "mi355_gated_delta_rule_fwd": [_I, _I, _I, _I, _I, _I, _P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _P],
     "mi355_causal_conv_silu_step": [_I, _I, _I, _P, _L, _P, _P, _P, _P],
     "mi355_gated_delta_rule_bwd": [_I, _I, _I, _I, _I, _I, _P, _P, _P, _L, _P, _P, _P, _P, _P, _P, _P, _L, _P, _P, _P, _L, _P, _P, _P],
+    "mi355_gdr_chunked_fwd": [_I, _I, _I, _I, _P, _P, _P, _L, _P, _P, _P, _P, _L, _I, _P, _P, _P],
+    "mi355_gdr_chunked_bwd": [_I, _I, _I, _I, _P, _P, _P, _L, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _P, _P, _L, _P, _P, _P],
     "mi355_gated_rmsnorm_fwd": [_L, _I, _I, _P, _P, _P, _L, _P, _P, _F, _P],
     "mi355_gated_rmsnorm_bwd": [_L, _I, _I, _P, _P, _P, _L, _P, _P, _P, _P, _L, _P, _I, _P],
     # input pipeline (csrc/pipeline.hip)
@@ -154,6 +156,8 @@ SIGNATURES = {
 QUERIES = {
     "mi355_gated_delta_rule_chunk": ([], _I),
     "mi355_gated_delta_rule_bwd_workspace_bytes": ([_I, _I, _I, _I, _I], _L),
+    "mi355_gdr_chunked_saved_bytes": ([_I, _I, _I], _L),
+    "mi355_gdr_chunked_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_rowconst_offset": ([_I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_qnorm_partials": ([_I, _I, _I], _L),

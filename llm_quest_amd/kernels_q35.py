@@ -264,16 +264,22 @@ def _check_gdr(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv):
             raise ValueError(f"gated_delta_rule: {n} must be contiguous fp32 [B*S, Hv]")
 
 
-def gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=True, want_state=False, state=None):
-    """Returns (o bf16 [B*S, Hv*Dv], checkpoints or None, final_state or None).  ``state`` fp32 [B, Hv, Dv, Dk]: carried-in recurrent
-    state, updated IN PLACE (and returned as final_state)."""
+GDR_CHUNKED_MIN = 64  # tokens from which the chunked kernels beat the token-by-token ones
+
+
+def gdr_chunked(v, S, Dk, Dv):
+    """Whether a layer's delta rule takes the chunked kernels (csrc/gdr_chunk.hip): heads of 128 | 128, value rows in 16-byte words, at least one whole chunk.
+    Both sides, forward + backward, 16 heads: one sequence of 64 tokens 151 / 139 us, of 333 779 / 240, four of 128 327 / 180, eight of 708 2 077 / 912."""
+    return Dk == 128 and Dv == 128 and S >= GDR_CHUNKED_MIN and v.stride(0) % 8 == 0 and v.data_ptr() % 16 == 0
+
+
+def gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=True, want_state=False, state=None, chunked=None):
+    """Returns (o bf16 [B*S, Hv*Dv], what the backward needs or None, final_state or None).  ``state`` fp32 [B, Hv, Dv, Dk]: carried-in recurrent
+    state, updated IN PLACE (and returned as final_state).  ``chunked``: False keeps to the token-by-token kernels whatever the sizes (operands that are not a layer's:
+    keys of any length, any alpha); default: ``gdr_chunked``."""
     L.require_gpu(q, k, v, beta, alpha)
     _check_gdr(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv)
     o = torch.empty((B * S, Hv * Dv), dtype=BF16, device=q.device)
-    ck = None
-    if keep:
-        ch = gdr_chunk()
-        ck = torch.empty((B, Hv, (S + ch - 1) // ch, Dv, Dk), dtype=F32, device=q.device)
     if state is not None:
         L.require_gpu(state)
         if not (state.dtype == F32 and state.is_contiguous() and tuple(state.shape) == (B, Hv, Dv, Dk)):
@@ -281,13 +287,21 @@ def gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=True,
         fin = state
     else:
         fin = torch.empty((B, Hv, Dv, Dk), dtype=F32, device=q.device) if want_state else None
+    if chunked is not False and gdr_chunked(v, S, Dk, Dv) and not (q.data_ptr() | k.data_ptr() | (0 if fin is None else fin.data_ptr())) % 16:
+        saved = torch.empty(L.load().mi355_gdr_chunked_saved_bytes(B, S, Hv) // 4, dtype=F32, device=q.device)
+        L.call("mi355_gdr_chunked_fwd", B, S, Hqk, Hv, L.ptr(q), L.ptr(k), L.ptr(v), v.stride(0), L.ptr(beta), L.ptr(alpha), L.ptr(o), L.ptr(saved), saved.numel() * 4, int(keep), L.ptr(state), L.ptr(fin))
+        return o, saved if keep else None, fin
+    ck = None
+    if keep:
+        ch = gdr_chunk()
+        ck = torch.empty((B, Hv, (S + ch - 1) // ch, Dv, Dk), dtype=F32, device=q.device)
     L.call("mi355_gated_delta_rule_fwd", B, S, Hqk, Hv, Dk, Dv, L.ptr(q), L.ptr(k), L.ptr(v), v.stride(0), L.ptr(beta), L.ptr(alpha), L.ptr(o), L.ptr(ck), L.ptr(state), L.ptr(fin))
     return o, ck, fin
 
 
 def gated_delta_rule_bwd(q, k, v, beta, alpha, ck, do, dv, B, S, Hqk, Hv, Dk, Dv, d_final=None, want_d_initial=False):
-    """dv: destination view [B*S, Hv*Dv].  Returns (dq, dk bf16 [B*S, Hqk*Dk], dbeta, dalpha fp32 [B*S, Hv]) -- and, with ``want_d_initial``, the fp32
-    [B, Hv, Dv, Dk] gradient of the carried-in state as a fifth element.  ``d_final``: the gradient arriving at the forward's final state (or None)."""
+    """dv: destination view [B*S, Hv*Dv]; ck: the forward's second result.  Returns (dq, dk bf16 [B*S, Hqk*Dk], dbeta, dalpha fp32 [B*S, Hv]) -- and, with ``want_d_initial``,
+    the fp32 [B, Hv, Dv, Dk] gradient of the carried-in state as a fifth element.  ``d_final``: the gradient arriving at the forward's final state (or None)."""
     L.require_gpu(q, k, v, beta, alpha, ck, do, dv, d_final)
     if d_final is not None and not (d_final.dtype == F32 and d_final.is_contiguous() and tuple(d_final.shape) == (B, Hv, Dv, Dk)):
         raise ValueError("gated_delta_rule_bwd: d_final must be contiguous fp32 [B, Hv, Dv, Dk]")
@@ -295,6 +309,21 @@ def gated_delta_rule_bwd(q, k, v, beta, alpha, ck, do, dv, B, S, Hqk, Hv, Dk, Dv
     _cols(dv, "gated_delta_rule_bwd(dv)")
     if not (do.dtype == BF16 and do.is_contiguous() and tuple(do.shape) == (B * S, Hv * Dv)) or tuple(dv.shape) != (B * S, Hv * Dv):
         raise ValueError("gated_delta_rule_bwd: do contiguous bf16 [B*S, Hv*Dv], dv a view of that shape")
+    dq = torch.empty_like(q)
+    dk = torch.empty_like(k)
+    dbeta = torch.empty_like(beta)
+    dalpha = torch.empty_like(alpha)
+    d_init = torch.empty((B, Hv, Dv, Dk), dtype=F32, device=q.device) if want_d_initial else None
+    if ck.dim() == 1:  # the chunked forward's
+        if do.data_ptr() % 16:
+            do = do.clone()
+        if d_final is not None and d_final.data_ptr() % 16:
+            d_final = d_final.clone()
+        need = L.load().mi355_gdr_chunked_bwd_workspace_bytes(B, S, Hqk, Hv)
+        ws = torch.empty(need // 4, dtype=F32, device=q.device)
+        L.call("mi355_gdr_chunked_bwd", B, S, Hqk, Hv, L.ptr(q), L.ptr(k), L.ptr(v), v.stride(0), L.ptr(beta), L.ptr(alpha), L.ptr(ck), ck.numel() * 4, L.ptr(do), L.ptr(dq), L.ptr(dk),
+               L.ptr(dv), dv.stride(0), L.ptr(dbeta), L.ptr(dalpha), L.ptr(ws), need, L.ptr(d_final), L.ptr(d_init))
+        return (dq, dk, dbeta, dalpha, d_init) if want_d_initial else (dq, dk, dbeta, dalpha)
     need = L.load().mi355_gated_delta_rule_bwd_workspace_bytes(B, S, Hv, Dk, Dv)
     key = str(q.device)
     ws = _WS.get(key)
@@ -302,11 +331,6 @@ def gated_delta_rule_bwd(q, k, v, beta, alpha, ck, do, dv, B, S, Hqk, Hv, Dk, Dv
         _WS.pop(key, None)
         ws = torch.empty((need + 3) // 4, dtype=F32, device=q.device)
         _WS[key] = ws
-    dq = torch.empty_like(q)
-    dk = torch.empty_like(k)
-    dbeta = torch.empty_like(beta)
-    dalpha = torch.empty_like(alpha)
-    d_init = torch.empty((B, Hv, Dv, Dk), dtype=F32, device=q.device) if want_d_initial else None
     L.call("mi355_gated_delta_rule_bwd", B, S, Hqk, Hv, Dk, Dv, L.ptr(q), L.ptr(k), L.ptr(v), v.stride(0), L.ptr(beta), L.ptr(alpha), L.ptr(ck), L.ptr(do),
            L.ptr(dq), L.ptr(dk), L.ptr(dv), dv.stride(0), L.ptr(dbeta), L.ptr(dalpha), L.ptr(ws), ws.numel() * 4, L.ptr(d_final), L.ptr(d_init))
     return (dq, dk, dbeta, dalpha, d_init) if want_d_initial else (dq, dk, dbeta, dalpha)

@@ -358,7 +358,7 @@ class GatedDeltaRuleFn(torch.autograd.Function):
         al = alpha.to(F32).permute(0, 2, 1).reshape(b * s, h).contiguous()
         # a carried-in state (reference :103: prev_state) is copied: the kernel advances the state in place, the caller's tensor stays as it was
         state = None if prev_state is None else prev_state.detach().to(F32).contiguous().clone()
-        o, ck, fin = Q.gated_delta_rule_fwd(q2, k2, v2, be, al, b, s, h, h, dk, dv, keep=True, want_state=True, state=state)
+        o, ck, fin = Q.gated_delta_rule_fwd(q2, k2, v2, be, al, b, s, h, h, dk, dv, keep=True, want_state=True, state=state, chunked=False)
         ctx.saved = (q2, k2, v2, be, al, ck)
         ctx.meta = (b, h, s, dk, dv, q.dtype, k.dtype, v.dtype, beta.dtype, alpha.dtype, None if prev_state is None else prev_state.dtype)
         ctx.set_materialize_grads(False)  # an unused last state arrives as None, not as a zero tensor the kernel would have to read

@@ -733,3 +733,56 @@ def test_gated_delta_rule_trains_through_a_carried_state(dk, dv, s1, s2):
     assert torch.equal(torch.cat([oa, ob], dim=2), o1) or rel_l2(torch.cat([oa, ob], dim=2), o1) < 2e-3
     for name, two, one in zip(("q", "k", "v", "beta", "alpha", "prev_state"), c, a):
         assert rel_l2(two.grad, one.grad) < 6e-3, (name, rel_l2(two.grad, one.grad))
+
+
+# ------------------------------------------------------------------------------------------------- the chunked kernels of the gated delta rule
+@pytest.mark.parametrize("b,hqk,hv,s,decay", [(1, 1, 1, 64, "mix"), (2, 1, 2, 65, "mix"), (1, 2, 2, 127, "slow"), (1, 1, 3, 128, "tiny"), (2, 2, 2, 200, "zero"), (1, 1, 1, 333, "keys")])
+def test_chunked_gated_delta_rule_matches_the_token_by_token_kernels(b, hqk, hv, s, decay):
+    """csrc/gdr_chunk.hip against the sequential kernels on the same operands (one chunk, chunks with a remainder, shared q / k heads; decays near one, far below fp32's
+    resolution of their sums, and exactly zero; nearly parallel keys), carried-in state and its gradient included.  bf16 results: a rounding flips where two fp32 sums
+    straddle a boundary (2^-9 of few elements); fp32 results: both sides are sums of 64 ... 128 fp32 products behind at most 64 steps of substitution."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    g = torch.Generator().manual_seed(s + hv)
+    D = 128
+    keys = torch.randn(b, s, hqk, D, generator=g) + (3.0 if decay == "keys" else 0.0)
+    q = torch.nn.functional.normalize(torch.randn(b, s, hqk, D, generator=g), dim=-1).to(BF16).reshape(b * s, -1).cuda()
+    k = torch.nn.functional.normalize(keys, dim=-1).to(BF16).reshape(b * s, -1).cuda()
+    wide = torch.randn(b * s, hv * D + 8, generator=g).to(BF16).cuda()
+    v = wide[:, : hv * D]
+    be = torch.sigmoid(torch.randn(b * s, hv, generator=g)).cuda()
+    rate = {"slow": -9.0, "tiny": 2.5}.get(decay, -3.0)
+    al = torch.exp(-torch.exp(rate + 2.0 * torch.rand(b * s, hv, generator=g))).cuda()
+    if decay == "zero":
+        al[::7] = 0.0
+    go = torch.randn(b * s, hv * D, generator=g).to(BF16).cuda()
+    s0, gs = (0.1 * torch.randn(b, hv, D, D, generator=g)).cuda(), (0.1 * torch.randn(b, hv, D, D, generator=g)).cuda()
+    out = []
+    for chunked in (False, None):
+        assert Q.gdr_chunked(v, s, D, D)
+        o, ck, fin = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, hqk, hv, D, D, state=s0.clone(), chunked=chunked)
+        assert (ck.dim() == 1) == (chunked is None)
+        dv = torch.zeros_like(wide)
+        res = Q.gated_delta_rule_bwd(q, k, v, be, al, ck, go, dv[:, : hv * D], b, s, hqk, hv, D, D, d_final=gs, want_d_initial=True)
+        assert bool((dv[:, hv * D :] == 0).all())
+        o2, ck2, fin2 = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, hqk, hv, D, D, keep=False, state=s0.clone(), chunked=chunked)
+        assert ck2 is None and torch.equal(o, o2) and torch.equal(fin, fin2)
+        out.append((o, res[0], res[1], dv[:, : hv * D], fin, res[2], res[3], res[4]))
+    for i, (one, two) in enumerate(zip(*out)):
+        if i == 6 and decay == "zero":  # d(alpha) where alpha is zero: the sums that span such a token hold alpha itself (as 1e-30), its factor at fp32's lower end
+            keep = al > 0
+            one, two = one[keep], two[keep]
+        assert bool(torch.isfinite(two.float()).all()) and rel_l2(two, one) < (1e-3 if i < 4 else 2e-6), (i, rel_l2(two, one))
+
+
+def test_chunked_gated_delta_rule_refuses_what_it_cannot_read():
+    from llm_quest_amd import _lib as L
+    from llm_quest_amd import kernels_q35 as Q
+
+    t = torch.zeros(64 * 130, dtype=BF16, device="cuda")
+    assert not Q.gdr_chunked(t.view(64, 130)[:, :128], 64, 128, 128) and not Q.gdr_chunked(t[1:].view(-1)[: 64 * 128].view(64, 128), 64, 128, 128)
+    assert not Q.gdr_chunked(torch.zeros(63, 128, dtype=BF16, device="cuda"), 63, 128, 128) and not Q.gdr_chunked(torch.zeros(64, 16, dtype=BF16, device="cuda"), 64, 16, 16)
+    x, f = torch.zeros(64, 128, dtype=BF16, device="cuda"), torch.zeros(64, 1, device="cuda")
+    L.require_gpu(x)
+    with pytest.raises(RuntimeError, match="too small"):
+        L.call("mi355_gdr_chunked_fwd", 1, 64, 1, 1, L.ptr(x), L.ptr(x), L.ptr(x), 128, L.ptr(f), L.ptr(f), L.ptr(x), L.ptr(f), 16, 0, None, None)
