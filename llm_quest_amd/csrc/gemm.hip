@@ -2377,6 +2377,20 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         cfg = (pp_mask() & kind_bit) ? 8 : 7;
         if (walk_on(N, K)) p.ablate |= 8;
     }
+    // A last round of few 256x256 tiles costs as much as a full one.  Where they are few -- one to three full rounds and a remainder that 128x128 tiles (split over K as ever)
+    // cover with at most one workgroup per CU -- the row panels of the full rounds go first and the remaining rows follow on the small tiles.  17 016 rows (24 samples of 709
+    // tokens), N = 1024 (268 tiles), us, one launch -> two: K = 2048 109 -> 76, 3072 150 -> 102, 4096 187 -> 127, 6144 278 -> 182; N = 2048 (536 tiles) 82 -> 74; 25 216 rows,
+    // N = 768 (297 tiles): K = 768 53 -> 42, 3072 147 -> 119.  Four rounds and more gain nothing (1072 tiles 131 / 132) or lose (1188 tiles 109 / 118: a remainder of 648 small tiles).
+    if (tile_hint == 0 && ablate == 0 && !split3 && form != MI355_GEMM_TN && (cfg == 2 || cfg == 3 || cfg == 7)) {
+        const int64_t tn = (N + 255) / 256, tiles256 = ((M + 255) / 256) * tn, rounds = tiles256 / 256, m_main = rounds * 256 / tn * 256;
+        const int64_t tail128 = ((M - m_main + 127) / 128) * ((N + 127) / 128), most[4] = {0, 256, 160, 128};
+        if (rounds >= 1 && rounds <= 3 && tiles256 % 256 != 0 && m_main >= 256 && m_main < M && tail128 <= most[rounds]) {
+            const int64_t esz = out_dtype == MI355_DT_F32 ? 4 : 2, rsz = epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_GELU_ERF ? esz : 2;
+            if (int rc = mi355_gemm_bf16(form, m_main, N, K, A, lda, B, ldb, C, ldc, out_dtype, bias, residual, ldr, epilogue, workspace, workspace_bytes, 0, stream)) return rc;
+            return mi355_gemm_bf16(form, M - m_main, N, K, (const bf16_t*)A + m_main * lda, lda, B, ldb, (char*)C + m_main * ldc * esz, ldc, out_dtype, bias,
+                                   residual ? (const char*)residual + m_main * ldr * rsz : nullptr, ldr, epilogue, workspace, workspace_bytes, 1, stream);
+        }
+    }
     if (cfg == 8) {  // ping-pong form: needs at least as many K-tiles as write-out slots
         if (persist_ok && K >= 64 * 5) return mi355_gemm_pp_part6(&p, s);
         cfg = 7;

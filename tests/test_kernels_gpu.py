@@ -1122,3 +1122,36 @@ def test_embedding_backward_sorted_long_runs_span_blocks(K, T):
     assert torch.equal(got[~named], torch.full((V, W), 7.0).to(BF16)[~named])
     err = (got[named].double() - ref[named]).abs().max() / ref[named].abs().max()
     assert err < 6e-3, float(err)  # one bf16 rounding of sums of up to thousands of rows
+
+
+@pytest.mark.parametrize("form,M,N,K,case", [("nt", 17016, 1024, 128, "res"), ("nn", 17016, 1024, 64, "plain"), ("nt", 16386, 1024, 72, "f32"), ("nt", 25216, 768, 192, "bias_gelu"),
+                                             ("nt", 33000, 1024, 128, "plain"), ("nt", 17016, 3072, 128, "plain"), ("nt", 3000, 6144, 128, "swiglu"), ("nt", 16385, 1016, 128, "res")])
+def test_products_in_two_launches_equal_one(form, M, N, K, case):
+    """Full rounds on 256x256 tiles, the rows behind them on 128x128 tiles: the same numbers as the large tile alone (small-integer operands: every sum is exact), no row missed or
+    written twice, operands and outputs in wider rows."""
+    from llm_quest_amd import _lib as L
+    from llm_quest_amd import kernels as KK
+
+    g = torch.Generator(device="cuda").manual_seed(M + N)
+    ints = lambda r, c, pad=0: torch.randint(-2, 3, (r, c + pad), generator=g, device="cuda").to(torch.bfloat16)[:, :c]
+    a = ints(M, K, 8)
+    b = ints(N, K, 8) if form == "nt" else ints(K, N)
+    f = L.GEMM_NT if form == "nt" else L.GEMM_NN
+    if case == "swiglu":
+        gu, act = KK.gemm_gateup_swiglu(a.contiguous(), b.contiguous())
+        one = KK.gemm(f, a, b, tile=2)
+        assert torch.equal(gu, one) and torch.equal(act, KK.swiglu_fwd(one, N // 2))
+        return
+    dt = torch.float32 if case == "f32" else torch.bfloat16
+    kw = {}
+    if case == "res":
+        kw["residual"] = ints(M, N, 8)
+    if case == "bias_gelu":
+        kw.update(bias=torch.randint(-2, 3, (N,), generator=g, device="cuda").float(), gelu=True)
+    outs = []
+    for tile in (0, 2 if form == "nt" else 3):
+        buf = torch.full((M + 1, N + 8), 7.0, dtype=dt, device="cuda")
+        KK.gemm(f, a, b, out=buf[:M, :N], tile=tile, **kw)
+        assert bool((buf[M] == 7).all()) and bool((buf[:, N:] == 7).all())
+        outs.append(buf[:M, :N])
+    assert torch.equal(*outs)
