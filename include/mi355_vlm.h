@@ -633,6 +633,15 @@ int mi355_qkv_rows_append(int64_t tokens, int H, int G, int d, int dv, const voi
 int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
                             int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
                             const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream);
+/* The same rule -- or, with head_decay, linear attention with one decay per head (k times kscale, q times qscale) -- in chunks of 64 tokens on the fp32 matrix pipe:
+ * heads of 128 | 128, fp32 rows, state fp32 [slots, H, 128, 128] read and written at slot.  tok: mi355_delta_rule_tokens' result (four floats per token and head).
+ * max_new: the most new tokens of one sequence.  workspace: mi355_delta_chunked_workspace_bytes, 16-byte aligned. */
+int mi355_delta_rule_tokens(int64_t tokens, int H, int G, int dk, const void* q, const void* k, int qk_dt, int64_t ldq, int64_t ldk, const void* b, const void* a, int ba_dt,
+                            int64_t ldb, int64_t lda, const float* A_log, const float* dt_bias, float qscale, float* ws, void* stream);
+int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H);
+int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
+                        const float* v, int64_t ldv, const float* tok, const float* head_decay, float qscale, float kscale, float* state, float* o, void* workspace,
+                        int64_t workspace_bytes, void* stream);
 /* Gated feed-forward activation on rows [gate (F) | up (F)] -> [F].  kind 0: gelu_tanh(gate) * up.  kind 1: g = min(gate, limit), u = clamp(up, -limit, limit),
  * g * sigmoid(1.702 g) * (u + 1).  kind 2: silu(gate) * up. */
 int mi355_glu_rows(int64_t rows, int F, const void* in, int in_dt, int64_t ld_in, int kind, float limit, void* out, int out_dt, int64_t ld_out, void* stream);

@@ -108,6 +108,8 @@ SIGNATURES = {
     "mi355_embed_hash_fwd": [_L, _I, _I, _P, _P, _P, _F, _P, _I, _I, _I, _P, _P],
     "mi355_add_layernorm_fwd": [_L, _I, _P, _F, _P, _I, _L, _I, _P, _P, _F, _P, _P, _I, _P],
     "mi355_rmsnorm_rows": [_L, _I, _P, _I, _L, _P, _F, _P, _I, _L, _P],
+    "mi355_delta_rule_tokens": [_L, _I, _I, _I, _P, _P, _I, _L, _L, _P, _P, _I, _L, _L, _P, _P, _F, _P, _P],
+    "mi355_delta_chunked": [_L, _I, _I, _P, _P, _I, _I, _P, _L, _P, _L, _P, _L, _P, _P, _F, _F, _P, _P, _P, _L, _P],
     "mi355_latent_kv_append": [_L, _I, _I, _P, _I, _L, _P, _F, _P, _P, _P, _I, _I, _P, _I, _L, _P],
     "mi355_rope_heads": [_L, _I, _I, _P, _I, _L, _I, _I, _P, _L, _I, _I, _I, _I, _I, _P, _P, _P],
     "mi355_gated_headnorm": [_L, _I, _I, _P, _P, _P, _I, _L, _F, _P, _I, _L, _P],
@@ -156,6 +158,7 @@ SIGNATURES = {
 QUERIES = {
     "mi355_gated_delta_rule_chunk": ([], _I),
     "mi355_gated_delta_rule_bwd_workspace_bytes": ([_I, _I, _I, _I, _I], _L),
+    "mi355_delta_chunked_workspace_bytes": ([_L, _I, _I], _L),
     "mi355_gdr_chunked_saved_bytes": ([_I, _I, _I], _L),
     "mi355_gdr_chunked_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),

@@ -368,7 +368,7 @@ class Retention(_Frozen):
         qk = torch.empty((h.shape[0], b), dtype=F32, device=h.device)
         S.rope_heads(proj, 2 * H, dk, dk, 0, qk, dk, 0, 0, self.rot_dims, self.freq, st.pos, layout=1)  # q and k heads side by side: 2 H heads of dim
         o = S.gla(qk[:, :a], qk[:, a:b], proj[:, b:c], None, None, 1.0, 1.0, st.seq_off, st.slots, st.cache.state(self.layer_idx, "S"), H, dk, dv,
-                  head_decay=self.decay32, kscale=dk ** -0.5)
+                  head_decay=self.decay32, kscale=dk ** -0.5, max_new=st.max_new)
         mix = S.gated_headnorm(o, self.ones, proj[:, c:], H, dv, self.eps, st.act_dtype)
         return S.linear(mix, self.w_o)
 
@@ -556,7 +556,7 @@ class GatedDeltaRule(_Frozen):
         a, b = G * dk, 2 * G * dk
         gate0 = C + H * dv
         o = S.delta_rule(qkv[:, :a], qkv[:, a:b], qkv[:, b:], proj[:, gate0 : gate0 + H], proj[:, gate0 + H :], self.A_log32, self.dt_bias32, dk ** -0.5, st.seq_off, st.slots,
-                         st.cache.state(self.layer_idx, "S"), H, G, dk, dv)
+                         st.cache.state(self.layer_idx, "S"), H, G, dk, dv, max_new=st.max_new)
         mix = S.gated_headnorm(o, self.norm32, proj[:, C:gate0], H, dv, self.eps, st.act_dtype)
         return S.linear(mix, self.w_o)
 

@@ -1,0 +1,269 @@
+// Linear recurrences of served decoders over the new tokens of a ragged batch, in chunks of 64 tokens on the fp32 matrix pipe (gfx950 only), heads of 128 | 128:
+// the gated delta rule (unit keys, decay and beta per token) and retention (one decay per head, no correction).  The mathematics of a chunk is that of gdr_chunk.hip;
+// here operands are fp32 rows of a packed batch, the state is [dk][dv] per slot, and nothing is kept for a backward pass.
+//     delta:      U = R (b V) - Kw S,  O = gam q S + P U,  S <- gam_63 S + (Gp K)^T U
+//     retention:  U = V,               the same
+// A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
+// the chip could multiply; the chunks take 363 us (prep 142, scan 203) and 183 us (scan 173).  Bound: the scan's chain of chunks (two products behind two barriers each), not the
+// pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
+// (A row that is not finite makes the rows before it in its own chunk NaN as well: the triangle's zeros are multiplied, not skipped.  The rows after it are lost either way.)
+#include "gdr_chunk.h"
+
+#define ST(s) ((hipStream_t)(s))
+
+namespace {
+
+// one chunk of one head in the workspace (floats): Kw [64][128], Uv [64][128] (delta only), P [64][64], then per token gam x query factor, Gp x key factor, and the chunk's decay
+constexpr int D_KW = 0, D_U = GC * GD, D_P = 2 * GC * GD, D_G = D_P + GC * GC, D_BLOCK = D_G + 2 * GC + 4;
+
+struct DChunkArgs {
+    const int *seq_off, *slot;
+    const float *q, *k, *v;
+    int64_t ldq, ldk, ldv;
+    const f32x4* tok;         // delta: [tokens, H] decay, beta, key factor, query factor
+    const float* head_decay;  // retention: [H]
+    float qscale, kscale;     // retention
+    int H, G, heads;  // heads: of all sequences
+    float *state, *o, *ws;
+};
+
+// chunks are packed: those of sequence s start at seq_off[s] / 64 + s (never less than the sum of the sequences' chunks before it)
+__device__ __forceinline__ float* chunk_block(const DChunkArgs& p, int s, int h, int n) { return p.ws + ((int64_t)(p.seq_off[s] / GC + s + n) * p.H + h) * D_BLOCK; }
+
+template <bool DELTA>
+__global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
+    __shared__ __attribute__((aligned(16))) float Ks[GC][GD + 4];
+    __shared__ __attribute__((aligned(16))) float N[DELTA ? GC : 1][GC + 4];
+    __shared__ __attribute__((aligned(16))) float T[DELTA ? GC : 1][GC + 4];
+    __shared__ double gd[GC];
+    __shared__ float be[GC], gam[GC], qf[GC];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
+    const int n = blockIdx.x, h = blockIdx.y, s = blockIdx.z, hq = h / (p.H / p.G), t0 = p.seq_off[s] + n * GC, cnt = min(GC, p.seq_off[s + 1] - t0);
+    if (cnt <= 0) return;
+    const float *qp = p.q + (int64_t)t0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)t0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)t0 * p.ldv + (int64_t)h * GD;
+    float* blk = chunk_block(p, s, h, n);
+    if (wave == 0) {
+        f32x4 c = {1.f, 0.f, 0.f, 0.f};
+        if (lane < cnt) {
+            if (DELTA) c = p.tok[((int64_t)t0 + lane) * p.H + h];
+            else c = f32x4{p.head_decay[h], 1.f, p.kscale, p.qscale};
+        }
+        const double g = cumulated_log64(decay_at_least(c[0])), g63 = __shfl(g, 63, 64);
+        gd[lane] = g;
+        be[lane] = c[1];
+        gam[lane] = expf((float)g);
+        qf[lane] = c[3];
+        blk[D_G + lane] = expf((float)g) * c[3];
+        blk[D_G + GC + lane] = expf((float)(g63 - g)) * c[2];
+        if (lane == 0) blk[D_G + 2 * GC] = expf((float)g63);
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {  // keys, made unit vectors (resp. scaled) on the way
+        const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
+        f32x4 kv = {0.f, 0.f, 0.f, 0.f};
+        if (r < cnt) kv = *reinterpret_cast<const f32x4*>(kp + r * p.ldk + c) * (DELTA ? p.tok[((int64_t)t0 + r) * p.H + h][2] : p.kscale);
+        *reinterpret_cast<f32x4*>(&Ks[r][c]) = kv;
+    }
+    __syncthreads();
+    {  // K K^T and Q K^T: wave = tile (ti, tj); the tile above the diagonal is zero
+        const int ti = wave >> 1, tj = wave & 1;
+        f32x16 kk = zero16(), qk = zero16();
+        if (wave != 1) {
+            const int qr = 32 * ti + ln;
+#pragma unroll 4
+            for (int c = 0; c < GD; c += 8) {
+                const f32x4 qv = qr < cnt ? *reinterpret_cast<const f32x4*>(qp + qr * p.ldq + c + 4 * hf) : f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 bv = *reinterpret_cast<const f32x4*>(&Ks[32 * tj + ln][c + 4 * hf]);
+                const f32x4 av = *reinterpret_cast<const f32x4*>(&Ks[32 * ti + ln][c + 4 * hf]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    qk = mfma2(qv[j], bv[j], qk);
+                    if (DELTA) kk = mfma2(av[j], bv[j], kk);
+                }
+            }
+        }
+        const int j = 32 * tj + ln;
+        const double gj = gd[j];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int i = 32 * ti + c_row(e, hf);
+            const float D = i >= j ? expf((float)(gd[i] - gj)) : 0.f;
+            if (DELTA) N[i][j] = i > j ? be[i] * kk[e] * D : 0.f;
+            blk[D_P + i * GC + j] = i >= j ? qf[i] * qk[e] * D : 0.f;
+        }
+    }
+    if constexpr (DELTA) {
+        __syncthreads();
+        invert_unit_lower64(N, T);
+        // Uv = R (b V), Kw = R (b gam K): wave = 32 columns, both row halves (the upper one ends at token 32)
+        f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16();
+        const int col = 32 * wave + ln;
+#pragma unroll 2
+        for (int kb = 0; kb < GC; kb += 8) {
+            const f32x4 a1 = *reinterpret_cast<const f32x4*>(&T[32 + ln][kb + 4 * hf]);
+            f32x4 a0 = {0.f, 0.f, 0.f, 0.f};
+            if (kb < 32) a0 = *reinterpret_cast<const f32x4*>(&T[ln][kb + 4 * hf]);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int t = kb + 4 * hf + j;
+                const float bv = t < cnt ? vp[t * p.ldv + col] * be[t] : 0.f, bk = Ks[t][col] * (be[t] * gam[t]);
+                u1 = mfma2(a1[j], bv, u1);
+                w1 = mfma2(a1[j], bk, w1);
+                if (kb < 32) {
+                    u0 = mfma2(a0[j], bv, u0);
+                    w0 = mfma2(a0[j], bk, w0);
+                }
+            }
+        }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {
+            const int r = c_row(e, hf);
+            blk[D_U + r * GD + col] = u0[e];
+            blk[D_U + (32 + r) * GD + col] = u1[e];
+            blk[D_KW + r * GD + col] = w0[e];
+            blk[D_KW + (32 + r) * GD + col] = w1[e];
+        }
+    }
+}
+
+// One workgroup per sequence, head and 32 value columns, chunk by chunk.  Waves 0, 1 take Kw S (row halves), waves 2, 3 q S and then P U; the state's four tiles of 32 key
+// channels go one to a wave.
+template <bool DELTA>
+__global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
+    __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];  // [value column][key channel]
+    __shared__ __attribute__((aligned(16))) float Us[GC][GV + 8];
+    __shared__ __attribute__((aligned(16))) float Ks[GC][GD + 4];
+    __shared__ float gg[2 * GC], gC;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
+    // the four value ranges of a head read the same rows: to one XCD (workgroups are dealt to the eight XCDs in turn), side by side
+    const int id = blockIdx.x, at = (id >> 5) * 8 + (id & 7), v0 = ((id >> 3) & 3) * GV;
+    if (at >= p.heads) return;
+    const int h = at % p.H, s = at / p.H, hq = h / (p.H / p.G), s0 = p.seq_off[s], len = p.seq_off[s + 1] - s0, NC = (len + GC - 1) / GC;
+    const bool qside = wave >= 2;
+    const float *qp = p.q + (int64_t)s0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)s0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)s0 * p.ldv + (int64_t)h * GD + v0;
+    float* state = p.state + ((int64_t)p.slot[s] * p.H + h) * GD * GD + v0;
+    if (NC <= 0) return;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;
+        Ss[c][r] = state[(int64_t)r * GD + c];
+    }
+    for (int n = 0; n < NC; ++n) {
+        const float* blk = chunk_block(p, s, h, n);
+        const int t0 = n * GC, cnt = min(GC, len - t0);
+        // a Kw row (waves 0, 1) or a q row (waves 2, 3) in fragment form, eight words in flight
+        const int row = 32 * rh + ln;
+        const float* src = qside ? qp + (t0 + row) * p.ldq + 4 * hf : DELTA ? blk + D_KW + row * GD + 4 * hf : nullptr;
+        if (qside && row >= cnt) src = nullptr;
+        f32x4 fr[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) fr[i] = src ? *reinterpret_cast<const f32x4*>(src + 8 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+        __syncthreads();  // the state is whole, the last chunk's keys and U are read
+        f32x4 kr[8], pr[8];
+        float uv[16];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
+            kr[i] = r < cnt ? *reinterpret_cast<const f32x4*>(kp + (t0 + r) * p.ldk + c) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (!qside) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = 32 * rh + c_row(e, hf);
+                if (DELTA) uv[e] = blk[D_U + r * GD + v0 + ln];
+                else uv[e] = r < cnt ? vp[(t0 + r) * p.ldv + ln] : 0.f;
+            }
+        }
+        if (tid < 2 * GC) gg[tid] = blk[D_G + tid];
+        if (tid == 0) gC = blk[D_G + 2 * GC];
+        f32x16 acc = zero16();
+        if (DELTA || qside) {
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                const f32x4 c = *reinterpret_cast<const f32x4*>(&Ss[ln][8 * i + 4 * hf]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc = mfma2(fr[i % 8][j], c[j], acc);
+                if (i < 8) fr[i] = src ? *reinterpret_cast<const f32x4*>(src + 8 * (i + 8)) : f32x4{0.f, 0.f, 0.f, 0.f};
+                if (i % 4 == 3) asm volatile("" ::: "memory");  // keep the state reads of later steps where they are: all sixteen at once cost more registers than there are
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
+            *reinterpret_cast<f32x4*>(&Ks[r][c]) = kr[i];
+        }
+        if (qside) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pr[i] = *reinterpret_cast<const f32x4*>(blk + D_P + (32 * rh + ln) * GC + 8 * i + 4 * hf);
+        } else {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) Us[32 * rh + c_row(e, hf)][ln] = uv[e] - acc[e];
+        }
+        __syncthreads();
+        if (qside) {
+#pragma unroll
+            for (int e = 0; e < 16; ++e) acc[e] *= gg[32 * rh + c_row(e, hf)];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                if (rh == 0 && i >= 4) break;  // P is lower triangular
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc = mfma2(pr[i][j], Us[8 * i + 4 * hf + j][ln], acc);
+            }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int r = 32 * rh + c_row(e, hf);
+                if (r < cnt) p.o[((int64_t)s0 + t0 + r) * p.H * GD + (int64_t)h * GD + v0 + ln] = acc[e];
+            }
+        }
+        f32x16 c;
+#pragma unroll
+        for (int e = 0; e < 16; ++e) c[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
+#pragma unroll 2
+        for (int kb = 0; kb < GC; kb += 8)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int t = kb + 4 * hf + j;
+                c = mfma2(Us[t][ln] * gg[GC + t], Ks[t][32 * wave + ln], c);
+            }
+#pragma unroll
+        for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = c[e];  // read by this wave alone since the last barrier
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+        const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;
+        state[(int64_t)r * GD + c] = Ss[c][r];
+    }
+}
+
+}  // namespace
+
+extern "C" int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H) {
+    return tokens > 0 && n_seq > 0 && H > 0 ? (tokens / GC + n_seq) * (int64_t)H * D_BLOCK * 4 : 0;
+}
+
+extern "C" int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
+                                   const float* v, int64_t ldv, const float* tok, const float* head_decay, float qscale, float kscale, float* state, float* o, void* workspace,
+                                   int64_t workspace_bytes, void* stream) {
+    MI355_REQUIRE(tokens > 0 && n_seq > 0 && n_seq <= 65535 && (int64_t)n_seq * H <= (1 << 26) && max_new > 0 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && q && k && v && state && o && workspace &&
+                      (tok != nullptr) != (head_decay != nullptr),
+                  "delta_chunked: bad arguments (either a decay per head or four numbers per token and head)");
+    MI355_REQUIRE(ldq >= (int64_t)G * GD && ldk >= (int64_t)G * GD && ldv >= (int64_t)H * GD && ldq % 4 == 0 && ldk % 4 == 0, "delta_chunked: rows too short, or query / key pitches no multiple of 4");
+    MI355_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)tok | (uintptr_t)workspace) & 15) == 0, "delta_chunked: queries, keys and the workspace must be 16-byte aligned");
+    MI355_REQUIRE(workspace_bytes >= mi355_delta_chunked_workspace_bytes(tokens, n_seq, H), "delta_chunked: workspace too small (%lld bytes)", (long long)workspace_bytes);
+    DChunkArgs p;
+    p.seq_off = seq_off, p.slot = slot, p.q = q, p.k = k, p.v = v, p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.tok = (const f32x4*)tok, p.head_decay = head_decay;
+    p.qscale = qscale, p.kscale = kscale, p.H = H, p.G = G, p.heads = n_seq * H, p.state = state, p.o = o, p.ws = (float*)workspace;
+    const dim3 prep((max_new + GC - 1) / GC, H, n_seq), scan((unsigned)((n_seq * (int64_t)H + 7) / 8 * 32));
+    if (tok) {
+        dchunk_prep_kernel<true><<<prep, 256, 0, ST(stream)>>>(p);
+        MI355_LAUNCH_CHECK("delta_chunked(prep)");
+        dchunk_scan_kernel<true><<<scan, 256, 0, ST(stream)>>>(p);
+    } else {
+        dchunk_prep_kernel<false><<<prep, 256, 0, ST(stream)>>>(p);
+        MI355_LAUNCH_CHECK("delta_chunked(prep)");
+        dchunk_scan_kernel<false><<<scan, 256, 0, ST(stream)>>>(p);
+    }
+    MI355_LAUNCH_CHECK("delta_chunked");
+    return 0;
+}

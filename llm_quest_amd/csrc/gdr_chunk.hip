@@ -11,54 +11,35 @@
 // in fp64, so a difference of two large ones keeps its digits.  d(alpha) is taken from sums over the pairs that span a token -- never as a difference of
 // larger sums, so it keeps its digits where alpha is tiny (below 1e-30 alpha counts as 1e-30).
 // Bound: the fp32 matrix pipe (256 FLOP a clock and CU).  The products of one 64-token chunk of one head: 37 MFLOP forward and backward together.
-#include "common.h"
-#include "lane_sums.h"
+#include "gdr_chunk.h"
 
 #define ST(s) ((hipStream_t)(s))
 
 namespace {
 
-constexpr int GC = 64, GD = 128, GV = 32;  // tokens of a chunk, head width (keys and values), value rows of a scan's workgroup
 // one chunk of one head in the saved buffer (floats): state at its start [128 dv][128 dk], Kw [64][128], U [64][128], P [64][64], R [64][64], gam [64], Gp [64]
 constexpr int G_KW = GD * GD, G_U = G_KW + GC * GD, G_P = G_U + GC * GD, G_R = G_P + GC * GC, G_GAM = G_R + GC * GC, G_BLOCK = G_GAM + 2 * GC;
 constexpr int W_DU = GD * GD, W_BLOCK = W_DU + GC * GD;  // backward workspace of a chunk: dS at its end, dU
 
-__device__ __forceinline__ f32x16 mfma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-__device__ __forceinline__ f32x4 widen4(u32x2 w) {
-    return f32x4{__uint_as_float(w[0] << 16), __uint_as_float(w[0] & 0xffff0000u), __uint_as_float(w[1] << 16), __uint_as_float(w[1] & 0xffff0000u)};
-}
-__device__ __forceinline__ f32x16 zero16() {
-    f32x16 z;
-#pragma unroll
-    for (int e = 0; e < 16; ++e) z[e] = 0.f;
-    return z;
-}
-// accumulator register e of lane (ln, hf) holds row c_row(e, hf), column ln of a 32 x 32 tile
-__device__ __forceinline__ constexpr int c_row(int e, int hf) { return 8 * (e >> 2) + 4 * hf + (e & 3); }
-__device__ __forceinline__ float half_sum(float v) {  // sum over the 32 lanes of a half wave
-    v = lanes_sum<16>(v);
-    return v + __shfl_xor(v, 16, 64);
-}
 // four consecutive bf16 of row `r` of a [tokens, ld] operand, zeros beyond the sequence
 __device__ __forceinline__ u32x2 row4(const bf16_t* p, int64_t ld, int r, int cnt, int c) {
     return r < cnt ? *reinterpret_cast<const u32x2*>(p + r * ld + c) : u32x2{0u, 0u};
 }
 __device__ __forceinline__ float one(const bf16_t* p, int64_t ld, int r, int cnt, int c) { return r < cnt ? bf2f(p[r * ld + c]) : 0.f; }
 
-// log decays of a chunk, cumulated in fp64 by one wave (lane = token); beyond the sequence alpha = 1, beta = 0
 __device__ __forceinline__ double cumulated_log(const float* alpha, int64_t idx, bool in, float& a_out) {
-    float a = in ? alpha[idx] : 1.f;
-    a = a < 1e-30f ? 1e-30f : a;  // (a NaN stays one)
-    a_out = a;
-    double g = log((double)a);
-    const int lane = threadIdx.x & 63;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        const double u = __shfl_up(g, o, 64);
-        if (lane >= o) g += u;
-    }
-    return g;
+    a_out = decay_at_least(in ? alpha[idx] : 1.f);
+    return cumulated_log64(a_out);
 }
+
+// The scans' workgroups: the four value ranges of a head read the same Kw / P / Q / K, so they go to one XCD (workgroups are dealt to the eight XCDs in turn), side by side.
+__device__ __forceinline__ bool scan_place(int heads, int& head, int& v0) {
+    const int id = blockIdx.x;
+    head = (id >> 5) * 8 + (id & 7);
+    v0 = ((id >> 3) & 3) * GV;
+    return head < heads;
+}
+static_assert(GD / GV == 4, "four value ranges to a head");
 
 // ------------------------------------------------------------------------------------------- prep: everything of a chunk that needs no state
 __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
@@ -121,46 +102,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
         }
     }
     __syncthreads();
-    if (wave < 2) {  // R of the two diagonal 32 x 32 blocks: lane = column, forward substitution down the rows
-        if (lane < 32) {
-            float r[32];
-#pragma unroll
-            for (int i = 0; i < 32; ++i) {
-                float s = i == ln ? 1.f : 0.f;
-#pragma unroll
-                for (int m = 0; m < i; ++m) s = fmaf(-N[32 * wave + i][32 * wave + m], r[m], s);
-                r[i] = s;
-                T[32 * wave + i][32 * wave + ln] = s;
-            }
-        }
-    } else {
-        for (int idx = tid - 128; idx < 32 * 32; idx += 128) T[idx >> 5][32 + (idx & 31)] = 0.f;
-    }
-    __syncthreads();
-    if (wave == 0) {  // R21 = -R22 (A21 R11): the inner product parks above N's diagonal
-        f32x16 y = zero16();
-#pragma unroll
-        for (int kb = 0; kb < 32; kb += 8) {
-            const f32x4 a = *reinterpret_cast<const f32x4*>(&N[32 + ln][kb + 4 * hf]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) y = mfma2(a[j], T[kb + 4 * hf + j][ln], y);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) N[c_row(e, hf)][32 + ln] = y[e];
-    }
-    __syncthreads();
-    if (wave == 0) {
-        f32x16 y = zero16();
-#pragma unroll
-        for (int kb = 0; kb < 32; kb += 8) {
-            const f32x4 a = *reinterpret_cast<const f32x4*>(&T[32 + ln][32 + kb + 4 * hf]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) y = mfma2(a[j], N[kb + 4 * hf + j][32 + ln], y);
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) T[32 + c_row(e, hf)][ln] = -y[e];
-    }
-    __syncthreads();
+    invert_unit_lower64(N, T);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 4;
@@ -198,18 +140,21 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
 }
 
 // ------------------------------------------------------------------------------------------- scan: the state chunk by chunk, 32 value rows per workgroup
-// Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave.  What a chunk reads from memory (Kw / Q / P rows in
-// fragment form, K through LDS, Uv) is requested while the chunk before it multiplies.
-__global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, float* __restrict__ saved,
+// Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave.  Bound: the chain
+// of chunks -- reads in flight, then two products behind two barriers.  Everything a chunk reads first is requested at its top, all at once: 167 us at 8 x 708 tokens x 16
+// heads; requested a chunk ahead 189 (the registers spill), in two halves 187, and 177 with the value ranges of a head on different XCDs.
+__global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, float* __restrict__ saved,
                                                            bf16_t* __restrict__ o, const float* initial_state, float* final_state, int keep, float qscale) {
     __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];
     __shared__ __attribute__((aligned(16))) float Us[GC][GV + 8];
     __shared__ __attribute__((aligned(16))) bf16_t Ks[GC][GD + 8];
     __shared__ float gg[2 * GC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
-    const int v0 = blockIdx.x * GV, h = blockIdx.y, b = blockIdx.z, hq = h / (Hv / Hqk);
+    int at, v0;
+    if (!scan_place(heads, at, v0)) return;
+    const int h = at % Hv, b = at / Hv, hq = h / (Hv / Hqk);
     const bool qside = wave >= 2;
-    const int64_t ldqk = (int64_t)Hqk * GD, head = (int64_t)b * Hv + h;
+    const int64_t ldqk = (int64_t)Hqk * GD, head = at;
     const bf16_t *qp = q + (int64_t)b * S * ldqk + hq * GD, *kp = k + (int64_t)b * S * ldqk + hq * GD;
     float* base = saved + head * NC * G_BLOCK;
 #pragma unroll
@@ -219,35 +164,31 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int S, int NC, int Hq
         if (initial_state) s = *reinterpret_cast<const f32x4*>(initial_state + (head * GD + v0 + r) * GD + c);
         *reinterpret_cast<f32x4*>(&Ss[r][c]) = s;
     }
-    f32x4 fr[16];  // waves 0, 1: a Kw row; waves 2, 3: a Q row (raw, two groups of four to a register quad) and a P row
-    float gr = 0.f;
-    auto request = [&](int n) {
-        const float* blk = base + (int64_t)n * G_BLOCK;
-        const int t0 = n * GC, cnt = min(GC, S - t0), row = 32 * rh + ln;
+    for (int n = 0; n < NC; ++n) {
+        float* blk = base + (int64_t)n * G_BLOCK;
+        const int t0 = n * GC, cnt = min(GC, S - t0);
+        // a Kw row (waves 0, 1) or, in half the words, a Q row (waves 2, 3) in fragment form, all of it in flight at once
+        const int row = 32 * rh + ln;
+        const float* kw = blk + G_KW + row * GD + 4 * hf;
+        f32x4 fr[16];
         if (!qside) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(blk + G_KW + row * GD + 8 * i + 4 * hf);
+            for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(kw + 8 * i);
         } else {
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 const u32x2 w0 = row4(qp + t0 * ldqk, ldqk, row, cnt, 16 * i + 4 * hf), w1 = row4(qp + t0 * ldqk, ldqk, row, cnt, 16 * i + 8 + 4 * hf);
                 fr[i] = f32x4{__uint_as_float(w0[0]), __uint_as_float(w0[1]), __uint_as_float(w1[0]), __uint_as_float(w1[1])};
-                fr[8 + i] = *reinterpret_cast<const f32x4*>(blk + G_P + row * GC + 8 * i + 4 * hf);
             }
         }
-        if (tid < 2 * GC) gr = blk[G_GAM + tid];
-    };
-    request(0);
-    for (int n = 0; n < NC; ++n) {
-        float* blk = base + (int64_t)n * G_BLOCK;
-        const int t0 = n * GC, cnt = min(GC, S - t0);
-        __syncthreads();  // the state is whole, the last chunk's K and U are read
         u32x4 kr[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
             kr[i] = r < cnt ? *reinterpret_cast<const u32x4*>(kp + (t0 + r) * ldqk + c) : u32x4{0u, 0u, 0u, 0u};
         }
+        const float gr = tid < 2 * GC ? blk[G_GAM + tid] : 0.f;
+        __syncthreads();  // the state is whole, the last chunk's K and U are read
         if (tid < 2 * GC) gg[tid] = gr;
         if (keep) {
 #pragma unroll
@@ -278,8 +219,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int S, int NC, int Hq
         }
         f32x4 pr[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) pr[i] = fr[8 + i];
-        if (n + 1 < NC) request(n + 1);
+        for (int i = 0; i < 8; ++i) pr[i] = qside ? *reinterpret_cast<const f32x4*>(blk + G_P + (32 * rh + ln) * GC + 8 * i + 4 * hf) : f32x4{0.f, 0.f, 0.f, 0.f};
         if (!qside) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
@@ -330,7 +270,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int S, int NC, int Hq
 }
 
 // ------------------------------------------------------------------------------------------- reverse scan: the state's gradient, 32 value rows per workgroup
-__global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ saved,
+__global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ saved,
                                                             const bf16_t* __restrict__ d_o, float* __restrict__ ws, const float* d_final, float* d_initial, float qscale) {
     __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];
     __shared__ float Us[GC][GV + 4];
@@ -339,8 +279,10 @@ __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int S, int NC, int H
     __shared__ __attribute__((aligned(16))) bf16_t Os[GC][GV];  // (unpadded: two workgroups of this kernel fill a CU's LDS to the byte)
     __shared__ float gg[2 * GC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1, kh = wave >> 1;
-    const int v0 = blockIdx.x * GV, h = blockIdx.y, b = blockIdx.z, hq = h / (Hv / Hqk);
-    const int64_t ldqk = (int64_t)Hqk * GD, ldo = (int64_t)Hv * GD, head = (int64_t)b * Hv + h;
+    int at, v0;
+    if (!scan_place(heads, at, v0)) return;
+    const int h = at % Hv, b = at / Hv, hq = h / (Hv / Hqk);
+    const int64_t ldqk = (int64_t)Hqk * GD, ldo = (int64_t)Hv * GD, head = at;
     const bf16_t *qp = q + (int64_t)b * S * ldqk + hq * GD, *kp = k + (int64_t)b * S * ldqk + hq * GD, *gp = d_o + (int64_t)b * S * ldo + (int64_t)h * GD + v0;
     const float* base = saved + head * NC * G_BLOCK;
     float* wbase = ws + head * NC * W_BLOCK;
@@ -775,7 +717,7 @@ __global__ __launch_bounds__(256) void gdrc_heads_kernel(int S, int Hqk, int Hv,
 
 static int check_gdrc(const char* who, int B, int S, int Hqk, int Hv) {
     MI355_REQUIRE(B > 0 && S > 0 && Hqk > 0 && Hv > 0 && Hv % Hqk == 0, "%s: value heads (%d) must be a multiple of q/k heads (%d)", who, Hv, Hqk);
-    MI355_REQUIRE(Hv <= 65535 && B <= 65535, "%s: grid limits", who);
+    MI355_REQUIRE(Hv <= 65535 && B <= 65535 && (int64_t)B * Hv <= (1 << 28), "%s: grid limits", who);
     return 0;
 }
 
@@ -797,7 +739,7 @@ extern "C" int mi355_gdr_chunked_fwd(int B, int S, int Hqk, int Hv, const void* 
     const float qs = 1.0f / sqrtf((float)GD);
     gdrc_prep_kernel<<<dim3(NC, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, qs);
     MI355_LAUNCH_CHECK("gdr_chunked_fwd(prep)");
-    gdrc_scan_kernel<<<dim3(GD / GV, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, saved, (bf16_t*)o, initial_state, final_state, keep, qs);
+    gdrc_scan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, saved, (bf16_t*)o, initial_state, final_state, keep, qs);
     MI355_LAUNCH_CHECK("gdr_chunked_fwd");
     return 0;
 }
@@ -816,7 +758,7 @@ extern "C" int mi355_gdr_chunked_bwd(int B, int S, int Hqk, int Hv, const void* 
     float* ws = (float*)workspace;
     float* pdq = Hv > Hqk ? ws + (int64_t)B * Hv * NC * W_BLOCK : nullptr;
     float* pdk = pdq ? pdq + (int64_t)B * Hv * S * GD : nullptr;
-    gdrc_rscan_kernel<<<dim3(GD / GV, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, saved, (const bf16_t*)d_o, ws, d_final_state, d_initial_state, qs);
+    gdrc_rscan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, saved, (const bf16_t*)d_o, ws, d_final_state, d_initial_state, qs);
     MI355_LAUNCH_CHECK("gdr_chunked_bwd(scan)");
     gdrc_bwd_kernel<<<dim3(NC, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, ws, (const bf16_t*)d_o, (bf16_t*)dq,
                                                              (bf16_t*)dk, (bf16_t*)dv, lddv, dbeta, dalpha, pdq, pdk, qs);

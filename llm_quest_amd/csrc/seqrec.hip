@@ -699,6 +699,20 @@ extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq
     return 0;
 }
 
+// The per-token numbers alone (the chunked kernels of delta_chunk.hip take them): ws [tokens, H] x {decay, beta, key factor, query factor x qscale}.
+extern "C" int mi355_delta_rule_tokens(int64_t tokens, int H, int G, int dk, const void* q, const void* k, int qk_dt, int64_t ldq, int64_t ldk, const void* b, const void* a, int ba_dt,
+                                       int64_t ldb, int64_t lda, const float* A_log, const float* dt_bias, float qscale, float* ws, void* stream) {
+    MI355_REQUIRE(tokens > 0 && H > 0 && G > 0 && H % G == 0 && dk > 0 && q && k && b && a && A_log && dt_bias && ws, "delta_rule_tokens: bad arguments");
+    MI355_REQUIRE(rec_dt_ok(qk_dt) && rec_dt_ok(ba_dt) && ldq >= (int64_t)G * dk && ldk >= (int64_t)G * dk && ldb >= H && lda >= H && ((uintptr_t)ws & 15) == 0,
+                  "delta_rule_tokens: rows too short, or the result not 16-byte aligned");
+    DeltaArgs p = {};
+    p.q = q, p.k = k, p.b = b, p.a = a, p.A_log = A_log, p.dt_bias = dt_bias, p.ws = (f32x4*)ws;
+    p.ldq = ldq, p.ldk = ldk, p.ldb = ldb, p.lda = lda, p.H = H, p.G = G, p.dk = dk, p.qk_dt = qk_dt, p.ba_dt = ba_dt, p.qscale = qscale;
+    delta_prep_kernel<<<rec_rows_grid(tokens * H, 4), 256, 0, ST(stream)>>>(tokens, p);
+    MI355_LAUNCH_CHECK("delta_rule_tokens");
+    return 0;
+}
+
 // ------------------------------------------------------------------------------------------- gated feed-forward activations
 // in[r] = [gate (F) | up (F)] -> out[r, i] (F wide).  kind 0: gelu_tanh(gate) * up.  kind 1: g = min(gate, limit), u = clamp(up, -limit, limit),
 // out = g * sigmoid(1.702 g) * (u + 1).  kind 2: silu(gate) * up.

@@ -365,6 +365,51 @@ def test_delta_rule_carries_state_over_cuts(dk, dv, H, G):
         assert row_err(torch.cat(got[i]), want.reshape(T, -1)) < 1e-5
 
 
+@pytest.mark.parametrize("rule,H,G,decay", [("delta", 4, 2, "slow"), ("delta", 2, 2, "wild"), ("delta", 6, 2, "none"), ("retention", 3, 3, "slow"), ("retention", 2, 2, "none")])
+def test_recurrences_in_chunks_equal_those_by_token(rule, H, G, decay):
+    """Steps with a chunk or more of new tokens take the chunked kernels: the same outputs and states as token by token and as the oracle in fp64, over lengths around a chunk,
+    sequences without tokens, slots out of order, states carried in, and rows of any even pitch.  Bound: fp32 sums of up to 128 + 64 terms each chunk, 1e-5 as above."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(7 * H + G)
+    D, lens, slots = 128, [1, 63, 0, 64, 65, 130, 200], [4, 0, 7, 2, 6, 1, 3]
+    T, d = sum(lens), _Slots(lens, slots)
+    wide = torch.randn(T, (2 * G + H) * D + 8, generator=g)
+    wide[:, G * D : 2 * G * D] *= 3.0
+    x = wide.to(DEV)
+    q, k, v = x[:, : G * D], x[:, G * D : 2 * G * D], x[:, 2 * G * D : (2 * G + H) * D]
+    start = torch.randn(8, H, D, D, generator=g)
+    states = [start.clone().to(DEV) for _ in range(2)]
+    if rule == "delta":
+        b, a = torch.randn(T, H, generator=g) * 2, torch.randn(T, H, generator=g) * 2
+        A_log, dt_bias = {"slow": torch.full((H,), -6.0), "wild": torch.full((H,), 3.0), "none": torch.full((H,), -80.0)}[decay], torch.randn(H, generator=g) * 0.5
+        run = lambda st, n: S.delta_rule(q, k, v, b.to(DEV), a.to(DEV), A_log.to(DEV), dt_bias.to(DEV), D ** -0.5, d.seq_off, d.slots, st, H, G, D, D, max_new=n)
+    else:
+        dec = {"slow": [0.999, 0.97, 0.5], "none": [1.0, 1e-20]}[decay]
+        run = lambda st, n: S.gla(q, k, v, None, None, 1.0, 1.0, d.seq_off, d.slots, st, H, D, D, head_decay=torch.tensor(dec, device=DEV), kscale=D ** -0.5, max_new=n)
+    assert S._delta_chunked(q, k, v, D, D, 200) and not S._delta_chunked(q, k, v, D, D, 63) and not S._delta_chunked(x[:, 1 : G * D + 1], k, v, D, D, 200)
+    by_token, chunked = run(states[0], 0), run(states[1], max(lens))
+    assert row_err(chunked, by_token.cpu()) < 1e-5
+    for s in range(8):
+        assert row_err(states[1][s].reshape(H * D, D), states[0][s].reshape(H * D, D).cpu()) < 1e-5, f"state in slot {s}"
+    assert torch.equal(states[1][5].cpu(), start[5]) and torch.equal(states[1][7].cpu(), start[7])  # no sequence's, and one without new tokens
+    w, at = wide.double(), lens[0]  # the second sequence against fp64, from its carried state
+    for i in (1, 5):
+        at, n = d.off[i], lens[i]
+        qi, ki, vi = (w[at : at + n, lo * D : hi * D].reshape(n, -1, D).repeat_interleave(H // (hi - lo), 1) for lo, hi in ((0, G), (G, 2 * G), (2 * G, 2 * G + H)))
+        st, want = start[slots[i]].double(), torch.empty(n, H, D, dtype=F64)
+        for t in range(n):
+            if rule == "delta":
+                qt, kt = (z[t] / torch.sqrt((z[t] ** 2).sum(-1, keepdim=True) + 1e-6) for z in (qi, ki))
+                st = st * torch.exp(-torch.exp(A_log.double()) * torch.nn.functional.softplus(a[at + t].double() + dt_bias.double()))[:, None, None]
+                st = st + kt[:, :, None] * (torch.sigmoid(b[at + t].double())[:, None] * (vi[t] - (kt[:, :, None] * st).sum(1)))[:, None, :]
+                qt = qt * D ** -0.5
+            else:
+                st, qt = st * torch.tensor(dec, dtype=F64)[:, None, None] + (ki[t] * D ** -0.5)[:, :, None] * vi[t][:, None, :], qi[t]
+            want[t] = (qt[:, :, None] * st).sum(1)
+        assert row_err(chunked[at : at + n], want.reshape(n, -1)) < 1e-5
+
+
 def _attention_case(dt, H, G, d, dv, size, keep, past, n_new, hot):
     """One sequence with ``past`` cached keys and ``n_new`` queries.  Every key is small noise except the ``hot`` ones, which match the query direction
     with a large score and carry a marked value: whether a query's output shows the mark says whether it saw the key."""
