@@ -97,6 +97,7 @@ SIGNATURES = {
     "mi355_gemv_bf16": [_I, _L, _I, _P, _L, _P, _L, _P, _L, _P, _L, _P],
     "mi355_gemv_bf16_f32out": [_I, _L, _I, _P, _L, _P, _L, _P, _L, _P, _P],
     "mi355_gemv_bf16_pro": [_I, _L, _I, _P, _L, _I, _P, _F, _P, _L, _P, _L, _P, _L, _P],
+    "mi355_decode_block": [_I, _I, _I, _I, _I, _I, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _P, _P, _P, _L, _P, _P, _P, _P, _F, _F, _I, _P, _L, _P, _P],
     "mi355_attn_decode_qkv": [_I, _I, _I, _I, _P, _L, _P, _P, _P, _P, _P, _P, _P, _L, _L, _I, _P, _P, _P, _L, _P, _F, _F, _I, _P, _P],
     "mi355_decode_advance": [_I, _P, _P, _P, _P, _P, _P],
     "mi355_attn_decode": [_I, _I, _I, _I, _P, _P, _P, _L, _L, _I, _P, _P, _L, _P, _F, _I, _P, _P],
@@ -161,6 +162,7 @@ QUERIES = {
     "mi355_delta_chunked_workspace_bytes": ([_L, _I, _I], _L),
     "mi355_gdr_chunked_saved_bytes": ([_I, _I, _I], _L),
     "mi355_gdr_chunked_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
+    "mi355_decode_block_scratch_bytes": ([_I, _I, _I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_rowconst_offset": ([_I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_qnorm_partials": ([_I, _I, _I], _L),

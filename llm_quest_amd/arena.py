@@ -53,6 +53,7 @@ class ParamArena:
         self.data = data
         self.grad = torch.zeros(total, dtype=p0.dtype, device=p0.device)
         self._fresh = [True] * len(self.params)
+        self._spans = {}  # (first, last) -> (offset, rows, columns) of the fused views of THIS layout
         self._ptrs = tuple(p.data_ptr() for p in self.params)
         return True
 
@@ -64,15 +65,24 @@ class ParamArena:
 
     def fused(self, first, last):
         """2-D view [sum(rows), K] over the consecutive 2-D parameters first..last (inclusive)."""
-        i, j = self.index(first), self.index(last)
-        k = first.shape[1]
-        rows = 0
-        for t in range(i, j + 1):
-            p = self.params[t]
-            if p.dim() != 2 or p.shape[1] != k or self.offsets[t] != self.offsets[i] + rows * k:
-                raise RuntimeError("ParamArena.fused: parameters are not adjacent row blocks")
-            rows += p.shape[0]
-        return self.data[self.offsets[i] : self.offsets[i] + rows * k].view(rows, k)
+        off, rows, k = self._span(self.index(first), self.index(last))
+        return self.data[off : off + rows * k].view(rows, k)
+
+    def fused_ptr(self, first, last):
+        """Address of ``fused(first, last)``."""
+        return self.data.data_ptr() + self._span(self.index(first), self.index(last))[0] * self.data.element_size()
+
+    def _span(self, i, j):
+        span = self._spans.get((i, j))
+        if span is None:
+            k, rows = self.params[i].shape[1], 0
+            for t in range(i, j + 1):
+                p = self.params[t]
+                if p.dim() != 2 or p.shape[1] != k or self.offsets[t] != self.offsets[i] + rows * k:
+                    raise RuntimeError("ParamArena.fused: parameters are not adjacent row blocks")
+                rows += p.shape[0]
+            span = self._spans[(i, j)] = (self.offsets[i], rows, k)
+        return span
 
     # ------------------------------------------------------------------ gradients
     def grad_view(self, i):

@@ -666,6 +666,36 @@ extern "C" int mi355_attn_decode_qkv(int B, int Hq, int Hkv, int D, const void* 
     return 0;
 }
 
+// One layer of a one-token step (M = B <= 8 rows): the step's launches behind one call.  A launch costs the host 3.5 us and its Python around it as much again and more (checks,
+// an allocation, parameter look-ups): 28 layers x 5 launches of ~ 8 us were 2.4 ms of host time a token beside 1.3 ms of kernels.
+namespace {
+constexpr int64_t pad8(int64_t n) { return (n + 7) / 8 * 8; }
+}  // namespace
+
+extern "C" int64_t mi355_decode_block_scratch_bytes(int B, int d, int F, int Hq, int Hkv, int D, int splits) {
+    if (B < 1 || d < 1 || F < 1 || Hq < 1 || Hkv < 1 || D < 1 || splits < 1) return 0;
+    const int64_t rows = pad8((int64_t)(Hq + 2 * Hkv) * D) + pad8((int64_t)Hq * D) + pad8(d) + pad8(2 * (int64_t)F);
+    return B * rows * 2 + (splits > 1 ? (int64_t)B * Hq * splits * (D + 2) * 4 : 0);
+}
+
+extern "C" int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, const void* h, const void* norm1_w, const void* w_qkv, const void* q_norm_w, const void* k_norm_w,
+                                  const float* cos, const float* sin, const int32_t* pos, void* k_cache, void* v_cache, int64_t batch_stride, int64_t ld, int capacity,
+                                  const int32_t* write_pos, const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, const void* w_out, const void* norm2_w,
+                                  const void* w_gate_up, const void* w_down, float scale, float eps, int splits, void* scratch, int64_t scratch_bytes, void* out, void* stream) {
+    MI355_REQUIRE(B >= 1 && B <= 8 && d > 0 && F > 0 && Hq > 0 && Hkv > 0 && D > 0 && scratch && out && out != h && splits >= 1, "decode_block: bad arguments");
+    MI355_REQUIRE(scratch_bytes >= mi355_decode_block_scratch_bytes(B, d, F, Hq, Hkv, D, splits) && ((uintptr_t)scratch & 15) == 0, "decode_block: scratch too small (%lld bytes) or not 16-byte aligned",
+                  (long long)scratch_bytes);
+    const int64_t nq = (int64_t)(Hq + 2 * Hkv) * D, lq = pad8(nq), nc = (int64_t)Hq * D, lc = pad8(nc), l1 = pad8(d), lg = pad8(2 * (int64_t)F);
+    bf16_t *qkv = (bf16_t*)scratch, *ctx = qkv + B * lq, *h1 = ctx + B * lc, *gu = h1 + B * l1;
+    MI355_REQUIRE(lc == nc, "decode_block: Hq * D must be a multiple of 8");
+    if (int rc = mi355_gemv_bf16_pro(B, nq, d, h, d, 1, norm1_w, eps, w_qkv, d, qkv, lq, nullptr, 0, stream)) return rc;
+    if (int rc = mi355_attn_decode_qkv(B, Hq, Hkv, D, qkv, lq, q_norm_w, k_norm_w, cos, sin, pos, k_cache, v_cache, batch_stride, ld, capacity, write_pos, len_dev, key_mask, ldm, ctx,
+                                       scale, eps, splits, (float*)(gu + B * lg), stream)) return rc;
+    if (int rc = mi355_gemv_bf16(B, d, (int)nc, ctx, nc, w_out, nc, h1, l1, h, d, stream)) return rc;
+    if (int rc = mi355_gemv_bf16_pro(B, 2 * (int64_t)F, d, h1, l1, 1, norm2_w, eps, w_gate_up, d, gu, lg, nullptr, 0, stream)) return rc;
+    return mi355_gemv_bf16_pro(B, d, F, gu, lg, 2, nullptr, eps, w_down, F, out, d, h1, l1, stream);
+}
+
 extern "C" int mi355_decode_advance(int B, const int64_t* next_ids, int64_t* tok, int32_t* rope_pos, int32_t* write_pos, int32_t* length, void* stream) {
     MI355_REQUIRE(B > 0 && next_ids && tok && rope_pos && write_pos && length, "decode_advance: bad arguments");
     decode_advance_kernel<<<(B + 63) / 64, 64, 0, ST(stream)>>>(B, next_ids, tok, rope_pos, write_pos, length);

@@ -189,7 +189,7 @@ def attention_cached(att, h1, B, S, cos, sin, pos, km, kv_cache, dev_state=None,
         return lin(ctx, att.out_proj.weight, residual=residual)
     if decode and dev_state is None and D in (64, 128) and kv_cache.keys_cache[att.layer_idx].shape[0] == B and kv_cache.keys_cache[att.layer_idx].dtype == qkv.dtype:
         # the same launch where the host knows the position: 6 launches a layer instead of 8 + 2 per sequence, the same bits (28 layers: a
-        # 580-token prompt and 16 tokens 55.5 -> 41.3 ms, six 61-token prompts and 24 tokens 136 -> 57 ms; the steps are bound by their launches)
+        # 580-token prompt and 16 tokens 55.5 -> 41.3 ms, six 61-token prompts and 24 tokens 136 -> 57 ms)
         write_pos, len_dev = step_counters(kv_cache, h1.device) if counters is None else counters
         kc, vc, end = kv_cache.claim_rows(att.layer_idx, 1)
         ctx = attn_decode_qkv(qkv, att.q_norm.weight, att.k_norm.weight, cos, sin, pos, Hq, Hkv, D, kc[:, :end], vc[:, :end], write_pos, len_dev, key_mask=km, scale=att.att_scaling,
@@ -211,15 +211,67 @@ def attention_cached(att, h1, B, S, cos, sin, pos, km, kv_cache, dev_state=None,
     return lin(ctx, att.out_proj.weight, residual=residual)
 
 
+def block_scratch(blk, B, splits, device):
+    """Scratch of one layer's ``mi355_decode_block``; the layers of a step, one after the other on one stream, share it."""
+    att = blk.att
+    return torch.empty(L.load().mi355_decode_block_scratch_bytes(B, att.out_proj.weight.shape[0], blk.ffn.lin1.weight.shape[0], att.num_heads, att.num_kv_groups, att.head_dim, splits),
+                       dtype=torch.uint8, device=device)
+
+
+def _block_step(blk, att, ffn, arena, h, B, F, cos, sin, pos, km, kv_cache, dev_state, counters, scratch):
+    """``block_cached`` of a one-token step as one native call (``mi355_decode_block``): the same launches in the same order, the same bits.  None where the separate calls have
+    to take it (operands that the fused attention does not).  28 layers, both sides: a 580-token prompt and 16 tokens
+    40.8 -> 24.0 ms, six 61-token prompts and 24 tokens 56.3 -> 40.2 ms (the kernels are what is left)."""
+    Hq, Hkv, D, layer = att.num_heads, att.num_kv_groups, att.head_dim, att.layer_idx
+    if (D != 64 and D != 128) or not kv_cache.keys_cache:
+        return None
+    kc, d = kv_cache.keys_cache[layer], h.shape[1]
+    if kc.dtype != BF16 or kc.shape[0] != B or h.dtype != BF16 or not h.is_contiguous() or arena.data.dtype != BF16 or not (cos.dtype == sin.dtype == torch.float32):
+        return None
+    wo, wd = att.out_proj.weight, ffn.lin2.weight
+    if wo.shape[0] != d or wo.shape[1] != Hq * D or wd.shape[1] != F or wd.shape[0] != d:
+        return None
+    if dev_state is not None:
+        if km is not None and km.shape[1] < kc.shape[1]:
+            return None
+        write_pos, len_dev, splits = dev_state[1], dev_state[2], dev_state[3] if len(dev_state) > 3 else 1
+        vc, end = kv_cache.values_cache[layer], kc.shape[1]
+    else:
+        write_pos, len_dev = step_counters(kv_cache, h.device) if counters is None else counters
+        kc, vc, end = kv_cache.claim_rows(layer, 1)
+        splits = decode_splits(end, B, Hq)
+    L.require_gpu(h, arena.data, cos, sin, pos, kc, vc, write_pos, len_dev, km)
+    strides = kc.stride()
+    if (kc.shape != vc.shape or strides != vc.stride() or kc.shape[2] != Hkv * D or strides[2] != 1 or pos.dtype != torch.int32 or pos.numel() != B or write_pos.dtype != torch.int32
+            or len_dev.dtype != torch.int32):
+        raise ValueError("decode step: caches [B, capacity, Hkv D] of one layout, int32 positions / length on the device")
+    ldm = 0
+    if km is not None:
+        if km.dtype != torch.uint8 or km.shape[0] != B or km.shape[1] < end or km.stride(1) != 1:
+            raise ValueError("decode step: key_mask uint8 [B, >= capacity]")
+        ldm = km.stride(0)
+    if scratch is None:
+        scratch = block_scratch(blk, B, splits, h.device)
+    out = torch.empty_like(h)
+    L.call("mi355_decode_block", B, d, F, Hq, Hkv, D, h.data_ptr(), blk.norm1.weight.data_ptr(), arena.fused_ptr(att.w_queries.weight, att.w_values.weight), att.q_norm.weight.data_ptr(),
+           att.k_norm.weight.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), kc.data_ptr(), vc.data_ptr(), strides[0], strides[1], end, write_pos.data_ptr(), len_dev.data_ptr(),
+           L.ptr(km), ldm, wo.data_ptr(), blk.norm2.weight.data_ptr(), arena.fused_ptr(ffn.lin1.weight, ffn.lin_gate.weight), wd.data_ptr(), att.att_scaling, 1e-6, splits,
+           scratch.data_ptr(), scratch.numel(), out.data_ptr())
+    return out
+
+
 @torch.no_grad()
-def block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state=None, counters=None):
-    """``TransformerBlock.forward(..., kv_cache=...)`` (reference qwen3_transformer_block.py:91-112) on the bf16 residual rows h [B*S, d]."""
+def block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state=None, counters=None, scratch=None):
+    """``TransformerBlock.forward(..., kv_cache=...)`` (reference qwen3_transformer_block.py:91-112) on the bf16 residual rows h [B*S, d].  ``scratch``: ``block_scratch`` of this
+    step, if the caller has it already."""
     arena = ops.arena_for(blk)
     ffn = blk.ffn
     decode = kv_cache.start_pos > 0
     lin = _lin(decode)
     F = ffn.lin1.weight.shape[0]
     if decode and fused_rows(B * S, max(h.shape[1], F)):  # one-token step: 6 launches instead of 10 (the norms and the activation ride in the weight streams)
+        if S == 1 and (out := _block_step(blk, blk.att, ffn, arena, h, B, F, cos, sin, pos, km, kv_cache, dev_state, counters, scratch)) is not None:
+            return out
         h = attention_cached(blk.att, h, B, S, cos, sin, pos, km, kv_cache, dev_state, residual=h, pre_norm=blk.norm1.weight, counters=counters)
         gu = gemv_pro(h, arena.fused(ffn.lin1.weight, ffn.lin_gate.weight), "rmsnorm", blk.norm2.weight)
         return gemv_pro(gu, ffn.lin2.weight, "swiglu", residual=h)
@@ -265,8 +317,12 @@ def qwen3_forward_cached(model, x, kv_cache, attn_mask=None, position_ids=None, 
         if km.shape[0] != B or km.shape[1] < start + S:
             raise ValueError(f"attn_mask must cover the cached sequence: (b, >= {start + S}), got {tuple(km.shape)}")
     counters = step_counters(kv_cache, h.device) if decode and dev_state is None else None
-    for blk in model.trf_blocks:
-        h = block_cached(blk, h, B, S, model.cos, model.sin, pos, km, kv_cache, dev_state, counters)
+    cos, sin, scratch, blocks = model.cos, model.sin, None, model.trf_blocks
+    if decode and len(blocks) and B <= 8:
+        heads = blocks[0].att.num_heads
+        scratch = block_scratch(blocks[0], B, decode_splits(start + 1, B, heads) if dev_state is None else dev_state[3] if len(dev_state) > 3 else 1, h.device)
+    for blk in blocks:
+        h = block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state, counters, scratch)
     if decode and fused_rows(B * S, h.shape[1]):
         return gemv_pro(h, model.out_head.weight, "rmsnorm", model.final_norm.weight).view(B, S, -1)
     lin = _lin(decode)
