@@ -453,7 +453,7 @@ int mi355_attn_decode_qkv(int B, int Hq, int Hkv, int D, const void* qkv, int64_
                           float* workspace, void* stream);
 /* One Qwen3 layer of a one-token step behind one call (TransformerBlock.forward with a KV cache, qwen3_transformer_block.py:91-112), B <= 8 rows h bf16 [B, d]:
  * mi355_gemv_bf16_pro (norm1, q | k | v), mi355_attn_decode_qkv, mi355_gemv_bf16 (out projection + h), mi355_gemv_bf16_pro (norm2, lin1 | lin_gate),
- * mi355_gemv_bf16_pro (SwiGLU, lin2 + residual) -> out bf16 [B, d] (not h).  scratch: mi355_decode_block_scratch_bytes, 16-byte aligned. */
+ * mi355_gemv_bf16 (lin2 + residual) -> out bf16 [B, d] (not h); SwiGLU is the epilogue of the lin1 | lin_gate stream (the rounding of mi355_swiglu_fwd).  scratch: mi355_decode_block_scratch_bytes, 16-byte aligned. */
 int64_t mi355_decode_block_scratch_bytes(int B, int d, int F, int Hq, int Hkv, int D, int splits);
 int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, const void* h, const void* norm1_w, const void* w_qkv, const void* q_norm_w, const void* k_norm_w,
                        const float* cos, const float* sin, const int32_t* pos, void* k_cache, void* v_cache, int64_t batch_stride, int64_t ld, int capacity,

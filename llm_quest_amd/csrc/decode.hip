@@ -2,11 +2,11 @@
 // (llm_quest/generate.py:97-151) through Qwen3 with utils.KVCache (utils.py:409-531).  One new token per sequence makes every
 // linear layer a matrix-VECTOR product and attention one query row against the cache: both are HBM-bound byte streams (weights,
 // resp. cached K/V read exactly once per token), so the kernels here are bandwidth kernels, not MFMA kernels.
-//   gemv            y[m, :] = x[m, :] W^T (+ residual), m < 8 rows: one wave per output column, 16-byte weight loads, fp32 accumulate
+//   gemv            y[m, :] = x[m, :] W^T (+ residual), m < 8 rows: 16 weight rows at a time on the matrix pipe (one operand row: a wave per weight row), fp32 accumulate
 //   attn_decode     one query per (batch, head) over `len` cached keys: 4 waves split the keys (flash-decoding), scores with the
 //                   key on the lane, P V with the feature on the lane, combined through LDS; reference mask semantics (finite fill)
 //   gemv_pro        the same weight stream with the row operation that feeds it folded in (PRO 1: RMSNorm of x, PRO 2: SwiGLU of a gate-up row): every
-//                   workgroup rebuilds the <= 8 operand rows in LDS (a few KB) instead of a launch of its own writing them -- a decode step is launch-bound
+//                   workgroup rebuilds the <= 8 operand rows (a few KB) instead of a launch of its own writing them
 //   attn_decode_qkv the same attention started from the fused QKV stream's raw row: QK-RMSNorm + RoPE of the head's query and of its kv head's new key inside the launch,
 //                   key and value head written to the cache row at the device-side position (qknorm_rope_fwd + kv_append + attn_decode in one launch)
 //   argmax_rows     greedy sampling: first index of the row maximum (torch.argmax tie rule on ties is unspecified; first is used)
@@ -26,67 +26,15 @@ __device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8]) {
 }
 
 // ------------------------------------------------------------------------------------------- skinny GEMM (NT), M <= 8
-template <int MT>
-__global__ __launch_bounds__(256) void gemv_kernel(int M, int64_t N, int K, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ W,
-                                                   int64_t ldw, bf16_t* __restrict__ y, int64_t ldy, const bf16_t* __restrict__ res, int64_t ldr) {
-    const int lane = threadIdx.x & 63;
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= N) return;
-    const bf16_t* w = W + n * ldw;
-    float acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = 0.f;
-    for (int k0 = lane * 8; k0 < K; k0 += 512) {
-        float wf[8];
-        unpack8(*reinterpret_cast<const u32x4*>(w + k0), wf);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (m >= M) break;  // MT is the next power of two: rows M..MT-1 do not exist
-            float xf[8];
-            unpack8(*reinterpret_cast<const u32x4*>(x + m * ldx + k0), xf);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[m] = fmaf(wf[e], xf[e], acc[m]);
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        if (m >= M) break;
-        const float s = wave_sum(acc[m]);
-        if (lane == 0) y[m * ldy + n] = f2bf(res ? s + bf2f(res[m * ldr + n]) : s);
-    }
-}
-
-// The same weight stream with fp32 results (+ an fp32 bias per column): rows whose consumer works in fp32 (rotary, norms, gates of a recurrence).
-template <int MT>
-__global__ __launch_bounds__(256) void gemv_f32out_kernel(int M, int64_t N, int K, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ W,
-                                                          int64_t ldw, float* __restrict__ y, int64_t ldy, const float* __restrict__ bias) {
-    const int lane = threadIdx.x & 63;
-    const int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (n >= N) return;
-    const bf16_t* w = W + n * ldw;
-    float acc[MT];
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[m] = 0.f;
-    for (int k0 = lane * 8; k0 < K; k0 += 512) {
-        float wf[8];
-        unpack8(*reinterpret_cast<const u32x4*>(w + k0), wf);
-#pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (m >= M) break;
-            float xf[8];
-            unpack8(*reinterpret_cast<const u32x4*>(x + m * ldx + k0), xf);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[m] = fmaf(wf[e], xf[e], acc[m]);
-        }
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        if (m >= M) break;
-        const float s = wave_sum(acc[m]);
-        if (lane == 0) y[m * ldy + n] = bias ? s + bias[n] : s;
-    }
-}
-
+// A workgroup takes 16 weight rows at a time; its NW waves share k out in consecutive runs of `steps` x 32.  A weight row is an A row of v_mfma_f32_16x16x32_bf16, an operand row a
+// B column (eight of the sixteen stay idle: the pipe has nothing else to do), the waves' sums meet in LDS and are added in wave order -- which sums a result is made of
+// depends on N and K alone.  The operand rows go straight to fragments, finished there by the row operation that feeds the stream: PRO 1 RMSNorm(x[m]) * nw in the arithmetic
+// and summation order of rmsnorm_fwd_generic (norm_rope.hip; == rmsnorm_fwd_kernel<2> at width 1024), PRO 2 x holds gate-up rows [M, 2K] (up | gate, as the fused
+// lin1 | lin_gate projection writes them), swiglu_act(up, gate) as swiglu_fwd_kernel rounds it: fused == the two launches bit for bit.  GLU: W holds 2N rows (up | gate) and the
+// activation is the epilogue -- eight up rows and their gate rows make a group; every activation is worked out once, not once a workgroup.
+// Bound: a launch of a few MB is a chain of memory round trips (operand rows, row sums, weights, results), so the weights' trip runs under the operands': loads return in
+// order, hence operand loads first, weights behind them, and the next 16 rows' weights under this one's products.
+constexpr int GEMV_STEPS = 8;  // of 32 k in flight per wave: 8 x 16 bytes a lane
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
     u32x4 o;
 #pragma unroll
@@ -95,112 +43,262 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
 }
 __device__ __forceinline__ float rbf(float x) { return bf2f(f2bf(x)); }
 
-// The weight stream with its operand rows built in LDS first.  PRO 1: xs[m] = RMSNorm(x[m]) * nw, the arithmetic and summation order of rmsnorm_fwd_generic
-// (norm_rope.hip; == rmsnorm_fwd_kernel<2> at width 1024), so fused == the two launches bit for bit.  PRO 2: x holds gate-up rows [M, 2K] (up | gate, as the fused
-// lin1 | lin_gate projection writes them), xs[m] = swiglu_act(up, gate) as swiglu_fwd_kernel rounds it.  Each wave then walks output columns wave, wave + 4 * grid, ...
-template <int MT, int PRO>
-__global__ __launch_bounds__(256) void gemv_pro_kernel(int M, int64_t N, int K, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ nw, float eps,
-                                                       const bf16_t* __restrict__ W, int64_t ldw, bf16_t* __restrict__ y, int64_t ldy,
-                                                       const bf16_t* __restrict__ res, int64_t ldr) {
-    extern __shared__ __attribute__((aligned(16))) bf16_t xs[];  // [M][K]
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int nvec = K >> 3;
-    if constexpr (PRO == 1) {
-        __shared__ float rs[8];
-        {  // the row kernel's sum, in its order: one wave per row, rows wave and wave + 4 side by side
-            const int m0 = wave, m1 = wave + 4;
-            float ss0 = 0.f, ss1 = 0.f;
-            for (int i = lane; i < nvec; i += 64) {
-                float v0[8], v1[8];
-                const u32x4 r0 = m0 < M ? *reinterpret_cast<const u32x4*>(x + m0 * ldx + i * 8) : (u32x4){0u, 0u, 0u, 0u};
-                const u32x4 r1 = m1 < M ? *reinterpret_cast<const u32x4*>(x + m1 * ldx + i * 8) : (u32x4){0u, 0u, 0u, 0u};
-                unpack8(r0, v0);
-                unpack8(r1, v1);
+template <int NW, int PRO, bool F32, bool GLU>
+__global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, int steps, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ nw, float eps,
+                                                       const bf16_t* __restrict__ W, int64_t ldw, void* __restrict__ y, int64_t ldy, const void* __restrict__ res, int64_t ldr) {
+    constexpr int T = GEMV_STEPS;
+    __shared__ float rs[8];
+    __shared__ __attribute__((aligned(16))) float part[2][NW][8][16];
+    __shared__ __attribute__((aligned(16))) bf16_t act[PRO == 2 ? NW : 1][8][PRO == 2 ? 32 * T + 8 : 8];  // PRO 2: a wave's run of the activated rows
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = (lane >> 4) * 8;
+    const int nvec = K >> 3, chunks = (steps + T - 1) / T;
+    const int k_lo = wave * steps * 32, k_hi = min(K, k_lo + steps * 32);
+    constexpr int GN = GLU ? 8 : 16;  // columns of a group
+    const int64_t groups = (N + GN - 1) / GN;
+    const u32x4 z4 = {0u, 0u, 0u, 0u};
+    u32x4 xf[T], gf[PRO ? T : 1], w0[T], w1[T];
+    auto request_x = [&](int c) {
+        if constexpr (PRO == 2) {  // whole rows dealt to the lanes: an activation costs ~ 100 clocks, fragments have eight or more lanes of sixteen idle
 #pragma unroll
-                for (int e = 0; e < 8; ++e) { ss0 += v0[e] * v0[e]; ss1 += v1[e] * v1[e]; }
+            for (int t = 0; t < T / 2; ++t) {
+                const int m = 2 * t + (lane >> 5), k = k_lo + c * T * 32 + (lane & 31) * 8;
+                const bool in = m < M && k < k_hi;
+                xf[t] = in ? *reinterpret_cast<const u32x4*>(x + m * ldx + k) : z4;
+                gf[t] = in ? *reinterpret_cast<const u32x4*>(x + m * ldx + K + k) : z4;
             }
-            ss0 = wave_sum(ss0);
-            ss1 = wave_sum(ss1);
-            if (lane == 0 && m0 < M) rs[m0] = rsqrtf(ss0 / (float)K + eps);
-            if (lane == 0 && m1 < M) rs[m1] = rsqrtf(ss1 / (float)K + eps);
+        } else {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const int k = k_lo + (c * T + t) * 32 + kg;
+                const bool in = r16 < M && k < k_hi;
+                xf[t] = in ? *reinterpret_cast<const u32x4*>(x + r16 * ldx + k) : z4;
+                if constexpr (PRO == 1) gf[t] = in ? *reinterpret_cast<const u32x4*>(nw + k) : z4;
+            }
+        }
+    };
+    auto request_w = [&](u32x4 (&w)[T], int64_t g, int c) {
+        const int64_t n = g * GN + (r16 & (GN - 1));
+        const bf16_t* row = W + ((n < N ? n : N - 1) + (GLU && r16 >= 8 ? N : 0)) * ldw;
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int k = k_lo + (c * T + t) * 32 + kg;
+            w[t] = k < k_hi ? *reinterpret_cast<const u32x4*>(row + k) : z4;
+        }
+    };
+    float r = 0.f;  // PRO 1: 1 / rms of the lane's operand row
+    auto finish_x = [&]() {
+        if constexpr (PRO == 1) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                float a[8], b[8], o[8];
+                unpack8(xf[t], a);
+                unpack8(gf[t], b);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = a[e] * r * b[e];
+                xf[t] = r16 < M ? pack8(o) : z4;
+            }
+        } else if constexpr (PRO == 2) {
+#pragma unroll
+            for (int t = 0; t < T / 2; ++t) {
+                if (2 * t >= M) break;
+                float a[8], b[8], o[8];
+                unpack8(xf[t], a);
+                unpack8(gf[t], b);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = swiglu_act(a[e], b[e]);
+                *reinterpret_cast<u32x4*>(&act[wave][2 * t + (lane >> 5)][(lane & 31) * 8]) = pack8(o);
+            }
+            __builtin_amdgcn_wave_barrier();  // written and read by this wave alone, in order
+#pragma unroll
+            for (int t = 0; t < T; ++t) xf[t] = r16 < M ? *reinterpret_cast<const u32x4*>(&act[wave][r16 & 7][t * 32 + kg]) : z4;
+            __builtin_amdgcn_wave_barrier();
+        }
+    };
+    int64_t g = blockIdx.x;
+    if constexpr (PRO == 1) {  // row sums: rows wave, wave + NW
+        u32x4 v0[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v0[i] = wave < M && lane + 64 * i < nvec ? *reinterpret_cast<const u32x4*>(x + wave * ldx + (lane + 64 * i) * 8) : z4;
+        request_x(0);
+        request_w(w0, g, 0);
+        for (int m = wave; m < M; m += NW) {
+            float ss = 0.f, v[8];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                if (lane + 64 * i < nvec) {
+                    unpack8(m == wave ? v0[i] : *reinterpret_cast<const u32x4*>(x + m * ldx + (lane + 64 * i) * 8), v);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+                }
+            for (int i = lane + 256; i < nvec; i += 64) {
+                unpack8(*reinterpret_cast<const u32x4*>(x + m * ldx + i * 8), v);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+            }
+            ss = wave_sum(ss);
+            if (lane == 0) rs[m] = rsqrtf(ss / (float)K + eps);
         }
         __syncthreads();
-        for (int idx0 = threadIdx.x; idx0 < M * nvec; idx0 += 1024) {  // every thread a vector of some row; four requested together (eight rows: a chain of four round trips otherwise)
-            u32x4 xv[4], nv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = idx0 + u * 256;
-                if (idx < M * nvec) {
-                    const int m = idx / nvec, i = idx - m * nvec;
-                    xv[u] = *reinterpret_cast<const u32x4*>(x + m * ldx + i * 8);
-                    nv[u] = *reinterpret_cast<const u32x4*>(nw + i * 8);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = idx0 + u * 256;
-                if (idx < M * nvec) {
-                    const int m = idx / nvec, i = idx - m * nvec;
-                    const float r = rs[m];
-                    float v[8], wv[8], o[8];
-                    unpack8(xv[u], v);
-                    unpack8(nv[u], wv);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) o[e] = v[e] * r * wv[e];
-                    *reinterpret_cast<u32x4*>(xs + m * K + i * 8) = pack8(o);
-                }
-            }
-        }
+        r = rs[r16 & 7];
     } else {
-        for (int idx0 = threadIdx.x; idx0 < M * nvec; idx0 += 1024) {
-            u32x4 uv[4], gv[4];
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = idx0 + u * 256;
-                if (idx < M * nvec) {
-                    const int m = idx / nvec, i = idx - m * nvec;
-                    uv[u] = *reinterpret_cast<const u32x4*>(x + m * ldx + i * 8);
-                    gv[u] = *reinterpret_cast<const u32x4*>(x + m * ldx + K + i * 8);
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < 4; ++u) {
-                const int idx = idx0 + u * 256;
-                if (idx < M * nvec) {
-                    const int m = idx / nvec, i = idx - m * nvec;
-                    float uf[8], g[8], o[8];
-                    unpack8(uv[u], uf);
-                    unpack8(gv[u], g);
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) o[e] = swiglu_act(uf[e], g[e]);
-                    *reinterpret_cast<u32x4*>(xs + m * K + i * 8) = pack8(o);
-                }
-            }
-        }
+        request_x(0);
+        request_w(w0, g, 0);
     }
-    __syncthreads();
-    for (int64_t n = (int64_t)blockIdx.x * 4 + wave; n < N; n += (int64_t)gridDim.x * 4) {
-        const bf16_t* w = W + n * ldw;
-        float acc[MT];
+    finish_x();
+    f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    int c = 0, flip = 0;
+    // one chunk of one group: the next one's weights are requested first
+    auto work = [&](u32x4 (&now)[T], u32x4 (&next)[T]) {
+        int64_t gn = g;
+        int cn = c + 1;
+        const int m = threadIdx.x >> 4;
+        const int64_t n = g * GN + r16;
+        float add = 0.f;
+        if (cn == chunks) {
+            cn = 0, gn += gridDim.x;
+            if (res && m < M && n < N && r16 < GN) add = F32 ? ((const float*)res)[n] : bf2f(((const bf16_t*)res)[m * ldr + n]);
+        }
+        if (gn < groups) request_w(next, gn, cn);
 #pragma unroll
-        for (int m = 0; m < MT; ++m) acc[m] = 0.f;
-        for (int k0 = lane * 8; k0 < K; k0 += 512) {
-            float wf[8];
-            unpack8(*reinterpret_cast<const u32x4*>(w + k0), wf);
+        for (int t = 0; t < T; ++t)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, now[t]), __builtin_bit_cast(bf16x8, xf[t]), acc, 0, 0, 0);
+        if (cn == 0) {
+            if (r16 < 8) *reinterpret_cast<f32x4*>(&part[flip][wave][r16][lane >> 4 << 2]) = acc;
+            __syncthreads();
+            if (m < M && n < N && r16 < GN) {
+                float s = part[flip][0][m][r16];
 #pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                if (m >= M) break;
-                float xf[8];
-                unpack8(*reinterpret_cast<const u32x4*>(xs + m * K + k0), xf);
+                for (int i = 1; i < NW; ++i) s += part[flip][i][m][r16];
+                if constexpr (GLU) {
+                    float gate = part[flip][0][m][8 + (r16 & 7)];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) acc[m] = fmaf(wf[e], xf[e], acc[m]);
+                    for (int i = 1; i < NW; ++i) gate += part[flip][i][m][8 + (r16 & 7)];
+                    ((bf16_t*)y)[m * ldy + n] = f2bf(swiglu_act(rbf(s), rbf(gate)));
+                } else if constexpr (F32) ((float*)y)[m * ldy + n] = res ? s + add : s;
+                else ((bf16_t*)y)[m * ldy + n] = f2bf(res ? s + add : s);
+            }
+            flip ^= 1;  // (the next group's sums go beside these: its barrier is behind every read of them)
+            acc = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        if (chunks > 1 && gn < groups) {
+            request_x(cn);
+            finish_x();
+        }
+        g = gn, c = cn;
+    };
+    while (g < groups) {
+        work(w0, w1);
+        if (g >= groups) break;
+        work(w1, w0);
+    }
+}
+
+// One operand row: a matrix pipe with one column at work gains nothing, and a row fits the registers of every wave in the layout of the weights' strips (512 k, 8 per lane), so
+// there is neither an image nor a barrier between the loads and the products (PRO 2 alone shares its activations through LDS: each costs ~ 100 clocks).  One wave = one
+// column (GLU: an up column and its gate column), the workgroups walk the columns.  Arithmetic of the prologues and of GLU as above; a sum is a lane's strips in order, then wave_sum.
+template <int T, int PRO, bool F32, bool GLU>
+__global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const bf16_t* __restrict__ x, const bf16_t* __restrict__ nw, float eps, const bf16_t* __restrict__ W, int64_t ldw,
+                                                       void* __restrict__ y, const void* __restrict__ res) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t act[];  // PRO 2: [K]
+    constexpr int C = GLU ? 2 : 1;  // columns of a wave; T strips in registers (the smallest of 2, 4, 8 that holds the row; longer rows go through eight at a time)
+    const int lane = threadIdx.x & 63, its = (K + 511) >> 9;
+    const u32x4 z4 = {0u, 0u, 0u, 0u};
+    u32x4 xr[T], nr[PRO == 1 ? T : 1], w[C][T];
+    auto request_x = [&](int base) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            const int k = (base + t) * 512 + lane * 8;
+            xr[t] = k < K ? *reinterpret_cast<const u32x4*>((PRO == 2 ? act : x) + k) : z4;
+            if constexpr (PRO == 1) nr[t] = k < K ? *reinterpret_cast<const u32x4*>(nw + k) : z4;
+        }
+    };
+    auto request_w = [&](int64_t n, int base) {
+#pragma unroll
+        for (int c = 0; c < C; ++c)
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                const int k = (base + t) * 512 + lane * 8;
+                w[c][t] = k < K ? *reinterpret_cast<const u32x4*>(W + (n + c * N) * ldw + k) : z4;
+            }
+    };
+    float r = 0.f;
+    auto finish_x = [&]() {
+        if constexpr (PRO == 1) {
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                float a[8], b[8], o[8];
+                unpack8(xr[t], a);
+                unpack8(nr[t], b);
+#pragma unroll
+                for (int e = 0; e < 8; ++e) o[e] = a[e] * r * b[e];
+                xr[t] = pack8(o);
+            }
+        }
+    };
+    const int64_t stride = (int64_t)gridDim.x * 4;
+    int64_t n = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if constexpr (PRO == 2) {
+        for (int k = threadIdx.x * 8; k < K; k += 2048) {
+            float u[8], g[8], o[8];
+            unpack8(*reinterpret_cast<const u32x4*>(x + k), u);
+            unpack8(*reinterpret_cast<const u32x4*>(x + K + k), g);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) o[e] = swiglu_act(u[e], g[e]);
+            *reinterpret_cast<u32x4*>(act + k) = pack8(o);
+        }
+        __syncthreads();
+    }
+    if (n >= N) return;  // (no barrier behind this)
+    request_x(0);
+    request_w(n, 0);
+    if constexpr (PRO == 1) {
+        float ss = 0.f, v[8];
+#pragma unroll
+        for (int t = 0; t < T; ++t) {
+            unpack8(xr[t], v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+        }
+        for (int k = T * 512 + lane * 8; k < K; k += 512) {
+            unpack8(*reinterpret_cast<const u32x4*>(x + k), v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
+        }
+        r = rsqrtf(wave_sum(ss) / (float)K + eps);
+    }
+    finish_x();
+    for (bool first = true; n < N; n += stride) {
+        float acc[C];
+#pragma unroll
+        for (int c = 0; c < C; ++c) acc[c] = 0.f;
+        float add = 0.f;
+        if (res) add = F32 ? ((const float*)res)[n] : bf2f(((const bf16_t*)res)[n]);
+        for (int base = 0; base < its; base += T) {
+            if (!first) {
+                if (its > T) request_x(base);
+                request_w(n, base);
+                if (its > T) finish_x();
+            }
+            first = false;
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                if (base + t >= its) break;
+                float xf[8], wf[8];
+                unpack8(xr[t], xf);
+#pragma unroll
+                for (int c = 0; c < C; ++c) {
+                    unpack8(w[c][t], wf);
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) acc[c] = fmaf(wf[e], xf[e], acc[c]);
+                }
             }
         }
 #pragma unroll
-        for (int m = 0; m < MT; ++m) {
-            if (m >= M) break;
-            const float s = wave_sum(acc[m]);
-            if (lane == 0) y[m * ldy + n] = f2bf(res ? s + bf2f(res[m * ldr + n]) : s);
+        for (int c = 0; c < C; ++c) acc[c] = wave_sum(acc[c]);
+        if (lane == 0) {
+            if constexpr (GLU) ((bf16_t*)y)[n] = f2bf(swiglu_act(rbf(acc[0]), rbf(acc[C - 1])));
+            else if constexpr (F32) ((float*)y)[n] = res ? acc[0] + add : acc[0];
+            else ((bf16_t*)y)[n] = f2bf(res ? acc[0] + add : acc[0]);
         }
     }
 }
@@ -552,15 +650,36 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(const float* __restric
 
 #define ST(s) ((hipStream_t)(s))
 
+// One row: gemv_one_kernel.  Two to eight: eight waves and at most a workgroup for each CU; four waves and two workgroups a CU where they walk many groups (a table of 151 936
+// rows: 56 us so, 64 with eight waves and 59 with four workgroups; 6144 x 1024: 7.9 us with eight waves, 8.7 with four; sixteen waves spill under a prologue).
+// us of one launch, weights from memory, before (a column per wave on the vector pipe for up to eight rows) -> now:   N x K      1 row          6 rows
+//     RMSNorm + 4096 x 1024    4.9 -> 4.5     9.0 -> 6.2          |   1024 x 3072 (from activated rows)    4.6 -> 3.5     7.9 -> 5.8
+//     RMSNorm + 6144 x 1024    6.6 -> 5.7    11.3 -> 7.9          |   1024 x 2048                          3.8 -> 2.9     6.3 -> 4.5
+//     RMSNorm + 151936 x 1024   52 -> 52      152 -> 56           |   3072 x 4096                          8.5 -> 7.1    14.0 -> 9.0
+template <int PRO, bool F32, bool GLU = false>
+static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, const void* nw, float eps, const void* W, int64_t ldw, void* y, int64_t ldy, const void* res, int64_t ldr, void* stream) {
+    if (M == 1) {
+        const int64_t blocks = (N + 3) / 4;
+#define GEMV(T) gemv_one_kernel<T, PRO, F32, GLU><<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO == 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res)
+        if (K <= 1024) GEMV(2); else if (K <= 2048) GEMV(4); else GEMV(8);
+#undef GEMV
+        return;
+    }
+    const int all = (K + 31) / 32;
+    const int64_t groups = ((GLU ? 2 * N : N) + 15) / 16;
+    const int waves = groups >= 1024 ? 4 : 8, most = 2048 / waves;
+    const int grid = (int)(groups < most ? groups : most), steps = (all + waves - 1) / waves;
+#define GEMV(NW) gemv_kernel<NW, PRO, F32, GLU><<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, ldy, res, ldr)
+    if (waves == 4) GEMV(4); else GEMV(8);
+#undef GEMV
+}
+
 extern "C" int mi355_gemv_bf16(int M, int64_t N, int K, const void* x, int64_t ldx, const void* W, int64_t ldw, void* y, int64_t ldy,
                                const void* residual, int64_t ldr, void* stream) {
     MI355_REQUIRE(M >= 1 && M <= 8, "gemv_bf16: 1..8 rows (got %d); larger batches go through mi355_gemm_bf16", M);
     MI355_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= K && ldw >= K && ldy >= N, "gemv_bf16: K and the leading dimensions of x / W must be multiples of 8");
     MI355_REQUIRE(x && W && y && (!residual || ldr >= N), "gemv_bf16: null pointer or residual pitch too small");
-    const int grid = (int)((N + 3) / 4);
-#define LAUNCH(MT) gemv_kernel<MT><<<grid, 256, 0, ST(stream)>>>(M, N, K, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw, (bf16_t*)y, ldy, (const bf16_t*)residual, ldr)
-    if (M == 1) LAUNCH(1); else if (M == 2) LAUNCH(2); else if (M <= 4) LAUNCH(4); else LAUNCH(8);
-#undef LAUNCH
+    gemv_launch<0, false>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);
     MI355_LAUNCH_CHECK("gemv_bf16");
     return 0;
 }
@@ -570,10 +689,7 @@ extern "C" int mi355_gemv_bf16_f32out(int M, int64_t N, int K, const void* x, in
     MI355_REQUIRE(M >= 1 && M <= 8, "gemv_bf16_f32out: 1..8 rows (got %d)", M);
     MI355_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= K && ldw >= K && ldy >= N, "gemv_bf16_f32out: K and the leading dimensions of x / W must be multiples of 8");
     MI355_REQUIRE(x && W && y, "gemv_bf16_f32out: null pointer");
-    const int grid = (int)((N + 3) / 4);
-#define LAUNCH(MT) gemv_f32out_kernel<MT><<<grid, 256, 0, ST(stream)>>>(M, N, K, (const bf16_t*)x, ldx, (const bf16_t*)W, ldw, y, ldy, bias)
-    if (M == 1) LAUNCH(1); else if (M == 2) LAUNCH(2); else if (M <= 4) LAUNCH(4); else LAUNCH(8);
-#undef LAUNCH
+    gemv_launch<0, true>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, bias, 0, stream);
     MI355_LAUNCH_CHECK("gemv_bf16_f32out");
     return 0;
 }
@@ -584,15 +700,11 @@ extern "C" int mi355_gemv_bf16_pro(int M, int64_t N, int K, const void* x, int64
     MI355_REQUIRE(prologue == 1 || prologue == 2, "gemv_bf16_pro: prologue 1 (RMSNorm of x) or 2 (SwiGLU of gate-up rows), got %d", prologue);
     MI355_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= (prologue == 2 ? 2 * K : K) && ldw >= K && ldy >= N,
                   "gemv_bf16_pro: K and the leading dimensions must be multiples of 8 (x rows hold 2K elements under prologue 2)");
-    // (the RMSNorm prologue keeps eight row sums in 32 bytes of static LDS beside the dynamic image: together they must stay within the 64 KiB a launch gets by default)
+    // (32 bytes beside the operand rows have always been refused with them: callers ask ops_decode.fused_rows, which knows that line)
     MI355_REQUIRE((int64_t)M * K * 2 + 32 <= 65536, "gemv_bf16_pro: the operand rows (%d x %d bf16) plus 32 bytes of row sums exceed the 64 KiB LDS image", M, K);
     MI355_REQUIRE(x && W && y && (!residual || ldr >= N) && (prologue != 1 || norm_w), "gemv_bf16_pro: null pointer or residual pitch too small");
-    const int grid = (int)((N + 3) / 4 < 2048 ? (N + 3) / 4 : 2048);
-    const size_t lds = (size_t)M * K * 2;
-#define LAUNCH(MT, PRO) gemv_pro_kernel<MT, PRO><<<grid, 256, lds, ST(stream)>>>(M, N, K, (const bf16_t*)x, ldx, (const bf16_t*)norm_w, eps, (const bf16_t*)W, ldw, (bf16_t*)y, ldy, (const bf16_t*)residual, ldr)
-    if (prologue == 1) { if (M == 1) LAUNCH(1, 1); else if (M == 2) LAUNCH(2, 1); else if (M <= 4) LAUNCH(4, 1); else LAUNCH(8, 1); }
-    else { if (M == 1) LAUNCH(1, 2); else if (M == 2) LAUNCH(2, 2); else if (M <= 4) LAUNCH(4, 2); else LAUNCH(8, 2); }
-#undef LAUNCH
+    if (prologue == 1) gemv_launch<1, false>(M, N, K, x, ldx, norm_w, eps, W, ldw, y, ldy, residual, ldr, stream);
+    else gemv_launch<2, false>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);
     MI355_LAUNCH_CHECK("gemv_bf16_pro");
     return 0;
 }
@@ -674,7 +786,7 @@ constexpr int64_t pad8(int64_t n) { return (n + 7) / 8 * 8; }
 
 extern "C" int64_t mi355_decode_block_scratch_bytes(int B, int d, int F, int Hq, int Hkv, int D, int splits) {
     if (B < 1 || d < 1 || F < 1 || Hq < 1 || Hkv < 1 || D < 1 || splits < 1) return 0;
-    const int64_t rows = pad8((int64_t)(Hq + 2 * Hkv) * D) + pad8((int64_t)Hq * D) + pad8(d) + pad8(2 * (int64_t)F);
+    const int64_t rows = pad8((int64_t)(Hq + 2 * Hkv) * D) + pad8((int64_t)Hq * D) + pad8(d) + pad8(F);
     return B * rows * 2 + (splits > 1 ? (int64_t)B * Hq * splits * (D + 2) * 4 : 0);
 }
 
@@ -685,15 +797,16 @@ extern "C" int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, c
     MI355_REQUIRE(B >= 1 && B <= 8 && d > 0 && F > 0 && Hq > 0 && Hkv > 0 && D > 0 && scratch && out && out != h && splits >= 1, "decode_block: bad arguments");
     MI355_REQUIRE(scratch_bytes >= mi355_decode_block_scratch_bytes(B, d, F, Hq, Hkv, D, splits) && ((uintptr_t)scratch & 15) == 0, "decode_block: scratch too small (%lld bytes) or not 16-byte aligned",
                   (long long)scratch_bytes);
-    const int64_t nq = (int64_t)(Hq + 2 * Hkv) * D, lq = pad8(nq), nc = (int64_t)Hq * D, lc = pad8(nc), l1 = pad8(d), lg = pad8(2 * (int64_t)F);
-    bf16_t *qkv = (bf16_t*)scratch, *ctx = qkv + B * lq, *h1 = ctx + B * lc, *gu = h1 + B * l1;
-    MI355_REQUIRE(lc == nc, "decode_block: Hq * D must be a multiple of 8");
+    const int64_t nq = (int64_t)(Hq + 2 * Hkv) * D, lq = pad8(nq), nc = (int64_t)Hq * D, lc = pad8(nc), l1 = pad8(d), la = pad8(F);
+    bf16_t *qkv = (bf16_t*)scratch, *ctx = qkv + B * lq, *h1 = ctx + B * lc, *act = h1 + B * l1;
+    MI355_REQUIRE(lc == nc && norm2_w && w_gate_up && w_down, "decode_block: Hq * D must be a multiple of 8; null pointer");
     if (int rc = mi355_gemv_bf16_pro(B, nq, d, h, d, 1, norm1_w, eps, w_qkv, d, qkv, lq, nullptr, 0, stream)) return rc;
     if (int rc = mi355_attn_decode_qkv(B, Hq, Hkv, D, qkv, lq, q_norm_w, k_norm_w, cos, sin, pos, k_cache, v_cache, batch_stride, ld, capacity, write_pos, len_dev, key_mask, ldm, ctx,
-                                       scale, eps, splits, (float*)(gu + B * lg), stream)) return rc;
+                                       scale, eps, splits, (float*)(act + B * la), stream)) return rc;
     if (int rc = mi355_gemv_bf16(B, d, (int)nc, ctx, nc, w_out, nc, h1, l1, h, d, stream)) return rc;
-    if (int rc = mi355_gemv_bf16_pro(B, 2 * (int64_t)F, d, h1, l1, 1, norm2_w, eps, w_gate_up, d, gu, lg, nullptr, 0, stream)) return rc;
-    return mi355_gemv_bf16_pro(B, d, F, gu, lg, 2, nullptr, eps, w_down, F, out, d, h1, l1, stream);
+    gemv_launch<1, false, true>(B, F, d, h1, l1, norm2_w, eps, w_gate_up, d, act, la, nullptr, 0, stream);
+    MI355_LAUNCH_CHECK("decode_block(gate, up)");
+    return mi355_gemv_bf16(B, d, F, act, la, w_down, F, out, d, h1, l1, stream);
 }
 
 extern "C" int mi355_decode_advance(int B, const int64_t* next_ids, int64_t* tok, int32_t* rope_pos, int32_t* write_pos, int32_t* length, void* stream) {
