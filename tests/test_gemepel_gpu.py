@@ -503,3 +503,46 @@ def test_fp32_grouped_product_on_split_operands(T, top, epi):
         y = torch.relu(y) ** 2
     want = y * sc.double()[:, None]
     assert float((out.double() - want).norm() / want.norm()) < 2e-6  # fp32 sums of 200 products and the epilogue's few roundings
+
+
+@pytest.mark.parametrize("rows,n,K,epi,out", [([1, 0, 31, 257, 600, 256, 65], 2560, 64, 0, F32), ([300, 5, 513], 5700, 128, 1, BF16), ([0, 700, 33, 129], 4096, 192, 4, BF16),
+                                              ([2] * 70 + [90], 250, 64, 2, F32), (None, 2050, 64, 0, BF16)])
+def test_bf16_product_on_wide_tiles(rows, n, K, epi, out):
+    """256 x 256 tiles: groups of uneven rows (none, one, around 32 / 64 / 128 / 256, more groups than lanes), gathered and scattered rows, columns that are no whole words, gated
+    blocks; and a plain batch.  fp32 sums of K exact products: results within a few fp32 roundings, resp. one bf16 rounding, of fp64."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(n + K)
+    batch, per = (len(rows), None) if rows else (3, 4100)
+    R = sum(rows) if rows else per
+    gated = epi in (2, 4)
+    n_out, n_rows = (n, 64 * -(-n // 32)) if gated else (n, n)
+    x = torch.randn(R if rows else batch * R, K + 8, generator=g).to(BF16).cuda()[:, :K]
+    w = (torch.randn(batch, n_rows, K, generator=g) / K ** 0.5).to(BF16).cuda()
+    total = x.shape[0]
+    c = torch.full((total, n_out + 2), 7.0, dtype=out, device="cuda")
+    grp, perm, sc = None, None, None
+    if rows:
+        offs = [0]
+        for r in rows:
+            offs.append(offs[-1] + r)
+        grp, perm = torch.tensor(offs, dtype=torch.int32, device="cuda"), torch.randperm(R, generator=g).to(torch.int32).cuda()
+        sc = torch.rand(R, generator=g).cuda()
+    S.bgemm(x, w, c, R, n_rows, K, batch=batch, a_bs=0 if rows else R * x.stride(0), sbn=K, b_bs=n_rows * K, c_bs=0 if rows else R * c.stride(0), grp_offs=grp, a_rows=perm, c_rows=perm,
+            row_scale=sc, epi=epi, limit=2.5, n_out=n_out if gated else 0)
+    bad = 0.0
+    for b in range(batch):
+        r = perm[offs[b] : offs[b + 1]].long() if rows else torch.arange(b * R, (b + 1) * R, device="cuda")
+        if not r.numel():
+            continue
+        y = x[r].double() @ w[b].double().T
+        if gated:
+            v = y.view(len(r), -1, 2, 32)
+            gt, up = (v[:, :, i].flatten(1)[:, :n] for i in (0, 1))
+            y = gt.clamp(max=2.5) * torch.sigmoid(1.702 * gt.clamp(max=2.5)) * (up.clamp(-2.5, 2.5) + 1) if epi == 2 else torch.nn.functional.silu(gt) * up
+        elif epi == 1:
+            y = torch.relu(y) ** 2
+        y = y * sc[r].double()[:, None] if rows else y
+        bad = max(bad, float((c[r, :n_out].double() - y).norm() / y.norm()))
+    assert bad < (2e-6 if out == F32 else 2.5e-3)
+    assert bool((c[:, n_out:] == 7.0).all())  # nothing beside the columns
