@@ -42,6 +42,13 @@ from llm_quest_amd import kernels_seq as S
 BF16, F32, I32 = torch.bfloat16, torch.float32, torch.int32
 
 
+def host_staging(n, dtype, device):
+    """Host memory for a copy to ``device`` that nobody waits for: pinned where the device is a GPU (the caching allocator keeps it until the copy is done).  A step's descriptors
+    in pageable memory made the host wait for all that was queued before it could prepare the step: six 900-token prompts and four steps 6.6 -> 4.4 ms, a fp32
+    replay of three 150-token prompts and four steps 6.0 -> 5.1."""
+    return torch.empty(n, dtype=dtype, pin_memory=torch.device(device).type == "cuda")
+
+
 class SeqStep:
     """One step of a ragged batch: ``entries`` = [(slot, new tokens)], the cache gives every sequence's length and last token.  Holds the device-side
     descriptors the kernels read.  ``fresh``: every sequence starts at its first token (prompts; attention may rebuild keys and values from this step's rows)."""
@@ -68,7 +75,8 @@ class SeqStep:
         row0 = [s * cap for s in slots]
         # rows of the descriptor block: tokens | previous token | position | cache row | per-sequence arrays | 0 .. T-1 | sequence of a row; one
         # host-to-device copy for all
-        buf = np.empty(6 * T + 5 * n + 1, dtype=np.int32)
+        host = host_staging(6 * T + 5 * n + 1, I32, device)
+        buf = host.numpy()
         tok, prev, pos, dst = buf[0:T], buf[T : 2 * T], buf[2 * T : 3 * T], buf[3 * T : 4 * T]
         for i, (slot, new) in enumerate(entries):
             a, b = seq_off[i], seq_off[i + 1]
@@ -83,7 +91,7 @@ class SeqStep:
             at += len(arr)
         buf[at : at + T] = np.arange(T, dtype=np.int32)
         buf[at + T : at + 2 * T] = np.repeat(np.arange(n, dtype=np.int32), n_new)
-        buf = torch.from_numpy(buf).to(device, non_blocking=False)
+        buf = host.to(device, non_blocking=True)
         cuts = [T, T, T, T, n + 1, n, n, n, n, T, T]
         parts, at = [], 0
         for c in cuts:

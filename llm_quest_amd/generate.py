@@ -189,7 +189,7 @@ class RaggedBatch:
     def step(self, entries, want=None, return_layers=False):
         """entries: [(seq_id, [token, ...])] in batch order.  want: per entry the positions among ITS new tokens whose logits are asked for (default:
         the last one).  Returns fp32 [rows asked for, vocab] in the order of the entries and of ``want`` (None if nothing is asked for)."""
-        from .common.mixers import SeqStep
+        from .common.mixers import SeqStep, host_staging
 
         if not entries:
             return None
@@ -212,7 +212,9 @@ class RaggedBatch:
                     raise ValueError("a wanted position lies outside the entry's tokens")
                 rows.append(st.host_seq_off[i] + p)
         # the whole stack runs even when no logits are asked for: the step still has to leave its rows and state behind
-        want_rows = torch.tensor(rows if rows else [0], dtype=torch.long).to(self.device)
+        host = host_staging(max(1, len(rows)), torch.long, self.device)
+        host.copy_(torch.tensor(rows if rows else [0], dtype=torch.long))
+        want_rows = host.to(self.device, non_blocking=True)
         out = self.model.step(st, want_rows, return_layers=return_layers)
         for slot, toks in slotted:
             cache.advance(slot, toks)
