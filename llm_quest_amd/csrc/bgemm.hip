@@ -366,12 +366,12 @@ __global__ __launch_bounds__(256) void bgemm_mfma128_kernel(BgemmArgs p) {
 // ---- MFMA path, 256 x 256 tile: eight waves of 128 x 64 (4 x 2 blocks of v_mfma_f32_32x32x16_bf16), k in steps of 64, operands HBM -> LDS by DMA (16 bytes a lane, rows gathered by
 // the lanes' addresses), two stages of 64 KiB: the next step's DMA is in flight while this one multiplies, one barrier a step.  A wave's six LDS fragments feed eight MFMAs (the
 // 128 x 128 kernel's four feed four, behind writes through registers: LDS-bound).  The DMA writes lanes in order, so rows of 128 bytes are swizzled on the source address:
-// 16-byte word c of row r lies at c ^ ((r >> 1) & 7).  Groups: a group's rows are dealt evenly over its ceil(rows / 256) tiles, blocks of 64 rows beyond a tile's end are
+// 16-byte word c of row r lies at c ^ ((r >> 1) & 7).  Groups: a group's rows are dealt evenly over its ceil(rows / 256) tiles, blocks of 32 rows beyond a tile's end are
 // not multiplied; the grid holds what M sorted rows can need at most and a workgroup finds its tile from the offsets (a grid of row tiles x groups would be
 // mostly empty: 114 688 workgroups for 16 groups of 16 384 rows).  Tiles are walked rows first, then columns, then groups, an XCD in one piece: what the tiles of an XCD
 // share stays in its L2.  The write-out goes through LDS: a value by value one (a row look-up and a 2-byte store each) cost as much as 2048 k of products.
-// 16 384 rows in 16 groups, us, before -> now: 2048 -> 2 x 3584 gated 816 -> 706 (690 TFLOP/s), 3584 -> 2048 402 -> 344; 2 048 rows 165 -> 148, 110 -> 89.  What is left: half of
-// the steps' time is not products (one workgroup a CU: fragments are read and DMA waited for behind every barrier), and the gated activation's exponentials run alone.
+// 16 384 rows in 16 groups, us, before -> now: 2048 -> 2 x 3584 gated 816 -> 644 (750 TFLOP/s), 3584 -> 2048 402 -> 318; 2 048 rows 165 -> 148, 110 -> 89.  What is left: half of
+// the steps' time is not products (one workgroup a CU: fragments are read and DMA waited for behind every barrier), and the gated activation's exponentials run alone (90 us).
 // 128 x 256 tiles, three stages of 32 k, two workgroups a CU: 726 and 360 (64-byte rows: twice the requests per byte); turning each column panel's k by some steps: the same.
 constexpr int WTM = 256, WTN = 256, WK = 64, WSTAGES = 2, WSTAGE = (WTM + WTN) * WK * 2;
 __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int batch, int tn) {
@@ -427,10 +427,11 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
             src[i] = (const char*)((const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)min(n0 + r, p.N - 1) * p.sbn + c * 8);
         }
     }
-    auto issue = [&](int t, int stage) {
+    auto issue = [&](int t, int stage, int lo, int hi) {  // (lo, hi: 0, 4 the A pieces, 4, 8 the B pieces)
 #pragma unroll
         for (int i = 0; i < 8; ++i)
-            __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)t * (WK * 2)),
+            if (i >= lo && i < hi)
+                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)t * (WK * 2)),
                                              (__attribute__((address_space(3))) void*)(lds + stage * WSTAGE + (i < 4 ? 0 : WTM * WK * 2) + piece(i) * 1024), 16, 0, 0);
     };
     const int wm = (wave >> 2) * 128, wn = (wave & 3) * 64, nt = p.K / WK;
@@ -451,14 +452,13 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-        issue(0, 0);
+        issue(0, 0, 0, 8);
         rows_of_tile();
         for (int t = 0; t < nt; ++t) {
             // this wave's pieces of the step have landed and its reads of the step before are done -- behind the barrier everyone's
             asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
             __builtin_amdgcn_s_barrier();
             asm volatile("" ::: "memory");
-            if (t + 1 < nt) issue(t + 1, (t + 1) & 1);
             if constexpr (NB > 0) {
                 const char *sa = lds + (t & 1) * WSTAGE, *sb = sa + WTM * WK * 2;
                 bf16x8 fa[2][NB], fb[2][2];  // the fragments of the next 16 k are requested in front of the products of this one
@@ -468,16 +468,18 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
 #pragma unroll
                     for (int i = 0; i < NB; ++i) fa[kk & 1][i] = frag(sa, wm + 32 * i + ln, kk);
                 };
-                read(0);
+                read(0);  // (in front of the DMA's issue, and that in two parts: with all of it first 8192^3 takes 1 020 us instead of 944)
+                if (t + 1 < nt) issue(t + 1, (t + 1) & 1, 0, 4);
 #pragma unroll
                 for (int kk = 0; kk < 4; ++kk) {
                     if (kk < 3) read(kk + 1);
+                    if (kk == 1 && t + 1 < nt) issue(t + 1, (t + 1) & 1, 4, 8);
 #pragma unroll
                     for (int i = 0; i < NB; ++i)
 #pragma unroll
                         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk & 1][i], fb[kk & 1][j], acc[i][j], 0, 0, 0);
                 }
-            }
+            } else if (t + 1 < nt) issue(t + 1, (t + 1) & 1, 0, 8);
         }
         // write-out through the stages' LDS, which nobody reads any more: 64 rows of a wave at a time as fp32, then whole 4-column words of a row to a lane
         __syncthreads();
@@ -489,9 +491,9 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
         for (int j = 0; j < 4; ++j) bias[j] = p.bias && nq + j < n_end ? p.bias[nq + j] : 0.f;
         const bool words = nq + 4 <= n_end && p.ldc % 4 == 0 && p.c_bs % 4 == 0 && ((uintptr_t)p.C & 15) == 0;
 #pragma unroll
-        for (int h = 0; h < NB / 2; ++h) {
+        for (int h = 0; h < (NB + 1) / 2; ++h) {
 #pragma unroll
-            for (int i = 0; i < 2; ++i)
+            for (int i = 0; i < (NB - 2 * h < 2 ? NB - 2 * h : 2); ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
@@ -530,7 +532,8 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
             __builtin_amdgcn_wave_barrier();
         }
     };
-    if (cnt - wm > 64) run(std::integral_constant<int, 4>{});
+    if (cnt - wm > 96) run(std::integral_constant<int, 4>{});
+    else if (cnt - wm > 64) run(std::integral_constant<int, 3>{});
     else if (cnt > wm) run(std::integral_constant<int, 2>{});
     else run(std::integral_constant<int, 0>{});
 }
