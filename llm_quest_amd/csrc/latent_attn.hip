@@ -34,13 +34,16 @@ __device__ __forceinline__ bool key_visible(int j, int lim, int window, int keep
     return j <= lim && (window <= 0 || lim - j < window || j < keep_first) && (chunk <= 0 || j >= lim / chunk * chunk);
 }
 
-__device__ __forceinline__ float lda_dt(const void* p, int dt, int64_t i) { return dt == MI355_DT_F32 ? ((const float*)p)[i] : bf2f(((const bf16_t*)p)[i]); }
+__device__ __forceinline__ float as_f32(float x) { return x; }
+__device__ __forceinline__ float as_f32(bf16_t x) { return bf2f(x); }
 
 #define AM 32  // query rows per tile of the FMA kernel
 #define AN 64  // keys per step
 #define AC 32  // feature chunk of the score product
 
-template <int NC>
+// Bound: a served step has few workgroups (one a sequence, folded form), each a chain of memory round trips; so the next feature chunk of keys and queries is requested while this one
+// is multiplied, and values eight keys at a time (one by one they were 64 round trips a key step): three sequences of 150 keys, 8 heads, 256 + 64 | 256 wide, 248 -> 118 us; a prompt of 150 tokens (128 + 64 | 128) 159 -> 80. The order of every sum is as before.
+template <int NC, typename KV>
 __global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p) {
     __shared__ float Qs[AM][AC + 1];
     __shared__ float Ks[AN][AC + 1];
@@ -96,27 +99,35 @@ __global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p) {
             if (j0 >= n_keys) break;
             if (j0 + AN <= win_lo && j0 >= p.keep_first) continue;  // block-uniform: no row sees a key of this step
         }
-        const void* Kp = seg ? p.PK : p.K1;
-        const void* Vp = seg ? p.PV : p.V;
+        const KV* Kp = (const KV*)(seg ? p.PK : p.K1);
+        const KV* Vp = (const KV*)(seg ? p.PV : p.V);
         const int64_t kr = seg ? pr0 : k1r0, vr = seg ? pr0 : vr0, ldk = seg ? p.ldp : p.ldk1, ldvv = seg ? p.ldp : p.ldv;
         float acc[2][4] = {};
-        for (int d0 = 0; d0 < DK; d0 += AC) {
-            __syncthreads();
+        float qn[4];
+        KV kn[8];
+        auto request = [&](int d0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {  // Q chunk: 32 rows x 32 features
                 const int e = tid + 256 * i, d = d0 + (e & 31), r = e >> 5;
                 const int tok = tok0 + r / p.hm, head = head0 + r % p.hm;
-                Qs[r][e & 31] = (d < DK && tok < n_new && head < p.H) ? p.Q[(qr0 + tok) * p.ldq + (int64_t)head * p.q_hs + d] : 0.f;
+                qn[i] = (d < DK && tok < n_new && head < p.H) ? p.Q[(qr0 + tok) * p.ldq + (int64_t)head * p.q_hs + d] : 0.f;
             }
 #pragma unroll
             for (int i = 0; i < 8; ++i) {  // K chunk: 64 keys x 32 features
                 const int e = tid + 256 * i, d = d0 + (e & 31), j = j0 + (e >> 5);
-                float v = 0.f;
-                if (j < n_here && d < DK)
-                    v = d < p.D1 ? lda_dt(Kp, p.dt, (kr + j) * ldk + (int64_t)kvh * p.k1_hs + d) : lda_dt(p.K2, p.dt, (k2r0 + j) * p.ldk2 + (d - p.D1));
-                Ks[e >> 5][e & 31] = v;
+                kn[i] = (KV)0;
+                if (j < n_here && d < DK) kn[i] = d < p.D1 ? Kp[(kr + j) * ldk + (int64_t)kvh * p.k1_hs + d] : ((const KV*)p.K2)[(k2r0 + j) * p.ldk2 + (d - p.D1)];
             }
+        };
+        request(0);
+        for (int d0 = 0; d0 < DK; d0 += AC) {
             __syncthreads();
+#pragma unroll
+            for (int i = 0; i < 4; ++i) Qs[(tid + 256 * i) >> 5][tid & 31] = qn[i];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) Ks[(tid + 256 * i) >> 5][tid & 31] = as_f32(kn[i]);
+            __syncthreads();
+            if (d0 + AC < DK) request(d0 + AC);
 #pragma unroll
             for (int d = 0; d < AC; ++d) {
                 const float q0 = Qs[2 * ty][d], q1 = Qs[2 * ty + 1][d];
@@ -166,18 +177,26 @@ __global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p) {
 #pragma unroll
             for (int i = 0; i < NC; ++i) o[r][i] *= f;
         }
-        for (int j = 0; j < nk; ++j) {
-            float vv[NC];
+        constexpr int VG = NC <= 4 ? 8 : 4;  // keys requested together
+        for (int jg = 0; jg < nk; jg += VG) {
+            KV vv[VG][NC];
 #pragma unroll
-            for (int i = 0; i < NC; ++i) {
-                const int col = c + 64 * i;
-                vv[i] = col < p.DV ? lda_dt(Vp, p.dt, (vr + j0 + j) * ldvv + (int64_t)kvh * p.v_hs + col) : 0.f;
-            }
+            for (int u = 0; u < VG; ++u)
 #pragma unroll
-            for (int r = 0; r < 8; ++r) {
-                const float pj = Ps[8 * rg + r][j];
+                for (int i = 0; i < NC; ++i) {
+                    const int col = c + 64 * i;
+                    vv[u][i] = (KV)0;
+                    if (jg + u < nk && col < p.DV) vv[u][i] = Vp[(vr + j0 + jg + u) * ldvv + (int64_t)kvh * p.v_hs + col];
+                }
 #pragma unroll
-                for (int i = 0; i < NC; ++i) o[r][i] = fmaf(pj, vv[i], o[r][i]);
+            for (int u = 0; u < VG; ++u) {
+                if (jg + u >= nk) break;
+#pragma unroll
+                for (int r = 0; r < 8; ++r) {
+                    const float pj = Ps[8 * rg + r][jg + u];
+#pragma unroll
+                    for (int i = 0; i < NC; ++i) o[r][i] = fmaf(pj, as_f32(vv[u][i]), o[r][i]);
+                }
             }
         }
     }
@@ -592,10 +611,9 @@ extern "C" int mi355_latent_attn(int n_seq, int max_new, int H, int hm, int D1, 
         }
         return 0;
     }
-    if (DV <= 64) latent_attn_fma_kernel<1><<<grid, 256, 0, ST(stream)>>>(p);
-    else if (DV <= 128) latent_attn_fma_kernel<2><<<grid, 256, 0, ST(stream)>>>(p);
-    else if (DV <= 256) latent_attn_fma_kernel<4><<<grid, 256, 0, ST(stream)>>>(p);
-    else latent_attn_fma_kernel<8><<<grid, 256, 0, ST(stream)>>>(p);
+#define FMA(NC) do { if (dt == MI355_DT_F32) latent_attn_fma_kernel<NC, float><<<grid, 256, 0, ST(stream)>>>(p); else latent_attn_fma_kernel<NC, bf16_t><<<grid, 256, 0, ST(stream)>>>(p); } while (0)
+    if (DV <= 64) FMA(1); else if (DV <= 128) FMA(2); else if (DV <= 256) FMA(4); else FMA(8);
+#undef FMA
     MI355_LAUNCH_CHECK("latent_attn");
     return 0;
 }
