@@ -260,6 +260,12 @@ int mi355_layernorm_fwd(int64_t rows, int width, const float* x, const float* sc
 int mi355_layernorm_bwd(int64_t rows, int width, const float* x, const float* scale, const float* mean, const float* rsig,
                         const void* dy, int dy_dtype, const float* dres, float* dx, float* dparam_partial, int parts,
                         float eps, int mode, void* stream);
+/* mi355_layernorm_bwd that also leaves dx as bf16 and its column sums (of the bf16 values: the bias gradient of the layer whose output dx belongs to): partial fp32
+ * [parts][3 * width] = dscale | dshift | column sums.  width 768 or 1024, operands 16-byte aligned. */
+int mi355_layernorm_bwd_bf16(int64_t rows, int width, const float* x, const float* scale, const float* mean, const float* rsig, const void* dy, int dy_dtype,
+                             const float* dres, float* dx, void* dx_bf16, float* partial, int parts, float eps, int mode, void* stream);
+/* mi355_reduce_rows_f32 over partial [parts][segments * n], every segment into a destination of its own (NULL: dropped; bit i of accumulate: added to). */
+int mi355_reduce_rows_into(int parts, int segments, int64_t n, const float* partial, float* d0, float* d1, float* d2, float* d3, int accumulate, void* stream);
 
 /* dtype conversion / elementwise helpers */
 int mi355_cast(int64_t n, const void* src, int src_dtype, void* dst, int dst_dtype, void* stream);

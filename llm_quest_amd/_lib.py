@@ -52,6 +52,8 @@ SIGNATURES = {
     "mi355_transpose_bf16": [_L, _L, _P, _L, _P, _L, _P],
     "mi355_patchify": [_I, _I, _I, _I, _I, _P, _P, _I, _P],
     "mi355_layernorm_fwd": [_L, _I, _P, _P, _P, _P, _I, _P, _P, _F, _I, _P],
+    "mi355_layernorm_bwd_bf16": [_L, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _F, _I, _P],
+    "mi355_reduce_rows_into": [_I, _I, _L, _P, _P, _P, _P, _P, _I, _P],
     "mi355_layernorm_bwd": [_L, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _F, _I, _P],
     "mi355_cast": [_L, _P, _I, _P, _I, _P],
     "mi355_vit_embed_assemble": [_I, _I, _I, _P, _P, _P, _P, _P],

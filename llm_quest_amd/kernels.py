@@ -839,8 +839,9 @@ def gelu_bwd(x, dy, tanh=False):
     return dx
 
 
-def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=None, dshift_out=None, accumulate=False, mode=0):
-    """Returns dx fp32 (+ dres).  dscale/dshift go to the given fp32 destinations (optionally accumulated) or new tensors."""
+def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=None, dshift_out=None, accumulate=False, mode=0, dests=None):
+    """Returns dx fp32 (+ dres).  dscale/dshift go to the given fp32 destinations (optionally accumulated) or new tensors.  ``dests`` (two, see ``reduce_rows_into``): straight into
+    them, and only dx is returned."""
     L.require_gpu(x2d, dy, dres)
     rows, width = x2d.shape
     if x2d.dtype != F32 or not x2d.is_contiguous() or not dy.is_contiguous() or dy.shape != x2d.shape:
@@ -851,6 +852,9 @@ def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=No
     parts = min(1024, (rows + 3) // 4)
     part = torch.empty((parts, 2 * width), dtype=F32, device=x2d.device)
     L.call("mi355_layernorm_bwd", rows, width, L.ptr(x2d), L.ptr(scale), L.ptr(mean), L.ptr(rsig), L.ptr(dy), L.dt_code(dy.dtype), L.ptr(dres), L.ptr(dx), L.ptr(part), parts, eps, mode)
+    if dests is not None:
+        reduce_rows_into(part, parts, width, dests)
+        return dx
     both = torch.empty(2 * width, dtype=F32, device=x2d.device)
     L.call("mi355_reduce_rows_f32", parts, 2 * width, L.ptr(part), L.ptr(both), L.DT_F32, 0)
     outs = []
@@ -864,6 +868,34 @@ def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=No
                 L.call("mi355_reduce_rows_f32", 1, width, L.ptr(src.contiguous()), L.ptr(dst), L.DT_F32, 0)
             outs.append(dst)
     return dx, outs[0], outs[1]
+
+
+def reduce_rows_into(partial, parts, width, dests):
+    """``dests`` = one (fp32 tensor of ``width`` elements, accumulate) or None per segment of partial [parts, len(dests) * width]: the segments' column sums in one launch."""
+    if any(d is not None for d in dests):
+        ptrs = [None if d is None else d[0].data_ptr() for d in dests] + [None] * (4 - len(dests))
+        L.call("mi355_reduce_rows_into", parts, len(dests), width, L.ptr(partial), *ptrs, sum(1 << i for i, d in enumerate(dests) if d is not None and d[1]))
+
+
+def layernorm_bwd_bf16_fits(x2d, scale, dy, dres):
+    """Whether ``layernorm_bwd_bf16`` holds these operands (the widths whose rows stay in registers, 16-byte words)."""
+    return x2d.shape[1] in (768, 1024) and not (x2d.data_ptr() | dy.data_ptr() | scale.data_ptr() | (0 if dres is None else dres.data_ptr())) % 16
+
+
+def layernorm_bwd_bf16(x2d, scale, mean, rsig, dy, dres, dests, eps=1e-5, mode=0):
+    """``layernorm_bwd`` -> (dx fp32, dx bf16); ``dests`` = destinations (see ``reduce_rows_into``) of the gradients of scale, shift and of the bias whose output dx is the gradient of."""
+    L.require_gpu(x2d, dy, dres)
+    rows, width = x2d.shape
+    if x2d.dtype != F32 or not x2d.is_contiguous() or not dy.is_contiguous() or dy.shape != x2d.shape:
+        raise ValueError("layernorm_bwd: x fp32 contiguous, dy contiguous of the same shape")
+    if dres is not None and (dres.dtype != F32 or not dres.is_contiguous() or dres.shape != x2d.shape):
+        raise ValueError("layernorm_bwd: dres must be contiguous fp32 like x")
+    dx, dxb = torch.empty_like(x2d), torch.empty((rows, width), dtype=BF16, device=x2d.device)
+    parts = min(1024, (rows + 3) // 4)
+    part = torch.empty((parts, 3 * width), dtype=F32, device=x2d.device)
+    L.call("mi355_layernorm_bwd_bf16", rows, width, L.ptr(x2d), L.ptr(scale), L.ptr(mean), L.ptr(rsig), L.ptr(dy), L.dt_code(dy.dtype), L.ptr(dres), L.ptr(dx), L.ptr(dxb), L.ptr(part), parts, eps, mode)
+    reduce_rows_into(part, parts, width, dests)
+    return dx, dxb
 
 
 def patchify3d(video, patch, tpatch, out_dtype=BF16):

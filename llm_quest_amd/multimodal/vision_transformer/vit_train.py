@@ -60,11 +60,21 @@ def _bgrad(p, dy):
     K.colsum(dy, out=dst.view(-1), accumulate=acc)
 
 
+def _dest(p):
+    """Destination of ``K.reduce_rows_into`` for parameter p."""
+    return _grad_buf(p) if p is not None and p.requires_grad else None
+
+
+def _ln_bwd_bf16(ln, x2d, mean, rsig, dy, dres, bias):
+    """LayerNorm backward whose result is the gradient of a Linear's output (``bias``): (dx, dx in bf16 with the bias gradient done, or None -- the Linear's backward makes its own)."""
+    scale = ln.scale.detach()
+    if not K.layernorm_bwd_bf16_fits(x2d, scale, dy, dres):
+        return _ln_bwd(ln, x2d, mean, rsig, dy, dres), None
+    return K.layernorm_bwd_bf16(x2d, scale, mean, rsig, dy, dres, (_dest(ln.scale), _dest(ln.shift), _dest(bias)), eps=ln.eps)
+
+
 def _ln_bwd(ln, x2d, mean, rsig, dy, dres):
-    dx, dsc, dsh = K.layernorm_bwd(x2d, ln.scale.detach(), mean, rsig, dy, dres=dres, eps=ln.eps)
-    _acc(ln.scale, dsc.contiguous())
-    _acc(ln.shift, dsh.contiguous())
-    return dx
+    return K.layernorm_bwd(x2d, ln.scale.detach(), mean, rsig, dy, dres=dres, eps=ln.eps, dests=(_dest(ln.scale), _dest(ln.shift)))
 
 
 
@@ -112,19 +122,22 @@ def att_forward(att, h1, B, S, training, residual=None, out_dtype=F32, p_res=0.0
     return y, (h1, qkv, ctx, lse, (B, S), (p_att, s_att, p_res, s_proj))
 
 
-def att_backward(att, saved, dy, wg=None):
-    """dy: gradient of the piece's output (fp32 or bf16 rows).  Returns d(h1) bf16; weight / bias gradients land in ``.grad``."""
+def att_backward(att, saved, dy, wg=None, dyb=None):
+    """dy: gradient of the piece's output (fp32 or bf16 rows).  Returns d(h1) bf16; weight / bias gradients land in ``.grad``.  ``dyb``: dy in bf16, the gradient of the output
+    projection's bias already taken from it (no residual dropout)."""
     h1, qkv, ctx, lse, (B, S), (p_att, s_att, p_res, s_proj) = saved
     d, H, Dh = att.d_out, att.num_heads, att.head_dim
+    bias_done = dyb is not None
     if p_res > 0:
         dyb = K.dropout(dy if dy.dtype == F32 else K.cast(dy, F32), p_res, *s_proj, out_dtype=BF16)
-    else:
+    elif dyb is None:
         dyb = dy if dy.dtype == BF16 else K.cast(dy, BF16)
     own = wg is None
     wg = [] if own else wg
     dctx = K.dgrad(dyb, bf16_cached(att, "wo", [att.out_proj.weight]))
     _wgrad(att.out_proj.weight, dyb, ctx, wg)
-    _bgrad(att.out_proj.bias, dyb)
+    if not bias_done:
+        _bgrad(att.out_proj.bias, dyb)
     dqkv = torch.empty_like(qkv)
     if p_att > 0:
         K.attn_dropout_bwd(qkv[:, :d], qkv[:, d : 2 * d], qkv[:, 2 * d :], ctx, dctx, lse, B, S, H, H, Dh,
@@ -137,9 +150,7 @@ def att_backward(att, saved, dy, wg=None):
     for i, lin in enumerate((att.w_queries, att.w_keys, att.w_values)):
         _wgrad(lin.weight, dqkv[:, i * d : (i + 1) * d], h1, wg)
     if att.w_queries.bias is not None:
-        gb = K.colsum(dqkv)
-        for i, lin in enumerate((att.w_queries, att.w_keys, att.w_values)):
-            _acc(lin.bias, gb[i * d : (i + 1) * d])
+        K.reduce_rows_into(K.colsum(dqkv), 1, d, [_dest(lin.bias) for lin in (att.w_queries, att.w_keys, att.w_values)])
     if own:
         ops._flush_wgrads(wg)
     return dh1
@@ -159,17 +170,20 @@ def ffn_forward(ffn, h2, residual=None, out_dtype=F32, p_res=0.0):
     return y, (h2, y1, f, (p_res, s_ffn))
 
 
-def ffn_backward(ffn, saved, dy, wg=None):
+def ffn_backward(ffn, saved, dy, wg=None, dyb=None):
+    """``dyb``: dy in bf16, the gradient of the second layer's bias already taken from it (no residual dropout)."""
     h2, y1, f, (p_res, s_ffn) = saved
+    bias_done = dyb is not None
     if p_res > 0:  # the dropout site's backward is the same mask on the gradient, fused with the bf16 cast
         dyb = K.dropout(dy if dy.dtype == F32 else K.cast(dy, F32), p_res, *s_ffn, out_dtype=BF16)
-    else:
+    elif dyb is None:
         dyb = dy if dy.dtype == BF16 else K.cast(dy, BF16)
     own = wg is None
     wg = [] if own else wg
     dy1 = K.gemm_dgrad_gelu_bwd(dyb, bf16_cached(ffn, "w2", [ffn.layers[2].weight]), y1)  # GELU backward in the dgrad epilogue
     _wgrad(ffn.layers[2].weight, dyb, f, wg)
-    _bgrad(ffn.layers[2].bias, dyb)
+    if not bias_done:
+        _bgrad(ffn.layers[2].bias, dyb)
     dh2 = K.dgrad(dy1, bf16_cached(ffn, "w1", [ffn.layers[0].weight]))
     _wgrad(ffn.layers[0].weight, dy1, h2, wg)
     _bgrad(ffn.layers[0].bias, dy1)
@@ -190,14 +204,26 @@ def block_forward(blk, x, B, S, training):
 
 def block_backward(blk, saved, dx, B, S):
     """dx fp32 [B*S, d] = gradient of the block's output; returns the gradient of its input; one grouped launch for the six weight gradients."""
+    return chained_block_backward(blk, saved, dx, B, S)[0]
+
+
+def chained_block_backward(blk, saved, dx, B, S, dxb=None, below=None):
+    """``block_backward`` of one block of a stack: returns (the gradient of its input, ``dxb`` of the block ``below`` it or None).  ``dxb``: dx in bf16 from the LayerNorm backward above, with this block's last bias gradient done; ``below``: the block to do the same for (without residual dropout).  A LayerNorm's backward has its result in registers: it rounds it
+    for the products below and sums its columns there (22 launches a block instead of 34)."""
     x, mean1, rsig1, sv_att, x2, mean2, rsig2, sv_ffn = saved
     wg = []
-    dh2 = ffn_backward(blk.ffn, sv_ffn, dx, wg)
-    dx2 = _ln_bwd(blk.ln_2, x2, mean2, rsig2, dh2, dx)
-    dh1 = att_backward(blk.att, sv_att, dx2, wg)
-    dxin = _ln_bwd(blk.ln_1, x, mean1, rsig1, dh1, dx2)
+    dh2 = ffn_backward(blk.ffn, sv_ffn, dx, wg, dxb)
+    if sv_att[5][2] > 0:  # residual dropout: the products' operand is the masked gradient
+        dx2, dx2b = _ln_bwd(blk.ln_2, x2, mean2, rsig2, dh2, dx), None
+    else:
+        dx2, dx2b = _ln_bwd_bf16(blk.ln_2, x2, mean2, rsig2, dh2, dx, blk.att.out_proj.bias)
+    dh1 = att_backward(blk.att, sv_att, dx2, wg, dx2b)
+    if below is not None:
+        dxin, dxb = _ln_bwd_bf16(blk.ln_1, x, mean1, rsig1, dh1, dx2, below.ffn.layers[2].bias)
+    else:
+        dxin, dxb = _ln_bwd(blk.ln_1, x, mean1, rsig1, dh1, dx2), None
     ops._flush_wgrads(wg)
-    return dxin
+    return dxin, dxb
 
 
 class PieceFn(torch.autograd.Function):
@@ -292,8 +318,10 @@ def vit_backward(m, saved, dout):
         dcls = _ln_bwd(ln, cls_rows, meanf, rsigf, dcls_n, None)
         dx = torch.zeros((B * S, d), dtype=F32, device=dcls.device)
         K.copy2d(dcls, dx.view(B, S * d)[:, :d])
-    for blk, sv in zip(reversed(m.transformer_blocks), reversed(saved_blocks)):
-        dx = block_backward(blk, sv, dx, B, S)
+    blocks, dxb = list(m.transformer_blocks), None
+    for i in reversed(range(len(blocks))):
+        masked = i > 0 and saved_blocks[i - 1][7][3][0] > 0  # residual dropout of the block below: what its forward did, whatever mode it is in now
+        dx, dxb = chained_block_backward(blocks[i], saved_blocks[i], dx, B, S, dxb, blocks[i - 1] if i > 0 and not masked else None)
     # ---- embedding: dropout site, pos / cls sums over the batch, patch projection wgrad
     if p_emb > 0:
         dx = K.dropout(dx, p_emb, *s_emb)

@@ -1155,3 +1155,28 @@ def test_products_in_two_launches_equal_one(form, M, N, K, case):
         assert bool((buf[M] == 7).all()) and bool((buf[:, N:] == 7).all())
         outs.append(buf[:M, :N])
     assert torch.equal(*outs)
+
+
+@pytest.mark.parametrize("rows,width,dt,res", [(5, 768, torch.bfloat16, True), (985, 768, torch.float32, False), (4099, 1024, torch.bfloat16, True), (1, 1024, torch.float32, True)])
+def test_layernorm_backward_with_bf16_result_and_column_sums(rows, width, dt, res):
+    """mi355_layernorm_bwd_bf16 + mi355_reduce_rows_into against the separate launches: the same dx, its bf16 rounding, its column sums (fp32 sums of `rows` terms), and every
+    destination written, added to or left out as asked for."""
+    from llm_quest_amd import kernels as KK
+
+    g = torch.Generator().manual_seed(rows + width)
+    x, scale, dy = torch.randn(rows, width, generator=g).cuda(), torch.randn(width, generator=g).cuda(), torch.randn(rows, width, generator=g).to(dt).cuda()
+    dres = torch.randn(rows, width, generator=g).cuda() if res else None
+    _, mean, rsig = KK.layernorm_fwd(x, scale, torch.zeros(width, device="cuda"), out_dtype=torch.bfloat16, eps=1e-5, want_stats=True)
+    want_dx, want_sc, want_sh = KK.layernorm_bwd(x, scale, mean, rsig, dy, dres=dres)
+    assert KK.layernorm_bwd_bf16_fits(x, scale, dy, dres) and not KK.layernorm_bwd_bf16_fits(x[:, : width - 64], scale, dy, dres)
+    old = torch.randn(width, generator=g).cuda()
+    dsc, bias = old.clone(), torch.full((width,), float("nan"), device="cuda")
+    dx, dxb = KK.layernorm_bwd_bf16(x, scale, mean, rsig, dy, dres, ((dsc, True), None, (bias, False)))
+    assert torch.equal(dx, want_dx) and torch.equal(dxb, want_dx.to(torch.bfloat16))
+    assert torch.equal(dsc, old + want_sc)
+    exact = dxb.double().sum(0)
+    assert bool(((bias.double() - exact).abs() <= 2.0 ** -24 * rows * dxb.double().abs().sum(0)).all())
+    dsh = torch.empty(width, device="cuda")
+    assert torch.equal(KK.layernorm_bwd(x, scale, mean, rsig, dy, dres=dres, dests=(None, (dsh, False))), want_dx) and torch.equal(dsh, want_sh)
+    with pytest.raises(RuntimeError, match="width"):
+        KK.L.call("mi355_layernorm_bwd_bf16", 1, 512, *([x.data_ptr()] * 5), 1, None, *([dx.data_ptr()] * 3), 1, 1e-5, 0)
