@@ -201,6 +201,32 @@ def test_causal_conv_silu(B, S, C):
     assert not dbuf.cpu()[:, C:].any()
 
 
+@pytest.mark.parametrize("B,S,C", [(1, 1, 8), (2, 3, 24), (3, 32, 2056), (1, 33, 64), (2, 35, 136), (1, 101, 8)])
+def test_causal_conv_silu_backward_at_chunk_edges(B, S, C):
+    """One pass over chunks of 32 tokens with the three behind them: sequences around a chunk's end and shorter than the window; against the same arithmetic (dc rounded to bf16)
+    in fp64, and the same bits where dx overwrites x's or dy's rows."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    torch.manual_seed(S + C)
+    x, w, g = torch.randn(B * S, C + 16).to(BF16), (0.5 * torch.randn(C, 1, 4)).to(BF16), torch.randn(B * S, C).to(BF16)
+    xd, gd, dx = x.cuda(), g.cuda(), torch.full((B * S, C + 8), 5.0, dtype=BF16, device="cuda")
+    dw = Q.causal_conv_silu_bwd(xd[:, :C], w.cuda(), gd, dx[:, :C], B, S)
+    p = torch.nn.functional.pad(x[:, :C].double().view(B, S, C), (0, 0, 3, 0))
+    win = torch.stack([p[:, j : j + S] for j in range(4)], -1)  # [B, S, C, 4]
+    c = (win * w.double().view(C, 4)).sum(-1).float().to(BF16).double()
+    sg = torch.sigmoid(c)
+    dc = (g.double().view(B, S, C) * sg * (1 + c * (1 - sg))).float().to(BF16).double()
+    q = torch.nn.functional.pad(dc, (0, 0, 0, 3))
+    want = sum(w.double().view(C, 4)[:, j] * q[:, 3 - j : 3 - j + S] for j in range(4))
+    assert rel_l2(dx[:, :C], want.reshape(B * S, C)) < 3e-3 and rel_l2(dw.view(C, 4), (dc.unsqueeze(-1) * win).sum((0, 1))) < 1e-3  # one bf16 rounding; a rounding of dc that falls the other way
+    assert bool((dx[:, C:] == 5.0).all())
+    ref = dx[:, :C].clone()
+    over_x, over_g = xd.clone(), gd.clone()
+    Q.causal_conv_silu_bwd(over_x[:, :C], w.cuda(), gd, over_x[:, :C], B, S)
+    Q.causal_conv_silu_bwd(xd[:, :C], w.cuda(), over_g, over_g, B, S)
+    assert torch.equal(over_x[:, :C], ref) and torch.equal(over_g, ref)
+
+
 def test_l2norm():
     from llm_quest_amd import kernels_q35 as Q
 
