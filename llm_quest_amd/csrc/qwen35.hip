@@ -13,6 +13,7 @@
 //                        independent recurrence, so rows are spread over lanes and the time loop runs inside the kernel
 //   gated_rmsnorm        RMSNorm(fp32) * silu(gate) -> bf16
 //   rowmask              x * padding_mask
+#include <initializer_list>
 #include "common.h"
 #include "lane_sums.h"
 
@@ -474,6 +475,135 @@ __global__ __launch_bounds__(256) void conv_silu_step_kernel(int B, int C, const
 #pragma unroll
     for (int c = 0; c < 8; ++c) o[c] = silu_f(rbf(acc[c]));
     *reinterpret_cast<u32x4*>(y + (int64_t)b * C + c0) = pack8(o);
+}
+
+// ------------------------------------------------------------------------------------------- rows of whole 16-byte pieces
+// The row kernels of q, k and the gated norm, with G = 8, 16 or 32 lanes to a row of D = 8 G values: a lane asks for 16 bytes of each operand, 64 / G rows share a
+// wavefront and a row's sums cross log2(G) lanes.  Bound: bytes; two bytes a lane and one row a wavefront left the loads too small and the six-step sums in the way.
+// 5 664 tokens x 16 heads of 128, a row a wavefront -> here: l2norm 20 -> 9 us, backward 35 -> 13; gated norm 40 -> 21 us, backward 88 -> 41.
+// Rows of other widths, offsets or pitches off 16 bytes, and 2^31 rows and more take a row a wavefront.
+template <int G>
+__device__ __forceinline__ float lanes_sum(float v) {
+#pragma unroll
+    for (int o = G / 2; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    return v;
+}
+__device__ __forceinline__ void load8(const bf16_t* p, float (&f)[8]) { unpack8(*reinterpret_cast<const u32x4*>(p), f); }
+__device__ __forceinline__ void store8(bf16_t* p, const float (&f)[8]) { *reinterpret_cast<u32x4*>(p) = pack8(f); }
+
+template <int G>
+__global__ __launch_bounds__(256) void l2norm_fwd_rows_kernel(unsigned total, int H, const bf16_t* __restrict__ x, int64_t ldx, bf16_t* __restrict__ y) {
+    constexpr int D = 8 * G, RPB = 256 / G;
+    const int c0 = (threadIdx.x % G) * 8;
+    const float floor_ = rbf(1e-6f);
+    for (unsigned item = blockIdx.x * RPB + threadIdx.x / G; item < total; item += gridDim.x * RPB) {
+        const unsigned t = item / (unsigned)H, h = item - t * (unsigned)H;
+        float v[8], ss = 0.f;
+        load8(x + (int64_t)t * ldx + (int64_t)h * D + c0, v);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) ss += v[c] * v[c];
+        ss = lanes_sum<G>(ss);
+        const float inv = rbf(1.f / fmaxf(rbf(sqrtf(ss)), floor_));
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v[c] *= inv;
+        store8(y + (int64_t)item * D + c0, v);
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void l2norm_bwd_rows_kernel(unsigned total, int H, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ dy,
+                                                              bf16_t* __restrict__ dx, int64_t lddx) {
+    constexpr int D = 8 * G, RPB = 256 / G;
+    const int c0 = (threadIdx.x % G) * 8;
+    for (unsigned item = blockIdx.x * RPB + threadIdx.x / G; item < total; item += gridDim.x * RPB) {
+        const unsigned t = item / (unsigned)H, h = item - t * (unsigned)H;
+        float v[8], g[8], ss = 0.f, dot = 0.f;
+        load8(x + (int64_t)t * ldx + (int64_t)h * D + c0, v);
+        load8(dy + (int64_t)item * D + c0, g);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            ss += v[c] * v[c];
+            dot += v[c] * g[c];
+        }
+        ss = lanes_sum<G>(ss);
+        dot = lanes_sum<G>(dot);
+        const float n = sqrtf(ss), inv = 1.f / fmaxf(n, 1e-6f);
+        const float k3 = n < 1e-6f ? 0.f : dot * inv * inv * inv;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) g[c] = g[c] * inv - v[c] * k3;
+        store8(dx + (int64_t)t * lddx + (int64_t)h * D + c0, g);
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void gated_rmsnorm_fwd_rows_kernel(unsigned total, int H, const bf16_t* __restrict__ o, const float* __restrict__ w,
+                                                                     const bf16_t* __restrict__ gate, int64_t ldg, bf16_t* __restrict__ out, float* __restrict__ rstd, float eps) {
+    constexpr int D = 8 * G, RPB = 256 / G;
+    const int c0 = (threadIdx.x % G) * 8;
+    float wv[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) wv[c] = w[c0 + c];
+    for (unsigned item = blockIdx.x * RPB + threadIdx.x / G; item < total; item += gridDim.x * RPB) {
+        const unsigned t = item / (unsigned)H, h = item - t * (unsigned)H;
+        float v[8], g[8], ss = 0.f;
+        load8(o + (int64_t)item * D + c0, v);
+        load8(gate + (int64_t)t * ldg + (int64_t)h * D + c0, g);
+#pragma unroll
+        for (int c = 0; c < 8; ++c) ss += v[c] * v[c];
+        ss = lanes_sum<G>(ss);
+        const float r = rsqrtf(ss / (float)D + eps);
+        if (c0 == 0) rstd[item] = r;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) v[c] = silu_f(g[c]) * (v[c] * r * wv[c]);
+        store8(out + (int64_t)item * D + c0, v);
+    }
+}
+
+template <int G>
+__global__ __launch_bounds__(256) void gated_rmsnorm_bwd_rows_kernel(unsigned total, int H, const bf16_t* __restrict__ o, const float* __restrict__ w,
+                                                                     const bf16_t* __restrict__ gate, int64_t ldg, const float* __restrict__ rstd,
+                                                                     const bf16_t* __restrict__ dout, bf16_t* __restrict__ d_o, bf16_t* __restrict__ dgate, int64_t lddg,
+                                                                     float* __restrict__ dw_partial) {
+    constexpr int D = 8 * G, RPB = 256 / G;
+    __shared__ float dw_lds[RPB][D];
+    const int c0 = (threadIdx.x % G) * 8, row = threadIdx.x / G;
+    float wv[8], dwacc[8];
+#pragma unroll
+    for (int c = 0; c < 8; ++c) {
+        wv[c] = w[c0 + c];
+        dwacc[c] = 0.f;
+    }
+    for (unsigned item = blockIdx.x * RPB + row; item < total; item += gridDim.x * RPB) {
+        const unsigned t = item / (unsigned)H, h = item - t * (unsigned)H;
+        float xh[8], g[8], dy[8], dot = 0.f;
+        load8(o + (int64_t)item * D + c0, xh);
+        load8(gate + (int64_t)t * ldg + (int64_t)h * D + c0, g);
+        load8(dout + (int64_t)item * D + c0, dy);
+        const float r = rstd[item];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            xh[c] *= r;
+            const float dn = dy[c] * silu_f(g[c]);
+            g[c] = dy[c] * (xh[c] * wv[c]) * dsilu_f(g[c]);
+            dwacc[c] += dn * xh[c];
+            dy[c] = dn * wv[c];
+            dot += dy[c] * xh[c];
+        }
+        dot = lanes_sum<G>(dot) / (float)D;
+#pragma unroll
+        for (int c = 0; c < 8; ++c) dy[c] = r * (dy[c] - xh[c] * dot);
+        store8(dgate + (int64_t)t * lddg + (int64_t)h * D + c0, g);
+        store8(d_o + (int64_t)item * D + c0, dy);
+    }
+#pragma unroll
+    for (int c = 0; c < 8; ++c) dw_lds[row][c0 + c] = dwacc[c];
+    __syncthreads();
+    for (int i = threadIdx.x; i < D; i += 256) {
+        float s = 0.f;
+#pragma unroll
+        for (int k = 0; k < RPB; ++k) s += dw_lds[k][i];
+        dw_partial[(int64_t)blockIdx.x * D + i] = s;
+    }
 }
 
 // ------------------------------------------------------------------------------------------- l2 norm of q / k heads
@@ -1095,10 +1225,20 @@ __global__ __launch_bounds__(256) void gated_rmsnorm_bwd_kernel(int64_t tokens, 
 }
 
 inline int grid1d(int64_t n, int per_block = 256) { return (int)((n + per_block - 1) / per_block); }
+// rows for the kernels above: lanes to a row (8, 16 or 32), or 0 for a row a wavefront
+inline int row_lanes(int64_t rows, int D, int64_t lds, std::initializer_list<const void*> ptrs) {
+    uintptr_t a = 0;
+    for (const void* p : ptrs) a |= (uintptr_t)p;
+    return (D == 64 || D == 128 || D == 256) && rows < (INT64_C(1) << 31) - (INT64_C(1) << 20) && lds % 8 == 0 && (a & 15) == 0 ? D / 8 : 0;
+}
+#define ROW_LANES(g, LAUNCH) \
+    if (g == 8) { LAUNCH(8); } else if (g == 16) { LAUNCH(16); } else { LAUNCH(32); }
+
 inline int wave_grid(int64_t items, int cap) {
     int64_t g = (items + 3) / 4;
     return (int)(g < 1 ? 1 : (g > cap ? cap : g));
 }
+inline int rows_grid(int64_t rows, int lanes) { return wave_grid((rows * lanes + 63) / 64, 2048); }
 
 }  // namespace
 
@@ -1240,6 +1380,13 @@ extern "C" int mi355_causal_conv_silu_step(int B, int C, int ksize, const void* 
 
 extern "C" int mi355_l2norm_fwd(int64_t tokens, int H, int D, const void* x, int64_t ldx, void* y, void* stream) {
     MI355_REQUIRE(tokens > 0 && H > 0 && D > 0 && D <= 256 && x && y && ldx >= (int64_t)H * D, "l2norm_fwd: bad arguments (head_dim <= 256)");
+    if (const int g = row_lanes(tokens * H, D, ldx, {x, y})) {
+#define RUN(G) l2norm_fwd_rows_kernel<G><<<rows_grid(tokens * H, G), 256, 0, ST(stream)>>>((unsigned)(tokens * H), H, (const bf16_t*)x, ldx, (bf16_t*)y)
+        ROW_LANES(g, RUN)
+#undef RUN
+        MI355_LAUNCH_CHECK("l2norm_fwd");
+        return 0;
+    }
     const int grid = wave_grid(tokens * H, 8192);
     if (D <= 64) l2norm_fwd_kernel<1><<<grid, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)x, ldx, (bf16_t*)y);
     else if (D <= 128) l2norm_fwd_kernel<2><<<grid, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)x, ldx, (bf16_t*)y);
@@ -1249,6 +1396,13 @@ extern "C" int mi355_l2norm_fwd(int64_t tokens, int H, int D, const void* x, int
 }
 extern "C" int mi355_l2norm_bwd(int64_t tokens, int H, int D, const void* x, int64_t ldx, const void* dy, void* dx, int64_t lddx, void* stream) {
     MI355_REQUIRE(tokens > 0 && H > 0 && D > 0 && D <= 256 && x && dy && dx && ldx >= (int64_t)H * D && lddx >= (int64_t)H * D, "l2norm_bwd: bad arguments (head_dim <= 256)");
+    if (const int g = row_lanes(tokens * H, D, ldx | lddx, {x, dy, dx})) {
+#define RUN(G) l2norm_bwd_rows_kernel<G><<<rows_grid(tokens * H, G), 256, 0, ST(stream)>>>((unsigned)(tokens * H), H, (const bf16_t*)x, ldx, (const bf16_t*)dy, (bf16_t*)dx, lddx)
+        ROW_LANES(g, RUN)
+#undef RUN
+        MI355_LAUNCH_CHECK("l2norm_bwd");
+        return 0;
+    }
     const int grid = wave_grid(tokens * H, 8192);
     if (D <= 64) l2norm_bwd_kernel<1><<<grid, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)x, ldx, (const bf16_t*)dy, (bf16_t*)dx, lddx);
     else if (D <= 128) l2norm_bwd_kernel<2><<<grid, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)x, ldx, (const bf16_t*)dy, (bf16_t*)dx, lddx);
@@ -1318,6 +1472,13 @@ extern "C" int mi355_gated_delta_rule_bwd(int B, int S, int Hqk, int Hv, int Dk,
 extern "C" int mi355_gated_rmsnorm_fwd(int64_t tokens, int H, int D, const void* o, const float* w, const void* gate, int64_t ldg, void* out,
                                        float* rstd, float eps, void* stream) {
     MI355_REQUIRE(tokens > 0 && H > 0 && D > 0 && D <= 256 && o && w && gate && out && rstd && ldg >= (int64_t)H * D, "gated_rmsnorm_fwd: bad arguments (head_dim <= 256)");
+    if (const int g = row_lanes(tokens * H, D, ldg, {o, gate, out})) {
+#define RUN(G) gated_rmsnorm_fwd_rows_kernel<G><<<rows_grid(tokens * H, G), 256, 0, ST(stream)>>>((unsigned)(tokens * H), H, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, (bf16_t*)out, rstd, eps)
+        ROW_LANES(g, RUN)
+#undef RUN
+        MI355_LAUNCH_CHECK("gated_rmsnorm_fwd");
+        return 0;
+    }
     const int grid = wave_grid(tokens * H, 8192);
     if (D <= 64) gated_rmsnorm_fwd_kernel<1><<<grid, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, (bf16_t*)out, rstd, eps);
     else if (D <= 128) gated_rmsnorm_fwd_kernel<2><<<grid, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, (bf16_t*)out, rstd, eps);
@@ -1329,6 +1490,13 @@ extern "C" int mi355_gated_rmsnorm_bwd(int64_t tokens, int H, int D, const void*
                                        const void* dout, void* d_o, void* dgate, int64_t lddg, float* dw_partial, int parts, void* stream) {
     MI355_REQUIRE(tokens > 0 && H > 0 && D > 0 && D <= 256 && o && w && gate && rstd && dout && d_o && dgate && dw_partial, "gated_rmsnorm_bwd: bad arguments (head_dim <= 256)");
     MI355_REQUIRE(ldg >= (int64_t)H * D && lddg >= (int64_t)H * D && parts >= 1 && parts <= 8192, "gated_rmsnorm_bwd: ld / parts out of range");
+    if (const int g = row_lanes(tokens * H, D, ldg | lddg, {o, gate, dout, d_o, dgate})) {
+#define RUN(G) gated_rmsnorm_bwd_rows_kernel<G><<<parts, 256, 0, ST(stream)>>>((unsigned)(tokens * H), H, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, rstd, (const bf16_t*)dout, (bf16_t*)d_o, (bf16_t*)dgate, lddg, dw_partial)
+        ROW_LANES(g, RUN)
+#undef RUN
+        MI355_LAUNCH_CHECK("gated_rmsnorm_bwd");
+        return 0;
+    }
     if (D <= 64) gated_rmsnorm_bwd_kernel<1><<<parts, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, rstd, (const bf16_t*)dout, (bf16_t*)d_o, (bf16_t*)dgate, lddg, dw_partial);
     else if (D <= 128) gated_rmsnorm_bwd_kernel<2><<<parts, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, rstd, (const bf16_t*)dout, (bf16_t*)d_o, (bf16_t*)dgate, lddg, dw_partial);
     else gated_rmsnorm_bwd_kernel<4><<<parts, 256, 0, ST(stream)>>>(tokens, H, D, (const bf16_t*)o, w, (const bf16_t*)gate, ldg, rstd, (const bf16_t*)dout, (bf16_t*)d_o, (bf16_t*)dgate, lddg, dw_partial);

@@ -247,6 +247,48 @@ def test_l2norm():
     assert rel_l2(dx[:, : H * D], xf.grad.reshape(tokens, H * D)) < 6e-3
 
 
+@pytest.mark.parametrize("tokens,H,D", [(1, 1, 64), (3, 5, 64), (1, 3, 128), (701, 7, 128), (33, 1, 256), (2, 3, 256)])
+@pytest.mark.parametrize("shift", [0, 1])
+def test_head_rows_by_pieces_and_by_waves(tokens, H, D, shift):
+    """l2 norm and gated RMSNorm, forward and backward, where 8, 16 or 32 lanes take a row (columns on 16 bytes) and where a wavefront does (shift 1): each against fp64."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    torch.manual_seed(D + tokens)
+    W = H * D
+    view = lambda a: torch.cat([torch.zeros(tokens, 8 + shift, dtype=BF16), a, torch.zeros(tokens, 16 - shift, dtype=BF16)], 1).cuda()[:, 8 + shift : 8 + shift + W]
+    hold = lambda: torch.full((tokens, W + 16), 3.0, dtype=BF16, device="cuda")
+    x, gate, dy, w = torch.randn(tokens, W).to(BF16), torch.randn(tokens, W).to(BF16), torch.randn(tokens, W).to(BF16), 1.0 + 0.1 * torch.randn(D)
+    x[0, :D] = 0  # the clamped branch
+    heads = lambda a: a.double().view(tokens, H, D)
+    close = lambda a, b: bool(((a.cpu().double().view(tokens, H, D) - b).abs() <= 2.0**-8 * b.abs() + 2e-6).all())  # one bf16 rounding (2^-9) and fp32 sums of 256 terms
+
+    y = Q.l2norm_fwd(view(x), H, D)
+    inv = (1 / heads(x).norm(dim=-1, keepdim=True).float().to(BF16).clamp_min(1e-6).float()).to(BF16).double()
+    assert bool(((y.cpu().double().view(tokens, H, D) - heads(x) * inv).abs() <= 2.0**-6 * (heads(x) * inv).abs()).all())  # the norm and its inverse may round the other way
+    out = hold()
+    Q.l2norm_bwd(view(x), dy.cuda(), out[:, shift : shift + W], H, D)
+    n = heads(x).norm(dim=-1, keepdim=True)
+    k3 = torch.where(n < 1e-6, 0.0, (heads(x) * heads(dy)).sum(-1, keepdim=True) / n.clamp_min(1e-6) ** 3)
+    want = heads(dy) / n.clamp_min(1e-6) - heads(x) * k3
+    assert bool(((out[:, shift : shift + W].cpu().double().view(tokens, H, D) - want).abs() <= 2.0**-8 * want.abs() + 2e-6 * (heads(dy).abs() / n.clamp_min(1e-6) + 1)).all())
+    assert bool((out[:, shift + W :] == 3.0).all()) and bool((out[:, :shift] == 3.0).all())
+
+    got, rstd = Q.gated_rmsnorm_fwd(x.cuda(), w.cuda(), view(gate), H, D)
+    r = torch.rsqrt(heads(x).pow(2).mean(-1, keepdim=True) + 1e-6)
+    g, d, wd = heads(gate), heads(dy), w.double()
+    sg = torch.sigmoid(g)
+    assert close(got, g * sg * heads(x) * r * wd)
+    dgate = hold()
+    d_o, dw = Q.gated_rmsnorm_bwd(x.cuda(), w.cuda(), view(gate), rstd, dy.cuda(), dgate[:, shift : shift + W], H, D)
+    xh = heads(x) * r
+    assert close(dgate[:, shift : shift + W], d * xh * wd * sg * (1 + g * (1 - sg)))
+    dn = d * g * sg
+    want = r * (dn * wd - xh * (dn * wd * xh).mean(-1, keepdim=True))
+    assert bool(((d_o.cpu().double().view(tokens, H, D) - want).abs() <= 2.0**-8 * want.abs() + 4e-6 * r * (1 + xh.abs())).all())
+    assert rel_l2(dw, (dn * xh).sum((0, 1))) < 1e-5
+    assert bool((dgate[:, shift + W :] == 3.0).all()) and bool((dgate[:, :shift] == 3.0).all())
+
+
 def test_gated_rmsnorm():
     from llm_quest_amd import kernels_q35 as Q
     from oracle import ops as OO
