@@ -812,6 +812,23 @@ def test_cross_entropy_large_vocab(K):
     assert rel_l2(loss_rows, ref) < 1e-5
 
 
+@pytest.mark.parametrize("V", [7, 2049, 8199, 32767, 32775, 155_663, 188_424, 248_320])
+def test_cross_entropy_two_read_kernel_at_trip_edges(K, V):
+    """Trips of four pieces a thread that end inside, at and behind the row, in both block sizes, with a run of masked (-inf) columns over whole trips: against fp64."""
+    g = torch.Generator().manual_seed(V)
+    lg = (torch.randn(3, V, generator=g) * 3).to(BF16)
+    lg[1, : V * 2 // 3] = float("-inf")
+    tg = torch.tensor([V // 2, V - 1, V - 2])
+    x = torch.zeros(3, (V + 7) // 8 * 8, dtype=BF16, device="cuda")[:, :V]
+    x.copy_(lg)
+    loss_rows, dl = K.cross_entropy(x, dev(tg), want_grad=True, grad_scale=dev(torch.ones(1)), inplace=True)
+    want = torch.nn.functional.cross_entropy(lg.double(), tg, reduction="none")
+    assert rel_l2(loss_rows, want) < 1e-5
+    grad = lg.double().softmax(-1) - torch.nn.functional.one_hot(tg, V)
+    # one bf16 rounding; exp(l - lse) to the fp32 rounding of an argument of at most 40
+    assert bool(((dl.cpu().double() - grad).abs() <= (2.0**-8 + 4e-5) * grad.abs() + 1e-6).all())
+
+
 @pytest.mark.parametrize("V", [1000, 8200, 32768, 32776, 151_936, 155_648, 155_656, 5003])
 @pytest.mark.parametrize("inplace", [True, False])
 def test_cross_entropy_forms_agree_with_fp32(K, V, inplace):
