@@ -125,6 +125,33 @@ def test_headnorm_rope_forward_backward(H, D, R, stride_mul):
             assert not dsrc.cpu()[:, h * hs + D : (h + 1) * hs].any()
 
 
+@pytest.mark.parametrize("tokens,H,D,R", [(1, 1, 64, 64), (37, 3, 64, 16), (5, 1, 128, 32), (700, 5, 128, 0), (3, 3, 256, 16), (61, 2, 256, 64)])
+def test_headnorm_rope_by_pieces_matches_waves(tokens, H, D, R):
+    """Rows by 16-byte pieces against a wavefront a row (the same columns one element further on): sums in another order, so an element may round the other way."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    torch.manual_seed(D + R)
+    hs = D + 24
+    src, g, w = torch.randn(tokens, H * hs).to(BF16), torch.randn(tokens, H * D).to(BF16).cuda(), (1 + 0.2 * torch.randn(D)).to(BF16).cuda()
+    tab = [torch.randn(tokens + 3, R).cuda() for _ in range(2)] if R else [None, None]
+    pos = torch.randint(0, tokens + 3, (tokens,), dtype=torch.int32).cuda() if R else None
+    got = []
+    for shift in (0, 1):
+        buf = torch.cat([torch.zeros(tokens, shift, dtype=BF16), src, torch.zeros(tokens, 8 - shift, dtype=BF16)], 1).cuda()
+        dbuf = torch.full_like(buf, 7.0)
+        view = buf[:, shift : shift + H * hs]
+        out, rstd = Q.headnorm_rope_fwd(view, H, D, hs, w, *tab, pos)
+        dw = Q.headnorm_rope_bwd(view, H, D, hs, w, *tab, pos, rstd, g, dbuf[:, shift : shift + H * hs], hs)
+        d = dbuf[:, shift : shift + H * hs].reshape(tokens, H, hs)
+        assert bool((d[:, :, D:] == 7.0).all())
+        got.append((out, rstd, d[:, :, :D], dw))
+    (o0, r0, d0, w0), (o1, r1, d1, w1) = got
+    assert rel_l2(r0, r1) < 1e-6 and rel_l2(w0, w1) < 1e-5
+    # a normed value off by an ulp (2^-8) turns into both columns of its pair, |cos| and |sin| up to 5
+    assert rel_l2(o0, o1) < 2e-3 and float((o0.float() - o1.float()).abs().max()) <= 2.0**-8 * 12 * float(o1.float().abs().max())
+    assert rel_l2(d0, d1) < 1e-3 and float((d0.float() - d1.float()).abs().max()) <= 2.0**-7 * float(d1.float().abs().max())
+
+
 def test_sigmoid_gate():
     from llm_quest_amd import kernels_q35 as Q
 
