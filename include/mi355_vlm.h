@@ -152,6 +152,9 @@ int mi355_swiglu_bwd(int64_t tokens, int F, const void* gu, const void* da, void
  * ViTMergeAdapter, qwen3_5_vision_model.py:408); kind 1: tanh approximation (Qwen3_5VisionFFN, qwen3_5_vision_model.py:122). */
 int mi355_gelu_fwd(int64_t n, const void* x, void* y, int kind, void* stream);
 int mi355_gelu_bwd(int64_t n, const void* x, const void* dy, void* dx, int kind, void* stream);
+/* mi355_gelu_bwd of [M, N] rows, N % 8 == 0, operands 16-byte aligned, that also leaves partial fp32 [parts][N]: column sums of the bf16 result (the bias gradient of
+ * vit_transformer_block.py:59-67's first Linear), to be added up by mi355_reduce_rows_into. */
+int mi355_gelu_bwd_colsum(int64_t M, int64_t N, const void* x, const void* dy, void* dx, float* partial, int parts, int kind, void* stream);
 
 /* Flash-style attention, token-major operands, never materialising SxS (replaces qwen3_attention.py:121-146,
  * vit_attention.py:74-86).  q [B*S, Hq*D] ld=ldq, k/v [B*S, Hkv*D] ld=ldk/ldv, o [B*S, Hq*D] ld=ldo, bf16;

@@ -65,6 +65,7 @@ SIGNATURES = {
     "mi355_scale_bf16": [_L, _P, _P, _P, _P],
     "mi355_gelu_fwd": [_L, _P, _P, _I, _P],
     "mi355_gelu_bwd": [_L, _P, _P, _P, _I, _P],
+    "mi355_gelu_bwd_colsum": [_L, _L, _P, _P, _P, _P, _I, _I, _P],
     "mi355_patchify3d": [_I, _I, _I, _I, _I, _I, _I, _P, _P, _I, _P],
     "mi355_merge_patches": [_L, _I, _I, _I, _L, _P, _P, _I, _P],
     "mi355_scatter_rows": [_L, _L, _P, _P, _P, _P, _P, _P, _I, _P],

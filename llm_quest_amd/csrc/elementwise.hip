@@ -101,6 +101,47 @@ __global__ __launch_bounds__(256) void gelu_bwd_kernel(int64_t n, const bf16_t* 
     }
 }
 
+// The same with the result's column sums (the bias gradient of the layer below), which otherwise read dx again.  A block takes 512 columns of every parts-th group of four rows,
+// a wavefront one row of a group, two groups requested at a time.  Bound: bytes (2 reads, 1 write).  25 216 x 3 072: 91 us without the sums, 94 with them (+ 6 us to add
+// up 256 parts), and the pass that read dx again is gone: 41 us a layer less in the training step of 128 images.
+template <int KIND>
+__global__ __launch_bounds__(256) void gelu_bwd_colsum_kernel(int64_t M, int64_t N, const bf16_t* __restrict__ x, const bf16_t* __restrict__ dy, bf16_t* __restrict__ dx,
+                                                              float* __restrict__ partial) {
+    __shared__ float red[4][512];
+    const int chunk = threadIdx.x & 63, rl = threadIdx.x >> 6;
+    const int64_t col = (int64_t)blockIdx.x * 512 + chunk * 8, step = 4 * (int64_t)gridDim.y;
+    float s[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto row = [&](int64_t r, const u32x4 xr, const u32x4 gr) {
+        float v[8], g[8];
+        unpack8(xr, v);
+        unpack8(gr, g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) g[e] *= gelu_grad<KIND>(v[e]);
+        const u32x4 o = pack8(g);
+        *reinterpret_cast<u32x4*>(dx + r * N + col) = o;
+        unpack8(o, g);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += g[e];
+    };
+    if (col < N) {
+        int64_t r = (int64_t)blockIdx.y * 4 + rl;
+        for (; r + step < M; r += 2 * step) {
+            const u32x4 x0 = *reinterpret_cast<const u32x4*>(x + r * N + col), g0 = *reinterpret_cast<const u32x4*>(dy + r * N + col);
+            const u32x4 x1 = *reinterpret_cast<const u32x4*>(x + (r + step) * N + col), g1 = *reinterpret_cast<const u32x4*>(dy + (r + step) * N + col);
+            row(r, x0, g0);
+            row(r + step, x1, g1);
+        }
+        if (r < M) row(r, *reinterpret_cast<const u32x4*>(x + r * N + col), *reinterpret_cast<const u32x4*>(dy + r * N + col));
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) red[rl][chunk * 8 + e] = s[e];
+    __syncthreads();
+    for (int c = threadIdx.x; c < 512; c += 256) {
+        const int64_t gc = (int64_t)blockIdx.x * 512 + c;
+        if (gc < N) partial[(int64_t)blockIdx.y * N + gc] = (red[0][c] + red[1][c]) + (red[2][c] + red[3][c]);
+    }
+}
+
 // 3-D patch gather for Conv3d(k = s = (TP, P, P)) (qwen3_5_vision_model.py:79-107): tokens ordered (t', ph, pw), K ordered (c, dt, i, j)
 template <int OUT_DT>
 __global__ __launch_bounds__(256) void patchify3d_kernel(int B, int C, int T, int H, int W, int P, int TP, const float* __restrict__ img, void* __restrict__ rows) {
@@ -740,6 +781,16 @@ extern "C" int mi355_gelu_bwd(int64_t n, const void* x, const void* dy, void* dx
     if (kind == 0) hipLaunchKernelGGL(gelu_bwd_kernel<0>, dim3(grid_for(n >> 3, 256)), dim3(256), 0, STREAM, n, (const bf16_t*)x, (const bf16_t*)dy, (bf16_t*)dx);
     else hipLaunchKernelGGL(gelu_bwd_kernel<1>, dim3(grid_for(n >> 3, 256)), dim3(256), 0, STREAM, n, (const bf16_t*)x, (const bf16_t*)dy, (bf16_t*)dx);
     MI355_LAUNCH_CHECK("mi355_gelu_bwd");
+    return 0;
+}
+
+extern "C" int mi355_gelu_bwd_colsum(int64_t M, int64_t N, const void* x, const void* dy, void* dx, float* partial, int parts, int kind, void* stream) {
+    MI355_REQUIRE(M > 0 && N > 0 && (N & 7) == 0 && x && dy && dx && partial && (kind == 0 || kind == 1), "mi355_gelu_bwd_colsum: N must be a positive multiple of 8, kind 0 or 1");
+    MI355_REQUIRE((((uintptr_t)x | (uintptr_t)dy | (uintptr_t)dx) & 15) == 0 && parts >= 1 && parts <= 65535, "mi355_gelu_bwd_colsum: operands must be 16-byte aligned, parts in 1 .. 65535");
+    const dim3 grid((unsigned)((N + 511) / 512), (unsigned)parts);
+    if (kind == 0) hipLaunchKernelGGL(gelu_bwd_colsum_kernel<0>, grid, dim3(256), 0, STREAM, M, N, (const bf16_t*)x, (const bf16_t*)dy, (bf16_t*)dx, partial);
+    else hipLaunchKernelGGL(gelu_bwd_colsum_kernel<1>, grid, dim3(256), 0, STREAM, M, N, (const bf16_t*)x, (const bf16_t*)dy, (bf16_t*)dx, partial);
+    MI355_LAUNCH_CHECK("mi355_gelu_bwd_colsum");
     return 0;
 }
 

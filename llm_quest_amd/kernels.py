@@ -839,6 +839,20 @@ def gelu_bwd(x, dy, tanh=False):
     return dx
 
 
+def gelu_bwd_colsum(x, dy, dest, tanh=False):
+    """``gelu_bwd`` of [rows, width], width % 8 == 0, with the result's column sums into ``dest`` (see ``reduce_rows_into``)."""
+    L.require_gpu(x, dy)
+    if x.dtype != BF16 or dy.dtype != BF16 or x.dim() != 2 or not x.is_contiguous() or not dy.is_contiguous() or dy.shape != x.shape or x.shape[1] % 8:
+        raise ValueError("gelu_bwd_colsum: contiguous bf16 [rows, width] with width % 8 == 0")
+    rows, width = x.shape
+    parts = max(1, min(256, rows // 32))
+    dx = torch.empty_like(x)
+    partial = torch.empty((parts, width), dtype=F32, device=x.device)
+    L.call("mi355_gelu_bwd_colsum", rows, width, L.ptr(x), L.ptr(dy), L.ptr(dx), L.ptr(partial), parts, 1 if tanh else 0)
+    reduce_rows_into(partial, parts, width, [dest])
+    return dx
+
+
 def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=None, dshift_out=None, accumulate=False, mode=0, dests=None):
     """Returns dx fp32 (+ dres).  dscale/dshift go to the given fp32 destinations (optionally accumulated) or new tensors.  ``dests`` (two, see ``reduce_rows_into``): straight into
     them, and only dx is returned."""

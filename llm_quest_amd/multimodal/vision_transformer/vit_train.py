@@ -180,13 +180,19 @@ def ffn_backward(ffn, saved, dy, wg=None, dyb=None):
         dyb = dy if dy.dtype == BF16 else K.cast(dy, BF16)
     own = wg is None
     wg = [] if own else wg
-    dy1 = K.gemm_dgrad_gelu_bwd(dyb, bf16_cached(ffn, "w2", [ffn.layers[2].weight]), y1)  # GELU backward in the dgrad epilogue
+    w2, b1 = bf16_cached(ffn, "w2", [ffn.layers[2].weight]), ffn.layers[0].bias
+    bias_in_pass = b1 is not None and b1.requires_grad and not K._FUSE_GELU and y1.shape[1] % 8 == 0
+    if bias_in_pass:
+        dy1 = K.gelu_bwd_colsum(y1, K.dgrad(dyb, w2), _dest(b1))
+    else:
+        dy1 = K.gemm_dgrad_gelu_bwd(dyb, w2, y1)
     _wgrad(ffn.layers[2].weight, dyb, f, wg)
     if not bias_done:
         _bgrad(ffn.layers[2].bias, dyb)
     dh2 = K.dgrad(dy1, bf16_cached(ffn, "w1", [ffn.layers[0].weight]))
     _wgrad(ffn.layers[0].weight, dy1, h2, wg)
-    _bgrad(ffn.layers[0].bias, dy1)
+    if not bias_in_pass:
+        _bgrad(b1, dy1)
     if own:
         ops._flush_wgrads(wg)
     return dh2

@@ -785,6 +785,21 @@ def test_attention_forward_lazy_rescale_branch_is_exercised(K, kernel):
         assert rel_l2(got, ref) < 8e-3, name
 
 
+@pytest.mark.parametrize("rows,width", [(1, 8), (5, 520), (63, 1024), (985, 3072), (2057, 504)])
+@pytest.mark.parametrize("tanh", [False, True])
+def test_gelu_backward_with_column_sums(K, rows, width, tanh):
+    """The same bits as the pass without the sums, and the sums of those rounded values, written and added to; rows around one, two and three trips of a block."""
+    g = torch.Generator().manual_seed(rows)
+    x, dy = dev(torch.randn(rows, width, generator=g).to(BF16)), dev(torch.randn(rows, width, generator=g).to(BF16))
+    want = K.gelu_bwd(x, dy, tanh=tanh)
+    total = want.double().sum(0)
+    scale = 1e-6 * want.double().abs().sum(0) + 1e-7  # fp32 sums of at most 2 057 terms in short chains
+    out = torch.full((width,), 7.0, device="cuda")
+    assert torch.equal(K.gelu_bwd_colsum(x, dy, (out, False), tanh=tanh), want) and bool(((out.double() - total).abs() <= scale).all())
+    K.gelu_bwd_colsum(x, dy, (out, True), tanh=tanh)
+    assert bool(((out.double() - 2 * total).abs() <= 3 * scale).all())
+
+
 # ----------------------------------------------------------------------------------------------- CE / embedding / gathers
 def test_cross_entropy_golden(K, golden):
     t = golden("per_op")
