@@ -2362,7 +2362,10 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         else if (form != MI355_GEMM_TN && tiles256 < 128) cfg = 1;  // measured: 92 tiles -> 128x128 wins (+2.8 % on the config-5 step), 180 tiles -> 256x256 wins
         // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Round 4, batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)
-        else if (form == MI355_GEMM_TN) cfg = (M * N > 5 * 1024 * 1024) ? 5 : 1;
+        // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,
+        // which the four waves have no partner to hide (151 936 x 1 024, tile 5 / 3 / 1: 61 tokens 117 / 96 / 100, 333 196 / 174 / 200, 602 259 / 248 / 275, 1 024 367 / 374 / 398;
+        // 50 256 x 768 (591 tiles): 61 tokens 36 / 28 / 25, 602 74 / 74 / 69, 1 500 136 / 147 / 144)
+        else if (form == MI355_GEMM_TN) cfg = M * N <= 5 * 1024 * 1024 || tiles256 < 160 ? 1 : K >= 1024 ? 5 : tiles256 >= 1024 ? 3 : 1;
         else if (form == MI355_GEMM_NT) cfg = 2;
         else cfg = 3;
     }
@@ -2442,7 +2445,7 @@ extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_pro
     MI355_REQUIRE(tile_hint == 0 || tile_hint == 1 || tile_hint == 3 || tile_hint == 4 || tile_hint == 5, "mi355_gemm_bf16_grouped: tile_hint must be 0 (auto), 1 (128x128), 3, 4 or 5 (256x256)");
     GroupTable tbl;
     tbl.count = count;
-    int64_t tiles256 = 0;
+    int64_t tiles256 = 0, longest = 0;
     bool small = false;
     for (int i = 0; i < count; ++i) {
         const mi355_gemm_problem& q = problems[i];
@@ -2454,11 +2457,37 @@ extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_pro
         p.ad_lse = nullptr; p.ad_delta = p.ad_nl2 = p.ad_ndl = nullptr; p.ad_S = p.ad_Hq = 0;
         p.split3 = 0;
         tiles256 += ((q.M + 255) / 256) * ((q.N + 255) / 256);
+        longest = q.K > longest ? q.K : longest;
         small |= q.M < 256 || q.N < 256;
     }
     for (int i = count; i < MAX_GROUP; ++i) tbl.g[i] = tbl.g[0];
     // 256x256 tiles (one workgroup per CU) once they cover most of the chip; otherwise 128x128 (two per CU, 4x the tiles)
-    const int cfg = tile_hint ? tile_hint : ((small || tiles256 < 160) ? 1 : (form == MI355_GEMM_TN ? 5 : 3));
+    int cfg = tile_hint ? tile_hint : ((small || tiles256 < 160) ? 1 : (form == MI355_GEMM_TN ? 5 : 3));
+    // Weight gradients whose 256x256 tiles are one round and up to half of a second.  Few tokens: 128x128 tiles, two per CU.  Many: the problems that fill the round best go on it
+    // and the others follow on 128x128 tiles, which all have a place at once.  us, one launch on 256x256 / one on 128x128 / two launches: 328 tiles (8 224, 7 168, 3 584 and 2 048 by
+    // 1 024) 333 tokens 45 / 39 / 39, 1 024 77 / 67 / 70, 2 048 121 / 109 / 106, 5 664 291 / 282 / 254; 288 tiles 2 048 tokens 114 / 92 / 91, 5 664 271 / 233 / 211; 320 tiles
+    // 333 tokens 42 / 33 / 39, 5 664 274 / 241 / 218; 384 tiles 1 500 tokens 93 / 91.  Not below one round (240 tiles, 2 048 tokens 64 / 74) nor from 672 tiles on (197 / 239).
+    if (tile_hint == 0 && cfg == 5 && tiles256 > 256 && tiles256 <= 384 && longest < 2048) cfg = 1;
+    if (tile_hint == 0 && cfg == 5 && tiles256 > 256 && tiles256 <= 384) {
+        unsigned best = 0;
+        int64_t best_tiles = 0;
+        for (unsigned pick = 1; pick + 1 < (1u << count); ++pick) {
+            int64_t t = 0;
+            for (int i = 0; i < count; ++i)
+                if (pick >> i & 1) t += ((problems[i].M + 255) / 256) * ((problems[i].N + 255) / 256);
+            if (t <= 256 && t > best_tiles) best_tiles = t, best = pick;
+        }
+        if (best && tiles256 - best_tiles <= 128) {
+            mi355_gemm_problem part[MAX_GROUP];
+            for (int rest = 0; rest < 2; ++rest) {
+                int n = 0;
+                for (int i = 0; i < count; ++i)
+                    if ((int)(best >> i & 1) != rest) part[n++] = problems[i];
+                if (int rc = mi355_gemm_bf16_grouped(form, n, part, out_dtype, rest ? 1 : 5, stream)) return rc;
+            }
+            return 0;
+        }
+    }
     hipStream_t s = (hipStream_t)stream;
     if (cfg == 5) return mi355_gemm_grouped_part5(form, &tbl, out_dtype, s);
     if (cfg == 4) return mi355_gemm_grouped_part4(form, &tbl, out_dtype, s);

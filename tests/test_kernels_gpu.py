@@ -785,6 +785,22 @@ def test_attention_forward_lazy_rescale_branch_is_exercised(K, kernel):
         assert rel_l2(got, ref) < 8e-3, name
 
 
+@pytest.mark.parametrize("K_,dims", [(72, [(8200, 1024), (7168, 1016), (1024, 3584)]), (333, [(5120, 2048), (2056, 1024), (4096, 1000), (264, 264)]), (2056, [(5120, 2048), (2056, 1024), (4096, 1000), (264, 264)]), (65, [(33_000, 512)])])
+def test_weight_gradients_of_more_than_one_round_of_tiles(K, K_, dims):
+    """Grouped weight gradients of 258, 264 and 300 tiles of 256 x 256, remainders in both directions: few tokens on small tiles, more (2 056) in two launches:
+    each against fp64, and one alone as a plain product."""
+    g = torch.Generator().manual_seed(K_)
+    probs, refs = [], []
+    for M, N in dims:
+        a, b = dev(torch.randn(K_, M, generator=g).to(BF16)), dev(torch.randn(K_, N, generator=g).to(BF16))
+        probs.append((a, b, torch.full((M, N), float("nan"), device="cuda"), None))
+        refs.append(a.double().T @ b.double())
+    K.gemm_grouped(K.L.GEMM_TN, probs)
+    for (a, b, c, _), ref in zip(probs, refs):
+        assert float((c.double() - ref).abs().max()) < 2.0**-22 * K_ * 16  # fp32 sums of K_ products of magnitude below 16
+        assert rel_l2(K.gemm(K.L.GEMM_TN, a, b, out_dtype=F32), ref) < 1e-5
+
+
 @pytest.mark.parametrize("rows,width", [(1, 8), (5, 520), (63, 1024), (985, 3072), (2057, 504)])
 @pytest.mark.parametrize("tanh", [False, True])
 def test_gelu_backward_with_column_sums(K, rows, width, tanh):
