@@ -150,3 +150,12 @@ def test_integration_md_stubs_match_the_binding_table():
                 cur += ch
         nargs += 1 if cur.strip() else 0
         assert nargs == len(_lib.SIGNATURES[name]), f"INTEGRATION.md calls {name} with {nargs} arguments, the ABI takes {len(_lib.SIGNATURES[name])}"
+
+
+@pytest.mark.parametrize("dest", [torch.zeros(16)[::2], torch.zeros(8, dtype=torch.float64), torch.zeros(7), torch.zeros(8, device="meta")])
+def test_gradient_destinations_are_checked(dest):
+    """A gradient that sums are written into by address: strided, of another type or width, or elsewhere is refused on the host."""
+    from llm_quest_amd import kernels
+
+    with pytest.raises(ValueError, match="contiguous fp32"):
+        kernels.reduce_rows_into(torch.zeros(2, 16), 2, 8, [None, (dest, False)])
