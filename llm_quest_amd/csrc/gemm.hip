@@ -2074,6 +2074,18 @@ int choose_ksplit(int64_t tiles, int64_t slots, int64_t K, int64_t M, int64_t N,
     int64_t ks = (slots + slots / 4 + tiles - 1) / tiles;
     if (ks > kt / 8) ks = kt / 8;
     if (ks > 16) ks = 16;
+    // Long loops (16 384 of K and more) are worth whole shares: the busiest CU's K-tiles (0.67 us each on a 128x128 tile among two or more; alone on its CU a workgroup has nothing
+    // to hide its waits, 1.4 times that) and the partial sums' way through memory at 4 TB/s.  us, from a
+    // quarter more workgroups than places -> here: NN by 1 024 columns, K = 248 320, 61 rows 317 -> 182, 333 346 -> 294, 1 300 (256x256) 1 174 -> 837; K = 20 000, 333 rows 40 -> 39, 1 300 112 -> 88;
+    // weight gradients 768 x 768 over 16 384 tokens 51 -> 41, 65 536 157 -> 120, 2 304 x 768 over 16 384 90 -> 88; 256 x 256 over 16 384 22 -> 24.
+    if (kt >= 256) {
+        double least = 0;
+        for (int64_t c = 1; c <= 32 && c * M * N * 4 <= ws_bytes; ++c) {
+            const int64_t share = (tiles * c + 255) / 256;
+            const double t = (share == 1 && slots > 256 ? 1.4 : (double)share) * (double)((kt + c - 1) / c) * (slots > 256 ? 0.67 : 2.0) + (c > 1 ? (double)(c * M * N) * 8 / 4e6 : 0);
+            if (c == 1 || t < least) least = t, ks = c;
+        }
+    }
     while (ks > 1 && ks * M * N * 4 > ws_bytes) --ks;
     return ks < 2 ? 1 : (int)ks;
 }
@@ -2358,7 +2370,12 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         // 256x256 tiles need at least half of the 256 CUs' worth of tiles; below that (small token counts: config 5 at B = 8 has 92 tiles for
         // its N = 1024 outputs) four times as many 128x128 tiles, two workgroups per CU, fill the chip instead
         const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
+        // input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
+        // 128x128 / 256x256: K = 248 320, 333 rows 294 / 304, 602 585 / 446, 2 048 1 298 / 1 092; K = 20 000, 708 rows 54 / 57, 1 300 88 / 82; by 768, K = 50 256, 602 rows 83 / 81
+        const bool long_split = form == MI355_GEMM_NN && workspace && !bias && epilogue == MI355_EPI_NONE && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3)) &&
+                                workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
         if (M < 256 || N < 256) cfg = 1;
+        else if (long_split && tiles256 < 128) cfg = 3;
         else if (form != MI355_GEMM_TN && tiles256 < 128) cfg = 1;  // measured: 92 tiles -> 128x128 wins (+2.8 % on the config-5 step), 180 tiles -> 256x256 wins
         // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Round 4, batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)

@@ -785,6 +785,21 @@ def test_attention_forward_lazy_rescale_branch_is_exercised(K, kernel):
         assert rel_l2(got, ref) < 8e-3, name
 
 
+@pytest.mark.parametrize("form,M,N,K_", [("NN", 61, 264, 16_384), ("NN", 333, 1000, 50_264), ("NN", 520, 264, 32_776), ("NN", 1030, 520, 16_392), ("TN", 264, 272, 16_390), ("TN", 768, 768, 25_216), ("NT", 130, 264, 20_008)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_long_products_split_over_k(K, form, M, N, K_, residual):
+    """K of 16 384 and more goes in shares of whole K-tiles (the last one shorter) on either tile, with the sum added to a residual or not: against fp64."""
+    g = torch.Generator().manual_seed(M)
+    a = dev(torch.randn(*((K_, M) if form == "TN" else (M, K_)), generator=g).to(BF16))
+    b = dev(torch.randn(*((N, K_) if form == "NT" else (K_, N)), generator=g).to(BF16))
+    r = dev(torch.randn(M, N, generator=g)) if residual else None
+    want = (a.double().T if form == "TN" else a.double()) @ (b.double().T if form == "NT" else b.double()) + (r.double() if residual else 0)
+    got = K.gemm(getattr(K.L, "GEMM_" + form), a, b, out_dtype=F32, residual=r)
+    assert rel_l2(got, want) < 2.0**-24 * K_**0.5  # fp32 sums: one rounding per addition, errors that add up as a walk
+    alone = K.gemm(getattr(K.L, "GEMM_" + form), a, b, out_dtype=F32, residual=r, allow_split_k=False)
+    assert rel_l2(alone, want) < 2.0**-24 * K_**0.5
+
+
 @pytest.mark.parametrize("K_,dims", [(72, [(8200, 1024), (7168, 1016), (1024, 3584)]), (333, [(5120, 2048), (2056, 1024), (4096, 1000), (264, 264)]), (2056, [(5120, 2048), (2056, 1024), (4096, 1000), (264, 264)]), (65, [(33_000, 512)])])
 def test_weight_gradients_of_more_than_one_round_of_tiles(K, K_, dims):
     """Grouped weight gradients of 258, 264 and 300 tiles of 256 x 256, remainders in both directions: few tokens on small tiles, more (2 056) in two launches:
