@@ -273,10 +273,10 @@ def gdr_chunked(v, S, Dk, Dv):
     return Dk == 128 and Dv == 128 and S >= GDR_CHUNKED_MIN and v.stride(0) % 8 == 0 and v.data_ptr() % 16 == 0
 
 
-def gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=True, want_state=False, state=None, chunked=None):
+def gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=True, want_state=False, state=None, chunked=False):
     """Returns (o bf16 [B*S, Hv*Dv], what the backward needs or None, final_state or None).  ``state`` fp32 [B, Hv, Dv, Dk]: carried-in recurrent
-    state, updated IN PLACE (and returned as final_state).  ``chunked``: False keeps to the token-by-token kernels whatever the sizes (operands that are not a layer's:
-    keys of any length, any alpha); default: ``gdr_chunked``."""
+    state, updated IN PLACE (and returned as final_state).  ``chunked``: None lets ``gdr_chunked`` choose, for the operands that a layer makes (unit keys, alpha in 0 .. 1);
+    False keeps to the token-by-token kernels, which take keys of any length and any alpha."""
     L.require_gpu(q, k, v, beta, alpha)
     _check_gdr(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv)
     o = torch.empty((B * S, Hv * Dv), dtype=BF16, device=q.device)

@@ -466,7 +466,7 @@ def q35_mixer_cached(att, arena, h1, st, i):
         qn, kn = Q.l2norm_fwd(y[:, :QK], Hqk, Dk), Q.l2norm_fwd(y[:, QK : 2 * QK], Hqk, Dk)
         beta, alpha = Q.gdn_gates_fwd(proj[:, C + VG : C + VG + Hv], proj[:, C + VG + Hv :], att.log_A, att.dt_bias)
         o, _, fin = Q.gated_delta_rule_fwd(qn, kn, y[:, 2 * QK :], beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=False, want_state=True,
-                                           state=cache.get_recurrent_state(i))
+                                           state=cache.get_recurrent_state(i), chunked=None)
         cache.set_recurrent_state(i, fin)
         mix, _ = Q.gated_rmsnorm_fwd(o, att.post_norm.weight, proj[:, C : C + VG], Hv, Dv, eps=att.post_norm.eps)
         return mix

@@ -162,7 +162,7 @@ def gdn_forward(att, arena, h1, rt, keep=True):
     qn = Q.l2norm_fwd(y[:, :QK], Hqk, Dk)
     kn = Q.l2norm_fwd(y[:, QK : 2 * QK], Hqk, Dk)
     beta, alpha = Q.gdn_gates_fwd(proj[:, C + VG : C + VG + Hv], proj[:, C + VG + Hv :], att.log_A, att.dt_bias)
-    o, ck, _ = Q.gated_delta_rule_fwd(qn, kn, y[:, 2 * QK :], beta, alpha, rt.B, rt.S, Hqk, Hv, Dk, Dv, keep=keep)
+    o, ck, _ = Q.gated_delta_rule_fwd(qn, kn, y[:, 2 * QK :], beta, alpha, rt.B, rt.S, Hqk, Hv, Dk, Dv, keep=keep, chunked=None)
     gated, rstd_p = Q.gated_rmsnorm_fwd(o, att.post_norm.weight, proj[:, C : C + VG], Hv, Dv, eps=att.post_norm.eps)
     return gated, (h1, proj, y, qn, kn, beta, alpha, o, ck, rstd_p)
 
@@ -358,7 +358,7 @@ class GatedDeltaRuleFn(torch.autograd.Function):
         al = alpha.to(F32).permute(0, 2, 1).reshape(b * s, h).contiguous()
         # a carried-in state (reference :103: prev_state) is copied: the kernel advances the state in place, the caller's tensor stays as it was
         state = None if prev_state is None else prev_state.detach().to(F32).contiguous().clone()
-        o, ck, fin = Q.gated_delta_rule_fwd(q2, k2, v2, be, al, b, s, h, h, dk, dv, keep=True, want_state=True, state=state, chunked=False)
+        o, ck, fin = Q.gated_delta_rule_fwd(q2, k2, v2, be, al, b, s, h, h, dk, dv, keep=True, want_state=True, state=state)
         ctx.saved = (q2, k2, v2, be, al, ck)
         ctx.meta = (b, h, s, dk, dv, q.dtype, k.dtype, v.dtype, beta.dtype, alpha.dtype, None if prev_state is None else prev_state.dtype)
         ctx.set_materialize_grads(False)  # an unused last state arrives as None, not as a zero tensor the kernel would have to read

@@ -592,6 +592,36 @@ def test_functional_gated_delta_rule_carries_a_previous_state(golden):
     assert torch.equal(o3.detach(), o2) and torch.equal(st3.detach(), st2) and torch.equal(st1, keep), "the differentiable path computes the same forward"
 
 
+@pytest.mark.parametrize("s", [64, 65, 130])
+def test_functional_gated_delta_rule_takes_any_decay_and_any_key(s):
+    """The public entry with a carried state, heads of 128 | 128 and whole chunks of tokens, on operands that no layer makes: decays below and at zero, keys that are not unit
+    vectors.  With and without gradients it is one recurrence (the same bits), and that of fp64: the state is fp32 (128 products a step, some 2^-24 sqrt(s) each), the output is
+    rounded to bf16 (2^-9)."""
+    from llm_quest_amd.qwen.qwen3_next.qwen3_next_attention import gated_delta_rule
+
+    g = torch.Generator().manual_seed(s)
+    b, h, D = 1, 2, 128
+    q, v = (torch.randn(b, h, s, D, generator=g).to(BF16) for _ in range(2))
+    k = (torch.randn(b, h, s, D, generator=g) * (0.7 / D**0.5)).to(BF16)
+    beta, alpha = torch.sigmoid(torch.randn(b, h, s, generator=g)), 0.5 + 0.5 * torch.rand(b, h, s, generator=g)
+    alpha[..., ::7] *= -1.0
+    alpha[..., 5::31] = 0.0
+    s0 = torch.randn(b, h, D, D, generator=g)
+    st, outs = s0.double(), []
+    for t in range(s):
+        kt, a = k[:, :, t].double(), alpha[:, :, t, None, None].double()
+        st = st * a
+        u = beta[:, :, t, None].double() * (v[:, :, t].double() - (st * kt[:, :, None, :]).sum(-1))
+        st = st + u[..., None] * kt[:, :, None, :]
+        outs.append((st * q[:, :, t].double()[:, :, None, :]).sum(-1) / D**0.5)
+    ref = torch.stack(outs, 2)
+    with torch.no_grad():
+        o, fin = gated_delta_rule(q.cuda(), k.cuda(), v.cuda(), beta.cuda(), alpha.cuda(), prev_state=s0.cuda())
+    o2, fin2 = gated_delta_rule(q.cuda().requires_grad_(True), k.cuda(), v.cuda(), beta.cuda(), alpha.cuda(), prev_state=s0.cuda())
+    assert torch.equal(o, o2.detach()) and torch.equal(fin, fin2.detach())
+    assert rel_l2(o.float(), ref.float()) < 4e-3 and rel_l2(fin, st.float()) < 1e-5
+
+
 def test_text_model_loss_path_and_determinism():
     """forward_hidden + lm_loss == CE of forward()'s logits; two identical steps give bit-identical gradients."""
     from llm_quest_amd.qwen.qwen3_5.qwen3_5_text_model import Qwen3_5TextModel
