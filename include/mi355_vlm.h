@@ -571,6 +571,10 @@ int mi355_gated_headnorm(int64_t tokens, int H, int D, const float* o, const flo
 int mi355_gla_fwd(int n_seq, const int* seq_off, const int* slot, int H, int dk, int dv, const void* q, const void* k, const void* v, const void* z, int dt,
                   int z_dt, int v_dt, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldz, const float* zbias, float inv_tau, float qscale, const float* head_decay,
                   float kscale, float* state, float* o, void* stream);
+/* The same for the sequences with fewer than `below` new tokens alone (0: all of them); the others' rows and states are left as they are. */
+int mi355_gla_fwd_below(int n_seq, const int* seq_off, const int* slot, int H, int dk, int dv, const void* q, const void* k, const void* v, const void* z, int dt,
+                  int z_dt, int v_dt, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldz, const float* zbias, float inv_tau, float qscale, const float* head_decay,
+                  float kscale, float* state, float* o, int below, void* stream);
 /* logits[t, e] = sum_k x[t, k] W[e, k]: fp32 rows (pitch ldx) against a bf16 matrix [E, K] (pitch ldw), fp32 FMA; out fp32 [tokens, E]. */
 int mi355_router_logits(int64_t tokens, int E, int K, const float* x, int64_t ldx, const void* W, int64_t ldw, float* out, void* stream);
 /* Grouped sigmoid router: s = sigmoid(logits), choice = s + correction (may be NULL); a group (E / groups neighbours) scores the sum of its two
@@ -650,13 +654,18 @@ int mi355_qkv_rows_append(int64_t tokens, int H, int G, int d, int dv, const voi
 int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
                             int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
                             const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream);
+/* The same for the sequences with fewer than `below` new tokens alone (0: all of them); ws is filled for every row of the step. */
+int mi355_delta_rule_ragged_below(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
+                            int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
+                            const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, int below, void* stream);
 /* The same rule -- or, with head_decay, linear attention with one decay per head (k times kscale, q times qscale) -- in chunks of 64 tokens on the fp32 matrix pipe:
  * heads of 128 | 128, fp32 rows, state fp32 [slots, H, 128, 128] read and written at slot.  tok: mi355_delta_rule_tokens' result (four floats per token and head).
- * max_new: the most new tokens of one sequence.  workspace: mi355_delta_chunked_workspace_bytes, 16-byte aligned. */
+ * max_new: the most new tokens of one sequence; sequences with fewer than `from` are left as they are (their kernels: the _below entries).  A fixed decay lies at 1e-30
+ * or above (what is below counts as 1e-30).  workspace: mi355_delta_chunked_workspace_bytes, 16-byte aligned. */
 int mi355_delta_rule_tokens(int64_t tokens, int H, int G, int dk, const void* q, const void* k, int qk_dt, int64_t ldq, int64_t ldk, const void* b, const void* a, int ba_dt,
                             int64_t ldb, int64_t lda, const float* A_log, const float* dt_bias, float qscale, float* ws, void* stream);
 int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H);
-int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
+int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, int from, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
                         const float* v, int64_t ldv, const float* tok, const float* head_decay, float qscale, float kscale, float* state, float* o, void* workspace,
                         int64_t workspace_bytes, void* stream);
 /* Gated feed-forward activation on rows [gate (F) | up (F)] -> [F].  kind 0: gelu_tanh(gate) * up.  kind 1: g = min(gate, limit), u = clamp(up, -limit, limit),

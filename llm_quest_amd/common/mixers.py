@@ -67,7 +67,7 @@ class SeqStep:
             n_new.append(len(new))
         cache.reserve(max(p + n for p, n in zip(past, n_new)))
         cap = cache.capacity
-        self.T, self.n_seq, self.max_new = seq_off[-1], len(slots), max(n_new)
+        self.T, self.n_seq, self.max_new, self.min_new = seq_off[-1], len(slots), max(n_new), min(n_new)
         self.max_keys = max(p + n for p, n in zip(past, n_new))
         self.fresh = all(p == 0 for p in past)
         self.host_seq_off, self.host_past, self.host_n_new = seq_off, past, n_new
@@ -376,7 +376,7 @@ class Retention(_Frozen):
         qk = torch.empty((h.shape[0], b), dtype=F32, device=h.device)
         S.rope_heads(proj, 2 * H, dk, dk, 0, qk, dk, 0, 0, self.rot_dims, self.freq, st.pos, layout=1)  # q and k heads side by side: 2 H heads of dim
         o = S.gla(qk[:, :a], qk[:, a:b], proj[:, b:c], None, None, 1.0, 1.0, st.seq_off, st.slots, st.cache.state(self.layer_idx, "S"), H, dk, dv,
-                  head_decay=self.decay32, kscale=dk ** -0.5, max_new=st.max_new)
+                  head_decay=self.decay32, kscale=dk ** -0.5, max_new=st.max_new, min_new=st.min_new)
         mix = S.gated_headnorm(o, self.ones, proj[:, c:], H, dv, self.eps, st.act_dtype)
         return S.linear(mix, self.w_o)
 
@@ -564,7 +564,7 @@ class GatedDeltaRule(_Frozen):
         a, b = G * dk, 2 * G * dk
         gate0 = C + H * dv
         o = S.delta_rule(qkv[:, :a], qkv[:, a:b], qkv[:, b:], proj[:, gate0 : gate0 + H], proj[:, gate0 + H :], self.A_log32, self.dt_bias32, dk ** -0.5, st.seq_off, st.slots,
-                         st.cache.state(self.layer_idx, "S"), H, G, dk, dv, max_new=st.max_new)
+                         st.cache.state(self.layer_idx, "S"), H, G, dk, dv, max_new=st.max_new, min_new=st.min_new)
         mix = S.gated_headnorm(o, self.norm32, proj[:, C:gate0], H, dv, self.eps, st.act_dtype)
         return S.linear(mix, self.w_o)
 

@@ -3,6 +3,7 @@
 // here operands are fp32 rows of a packed batch, the state is [dk][dv] per slot, and nothing is kept for a backward pass.
 //     delta:      U = R (b V) - Kw S,  O = gam q S + P U,  S <- gam_63 S + (Gp K)^T U
 //     retention:  U = V,               the same
+// Which sequences of a step go this way is their own number of new tokens' affair (`from`): beside a long prompt, a short one and a single token take the kernel they take alone.
 // A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
 // the chip could multiply; the chunks take 363 us (prep 142, scan 203) and 183 us (scan 173).  Bound: the scan's chain of chunks (two products behind two barriers each), not the
 // pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
@@ -24,6 +25,7 @@ struct DChunkArgs {
     const float* head_decay;  // retention: [H]
     float qscale, kscale;     // retention
     int H, G, heads;  // heads: of all sequences
+    int from;         // sequences with fewer new tokens are another kernel's
     float *state, *o, *ws;
 };
 
@@ -39,7 +41,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
     __shared__ float be[GC], gam[GC], qf[GC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
     const int n = blockIdx.x, h = blockIdx.y, s = blockIdx.z, hq = h / (p.H / p.G), t0 = p.seq_off[s] + n * GC, cnt = min(GC, p.seq_off[s + 1] - t0);
-    if (cnt <= 0) return;
+    if (cnt <= 0 || p.seq_off[s + 1] - p.seq_off[s] < p.from) return;
     const float *qp = p.q + (int64_t)t0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)t0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)t0 * p.ldv + (int64_t)h * GD;
     float* blk = chunk_block(p, s, h, n);
     if (wave == 0) {
@@ -142,7 +144,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
     const bool qside = wave >= 2;
     const float *qp = p.q + (int64_t)s0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)s0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)s0 * p.ldv + (int64_t)h * GD + v0;
     float* state = p.state + ((int64_t)p.slot[s] * p.H + h) * GD * GD + v0;
-    if (NC <= 0) return;
+    if (NC <= 0 || len < p.from) return;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;
@@ -242,7 +244,7 @@ extern "C" int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq
     return tokens > 0 && n_seq > 0 && H > 0 ? (tokens / GC + n_seq) * (int64_t)H * D_BLOCK * 4 : 0;
 }
 
-extern "C" int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
+extern "C" int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, int from, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
                                    const float* v, int64_t ldv, const float* tok, const float* head_decay, float qscale, float kscale, float* state, float* o, void* workspace,
                                    int64_t workspace_bytes, void* stream) {
     MI355_REQUIRE(tokens > 0 && n_seq > 0 && n_seq <= 65535 && (int64_t)n_seq * H <= (1 << 26) && max_new > 0 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && q && k && v && state && o && workspace &&
@@ -253,7 +255,7 @@ extern "C" int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, const
     MI355_REQUIRE(workspace_bytes >= mi355_delta_chunked_workspace_bytes(tokens, n_seq, H), "delta_chunked: workspace too small (%lld bytes)", (long long)workspace_bytes);
     DChunkArgs p;
     p.seq_off = seq_off, p.slot = slot, p.q = q, p.k = k, p.v = v, p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.tok = (const f32x4*)tok, p.head_decay = head_decay;
-    p.qscale = qscale, p.kscale = kscale, p.H = H, p.G = G, p.heads = n_seq * H, p.state = state, p.o = o, p.ws = (float*)workspace;
+    p.qscale = qscale, p.kscale = kscale, p.H = H, p.G = G, p.heads = n_seq * H, p.from = from, p.state = state, p.o = o, p.ws = (float*)workspace;
     const dim3 prep((max_new + GC - 1) / GC, H, n_seq), scan((unsigned)((n_seq * (int64_t)H + 7) / 8 * 32));
     if (tok) {
         dchunk_prep_kernel<true><<<prep, 256, 0, ST(stream)>>>(p);

@@ -375,7 +375,7 @@ __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - l
 __global__ void gla_kernel(const int* __restrict__ seq_off, const int* __restrict__ slot, int H, int dk, int dv, const void* __restrict__ q, const void* __restrict__ k,
                            const void* __restrict__ v, const void* __restrict__ z, int dt, int z_dt, int v_dt, int64_t ldq, int64_t ldk, int64_t ldv_, int64_t ldz,
                            const float* __restrict__ zbias, float inv_tau, float qscale, const float* __restrict__ head_decay, float kscale,
-                           float* __restrict__ state, float* __restrict__ o) {
+                           float* __restrict__ state, float* __restrict__ o, int below) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int RC = blockDim.x >> 6;
     float* sq = smem;                       // [TB][dk]
@@ -385,6 +385,7 @@ __global__ void gla_kernel(const int* __restrict__ seq_off, const int* __restric
     float* sp = sv + GLA_TB * 64;           // [TB][RC][64]
     const int s = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 64 + (threadIdx.x & 63), chunk = threadIdx.x >> 6;
     const int t0 = seq_off[s], t1 = seq_off[s + 1];
+    if (below && t1 - t0 >= below) return;  // (the same for the whole workgroup)
     const bool col_ok = col < dv;
     float* S = state + (((int64_t)slot[s] * H + h) * dk) * dv;
     float st[GLA_R];
@@ -485,10 +486,10 @@ __global__ void gla_kernel(const int* __restrict__ seq_off, const int* __restric
     }
 }
 
-extern "C" int mi355_gla_fwd(int n_seq, const int* seq_off, const int* slot, int H, int dk, int dv, const void* q, const void* k, const void* v, const void* z, int dt,
+extern "C" int mi355_gla_fwd_below(int n_seq, const int* seq_off, const int* slot, int H, int dk, int dv, const void* q, const void* k, const void* v, const void* z, int dt,
                              int z_dt, int v_dt, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldz, const float* zbias, float inv_tau, float qscale, const float* head_decay, float kscale,
-                             float* state, float* o, void* stream) {
-    MI355_REQUIRE(n_seq > 0 && n_seq <= 65535 && seq_off && slot && H > 0 && H <= 65535 && dk > 0 && dk <= 16 * GLA_R && dv > 0 && q && k && v && state && o && dt_ok(dt) && dt_ok(v_dt),
+                             float* state, float* o, int below, void* stream) {
+    MI355_REQUIRE(below >= 0 && n_seq > 0 && n_seq <= 65535 && seq_off && slot && H > 0 && H <= 65535 && dk > 0 && dk <= 16 * GLA_R && dv > 0 && q && k && v && state && o && dt_ok(dt) && dt_ok(v_dt),
                   "gla_fwd: bad arguments (key channels per head <= 256)");
     MI355_REQUIRE(head_decay || (z && zbias && dt_ok(z_dt) && ldz >= (int64_t)H * dk), "gla_fwd: the decay needs its rows and bias, or a constant per head");
     MI355_REQUIRE(ldq >= (int64_t)H * dk && ldk >= (int64_t)H * dk && ldv >= (int64_t)H * dv, "gla_fwd: rows too short");
@@ -496,9 +497,15 @@ extern "C" int mi355_gla_fwd(int n_seq, const int* seq_off, const int* slot, int
     const size_t lds_bytes = sizeof(float) * ((size_t)3 * GLA_TB * dk + (size_t)GLA_TB * 64 + (size_t)GLA_TB * RC * 64);
     MI355_REQUIRE(lds_bytes <= 64 * 1024, "gla_fwd: LDS budget exceeded");
     gla_kernel<<<dim3(n_seq, H, (dv + 63) / 64), 64 * RC, lds_bytes, ST(stream)>>>(seq_off, slot, H, dk, dv, q, k, v, z, dt, z_dt, v_dt, ldq, ldk, ldv, ldz, zbias, inv_tau, qscale,
-                                                                                   head_decay, kscale, state, o);
+                                                                                   head_decay, kscale, state, o, below);
     MI355_LAUNCH_CHECK("gla_fwd");
     return 0;
+}
+
+extern "C" int mi355_gla_fwd(int n_seq, const int* seq_off, const int* slot, int H, int dk, int dv, const void* q, const void* k, const void* v, const void* z, int dt,
+                             int z_dt, int v_dt, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldz, const float* zbias, float inv_tau, float qscale, const float* head_decay, float kscale,
+                             float* state, float* o, void* stream) {
+    return mi355_gla_fwd_below(n_seq, seq_off, slot, H, dk, dv, q, k, v, z, dt, z_dt, v_dt, ldq, ldk, ldv, ldz, zbias, inv_tau, qscale, head_decay, kscale, state, o, 0, stream);
 }
 
 // ------------------------------------------------------------------------------------------- router logits

@@ -563,6 +563,7 @@ struct DeltaArgs {
     int64_t ldq, ldk, ldv, ldb, lda;
     int H, G, dk, dv, qk_dt, v_dt, ba_dt;
     float qscale;
+    int below;  // 0: every sequence; else those with fewer new tokens
 };
 
 __global__ __launch_bounds__(256) void delta_prep_kernel(int64_t T, DeltaArgs p) {
@@ -598,6 +599,7 @@ __global__ __launch_bounds__(256) void delta_rule_kernel(DeltaArgs p) {
     const bool col_ok = col < p.dv;
     const int hq = h / (p.H / p.G), dk = p.dk;
     const int t0 = p.seq_off[s], t1 = p.seq_off[s + 1];
+    if (p.below && t1 - t0 >= p.below) return;
     float* S = p.state + (((int64_t)p.slot[s] * p.H + h) * dk) * p.dv;
     float st[CPL];
 #pragma unroll
@@ -675,10 +677,10 @@ static void launch_delta(const DeltaArgs& p, dim3 grid, bool vec, hipStream_t st
     else delta_rule_kernel<CPL, false><<<grid, 256, 0, st>>>(p);
 }
 
-extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
+extern "C" int mi355_delta_rule_ragged_below(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
                                        int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
-                                       const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream) {
-    MI355_REQUIRE(tokens > 0 && n_seq > 0 && n_seq <= 65535 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 32 * DR_LPR && dv > 0 && q && k && v &&
+                                       const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, int below, void* stream) {
+    MI355_REQUIRE(below >= 0 && tokens > 0 && n_seq > 0 && n_seq <= 65535 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 32 * DR_LPR && dv > 0 && q && k && v &&
                       b && a && A_log && dt_bias && state && o && ws,
                   "delta_rule_ragged: bad arguments (key channels per head <= 256, value heads a multiple of the query / key heads, workspace of 4 floats per token and head)");
     MI355_REQUIRE(rec_dt_ok(qk_dt) && rec_dt_ok(v_dt) && rec_dt_ok(ba_dt) && ldq >= (int64_t)G * dk && ldk >= (int64_t)G * dk && ldv >= (int64_t)H * dv && ldb >= H && lda >= H,
@@ -686,7 +688,7 @@ extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq
     MI355_REQUIRE(((uintptr_t)ws & 15) == 0, "delta_rule_ragged: the workspace must be 16-byte aligned");
     DeltaArgs p;
     p.seq_off = seq_off, p.slot = slot, p.q = q, p.k = k, p.v = v, p.b = b, p.a = a, p.A_log = A_log, p.dt_bias = dt_bias, p.state = state, p.o = o, p.ws = (f32x4*)ws;
-    p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.ldb = ldb, p.lda = lda, p.H = H, p.G = G, p.dk = dk, p.dv = dv, p.qk_dt = qk_dt, p.v_dt = v_dt, p.ba_dt = ba_dt, p.qscale = qscale;
+    p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.ldb = ldb, p.lda = lda, p.H = H, p.G = G, p.dk = dk, p.dv = dv, p.qk_dt = qk_dt, p.v_dt = v_dt, p.ba_dt = ba_dt, p.qscale = qscale, p.below = below;
     delta_prep_kernel<<<rec_rows_grid(tokens * H, 4), 256, 0, ST(stream)>>>(tokens, p);
     MI355_LAUNCH_CHECK("delta_rule_ragged(prep)");
     const bool vec = qk_dt == MI355_DT_F32 && dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ((uintptr_t)q & 15) == 0 && ((uintptr_t)k & 15) == 0;
@@ -697,6 +699,12 @@ extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq
     else launch_delta<32>(p, grid, vec, ST(stream));
     MI355_LAUNCH_CHECK("delta_rule_ragged");
     return 0;
+}
+
+extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
+                                       int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
+                                       const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream) {
+    return mi355_delta_rule_ragged_below(tokens, n_seq, seq_off, slot, H, G, dk, dv, q, k, qk_dt, ldq, ldk, v, v_dt, ldv, b, a, ba_dt, ldb, lda, A_log, dt_bias, qscale, state, o, ws, 0, stream);
 }
 
 // The per-token numbers alone (the chunked kernels of delta_chunk.hip take them): ws [tokens, H] x {decay, beta, key factor, query factor x qscale}.

@@ -133,7 +133,7 @@ DELTA_CHUNKED_MIN = 64  # new tokens of a sequence from which the chunked recurr
 
 def _delta_chunked(q, k, v, dk, dv, max_new):
     """Whether a step's recurrence takes the chunked kernels (csrc/delta_chunk.hip): heads of 128 | 128 on fp32 rows in 16-byte words, and a sequence with at least a whole chunk of
-    new tokens (a last chunk is worked out as a whole one).  Both sides with 16 heads, token by token / in chunks: 64 tokens 53 / 44 us
+    new tokens (a last chunk is worked out as a whole one).  Of such a step the sequences with fewer new tokens still go token by token, as they do alone.  Both sides with 16 heads, token by token / in chunks: 64 tokens 53 / 44 us
     (one decay per head: 41 / 20), 333 tokens 238 / 86 (182 / 51), six times 900 921 / 363 (504 / 183); below a chunk the delta rule loses: 32 tokens 31 / 41, six times 32 42 / 51."""
     return (max_new >= DELTA_CHUNKED_MIN and q.shape[0] > 0 and dk == 128 and dv == 128 and q.dtype == k.dtype == v.dtype == F32 and not (q.stride(0) | k.stride(0)) % 4
             and not (q.data_ptr() | k.data_ptr()) % 16)
@@ -143,20 +143,21 @@ def _run_chunked(q, k, v, tok, head_decay, qscale, kscale, seq_off, slot, state,
     T, n_seq = q.shape[0], slot.numel()
     need = L.load().mi355_delta_chunked_workspace_bytes(T, n_seq, H)
     ws = torch.empty(need // 4, dtype=F32, device=q.device)
-    L.call("mi355_delta_chunked", T, n_seq, int(max_new), L.ptr(seq_off), L.ptr(slot), H, G, L.ptr(q), q.stride(0), L.ptr(k), k.stride(0), L.ptr(v), v.stride(0), L.ptr(tok), L.ptr(head_decay),
+    L.call("mi355_delta_chunked", T, n_seq, int(max_new), DELTA_CHUNKED_MIN, L.ptr(seq_off), L.ptr(slot), H, G, L.ptr(q), q.stride(0), L.ptr(k), k.stride(0), L.ptr(v), v.stride(0), L.ptr(tok), L.ptr(head_decay),
            float(qscale), float(kscale), L.ptr(state), L.ptr(o), L.ptr(ws), need)
     return o
 
 
-def gla(q, k, v, z, zbias, inv_tau, qscale, seq_off, slot, state, H, dk, dv, head_decay=None, kscale=1.0, max_new=0):
+def gla(q, k, v, z, zbias, inv_tau, qscale, seq_off, slot, state, H, dk, dv, head_decay=None, kscale=1.0, max_new=0, min_new=0):
     """Gated linear attention over a ragged batch; ``state`` fp32 [slots, H, dk, dv] is read and written at ``slot``.  Returns fp32 [tokens, H * dv].
     ``head_decay`` (fp32 [H]): a fixed decay per head instead of the per-channel one from ``z`` (``z`` / ``zbias`` may then be None); keys are multiplied
-    by ``kscale``.  ``max_new``: the most new tokens of one sequence of the step (0: not known); long steps with a fixed decay go in chunks."""
+    by ``kscale``.  ``max_new`` and ``min_new``: the most and the least new tokens of one sequence of the step (0: not known); where the most is known and the decay fixed (at
+    1e-30 or above), long sequences go in chunks."""
     L.require_gpu(q, k, v, z, zbias, seq_off, slot, state, head_decay)
     if head_decay is not None:
         if head_decay.dtype != F32 or not head_decay.is_contiguous() or head_decay.numel() != H:
             raise ValueError("gla: head_decay fp32 [H]")
-        return _gla_fixed(q, k, v, head_decay, qscale, kscale, seq_off, slot, state, H, dk, dv, max_new)
+        return _gla_fixed(q, k, v, head_decay, qscale, kscale, seq_off, slot, state, H, dk, dv, max_new, min_new)
     for t, n, w in ((q, "q", H * dk), (k, "k", H * dk), (z, "z", H * dk), (v, "v", H * dv)):
         _rows(t, f"gla({n})")
         if t.shape[1] != w or (n != "z" and t.dtype != q.dtype) or t.shape[0] != q.shape[0]:
@@ -172,7 +173,7 @@ def gla(q, k, v, z, zbias, inv_tau, qscale, seq_off, slot, state, H, dk, dv, hea
     return o
 
 
-def _gla_fixed(q, k, v, head_decay, qscale, kscale, seq_off, slot, state, H, dk, dv, max_new=0):
+def _gla_fixed(q, k, v, head_decay, qscale, kscale, seq_off, slot, state, H, dk, dv, max_new=0, min_new=0):
     for t, n, w in ((q, "q", H * dk), (k, "k", H * dk), (v, "v", H * dv)):
         _rows(t, f"gla({n})")
         if t.shape[1] != w or (n != "v" and t.dtype != q.dtype) or t.shape[0] != q.shape[0]:
@@ -183,10 +184,12 @@ def _gla_fixed(q, k, v, head_decay, qscale, kscale, seq_off, slot, state, H, dk,
     if state.dtype != F32 or not state.is_contiguous() or tuple(state.shape[1:]) != (H, dk, dv):
         raise ValueError("gla: state fp32 [slots, H, dk, dv]")
     o = torch.empty((q.shape[0], H * dv), dtype=F32, device=q.device)
-    if _delta_chunked(q, k, v, dk, dv, max_new):
-        return _run_chunked(q, k, v, None, head_decay, qscale, kscale, seq_off, slot, state, o, H, H, max_new)
-    L.call("mi355_gla_fwd", n_seq, L.ptr(seq_off), L.ptr(slot), H, dk, dv, L.ptr(q), L.ptr(k), L.ptr(v), None, _dt(q), 0, _dt(v), q.stride(0), k.stride(0), v.stride(0),
-           0, None, 1.0, float(qscale), L.ptr(head_decay), float(kscale), L.ptr(state), L.ptr(o))
+    chunked = _delta_chunked(q, k, v, dk, dv, max_new)
+    if not chunked or min_new < DELTA_CHUNKED_MIN:
+        L.call("mi355_gla_fwd_below", n_seq, L.ptr(seq_off), L.ptr(slot), H, dk, dv, L.ptr(q), L.ptr(k), L.ptr(v), None, _dt(q), 0, _dt(v), q.stride(0), k.stride(0), v.stride(0),
+               0, None, 1.0, float(qscale), L.ptr(head_decay), float(kscale), L.ptr(state), L.ptr(o), DELTA_CHUNKED_MIN if chunked else 0)
+    if chunked:
+        _run_chunked(q, k, v, None, head_decay, qscale, kscale, seq_off, slot, state, o, H, H, max_new)
     return o
 
 
@@ -440,9 +443,9 @@ def qkv_rows_append(src, H, G, d, dv, bias, qw, kw, eps, qscale, dims, layout, f
     return q
 
 
-def delta_rule(q, k, v, b, a, A_log, dt_bias, qscale, seq_off, slot, state, H, G, dk, dv, max_new=0):
-    """Gated delta rule over a ragged batch (raw q / k rows: made unit vectors inside); ``state`` fp32 [slots, H, dk, dv].  Returns fp32 [tokens, H * dv].  ``max_new``: the most
-    new tokens of one sequence of the step (0: not known); long steps go in chunks."""
+def delta_rule(q, k, v, b, a, A_log, dt_bias, qscale, seq_off, slot, state, H, G, dk, dv, max_new=0, min_new=0):
+    """Gated delta rule over a ragged batch (raw q / k rows: made unit vectors inside); ``state`` fp32 [slots, H, dk, dv].  Returns fp32 [tokens, H * dv].  ``max_new`` and
+    ``min_new``: the most and the least new tokens of one sequence of the step (0: not known); where the most is known, long sequences go in chunks."""
     L.require_gpu(q, k, v, b, a, A_log, dt_bias, seq_off, slot, state)
     T = q.shape[0]
     for t, n, w in ((q, "q", G * dk), (k, "k", G * dk), (v, "v", H * dv), (b, "b", H), (a, "a", H)):
@@ -461,12 +464,15 @@ def delta_rule(q, k, v, b, a, A_log, dt_bias, qscale, seq_off, slot, state, H, G
             raise ValueError("delta_rule: A_log and dt_bias fp32 [H]")
     o = torch.empty((T, H * dv), dtype=F32, device=q.device)
     ws = torch.empty((T * H * 4,), dtype=F32, device=q.device)  # per token and head: decay, beta, the two unit-vector factors
-    if _delta_chunked(q, k, v, dk, dv, max_new):
+    chunked = _delta_chunked(q, k, v, dk, dv, max_new)
+    if not chunked or min_new < DELTA_CHUNKED_MIN:
+        L.call("mi355_delta_rule_ragged_below", T, n_seq, L.ptr(seq_off), L.ptr(slot), H, G, dk, dv, L.ptr(q), L.ptr(k), _dt(q), q.stride(0), k.stride(0), L.ptr(v), _dt(v), v.stride(0),
+               L.ptr(b), L.ptr(a), _dt(b), b.stride(0), a.stride(0), L.ptr(A_log), L.ptr(dt_bias), float(qscale), L.ptr(state), L.ptr(o), L.ptr(ws), DELTA_CHUNKED_MIN if chunked else 0)
+    else:
         L.call("mi355_delta_rule_tokens", T, H, G, dk, L.ptr(q), L.ptr(k), _dt(q), q.stride(0), k.stride(0), L.ptr(b), L.ptr(a), _dt(b), b.stride(0), a.stride(0), L.ptr(A_log), L.ptr(dt_bias),
                float(qscale), L.ptr(ws))
-        return _run_chunked(q, k, v, ws, None, 1.0, 1.0, seq_off, slot, state, o, H, G, max_new)
-    L.call("mi355_delta_rule_ragged", T, n_seq, L.ptr(seq_off), L.ptr(slot), H, G, dk, dv, L.ptr(q), L.ptr(k), _dt(q), q.stride(0), k.stride(0), L.ptr(v), _dt(v), v.stride(0),
-           L.ptr(b), L.ptr(a), _dt(b), b.stride(0), a.stride(0), L.ptr(A_log), L.ptr(dt_bias), float(qscale), L.ptr(state), L.ptr(o), L.ptr(ws))
+    if chunked:
+        _run_chunked(q, k, v, ws, None, 1.0, 1.0, seq_off, slot, state, o, H, G, max_new)
     return o
 
 

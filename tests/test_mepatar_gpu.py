@@ -410,6 +410,34 @@ def test_recurrences_in_chunks_equal_those_by_token(rule, H, G, decay):
         assert row_err(chunked[at : at + n], want.reshape(n, -1)) < 1e-5
 
 
+@pytest.mark.parametrize("rule,H,G", [("delta", 4, 2), ("retention", 3, 3)])
+def test_recurrences_of_a_sequence_do_not_know_what_shares_the_step(rule, H, G):
+    """Single tokens, portions below a chunk and long prompts in one step, heads of 128 | 128: every sequence's outputs and state are the bits that it gets in a step of its own."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(H)
+    D, lens, slots = 128, [1, 200, 63, 64, 1, 65], [4, 2, 0, 5, 1, 3]
+    d = _Slots(lens, slots)
+    x = torch.randn(sum(lens), (2 * G + H) * D, generator=g).to(DEV)
+    start = torch.randn(6, H, D, D, generator=g).to(DEV)
+    ba = (torch.randn(sum(lens), 2 * H, generator=g) * 2).to(DEV)
+    A_log, dt_bias, dec = torch.full((H,), -2.0, device=DEV), torch.zeros(H, device=DEV), torch.linspace(0.5, 0.99, H, device=DEV)
+
+    def run(rows, desc, state, n):
+        q, k, v = x[rows, : G * D], x[rows, G * D : 2 * G * D], x[rows, 2 * G * D :]
+        if rule == "delta":
+            return S.delta_rule(q, k, v, ba[rows, :H], ba[rows, H:], A_log, dt_bias, D ** -0.5, desc.seq_off, desc.slots, state, H, G, D, D, max_new=max(n), min_new=min(n))
+        return S.gla(q, k, v, None, None, 1.0, 1.0, desc.seq_off, desc.slots, state, H, D, D, head_decay=dec, kscale=D ** -0.5, max_new=max(n), min_new=min(n))
+
+    together = start.clone()
+    out = run(slice(0, sum(lens)), d, together, lens)
+    for i, n in enumerate(lens):
+        alone = start.clone()
+        rows = slice(d.off[i], d.off[i + 1])
+        assert torch.equal(run(rows, _Slots([n], [slots[i]]), alone, [n]), out[rows]), (i, n)
+        assert torch.equal(alone[slots[i]], together[slots[i]]), f"state in slot {slots[i]}"
+
+
 def _attention_case(dt, H, G, d, dv, size, keep, past, n_new, hot):
     """One sequence with ``past`` cached keys and ``n_new`` queries.  Every key is small noise except the ``hot`` ones, which match the query direction
     with a large score and carry a marked value: whether a query's output shows the mark says whether it saw the key."""
