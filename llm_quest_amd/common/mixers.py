@@ -353,6 +353,7 @@ class Retention(_Frozen):
         if rot_dims % 2 or rot_dims > dim:
             raise ValueError("Retention: the rotated entries are an even number <= dim")
         self.width, self.heads, self.dim, self.vdim, self.decay, self.rot_dims, self.rot_base, self.eps, self.layer_idx = width, heads, dim, vdim, [float(d) for d in decay], rot_dims, float(rot_base), float(eps), layer_idx
+        self.log_decay = all(1e-30 <= d <= 1.0 for d in self.decay)  # chunks of tokens work with the decay's logarithm: other decays go token by token
         self.w_in = self._param(2 * heads * dim + 2 * heads * vdim, width)  # [q | k | v | gate] rows -> one product
         self.w_o = self._param(width, heads * vdim)
         self._ready = None
@@ -376,7 +377,7 @@ class Retention(_Frozen):
         qk = torch.empty((h.shape[0], b), dtype=F32, device=h.device)
         S.rope_heads(proj, 2 * H, dk, dk, 0, qk, dk, 0, 0, self.rot_dims, self.freq, st.pos, layout=1)  # q and k heads side by side: 2 H heads of dim
         o = S.gla(qk[:, :a], qk[:, a:b], proj[:, b:c], None, None, 1.0, 1.0, st.seq_off, st.slots, st.cache.state(self.layer_idx, "S"), H, dk, dv,
-                  head_decay=self.decay32, kscale=dk ** -0.5, max_new=st.max_new, min_new=st.min_new)
+                  head_decay=self.decay32, kscale=dk ** -0.5, max_new=st.max_new if self.log_decay else 0, min_new=st.min_new)
         mix = S.gated_headnorm(o, self.ones, proj[:, c:], H, dv, self.eps, st.act_dtype)
         return S.linear(mix, self.w_o)
 

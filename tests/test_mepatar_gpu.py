@@ -438,6 +438,32 @@ def test_recurrences_of_a_sequence_do_not_know_what_shares_the_step(rule, H, G):
         assert torch.equal(alone[slots[i]], together[slots[i]]), f"state in slot {slots[i]}"
 
 
+def test_retention_with_any_fixed_decay_does_not_know_how_a_prompt_is_cut():
+    """Decays that have no logarithm (negative, zero), one below what the chunks of tokens hold and one above one, heads of 128 | 128: a prompt of more than a chunk is the same rows as
+    in two short portions (fp32 sums of 128 channels in the same order, equal up to the tiles of the products around them: 1e-5 as above; states head by head, their sizes are far apart)."""
+    from llm_quest_amd.common.mixers import Retention, SeqStep
+    from llm_quest_amd.utils import SlotStateCache
+
+    torch.manual_seed(5)
+    mod = Retention(64, 4, 128, 128, [-0.7, 0.0, 1e-35, 1.25], 0, 1e4, 1e-5, 0)
+    mod.w_in.data.copy_(torch.randn_like(mod.w_in.float()) / 8)
+    mod.w_o.data.copy_(torch.randn_like(mod.w_o.float()) / 16)
+    mod = mod.to(DEV)
+    h = torch.randn(100, 64, device=DEV)
+    rows = []
+    for cuts in ([100], [50, 50]):
+        cache = SlotStateCache([mod.cache_spec()], 4096, DEV, F32, slots=1)
+        slot, at = cache.open("a"), 0
+        for n in cuts:
+            rows.append(mod.step(h[at : at + n], SeqStep(cache, [(slot, [0] * n)], DEV, F32)))
+            cache.advance(slot, [0] * n)
+            at += n
+        rows.append(cache.state(0, "S")[slot].clone())
+    assert row_err(rows[0], torch.cat(rows[2:4])) < 1e-5
+    for i in range(4):
+        assert row_err(rows[1][i], rows[4][i]) < 1e-5, f"state of head {i}"
+
+
 def _attention_case(dt, H, G, d, dv, size, keep, past, n_new, hot):
     """One sequence with ``past`` cached keys and ``n_new`` queries.  Every key is small noise except the ``hot`` ones, which match the query direction
     with a large score and carry a marked value: whether a query's output shows the mark says whether it saw the key."""
