@@ -388,8 +388,8 @@ int mi355_gated_delta_rule_bwd(int B, int S, int Hqk, int Hv, int Dk, int Dv, co
  * (the state gradient's starting value) and where d(loss) / d(initial_state) is left -- training through a carried recurrent state
  * (gated_delta_rule(..., prev_state), qwen3_next_attention.py:103-159).  The forward must have run with that initial_state and checkpoints. */
 
-/* The same rule in chunks of 64 tokens on the fp32 matrix pipe, for heads of 128 | 128 and the operands a layer makes (unit keys, 0 <= alpha <= 1; alpha below
- * 1e-30 counts as 1e-30).  saved: mi355_gdr_chunked_saved_bytes, 16-byte aligned: the forward's scratch, and (keep != 0) what the backward reads; v's row pitch a
+/* The same rule in chunks of 64 tokens on the fp32 matrix pipe, for heads of 128 | 128 and the operands a layer makes (unit keys, alpha and beta in 0 .. 1; either
+ * below 1e-30 counts as 1e-30).  saved: mi355_gdr_chunked_saved_bytes, 16-byte aligned: the forward's scratch, and (keep != 0) what the backward reads; v's row pitch a
  * multiple of 8; states as above.  The backward's workspace: mi355_gdr_chunked_bwd_workspace_bytes. */
 int64_t mi355_gdr_chunked_saved_bytes(int B, int S, int Hv);
 int64_t mi355_gdr_chunked_bwd_workspace_bytes(int B, int S, int Hqk, int Hv);

@@ -36,6 +36,19 @@ __device__ __forceinline__ double cumulated_log64(float a) {
     return g;
 }
 
+// exp of a sum of log decays: expf takes the rounded sum, the first power of what was cut off comes back behind it (of -20 fp32 keeps two parts in 10^6)
+__device__ __forceinline__ float exp_of(double g) {
+    const float r = (float)g, e = expf(r);
+    return fmaf(e, (float)(g - (double)r), e);
+}
+__device__ __forceinline__ void add16(f32x16& to, f32x16& from) {  // a chain's sum so far to its total, and the chain begins anew: half the length, 0.7 of its error
+#pragma unroll
+    for (int e = 0; e < 16; ++e) {
+        to[e] += from[e];
+        from[e] = 0.f;
+    }
+}
+
 // T = (I + tril(N, -1))^-1, both [64][68] in LDS, by the four waves of a workgroup (N's upper right quarter is scratch): the two diagonal 32 x 32 blocks by forward
 // substitution (lane = column), the block below them as -R22 (N21 R11).
 __device__ __forceinline__ void invert_unit_lower64(float (&N)[GC][GC + 4], float (&T)[GC][GC + 4]) {

@@ -9,7 +9,12 @@
 // workgroup per chunk afterwards.  Four kernels: prep, scan, reverse scan (both per 32 value rows of the state: a row never meets another), and the rest.
 // All sums are fp32 FMAs on v_mfma_f32_32x32x2_f32 (the two products of bf16 operands alone, K K^T and Q K^T, on the bf16 shape: exact); the log decays are cumulated
 // in fp64, so a difference of two large ones keeps its digits.  d(alpha) is taken from sums over the pairs that span a token -- never as a difference of
-// larger sums, so it keeps its digits where alpha is tiny (below 1e-30 alpha counts as 1e-30).
+// larger sums, so it keeps its digits where alpha is tiny (below 1e-30 alpha counts as 1e-30); d(beta) as what reaches u times u / beta.
+// A matrix pipe's chain of 128 products rounds 128 times at its size where lanes sum 16 and meet in a tree; so the chains that show are cut (add16) and the state's gradient
+// gathers its terms from the last token to the first.  Distance to 64 bits, token-by-token kernels | here, 256 tokens, geometric mean of four draws: outputs, d(q), d(k), d(v)
+// 1.65e-3 | 1.65e-3 (their bf16); fp32: state 7.4e-8 | 8.6e-8, d(state) 9.0e-8 | 9.5e-8 (2.9e-7 from the first token on), d(beta) 1.5e-7 | 1.8e-7 (2.6e-7 with whole chains), d(alpha)
+// 1.7e-7 | 2.1e-7 (2.5e-7); decays near one 4.4e-7 | 3.6e-7, 5.0e-7 | 4.9e-7; nearly parallel keys 1.5e-7 | 2.3e-7, 2.1e-7 | 4.4e-7.  Cutting d(q)'s and d(k)'s chains as well:
+// d(alpha) 1.9e-7 for 50 us of a backward of 680 (registers spill).
 // Bound: the fp32 matrix pipe (256 FLOP a clock and CU).  The products of one 64-token chunk of one head: 37 MFLOP forward and backward together.
 #include "gdr_chunk.h"
 
@@ -31,6 +36,8 @@ __device__ __forceinline__ double cumulated_log(const float* alpha, int64_t idx,
     a_out = decay_at_least(in ? alpha[idx] : 1.f);
     return cumulated_log64(a_out);
 }
+// a token's beta; zero counts as 1e-30 (as the decays' floor: nothing that is kept changes, and u / beta is v minus what the state already holds)
+__device__ __forceinline__ float beta_of(const float* beta, int64_t idx, bool in) { return in ? decay_at_least(beta[idx]) : 0.f; }
 
 // The scans' workgroups: the four value ranges of a head read the same Kw / P / Q / K, so they go to one XCD (workgroups are dealt to the eight XCDs in turn), side by side.
 __device__ __forceinline__ bool scan_place(int heads, int& head, int& v0) {
@@ -72,10 +79,10 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
         const double g = cumulated_log(alpha, (tok0 + lane) * Hv + h, lane < cnt, a);
         const double g63 = __shfl(g, 63, 64);
         gd[lane] = g;
-        be[lane] = lane < cnt ? beta[(tok0 + lane) * Hv + h] : 0.f;
-        gam[lane] = expf((float)g);
-        blk[G_GAM + lane] = expf((float)g);
-        blk[G_GAM + GC + lane] = expf((float)(g63 - g));
+        be[lane] = beta_of(beta, (tok0 + lane) * Hv + h, lane < cnt);
+        gam[lane] = exp_of(g);
+        blk[G_GAM + lane] = exp_of(g);
+        blk[G_GAM + GC + lane] = exp_of(g63 - g);
     }
     __syncthreads();
     {  // K K^T and Q K^T: wave = tile (ti, tj); the tile above the diagonal is zero
@@ -96,7 +103,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int i = 32 * ti + c_row(e, hf);
-            const float D = i >= j ? expf((float)(gd[i] - gj)) : 0.f;
+            const float D = i >= j ? exp_of(gd[i] - gj) : 0.f;
             N[i][j] = i > j ? be[i] * kk[e] * D : 0.f;
             blk[G_P + i * GC + j] = i >= j ? qscale * qk[e] * D : 0.f;
         }
@@ -109,7 +116,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
         *reinterpret_cast<f32x4*>(blk + G_R + r * GC + c) = *reinterpret_cast<const f32x4*>(&T[r][c]);
     }
     {  // Uv = R (b V), Kw = R (b gam K): wave = 32 columns, both row halves (the upper one ends at token 32)
-        f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16();
+        f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16(), ut = zero16(), wt = zero16();
         const int col = 32 * wave + ln;
 #pragma unroll
         for (int kb = 0; kb < GC; kb += 8) {
@@ -127,7 +134,10 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
                     w0 = mfma2(a0[j], bk, w0);
                 }
             }
+            if (kb == 24) add16(ut, u1), add16(wt, w1);
         }
+        add16(u1, ut);
+        add16(w1, wt);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int r = c_row(e, hf);
@@ -197,7 +207,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
                 *reinterpret_cast<f32x4*>(blk + (v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
             }
         }
-        f32x16 uv, acc = zero16();
+        f32x16 uv = zero16(), acc = zero16();
         if (!qside) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) uv[e] = blk[G_U + (32 * rh + c_row(e, hf)) * GD + v0 + ln];
@@ -210,6 +220,13 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
             else a = widen4(i & 1 ? u32x2{__float_as_uint(fr[i >> 1][2]), __float_as_uint(fr[i >> 1][3])} : u32x2{__float_as_uint(fr[i >> 1][0]), __float_as_uint(fr[i >> 1][1])});
 #pragma unroll
             for (int j = 0; j < 4; ++j) acc = mfma2(a[j], s[j], acc);
+            if (i == 7) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    uv[e] -= acc[e];
+                    acc[e] = 0.f;
+                }
+            }
             if (i % 4 == 3) asm volatile("" ::: "memory");  // keep the state reads of later steps where they are: all sixteen at once cost more registers than there are
         }
 #pragma unroll
@@ -232,7 +249,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
         __syncthreads();
         if (qside) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] *= gg[32 * rh + c_row(e, hf)] * qscale;
+            for (int e = 0; e < 16; ++e) acc[e] = (acc[e] - uv[e]) * (gg[32 * rh + c_row(e, hf)] * qscale);
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 if (rh == 0 && i >= 4) break;  // P is lower triangular
@@ -338,7 +355,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, in
         }
         __syncthreads();
         // dU = P^T dO + Gp (K dS^T): wave = (row half, half of the contraction); the two halves of a contraction meet in LDS
-        f32x16 u = zero16(), pt = zero16();
+        f32x16 u = zero16(), ut = zero16(), pt = zero16();
         {
             f32x4 kf[8];
 #pragma unroll
@@ -357,7 +374,9 @@ __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, in
                 const f32x4 s = *reinterpret_cast<const f32x4*>(&Ss[ln][64 * kh + 8 * i + 4 * hf]);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) u = mfma2(kf[i][j], s[j], u);
+                if (i == 3) add16(ut, u);
             }
+            add16(u, ut);
             if (some) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
@@ -386,10 +405,11 @@ __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, in
         const float gC = gg[GC - 1];
 #pragma unroll
         for (int e = 0; e < 16; ++e) s[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
+        // from the last token to the first: what reaches the chunk's start grows that way (the other way around the large terms come first and every later sum rounds at their size)
 #pragma unroll 2
-        for (int kb = 0; kb < GC; kb += 8)
+        for (int kb = GC - 8; kb >= 0; kb -= 8)
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
+            for (int j = 3; j >= 0; --j) {
                 const int t = kb + 4 * hf + j;
                 s = mfma2(bf2f(Os[t][ln]) * (gg[t] * qscale), bf2f(Qs[t][32 * wave + ln]), s);
                 s = mfma2(-Us[t][ln], Ws[t][32 * wave + ln], s);
@@ -418,7 +438,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
     __shared__ __attribute__((aligned(16))) float M1[GC][LM];      // dR; later d(K K^T) + its transpose
     __shared__ __attribute__((aligned(16))) float M2[GC][LM];      // R
     __shared__ double gd[GC];
-    __shared__ float be[GC], al[GC], gam[GC], gp[GC], redG[4][GC], redP[4][GC], bc[2][GC], br[2][GC], dss[4];
+    __shared__ float be[GC], al[GC], gam[GC], gp[GC], redG[4][GC], redP[4][GC], redB[4][GC], dss[4];
     float(*M3)[LZ] = reinterpret_cast<float(*)[LZ]>(&Z[0][0]);
     float(*ME)[LZ] = reinterpret_cast<float(*)[LZ]>(&Z[0][0] + GC * LZ);
     static_assert(2 * GC * LZ <= GC * (GD + 4), "both late matrices fit the early one's space");
@@ -438,7 +458,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
         float a;
         gd[lane] = cumulated_log(alpha, (tok0 + lane) * Hv + h, lane < cnt, a);
         al[lane] = a;
-        be[lane] = lane < cnt ? beta[(tok0 + lane) * Hv + h] : 0.f;
+        be[lane] = beta_of(beta, (tok0 + lane) * Hv + h, lane < cnt);
         gam[lane] = blk[G_GAM + lane];
         gp[lane] = blk[G_GAM + GC + lane];
     }
@@ -473,7 +493,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
     const int ti = wave >> 1, tj = wave & 1, j0 = 32 * tj + ln;
     f32x16 lkk, e1, dqk;
     {
-        f32x16 kk = zero16(), qk = zero16(), dP = zero16(), dT = zero16(), tz = zero16();
+        f32x16 kk = zero16(), qk = zero16(), dP = zero16(), dT = zero16(), tz = zero16(), dPt = zero16();
         if (wave != 1) {
             const int ri = 32 * ti + ln, rj = 32 * tj + ln;
 #pragma unroll
@@ -495,30 +515,28 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
                     dT = mfma2(di[j], vj[j], dT);
                     tz = mfma2(zi[j], kj[j], tz);
                 }
+                if ((kb & 24) == 24) add16(dPt, dP);
             }
+            add16(dP, dPt);
         }
         const double gj = gd[j0];
-        float cs = 0.f;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int i = 32 * ti + c_row(e, hf);
             const bool in = i >= j0;
-            const float D = in ? expf((float)(gd[i] - gj)) : 0.f, t = in ? dT[e] + gam[j0] * tz[e] : 0.f, p = in ? qscale * dP[e] : 0.f;
+            const float D = in ? exp_of(gd[i] - gj) : 0.f, t = in ? dT[e] + gam[j0] * tz[e] : 0.f, p = in ? qscale * dP[e] : 0.f;
             lkk[e] = i > j0 ? kk[e] * D : 0.f;
             e1[e] = p * (qk[e] * D);
             dqk[e] = p * D;
-            cs = fmaf(t, M2[i][j0], cs);
             M1[i][j0] = t * be[j0];
         }
-        cs += __shfl_xor(cs, 32, 64);
-        if (hf == 0) bc[ti][j0] = cs;  // d(beta) through T = R diag(beta): column sums
     }
     __syncthreads();
     f32x16 w[2];  // dK, from here on
     {  // dV = T^T dU, d(gam K) = T^T Z: wave = 32 columns
-        f32x16 a[2] = {zero16(), zero16()}, g[2] = {zero16(), zero16()};
+        f32x16 a[2] = {zero16(), zero16()}, g[2] = {zero16(), zero16()}, at = zero16(), gt = zero16();
 #pragma unroll 2
-        for (int kb = 0; kb < GC; kb += 8)
+        for (int kb = 0; kb < GC; kb += 8) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = kb + 4 * hf + j;
@@ -530,11 +548,18 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
                     g[1] = mfma2(r1, bz, g[1]);
                 }
             }
+            if (kb == 24) add16(at, a[0]), add16(gt, g[0]);
+        }
+        add16(a[0], at);
+        add16(g[0], gt);
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int i = 32 * r + c_row(e, hf);
+                // d(beta): what reaches u = beta (v - the state's answer to k) times that difference, which is u / beta
+                const float sb = half_sum(a[r][e] * Up[i * GD + col]);
+                if (ln == 0) redB[wave][i] = sb;
                 if (i < cnt) dv[(tok0 + i) * lddv + (int64_t)h * GD + col] = f2bf(be[i] * a[r][e]);
                 const float d = be[i] * g[r][e];
                 w[r][e] = gam[i] * d;
@@ -570,9 +595,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
         for (int e = 0; e < 16; ++e) {
             const int i = 32 * ti + c_row(e, hf);
             const float d = i > j0 ? -dn[e] : 0.f;
-            const float rs = half_sum(d * lkk[e]);
-            if (ln == 0) br[tj][i] = rs;  // d(beta) through N = I + diag(beta) L: row sums
-            const float dl = be[i] * d, D = i > j0 ? expf((float)(gd[i] - gd[j0])) : 0.f;
+            const float dl = be[i] * d, D = i > j0 ? exp_of(gd[i] - gd[j0]) : 0.f;
             if (i > j0) M1[i][j0] = M1[j0][i] = dl * D;
             else if (i == j0) M1[i][i] = 0.f;
             M3[i][j0] = dqk[e];
@@ -584,7 +607,6 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
             const int i = c_row(e, hf);
             M3[i][j0] = 0.f;
             ME[i][j0] = 0.f;
-            if (ln == 0) br[1][i] = 0.f;
         }
     }
     __syncthreads();
@@ -673,26 +695,27 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
         }
     // d(log alpha_t): every pair (i, j) with j < t <= i, what reaches token i >= t from the chunk's first state, what token j < t leaves in its last, and the state passing through
     if (tid < GC) {
-        float run = 0.f, row[GC];
+        double run = 0.;
+        float row[GC];
 #pragma unroll
         for (int j = 0; j < GC; ++j) row[j] = ME[tid][j];
 #pragma unroll
         for (int j = 0; j < GC; ++j) {
             const float c = row[j];
-            ME[tid][j] = run;  // sum over the columns before j
+            ME[tid][j] = (float)run;  // sum over the columns before j
             run += c;
         }
     }
     __syncthreads();
     if (tid < cnt) {
         const int t = tid;
-        float s = gam[GC - 1] * ((dss[0] + dss[1]) + (dss[2] + dss[3]));
+        double s = gam[GC - 1] * ((dss[0] + dss[1]) + (dss[2] + dss[3]));
         for (int i = 0; i < GC; ++i) {
             if (i >= t) s += ME[i][t] + gam[i] * ((redG[0][i] + redG[1][i]) + (redG[2][i] + redG[3][i]));
             else s += gp[i] * ((redP[0][i] + redP[1][i]) + (redP[2][i] + redP[3][i]));
         }
-        dalpha[(tok0 + t) * Hv + h] = s / al[t];
-        dbeta[(tok0 + t) * Hv + h] = (bc[0][t] + bc[1][t]) + (br[0][t] + br[1][t]);
+        dalpha[(tok0 + t) * Hv + h] = (float)s / al[t];
+        dbeta[(tok0 + t) * Hv + h] = ((redB[0][t] + redB[1][t]) + (redB[2][t] + redB[3][t])) / be[t];
     }
 }
 

@@ -900,6 +900,49 @@ def test_chunked_gated_delta_rule_matches_the_token_by_token_kernels(b, hqk, hv,
         assert bool(torch.isfinite(two.float()).all()) and rel_l2(two, one) < (1e-3 if i < 4 else 2e-6), (i, rel_l2(two, one))
 
 
+@pytest.mark.parametrize("b,hqk,hv,s,decay", [(1, 1, 2, 64, "mix"), (2, 2, 2, 200, "mix"), (1, 1, 1, 333, "slow"), (1, 2, 2, 130, "tiny"), (1, 1, 2, 190, "zero"), (1, 2, 2, 128, "keys")])
+def test_chunked_gated_delta_rule_is_as_near_to_fp64_as_the_token_by_token_kernels(b, hqk, hv, s, decay):
+    """Forward and backward of both sets of kernels against the recurrence in fp64 and its autograd.  bf16 results: the rounding to bf16 is all that shows, so the two distances are the
+    same (1 % beside it).  fp32 results: chains of 32 ... 128 fp32 sums, each rounding at most 2^-24 of a partial sum, some behind 63 steps of substitution: 1e-6 holds
+    sqrt(128) of them and the amplification of nearly parallel keys.  ``zero``: decays and betas of exactly zero (they count as 1e-30)."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    g = torch.Generator().manual_seed(3 * s + hv)
+    D = 128
+    keys = torch.randn(b, s, hqk, D, generator=g) + (3.0 if decay == "keys" else 0.0)
+    q = torch.nn.functional.normalize(torch.randn(b, s, hqk, D, generator=g), dim=-1).to(BF16).reshape(b * s, -1).cuda()
+    k = torch.nn.functional.normalize(keys, dim=-1).to(BF16).reshape(b * s, -1).cuda()
+    v, go = (torch.randn(b * s, hv * D, generator=g).to(BF16).cuda() for _ in range(2))
+    be = torch.sigmoid(torch.randn(b * s, hv, generator=g)).cuda()
+    al = torch.exp(-torch.exp({"slow": -9.0, "tiny": 1.0}.get(decay, -3.0) + 2.0 * torch.rand(b * s, hv, generator=g))).cuda()
+    if decay == "zero":
+        al[5::9], be[3::11] = 0.0, 0.0
+    s0, gs = ((0.1 * torch.randn(b, hv, D, D, generator=g)).cuda() for _ in range(2))
+
+    heads = lambda t, h: t.double().view(b, s, h, -1).permute(0, 2, 1, 3).clone().requires_grad_(True)
+    q6, k6, v6, be6, al6 = heads(q, hqk), heads(k, hqk), heads(v, hv), heads(be, hv), heads(al, hv)
+    s6 = s0.double().requires_grad_(True)
+    qr, kr, st, outs = q6.repeat_interleave(hv // hqk, 1), k6.repeat_interleave(hv // hqk, 1), s6, []
+    for t in range(s):
+        st = st * al6[:, :, t, :, None]
+        st = st + (be6[:, :, t] * (v6[:, :, t] - (st * kr[:, :, t, None, :]).sum(-1)))[..., None] * kr[:, :, t, None, :]
+        outs.append((st * qr[:, :, t, None, :]).sum(-1) / D**0.5)
+    o6 = torch.stack(outs, 2)
+    ((o6 * go.double().view(b, s, hv, D).permute(0, 2, 1, 3)).sum() + (st * gs.double()).sum()).backward()
+    rows = lambda t: t.detach().permute(0, 2, 1, 3).reshape(b * s, -1)
+    want = [rows(o6), rows(q6.grad), rows(k6.grad), rows(v6.grad), st.detach(), rows(be6.grad), rows(al6.grad), s6.grad]
+    dist = []
+    for chunked in (False, None):
+        o, ck, fin = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, hqk, hv, D, D, state=s0.clone(), chunked=chunked)
+        dv = torch.empty_like(v)
+        dq, dk, dbe, dal, d0 = Q.gated_delta_rule_bwd(q, k, v, be, al, ck, go, dv, b, s, hqk, hv, D, D, d_final=gs, want_d_initial=True)
+        dist.append([rel_l2(x, w) for x, w in zip((o, dq, dk, dv, fin, dbe, dal, d0), want)])
+    for i, (one, two) in enumerate(zip(*dist)):
+        if i == 7 and decay == "zero":  # behind a decay of zero the first state's gradient is zero itself (here 1e-30 of what it was)
+            continue
+        assert two < (1.01 * one if i < 4 else 1e-6), (i, one, two)
+
+
 def test_chunked_gated_delta_rule_refuses_what_it_cannot_read():
     from llm_quest_amd import _lib as L
     from llm_quest_amd import kernels_q35 as Q
