@@ -654,13 +654,10 @@ int mi355_qkv_rows_append(int64_t tokens, int H, int G, int d, int dv, const voi
 int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
                             int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
                             const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream);
-/* The same for the sequences with fewer than `below` new tokens alone (0: all of them); ws is filled for every row of the step. */
-int mi355_delta_rule_ragged_below(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
-                            int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
-                            const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, int below, void* stream);
 /* The same rule -- or, with head_decay, linear attention with one decay per head (k times kscale, q times qscale) -- in chunks of 64 tokens on the fp32 matrix pipe:
  * heads of 128 | 128, fp32 rows, state fp32 [slots, H, 128, 128] read and written at slot.  tok: mi355_delta_rule_tokens' result (four floats per token and head).
- * max_new: the most new tokens of one sequence; sequences with fewer than `from` are left as they are (their kernels: the _below entries).  A fixed decay lies at 1e-30
+ * max_new: the most new tokens of one sequence; sequences with fewer than `from` go token by token under tok, and are
+ * left as they are under head_decay (mi355_gla_fwd_below takes them).  A fixed decay lies at 1e-30
  * or above (what is below counts as 1e-30).  workspace: mi355_delta_chunked_workspace_bytes, 16-byte aligned. */
 int mi355_delta_rule_tokens(int64_t tokens, int H, int G, int dk, const void* q, const void* k, int qk_dt, int64_t ldq, int64_t ldk, const void* b, const void* a, int ba_dt,
                             int64_t ldb, int64_t lda, const float* A_log, const float* dt_bias, float qscale, float* ws, void* stream);

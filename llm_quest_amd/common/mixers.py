@@ -565,7 +565,7 @@ class GatedDeltaRule(_Frozen):
         a, b = G * dk, 2 * G * dk
         gate0 = C + H * dv
         o = S.delta_rule(qkv[:, :a], qkv[:, a:b], qkv[:, b:], proj[:, gate0 : gate0 + H], proj[:, gate0 + H :], self.A_log32, self.dt_bias32, dk ** -0.5, st.seq_off, st.slots,
-                         st.cache.state(self.layer_idx, "S"), H, G, dk, dv, max_new=st.max_new, min_new=st.min_new)
+                         st.cache.state(self.layer_idx, "S"), H, G, dk, dv, max_new=st.max_new)
         mix = S.gated_headnorm(o, self.norm32, proj[:, C:gate0], H, dv, self.eps, st.act_dtype)
         return S.linear(mix, self.w_o)
 

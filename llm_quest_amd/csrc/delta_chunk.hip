@@ -3,11 +3,13 @@
 // here operands are fp32 rows of a packed batch, the state is [dk][dv] per slot, and nothing is kept for a backward pass.
 //     delta:      U = R (b V) - Kw S,  O = gam q S + P U,  S <- gam_63 S + (Gp K)^T U
 //     retention:  U = V,               the same
-// Which sequences of a step go this way is their own number of new tokens' affair (`from`): beside a long prompt, a short one and a single token take the kernel they take alone.
+// Which sequences of a step go this way is their own number of new tokens' affair (`from`): beside a long prompt, a short one and a single token
+// get the bits that they get alone -- of the delta rule inside the scan's launch, whose long chains hide them; of retention by mi355_gla_fwd_below.
 // A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
 // the chip could multiply; the chunks take 363 us (prep 142, scan 203) and 183 us (scan 173).  Bound: the scan's chain of chunks (two products behind two barriers each), not the
 // pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
 // (A row that is not finite makes the rows before it in its own chunk NaN as well: the triangle's zeros are multiplied, not skipped.  The rows after it are lost either way.)
+#include "delta_token.h"
 #include "gdr_chunk.h"
 
 #define ST(s) ((hipStream_t)(s))
@@ -25,7 +27,7 @@ struct DChunkArgs {
     const float* head_decay;  // retention: [H]
     float qscale, kscale;     // retention
     int H, G, heads;  // heads: of all sequences
-    int from;         // sequences with fewer new tokens are another kernel's
+    int from;         // sequences with fewer new tokens: retention leaves them alone, the delta rule goes token by token
     float *state, *o, *ws;
 };
 
@@ -144,7 +146,17 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
     const bool qside = wave >= 2;
     const float *qp = p.q + (int64_t)s0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)s0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)s0 * p.ldv + (int64_t)h * GD + v0;
     float* state = p.state + ((int64_t)p.slot[s] * p.H + h) * GD * GD + v0;
-    if (NC <= 0 || len < p.from) return;
+    if (NC <= 0) return;
+    if (len < p.from) {
+        if constexpr (DELTA) {
+            DeltaArgs d = {};
+            d.seq_off = p.seq_off, d.slot = p.slot, d.q = p.q, d.k = p.k, d.v = p.v, d.ldq = p.ldq, d.ldk = p.ldk, d.ldv = p.ldv, d.ws = const_cast<f32x4*>(p.tok);
+            d.H = p.H, d.G = p.G, d.dk = d.dv = GD, d.qk_dt = d.v_dt = MI355_DT_F32, d.state = p.state, d.o = p.o;
+            static_assert(GV == 4 * (64 / DR_LPR) && GD == 16 * DR_LPR, "a workgroup's columns and a lane's channels there and here");
+            delta_rule_columns<16, true>(d, s, h, v0 + wave * (64 / DR_LPR));
+        }
+        return;
+    }
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;

@@ -6,11 +6,11 @@
 // Conventions as in seqmix.hip: operands come as bf16 or fp32 (a MI355_DT_* code each); the residual stream, norm statistics, rotary angles, decays,
 // gates of a recurrence and recurrent state are fp32 in both modes.  A "row" is a token of the packed batch; sequences are described by int32 device arrays.
 #include "common.h"
+#include "delta_token.h"
 #include "lane_sums.h"
 
 #define ST(s) ((hipStream_t)(s))
 
-__device__ __forceinline__ float ldr_dt(const void* p, int dt, int64_t i) { return dt == MI355_DT_F32 ? ((const float*)p)[i] : bf2f(((const bf16_t*)p)[i]); }
 __device__ __forceinline__ void str_dt(void* p, int dt, int64_t i, float v) {
     if (dt == MI355_DT_F32) ((float*)p)[i] = v;
     else ((bf16_t*)p)[i] = f2bf(v);
@@ -545,27 +545,7 @@ extern "C" int mi355_qkv_rows_append(int64_t tokens, int H, int G, int d, int dv
 }
 
 // ------------------------------------------------------------------------------------------- gated delta rule, ragged, carried state
-// Per value head h a state S [dk, dv] (fp32, carried per sequence slot); its query / key head is h / (H / G).  Per token:
-//   k^ = k / sqrt(sum k^2 + 1e-6), q^ = q / sqrt(sum q^2 + 1e-6) * qscale   (unit vectors; raw q / k rows come in)
-//   beta = sigmoid(b), g = exp(-exp(A_log[h]) * softplus(a + dt_bias[h]))
-//   S <- g S;  u = beta (v - S^T k^);  S <- S + k^ u^T;  o = S^T q^
-// Column c of S obeys its own recurrence, so columns are spread over lanes and the time loop stays inside: DR_LPR lanes share a column (CPL key
-// channels each, in registers), the two dot products of a step close with lane sums -- no LDS, no barrier.  The per-token scalars (g, beta and the two
-// unit-vector factors, which multiply the dot products instead of the rows) are prepared once per (token, head) by delta_prep_kernel; the operands of
-// step t + 1 are requested before step t's arithmetic.
-#define DR_LPR 8
-struct DeltaArgs {
-    const int *seq_off, *slot;
-    const void *q, *k, *v, *b, *a;
-    const float *A_log, *dt_bias;
-    float *state, *o;
-    f32x4* ws;  // [tokens, H]: g, beta, key factor, query factor * qscale
-    int64_t ldq, ldk, ldv, ldb, lda;
-    int H, G, dk, dv, qk_dt, v_dt, ba_dt;
-    float qscale;
-    int below;  // 0: every sequence; else those with fewer new tokens
-};
-
+// (delta_token.h: the rule, and what a workgroup does)
 __global__ __launch_bounds__(256) void delta_prep_kernel(int64_t T, DeltaArgs p) {
     const int lane = threadIdx.x & 63;
     const int64_t items = T * p.H;
@@ -590,85 +570,8 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(int64_t T, DeltaArgs p)
 
 template <int CPL, bool VEC>
 __global__ __launch_bounds__(256) void delta_rule_kernel(DeltaArgs p) {
-    constexpr int RPW = 64 / DR_LPR;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int s = blockIdx.z, h = blockIdx.y;
-    const int col0 = (blockIdx.x * 4 + wave) * RPW;
-    if (col0 >= p.dv) return;  // whole wave out of range; no block-level synchronisation below
-    const int col = col0 + lane / DR_LPR, cg = lane % DR_LPR, ch0 = cg * CPL;
-    const bool col_ok = col < p.dv;
-    const int hq = h / (p.H / p.G), dk = p.dk;
-    const int t0 = p.seq_off[s], t1 = p.seq_off[s + 1];
-    if (p.below && t1 - t0 >= p.below) return;
-    float* S = p.state + (((int64_t)p.slot[s] * p.H + h) * dk) * p.dv;
-    float st[CPL];
-#pragma unroll
-    for (int i = 0; i < CPL; ++i) st[i] = (col_ok && ch0 + i < dk) ? S[(int64_t)(ch0 + i) * p.dv + col] : 0.f;
-    struct In {
-        float k[CPL], q[CPL];
-        f32x4 sc;
-        float v;
-    };
-    auto load_in = [&](In& in, int t) {
-        const int64_t ko = (int64_t)t * p.ldk + (int64_t)hq * dk + ch0, qo = (int64_t)t * p.ldq + (int64_t)hq * dk + ch0;
-        if (VEC) {
-#pragma unroll
-            for (int i = 0; i < CPL; i += 4) {
-                f32x4 kv = {0.f, 0.f, 0.f, 0.f}, qv = {0.f, 0.f, 0.f, 0.f};
-                if (ch0 + i < dk) {
-                    kv = *(const f32x4*)((const float*)p.k + ko + i);
-                    qv = *(const f32x4*)((const float*)p.q + qo + i);
-                }
-#pragma unroll
-                for (int e = 0; e < 4; ++e) in.k[i + e] = kv[e], in.q[i + e] = qv[e];
-            }
-        } else {
-#pragma unroll
-            for (int i = 0; i < CPL; ++i) {
-                const bool ok = ch0 + i < dk;
-                in.k[i] = ok ? ldr_dt(p.k, p.qk_dt, ko + i) : 0.f;
-                in.q[i] = ok ? ldr_dt(p.q, p.qk_dt, qo + i) : 0.f;
-            }
-        }
-        in.sc = p.ws[(int64_t)t * p.H + h];
-        in.v = col_ok ? ldr_dt(p.v, p.v_dt, (int64_t)t * p.ldv + (int64_t)h * p.dv + col) : 0.f;
-    };
-    auto step = [&](const In& in, int t) {
-        const float a = in.sc[0], b = in.sc[1], kn = in.sc[2], qn = in.sc[3];
-        float u0 = 0.f, u1 = 0.f;
-#pragma unroll
-        for (int i = 0; i < CPL; i += 2) {
-            st[i] *= a;
-            st[i + 1] *= a;
-            u0 = fmaf(st[i], in.k[i], u0);
-            u1 = fmaf(st[i + 1], in.k[i + 1], u1);
-        }
-        const float u = lanes_sum<DR_LPR>(u0 + u1) * kn;
-        const float c = b * (in.v - u) * kn;
-        float o0 = 0.f, o1 = 0.f;
-#pragma unroll
-        for (int i = 0; i < CPL; i += 2) {
-            st[i] = fmaf(c, in.k[i], st[i]);
-            st[i + 1] = fmaf(c, in.k[i + 1], st[i + 1]);
-            o0 = fmaf(st[i], in.q[i], o0);
-            o1 = fmaf(st[i + 1], in.q[i + 1], o1);
-        }
-        const float oo = lanes_sum<DR_LPR>(o0 + o1) * qn;
-        if (cg == 0 && col_ok) p.o[(int64_t)t * p.H * p.dv + (int64_t)h * p.dv + col] = oo;
-    };
-    In inA, inB;
-    if (t0 < t1) load_in(inA, t0);
-    for (int t = t0; t < t1; t += 2) {
-        if (t + 1 < t1) load_in(inB, t + 1);
-        step(inA, t);
-        if (t + 1 < t1) {
-            if (t + 2 < t1) load_in(inA, t + 2);
-            step(inB, t + 1);
-        }
-    }
-#pragma unroll
-    for (int i = 0; i < CPL; ++i)
-        if (col_ok && ch0 + i < dk) S[(int64_t)(ch0 + i) * p.dv + col] = st[i];
+    const int col0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / DR_LPR);
+    if (col0 < p.dv) delta_rule_columns<CPL, VEC>(p, blockIdx.z, blockIdx.y, col0);
 }
 
 template <int CPL>
@@ -677,10 +580,10 @@ static void launch_delta(const DeltaArgs& p, dim3 grid, bool vec, hipStream_t st
     else delta_rule_kernel<CPL, false><<<grid, 256, 0, st>>>(p);
 }
 
-extern "C" int mi355_delta_rule_ragged_below(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
+extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
                                        int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
-                                       const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, int below, void* stream) {
-    MI355_REQUIRE(below >= 0 && tokens > 0 && n_seq > 0 && n_seq <= 65535 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 32 * DR_LPR && dv > 0 && q && k && v &&
+                                       const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream) {
+    MI355_REQUIRE(tokens > 0 && n_seq > 0 && n_seq <= 65535 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && dk > 0 && dk <= 32 * DR_LPR && dv > 0 && q && k && v &&
                       b && a && A_log && dt_bias && state && o && ws,
                   "delta_rule_ragged: bad arguments (key channels per head <= 256, value heads a multiple of the query / key heads, workspace of 4 floats per token and head)");
     MI355_REQUIRE(rec_dt_ok(qk_dt) && rec_dt_ok(v_dt) && rec_dt_ok(ba_dt) && ldq >= (int64_t)G * dk && ldk >= (int64_t)G * dk && ldv >= (int64_t)H * dv && ldb >= H && lda >= H,
@@ -688,7 +591,7 @@ extern "C" int mi355_delta_rule_ragged_below(int64_t tokens, int n_seq, const in
     MI355_REQUIRE(((uintptr_t)ws & 15) == 0, "delta_rule_ragged: the workspace must be 16-byte aligned");
     DeltaArgs p;
     p.seq_off = seq_off, p.slot = slot, p.q = q, p.k = k, p.v = v, p.b = b, p.a = a, p.A_log = A_log, p.dt_bias = dt_bias, p.state = state, p.o = o, p.ws = (f32x4*)ws;
-    p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.ldb = ldb, p.lda = lda, p.H = H, p.G = G, p.dk = dk, p.dv = dv, p.qk_dt = qk_dt, p.v_dt = v_dt, p.ba_dt = ba_dt, p.qscale = qscale, p.below = below;
+    p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.ldb = ldb, p.lda = lda, p.H = H, p.G = G, p.dk = dk, p.dv = dv, p.qk_dt = qk_dt, p.v_dt = v_dt, p.ba_dt = ba_dt, p.qscale = qscale;
     delta_prep_kernel<<<rec_rows_grid(tokens * H, 4), 256, 0, ST(stream)>>>(tokens, p);
     MI355_LAUNCH_CHECK("delta_rule_ragged(prep)");
     const bool vec = qk_dt == MI355_DT_F32 && dk % 4 == 0 && ldq % 4 == 0 && ldk % 4 == 0 && ((uintptr_t)q & 15) == 0 && ((uintptr_t)k & 15) == 0;
@@ -699,12 +602,6 @@ extern "C" int mi355_delta_rule_ragged_below(int64_t tokens, int n_seq, const in
     else launch_delta<32>(p, grid, vec, ST(stream));
     MI355_LAUNCH_CHECK("delta_rule_ragged");
     return 0;
-}
-
-extern "C" int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const int* slot, int H, int G, int dk, int dv, const void* q, const void* k, int qk_dt,
-                                       int64_t ldq, int64_t ldk, const void* v, int v_dt, int64_t ldv, const void* b, const void* a, int ba_dt, int64_t ldb, int64_t lda,
-                                       const float* A_log, const float* dt_bias, float qscale, float* state, float* o, float* ws, void* stream) {
-    return mi355_delta_rule_ragged_below(tokens, n_seq, seq_off, slot, H, G, dk, dv, q, k, qk_dt, ldq, ldk, v, v_dt, ldv, b, a, ba_dt, ldb, lda, A_log, dt_bias, qscale, state, o, ws, 0, stream);
 }
 
 // The per-token numbers alone (the chunked kernels of delta_chunk.hip take them): ws [tokens, H] x {decay, beta, key factor, query factor x qscale}.

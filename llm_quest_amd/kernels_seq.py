@@ -443,9 +443,9 @@ def qkv_rows_append(src, H, G, d, dv, bias, qw, kw, eps, qscale, dims, layout, f
     return q
 
 
-def delta_rule(q, k, v, b, a, A_log, dt_bias, qscale, seq_off, slot, state, H, G, dk, dv, max_new=0, min_new=0):
-    """Gated delta rule over a ragged batch (raw q / k rows: made unit vectors inside); ``state`` fp32 [slots, H, dk, dv].  Returns fp32 [tokens, H * dv].  ``max_new`` and
-    ``min_new``: the most and the least new tokens of one sequence of the step (0: not known); where the most is known, long sequences go in chunks."""
+def delta_rule(q, k, v, b, a, A_log, dt_bias, qscale, seq_off, slot, state, H, G, dk, dv, max_new=0):
+    """Gated delta rule over a ragged batch (raw q / k rows: made unit vectors inside); ``state`` fp32 [slots, H, dk, dv].  Returns fp32 [tokens, H * dv].  ``max_new``: the most
+    new tokens of one sequence of the step (0: not known); where it is known, long sequences go in chunks."""
     L.require_gpu(q, k, v, b, a, A_log, dt_bias, seq_off, slot, state)
     T = q.shape[0]
     for t, n, w in ((q, "q", G * dk), (k, "k", G * dk), (v, "v", H * dv), (b, "b", H), (a, "a", H)):
@@ -464,15 +464,12 @@ def delta_rule(q, k, v, b, a, A_log, dt_bias, qscale, seq_off, slot, state, H, G
             raise ValueError("delta_rule: A_log and dt_bias fp32 [H]")
     o = torch.empty((T, H * dv), dtype=F32, device=q.device)
     ws = torch.empty((T * H * 4,), dtype=F32, device=q.device)  # per token and head: decay, beta, the two unit-vector factors
-    chunked = _delta_chunked(q, k, v, dk, dv, max_new)
-    if not chunked or min_new < DELTA_CHUNKED_MIN:
-        L.call("mi355_delta_rule_ragged_below", T, n_seq, L.ptr(seq_off), L.ptr(slot), H, G, dk, dv, L.ptr(q), L.ptr(k), _dt(q), q.stride(0), k.stride(0), L.ptr(v), _dt(v), v.stride(0),
-               L.ptr(b), L.ptr(a), _dt(b), b.stride(0), a.stride(0), L.ptr(A_log), L.ptr(dt_bias), float(qscale), L.ptr(state), L.ptr(o), L.ptr(ws), DELTA_CHUNKED_MIN if chunked else 0)
-    else:
+    if _delta_chunked(q, k, v, dk, dv, max_new):
         L.call("mi355_delta_rule_tokens", T, H, G, dk, L.ptr(q), L.ptr(k), _dt(q), q.stride(0), k.stride(0), L.ptr(b), L.ptr(a), _dt(b), b.stride(0), a.stride(0), L.ptr(A_log), L.ptr(dt_bias),
                float(qscale), L.ptr(ws))
-    if chunked:
-        _run_chunked(q, k, v, ws, None, 1.0, 1.0, seq_off, slot, state, o, H, G, max_new)
+        return _run_chunked(q, k, v, ws, None, 1.0, 1.0, seq_off, slot, state, o, H, G, max_new)
+    L.call("mi355_delta_rule_ragged", T, n_seq, L.ptr(seq_off), L.ptr(slot), H, G, dk, dv, L.ptr(q), L.ptr(k), _dt(q), q.stride(0), k.stride(0), L.ptr(v), _dt(v), v.stride(0),
+           L.ptr(b), L.ptr(a), _dt(b), b.stride(0), a.stride(0), L.ptr(A_log), L.ptr(dt_bias), float(qscale), L.ptr(state), L.ptr(o), L.ptr(ws))
     return o
 
 

@@ -426,7 +426,7 @@ def test_recurrences_of_a_sequence_do_not_know_what_shares_the_step(rule, H, G):
     def run(rows, desc, state, n):
         q, k, v = x[rows, : G * D], x[rows, G * D : 2 * G * D], x[rows, 2 * G * D :]
         if rule == "delta":
-            return S.delta_rule(q, k, v, ba[rows, :H], ba[rows, H:], A_log, dt_bias, D ** -0.5, desc.seq_off, desc.slots, state, H, G, D, D, max_new=max(n), min_new=min(n))
+            return S.delta_rule(q, k, v, ba[rows, :H], ba[rows, H:], A_log, dt_bias, D ** -0.5, desc.seq_off, desc.slots, state, H, G, D, D, max_new=max(n))
         return S.gla(q, k, v, None, None, 1.0, 1.0, desc.seq_off, desc.slots, state, H, D, D, head_decay=dec, kscale=D ** -0.5, max_new=max(n), min_new=min(n))
 
     together = start.clone()
