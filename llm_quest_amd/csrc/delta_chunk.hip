@@ -8,6 +8,8 @@
 // A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
 // the chip could multiply; the chunks take 363 us (prep 142, scan 203) and 183 us (scan 173).  Bound: the scan's chain of chunks (two products behind two barriers each), not the
 // pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
+// Chains of 128 products on the matrix pipe are cut (add16): outputs' distance to 64 bits, token by token | here with whole chains | here: 1.29e-7 | 2.32e-7 | 1.73e-7, decays near zero
+// 1.19e-7 | 2.27e-7 | 1.45e-7, nearly parallel keys 1.29e-7 | 2.67e-7 | 1.90e-7, decays near one 4.7e-7 | 5.0e-7 | 4.7e-7, retention 3.1e-7 | 3.0e-7 | 2.6e-7; the six prompts 363 -> 369 us.
 // (A row that is not finite makes the rows before it in its own chunk NaN as well: the triangle's zeros are multiplied, not skipped.  The rows after it are lost either way.)
 #include "delta_token.h"
 #include "gdr_chunk.h"
@@ -55,11 +57,11 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
         const double g = cumulated_log64(decay_at_least(c[0])), g63 = __shfl(g, 63, 64);
         gd[lane] = g;
         be[lane] = c[1];
-        gam[lane] = expf((float)g);
+        gam[lane] = exp_of(g);
         qf[lane] = c[3];
-        blk[D_G + lane] = expf((float)g) * c[3];
-        blk[D_G + GC + lane] = expf((float)(g63 - g)) * c[2];
-        if (lane == 0) blk[D_G + 2 * GC] = expf((float)g63);
+        blk[D_G + lane] = exp_of(g) * c[3];
+        blk[D_G + GC + lane] = exp_of(g63 - g) * c[2];
+        if (lane == 0) blk[D_G + 2 * GC] = exp_of(g63);
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {  // keys, made unit vectors (resp. scaled) on the way
@@ -71,7 +73,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
     __syncthreads();
     {  // K K^T and Q K^T: wave = tile (ti, tj); the tile above the diagonal is zero
         const int ti = wave >> 1, tj = wave & 1;
-        f32x16 kk = zero16(), qk = zero16();
+        f32x16 kk = zero16(), qk = zero16(), kkt = zero16(), qkt = zero16();
         if (wave != 1) {
             const int qr = 32 * ti + ln;
 #pragma unroll 4
@@ -84,14 +86,19 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
                     qk = mfma2(qv[j], bv[j], qk);
                     if (DELTA) kk = mfma2(av[j], bv[j], kk);
                 }
+                if ((c & 24) == 24) {
+                    add16(qkt, qk);
+                    if (DELTA) add16(kkt, kk);
+                }
             }
+            qk = qkt, kk = kkt;
         }
         const int j = 32 * tj + ln;
         const double gj = gd[j];
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int i = 32 * ti + c_row(e, hf);
-            const float D = i >= j ? expf((float)(gd[i] - gj)) : 0.f;
+            const float D = i >= j ? exp_of(gd[i] - gj) : 0.f;
             if (DELTA) N[i][j] = i > j ? be[i] * kk[e] * D : 0.f;
             blk[D_P + i * GC + j] = i >= j ? qf[i] * qk[e] * D : 0.f;
         }
@@ -100,7 +107,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
         __syncthreads();
         invert_unit_lower64(N, T);
         // Uv = R (b V), Kw = R (b gam K): wave = 32 columns, both row halves (the upper one ends at token 32)
-        f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16();
+        f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16(), ut = zero16(), wt = zero16();
         const int col = 32 * wave + ln;
 #pragma unroll 2
         for (int kb = 0; kb < GC; kb += 8) {
@@ -118,7 +125,10 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
                     w0 = mfma2(a0[j], bk, w0);
                 }
             }
+            if (kb == 24) add16(ut, u1), add16(wt, w1);
         }
+        add16(u1, ut);
+        add16(w1, wt);
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int r = c_row(e, hf);
@@ -174,7 +184,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
         for (int i = 0; i < 8; ++i) fr[i] = src ? *reinterpret_cast<const f32x4*>(src + 8 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
         __syncthreads();  // the state is whole, the last chunk's keys and U are read
         f32x4 kr[8], pr[8];
-        float uv[16];
+        f32x16 uv = zero16();
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
             const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
@@ -197,6 +207,13 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
                 const f32x4 c = *reinterpret_cast<const f32x4*>(&Ss[ln][8 * i + 4 * hf]);
 #pragma unroll
                 for (int j = 0; j < 4; ++j) acc = mfma2(fr[i % 8][j], c[j], acc);
+                if (i == 7) {  // (as add16: what is left of U, or minus the first half of q S)
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        uv[e] -= acc[e];
+                        acc[e] = 0.f;
+                    }
+                }
                 if (i < 8) fr[i] = src ? *reinterpret_cast<const f32x4*>(src + 8 * (i + 8)) : f32x4{0.f, 0.f, 0.f, 0.f};
                 if (i % 4 == 3) asm volatile("" ::: "memory");  // keep the state reads of later steps where they are: all sixteen at once cost more registers than there are
             }
@@ -216,7 +233,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
         __syncthreads();
         if (qside) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] *= gg[32 * rh + c_row(e, hf)];
+            for (int e = 0; e < 16; ++e) acc[e] = (acc[e] - uv[e]) * gg[32 * rh + c_row(e, hf)];
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
                 if (rh == 0 && i >= 4) break;  // P is lower triangular

@@ -438,6 +438,33 @@ def test_recurrences_of_a_sequence_do_not_know_what_shares_the_step(rule, H, G):
         assert torch.equal(alone[slots[i]], together[slots[i]]), f"state in slot {slots[i]}"
 
 
+@pytest.mark.parametrize("offset,rate", [(0.0, 3.0), (0.0, -2.0), (3.0, -2.0)])
+def test_delta_rule_in_chunks_is_about_as_near_to_fp64_as_by_token(offset, rate):
+    """Outputs of the chunked delta rule and of the one by token against fp64 (decays near zero; all kinds; nearly parallel keys).  A chunk's outputs have two more products of 128 terms
+    behind them than a token's; cut into runs of 32 their roundings stay below the others' (sqrt(32) of 2^-24 each, beside sqrt(128)): a distance within 1.6 of the token's."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(17)
+    H, G, D, T = 4, 2, 128, 150
+    x = torch.randn(T, (2 * G + H) * D, generator=g)
+    x[:, G * D : 2 * G * D] += offset
+    ba, start, A = torch.randn(T, 2 * H, generator=g) * 2, torch.randn(1, H, D, D, generator=g), torch.full((H,), rate)
+    w, st, want = x.double(), start[0].double(), torch.empty(T, H, D, dtype=F64)
+    for t in range(T):
+        qt, kt = (w[t, lo * D : hi * D].view(G, D).repeat_interleave(H // G, 0) for lo, hi in ((0, G), (G, 2 * G)))
+        qt, kt = (z / torch.sqrt((z ** 2).sum(-1, keepdim=True) + 1e-6) for z in (qt, kt))
+        st = st * torch.exp(-torch.exp(A.double()) * torch.nn.functional.softplus(ba[t, H:].double()))[:, None, None]
+        st = st + kt[:, :, None] * (torch.sigmoid(ba[t, :H].double())[:, None] * (w[t, 2 * G * D :].view(H, D) - (kt[:, :, None] * st).sum(1)))[:, None, :]
+        want[t] = (qt[:, :, None] * st).sum(1) * D ** -0.5
+    d, x, ba = _Slots([T]), x.to(DEV), ba.to(DEV)
+    dist = []
+    for n in (0, T):
+        o = S.delta_rule(x[:, : G * D], x[:, G * D : 2 * G * D], x[:, 2 * G * D :], ba[:, :H], ba[:, H:], A.to(DEV), torch.zeros(H, device=DEV), D ** -0.5, d.seq_off, d.slots,
+                         start.clone().to(DEV), H, G, D, D, max_new=n)
+        dist.append(float((o.double().cpu().view(T, H, D) - want).norm() / want.norm()))
+    assert dist[1] < 1.6 * dist[0], dist
+
+
 def test_retention_with_any_fixed_decay_does_not_know_how_a_prompt_is_cut():
     """Decays that have no logarithm (negative, zero), one below what the chunks of tokens hold and one above one, heads of 128 | 128: a prompt of more than a chunk is the same rows as
     in two short portions (fp32 sums of 128 channels in the same order, equal up to the tiles of the products around them: 1e-5 as above; states head by head, their sizes are far apart)."""
