@@ -10,7 +10,8 @@
 // pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
 // Chains of 128 products on the matrix pipe are cut (add16): outputs' distance to 64 bits, token by token | here with whole chains | here: 1.29e-7 | 2.32e-7 | 1.73e-7, decays near zero
 // 1.19e-7 | 2.27e-7 | 1.45e-7, nearly parallel keys 1.29e-7 | 2.67e-7 | 1.90e-7, decays near one 4.7e-7 | 5.0e-7 | 4.7e-7, retention 3.1e-7 | 3.0e-7 | 2.6e-7; the six prompts 363 -> 369 us.
-// (A row that is not finite makes the rows before it in its own chunk NaN as well: the triangle's zeros are multiplied, not skipped.  The rows after it are lost either way.)
+// A chunk whose U is not finite and all behind it go token by token inside the scan: the triangles' zeros are multiplied, not skipped, and a token's key, value, decay or beta that
+// is not finite would reach the rows before it.  (A query reaches its own row alone, a key under retention the rows behind it.)
 #include "delta_token.h"
 #include "gdr_chunk.h"
 
@@ -148,6 +149,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
     __shared__ __attribute__((aligned(16))) float Us[GC][GV + 8];
     __shared__ __attribute__((aligned(16))) float Ks[GC][GD + 4];
     __shared__ float gg[2 * GC], gC;
+    __shared__ int lost[2];  // a chunk's flag: set by its U, cleared a chunk later
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
     // the four value ranges of a head read the same rows: to one XCD (workgroups are dealt to the eight XCDs in turn), side by side
     const int id = blockIdx.x, at = (id >> 5) * 8 + (id & 7), v0 = ((id >> 3) & 3) * GV;
@@ -157,22 +159,27 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
     const float *qp = p.q + (int64_t)s0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)s0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)s0 * p.ldv + (int64_t)h * GD + v0;
     float* state = p.state + ((int64_t)p.slot[s] * p.H + h) * GD * GD + v0;
     if (NC <= 0) return;
+    auto by_token = [&](int ta, int tb, float* S, int64_t s_ch, int64_t s_col) {  // S: from this workgroup's first column on
+        DeltaArgs d = {};
+        d.q = p.q, d.k = p.k, d.v = p.v, d.ldq = p.ldq, d.ldk = p.ldk, d.ldv = p.ldv, d.ws = const_cast<f32x4*>(p.tok), d.o = p.o;
+        d.H = p.H, d.G = p.G, d.dk = d.dv = GD, d.qk_dt = d.v_dt = MI355_DT_F32;
+        static_assert(GV == 4 * (64 / DR_LPR) && GD == 16 * DR_LPR, "a workgroup's columns and a lane's channels there and here");
+        f32x4 fixed = {};
+        if (!DELTA) fixed = f32x4{p.head_decay[h], 1.f, p.kscale, p.qscale};
+        delta_rule_columns<16, true, DELTA>(d, h, v0 + wave * (64 / DR_LPR), ta, tb, S, s_ch, s_col, v0, fixed);
+    };
     if (len < p.from) {
-        if constexpr (DELTA) {
-            DeltaArgs d = {};
-            d.seq_off = p.seq_off, d.slot = p.slot, d.q = p.q, d.k = p.k, d.v = p.v, d.ldq = p.ldq, d.ldk = p.ldk, d.ldv = p.ldv, d.ws = const_cast<f32x4*>(p.tok);
-            d.H = p.H, d.G = p.G, d.dk = d.dv = GD, d.qk_dt = d.v_dt = MI355_DT_F32, d.state = p.state, d.o = p.o;
-            static_assert(GV == 4 * (64 / DR_LPR) && GD == 16 * DR_LPR, "a workgroup's columns and a lane's channels there and here");
-            delta_rule_columns<16, true>(d, s, h, v0 + wave * (64 / DR_LPR));
-        }
+        if (DELTA) by_token(s0, s0 + len, state, GD, 1);
         return;
     }
+    if (tid < 2) lost[tid] = 0;
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
         const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;
         Ss[c][r] = state[(int64_t)r * GD + c];
     }
-    for (int n = 0; n < NC; ++n) {
+    int n = 0;
+    for (; n < NC; ++n) {
         const float* blk = chunk_block(p, s, h, n);
         const int t0 = n * GC, cnt = min(GC, len - t0);
         // a Kw row (waves 0, 1) or a q row (waves 2, 3) in fragment form, eight words in flight
@@ -199,7 +206,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
             }
         }
         if (tid < 2 * GC) gg[tid] = blk[D_G + tid];
-        if (tid == 0) gC = blk[D_G + 2 * GC];
+        if (tid == 0) gC = blk[D_G + 2 * GC], lost[(n + 1) & 1] = 0;
         f32x16 acc = zero16();
         if (DELTA || qside) {
 #pragma unroll
@@ -228,9 +235,14 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
             for (int i = 0; i < 8; ++i) pr[i] = *reinterpret_cast<const f32x4*>(blk + D_P + (32 * rh + ln) * GC + 8 * i + 4 * hf);
         } else {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) Us[32 * rh + c_row(e, hf)][ln] = uv[e] - acc[e];
+            for (int e = 0; e < 16; ++e) {
+                acc[e] = uv[e] - acc[e];
+                Us[32 * rh + c_row(e, hf)][ln] = acc[e];
+            }
+            if (__any(lost16(acc)) && lane == 0) lost[n & 1] = 1;
         }
         __syncthreads();
+        const int gone = lost[n & 1];
         if (qside) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[e] = (acc[e] - uv[e]) * gg[32 * rh + c_row(e, hf)];
@@ -246,6 +258,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
                 if (r < cnt) p.o[((int64_t)s0 + t0 + r) * p.H * GD + (int64_t)h * GD + v0 + ln] = acc[e];
             }
         }
+        if (gone) break;  // (the same for the whole workgroup)
         f32x16 c;
 #pragma unroll
         for (int e = 0; e < 16; ++e) c[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
@@ -258,6 +271,11 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
             }
 #pragma unroll
         for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = c[e];  // read by this wave alone since the last barrier
+    }
+    if (n < NC) {
+        __threadfence();
+        __syncthreads();  // what the chunk wrote of its outputs lies below what comes
+        by_token(s0 + n * GC, s0 + len, &Ss[0][0], 1, GD + 4);
     }
     __syncthreads();
 #pragma unroll

@@ -26,18 +26,17 @@ struct DeltaArgs {
     float qscale;
 };
 
-// the columns col0 .. col0 + 64 / DR_LPR - 1 of head h of sequence s, one wave; no block-level synchronisation
-template <int CPL, bool VEC>
-__device__ __forceinline__ void delta_rule_columns(const DeltaArgs& p, int s, int h, int col0) {
+// the columns col0 .. col0 + 64 / DR_LPR - 1 of head h over the rows t0 .. t1 - 1, one wave; S: that head's state from column c0 on, entry (channel, column) at
+// channel * s_ch + (column - c0) * s_col; no block-level synchronisation.  RULE false: linear attention with the decay, key and query factors `fixed` of every token.
+template <int CPL, bool VEC, bool RULE = true>
+__device__ __forceinline__ void delta_rule_columns(const DeltaArgs& p, int h, int col0, int t0, int t1, float* S, int64_t s_ch, int64_t s_col, int c0 = 0, f32x4 fixed = {}) {
     const int lane = threadIdx.x & 63;
     const int col = col0 + lane / DR_LPR, cg = lane % DR_LPR, ch0 = cg * CPL;
     const bool col_ok = col < p.dv;
     const int hq = h / (p.H / p.G), dk = p.dk;
-    const int t0 = p.seq_off[s], t1 = p.seq_off[s + 1];
-    float* S = p.state + (((int64_t)p.slot[s] * p.H + h) * dk) * p.dv;
     float st[CPL];
 #pragma unroll
-    for (int i = 0; i < CPL; ++i) st[i] = (col_ok && ch0 + i < dk) ? S[(int64_t)(ch0 + i) * p.dv + col] : 0.f;
+    for (int i = 0; i < CPL; ++i) st[i] = (col_ok && ch0 + i < dk) ? S[(ch0 + i) * s_ch + (col - c0) * s_col] : 0.f;
     struct In {
         float k[CPL], q[CPL];
         f32x4 sc;
@@ -64,7 +63,7 @@ __device__ __forceinline__ void delta_rule_columns(const DeltaArgs& p, int s, in
                 in.q[i] = ok ? ldr_dt(p.q, p.qk_dt, qo + i) : 0.f;
             }
         }
-        in.sc = p.ws[(int64_t)t * p.H + h];
+        in.sc = RULE ? p.ws[(int64_t)t * p.H + h] : fixed;
         in.v = col_ok ? ldr_dt(p.v, p.v_dt, (int64_t)t * p.ldv + (int64_t)h * p.dv + col) : 0.f;
     };
     auto step = [&](const In& in, int t) {
@@ -77,7 +76,7 @@ __device__ __forceinline__ void delta_rule_columns(const DeltaArgs& p, int s, in
             u0 = fmaf(st[i], in.k[i], u0);
             u1 = fmaf(st[i + 1], in.k[i + 1], u1);
         }
-        const float u = lanes_sum<DR_LPR>(u0 + u1) * kn;
+        const float u = RULE ? lanes_sum<DR_LPR>(u0 + u1) * kn : 0.f;
         const float c = b * (in.v - u) * kn;
         float o0 = 0.f, o1 = 0.f;
 #pragma unroll
@@ -102,5 +101,5 @@ __device__ __forceinline__ void delta_rule_columns(const DeltaArgs& p, int s, in
     }
 #pragma unroll
     for (int i = 0; i < CPL; ++i)
-        if (col_ok && ch0 + i < dk) S[(int64_t)(ch0 + i) * p.dv + col] = st[i];
+        if (col_ok && ch0 + i < dk) S[(ch0 + i) * s_ch + (col - c0) * s_col] = st[i];
 }

@@ -49,6 +49,14 @@ __device__ __forceinline__ void add16(f32x16& to, f32x16& from) {  // a chain's 
     }
 }
 
+// whether any of 16 values is infinite or NaN
+__device__ __forceinline__ bool lost16(const f32x16& v) {
+    float z = 0.f;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) z = fmaf(v[e], 0.f, z);
+    return z != z;
+}
+
 // T = (I + tril(N, -1))^-1, both [64][68] in LDS, by the four waves of a workgroup (N's upper right quarter is scratch): the two diagonal 32 x 32 blocks by forward
 // substitution (lane = column), the block below them as -R22 (N21 R11).
 __device__ __forceinline__ void invert_unit_lower64(float (&N)[GC][GC + 4], float (&T)[GC][GC + 4]) {

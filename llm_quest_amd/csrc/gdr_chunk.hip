@@ -153,12 +153,14 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
 // Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave.  Bound: the chain
 // of chunks -- reads in flight, then two products behind two barriers.  Everything a chunk reads first is requested at its top, all at once: 167 us at 8 x 708 tokens x 16
 // heads; requested a chunk ahead 189 (the registers spill), in two halves 187, and 177 with the value ranges of a head on different XCDs.
-__global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, float* __restrict__ saved,
+__global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
+                                                           const bf16_t* __restrict__ v, int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha, float* __restrict__ saved,
                                                            bf16_t* __restrict__ o, const float* initial_state, float* final_state, int keep, float qscale) {
     __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];
     __shared__ __attribute__((aligned(16))) float Us[GC][GV + 8];
     __shared__ __attribute__((aligned(16))) bf16_t Ks[GC][GD + 8];
     __shared__ float gg[2 * GC];
+    __shared__ int lost[2];  // a chunk's flag: set by its U, cleared a chunk later
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
     int at, v0;
     if (!scan_place(heads, at, v0)) return;
@@ -174,7 +176,9 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
         if (initial_state) s = *reinterpret_cast<const f32x4*>(initial_state + (head * GD + v0 + r) * GD + c);
         *reinterpret_cast<f32x4*>(&Ss[r][c]) = s;
     }
-    for (int n = 0; n < NC; ++n) {
+    if (tid < 2) lost[tid] = 0;
+    int n = 0;
+    for (; n < NC; ++n) {
         float* blk = base + (int64_t)n * G_BLOCK;
         const int t0 = n * GC, cnt = min(GC, S - t0);
         // a Kw row (waves 0, 1) or, in half the words, a Q row (waves 2, 3) in fragment form, all of it in flight at once
@@ -200,6 +204,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
         const float gr = tid < 2 * GC ? blk[G_GAM + tid] : 0.f;
         __syncthreads();  // the state is whole, the last chunk's K and U are read
         if (tid < 2 * GC) gg[tid] = gr;
+        if (tid == 0) lost[(n + 1) & 1] = 0;
         if (keep) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -241,12 +246,14 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = 32 * rh + c_row(e, hf);
-                const float u = uv[e] - acc[e];
-                Us[r][ln] = u;
-                blk[G_U + r * GD + v0 + ln] = u;
+                acc[e] = uv[e] - acc[e];
+                Us[r][ln] = acc[e];
+                blk[G_U + r * GD + v0 + ln] = acc[e];
             }
+            if (__any(lost16(acc)) && lane == 0) lost[n & 1] = 1;
         }
         __syncthreads();
+        const int gone = lost[n & 1];
         if (qside) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) acc[e] = (acc[e] - uv[e]) * (gg[32 * rh + c_row(e, hf)] * qscale);
@@ -262,6 +269,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
                 if (r < cnt) o[((int64_t)b * S + t0 + r) * Hv * GD + (int64_t)h * GD + v0 + ln] = f2bf(acc[e]);
             }
         }
+        if (gone) break;  // (the same for the whole workgroup)
         f32x16 s;
         const float gC = gg[GC - 1];
 #pragma unroll
@@ -275,6 +283,44 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
             }
 #pragma unroll
         for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = s[e];  // read by this wave alone since the last barrier
+    }
+    // A chunk whose U is not finite, and all behind it: the recurrence itself, eight lanes to a value row.  (In a chunk the triangles' zeros are multiplied, not skipped: a token's key,
+    // value, decay or beta that is not finite reaches U and with it the rows before it.  A query reaches its own row alone.)
+    if (n < NC) {
+        __threadfence();
+        __syncthreads();  // what the chunk wrote of its outputs and U lies below what comes
+        const int r = tid >> 3, c = (tid & 7) * 16;
+        float st[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) st[i] = Ss[r][c + i];
+        for (int t = n * GC; t < S; ++t) {
+            float* blk = base + (int64_t)(t / GC) * G_BLOCK;
+            if (keep && t % GC == 0) {
+#pragma unroll
+                for (int i = 0; i < 16; ++i) blk[(v0 + r) * GD + c + i] = st[i];
+            }
+            const int64_t at_ = ((int64_t)b * S + t) * Hv + h;
+            const float a = alpha[at_];
+            float u = 0.f, x = 0.f;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                st[i] *= a;
+                u = fmaf(st[i], bf2f(kp[t * ldqk + c + i]), u);
+            }
+            u = beta[at_] * (bf2f(v[((int64_t)b * S + t) * ldv + (int64_t)h * GD + v0 + r]) - lanes_sum<8>(u));
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                st[i] = fmaf(u, bf2f(kp[t * ldqk + c + i]), st[i]);
+                x = fmaf(st[i], bf2f(qp[t * ldqk + c + i]), x);
+            }
+            x = lanes_sum<8>(x) * qscale;
+            if (c == 0) {
+                o[at_ * GD + v0 + r] = f2bf(x);
+                blk[G_U + t % GC * GD + v0 + r] = u;
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) Ss[r][c + i] = st[i];
     }
     if (final_state) {
         __syncthreads();
@@ -762,7 +808,8 @@ extern "C" int mi355_gdr_chunked_fwd(int B, int S, int Hqk, int Hv, const void* 
     const float qs = 1.0f / sqrtf((float)GD);
     gdrc_prep_kernel<<<dim3(NC, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, qs);
     MI355_LAUNCH_CHECK("gdr_chunked_fwd(prep)");
-    gdrc_scan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, saved, (bf16_t*)o, initial_state, final_state, keep, qs);
+    gdrc_scan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved,
+                                                                      (bf16_t*)o, initial_state, final_state, keep, qs);
     MI355_LAUNCH_CHECK("gdr_chunked_fwd");
     return 0;
 }

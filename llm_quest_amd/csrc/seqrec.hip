@@ -571,7 +571,8 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(int64_t T, DeltaArgs p)
 template <int CPL, bool VEC>
 __global__ __launch_bounds__(256) void delta_rule_kernel(DeltaArgs p) {
     const int col0 = (blockIdx.x * 4 + (threadIdx.x >> 6)) * (64 / DR_LPR);
-    if (col0 < p.dv) delta_rule_columns<CPL, VEC>(p, blockIdx.z, blockIdx.y, col0);
+    const int s = blockIdx.z, h = blockIdx.y;
+    if (col0 < p.dv) delta_rule_columns<CPL, VEC>(p, h, col0, p.seq_off[s], p.seq_off[s + 1], p.state + ((int64_t)p.slot[s] * p.H + h) * p.dk * p.dv, p.dv, 1);
 }
 
 template <int CPL>

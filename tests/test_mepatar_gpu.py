@@ -465,6 +465,41 @@ def test_delta_rule_in_chunks_is_about_as_near_to_fp64_as_by_token(offset, rate)
     assert dist[1] < 1.6 * dist[0], dist
 
 
+@pytest.mark.parametrize("rule", ["delta", "retention"])
+@pytest.mark.parametrize("what", ["key", "value", "query", "state"])
+def test_recurrences_in_chunks_keep_what_is_not_finite_to_the_rows_behind_it(rule, what):
+    """A NaN or an infinity in one token's operands (or a carried state) reaches the outputs that it reaches token by token and no row before it in the same chunk; the finite outputs and
+    states are the same (1e-5 as above)."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(23)
+    H = G = 2
+    D, lens, at = 128, [70, 200], 170
+    T, d = sum(lens), _Slots(lens)
+    x = torch.randn(T, 3 * H * D, generator=g)
+    start, ba = torch.randn(2, H, D, D, generator=g), (torch.randn(T, 2 * H, generator=g)).to(DEV)
+    if what == "state":
+        start[1, 1, 3, 40] = float("inf")
+    else:
+        x[at, {"query": 0, "key": H * D, "value": 2 * H * D}[what] + 9] = float("inf") if what == "value" else float("nan")
+    x = x.to(DEV)
+    q, k, v = x[:, : H * D], x[:, H * D : 2 * H * D], x[:, 2 * H * D :]
+    A, dec = torch.full((H,), -2.0, device=DEV), torch.tensor([0.9, 0.99], device=DEV)
+    out = []
+    for n in (0, max(lens)):
+        st = start.clone().to(DEV)
+        if rule == "delta":
+            o = S.delta_rule(q, k, v, ba[:, :H], ba[:, H:], A, torch.zeros(H, device=DEV), D ** -0.5, d.seq_off, d.slots, st, H, G, D, D, max_new=n)
+        else:
+            o = S.gla(q, k, v, None, None, 1.0, 1.0, d.seq_off, d.slots, st, H, D, D, head_decay=dec, kscale=D ** -0.5, max_new=n, min_new=min(lens) if n else 0)
+        out.append((o, st))
+    for one, two in zip(*out):
+        fine = torch.isfinite(one)
+        assert torch.equal(fine, torch.isfinite(two))
+        assert float((two[fine] - one[fine]).double().norm() / one[fine].double().norm()) < 1e-5
+    assert not bool(torch.isfinite(out[1][0]).all()) and bool(torch.isfinite(out[1][0][: (70 if what == "state" else at)]).all())
+
+
 def test_retention_with_any_fixed_decay_does_not_know_how_a_prompt_is_cut():
     """Decays that have no logarithm (negative, zero), one below what the chunks of tokens hold and one above one, heads of 128 | 128: a prompt of more than a chunk is the same rows as
     in two short portions (fp32 sums of 128 channels in the same order, equal up to the tiles of the products around them: 1e-5 as above; states head by head, their sizes are far apart)."""

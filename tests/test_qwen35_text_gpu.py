@@ -943,6 +943,38 @@ def test_chunked_gated_delta_rule_is_as_near_to_fp64_as_the_token_by_token_kerne
         assert two < (1.01 * one if i < 4 else 1e-6), (i, one, two)
 
 
+@pytest.mark.parametrize("what", ["key", "value", "query", "decay", "state"])
+def test_chunked_gated_delta_rule_keeps_what_is_not_finite_to_the_rows_behind_it(what):
+    """A NaN or an infinity in one token's operands (or the carried state) reaches the outputs that it reaches token by token -- later rows, for a value its own column, for a query its
+    own row -- and no row before it in the same chunk; the finite outputs are the same (bf16 rounding flips, as above)."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    g = torch.Generator().manual_seed(21)
+    D, s, hv, at = 128, 200, 2, 100
+    q, k = (torch.nn.functional.normalize(torch.randn(s, hv, D, generator=g), dim=-1).to(BF16).reshape(s, -1).cuda() for _ in range(2))
+    v = torch.randn(s, hv * D, generator=g).to(BF16).cuda()
+    be, al = torch.sigmoid(torch.randn(s, hv, generator=g)).cuda(), (0.5 + 0.5 * torch.rand(s, hv, generator=g)).cuda()
+    s0 = torch.randn(1, hv, D, D, generator=g).cuda()
+    if what == "key":
+        k[at, 5] = float("nan")
+    elif what == "value":
+        v[at, 7], v[at + 3, 130] = float("inf"), float("nan")
+    elif what == "query":
+        q[at, 9] = float("inf")
+    elif what == "decay":
+        al[at, 1] = float("nan")
+    else:
+        s0[0, 1, 40, 3] = float("inf")
+    out = []
+    for chunked in (False, None):
+        o, _, fin = Q.gated_delta_rule_fwd(q, k, v, be, al, 1, s, hv, hv, D, D, keep=False, state=s0.clone(), chunked=chunked)
+        out.append((o.float(), fin))
+    for one, two in zip(*out):
+        fine = torch.isfinite(one)
+        assert torch.equal(fine, torch.isfinite(two)) and rel_l2(two[fine], one[fine]) < 1e-3
+    assert not bool(torch.isfinite(out[1][0]).all()) and bool(torch.isfinite(out[1][0][: (0 if what == "state" else at)]).all())
+
+
 def test_chunked_gated_delta_rule_refuses_what_it_cannot_read():
     from llm_quest_amd import _lib as L
     from llm_quest_amd import kernels_q35 as Q
