@@ -544,7 +544,7 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
 // then joined in order, in EVERY kernel of this path: a row's bits depend neither on the rows beside it nor on which of the kernels its row count takes.
 // Against the FMA kernel (64 x 64 tile, scalar fp32: VALU-bound, and at few rows a chain of uncached 2-byte loads): a fp32 replay of three 150-token prompts and four
 // single tokens through four layers with experts 19.9 -> 6.0 ms, its logits' error against 64 bits 4.9e-6 -> 2.1e-6
-// (fewer roundings per sum).  Weights are finite: an infinite one would meet a zero part (NaN).
+// (fewer roundings per sum).  An infinite weight may meet a zero part, which would make NaN of an infinity: a result that is not finite is summed again the plain way.
 #define SW 8
 struct Split8 { u32x4 hi, mid, lo; };
 struct FragF32 { f32x4 a, b; };  // eight consecutive k of a row
@@ -567,6 +567,15 @@ __device__ __forceinline__ Split8 split8(const f32x4 a, const f32x4 b) {
     split_pair(b[0], b[1], h, m, l); r.hi[2] = h; r.mid[2] = m; r.lo[2] = l;
     split_pair(b[2], b[3], h, m, l); r.hi[3] = h; r.mid[3] = m; r.lo[3] = l;
     return r;
+}
+
+__device__ __forceinline__ float settled(const BgemmArgs& p, float v, int b, int r, int n) {  // sorted row r, column n
+    if (v - v == 0.f || n >= p.N) return v;
+    const float* a = (const float*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
+    const bf16_t* w = (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)n * p.sbn;
+    v = 0.f;
+    for (int k = 0; k < p.K; ++k) v = fmaf(a[k], bf2f(w[k]), v);
+    return v;
 }
 
 // Tile of 64 WM rows x 128 columns, four waves of 32 WM x 64 (2 x 2): k in steps of 32 through one LDS stage (A as three bf16 planes, split once per tile), the next
@@ -669,6 +678,25 @@ __global__ __launch_bounds__(256) void bgemm_f32_tile_kernel(BgemmArgs p) {
             for (int j = 0; j < 2; ++j)
 #pragma unroll
                 for (int e = 0; e < 16; ++e) tot[i][j][e] += acc[i][j][e];
+    }
+    float z = 0.f;
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) z = fmaf(tot[i][j][e], 0.f, z);
+    if (__any(z != z)) {
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int e = 0; e < 16; ++e) {
+                const int m = m0 + wm + 32 * i + 8 * (e >> 2) + 4 * hf + (e & 3);
+                if (m < rows) {
+#pragma unroll
+                    for (int j = 0; j < 2; ++j) tot[i][j][e] = settled(p, tot[i][j][e], b, row0 + m, n0 + wn + 32 * j + ln);
+                }
+            }
     }
 #pragma unroll
     for (int bi = 0; bi < WM; ++bi)
@@ -800,6 +828,10 @@ __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
         if (m >= rows || n >= (GLU ? p.n_out : p.N)) continue;
         const int r = row0 + m;
         const int64_t crow = p.c_rows ? p.c_rows[r] : r;
+        if constexpr (F32) {
+#pragma unroll
+            for (int j = 0; j < NB; ++j) v[j] = settled(p, v[j], b, r, n0 + 32 * j + ln);
+        }
         float x;
         if constexpr (GLU) {
             x = gated_act(p.epi, v[0], v[NB - 1], p.limit);

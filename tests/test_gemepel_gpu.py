@@ -479,6 +479,27 @@ def test_fp32_product_on_split_operands(M, N, K):
         assert float((out[2].double() - big).abs().max()) <= 2.0 ** -22 * float(big.abs().max()) and torch.equal(out[3:], got[3:])
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 200, 272), (200, 130, 96), (1024, 8192, 64)])
+def test_fp32_product_with_weights_that_are_not_finite(M, N, K):
+    """The fp32 product of the stream, the 64-row and the 128-row tiles with infinite and NaN weights: infinite, NaN and finite results are those of fp64, element by element (finite
+    columns to fp32 rounding of K exact products)."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(M)
+    x, w = torch.randn(M, K, generator=g), torch.randn(N, K, generator=g).to(BF16)
+    x[1, 7] = 0.0  # meets an infinity: NaN
+    x[2] = x[2].to(BF16).float()  # a bf16 number's second and third parts are zero
+    w[0, 7], w[33, K - 1], w[N - 1, 40] = float("inf"), -float("inf"), float("nan")
+    w[65, 3], w[65, 50] = float("inf"), -float("inf")
+    out = S.linear(x.to(DEV), w.to(DEV), out_dtype=F32).cpu()
+    cols = [0, 1, 33, 34, 64, 65, 66, N - 2, N - 1]
+    want = (x.double()[:, None, :] * w[cols].double()[None]).sum(-1)
+    got = out[:, cols].double()
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf()) and torch.equal(got[want.isinf()], want[want.isinf()])
+    fine = want.isfinite()
+    assert float((got[fine] - want[fine]).abs().max()) < 2e-5 * K**0.5 and bool(out[:, [c for c in range(N) if c not in (0, 33, 65, N - 1)]].isfinite().all())
+
+
 @pytest.mark.parametrize("T,top,epi", [(5, 2, 1), (70, 3, 0), (90, 2, 4), (400, 2, 4)])
 def test_fp32_grouped_product_on_split_operands(T, top, epi):
     """Experts (rows gathered, scaled and scattered; one expert without rows; gated blocks): stream and tile against fp64."""
