@@ -885,13 +885,22 @@ def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=No
 
 
 def reduce_rows_into(partial, parts, width, dests):
-    """``dests`` = one (fp32 tensor of ``width`` elements, accumulate) or None per segment of partial [parts, len(dests) * width]: the segments' column sums in one launch."""
+    """``dests`` = one (fp32 tensor of ``width`` elements, accumulate) or None per segment of partial [parts, len(dests) * width]: the segments' column sums in one launch -- and one
+    more for each time that a destination comes again (a parameter in two places: the workgroups of one launch are in no order)."""
     for d in dests:
         if d is not None and not (d[0].dtype == F32 and d[0].is_contiguous() and d[0].numel() == width and d[0].device == partial.device):
             raise ValueError("reduce_rows_into: a destination is contiguous fp32 with the segment's width, on the partial sums' device")
-    if any(d is not None for d in dests):
-        ptrs = [None if d is None else d[0].data_ptr() for d in dests] + [None] * (4 - len(dests))
-        L.call("mi355_reduce_rows_into", parts, len(dests), width, L.ptr(partial), *ptrs, sum(1 << i for i, d in enumerate(dests) if d is not None and d[1]))
+    while any(d is not None for d in dests):
+        taken, now, later = set(), [], []
+        for d in dests:
+            again = d is not None and d[0].data_ptr() in taken
+            now.append(None if again else d)
+            later.append(d if again else None)
+            if d is not None:
+                taken.add(d[0].data_ptr())
+        ptrs = [None if d is None else d[0].data_ptr() for d in now] + [None] * (4 - len(now))
+        L.call("mi355_reduce_rows_into", parts, len(now), width, L.ptr(partial), *ptrs, sum(1 << i for i, d in enumerate(now) if d is not None and d[1]))
+        dests = later
 
 
 def layernorm_bwd_bf16_fits(x2d, scale, dy, dres):

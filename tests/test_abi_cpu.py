@@ -159,3 +159,14 @@ def test_gradient_destinations_are_checked(dest):
 
     with pytest.raises(ValueError, match="contiguous fp32"):
         kernels.reduce_rows_into(torch.zeros(2, 16), 2, 8, [None, (dest, False)])
+
+
+def test_row_reductions_into_one_parameter_twice_go_one_after_the_other(monkeypatch):
+    """A launch's workgroups are in no order: a destination that comes again (one bias in two places) has a launch of its own."""
+    from llm_quest_amd import kernels
+
+    calls = []
+    monkeypatch.setattr(kernels.L, "call", lambda name, *a: calls.append(a))
+    a, b = torch.zeros(8), torch.zeros(8)
+    kernels.reduce_rows_into(torch.zeros(2, 32), 2, 8, [(a, False), (a, True), (b, True), None])
+    assert [(c[4:8], c[8]) for c in calls] == [((a.data_ptr(), None, b.data_ptr(), None), 4), ((None, a.data_ptr(), None, None), 2)]

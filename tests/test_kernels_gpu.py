@@ -1220,6 +1220,17 @@ def test_products_in_two_launches_equal_one(form, M, N, K, case):
     assert torch.equal(*outs)
 
 
+def test_row_reductions_of_one_parameter_in_two_places_add_up():
+    """Segments with one destination (a bias that two layers share) are added one after the other; three sums of 70 fp32 terms."""
+    from llm_quest_amd import kernels as KK
+
+    part = torch.randn(70, 3 * 200, generator=torch.Generator().manual_seed(2)).cuda()
+    dest = torch.full((200,), float("nan"), device="cuda")
+    KK.reduce_rows_into(part, 70, 200, [(dest, False), (dest, True), (dest, True)])
+    want = part.double().view(70, 3, 200).sum((0, 1))
+    assert float((dest.double() - want).abs().max()) <= 2.0 ** -24 * 73 * float(part.double().view(70, 3, 200).abs().sum((0, 1)).max())
+
+
 @pytest.mark.parametrize("rows,width,dt,res", [(5, 768, torch.bfloat16, True), (985, 768, torch.float32, False), (4099, 1024, torch.bfloat16, True), (1, 1024, torch.float32, True)])
 def test_layernorm_backward_with_bf16_result_and_column_sums(rows, width, dt, res):
     """mi355_layernorm_bwd_bf16 + mi355_reduce_rows_into against the separate launches: the same dx, its bf16 rounding, its column sums (fp32 sums of `rows` terms), and every
