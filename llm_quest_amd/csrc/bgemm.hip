@@ -391,151 +391,157 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
     };
     int all = 0;
     for (int b0 = 0; b0 < batch; b0 += 64) all += __shfl(scan(group_tiles(b0 + lane)), 63, 64);
-    const int useful = __builtin_amdgcn_readfirstlane(all) * tn, id = blockIdx.x;
-    if (id >= useful) return;
-    const int q = useful >> 3, r8 = useful & 7, xcd = id & 7;
-    const int at = (xcd < r8 ? xcd * (q + 1) : r8 * (q + 1) + (xcd - r8) * q) + (id >> 3);
-    int b = 0, before = 0, mine = 1;
-    for (int b0 = 0; b0 < batch; b0 += 64) {
-        const int n = group_tiles(b0 + lane), incl = before + scan(n);
-        const unsigned long long hit = __ballot(incl * tn > at);
-        if (hit) {
-            const int l = __ffsll(hit) - 1;
-            b = b0 + l;
-            mine = __shfl(n, l, 64);
-            before = __shfl(incl, l, 64) - mine;
-            break;
+    const int useful = __builtin_amdgcn_readfirstlane(all) * tn;
+    auto tile = [&](int id) __attribute__((always_inline)) {
+        const int q = useful >> 3, r8 = useful & 7, xcd = id & 7;
+        const int at = (xcd < r8 ? xcd * (q + 1) : r8 * (q + 1) + (xcd - r8) * q) + (id >> 3);
+        int b = 0, before = 0, mine = 1;
+        for (int b0 = 0; b0 < batch; b0 += 64) {
+            const int n = group_tiles(b0 + lane), incl = before + scan(n);
+            const unsigned long long hit = __ballot(incl * tn > at);
+            if (hit) {
+                const int l = __ffsll(hit) - 1;
+                b = b0 + l;
+                mine = __shfl(n, l, 64);
+                before = __shfl(incl, l, 64) - mine;
+                break;
+            }
+            before = __shfl(incl, 63, 64);
         }
-        before = __shfl(incl, 63, 64);
-    }
-    b = __builtin_amdgcn_readfirstlane(b);
-    mine = __builtin_amdgcn_readfirstlane(mine);
-    const int local = at - __builtin_amdgcn_readfirstlane(before) * tn, tm = local % mine, n0 = local / mine * WTN;
-    const int row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? p.grp_offs[b + 1] - row0 : p.M;
-    const int per = ((rows + mine - 1) / mine + 31) & ~31, m0 = tm * per, cnt = __builtin_amdgcn_readfirstlane(min(per, rows - m0));
-    if (cnt <= 0) return;  // (rounding up to 32 rows can leave the last tile without any)
-    // this wave's share of a stage: four pieces of A and four of B, eight rows of 128 bytes each (rows beyond the tile: the last one again, their results are not stored)
-    const char* src[8];
-    auto piece = [&](int i) { return wave * 4 + (i & 3); };
+        b = __builtin_amdgcn_readfirstlane(b);
+        mine = __builtin_amdgcn_readfirstlane(mine);
+        const int local = at - __builtin_amdgcn_readfirstlane(before) * tn, tm = local % mine, n0 = local / mine * WTN;
+        const int row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? p.grp_offs[b + 1] - row0 : p.M;
+        const int per = ((rows + mine - 1) / mine + 31) & ~31, m0 = tm * per, cnt = __builtin_amdgcn_readfirstlane(min(per, rows - m0));
+        if (cnt <= 0) return;  // (rounding up to 32 rows can leave the last tile without any)
+        // this wave's share of a stage: four pieces of A and four of B, eight rows of 128 bytes each (rows beyond the tile: the last one again, their results are not stored)
+        const char* src[8];
+        auto piece = [&](int i) { return wave * 4 + (i & 3); };
 #pragma unroll
-    for (int i = 0; i < 8; ++i) {
-        const int r = piece(i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
-        if (i < 4) {
-            const int ar = row0 + m0 + min(r, cnt - 1);
-            src[i] = (const char*)((const bf16_t*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[ar] / p.a_div : ar) * p.lda + c * 8);
-        } else {
-            src[i] = (const char*)((const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)min(n0 + r, p.N - 1) * p.sbn + c * 8);
+        for (int i = 0; i < 8; ++i) {
+            const int r = piece(i) * 8 + (lane >> 3), c = (lane & 7) ^ ((r >> 1) & 7);
+            if (i < 4) {
+                const int ar = row0 + m0 + min(r, cnt - 1);
+                src[i] = (const char*)((const bf16_t*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[ar] / p.a_div : ar) * p.lda + c * 8);
+            } else {
+                src[i] = (const char*)((const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)min(n0 + r, p.N - 1) * p.sbn + c * 8);
+            }
         }
-    }
-    auto issue = [&](int t, int stage, int lo, int hi) {  // (lo, hi: 0, 4 the A pieces, 4, 8 the B pieces)
+        auto issue = [&](int t, int stage, int lo, int hi) {  // (lo, hi: 0, 4 the A pieces, 4, 8 the B pieces)
 #pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (i >= lo && i < hi)
-                __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)t * (WK * 2)),
-                                             (__attribute__((address_space(3))) void*)(lds + stage * WSTAGE + (i < 4 ? 0 : WTM * WK * 2) + piece(i) * 1024), 16, 0, 0);
-    };
-    const int wm = (wave >> 2) * 128, wn = (wave & 3) * 64, nt = p.K / WK;
-    auto frag = [&](const char* tile, int r, int kk) { return *(const bf16x8*)(tile + r * 128 + (((kk * 2 + hf) ^ ((r >> 1) & 7)) << 4)); };
-    auto rows_of_tile = [&]() {  // where the tile's rows go, and what they are multiplied by
-        if (tid < cnt) {
-            const int r = row0 + m0 + tid, c = p.c_rows ? p.c_rows[r] : r;
-            to_row[tid] = c;
-            scale[tid] = p.row_scale ? p.row_scale[c] : 1.0f;
-        }
-    };
-    auto run = [&](auto nb) {
-        constexpr int NB = decltype(nb)::value;  // blocks of 32 rows
-        f32x16 acc[NB ? NB : 1][2];
+            for (int i = 0; i < 8; ++i)
+                if (i >= lo && i < hi)
+                    __builtin_amdgcn_global_load_lds((const __attribute__((address_space(1))) void*)(src[i] + (int64_t)t * (WK * 2)),
+                                                 (__attribute__((address_space(3))) void*)(lds + stage * WSTAGE + (i < 4 ? 0 : WTM * WK * 2) + piece(i) * 1024), 16, 0, 0);
+        };
+        const int wm = (wave >> 2) * 128, wn = (wave & 3) * 64, nt = p.K / WK;
+        auto frag = [&](const char* tile, int r, int kk) { return *(const bf16x8*)(tile + r * 128 + (((kk * 2 + hf) ^ ((r >> 1) & 7)) << 4)); };
+        auto rows_of_tile = [&]() {  // where the tile's rows go, and what they are multiplied by
+            if (tid < cnt) {
+                const int r = row0 + m0 + tid, c = p.c_rows ? p.c_rows[r] : r;
+                to_row[tid] = c;
+                scale[tid] = p.row_scale ? p.row_scale[c] : 1.0f;
+            }
+        };
+        auto run = [&](auto nb) {
+            constexpr int NB = decltype(nb)::value;  // blocks of 32 rows
+            f32x16 acc[NB ? NB : 1][2];
 #pragma unroll
-        for (int i = 0; i < NB; ++i)
-#pragma unroll
-            for (int j = 0; j < 2; ++j)
-#pragma unroll
-                for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
-        issue(0, 0, 0, 8);
-        rows_of_tile();
-        for (int t = 0; t < nt; ++t) {
-            // this wave's pieces of the step have landed and its reads of the step before are done -- behind the barrier everyone's
-            asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            asm volatile("" ::: "memory");
-            if constexpr (NB > 0) {
-                const char *sa = lds + (t & 1) * WSTAGE, *sb = sa + WTM * WK * 2;
-                bf16x8 fa[2][NB], fb[2][2];  // the fragments of the next 16 k are requested in front of the products of this one
-                auto read = [&](int kk) {
-#pragma unroll
-                    for (int j = 0; j < 2; ++j) fb[kk & 1][j] = frag(sb, wn + 32 * j + ln, kk);
-#pragma unroll
-                    for (int i = 0; i < NB; ++i) fa[kk & 1][i] = frag(sa, wm + 32 * i + ln, kk);
-                };
-                read(0);  // (in front of the DMA's issue, and that in two parts: with all of it first 8192^3 takes 1 020 us instead of 944)
-                if (t + 1 < nt) issue(t + 1, (t + 1) & 1, 0, 4);
-#pragma unroll
-                for (int kk = 0; kk < 4; ++kk) {
-                    if (kk < 3) read(kk + 1);
-                    if (kk == 1 && t + 1 < nt) issue(t + 1, (t + 1) & 1, 4, 8);
-#pragma unroll
-                    for (int i = 0; i < NB; ++i)
-#pragma unroll
-                        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk & 1][i], fb[kk & 1][j], acc[i][j], 0, 0, 0);
-                }
-            } else if (t + 1 < nt) issue(t + 1, (t + 1) & 1, 0, 8);
-        }
-        // write-out through the stages' LDS, which nobody reads any more: 64 rows of a wave at a time as fp32, then whole 4-column words of a row to a lane
-        __syncthreads();
-        float* mine = (float*)(lds + wave * 16384);
-        const bool glu = p.epi >= 2;
-        const int cols = glu ? 32 : 64, lanes = cols / 4, cq = (lane & (lanes - 1)) * 4, nq = glu ? ((n0 + wn) >> 1) + cq : n0 + wn + cq, n_end = glu ? p.n_out : p.N;
-        float bias[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) bias[j] = p.bias && nq + j < n_end ? p.bias[nq + j] : 0.f;
-        const bool words = nq + 4 <= n_end && p.ldc % 4 == 0 && p.c_bs % 4 == 0 && ((uintptr_t)p.C & 15) == 0;
-#pragma unroll
-        for (int h = 0; h < (NB + 1) / 2; ++h) {
-#pragma unroll
-            for (int i = 0; i < (NB - 2 * h < 2 ? NB - 2 * h : 2); ++i)
+            for (int i = 0; i < NB; ++i)
 #pragma unroll
                 for (int j = 0; j < 2; ++j)
 #pragma unroll
-                    for (int e = 0; e < 16; ++e) mine[(32 * i + 8 * (e >> 2) + 4 * hf + (e & 3)) * 64 + 32 * j + ln] = acc[2 * h + i][j][e];
-            __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses are in order)
-            for (int r = lane / lanes; r < 64; r += 64 / lanes) {
-                const int m = wm + 64 * h + r;
-                if (m >= cnt) break;
-                const float sc = scale[m];
-                const int64_t at = (int64_t)b * p.c_bs + (int64_t)to_row[m] * p.ldc + nq;
-                f32x4 v = *(const f32x4*)(mine + r * 64 + cq);
-                if (glu) {
-                    const f32x4 u = *(const f32x4*)(mine + r * 64 + 32 + cq);
+                    for (int e = 0; e < 16; ++e) acc[i][j][e] = 0.f;
+            issue(0, 0, 0, 8);
+            rows_of_tile();
+            for (int t = 0; t < nt; ++t) {
+                // this wave's pieces of the step have landed and its reads of the step before are done -- behind the barrier everyone's
+                asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                if constexpr (NB > 0) {
+                    const char *sa = lds + (t & 1) * WSTAGE, *sb = sa + WTM * WK * 2;
+                    bf16x8 fa[2][NB], fb[2][2];  // the fragments of the next 16 k are requested in front of the products of this one
+                    auto read = [&](int kk) {
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) v[j] = gated_act(p.epi, v[j], u[j], p.limit) * sc;
-                } else {
+                        for (int j = 0; j < 2; ++j) fb[kk & 1][j] = frag(sb, wn + 32 * j + ln, kk);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        v[j] += bias[j];
-                        if (p.epi == 1) v[j] = v[j] > 0.f ? v[j] * v[j] : 0.f;
-                        v[j] *= sc;
+                        for (int i = 0; i < NB; ++i) fa[kk & 1][i] = frag(sa, wm + 32 * i + ln, kk);
+                    };
+                    read(0);  // (in front of the DMA's issue, and that in two parts: with all of it first 8192^3 takes 1 020 us instead of 944)
+                    if (t + 1 < nt) issue(t + 1, (t + 1) & 1, 0, 4);
+#pragma unroll
+                    for (int kk = 0; kk < 4; ++kk) {
+                        if (kk < 3) read(kk + 1);
+                        if (kk == 1 && t + 1 < nt) issue(t + 1, (t + 1) & 1, 4, 8);
+#pragma unroll
+                        for (int i = 0; i < NB; ++i)
+#pragma unroll
+                            for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[kk & 1][i], fb[kk & 1][j], acc[i][j], 0, 0, 0);
+                    }
+                } else if (t + 1 < nt) issue(t + 1, (t + 1) & 1, 0, 8);
+            }
+            // write-out through the stages' LDS, which nobody reads any more: 64 rows of a wave at a time as fp32, then whole 4-column words of a row to a lane
+            __syncthreads();
+            float* mine = (float*)(lds + wave * 16384);
+            const bool glu = p.epi >= 2;
+            const int cols = glu ? 32 : 64, lanes = cols / 4, cq = (lane & (lanes - 1)) * 4, nq = glu ? ((n0 + wn) >> 1) + cq : n0 + wn + cq, n_end = glu ? p.n_out : p.N;
+            float bias[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) bias[j] = p.bias && nq + j < n_end ? p.bias[nq + j] : 0.f;
+            const bool words = nq + 4 <= n_end && p.ldc % 4 == 0 && p.c_bs % 4 == 0 && ((uintptr_t)p.C & 15) == 0;
+#pragma unroll
+            for (int h = 0; h < (NB + 1) / 2; ++h) {
+#pragma unroll
+                for (int i = 0; i < (NB - 2 * h < 2 ? NB - 2 * h : 2); ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) mine[(32 * i + 8 * (e >> 2) + 4 * hf + (e & 3)) * 64 + 32 * j + ln] = acc[2 * h + i][j][e];
+                __builtin_amdgcn_wave_barrier();  // (a wave's LDS accesses are in order)
+                for (int r = lane / lanes; r < 64; r += 64 / lanes) {
+                    const int m = wm + 64 * h + r;
+                    if (m >= cnt) break;
+                    const float sc = scale[m];
+                    const int64_t at = (int64_t)b * p.c_bs + (int64_t)to_row[m] * p.ldc + nq;
+                    f32x4 v = *(const f32x4*)(mine + r * 64 + cq);
+                    if (glu) {
+                        const f32x4 u = *(const f32x4*)(mine + r * 64 + 32 + cq);
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) v[j] = gated_act(p.epi, v[j], u[j], p.limit) * sc;
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            v[j] += bias[j];
+                            if (p.epi == 1) v[j] = v[j] > 0.f ? v[j] * v[j] : 0.f;
+                            v[j] *= sc;
+                        }
+                    }
+                    if (words) {
+                        if (p.c_dt == MI355_DT_F32) *(f32x4*)((float*)p.C + at) = v;
+                        else *(u32x2*)((bf16_t*)p.C + at) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; ++j)
+                            if (nq + j < n_end) {
+                                if (p.c_dt == MI355_DT_F32) ((float*)p.C)[at + j] = v[j];
+                                else ((bf16_t*)p.C)[at + j] = f2bf(v[j]);
+                            }
                     }
                 }
-                if (words) {
-                    if (p.c_dt == MI355_DT_F32) *(f32x4*)((float*)p.C + at) = v;
-                    else *(u32x2*)((bf16_t*)p.C + at) = u32x2{pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-                } else {
-#pragma unroll
-                    for (int j = 0; j < 4; ++j)
-                        if (nq + j < n_end) {
-                            if (p.c_dt == MI355_DT_F32) ((float*)p.C)[at + j] = v[j];
-                            else ((bf16_t*)p.C)[at + j] = f2bf(v[j]);
-                        }
-                }
+                __builtin_amdgcn_wave_barrier();
             }
-            __builtin_amdgcn_wave_barrier();
-        }
+        };
+        if (cnt - wm > 96) run(std::integral_constant<int, 4>{});
+        else if (cnt - wm > 64) run(std::integral_constant<int, 3>{});
+        else if (cnt > wm) run(std::integral_constant<int, 2>{});
+        else run(std::integral_constant<int, 0>{});
     };
-    if (cnt - wm > 96) run(std::integral_constant<int, 4>{});
-    else if (cnt - wm > 64) run(std::integral_constant<int, 3>{});
-    else if (cnt > wm) run(std::integral_constant<int, 2>{});
-    else run(std::integral_constant<int, 0>{});
+    if ((int)blockIdx.x < useful) tile(blockIdx.x);
+    for (int id = blockIdx.x + gridDim.x; id < useful; id += gridDim.x) {  // only where M counts the rows of one group, not of all
+        __syncthreads();  // the last tile's write-out has left the LDS
+        tile(id);
+    }
 }
 
 // ---- fp32 A times bf16 B on the matrix pipe, with the fp32 product's accuracy.  An fp32 number is the sum of three bf16 numbers exactly (its 24 significant bits cut into three

@@ -500,6 +500,23 @@ def test_fp32_product_with_weights_that_are_not_finite(M, N, K):
     assert float((got[fine] - want[fine]).abs().max()) < 2e-5 * K**0.5 and bool(out[:, [c for c in range(N) if c not in (0, 33, 65, N - 1)]].isfinite().all())
 
 
+@pytest.mark.parametrize("rows,groups", [(300, 16), (257, 20)])
+def test_grouped_product_with_m_as_the_rows_of_one_group(rows, groups):
+    """``M`` may count the rows of the largest group instead of all: the 256 x 256 tiles' grid is then smaller than the work and its workgroups go round.  bf16 operands, fp32 sums and
+    results: 2^-24 a sum of K exact products."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(rows)
+    N, K, T = 1024, 256, rows * groups
+    x, w = torch.randn(T, K, generator=g).to(BF16).to(DEV), torch.randn(groups, N, K, generator=g).to(BF16).to(DEV)
+    offs = torch.arange(0, T + 1, rows, dtype=torch.int32, device=DEV)
+    out = [torch.full((T, N), float("nan"), device=DEV) for _ in range(2)]
+    for o, m in zip(out, (T, rows)):
+        S.bgemm(x, w.view(-1, K), o, m, N, K, batch=groups, sbn=K, b_bs=N * K, grp_offs=offs)
+    want = torch.cat([x[i * rows : (i + 1) * rows].double() @ w[i].double().T for i in range(groups)])
+    assert float((out[0].double() - want).abs().max()) < K * 2.0 ** -24 * 60 and torch.equal(out[0], out[1])
+
+
 @pytest.mark.parametrize("T,top,epi", [(5, 2, 1), (70, 3, 0), (90, 2, 4), (400, 2, 4)])
 def test_fp32_grouped_product_on_split_operands(T, top, epi):
     """Experts (rows gathered, scaled and scattered; one expert without rows; gated blocks): stream and tile against fp64."""
