@@ -389,9 +389,11 @@ int mi355_gated_delta_rule_bwd(int B, int S, int Hqk, int Hv, int Dk, int Dv, co
  * (gated_delta_rule(..., prev_state), qwen3_next_attention.py:103-159).  The forward must have run with that initial_state and checkpoints. */
 
 /* The same rule in chunks of 64 tokens on the fp32 matrix pipe, for heads of 128 | 128 and the operands a layer makes (unit keys, alpha and beta in 0 .. 1; either
- * below 1e-30 counts as 1e-30).  saved: mi355_gdr_chunked_saved_bytes, 16-byte aligned: the forward's scratch, and (keep != 0) what the backward reads; v's row pitch a
+ * below 1e-30 counts as 1e-30).  saved, 16-byte aligned: with keep
+ * mi355_gdr_chunked_saved_bytes, what the backward reads; without, mi355_gdr_chunked_scratch_bytes, bounded for long sequences; v's row pitch a
  * multiple of 8; states as above.  The backward's workspace: mi355_gdr_chunked_bwd_workspace_bytes. */
 int64_t mi355_gdr_chunked_saved_bytes(int B, int S, int Hv);
+int64_t mi355_gdr_chunked_scratch_bytes(int B, int S, int Hv);
 int64_t mi355_gdr_chunked_bwd_workspace_bytes(int B, int S, int Hqk, int Hv);
 int mi355_gdr_chunked_fwd(int B, int S, int Hqk, int Hv, const void* q, const void* k, const void* v, int64_t ldv, const float* beta, const float* alpha, void* o,
                           float* saved, int64_t saved_bytes, int keep, const float* initial_state, float* final_state, void* stream);

@@ -22,8 +22,11 @@
 
 namespace {
 
-// one chunk of one head in the saved buffer (floats): state at its start [128 dv][128 dk], Kw [64][128], U [64][128], P [64][64], R [64][64], gam [64], Gp [64]
-constexpr int G_KW = GD * GD, G_U = G_KW + GC * GD, G_P = G_U + GC * GD, G_R = G_P + GC * GC, G_GAM = G_R + GC * GC, G_BLOCK = G_GAM + 2 * GC;
+// one chunk of one head in the saved buffer (floats): Kw [64][128], U [64][128], P [64][64], gam [64], Gp [64] (C_: from Kw on); for a backward the state at its start
+// [128 dv][128 dk] lies in front of them and R [64][64] behind (G_: from there on)
+constexpr int C_U = GC * GD, C_P = C_U + GC * GD, C_GAM = C_P + GC * GC, C_R = C_GAM + 2 * GC, G_SMALL = C_R, G_KW = GD * GD, G_U = G_KW + C_U, G_P = G_KW + C_P, G_GAM = G_KW + C_GAM,
+              G_R = G_KW + C_R, G_BLOCK = G_R + GC * GC;
+constexpr int64_t SPAN_BYTES = 256 << 20;  // of a forward that keeps nothing: what one span of chunks takes at most, if that holds four (a prompt of any length, bounded scratch)
 constexpr int W_DU = GD * GD, W_BLOCK = W_DU + GC * GD;  // backward workspace of a chunk: dS at its end, dU
 
 // four consecutive bf16 of row `r` of a [tokens, ld] operand, zeros beyond the sequence
@@ -49,7 +52,7 @@ __device__ __forceinline__ bool scan_place(int heads, int& head, int& v0) {
 static_assert(GD / GV == 4, "four value ranges to a head");
 
 // ------------------------------------------------------------------------------------------- prep: everything of a chunk that needs no state
-__global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
+__global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int n0, int keep, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                            const bf16_t* __restrict__ v, int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha,
                                                            float* __restrict__ saved, float qscale) {
     __shared__ __attribute__((aligned(16))) bf16_t Ks[GC][GD + 8];
@@ -59,10 +62,10 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
     __shared__ double gd[GC];
     __shared__ float be[GC], gam[GC];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
-    const int n = blockIdx.x, h = blockIdx.y, b = blockIdx.z, hq = h / (Hv / Hqk), t0 = n * GC, cnt = min(GC, S - t0);
+    const int n = blockIdx.x, h = blockIdx.y, b = blockIdx.z, hq = h / (Hv / Hqk), t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
     const int64_t tok0 = (int64_t)b * S + t0, ldqk = (int64_t)Hqk * GD;
     const bf16_t *qp = q + tok0 * ldqk + hq * GD, *kp = k + tok0 * ldqk + hq * GD, *vp = v + tok0 * ldv + (int64_t)h * GD;
-    float* blk = saved + (((int64_t)b * Hv + h) * NC + n) * G_BLOCK;
+    float* blk = saved + (((int64_t)b * Hv + h) * gridDim.x + n) * (keep ? G_BLOCK : G_SMALL) + (keep ? G_KW : 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
@@ -81,8 +84,8 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
         gd[lane] = g;
         be[lane] = beta_of(beta, (tok0 + lane) * Hv + h, lane < cnt);
         gam[lane] = exp_of(g);
-        blk[G_GAM + lane] = exp_of(g);
-        blk[G_GAM + GC + lane] = exp_of(g63 - g);
+        blk[C_GAM + lane] = exp_of(g);
+        blk[C_GAM + GC + lane] = exp_of(g63 - g);
     }
     __syncthreads();
     {  // K K^T and Q K^T: wave = tile (ti, tj); the tile above the diagonal is zero
@@ -105,15 +108,17 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
             const int i = 32 * ti + c_row(e, hf);
             const float D = i >= j ? exp_of(gd[i] - gj) : 0.f;
             N[i][j] = i > j ? be[i] * kk[e] * D : 0.f;
-            blk[G_P + i * GC + j] = i >= j ? qscale * qk[e] * D : 0.f;
+            blk[C_P + i * GC + j] = i >= j ? qscale * qk[e] * D : 0.f;
         }
     }
     __syncthreads();
     invert_unit_lower64(N, T);
+    if (keep) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 4;
-        *reinterpret_cast<f32x4*>(blk + G_R + r * GC + c) = *reinterpret_cast<const f32x4*>(&T[r][c]);
+        for (int i = 0; i < 4; ++i) {
+            const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 4;
+            *reinterpret_cast<f32x4*>(blk + C_R + r * GC + c) = *reinterpret_cast<const f32x4*>(&T[r][c]);
+        }
     }
     {  // Uv = R (b V), Kw = R (b gam K): wave = 32 columns, both row halves (the upper one ends at token 32)
         f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16(), ut = zero16(), wt = zero16();
@@ -141,10 +146,10 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int r = c_row(e, hf);
-            blk[G_U + r * GD + col] = u0[e];
-            blk[G_U + (32 + r) * GD + col] = u1[e];
-            blk[G_KW + r * GD + col] = w0[e];
-            blk[G_KW + (32 + r) * GD + col] = w1[e];
+            blk[C_U + r * GD + col] = u0[e];
+            blk[C_U + (32 + r) * GD + col] = u1[e];
+            blk[r * GD + col] = w0[e];
+            blk[(32 + r) * GD + col] = w1[e];
         }
     }
 }
@@ -153,7 +158,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int NC, int Hq
 // Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave.  Bound: the chain
 // of chunks -- reads in flight, then two products behind two barriers.  Everything a chunk reads first is requested at its top, all at once: 167 us at 8 x 708 tokens x 16
 // heads; requested a chunk ahead 189 (the registers spill), in two halves 187, and 177 with the value ranges of a head on different XCDs.
-__global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
+__global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int n0, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                            const bf16_t* __restrict__ v, int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha, float* __restrict__ saved,
                                                            bf16_t* __restrict__ o, const float* initial_state, float* final_state, int keep, float qscale) {
     __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];
@@ -168,7 +173,8 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
     const bool qside = wave >= 2;
     const int64_t ldqk = (int64_t)Hqk * GD, head = at;
     const bf16_t *qp = q + (int64_t)b * S * ldqk + hq * GD, *kp = k + (int64_t)b * S * ldqk + hq * GD;
-    float* base = saved + head * NC * G_BLOCK;
+    const int64_t block = keep ? G_BLOCK : G_SMALL;
+    float* base = saved + head * NC * block + (keep ? G_KW : 0);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
@@ -179,11 +185,11 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
     if (tid < 2) lost[tid] = 0;
     int n = 0;
     for (; n < NC; ++n) {
-        float* blk = base + (int64_t)n * G_BLOCK;
-        const int t0 = n * GC, cnt = min(GC, S - t0);
+        float* blk = base + n * block;
+        const int t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
         // a Kw row (waves 0, 1) or, in half the words, a Q row (waves 2, 3) in fragment form, all of it in flight at once
         const int row = 32 * rh + ln;
-        const float* kw = blk + G_KW + row * GD + 4 * hf;
+        const float* kw = blk + row * GD + 4 * hf;
         f32x4 fr[16];
         if (!qside) {
 #pragma unroll
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
             const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
             kr[i] = r < cnt ? *reinterpret_cast<const u32x4*>(kp + (t0 + r) * ldqk + c) : u32x4{0u, 0u, 0u, 0u};
         }
-        const float gr = tid < 2 * GC ? blk[G_GAM + tid] : 0.f;
+        const float gr = tid < 2 * GC ? blk[C_GAM + tid] : 0.f;
         __syncthreads();  // the state is whole, the last chunk's K and U are read
         if (tid < 2 * GC) gg[tid] = gr;
         if (tid == 0) lost[(n + 1) & 1] = 0;
@@ -209,13 +215,13 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-                *reinterpret_cast<f32x4*>(blk + (v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
+                *reinterpret_cast<f32x4*>(blk - G_KW + (v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
             }
         }
         f32x16 uv = zero16(), acc = zero16();
         if (!qside) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) uv[e] = blk[G_U + (32 * rh + c_row(e, hf)) * GD + v0 + ln];
+            for (int e = 0; e < 16; ++e) uv[e] = blk[C_U + (32 * rh + c_row(e, hf)) * GD + v0 + ln];
         }
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
@@ -241,14 +247,14 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
         }
         f32x4 pr[8];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) pr[i] = qside ? *reinterpret_cast<const f32x4*>(blk + G_P + (32 * rh + ln) * GC + 8 * i + 4 * hf) : f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < 8; ++i) pr[i] = qside ? *reinterpret_cast<const f32x4*>(blk + C_P + (32 * rh + ln) * GC + 8 * i + 4 * hf) : f32x4{0.f, 0.f, 0.f, 0.f};
         if (!qside) {
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = 32 * rh + c_row(e, hf);
                 acc[e] = uv[e] - acc[e];
                 Us[r][ln] = acc[e];
-                blk[G_U + r * GD + v0 + ln] = acc[e];
+                blk[C_U + r * GD + v0 + ln] = acc[e];
             }
             if (__any(lost16(acc)) && lane == 0) lost[n & 1] = 1;
         }
@@ -293,11 +299,11 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
         float st[16];
 #pragma unroll
         for (int i = 0; i < 16; ++i) st[i] = Ss[r][c + i];
-        for (int t = n * GC; t < S; ++t) {
-            float* blk = base + (int64_t)(t / GC) * G_BLOCK;
+        for (int t = (n0 + n) * GC; t < min(S, (n0 + NC) * GC); ++t) {
+            float* blk = base + (t / GC - n0) * block;
             if (keep && t % GC == 0) {
 #pragma unroll
-                for (int i = 0; i < 16; ++i) blk[(v0 + r) * GD + c + i] = st[i];
+                for (int i = 0; i < 16; ++i) (blk - G_KW)[(v0 + r) * GD + c + i] = st[i];
             }
             const int64_t at_ = ((int64_t)b * S + t) * Hv + h;
             const float a = alpha[at_];
@@ -316,7 +322,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
             x = lanes_sum<8>(x) * qscale;
             if (c == 0) {
                 o[at_ * GD + v0 + r] = f2bf(x);
-                blk[G_U + t % GC * GD + v0 + r] = u;
+                blk[C_U + t % GC * GD + v0 + r] = u;
             }
         }
 #pragma unroll
@@ -792,6 +798,16 @@ static int check_gdrc(const char* who, int B, int S, int Hqk, int Hv) {
 
 extern "C" int64_t mi355_gdr_chunked_saved_bytes(int B, int S, int Hv) { return B > 0 && S > 0 && Hv > 0 ? (int64_t)B * Hv * (((int64_t)S + GC - 1) / GC) * G_BLOCK * 4 : 0; }
 
+static int span_chunks(int B, int S, int Hv) {
+    const int64_t all = ((int64_t)S + GC - 1) / GC, fit = SPAN_BYTES / ((int64_t)B * Hv * G_SMALL * 4);
+    return (int)(fit >= all ? all : fit < 4 ? (all < 4 ? all : 4) : fit);
+}
+extern "C" int64_t mi355_gdr_chunked_scratch_bytes(int B, int S, int Hv) {
+    if (B <= 0 || S <= 0 || Hv <= 0) return 0;
+    const int64_t span = span_chunks(B, S, Hv);
+    return (int64_t)B * Hv * 4 * (span * G_SMALL + (span * GC < S ? GD * GD : 0));
+}
+
 extern "C" int64_t mi355_gdr_chunked_bwd_workspace_bytes(int B, int S, int Hqk, int Hv) {
     if (B <= 0 || S <= 0 || Hqk <= 0 || Hv <= 0) return 0;
     const int64_t blocks = (int64_t)B * Hv * (((int64_t)S + GC - 1) / GC) * W_BLOCK;
@@ -803,14 +819,20 @@ extern "C" int mi355_gdr_chunked_fwd(int B, int S, int Hqk, int Hv, const void* 
     if (check_gdrc("gdr_chunked_fwd", B, S, Hqk, Hv)) return 1;
     MI355_REQUIRE(q && k && v && beta && alpha && o && saved && ldv >= (int64_t)Hv * GD && ldv % 8 == 0, "gdr_chunked_fwd: null pointer, or v's row pitch too small or no multiple of 8");
     MI355_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)v | (uintptr_t)saved | (uintptr_t)initial_state | (uintptr_t)final_state) & 15) == 0, "gdr_chunked_fwd: operands must be 16-byte aligned");
-    MI355_REQUIRE(saved_bytes >= mi355_gdr_chunked_saved_bytes(B, S, Hv), "gdr_chunked_fwd: saved buffer too small (%lld bytes)", (long long)saved_bytes);
-    const int NC = (S + GC - 1) / GC;
+    MI355_REQUIRE(saved_bytes >= (keep ? mi355_gdr_chunked_saved_bytes(B, S, Hv) : mi355_gdr_chunked_scratch_bytes(B, S, Hv)), "gdr_chunked_fwd: saved buffer too small (%lld bytes)",
+                  (long long)saved_bytes);
+    const int all = (S + GC - 1) / GC, span = keep ? all : span_chunks(B, S, Hv);
     const float qs = 1.0f / sqrtf((float)GD);
-    gdrc_prep_kernel<<<dim3(NC, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, qs);
-    MI355_LAUNCH_CHECK("gdr_chunked_fwd(prep)");
-    gdrc_scan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved,
-                                                                      (bf16_t*)o, initial_state, final_state, keep, qs);
-    MI355_LAUNCH_CHECK("gdr_chunked_fwd");
+    // several spans: the state travels through final_state, or behind the blocks where nobody asks for it
+    float* carry = final_state ? final_state : saved + (int64_t)B * Hv * span * G_SMALL;
+    for (int n0 = 0; n0 < all; n0 += span) {
+        const int nc = all - n0 < span ? all - n0 : span;
+        gdrc_prep_kernel<<<dim3(nc, Hv, B), 256, 0, ST(stream)>>>(S, n0, keep, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, qs);
+        MI355_LAUNCH_CHECK("gdr_chunked_fwd(prep)");
+        gdrc_scan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, n0, nc, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, (bf16_t*)o,
+                                                                          n0 ? carry : initial_state, n0 + nc < all ? carry : final_state, keep, qs);
+        MI355_LAUNCH_CHECK("gdr_chunked_fwd");
+    }
     return 0;
 }
 

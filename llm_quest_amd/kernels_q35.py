@@ -288,7 +288,8 @@ def gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, Dk, Dv, keep=True,
     else:
         fin = torch.empty((B, Hv, Dv, Dk), dtype=F32, device=q.device) if want_state else None
     if chunked is not False and gdr_chunked(v, S, Dk, Dv) and not (q.data_ptr() | k.data_ptr() | (0 if fin is None else fin.data_ptr())) % 16:
-        saved = torch.empty(L.load().mi355_gdr_chunked_saved_bytes(B, S, Hv) // 4, dtype=F32, device=q.device)
+        need = L.load().mi355_gdr_chunked_saved_bytes if keep else L.load().mi355_gdr_chunked_scratch_bytes
+        saved = torch.empty(need(B, S, Hv) // 4, dtype=F32, device=q.device)
         L.call("mi355_gdr_chunked_fwd", B, S, Hqk, Hv, L.ptr(q), L.ptr(k), L.ptr(v), v.stride(0), L.ptr(beta), L.ptr(alpha), L.ptr(o), L.ptr(saved), saved.numel() * 4, int(keep), L.ptr(state), L.ptr(fin))
         return o, saved if keep else None, fin
     ck = None

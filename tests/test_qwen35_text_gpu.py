@@ -975,6 +975,40 @@ def test_chunked_gated_delta_rule_keeps_what_is_not_finite_to_the_rows_behind_it
     assert not bool(torch.isfinite(out[1][0]).all()) and bool(torch.isfinite(out[1][0][: (0 if what == "state" else at)]).all())
 
 
+@pytest.mark.parametrize("what", ["state kept", "state dropped", "not finite"])
+def test_chunked_gated_delta_rule_without_a_backward_goes_through_long_sequences_in_spans(what):
+    """A forward that keeps nothing has a scratch that does not grow with the sequence (here 18 chunks of 320 heads in spans of ten, 272 MiB for any length)
+    and the bits of the forward in one piece."""
+    from llm_quest_amd import _lib as L
+    from llm_quest_amd import kernels_q35 as Q
+
+    lib, b, hv, s, D = L.load(), 5, 64, 1100, 128
+    assert lib.mi355_gdr_chunked_scratch_bytes(b, s, hv) == lib.mi355_gdr_chunked_scratch_bytes(b, 10 * s, hv) < 272 << 20
+    assert lib.mi355_gdr_chunked_scratch_bytes(1, s, 16) < 64 << 20
+    g = torch.Generator(device="cuda").manual_seed(9)
+    r = lambda *z: torch.randn(*z, generator=g, device="cuda")
+    q, k = (torch.nn.functional.normalize(r(b * s, 2, D), dim=-1).to(BF16).reshape(b * s, -1) for _ in range(2))
+    v, be, al = r(b * s, hv * D).to(BF16), torch.sigmoid(r(b * s, hv)), torch.exp(-torch.exp(r(b * s, hv) - 3.0))
+    if what == "not finite":
+        v[2 * s + 700, 3] = float("nan")  # (the third sequence, second span)
+    s0 = r(b, hv, D, D)
+    o, _, fin = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, 2, hv, D, D, state=s0.clone(), chunked=None)
+    bits = lambda t: t.view(torch.int16 if t.dtype == BF16 else torch.int32)
+    if what == "state dropped":
+        zero, _, _ = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, 2, hv, D, D, chunked=None)
+        o2, _, none = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, 2, hv, D, D, keep=False, chunked=None)
+        assert none is None and torch.equal(bits(o2), bits(zero))
+    else:
+        o2, _, fin2 = Q.gated_delta_rule_fwd(q, k, v, be, al, b, s, 2, hv, D, D, keep=False, state=s0.clone(), chunked=None)
+        fine = torch.isfinite(o.float())
+        assert torch.equal(bits(fin2), bits(fin)) or what == "not finite"
+        assert torch.equal(fine, torch.isfinite(o2.float())) and torch.equal(torch.isfinite(fin), torch.isfinite(fin2)) and torch.isfinite(fin).any()
+        if what == "state kept":
+            assert torch.equal(bits(o2), bits(o))
+        else:  # (the NaN's column range goes token by token in both, the finite columns of it too)
+            assert not bool(fine.all()) and rel_l2(o2.float()[fine], o.float()[fine]) < 1e-3
+
+
 def test_chunked_gated_delta_rule_refuses_what_it_cannot_read():
     from llm_quest_amd import _lib as L
     from llm_quest_amd import kernels_q35 as Q
