@@ -28,7 +28,7 @@ __device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8]) {
 // ------------------------------------------------------------------------------------------- skinny GEMM (NT), M <= 8
 // A workgroup takes 16 weight rows at a time; its NW waves share k out in consecutive runs of `steps` x 32.  A weight row is an A row of v_mfma_f32_16x16x32_bf16, an operand row a
 // B column (eight of the sixteen stay idle: the pipe has nothing else to do), the waves' sums meet in LDS and are added in wave order -- which sums a result is made of
-// depends on N and K alone.  The operand rows go straight to fragments, finished there by the row operation that feeds the stream: PRO 1 RMSNorm(x[m]) * nw in the arithmetic
+// depends on N and K alone, for two to eight rows: one row goes through gemv_one_kernel, which sums in another order.  The operand rows go straight to fragments, finished there by the row operation that feeds the stream: PRO 1 RMSNorm(x[m]) * nw in the arithmetic
 // and summation order of rmsnorm_fwd_generic (norm_rope.hip; == rmsnorm_fwd_kernel<2> at width 1024), PRO 2 x holds gate-up rows [M, 2K] (up | gate, as the fused
 // lin1 | lin_gate projection writes them), swiglu_act(up, gate) as swiglu_fwd_kernel rounds it: fused == the two launches bit for bit.  GLU: W holds 2N rows (up | gate) and the
 // activation is the epilogue -- eight up rows and their gate rows make a group; every activation is worked out once, not once a workgroup.
@@ -700,8 +700,9 @@ extern "C" int mi355_gemv_bf16_pro(int M, int64_t N, int K, const void* x, int64
     MI355_REQUIRE(prologue == 1 || prologue == 2, "gemv_bf16_pro: prologue 1 (RMSNorm of x) or 2 (SwiGLU of gate-up rows), got %d", prologue);
     MI355_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= (prologue == 2 ? 2 * K : K) && ldw >= K && ldy >= N,
                   "gemv_bf16_pro: K and the leading dimensions must be multiples of 8 (x rows hold 2K elements under prologue 2)");
-    // (32 bytes beside the operand rows have always been refused with them: callers ask ops_decode.fused_rows, which knows that line)
-    MI355_REQUIRE((int64_t)M * K * 2 + 32 <= 65536, "gemv_bf16_pro: the operand rows (%d x %d bf16) plus 32 bytes of row sums exceed the 64 KiB LDS image", M, K);
+    // Where the entry ends, and ops_decode.fused_rows with it; beyond, the row operation has a launch of its own.  Only one row's activations (prologue 2) are in LDS as a whole; the line
+    // is where an earlier image of all rows ended, and is kept because it decides which launches, and so which bits, a step of that size has.
+    MI355_REQUIRE((int64_t)M * K * 2 + 32 <= 65536, "gemv_bf16_pro: takes operand rows (here %d x %d bf16) up to 64 KiB less 32 bytes", M, K);
     MI355_REQUIRE(x && W && y && (!residual || ldr >= N) && (prologue != 1 || norm_w), "gemv_bf16_pro: null pointer or residual pitch too small");
     if (prologue == 1) gemv_launch<1, false>(M, N, K, x, ldx, norm_w, eps, W, ldw, y, ldy, residual, ldr, stream);
     else gemv_launch<2, false>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);

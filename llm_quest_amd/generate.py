@@ -178,7 +178,9 @@ class RaggedBatch:
     """Scheduler of the serving models of ``registry`` (``model.step`` + ``utils.SlotStateCache``): sequences of different lengths run as ONE packed
     batch without padding.  A step brings, for every sequence in it, its next tokens -- a whole prompt for a sequence that starts, one token (or more) for
     one that goes on -- and returns fp32 logits of the rows asked for.  Sequences are named by the caller; ``finish`` gives a sequence's slot back, and
-    the next sequence to start takes it.  A row's logits do not depend on which other sequences share the step."""
+    the next sequence to start takes it.  A row's logits do not depend on which other sequences share the step, except
+    that in bf16 the step's rows and sequences pick the kernel of a product (one row, two to eight, tiles) and the parts that attention's keys are dealt to, and with them the order
+    of fp32 sums."""
 
     def __init__(self, model, max_tokens=0, slots=4, device=None):
         self.model = model

@@ -49,8 +49,8 @@ def gemv_pro(x2d, w, prologue, norm_w=None, eps=1e-6, residual=None):
 
 
 def fused_rows(M, Kd):
-    """Whether a one-token step of M sequences takes the fused streams (the operand rows must fit the kernel's 64-KiB LDS image)."""
-    return M <= 8 and M * Kd * 2 + 32 <= 65536  # (csrc/decode.hip: the operand image plus 32 bytes of row sums within 64 KiB)
+    """Whether a one-token step of M sequences takes the fused streams (``mi355_gemv_bf16_pro``: eight rows, 64 KiB of them less 32 bytes)."""
+    return M <= 8 and M * Kd * 2 + 32 <= 65536
 
 
 def decode_splits(n_keys, B, Hq):
