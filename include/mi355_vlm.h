@@ -358,7 +358,7 @@ int mi355_gdn_gates_bwd(int64_t tokens, int Hv, const void* b_lin, const void* a
 /* Depthwise causal Conv1d(kernel 4, left padding 3, cropped to S) + SiLU over the sequence axis of the token-major fused QKV
  * projection (qwen3_5_text_model.py:81-90,138-140).  x bf16 [B*S, C] row pitch ldx; w bf16 [C, 4]; y bf16 [B*S, C]. */
 int mi355_causal_conv_silu_fwd(int B, int S, int C, int ksize, const void* x, int64_t ldx, const void* w, void* y, void* stream);
-/* dc_ws bf16 [B*S, C] scratch (used where dx lies among x's or dy's rows); dx row pitch lddx; dw_partial fp32 [B*ceil(S/token_chunk), C*4]. */
+/* dc_ws bf16 [B*S, C] scratch where dx lies among x's or dy's rows (else it may be NULL); dx row pitch lddx; dw_partial fp32 [B*ceil(S/token_chunk), C*4]. */
 int mi355_causal_conv_silu_bwd(int B, int S, int C, int ksize, const void* x, int64_t ldx, const void* w, const void* dy, void* dc_ws, void* dx,
                                int64_t lddx, float* dw_partial, int token_chunk, void* stream);
 

@@ -6,10 +6,10 @@
 // Which sequences of a step go this way is their own number of new tokens' affair (`from`): beside a long prompt, a short one and a single token
 // get the bits that they get alone -- of the delta rule inside the scan's launch, whose long chains hide them; of retention by mi355_gla_fwd_below.
 // A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
-// the chip could multiply; the chunks take 363 us (prep 142, scan 203) and 183 us (scan 173).  Bound: the scan's chain of chunks (two products behind two barriers each), not the
+// the chip could multiply; the chunks take 359 us and 188 us.  Bound: the scan's chain of chunks (two products behind two barriers each), not the
 // pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
 // Chains of 128 products on the matrix pipe are cut (add16): outputs' distance to 64 bits, token by token | here with whole chains | here: 1.29e-7 | 2.32e-7 | 1.73e-7, decays near zero
-// 1.19e-7 | 2.27e-7 | 1.45e-7, nearly parallel keys 1.29e-7 | 2.67e-7 | 1.90e-7, decays near one 4.7e-7 | 5.0e-7 | 4.7e-7, retention 3.1e-7 | 3.0e-7 | 2.6e-7; the six prompts 363 -> 369 us.
+// 1.19e-7 | 2.27e-7 | 1.45e-7, nearly parallel keys 1.29e-7 | 2.67e-7 | 1.90e-7, decays near one 4.7e-7 | 5.0e-7 | 4.7e-7, retention 3.1e-7 | 3.0e-7 | 2.6e-7; 6 of the 363 us that the six prompts took.
 // A chunk whose U is not finite and all behind it go token by token inside the scan: the triangles' zeros are multiplied, not skipped, and a token's key, value, decay or beta that
 // is not finite would reach the rows before it.  (A query reaches its own row alone, a key under retention the rows behind it.)
 #include "delta_token.h"

@@ -1455,7 +1455,7 @@ extern "C" int mi355_causal_conv_silu_bwd(int B, int S, int C, int ksize, const 
                                           void* dx, int64_t lddx, float* dw_partial, int token_chunk, void* stream) {
     MI355_REQUIRE(B > 0 && S > 0 && C > 0 && C % 8 == 0 && ldx % 8 == 0 && lddx % 8 == 0 && ldx >= C && lddx >= C, "causal_conv_silu: channels and ld must be multiples of 8");
     MI355_REQUIRE(ksize == 4, "causal_conv_silu: kernel size %d not built (4 only)", ksize);
-    MI355_REQUIRE(x && w && dy && dc_ws && dx && dw_partial && token_chunk >= 1, "causal_conv_silu_bwd: bad arguments");
+    MI355_REQUIRE(x && w && dy && dx && dw_partial && token_chunk >= 1, "causal_conv_silu_bwd: bad arguments");
     // a chunk reads rows of its neighbours: where dx shares memory with x or dy it goes through dc_ws
     const int64_t rows = (int64_t)B * S;
     auto meets = [&](const void* p, int64_t ld, const void* out, int64_t ldo) {
@@ -1463,7 +1463,7 @@ extern "C" int mi355_causal_conv_silu_bwd(int B, int S, int C, int ksize, const 
         return a < d + (uintptr_t)(((rows - 1) * ldo + C) * 2) && d < a + (uintptr_t)(((rows - 1) * ld + C) * 2);
     };
     if (meets(x, ldx, dx, lddx) || meets(dy, C, dx, lddx)) {
-        MI355_REQUIRE(!meets(x, ldx, dc_ws, C) && !meets(dy, C, dc_ws, C), "causal_conv_silu_bwd: dc_ws must not overlap x or dy");
+        MI355_REQUIRE(dc_ws && !meets(x, ldx, dc_ws, C) && !meets(dy, C, dc_ws, C), "causal_conv_silu_bwd: where dx overlaps x or dy it takes dc_ws, which must not");
         if (int rc = mi355_causal_conv_silu_bwd(B, S, C, ksize, x, ldx, w, dy, dx, dc_ws, C, dw_partial, token_chunk, stream)) return rc;
         return mi355_copy2d(rows, (int64_t)C * 2, dc_ws, (int64_t)C * 2, dx, lddx * 2, stream);
     }

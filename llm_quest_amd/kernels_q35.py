@@ -222,7 +222,8 @@ def causal_conv_silu_bwd(x, w, dy, dx, B, S):
     C, ks = x.shape[1], w.shape[-1]
     if not (dy.dtype == BF16 and dy.is_contiguous() and tuple(dy.shape) == (B * S, C)) or tuple(dx.shape) != (B * S, C):
         raise ValueError("causal_conv_silu_bwd: dy contiguous bf16 [B*S, C], dx a [B*S, C] view")
-    ws = torch.empty((B * S, C), dtype=BF16, device=x.device)
+    mine = dx.untyped_storage().data_ptr()  # only a gradient that overwrites its operands needs scratch
+    ws = torch.empty((B * S, C), dtype=BF16, device=x.device) if mine in (x.untyped_storage().data_ptr(), dy.untyped_storage().data_ptr()) else None
     chunks = B * ((S + CONV_TOKEN_CHUNK - 1) // CONV_TOKEN_CHUNK)
     part = torch.empty((chunks, C * ks), dtype=F32, device=x.device)
     L.call("mi355_causal_conv_silu_bwd", B, S, C, ks, L.ptr(x), x.stride(0), L.ptr(w), L.ptr(dy), L.ptr(ws), L.ptr(dx), dx.stride(0), L.ptr(part), CONV_TOKEN_CHUNK)
@@ -269,7 +270,7 @@ GDR_CHUNKED_MIN = 64  # tokens from which the chunked kernels beat the token-by-
 
 def gdr_chunked(v, S, Dk, Dv):
     """Whether a layer's delta rule takes the chunked kernels (csrc/gdr_chunk.hip): heads of 128 | 128, value rows in 16-byte words, at least one whole chunk.
-    Both sides, forward + backward, 16 heads: one sequence of 64 tokens 151 / 139 us, of 333 779 / 240, four of 128 327 / 180, eight of 708 2 077 / 912."""
+    Both sides, forward + backward, 16 heads: one sequence of 64 tokens 151 / 139 us, of 333 779 / 240, four of 128 327 / 180, eight of 708 2 077 / 910."""
     return Dk == 128 and Dv == 128 and S >= GDR_CHUNKED_MIN and v.stride(0) % 8 == 0 and v.data_ptr() % 16 == 0
 
 

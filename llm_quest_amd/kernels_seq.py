@@ -134,7 +134,7 @@ DELTA_CHUNKED_MIN = 64  # new tokens of a sequence from which the chunked recurr
 def _delta_chunked(q, k, v, dk, dv, max_new):
     """Whether a step's recurrence takes the chunked kernels (csrc/delta_chunk.hip): heads of 128 | 128 on fp32 rows in 16-byte words, and a sequence with at least a whole chunk of
     new tokens (a last chunk is worked out as a whole one).  Of such a step the sequences with fewer new tokens still go token by token, as they do alone.  Both sides with 16 heads, token by token / in chunks: 64 tokens 53 / 44 us
-    (one decay per head: 41 / 20), 333 tokens 238 / 86 (182 / 51), six times 900 921 / 363 (504 / 183); below a chunk the delta rule loses: 32 tokens 31 / 41, six times 32 42 / 51."""
+    (one decay per head: 41 / 20), 333 tokens 238 / 86 (182 / 51), six times 900 921 / 359 (504 / 188); below a chunk the delta rule loses: 32 tokens 31 / 41, six times 32 42 / 51."""
     return (max_new >= DELTA_CHUNKED_MIN and q.shape[0] > 0 and dk == 128 and dv == 128 and q.dtype == k.dtype == v.dtype == F32 and not (q.stride(0) | k.stride(0)) % 4
             and not (q.data_ptr() | k.data_ptr()) % 16)
 

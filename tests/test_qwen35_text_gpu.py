@@ -254,6 +254,20 @@ def test_causal_conv_silu_backward_at_chunk_edges(B, S, C):
     assert torch.equal(over_x[:, :C], ref) and torch.equal(over_g, ref)
 
 
+def test_causal_conv_silu_backward_takes_scratch_only_where_it_overwrites_its_operands():
+    from llm_quest_amd import kernels_q35 as Q
+
+    rows, C = 4096, 1024
+    x, g, w, dx = (torch.randn(*z, device="cuda").to(BF16) for z in ((rows, C), (rows, C), (C, 1, 4), (rows, C)))
+    peak = []
+    for out in (dx, x):
+        torch.cuda.reset_peak_memory_stats()
+        before = torch.cuda.memory_allocated()
+        Q.causal_conv_silu_bwd(x, w, g, out, 1, rows)
+        peak.append(torch.cuda.max_memory_allocated() - before)
+    assert peak[1] - peak[0] == rows * C * 2 and peak[0] < rows * C * 2
+
+
 def test_l2norm():
     from llm_quest_amd import kernels_q35 as Q
 
