@@ -664,7 +664,7 @@ int mi355_delta_rule_ragged(int64_t tokens, int n_seq, const int* seq_off, const
  * or above (what is below counts as 1e-30).  workspace: mi355_delta_chunked_workspace_bytes, 16-byte aligned. */
 int mi355_delta_rule_tokens(int64_t tokens, int H, int G, int dk, const void* q, const void* k, int qk_dt, int64_t ldq, int64_t ldk, const void* b, const void* a, int ba_dt,
                             int64_t ldb, int64_t lda, const float* A_log, const float* dt_bias, float qscale, float* ws, void* stream);
-int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H);
+int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H, int from);
 int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, int from, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
                         const float* v, int64_t ldv, const float* tok, const float* head_decay, float qscale, float kscale, float* state, float* o, void* workspace,
                         int64_t workspace_bytes, void* stream);

@@ -163,7 +163,7 @@ SIGNATURES = {
 QUERIES = {
     "mi355_gated_delta_rule_chunk": ([], _I),
     "mi355_gated_delta_rule_bwd_workspace_bytes": ([_I, _I, _I, _I, _I], _L),
-    "mi355_delta_chunked_workspace_bytes": ([_L, _I, _I], _L),
+    "mi355_delta_chunked_workspace_bytes": ([_L, _I, _I, _I], _L),
     "mi355_gdr_chunked_saved_bytes": ([_I, _I, _I], _L),
     "mi355_gdr_chunked_scratch_bytes": ([_I, _I, _I], _L),
     "mi355_gdr_chunked_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),

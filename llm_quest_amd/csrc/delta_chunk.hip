@@ -31,11 +31,16 @@ struct DChunkArgs {
     float qscale, kscale;     // retention
     int H, G, heads;  // heads: of all sequences
     int from;         // sequences with fewer new tokens: retention leaves them alone, the delta rule goes token by token
+    int by_tokens;    // where a sequence's chunks lie (chunk_block)
     float *state, *o, *ws;
 };
 
-// chunks are packed: those of sequence s start at seq_off[s] / 64 + s (never less than the sum of the sequences' chunks before it)
-__device__ __forceinline__ float* chunk_block(const DChunkArgs& p, int s, int h, int n) { return p.ws + ((int64_t)(p.seq_off[s] / GC + s + n) * p.H + h) * D_BLOCK; }
+// Chunks are packed: those of sequence s start at seq_off[s] / 64 + s, never less than the chunks of the sequences before it.  Where most sequences are short ones (501 sequences of 564
+// tokens: 660 MB for the one that has chunks) at 2 seq_off[s] / 64: a sequence of 64 tokens and more has no more chunks than twice its tokens hold.
+__host__ __device__ __forceinline__ bool by_tokens(int64_t tokens, int n_seq, int from) { return from >= GC && tokens * 2 / GC < tokens / GC + n_seq; }
+__device__ __forceinline__ float* chunk_block(const DChunkArgs& p, int s, int h, int n) {
+    return p.ws + ((int64_t)((p.by_tokens ? p.seq_off[s] * 2 / GC : p.seq_off[s] / GC + s) + n) * p.H + h) * D_BLOCK;
+}
 
 template <bool DELTA>
 __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
@@ -287,22 +292,22 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
 
 }  // namespace
 
-extern "C" int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H) {
-    return tokens > 0 && n_seq > 0 && H > 0 ? (tokens / GC + n_seq) * (int64_t)H * D_BLOCK * 4 : 0;
+extern "C" int64_t mi355_delta_chunked_workspace_bytes(int64_t tokens, int n_seq, int H, int from) {
+    return tokens > 0 && n_seq > 0 && H > 0 ? (by_tokens(tokens, n_seq, from) ? tokens * 2 / GC : tokens / GC + n_seq) * (int64_t)H * D_BLOCK * 4 : 0;
 }
 
 extern "C" int mi355_delta_chunked(int64_t tokens, int n_seq, int max_new, int from, const int* seq_off, const int* slot, int H, int G, const float* q, int64_t ldq, const float* k, int64_t ldk,
                                    const float* v, int64_t ldv, const float* tok, const float* head_decay, float qscale, float kscale, float* state, float* o, void* workspace,
                                    int64_t workspace_bytes, void* stream) {
-    MI355_REQUIRE(tokens > 0 && n_seq > 0 && n_seq <= 65535 && (int64_t)n_seq * H <= (1 << 26) && max_new > 0 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && q && k && v && state && o && workspace &&
+    MI355_REQUIRE(tokens > 0 && tokens < (1 << 30) && n_seq > 0 && n_seq <= 65535 && (int64_t)n_seq * H <= (1 << 26) && max_new > 0 && seq_off && slot && H > 0 && H <= 65535 && G > 0 && H % G == 0 && q && k && v && state && o && workspace &&
                       (tok != nullptr) != (head_decay != nullptr),
                   "delta_chunked: bad arguments (either a decay per head or four numbers per token and head)");
     MI355_REQUIRE(ldq >= (int64_t)G * GD && ldk >= (int64_t)G * GD && ldv >= (int64_t)H * GD && ldq % 4 == 0 && ldk % 4 == 0, "delta_chunked: rows too short, or query / key pitches no multiple of 4");
     MI355_REQUIRE((((uintptr_t)q | (uintptr_t)k | (uintptr_t)tok | (uintptr_t)workspace) & 15) == 0, "delta_chunked: queries, keys and the workspace must be 16-byte aligned");
-    MI355_REQUIRE(workspace_bytes >= mi355_delta_chunked_workspace_bytes(tokens, n_seq, H), "delta_chunked: workspace too small (%lld bytes)", (long long)workspace_bytes);
+    MI355_REQUIRE(workspace_bytes >= mi355_delta_chunked_workspace_bytes(tokens, n_seq, H, from), "delta_chunked: workspace too small (%lld bytes)", (long long)workspace_bytes);
     DChunkArgs p;
     p.seq_off = seq_off, p.slot = slot, p.q = q, p.k = k, p.v = v, p.ldq = ldq, p.ldk = ldk, p.ldv = ldv, p.tok = (const f32x4*)tok, p.head_decay = head_decay;
-    p.qscale = qscale, p.kscale = kscale, p.H = H, p.G = G, p.heads = n_seq * H, p.from = from, p.state = state, p.o = o, p.ws = (float*)workspace;
+    p.qscale = qscale, p.kscale = kscale, p.H = H, p.G = G, p.heads = n_seq * H, p.from = from, p.by_tokens = by_tokens(tokens, n_seq, from), p.state = state, p.o = o, p.ws = (float*)workspace;
     const dim3 prep((max_new + GC - 1) / GC, H, n_seq), scan((unsigned)((n_seq * (int64_t)H + 7) / 8 * 32));
     if (tok) {
         dchunk_prep_kernel<true><<<prep, 256, 0, ST(stream)>>>(p);

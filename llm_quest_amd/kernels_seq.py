@@ -141,7 +141,7 @@ def _delta_chunked(q, k, v, dk, dv, max_new):
 
 def _run_chunked(q, k, v, tok, head_decay, qscale, kscale, seq_off, slot, state, o, H, G, max_new):
     T, n_seq = q.shape[0], slot.numel()
-    need = L.load().mi355_delta_chunked_workspace_bytes(T, n_seq, H)
+    need = L.load().mi355_delta_chunked_workspace_bytes(T, n_seq, H, DELTA_CHUNKED_MIN)
     ws = torch.empty(need // 4, dtype=F32, device=q.device)
     L.call("mi355_delta_chunked", T, n_seq, int(max_new), DELTA_CHUNKED_MIN, L.ptr(seq_off), L.ptr(slot), H, G, L.ptr(q), q.stride(0), L.ptr(k), k.stride(0), L.ptr(v), v.stride(0), L.ptr(tok), L.ptr(head_decay),
            float(qscale), float(kscale), L.ptr(state), L.ptr(o), L.ptr(ws), need)

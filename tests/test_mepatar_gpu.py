@@ -410,16 +410,17 @@ def test_recurrences_in_chunks_equal_those_by_token(rule, H, G, decay):
         assert row_err(chunked[at : at + n], want.reshape(n, -1)) < 1e-5
 
 
+@pytest.mark.parametrize("lens", [[1, 200, 63, 64, 1, 65], [1] * 20 + [64, 130] + [1] * 9 + [95, 65, 1, 129]], ids=["few", "many"])
 @pytest.mark.parametrize("rule,H,G", [("delta", 4, 2), ("retention", 3, 3)])
-def test_recurrences_of_a_sequence_do_not_know_what_shares_the_step(rule, H, G):
+def test_recurrences_of_a_sequence_do_not_know_what_shares_the_step(rule, H, G, lens):
     """Single tokens, portions below a chunk and long prompts in one step, heads of 128 | 128: every sequence's outputs and state are the bits that it gets in a step of its own."""
     from llm_quest_amd import kernels_seq as S
 
     g = torch.Generator().manual_seed(H)
-    D, lens, slots = 128, [1, 200, 63, 64, 1, 65], [4, 2, 0, 5, 1, 3]
+    D, slots = 128, [(5 * i + 2) % len(lens) for i in range(len(lens))] if len(lens) % 5 else list(range(len(lens)))[::-1]
     d = _Slots(lens, slots)
     x = torch.randn(sum(lens), (2 * G + H) * D, generator=g).to(DEV)
-    start = torch.randn(6, H, D, D, generator=g).to(DEV)
+    start = torch.randn(len(lens), H, D, D, generator=g).to(DEV)
     ba = (torch.randn(sum(lens), 2 * H, generator=g) * 2).to(DEV)
     A_log, dt_bias, dec = torch.full((H,), -2.0, device=DEV), torch.zeros(H, device=DEV), torch.linspace(0.5, 0.99, H, device=DEV)
 
