@@ -157,7 +157,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int n0, int ke
 // ------------------------------------------------------------------------------------------- scan: the state chunk by chunk, 32 value rows per workgroup
 // Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave.  Bound: the chain
 // of chunks -- reads in flight, then two products behind two barriers.  Everything a chunk reads first is requested at its top, all at once: 172 us at 8 x 708 tokens x 16
-// heads; requested a chunk ahead 189 (the registers spill), in two halves 187, and 177 with the value ranges of a head on different XCDs.
+// heads (167 before its chains were cut, and so measured: requested a chunk ahead 189, the registers spill; in two halves 187; the value ranges of a head on different XCDs 177).
 __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int n0, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                            const bf16_t* __restrict__ v, int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha, float* __restrict__ saved,
                                                            bf16_t* __restrict__ o, const float* initial_state, float* final_state, int keep, float qscale) {
