@@ -7,6 +7,7 @@ fallback.  ``build()`` compiles it in-tree with hipcc for gfx950 (cross-compiles
 import ctypes
 import os
 import subprocess
+import sys
 
 import torch
 
@@ -179,13 +180,21 @@ _lib = None
 
 def build(verbose=False, force=False):
     """Compile libmi355vlm.so in-tree (hipcc --offload-arch=gfx950); ``force``: every object, also where nothing changed."""
-    cmd = ["make", "-C", CSRC, "-j8"] + (["-B"] if force else [])
+    cmd = ["make", "-C", CSRC, "-j8", "PYTHON=" + sys.executable] + (["-B"] if force else [])
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError("building libmi355vlm.so failed:\n" + res.stdout[-4000:] + res.stderr[-4000:])
     if verbose:
         print(res.stdout[-2000:])
     return LIB_PATH
+
+
+try:
+    from . import _launch  # built beside the library (csrc/Makefile); without it the launches below go through ctypes, with the same results
+except ImportError:
+    _launch = None
+if not hasattr(torch._C, "_cuda_getDevice"):
+    _launch = None
 
 
 def load():
@@ -214,6 +223,8 @@ def load():
             raise
         fn.argtypes = argtypes
         fn.restype = ctypes.c_int
+        if _launch is not None:
+            _launch.bind(name, ctypes.cast(fn, _P).value)
     for name, (argtypes, restype) in QUERIES.items():
         try:
             fn = getattr(lib, name)
@@ -240,7 +251,7 @@ def ptr(t):
 
 import threading
 
-_tls = threading.local()  # .device: device of the tensors checked by this THREAD's last require_gpu() -- the launches that follow run there
+_tls = threading.local()  # .device: device of the tensors checked by this THREAD's last require_gpu() -- the launches that follow run there (with _launch: kept on its side)
 # (autograd runs one thread per device: a module-level global would let one thread's require_gpu steer another thread's launch)
 
 
@@ -257,14 +268,21 @@ def call(name, *args):
     ``require_gpu``: a wrapper that launches several kernels (a backward followed by its partial-sum reductions) checks its operands
     once and every launch of it lands on their device."""
     lib = load()
-    dev = getattr(_tls, "device", None)
+    if _launch is None:
+        dev = getattr(_tls, "device", None)
+    else:
+        dev = torch.device("cuda", _launch.device()) if _launch.device() >= 0 else None
     if dev is not None and dev.index is not None and dev.index != torch.cuda.current_device():
         with torch.cuda.device(dev):
             rc = getattr(lib, name)(*args, stream(dev))
     else:
         rc = getattr(lib, name)(*args, stream(dev))
     if rc != 0:
-        raise RuntimeError(f"{name} failed (rc={rc}): {lib.mi355_last_error().decode()}")
+        _fail(name, rc)
+
+
+def _fail(name, rc):
+    raise RuntimeError(f"{name} failed (rc={rc}): {load().mi355_last_error().decode()}")
 
 
 def require_gpu(*tensors):
@@ -283,7 +301,17 @@ def require_gpu(*tensors):
             dev = t.device
         elif t.device != dev:
             raise RuntimeError(f"llm_quest_amd ops: operands live on different devices ({dev} and {t.device})")
-    _tls.device = dev
+    if _launch is None:
+        _tls.device = dev
+    else:
+        _launch.set_device(-1 if dev is None else torch.cuda.current_device() if dev.index is None else dev.index)
+
+
+# The native forms of the three functions that every launch goes through (csrc/launch.cpp); what they do not take, they hand to those above.
+_python_call, _python_require_gpu = call, require_gpu
+if _launch is not None:
+    _launch.setup(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, _python_call, _python_require_gpu, _fail)
+    call, require_gpu, ptr = _launch.call, _launch.require_gpu, _launch.ptr
 
 
 def dt_code(dtype):

@@ -36,7 +36,7 @@ WS_BYTES = 512 << 20  # split-K scratch per device (fp32 slabs of the largest we
 
 def _workspace(device):
     """Split-K scratch of the (device, stream) the launch goes to: two streams issuing split-K GEMMs never share slabs."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, L.stream(device))
     ws = _WS.get(key)
     if ws is None:
         ws = torch.empty(WS_BYTES // 4, dtype=F32, device=device)
@@ -220,7 +220,7 @@ def gemm_grouped(form, problems, tile=0):
             if residual.dtype != odt or tuple(residual.shape) != (M, N):
                 raise ValueError("gemm_grouped: residual must match the output's shape and dtype")
             q.residual, q.ldr = residual.data_ptr(), residual.stride(0)
-    L.call("mi355_gemm_bf16_grouped", form, len(problems), _c.cast(table, _c.c_void_p), L.dt_code(odt), tile or _TILE_BY_FORM[form] or (_TILE_OVERRIDE if _TILE_OVERRIDE in (1, 3, 4, 5) else 0))
+    L.call("mi355_gemm_bf16_grouped", form, len(problems), _c.addressof(table), L.dt_code(odt), tile or _TILE_BY_FORM[form] or (_TILE_OVERRIDE if _TILE_OVERRIDE in (1, 3, 4, 5) else 0))
 
 
 # Measured (ViT-B/16 training step, B = 256, same box): fused 65.5 ms, separate kernels 64.1 ms -- erf / tanh in the epilogue sit on the tile's critical
@@ -431,7 +431,7 @@ def _attn_scratch(device, nbytes):
     allocated -- the caller then runs the recompute form.  A buffer more than 4x the request is replaced by a fitting one."""
     if nbytes > _ATTN_DS_SPILL_MAX:
         return None
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, L.stream(device))
     ws = _ATTN_WS.pop(key, None)
     if ws is not None and (ws.numel() < nbytes or ws.numel() > 4 * nbytes):
         ws = None
@@ -771,7 +771,7 @@ _SUMSQ_PARTS = {}
 
 def _sumsq_parts(device):
     """Per (device, stream) scratch of mi355_sumsq's per-block partial sums (4096 floats): calls on different streams never share one."""
-    key = (device, torch.cuda.current_stream(device).cuda_stream)
+    key = (device, L.stream(device))
     buf = _SUMSQ_PARTS.get(key)
     if buf is None:
         if len(_SUMSQ_PARTS) > 16:
