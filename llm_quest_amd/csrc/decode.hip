@@ -11,6 +11,7 @@
 //                   key and value head written to the cache row at the device-side position (qknorm_rope_fwd + kv_append + attn_decode in one launch)
 //   argmax_rows     greedy sampling: first index of the row maximum (torch.argmax tie rule on ties is unspecified; first is used)
 #include "common.h"
+#include "lane_sums.h"
 
 namespace {
 
@@ -26,7 +27,7 @@ __device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8]) {
 }
 
 // ------------------------------------------------------------------------------------------- skinny GEMM (NT), M <= 8
-// A workgroup takes 16 weight rows at a time; its NW waves share k out in consecutive runs of `steps` x 32.  A weight row is an A row of v_mfma_f32_16x16x32_bf16, an operand row a
+// A workgroup takes 16 weight rows (ROWS: or 8) at a time; its NW waves share k out in consecutive runs of `steps` x 32.  A weight row is an A row of v_mfma_f32_16x16x32_bf16, an operand row a
 // B column (eight of the sixteen stay idle: the pipe has nothing else to do), the waves' sums meet in LDS and are added in wave order -- which sums a result is made of
 // depends on N and K alone, for two to eight rows: one row goes through gemv_one_kernel, which sums in another order.  The operand rows go straight to fragments, finished there by the row operation that feeds the stream: PRO 1 RMSNorm(x[m]) * nw in the arithmetic
 // and summation order of rmsnorm_fwd_generic (norm_rope.hip; == rmsnorm_fwd_kernel<2> at width 1024), PRO 2 x holds gate-up rows [M, 2K] (up | gate, as the fused
@@ -43,7 +44,7 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
 }
 __device__ __forceinline__ float rbf(float x) { return bf2f(f2bf(x)); }
 
-template <int NW, int PRO, bool F32, bool GLU>
+template <int NW, int PRO, bool F32, bool GLU, int ROWS>
 __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, int steps, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ nw, float eps,
                                                        const bf16_t* __restrict__ W, int64_t ldw, void* __restrict__ y, int64_t ldy, const void* __restrict__ res, int64_t ldr) {
     constexpr int T = GEMV_STEPS;
@@ -53,7 +54,8 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = (lane >> 4) * 8;
     const int nvec = K >> 3, chunks = (steps + T - 1) / T;
     const int k_lo = wave * steps * 32, k_hi = min(K, k_lo + steps * 32);
-    constexpr int GN = GLU ? 8 : 16;  // columns of a group
+    constexpr int GN = GLU ? 8 : ROWS;  // columns of a group
+    const bool on = GLU || r16 < ROWS;  // lanes that hold a weight row
     const int64_t groups = (N + GN - 1) / GN;
     const u32x4 z4 = {0u, 0u, 0u, 0u};
     u32x4 xf[T], gf[PRO ? T : 1], w0[T], w1[T];
@@ -82,7 +84,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const int k = k_lo + (c * T + t) * 32 + kg;
-            w[t] = k < k_hi ? *reinterpret_cast<const u32x4*>(row + k) : z4;
+            w[t] = on && k < k_hi ? *reinterpret_cast<const u32x4*>(row + k) : z4;
         }
     };
     float r = 0.f;  // PRO 1: 1 / rms of the lane's operand row
@@ -196,10 +198,52 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
 // One operand row: a matrix pipe with one column at work gains nothing, and a row fits the registers of every wave in the layout of the weights' strips (512 k, 8 per lane), so
 // there is neither an image nor a barrier between the loads and the products (PRO 2 alone shares its activations through LDS: each costs ~ 100 clocks).  One wave = one
 // column (GLU: an up column and its gate column), the workgroups walk the columns.  Arithmetic of the prologues and of GLU as above; a sum is a lane's strips in order, then wave_sum.
+// PRO 3: the row is a context that the decode attention left in `fold.S` splits; every workgroup folds it, as attn_decode_combine_kernel would (the same bits), into LDS -- S x 8 KB
+// from L2 under the weights' flight against a launch of its own: at 590 keys in five splits 3.3 us and the gap behind it.
+struct SplitRow {
+    const float* ws; int D, S;
+};
+__device__ __forceinline__ void fold_splits8(const SplitRow& fold, int k, float (&o)[8]) {  // features k .. k + 7 (of one head)
+    const int head = k / fold.D, i = k - head * fold.D, pitch = fold.D + 2;
+    const float* src = fold.ws + (int64_t)head * fold.S * pitch;
+    constexpr int AT = 8;  // splits requested at a time
+    float ms[AT], ls[AT];
+    f32x2 v[AT][4];
+    auto request = [&](int s0) {
+#pragma unroll
+        for (int j = 0; j < AT; ++j) {
+            const float* p = src + min(s0 + j, fold.S - 1) * pitch;
+            ms[j] = p[fold.D], ls[j] = p[fold.D + 1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[j][e] = *reinterpret_cast<const f32x2*>(p + i + 2 * e);
+        }
+    };
+    request(0);
+    float mg = -__builtin_huge_valf();
+#pragma unroll
+    for (int j = 0; j < AT; ++j) mg = fmaxf(mg, ms[j]);
+    for (int s = AT; s < fold.S; ++s) mg = fmaxf(mg, src[s * pitch + fold.D]);
+    float lg = 0.f, out[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) out[e] = 0.f;
+    for (int s0 = 0; s0 < fold.S; s0 += AT) {
+        if (s0) request(s0);
+#pragma unroll
+        for (int j = 0; j < AT; ++j) {
+            if (s0 + j >= fold.S) break;
+            const float f = ms[j] == -__builtin_huge_valf() ? 0.f : exp2f(ms[j] - mg);  // (a split without keys)
+            lg += ls[j] * f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) out[e] += v[j][e >> 1][e & 1] * f;
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[e] = out[e] / lg;
+}
 template <int T, int PRO, bool F32, bool GLU>
 __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const bf16_t* __restrict__ x, const bf16_t* __restrict__ nw, float eps, const bf16_t* __restrict__ W, int64_t ldw,
-                                                       void* __restrict__ y, const void* __restrict__ res) {
-    extern __shared__ __attribute__((aligned(16))) bf16_t act[];  // PRO 2: [K]
+                                                       void* __restrict__ y, const void* __restrict__ res, SplitRow fold) {
+    extern __shared__ __attribute__((aligned(16))) bf16_t act[];  // PRO 2, 3: [K]
     constexpr int C = GLU ? 2 : 1;  // columns of a wave; T strips in registers (the smallest of 2, 4, 8 that holds the row; longer rows go through eight at a time)
     const int lane = threadIdx.x & 63, its = (K + 511) >> 9;
     const u32x4 z4 = {0u, 0u, 0u, 0u};
@@ -208,7 +252,7 @@ __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const b
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const int k = (base + t) * 512 + lane * 8;
-            xr[t] = k < K ? *reinterpret_cast<const u32x4*>((PRO == 2 ? act : x) + k) : z4;
+            xr[t] = k < K ? *reinterpret_cast<const u32x4*>((PRO >= 2 ? act : x) + k) : z4;
             if constexpr (PRO == 1) nr[t] = k < K ? *reinterpret_cast<const u32x4*>(nw + k) : z4;
         }
     };
@@ -248,9 +292,18 @@ __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const b
         }
         __syncthreads();
     }
+    if constexpr (PRO == 3) {
+        request_w(n < N ? n : N - 1, 0);
+        for (int k = threadIdx.x * 8; k < K; k += 2048) {
+            float o[8];
+            fold_splits8(fold, k, o);
+            *reinterpret_cast<u32x4*>(act + k) = pack8(o);
+        }
+        __syncthreads();
+    }
     if (n >= N) return;  // (no barrier behind this)
     request_x(0);
-    request_w(n, 0);
+    if constexpr (PRO != 3) request_w(n, 0);
     if constexpr (PRO == 1) {
         float ss = 0.f, v[8];
 #pragma unroll
@@ -312,44 +365,58 @@ struct QkvPost {
     const bf16_t* qkv; int64_t ldqkv; const bf16_t* qw; const bf16_t* kw; const float* cosT; const float* sinT; const int32_t* pos; const int32_t* write_pos; int capacity; float eps;
 };
 
-// QK-RMSNorm + RoPE of one head in two stages (request the operands; later, finish): lanes 0 .. LPH-1 hold the head, 8 features of each half per lane.
+// Sums and maxima over lanes on the VALU: a ds_bpermute (what __shfl_xor compiles to) is an LDS round trip, and a one-token step's attention is a chain of them.
+__device__ __forceinline__ float other16(float v, bool max) {  // with the lane whose number differs in bit 4
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return max ? fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) : __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float other32(float v, bool max) {
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return max ? fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1])) : __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+template <int CH>
+__device__ __forceinline__ float chunk_sum(float v) {  // over the CH lanes that hold a key's features
+    if constexpr (CH <= 16) return lanes_sum<CH>(v);
+    else return other16(lanes_sum<16>(v), false);
+}
+template <int CH>
+__device__ __forceinline__ float across_groups(float v, bool max) {  // over the 64 / CH lanes of one chunk
+#pragma unroll
+    for (int o = CH; o < 16; o <<= 1) {
+        const float w = __shfl_xor(v, o, 64);
+        v = max ? fmaxf(v, w) : v + w;
+    }
+    if constexpr (CH <= 16) v = other16(v, max);
+    return other32(v, max);
+}
+
+// QK-RMSNorm + RoPE of one head in two stages (request the operands; later, finish): lane i < D / 2 holds features i and D / 2 + i.  The bits of qknorm_rope_fwd_kernel
+// (norm_rope.hip), whose lanes hold eight features of each half: the sum of squares is taken in that order -- eight neighbours one after the other, then the groups of eight in a
+// tree -- but an element's arithmetic runs once, not eight times over (a wave's whole norm and rotation 1 500 -> 500 clocks, at the head of a one-token step's chain).
 struct HeadOperands {
-    u32x4 w1, w2, x1, x2;
-    f32x4 c1a, c1b, s1a, s1b, c2a, c2b, s2a, s2b;
+    bf16_t w1, w2, x1, x2;
+    float c1, s1, c2, s2;
     template <int D>
     __device__ __forceinline__ void load(const bf16_t* __restrict__ src, const bf16_t* __restrict__ w, const float* __restrict__ cosT, const float* __restrict__ sinT, int64_t p, int lane) {
-        constexpr int HALF = D / 2, LPH = HALF / 8;
-        const int i = (lane % LPH) * 8;
-        x1 = *reinterpret_cast<const u32x4*>(src + i);
-        x2 = *reinterpret_cast<const u32x4*>(src + HALF + i);
-        w1 = *reinterpret_cast<const u32x4*>(w + i);
-        w2 = *reinterpret_cast<const u32x4*>(w + HALF + i);
-        const f32x4 *c1 = reinterpret_cast<const f32x4*>(cosT + p * D + i), *s1 = reinterpret_cast<const f32x4*>(sinT + p * D + i);
-        const f32x4 *c2 = reinterpret_cast<const f32x4*>(cosT + p * D + HALF + i), *s2 = reinterpret_cast<const f32x4*>(sinT + p * D + HALF + i);
-        c1a = c1[0]; c1b = c1[1]; s1a = s1[0]; s1b = s1[1]; c2a = c2[0]; c2b = c2[1]; s2a = s2[0]; s2b = s2[1];
+        constexpr int HALF = D / 2;
+        const int i = lane % HALF;
+        x1 = src[i], x2 = src[HALF + i], w1 = w[i], w2 = w[HALF + i];
+        c1 = cosT[p * D + i], s1 = sinT[p * D + i], c2 = cosT[p * D + HALF + i], s2 = sinT[p * D + HALF + i];
     }
     template <int D>
-    __device__ __forceinline__ void finish(float eps, float (&y1)[8], float (&y2)[8]) const {
-        constexpr int HALF = D / 2, LPH = HALF / 8;
-        float wf1[8], wf2[8], xf1[8], xf2[8], cb1[8], sb1[8], cb2[8], sb2[8];
-        unpack8(w1, wf1); unpack8(w2, wf2); unpack8(x1, xf1); unpack8(x2, xf2);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-            cb1[e] = rbf(c1a[e]); cb1[4 + e] = rbf(c1b[e]); sb1[e] = rbf(s1a[e]); sb1[4 + e] = rbf(s1b[e]);
-            cb2[e] = rbf(c2a[e]); cb2[4 + e] = rbf(c2b[e]); sb2[e] = rbf(s2a[e]); sb2[4 + e] = rbf(s2b[e]);
-        }
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) ss += xf1[e] * xf1[e] + xf2[e] * xf2[e];
-#pragma unroll
-        for (int o = LPH / 2; o > 0; o >>= 1) ss += __shfl_xor(ss, o, 64);
+    __device__ __forceinline__ void finish(float eps, float& y1, float& y2) const {
+        const float xf1 = bf2f(x1), xf2 = bf2f(x2), t = xf1 * xf1 + xf2 * xf2;
+        float ss = 0.f;  // of eight lanes, at the first of them (row_shl:k brings the value of the lane k further on)
+        ss += t;
+        ss += dpp_f<0x101>(t), ss += dpp_f<0x102>(t), ss += dpp_f<0x103>(t), ss += dpp_f<0x104>(t), ss += dpp_f<0x105>(t), ss += dpp_f<0x106>(t), ss += dpp_f<0x107>(t);
+        if constexpr (D == 128) ss = other32(ss, false);
+        ss = other16(ss, false);
+        ss += dpp_f<0x128>(ss);  // row_ror:8
+        ss = __int_as_float(__builtin_amdgcn_readfirstlane(__float_as_int(ss)));
         const float r = rsqrtf(ss / (float)D + eps);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-            const float n1 = rbf(xf1[e] * r * wf1[e]), n2 = rbf(xf2[e] * r * wf2[e]);
-            y1[e] = rbf(rbf(cb1[e] * n1) + rbf(sb1[e] * (-n2)));
-            y2[e] = rbf(rbf(cb2[e] * n2) + rbf(sb2[e] * n1));
-        }
+        const float n1 = rbf(xf1 * r * bf2f(w1)), n2 = rbf(xf2 * r * bf2f(w2));
+        y1 = rbf(rbf(rbf(c1) * n1) + rbf(rbf(s1) * (-n2)));
+        y2 = rbf(rbf(rbf(c2) * n2) + rbf(rbf(s2) * n1));
     }
 };
 
@@ -358,93 +425,84 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(int Hq, int Hkv
                                                                  int64_t ld, int len, const int32_t* __restrict__ len_dev, const uint8_t* __restrict__ key_mask, int64_t ldm,
                                                                  bf16_t* __restrict__ o, float scale_log2, QkvPost post, float* __restrict__ ws) {
     // One mapping for both products: lane = (key group kg, 16-byte feature chunk ch); a load instruction covers KG whole key rows, coalesced.  Scores: 8 features per lane,
-    // folded over the CH lanes of a key by a butterfly, so every lane of a key group holds the scores of its NT keys and the probabilities never leave registers.
-    // A one-token step is a chain of memory round trips, so the chain is kept at two: (1) the device-side length / positions, (2) EVERYTHING else at once -- the wave's
-    // first chunk of key AND value rows is requested before the query exists (and before the QKV post-processing of POST runs); the new token's own key / value never
-    // come back from memory (POST: they are used from LDS, the cache row is written for the later steps only).
+    // folded over the CH lanes of a key; P V: the key groups are folded at the end.  Rows of the new token never come back from memory (POST: they are used from LDS, the cache
+    // row is written for the later steps only).
+    // Bound: one wave's chain -- arguments, position, angles, norm and rotation; cache rows; scores, softmax, P V -- of which the arithmetic was the longer half (a wave's vector
+    // instruction takes four clocks whatever it does): few keys per wave, no per-lane branch round a load, the new token's norm and rotation on waves without keys.  Eight keys a
+    // lane and everything behind the position's load -> now: 1 sequence x 100 keys 8.2 -> 5.4 us, 6 x 80 8.3 -> 5.5, 590 keys in three splits 9.5 -> 6.7, in five 5.8.  (Sixteen waves
+    // instead of a second round: 7.3 for the 6.7.)
     constexpr int CH = D / 8, KG = 64 / CH;
-    constexpr int NT = CH < 8 ? CH : 8;    // keys per lane and chunk: 2 x NT 16-byte rows in flight per lane
-    constexpr int CK = NT * KG;           // keys per chunk; chunk c belongs to split c % S (blockIdx.z of S = gridDim.z), there to wave (c / S) % WAVES
-    // S > 1 (long caches; a workgroup streams ~ 256 keys per memory round trip): every split leaves its un-normalised context, maximum and sum in `ws`
-    // ([B, Hq, S, D + 2] floats), attn_decode_combine_kernel folds them in split order.
+    constexpr int NT = 4;        // keys per lane and chunk: 2 x NT 16-byte rows in flight per lane
+    constexpr int CK = NT * KG;  // keys per chunk; chunk c belongs to split c % S (blockIdx.z of S = gridDim.z), there to wave (c / S) % WAVES
+    // S > 1 (long caches): every split leaves its un-normalised context, maximum and sum in `ws` ([B, Hq, S, D + 2] floats), folded in split order by who reads them.
     __shared__ float qs[D];
-    __shared__ float ksn[POST ? D : 1], vsn[POST ? D : 1];
+    __shared__ __attribute__((aligned(16))) bf16_t ksn[POST ? D : 8], vsn[POST ? D : 8];
     __shared__ float part[WAVES][D + 2];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int kg = lane / CH, ch = lane % CH;
     const int h = blockIdx.x, b = blockIdx.y, hk = h / (Hq / Hkv);
     const int S = gridDim.z, sp = blockIdx.z;
     const int c0 = sp + S * wave, cstep = S * WAVES;
-    if (len_dev) len = min(len, *len_dev);  // graph replay: the current length lives on the device, `len` is the capacity bound
-    int wp = -1;                            // POST: the cache row of the new token (its key / value are taken from LDS)
-    int64_t p = 0;
-    if constexpr (POST) {
-        wp = *post.write_pos;
-        p = post.pos[b];
-    }
+    // A wave's first rows are requested by the bound that the host knows, in front of what the device alone knows (the length, the new token's row and position: a memory round
+    // trip), where the bound is no longer than four rounds of the workgroups; what is read past the length is dropped below.  POST: the row at the bound's end is left out, for
+    // where the host knows the length it is the new token's, being written now by the heads that share it.
+    const bool early = len <= 4 * CK * WAVES * S;
+    const int bound = len;
+    int first = POST ? max(bound - 1, 1) : bound;
+    if (!early && len_dev) first = min(bound, *len_dev);
+    int wp = -1;  // POST: the cache row of the new token (its key / value are taken from LDS)
     const bf16_t* kb = kc + b * batch_stride + (int64_t)hk * D + ch * 8;
     const bf16_t* vb = vc + b * batch_stride + (int64_t)hk * D + ch * 8;
     u32x4 kraw[NT], vraw[NT];
-    auto request_k = [&](int base) {
+    auto request = [&](u32x4 (&r)[NT], const bf16_t* from, int base, int bound) {  // (rows past the bound: the last one; the new token's row, being written now, is read and not used)
+        if (base >= bound) return;
 #pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int j = base + t * KG + kg;
-            kraw[t] = (j < len && j != wp) ? *reinterpret_cast<const u32x4*>(kb + (int64_t)j * ld) : (u32x4){0u, 0u, 0u, 0u};
-        }
-    };
-    auto request_v = [&](int base) {
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-            const int j = base + t * KG + kg;
-            vraw[t] = (j < len && j != wp) ? *reinterpret_cast<const u32x4*>(vb + (int64_t)j * ld) : (u32x4){0u, 0u, 0u, 0u};
-        }
+        for (int t = 0; t < NT; ++t) r[t] = *reinterpret_cast<const u32x4*>(from + (int64_t)min(base + t * KG + kg, bound - 1) * ld);
     };
     if constexpr (POST) {
         static_assert(D == 64 || D == 128, "QK-norm + RoPE geometry: 8 features per lane and half");
-        constexpr int HALF = D / 2, LPH = HALF / 8;
-        const bool room = wp >= 0 && wp < post.capacity;  // never write outside the cache
+        constexpr int HALF = D / 2;
         const bf16_t* row = post.qkv + b * post.ldqkv;
-        const int i = (lane % LPH) * 8;
-        // loads return in order: the post-processing operands (hot in L2) are requested in front of the cache rows (HBM), their arithmetic runs under the rows' flight
+        // The last waves, which short caches leave without keys, finish the query, the new key and the new value.  Loads return in order: their operands are requested in front
+        // of their cache rows, and their arithmetic runs under the rows' flight.
         HeadOperands hop;
         u32x4 vnew = {0u, 0u, 0u, 0u};
-        if (wave == 0) hop.load<D>(row + (int64_t)h * D, post.qw, post.cosT, post.sinT, p, lane);
-        else if (wave == 1) hop.load<D>(row + (int64_t)(Hq + hk) * D, post.kw, post.cosT, post.sinT, p, lane);
-        else if (wave == 2 && lane < D / 8) vnew = *reinterpret_cast<const u32x4*>(row + (int64_t)(Hq + Hkv + hk) * D + lane * 8);
-        request_k(c0 * CK);
-        request_v(c0 * CK);
-        if (wave == 0) {
-            float y1[8], y2[8];
+        const int role = WAVES - 1 - wave;
+        if (role < 2) hop.load<D>(row + (int64_t)(role == 0 ? h : Hq + hk) * D, role == 0 ? post.qw : post.kw, post.cosT, post.sinT, post.pos[b], lane);
+        else if (role == 2 && lane < D / 8) vnew = *reinterpret_cast<const u32x4*>(row + (int64_t)(Hq + Hkv + hk) * D + lane * 8);
+        request(kraw, kb, c0 * CK, first);
+        request(vraw, vb, c0 * CK, first);
+        wp = *post.write_pos;
+        len = min(len, *len_dev);
+        const bool room = wp >= 0 && wp < post.capacity;  // never write outside the cache
+        if (early && len == bound && wp != bound - 1) {   // (the row that was left out is an old one)
+            request(kraw, kb, c0 * CK, bound);
+            request(vraw, vb, c0 * CK, bound);
+        }
+        if (role < 2) {
+            float y1, y2;
             hop.finish<D>(post.eps, y1, y2);
-            if (lane < LPH) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { qs[i + e] = y1[e]; qs[HALF + i + e] = y2[e]; }
-            }
-        } else if (wave == 1) {
-            float y1[8], y2[8];
-            hop.finish<D>(post.eps, y1, y2);
-            if (lane < LPH) {
-#pragma unroll
-                for (int e = 0; e < 8; ++e) { ksn[i + e] = y1[e]; ksn[HALF + i + e] = y2[e]; }
-                if (room) {
-                    bf16_t* dst = const_cast<bf16_t*>(kc) + b * batch_stride + (int64_t)wp * ld + (int64_t)hk * D;
-                    *reinterpret_cast<u32x4*>(dst + i) = pack8(y1);
-                    *reinterpret_cast<u32x4*>(dst + HALF + i) = pack8(y2);
+            if (lane < HALF) {
+                if (role == 0) {
+                    qs[lane] = y1, qs[HALF + lane] = y2;
+                } else {
+                    const bf16_t p1 = f2bf(y1), p2 = f2bf(y2);
+                    ksn[lane] = p1, ksn[HALF + lane] = p2;
+                    if (room) {
+                        bf16_t* dst = const_cast<bf16_t*>(kc) + b * batch_stride + (int64_t)wp * ld + (int64_t)hk * D;
+                        dst[lane] = p1, dst[HALF + lane] = p2;
+                    }
                 }
             }
-        } else if (wave == 2) {
-            if (lane < D / 8) {
-                float vf[8];
-                unpack8(vnew, vf);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) vsn[lane * 8 + e] = vf[e];
-                if (room) *reinterpret_cast<u32x4*>(const_cast<bf16_t*>(vc) + b * batch_stride + (int64_t)wp * ld + (int64_t)hk * D + lane * 8) = vnew;
-            }
+        } else if (role == 2 && lane < D / 8) {
+            *reinterpret_cast<u32x4*>(vsn + lane * 8) = vnew;
+            if (room) *reinterpret_cast<u32x4*>(const_cast<bf16_t*>(vc) + b * batch_stride + (int64_t)wp * ld + (int64_t)hk * D + lane * 8) = vnew;
         }
     } else {
         for (int i = threadIdx.x; i < D; i += 64 * WAVES) qs[i] = bf2f(q[((int64_t)b * Hq + h) * D + i]);
-        request_k(c0 * CK);
-        request_v(c0 * CK);
+        request(kraw, kb, c0 * CK, first);
+        request(vraw, vb, c0 * CK, first);
+        if (len_dev) len = min(len, *len_dev);  // graph replay: the current length lives on the device, `len` is the capacity bound
     }
     __syncthreads();
     const uint8_t* km = key_mask ? key_mask + b * ldm : nullptr;
@@ -456,65 +514,59 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(int Hq, int Hkv
     for (int e = 0; e < 8; ++e) acc[e] = 0.f;
     for (int base = c0 * CK; base < len; base += cstep * CK) {
         const int nb = base + cstep * CK;
+        u32x4 kn = {0u, 0u, 0u, 0u}, vn = kn;
+        if constexpr (POST) kn = *reinterpret_cast<const u32x4*>(ksn + ch * 8), vn = *reinterpret_cast<const u32x4*>(vsn + ch * 8);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {  // (selects, no branches: cold code would cost the one wave that meets the new token or the end more than these cost all)
+            const int j = base + t * KG + kg;
+            if constexpr (POST) kraw[t] = j == wp ? kn : kraw[t], vraw[t] = j == wp ? vn : vraw[t];
+            vraw[t] = j < len ? vraw[t] : u32x4{0u, 0u, 0u, 0u};  // (a probability of 0 times whatever lies there)
+        }
         float sc[NT];
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const int j = base + t * KG + kg;
             float kf[8];
             unpack8(kraw[t], kf);
-            if constexpr (POST) {
-                if (j == wp) {
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) kf[e] = ksn[ch * 8 + e];
-                }
-            }
             float d = 0.f;
 #pragma unroll
             for (int e = 0; e < 8; ++e) d = fmaf(kf[e], qf[e], d);
-#pragma unroll
-            for (int o = 1; o < CH; o <<= 1) d += __shfl_xor(d, o, 64);
-            sc[t] = j < len ? ((km && !km[j]) ? MASK_T : d * scale_log2) : -__builtin_huge_valf();  // keys beyond the cache do not exist
+            sc[t] = chunk_sum<CH>(d) * scale_log2;
         }
-        if (nb < len) request_k(nb);  // the next round's rows travel under this round's arithmetic
-        float mc = sc[0];
+        if (nb < len) request(kraw, kb, nb, len);  // the next round's rows travel under this round's arithmetic
+        if (km) {
 #pragma unroll
-        for (int t = 1; t < NT; ++t) mc = fmaxf(mc, sc[t]);
+            for (int t = 0; t < NT; ++t)
+                if (!km[min(base + t * KG + kg, len - 1)]) sc[t] = MASK_T;
+        }
 #pragma unroll
-        for (int o = CH; o < 64; o <<= 1) mc = fmaxf(mc, __shfl_xor(mc, o, 64));
+        for (int t = 0; t < NT; ++t) sc[t] = base + t * KG + kg < len ? sc[t] : -__builtin_huge_valf();  // keys beyond the cache do not exist
+        float mc = fmaxf(fmaxf(sc[0], sc[1]), fmaxf(sc[2], sc[3]));
+        mc = across_groups<CH>(mc, true);
         const float mn = fmaxf(m, mc);
-        const float alpha = exp2f(m - mn);  // m = -inf on the first chunk -> 0
+        const float alpha = __builtin_amdgcn_exp2f(m - mn);  // m = -inf on the first chunk -> 0
         float psum = 0.f;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            sc[t] = exp2f(sc[t] - mn);  // -inf -> 0
+            sc[t] = __builtin_amdgcn_exp2f(sc[t] - mn);  // -inf -> 0
             psum += sc[t];
         }
-#pragma unroll
-        for (int o = CH; o < 64; o <<= 1) psum += __shfl_xor(psum, o, 64);
+        psum = across_groups<CH>(psum, false);
         l = l * alpha + psum;
         m = mn;
 #pragma unroll
         for (int e = 0; e < 8; ++e) acc[e] *= alpha;
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
-            const int j = base + t * KG + kg;
             float vf[8];
             unpack8(vraw[t], vf);
-            if constexpr (POST) {
-                if (j == wp) {
 #pragma unroll
-                    for (int e = 0; e < 8; ++e) vf[e] = vsn[ch * 8 + e];
-                }
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) acc[e] = fmaf(sc[t], vf[e], acc[e]);  // rows beyond the cache: probability 0 times a zero row
+            for (int e = 0; e < 8; ++e) acc[e] = fmaf(sc[t], vf[e], acc[e]);
         }
-        if (nb < len) request_v(nb);
+        if (nb < len) request(vraw, vb, nb, len);
     }
     // fold the key groups of the wave (lanes with the same chunk), then combine the waves' key ranges
 #pragma unroll
-    for (int e = 0; e < 8; ++e)
-        for (int o = CH; o < 64; o <<= 1) acc[e] += __shfl_xor(acc[e], o, 64);
+    for (int e = 0; e < 8; ++e) acc[e] = across_groups<CH>(acc[e], false);
     if (kg == 0) {
 #pragma unroll
         for (int e = 0; e < 8; ++e) part[wave][ch * 8 + e] = acc[e];
@@ -525,12 +577,13 @@ __global__ __launch_bounds__(64 * WAVES) void attn_decode_kernel(int Hq, int Hkv
     }
     __syncthreads();
     for (int i = threadIdx.x; i < D; i += 64 * WAVES) {
-        float mg = -__builtin_huge_valf();
-        for (int w = 0; w < WAVES; ++w) mg = fmaxf(mg, part[w][D]);
+        float mw[WAVES], mg = -__builtin_huge_valf();
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) mg = fmaxf(mg, mw[w] = part[w][D]);
         float lg = 0.f, out = 0.f;
+#pragma unroll
         for (int w = 0; w < WAVES; ++w) {
-            const float mw = part[w][D];
-            const float f = mw == -__builtin_huge_valf() ? 0.f : exp2f(mw - mg);
+            const float f = mw[w] == -__builtin_huge_valf() ? 0.f : __builtin_amdgcn_exp2f(mw[w] - mg);
             lg += part[w][D + 1] * f;
             out += part[w][i] * f;
         }
@@ -651,27 +704,38 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(const float* __restric
 #define ST(s) ((hipStream_t)(s))
 
 // One row: gemv_one_kernel.  Two to eight: eight waves and at most a workgroup for each CU; four waves and two workgroups a CU where they walk many groups (a table of 151 936
-// rows: 56 us so, 64 with eight waves and 59 with four workgroups; 6144 x 1024: 7.9 us with eight waves, 8.7 with four; sixteen waves spill under a prologue).
-// us of one launch, weights from memory, before (a column per wave on the vector pipe for up to eight rows) -> now:   N x K      1 row          6 rows
+// rows: 56 us so, 64 with eight waves and 59 with four workgroups; 6144 x 1024: 7.9 us with eight waves, 8.7 with four; sixteen waves spill under a prologue).  Twelve waves where
+// eight would take a second chunk and half of it empty (K of 2 049 to 3 072): its operands are only requested behind the first one's products.  Groups of eight weight rows, not
+// sixteen, while those leave half the CUs without one: a CU's loads, 64 bytes a clock, are what a group takes longest for.  Both together: 1024 x 2048 and 1024 x 3072, six rows, 5.7
+// us in the mean of the two (by the profiler's clock) -> 4.4 and 5.4.  How many waves share a sum depends on N and K alone, so a product with its prologue keeps the bits of the two launches.
+// us of one launch, weights from memory, before (a column per wave on the vector pipe for up to eight rows) -> the matrix pipe in groups of 16:   N x K      1 row          6 rows
 //     RMSNorm + 4096 x 1024    4.9 -> 4.5     9.0 -> 6.2          |   1024 x 3072 (from activated rows)    4.6 -> 3.5     7.9 -> 5.8
 //     RMSNorm + 6144 x 1024    6.6 -> 5.7    11.3 -> 7.9          |   1024 x 2048                          3.8 -> 2.9     6.3 -> 4.5
 //     RMSNorm + 151936 x 1024   52 -> 52      152 -> 56           |   3072 x 4096                          8.5 -> 7.1    14.0 -> 9.0
 template <int PRO, bool F32, bool GLU = false>
-static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, const void* nw, float eps, const void* W, int64_t ldw, void* y, int64_t ldy, const void* res, int64_t ldr, void* stream) {
+static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, const void* nw, float eps, const void* W, int64_t ldw, void* y, int64_t ldy, const void* res, int64_t ldr, void* stream, SplitRow fold = {}) {
     if (M == 1) {
         const int64_t blocks = (N + 3) / 4;
-#define GEMV(T) gemv_one_kernel<T, PRO, F32, GLU><<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO == 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res)
+#define GEMV(T) gemv_one_kernel<T, PRO, F32, GLU><<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO >= 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res, fold)
         if (K <= 1024) GEMV(2); else if (K <= 2048) GEMV(4); else GEMV(8);
 #undef GEMV
         return;
     }
-    const int all = (K + 31) / 32;
-    const int64_t groups = ((GLU ? 2 * N : N) + 15) / 16;
-    const int waves = groups >= 1024 ? 4 : 8, most = 2048 / waves;
-    const int grid = (int)(groups < most ? groups : most), steps = (all + waves - 1) / waves;
-#define GEMV(NW) gemv_kernel<NW, PRO, F32, GLU><<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, ldy, res, ldr)
-    if (waves == 4) GEMV(4); else GEMV(8);
+    if constexpr (PRO != 3) {
+        const int all = (K + 31) / 32;
+        const int64_t groups = ((GLU ? 2 * N : N) + 15) / 16;
+        const int waves = groups >= 1024 ? 4 : all > 8 * GEMV_STEPS && all <= 12 * GEMV_STEPS ? 12 : 8, most = waves == 4 ? 512 : 256;
+        const bool half = !GLU && groups <= 128;
+        const int64_t work = half ? (N + 7) / 8 : groups;
+        const int grid = (int)(work < most ? work : most), steps = (all + waves - 1) / waves;
+#define GEMV(NW, R) gemv_kernel<NW, PRO, F32, GLU, R><<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, (void*)y, ldy, res, ldr)
+        if (waves == 4) GEMV(4, 16);
+        else if (half && !GLU) {
+            if (waves == 12) GEMV(12, GLU ? 16 : 8); else GEMV(8, GLU ? 16 : 8);
+        } else if (waves == 12) GEMV(12, 16);
+        else GEMV(8, 16);
 #undef GEMV
+    }
 }
 
 extern "C" int mi355_gemv_bf16(int M, int64_t N, int K, const void* x, int64_t ldx, const void* W, int64_t ldw, void* y, int64_t ldy,
@@ -737,7 +801,7 @@ extern "C" int mi355_kv_append_rows(int B, int S, int64_t width_bytes, const voi
 
 static int attn_decode_launch(const char* who, int B, int Hq, int Hkv, int D, const void* q, const void* k_cache, const void* v_cache, int64_t batch_stride, int64_t ld, int len,
                               const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, void* o, float scale, const QkvPost* post, int splits, float* workspace,
-                              void* stream) {
+                              void* stream, bool combine = true) {
     MI355_REQUIRE(B > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 && len > 0, "%s: bad sizes", who);
     MI355_REQUIRE(k_cache && v_cache && o && ld >= (int64_t)Hkv * D && ld % 8 == 0 && batch_stride >= (int64_t)len * ld, "%s: cache pitch / stride too small", who);
     MI355_REQUIRE(!key_mask || ldm >= len, "%s: key mask pitch smaller than the cache length", who);
@@ -752,7 +816,7 @@ static int attn_decode_launch(const char* who, int B, int Hq, int Hkv, int D, co
         if (D == 32) LAUNCH(32, 8, false); else if (D == 64) LAUNCH(64, 8, false); else if (D == 128) LAUNCH(128, 8, false); else LAUNCH(256, 8, false);
     }
 #undef LAUNCH
-    if (splits > 1) attn_decode_combine_kernel<<<dim3(Hq, B), D, 0, ST(stream)>>>(Hq, D, splits, workspace, (bf16_t*)o);
+    if (splits > 1 && combine) attn_decode_combine_kernel<<<dim3(Hq, B), D, 0, ST(stream)>>>(Hq, D, splits, workspace, (bf16_t*)o);
     return 0;
 }
 
@@ -766,17 +830,25 @@ extern "C" int mi355_attn_decode(int B, int Hq, int Hkv, int D, const void* q, c
     return 0;
 }
 
-extern "C" int mi355_attn_decode_qkv(int B, int Hq, int Hkv, int D, const void* qkv, int64_t ldqkv, const void* q_norm_w, const void* k_norm_w, const float* cos,
+static int attn_decode_qkv(int B, int Hq, int Hkv, int D, const void* qkv, int64_t ldqkv, const void* q_norm_w, const void* k_norm_w, const float* cos,
                                      const float* sin, const int32_t* pos, void* k_cache, void* v_cache, int64_t batch_stride, int64_t ld, int capacity,
                                      const int32_t* write_pos, const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, void* o, float scale, float eps, int splits,
-                                     float* workspace, void* stream) {
+                           float* workspace, void* stream, bool combine) {
     MI355_REQUIRE(D == 128 || D == 64, "attn_decode_qkv: head_dim must be 64 or 128 (got %d)", D);
     MI355_REQUIRE(Hq > 0 && Hkv > 0 && ldqkv >= (int64_t)(Hq + 2 * Hkv) * D && ldqkv % 8 == 0, "attn_decode_qkv: the qkv row holds (Hq + 2 Hkv) * D elements, pitch a multiple of 8");
     MI355_REQUIRE(qkv && q_norm_w && k_norm_w && cos && sin && pos && write_pos && len_dev, "attn_decode_qkv: null pointer (the write position and the length live on the device)");
     const QkvPost post = {(const bf16_t*)qkv, ldqkv, (const bf16_t*)q_norm_w, (const bf16_t*)k_norm_w, cos, sin, pos, write_pos, capacity, eps};
-    if (int rc = attn_decode_launch("attn_decode_qkv", B, Hq, Hkv, D, nullptr, k_cache, v_cache, batch_stride, ld, capacity, len_dev, key_mask, ldm, o, scale, &post, splits, workspace, stream)) return rc;
+    if (int rc = attn_decode_launch("attn_decode_qkv", B, Hq, Hkv, D, nullptr, k_cache, v_cache, batch_stride, ld, capacity, len_dev, key_mask, ldm, o, scale, &post, splits, workspace, stream, combine)) return rc;
     MI355_LAUNCH_CHECK("attn_decode_qkv");
     return 0;
+}
+
+extern "C" int mi355_attn_decode_qkv(int B, int Hq, int Hkv, int D, const void* qkv, int64_t ldqkv, const void* q_norm_w, const void* k_norm_w, const float* cos,
+                                     const float* sin, const int32_t* pos, void* k_cache, void* v_cache, int64_t batch_stride, int64_t ld, int capacity,
+                                     const int32_t* write_pos, const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, void* o, float scale, float eps, int splits,
+                                     float* workspace, void* stream) {
+    return attn_decode_qkv(B, Hq, Hkv, D, qkv, ldqkv, q_norm_w, k_norm_w, cos, sin, pos, k_cache, v_cache, batch_stride, ld, capacity, write_pos, len_dev, key_mask, ldm, o, scale, eps,
+                           splits, workspace, stream, true);
 }
 
 // One layer of a one-token step (M = B <= 8 rows): the step's launches behind one call.  A launch costs the host 3.5 us and its Python around it as much again and more (checks,
@@ -802,9 +874,15 @@ extern "C" int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, c
     bf16_t *qkv = (bf16_t*)scratch, *ctx = qkv + B * lq, *h1 = ctx + B * lc, *act = h1 + B * l1;
     MI355_REQUIRE(lc == nc && norm2_w && w_gate_up && w_down, "decode_block: Hq * D must be a multiple of 8; null pointer");
     if (int rc = mi355_gemv_bf16_pro(B, nq, d, h, d, 1, norm1_w, eps, w_qkv, d, qkv, lq, nullptr, 0, stream)) return rc;
-    if (int rc = mi355_attn_decode_qkv(B, Hq, Hkv, D, qkv, lq, q_norm_w, k_norm_w, cos, sin, pos, k_cache, v_cache, batch_stride, ld, capacity, write_pos, len_dev, key_mask, ldm, ctx,
-                                       scale, eps, splits, (float*)(act + B * la), stream)) return rc;
-    if (int rc = mi355_gemv_bf16(B, d, (int)nc, ctx, nc, w_out, nc, h1, l1, h, d, stream)) return rc;
+    float* parts = (float*)(act + B * la);
+    const bool fold = B == 1 && splits > 1 && nc <= 32768;  // (two rows and more go through the matrix pipe, whose operands have no image to fold into; 64 KiB of LDS)
+    if (int rc = attn_decode_qkv(B, Hq, Hkv, D, qkv, lq, q_norm_w, k_norm_w, cos, sin, pos, k_cache, v_cache, batch_stride, ld, capacity, write_pos, len_dev, key_mask, ldm, ctx,
+                                 scale, eps, splits, parts, stream, !fold)) return rc;
+    if (fold) {
+        MI355_REQUIRE(w_out, "decode_block: null pointer");
+        gemv_launch<3, false>(1, d, (int)nc, ctx, nc, nullptr, 0.f, w_out, nc, h1, l1, h, d, stream, SplitRow{parts, D, splits});
+        MI355_LAUNCH_CHECK("decode_block(out)");
+    } else if (int rc = mi355_gemv_bf16(B, d, (int)nc, ctx, nc, w_out, nc, h1, l1, h, d, stream)) return rc;
     gemv_launch<1, false, true>(B, F, d, h1, l1, norm2_w, eps, w_gate_up, d, act, la, nullptr, 0, stream);
     MI355_LAUNCH_CHECK("decode_block(gate, up)");
     return mi355_gemv_bf16(B, d, F, act, la, w_down, F, out, d, h1, l1, stream);
