@@ -740,7 +740,10 @@ __global__ __launch_bounds__(256) void bgemm_f32_tile_kernel(BgemmArgs p) {
 
 // ---- MFMA path for few rows per group (one-token steps through a mixture's experts): bound by the stream of the weights.  A workgroup is eight waves on 32 rows x 32
 // columns (GLU: the 32 gate and the 32 up columns of one block); the waves deal the k range among themselves, read both operands straight from memory in
-// fragment form -- 16 bytes per lane, SU steps of 16 in flight while the previous SU multiply -- and their partial sums meet in LDS.
+// fragment form -- 16 bytes per lane, two stages of SU steps of 16 in flight -- and their partial sums meet in LDS.  A workgroup lives for a few memory round trips, so what
+// depends on nothing goes first: the weights in front of the row list that says which operand rows meet them, and where the results go is looked up under the stream.
+// (One stage held the other up: its registers were copied, and so waited for, before the next was requested: six rows of 16 experts, 1024 x 1792 gated 13.3 -> 11.0 us,
+// 896 x 1024 9.0 -> 8.4; 24 rows 26.7 -> 21.2, 18.1 -> 16.3.  Eight steps a stage: 8.9 and 17.8.)
 #define SU 4
 #define F32_STREAM_ROWS 128  // fp32 A: beyond this many rows the tile kernel's one split per 128 columns beats the stream's one per 32 (450 rows: a third of the time)
 #define STREAM_ROWS 256  // up to this many sorted rows in all groups together
@@ -754,67 +757,93 @@ __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
     const int b = blockIdx.z, row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? p.grp_offs[b + 1] - row0 : p.M;
     const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32 * NB;
     if (m0 >= rows) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5;
+    const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    struct Stage {
+        frag_t a[SU];
+        u32x4 b[SU][NB];
+    };
+    Stage x, y;
+    const bf16_t* b_row[NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) b_row[j] = (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)min(n0 + 32 * j + ln, p.N - 1) * p.sbn + 8 * hf;  // (columns past N are not stored)
+    auto request_b = [&](Stage& t, int st) {
+        if (st + SU <= s1 && (st + SU) * 16 <= p.K) {
+#pragma unroll
+            for (int u = 0; u < SU; ++u)
+#pragma unroll
+                for (int j = 0; j < NB; ++j) t.b[u][j] = *(const u32x4*)(b_row[j] + (st + u) * 16);
+        } else {
+#pragma unroll
+            for (int u = 0; u < SU; ++u) {
+                const bool in = st + u < s1 && (st + u) * 16 + 8 * hf < p.K;  // K is a multiple of 8
+#pragma unroll
+                for (int j = 0; j < NB; ++j) t.b[u][j] = in ? *(const u32x4*)(b_row[j] + (st + u) * 16) : zero;
+            }
+        }
+    };
+    request_b(x, s0);
     const elem_t* a_row = nullptr;
     if (m0 + ln < rows) {
         const int r = row0 + m0 + ln;
         a_row = (const elem_t*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
     }
-    const bf16_t* b_row[NB];
-#pragma unroll
-    for (int j = 0; j < NB; ++j) b_row[j] = n0 + 32 * j + ln < p.N ? (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)(n0 + 32 * j + ln) * p.sbn : nullptr;
-    const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
-    const u32x4 zero = {0u, 0u, 0u, 0u};
-    frag_t fa[SU];
-    u32x4 fb[SU][NB];
-    auto fetch = [&](int st) {
+    auto request_a = [&](Stage& t, int st) {
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
-            const int k = (st + u) * 16 + 8 * hf;  // K is a multiple of 8
-            const bool in = st + u < s1 && k < p.K;
+            const int k = (st + u) * 16 + 8 * hf;
+            const bool in = a_row && st + u < s1 && k < p.K;
             if constexpr (F32) {
-                fa[u].a = in && a_row ? *(const f32x4*)(a_row + k) : (f32x4){0.f, 0.f, 0.f, 0.f};
-                fa[u].b = in && a_row ? *(const f32x4*)(a_row + k + 4) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                t.a[u].a = in ? *(const f32x4*)(a_row + k) : (f32x4){0.f, 0.f, 0.f, 0.f};
+                t.a[u].b = in ? *(const f32x4*)(a_row + k + 4) : (f32x4){0.f, 0.f, 0.f, 0.f};
             } else {
-                fa[u] = in && a_row ? *(const u32x4*)(a_row + k) : zero;
+                t.a[u] = in ? *(const u32x4*)(a_row + k) : zero;
             }
-#pragma unroll
-            for (int j = 0; j < NB; ++j) fb[u][j] = in && b_row[j] ? *(const u32x4*)(b_row[j] + k) : zero;
         }
     };
+    request_a(x, s0);
+    // this thread's results: rows m0 + 8 (e >> 2) + 4 hf + (e & 3), e = wave * 16 / SW + q
+    int64_t crow[16 / SW];
+    float scale[16 / SW];
+#pragma unroll
+    for (int q = 0; q < 16 / SW; ++q) {
+        const int e = wave * (16 / SW) + q, r = row0 + min(m0 + 8 * (e >> 2) + 4 * hf + (e & 3), rows - 1);
+        crow[q] = p.c_rows ? p.c_rows[r] : r;
+    }
     f32x16 acc[NB];
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
         for (int e = 0; e < 16; ++e) acc[j][e] = 0.f;
-    fetch(s0);
-    for (int st = s0; st < s1; st += SU) {
-        frag_t ca[SU];
-        u32x4 cb[SU][NB];
-#pragma unroll
-        for (int u = 0; u < SU; ++u) {
-            ca[u] = fa[u];
-#pragma unroll
-            for (int j = 0; j < NB; ++j) cb[u][j] = fb[u][j];
+    auto work = [&](Stage& now, Stage& next, int st) {
+        if (st + SU < s1) {
+            request_b(next, st + SU);
+            request_a(next, st + SU);
         }
-        if (st + SU < s1) fetch(st + SU);
 #pragma unroll
         for (int u = 0; u < SU; ++u) {
             if constexpr (F32) {
-                const Split8 t = split8(ca[u].a, ca[u].b);
+                const Split8 t = split8(now.a[u].a, now.a[u].b);
 #pragma unroll
                 for (int j = 0; j < NB; ++j) {
-                    const bf16x8 w = __builtin_bit_cast(bf16x8, cb[u][j]);
+                    const bf16x8 w = __builtin_bit_cast(bf16x8, now.b[u][j]);
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.lo), w, acc[j], 0, 0, 0);
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.mid), w, acc[j], 0, 0, 0);
                     acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.hi), w, acc[j], 0, 0, 0);
                 }
             } else {
 #pragma unroll
-                for (int j = 0; j < NB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ca[u]), __builtin_bit_cast(bf16x8, cb[u][j]), acc[j], 0, 0, 0);
+                for (int j = 0; j < NB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, now.a[u]), __builtin_bit_cast(bf16x8, now.b[u][j]), acc[j], 0, 0, 0);
             }
         }
+    };
+    for (int st = s0; st < s1; st += 2 * SU) {
+        work(x, y, st);
+        if (st + SU < s1) work(y, x, st + SU);
     }
+#pragma unroll
+    for (int q = 0; q < 16 / SW; ++q) scale[q] = p.row_scale ? p.row_scale[crow[q]] : 1.0f;
 #pragma unroll
     for (int j = 0; j < NB; ++j)
 #pragma unroll
@@ -832,23 +861,130 @@ __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
             for (int w = 0; w < SW; ++w) v[j] += red[w][j][e][lane];
         }
         if (m >= rows || n >= (GLU ? p.n_out : p.N)) continue;
-        const int r = row0 + m;
-        const int64_t crow = p.c_rows ? p.c_rows[r] : r;
         if constexpr (F32) {
 #pragma unroll
-            for (int j = 0; j < NB; ++j) v[j] = settled(p, v[j], b, r, n0 + 32 * j + ln);
+            for (int j = 0; j < NB; ++j) v[j] = settled(p, v[j], b, row0 + m, n0 + 32 * j + ln);
         }
-        float x;
+        float o;
         if constexpr (GLU) {
-            x = gated_act(p.epi, v[0], v[NB - 1], p.limit);
+            o = gated_act(p.epi, v[0], v[NB - 1], p.limit);
         } else {
-            x = v[0] + (p.bias ? p.bias[n] : 0.f);
-            if (p.epi == 1) x = x > 0.f ? x * x : 0.f;
+            o = v[0] + (p.bias ? p.bias[n] : 0.f);
+            if (p.epi == 1) o = o > 0.f ? o * o : 0.f;
         }
-        x *= p.row_scale ? p.row_scale[crow] : 1.0f;
-        const int64_t ci = (int64_t)b * p.c_bs + crow * p.ldc + n;
-        if (p.c_dt == MI355_DT_F32) ((float*)p.C)[ci] = x;
-        else ((bf16_t*)p.C)[ci] = f2bf(x);
+        o *= scale[q];
+        const int64_t ci = (int64_t)b * p.c_bs + crow[q] * p.ldc + n;
+        if (p.c_dt == MI355_DT_F32) ((float*)p.C)[ci] = o;
+        else ((bf16_t*)p.C)[ci] = f2bf(o);
+    }
+}
+
+// The same product of fp32 rows where few rows meet the weights: in the kernel above every wave splits its operand fragments in registers, for 32 rows whether they exist or not
+// (90 vector instructions a step of 16: 12 us of a 2048 x 1024 product of three rows).  Here the workgroup splits the rows that exist once, into three bf16 planes in LDS, under the
+// weights' flight; a lane without a row reads a row of zeros.  The same parts meet the same weights in the same order: the bits are those of the other kernels of this path.
+// Three rows, K x N: 2048 x 1024 12.4 -> 6.7 us, 1024 x 4096 9.2 -> 6.1, 1024 x 8256 16.5 -> 8.7, 1024 x 32000 32.9 -> 17.1 (the kernel above as it is now: 11.8, 8.4, 14.4, 28.5); one row
+// 1024 x 512 7.7 -> 4.6; 32 rows 1024 x 1024 10.1 -> 9.4 (the kernel above: 9.4); six rows of 16 experts 1792 x 1024 13.1 -> 10.5 (above: 11.9).  Gated epilogues stay above: two
+// accumulators want the registers of the second stage (six rows of 16 experts, 1024 x 1792: 12.7 here, 11.0 there).
+// Columns a workgroup: 32 is what a product of the matrix pipe holds; fewer idle its lanes, and pay while the workgroups with work leave CUs without any.  8 / 16 / 32 columns, by tiles
+// of 32: 16 tiles 4.6 / 4.9 / 5.2 us, 32 tiles 6.7 / 7.3 / 8.3; 128 tiles 7.1 / 6.0 / 6.3; 192 tiles with 1792 deep 12.3 / 10.5 / 12.0, 896 deep 9.4 / 7.3 / 6.4; 258 tiles 13.2 / 10.1 / 8.8.
+#define F32_ROWS_LDS (144 * 1024)
+#define F32_ROWS_HALF 192
+static inline int64_t f32_rows_pitch(int64_t K) { return (K + 15) / 16 * 16 + 8; }  // (8: rows start in different banks)
+template <int COLS>
+__global__ __launch_bounds__(64 * SW) void bgemm_f32_rows_kernel(BgemmArgs p, int cap, int pitch) {
+    constexpr int RU = 8;  // steps of a stage: two stages hold a wave's run up to K = 2048
+    extern __shared__ __attribute__((aligned(16))) char smem[];  // planes [3][cap + 1][pitch]; then the waves' sums [SW][16][64]
+    bf16_t* planes = (bf16_t*)smem;
+    float* red = (float*)smem;
+    const int b = blockIdx.z, row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? min(p.grp_offs[b + 1] - row0, cap) : p.M;
+    const int n0 = blockIdx.x * COLS;
+    if (rows <= 0) return;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5;
+    const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
+    const u32x4 zero = {0u, 0u, 0u, 0u};
+    u32x4 x[RU], y[RU];
+    const bf16_t* b_row = (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)min(n0 + ln, p.N - 1) * p.sbn + 8 * hf;  // (columns past N are not stored)
+    auto request = [&](u32x4 (&t)[RU], int st) {
+        if (COLS < 32 && ln >= COLS) return;
+        if (st + RU <= s1 && (st + RU) * 16 <= p.K) {
+#pragma unroll
+            for (int u = 0; u < RU; ++u) t[u] = *(const u32x4*)(b_row + (st + u) * 16);
+        } else {
+#pragma unroll
+            for (int u = 0; u < RU; ++u) {
+                const bool in = st + u < s1 && (st + u) * 16 + 8 * hf < p.K;  // K is a multiple of 8
+                t[u] = in ? *(const u32x4*)(b_row + (st + u) * 16) : zero;
+            }
+        }
+    };
+    if constexpr (COLS < 32) {
+#pragma unroll
+        for (int u = 0; u < RU; ++u) x[u] = y[u] = zero;
+    }
+    request(x, s0);
+    if (s0 + RU < s1) request(y, s0 + RU);
+    const int words = (pitch - 8) / 8, plane = (cap + 1) * pitch;  // 8 k at a time
+    for (int c = tid; c < (rows + 1) * words; c += 64 * SW) {
+        const int i = c / words, k = (c - i * words) * 8;
+        Split8 t = {zero, zero, zero};
+        if (i < rows && k < p.K) {
+            const int r = row0 + i;
+            const float* a = (const float*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda + k;
+            t = split8(*(const f32x4*)a, *(const f32x4*)(a + 4));
+        }
+        bf16_t* to = planes + i * pitch + k;  // (row `rows` is the row of zeros)
+        *(u32x4*)to = t.hi;
+        *(u32x4*)(to + plane) = t.mid;
+        *(u32x4*)(to + 2 * plane) = t.lo;
+    }
+    int64_t crow[16 / SW];
+#pragma unroll
+    for (int q = 0; q < 16 / SW; ++q) {
+        const int e = wave * (16 / SW) + q, r = row0 + min(8 * (e >> 2) + 4 * hf + (e & 3), rows - 1);
+        crow[q] = p.c_rows ? p.c_rows[r] : r;
+    }
+    __syncthreads();
+    const bf16_t* a_row = planes + min(ln, rows) * pitch + 8 * hf;
+    f32x16 acc;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) acc[e] = 0.f;
+    auto work = [&](u32x4 (&t)[RU], int st) {
+#pragma unroll
+        for (int u = 0; u < RU; ++u) {
+            if (st + u >= s1) break;
+            const bf16x8 hi = *(const bf16x8*)(a_row + (st + u) * 16), mid = *(const bf16x8*)(a_row + plane + (st + u) * 16), lo = *(const bf16x8*)(a_row + 2 * plane + (st + u) * 16);
+            const bf16x8 w = __builtin_bit_cast(bf16x8, t[u]);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(lo, w, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(mid, w, acc, 0, 0, 0);
+            acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(hi, w, acc, 0, 0, 0);
+        }
+        if (st + 2 * RU < s1) request(t, st + 2 * RU);
+    };
+    for (int st = s0; st < s1; st += 2 * RU) {
+        work(x, st);
+        if (st + RU < s1) work(y, st + RU);
+    }
+    float scale[16 / SW];
+#pragma unroll
+    for (int q = 0; q < 16 / SW; ++q) scale[q] = p.row_scale ? p.row_scale[crow[q]] : 1.0f;
+    __syncthreads();
+#pragma unroll
+    for (int e = 0; e < 16; ++e) red[(wave * 16 + e) * 64 + lane] = acc[e];
+    __syncthreads();
+    const int n = n0 + ln;
+#pragma unroll
+    for (int q = 0; q < 16 / SW; ++q) {
+        const int e = wave * (16 / SW) + q, m = 8 * (e >> 2) + 4 * hf + (e & 3);
+        float v = 0.f;
+#pragma unroll
+        for (int w = 0; w < SW; ++w) v += red[(w * 16 + e) * 64 + lane];
+        if (m >= rows || ln >= COLS || n >= p.N) continue;
+        float o = settled(p, v, b, row0 + m, n) + (p.bias ? p.bias[n] : 0.f);
+        if (p.epi == 1) o = o > 0.f ? o * o : 0.f;
+        o *= scale[q];
+        const int64_t ci = (int64_t)b * p.c_bs + crow[q] * p.ldc + n;
+        if (p.c_dt == MI355_DT_F32) ((float*)p.C)[ci] = o;
+        else ((bf16_t*)p.C)[ci] = f2bf(o);
     }
 }
 
@@ -905,7 +1041,15 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
         MI355_REQUIRE(ty <= 65535, "bgemm: too many row tiles");
         if (M <= F32_STREAM_ROWS) {
             const dim3 grid((N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
-            if (epi >= 2) bgemm_stream_kernel<true, true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
+            const int64_t pitch = f32_rows_pitch(K), planes = 6 * (M + 1) * pitch, sums = SW * 16 * 64 * 4;
+            if (epi < 2 && M <= 32 && planes <= F32_ROWS_LDS) {  // (M bounds the rows of every group)
+                const unsigned lds = (unsigned)(planes > sums ? planes : sums);
+                // (a group without rows is no work)
+                const int64_t tiles = (int64_t)grid.x * (grp_offs && M < batch ? M : batch);
+#define ROWS(C) bgemm_f32_rows_kernel<C><<<dim3((N + C - 1) / C, 1, batch), 64 * SW, lds, ST(stream)>>>(p, M, (int)pitch)
+                if (tiles <= 32) ROWS(8); else if (tiles <= F32_ROWS_HALF) ROWS(16); else ROWS(32);
+#undef ROWS
+            } else if (epi >= 2) bgemm_stream_kernel<true, true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
             else bgemm_stream_kernel<false, true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
         } else {
             const int64_t tn = (N + 127) / 128, tiles = (grp_offs ? 1 : batch) * tn * ((M + 127) / 128);
