@@ -17,6 +17,7 @@
 //
 // Three compute paths: fp32 FMA through LDS (any operand type: the true-fp32 mode), bf16 MFMA (v_mfma_f32_32x32x8_bf16_1k) for bf16 keys / values with every
 // option, and -- latent_attn_full.h -- a leaner bf16 MFMA kernel for aligned rows without pooled blocks (sigmoid weights: only where every key j <= i is seen).
+#include "lane_sums.h"
 #include "latent_attn.h"
 
 #define ST(s) ((hipStream_t)(s))
@@ -44,7 +45,7 @@ __device__ __forceinline__ float as_f32(bf16_t x) { return bf2f(x); }
 // Bound: a served step has few workgroups (one a sequence, folded form), each a chain of memory round trips; so the next feature chunk of keys and queries is requested while this one
 // is multiplied, and values eight keys at a time (one by one they were 64 round trips a key step): three sequences of 150 keys, 8 heads, 256 + 64 | 256 wide, 248 -> 118 us; a prompt of 150 tokens (128 + 64 | 128) 159 -> 80. The order of every sum is as before.
 template <int NC, typename KV>
-__global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p) {
+__global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p, int from) {  // sequences with fewer new tokens than `from` are not its own
     __shared__ float Qs[AM][AC + 1];
     __shared__ float Ks[AN][AC + 1];
     __shared__ float Ps[AM][AN + 4];
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p) {
     const int s = blockIdx.z, tm = AM / p.hm;
     const int tok0 = blockIdx.x * tm, head0 = blockIdx.y * p.hm;
     const int n_new = p.n_new[s], past = p.past[s];
-    if (tok0 >= n_new) return;
+    if (tok0 >= n_new || n_new < from) return;
     const int64_t qr0 = p.q_row0[s], k1r0 = p.k1_row0[s], k2r0 = p.k2_row0[s], vr0 = p.v_row0[s];
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     const int DK = p.D1 + p.D2;
@@ -234,6 +235,181 @@ __global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p) {
     }
 }
 
+
+// ---- The same FMA product for sequences with one or two new tokens.  The tile above has 32 query rows and walks 64 keys at a time through LDS, two barriers for every 32 features:
+// one token of eight heads fills eight of the rows, and three sequences were three workgroups, each a chain of barriers (150 keys, 8 heads, 256 + 64 | 256 wide: 118 us).  Here a
+// workgroup is one token and `hg` <= 4 heads of one key / value head; its eight waves take four keys at a time in turn, a lane 1 / 64 of every row (coalesced, no LDS, no
+// barrier in the loop): the four heads' partial scores of a key fold into one register -- heads by rows of 16 lanes -- in six swaps and adds, and the weights come back to all lanes
+// as scalars.  Which of the two a sequence takes depends on its own new tokens alone, so a row's bits do not depend on the rest of the step.  118 -> 20.7 us
+// (keys dealt to 8 waves; what is left is two rounds of a wave's keys from memory, the exchange and the launch).
+constexpr int STEP_NEW = 2, STEP_WAVES = 8, STEP_KB = 4;
+__device__ __forceinline__ float fold32(float a, float b) {  // lanes 0 .. 31: a folded over the halves, 32 .. 63: b
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float fold16(float a, float b) {  // even rows of 16 lanes: a folded over the row pairs, odd ones: b
+    const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(a), __float_as_uint(b), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+__device__ __forceinline__ float from_row(float v, int row) { return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), row * 16)); }
+
+template <int NQ, int NV, bool SAME, typename KV>  // SAME: the values are the first features of the keys' main part
+__global__ __launch_bounds__(64 * STEP_WAVES) void latent_attn_step_kernel(LatAttnArgs p, int hg) {
+    __shared__ float part[STEP_WAVES][4][64 * NV];
+    __shared__ float ms[STEP_WAVES][4], lsum[STEP_WAVES][4];
+    const int head0 = blockIdx.x * hg, tok = blockIdx.y, s = blockIdx.z, n_new = p.n_new[s];
+    if (n_new > STEP_NEW || tok >= n_new) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), row = lane >> 4;
+    const int hr = (row & 1) * 2 + (row >> 1);  // the head of a row of lanes: 0, 2, 1, 3
+    const int DK = p.D1 + p.D2, lim = p.past[s] + tok, kvh = head0 / p.kv_rep;
+    const int64_t qrow = p.q_row0[s] + tok;
+    const int c0 = p.chunk > 0 ? lim / p.chunk * p.chunk : 0, lo = max(tile_key_floor(lim, p.window, p.chunk), 0);
+    const int n_keep = p.window > 0 ? max(min(p.keep_first, lo) - c0, 0) : 0, total = n_keep + lim + 1 - lo;  // keys the token sees: kept ones, then its window
+    auto key = [&](int u) { return u < n_keep ? c0 + u : lo + u - n_keep; };
+    float q[4][NQ];
+    const KV* at[NQ];
+    bool main_part[NQ];
+#pragma unroll
+    for (int i = 0; i < NQ; ++i) {
+        const int d = lane + 64 * i, e = min(d, DK - 1);
+        main_part[i] = e < p.D1;
+        at[i] = main_part[i] ? (const KV*)p.K1 + p.k1_row0[s] * p.ldk1 + (int64_t)kvh * p.k1_hs + e : (const KV*)p.K2 + p.k2_row0[s] * p.ldk2 + (e - p.D1);
+#pragma unroll
+        for (int h = 0; h < 4; ++h) q[h][i] = h < hg && head0 + h < p.H && d < DK ? p.Q[qrow * p.ldq + (int64_t)(head0 + h) * p.q_hs + d] : 0.f;
+    }
+    const KV* vat = (const KV*)p.V + p.v_row0[s] * p.ldv + (int64_t)kvh * p.v_hs;
+    struct Keys {
+        KV k[STEP_KB][NQ], v[SAME ? 1 : STEP_KB][SAME ? 1 : NV];
+    };
+    auto request = [&](Keys& t, int u0) {
+#pragma unroll
+        for (int u = 0; u < STEP_KB; ++u) {
+            const int64_t j = key(min(u0 + u, total - 1));
+            const int64_t o1 = j * p.ldk1, o2 = j * p.ldk2;
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                if (64 * i >= DK) break;
+                t.k[u][i] = at[i][main_part[i] ? o1 : o2];
+            }
+            if constexpr (!SAME) {
+#pragma unroll
+                for (int i = 0; i < NV; ++i) t.v[u][i] = vat[j * p.ldv + min(lane + 64 * i, p.DV - 1)];
+            }
+        }
+    };
+    const int head = min(head0 + min(hr, hg - 1), p.H - 1);
+    const float sl = p.slope ? p.slope[head] : 0.f, sb = p.sig_bias ? p.sig_bias[head] : 0.f;
+    float m = -__builtin_huge_valf(), l = 0.f, o[4][NV];
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) o[h][i] = 0.f;
+    auto work = [&](const Keys& t, int u0) {
+        float e[STEP_KB], mx = -__builtin_huge_valf();
+#pragma unroll
+        for (int u = 0; u < STEP_KB; ++u) {
+            float d[4] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int i = 0; i < NQ; ++i) {
+                if (64 * i >= DK) break;
+                const float kf = lane + 64 * i < DK ? as_f32(t.k[u][i]) : 0.f;  // (an infinity there must not meet the zero of q)
+#pragma unroll
+                for (int h = 0; h < 4; ++h) d[h] = fmaf(q[h][i], kf, d[h]);
+            }
+            const float sc = lanes_sum<16>(fold16(fold32(d[0], d[1]), fold32(d[2], d[3])));
+            e[u] = cap_score(sc * p.scale, p.softcap) - sl * (float)(lim - key(min(u0 + u, total - 1)));
+            if (u0 + u >= total) e[u] = -__builtin_huge_valf();
+            mx = fmaxf(mx, e[u]);
+        }
+        if (p.sig_bias) {
+#pragma unroll
+            for (int u = 0; u < STEP_KB; ++u) e[u] = 1.0f / (1.0f + expf(-(e[u] + sb)));
+        } else {
+            const float m_new = fmaxf(m, mx), base = m_new == -__builtin_huge_valf() ? 0.f : m_new;
+            if (__any(m_new > m)) {
+                const float f = expf(m - base);
+                l *= f;
+#pragma unroll
+                for (int h = 0; h < 4; ++h) {
+                    const float fh = from_row(f, (h & 1) * 2 + (h >> 1));
+#pragma unroll
+                    for (int i = 0; i < NV; ++i) o[h][i] *= fh;
+                }
+            }
+            m = m_new;
+#pragma unroll
+            for (int u = 0; u < STEP_KB; ++u) {
+                e[u] = expf(e[u] - base);
+                l += e[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < STEP_KB; ++u) {
+            if (u0 + u >= total) break;
+#pragma unroll
+            for (int h = 0; h < 4; ++h) {
+                const float w = from_row(e[u], (h & 1) * 2 + (h >> 1));
+#pragma unroll
+                for (int i = 0; i < NV; ++i) o[h][i] = fmaf(w, as_f32(SAME ? t.k[u][i] : t.v[SAME ? 0 : u][SAME ? 0 : i]), o[h][i]);
+            }
+        }
+    };
+    constexpr int STRIDE = STEP_WAVES * STEP_KB;
+    Keys x, y;
+    int u0 = wave * STEP_KB;
+    if (u0 < total) request(x, u0);
+    for (; u0 < total; u0 += 2 * STRIDE) {
+        if (u0 + STRIDE < total) request(y, u0 + STRIDE);
+        work(x, u0);
+        if (u0 + STRIDE >= total) break;
+        if (u0 + 2 * STRIDE < total) request(x, u0 + 2 * STRIDE);
+        work(y, u0 + STRIDE);
+    }
+#pragma unroll
+    for (int h = 0; h < 4; ++h)
+#pragma unroll
+        for (int i = 0; i < NV; ++i) part[wave][h][lane + 64 * i] = o[h][i];
+    if ((lane & 15) == 0) ms[wave][hr] = m, lsum[wave][hr] = l;
+    __syncthreads();
+    for (int x0 = threadIdx.x; x0 < hg * p.DV; x0 += 64 * STEP_WAVES) {
+        const int h = x0 / p.DV, col = x0 - h * p.DV, hd = head0 + h;
+        if (hd >= p.H) break;
+        float mm = -__builtin_huge_valf(), ll = 0.f, v = 0.f;
+        if (!p.sig_bias) {
+#pragma unroll
+            for (int w = 0; w < STEP_WAVES; ++w) mm = fmaxf(mm, ms[w][h]);
+            if (p.sink) mm = fmaxf(mm, p.sink[hd]);
+        }
+#pragma unroll
+        for (int w = 0; w < STEP_WAVES; ++w) {
+            const float f = p.sig_bias ? 1.f : ms[w][h] == -__builtin_huge_valf() ? 0.f : expf(ms[w][h] - mm);  // (a wave without keys)
+            ll += lsum[w][h] * f;
+            v += part[w][h][col] * f;
+        }
+        if (p.sink) ll += expf(p.sink[hd] - mm);  // the sink joins the denominator
+        if (!p.sig_bias) v /= ll;
+        if (p.gate) v *= gate_of(p.gate[qrow * p.ldg + (int64_t)hd * p.DV + col]);
+        const int64_t ob = qrow * p.ldo + (int64_t)hd * p.o_hs + col;
+        if (p.o_dt == MI355_DT_F32) ((float*)p.O)[ob] = v;
+        else ((bf16_t*)p.O)[ob] = f2bf(v);
+    }
+}
+
+// Launches it if it holds these sizes (no pooled rows; a whole wave's keys must share their row).
+static bool latent_attn_step_launch(const LatAttnArgs& p, int max_new, int n_seq, hipStream_t st) {
+    const int DK = p.D1 + p.D2;
+    if (p.pool > 0 || DK > 640 || p.DV > 512) return false;
+    const bool shared = p.k1_hs == 0 && p.v_hs == 0;
+    const int hg = shared || p.kv_rep % 4 == 0 ? 4 : p.kv_rep % 2 == 0 ? 2 : 1;
+    const bool same = p.V == p.K1 && p.ldv == p.ldk1 && p.v_hs == p.k1_hs && p.v_row0 == p.k1_row0 && p.DV <= p.D1;
+    const dim3 grid((p.H + hg - 1) / hg, max_new < STEP_NEW ? max_new : STEP_NEW, n_seq);
+#define STEP2(NQ, NV, KV) do { if (same) latent_attn_step_kernel<NQ, NV, true, KV><<<grid, 64 * STEP_WAVES, 0, st>>>(p, hg); else latent_attn_step_kernel<NQ, NV, false, KV><<<grid, 64 * STEP_WAVES, 0, st>>>(p, hg); } while (0)
+#define STEP(NQ, NV) do { if (p.dt == MI355_DT_F32) STEP2(NQ, NV, float); else STEP2(NQ, NV, bf16_t); } while (0)
+    if (DK <= 128 && p.DV <= 128) STEP(2, 2); else if (DK <= 256 && p.DV <= 256) STEP(4, 4); else if (DK <= 384 && p.DV <= 256) STEP(6, 4); else STEP(10, 8);
+#undef STEP
+#undef STEP2
+    return true;
+}
 
 // ---- MFMA path (bf16 keys / values).  A workgroup is four waves; wave w owns query rows 32 w .. 32 w + 31 of a 128-row tile and keeps their Q fragments
 // (bf16) in registers.  Scores are computed transposed, S^T = K Q^T (v_mfma_f32_32x32x8_bf16_1k: A = 32 keys x 8 features from LDS, B = the lane's own
@@ -611,7 +787,13 @@ extern "C" int mi355_latent_attn(int n_seq, int max_new, int H, int hm, int D1, 
         }
         return 0;
     }
-#define FMA(NC) do { if (dt == MI355_DT_F32) latent_attn_fma_kernel<NC, float><<<grid, 256, 0, ST(stream)>>>(p); else latent_attn_fma_kernel<NC, bf16_t><<<grid, 256, 0, ST(stream)>>>(p); } while (0)
+    int from = 0;
+    if ((max_new <= STEP_NEW || n_seq > 1) && latent_attn_step_launch(p, max_new, n_seq, ST(stream))) {  // (one sequence of more tokens is none of its)
+        MI355_LAUNCH_CHECK("latent_attn(step)");
+        if (max_new <= STEP_NEW) return 0;
+        from = STEP_NEW + 1;
+    }
+#define FMA(NC) do { if (dt == MI355_DT_F32) latent_attn_fma_kernel<NC, float><<<grid, 256, 0, ST(stream)>>>(p, from); else latent_attn_fma_kernel<NC, bf16_t><<<grid, 256, 0, ST(stream)>>>(p, from); } while (0)
     if (DV <= 64) FMA(1); else if (DV <= 128) FMA(2); else if (DV <= 256) FMA(4); else FMA(8);
 #undef FMA
     MI355_LAUNCH_CHECK("latent_attn");

@@ -58,3 +58,94 @@ def test_experts_of_few_rows(counts, K, N, epi, dt):
             y, err = torch.relu(y) ** 2, 2 * mag * err
         s = sc[r].double()[:, None]
         assert bool(((out[r].double() - y * s).abs() <= err * s + 4 * EPS * (y * s).abs()).all())
+
+
+CASES = [dict(), dict(shared=True, D2=8), dict(shared=True, values_are_keys=True, D1=256, D2=64, DV=256, H=8), dict(H=6, rep=3, DV=70), dict(H=8, rep=4, window=37, keep=5), dict(H=4, rep=2, chunk=48),
+         dict(H=3, window=20, chunk=64, softcap=3.0), dict(H=5, shared=True, sink=True, slope=True), dict(H=2, sig=True, window=33), dict(H=4, gate=True, softcap=2.0, D1=130, DV=257),
+         dict(H=9, shared=True, D1=512, D2=128, DV=512, values_are_keys=True), dict(H=2, D1=100, DV=129, window=1), dict(H=4, rep=4, sink=True, window=16, keep=64)]
+
+
+@pytest.mark.parametrize("opt", CASES, ids=lambda o: "-".join(f"{k}{int(v)}" for k, v in o.items()) or "plain")
+@pytest.mark.parametrize("dt", [F32, BF16])
+def test_attention_of_one_or_two_new_tokens(opt, dt):
+    """Sequences of 1, 2 and 3 new tokens after 0 .. 200 keys in one step, every option; the rows of a sequence are bit by bit those it has alone.  Scores are sums of D products and
+    a weight's relative error is its score's error; the values' sum over n keys rounds n times: 64 bits within 2^-24 (n + |q||k| scale (D + 4)) of the largest weighted value."""
+    from llm_quest_amd import kernels_seq as S
+
+    H, D1, D2, DV = opt.get("H", 2), opt.get("D1", 64), opt.get("D2", 0), opt.get("DV", 48)
+    rep, shared, same = opt.get("rep", 1), opt.get("shared", False), opt.get("values_are_keys", False)
+    window, keep, chunk, cap = opt.get("window", 0), opt.get("keep", 0), opt.get("chunk", 0), opt.get("softcap", 0.0)
+    new, past = [1, 2, 3, 1, 2, 1, 1], [0, 0, 5, 31, 64, 129, 200]
+    g = torch.Generator().manual_seed(H * D1 + DV)
+    G = 1 if shared else H // rep
+    total = [n + p for n, p in zip(new, past)]
+    T, R = sum(total), sum(new)
+    k1, k2 = torch.randn(T, G * D1, generator=g).to(dt).cuda(), torch.randn(T, max(D2, 1), generator=g).to(dt).cuda()
+    v = k1 if same else torch.randn(T, G * DV, generator=g).to(dt).cuda()
+    q = (torch.randn(R, H * (D1 + D2), generator=g)).cuda()
+    sink, slope, sig = [torch.randn(H, generator=g).cuda() if opt.get(n) else None for n in ("sink", "slope", "sig")]
+    slope = slope.abs() * 0.1 if slope is not None else None
+    gate = torch.randn(R, H * DV, generator=g).cuda() if opt.get("gate") else None
+    scale = (D1 + D2) ** -0.5
+    cum = lambda a: [sum(a[:i]) for i in range(len(a))]
+    q0, k0 = cum(new), cum(total)
+
+    def run(seqs):
+        out = torch.full((R, H * DV), float("nan"), device="cuda")
+        pick = lambda a: i32([a[i] for i in seqs])
+        desc = (pick(q0), pick(new), pick(past), pick(k0), pick(k0), pick(k0))
+        hm = 1
+        while hm * 2 <= 8 and (shared or rep % (hm * 2) == 0):
+            hm *= 2
+        return _fp32_path(S, q, k1, k2 if D2 else None, v, out, H, hm, D1, D2, DV, shared, desc, max(new[i] for i in seqs), scale, 1 if shared else rep, window, keep, cap, sink, chunk, sig, slope, gate)
+
+    got = run(list(range(len(new))))
+    for i in range(len(new)):
+        rows = slice(q0[i], q0[i] + new[i])
+        assert torch.equal(got[rows], run([i])[rows])
+        if i >= 2:
+            assert torch.equal(got[rows], run([0, i])[rows]) and torch.equal(got[rows], run([i, 2] if i != 2 else [2, 6])[rows])
+        n = total[i]
+        ks = k1[k0[i] : k0[i] + n].double().view(n, G, D1).expand(n, H, D1) if shared else k1[k0[i] : k0[i] + n].double().view(n, G, D1).repeat_interleave(rep, 1)
+        if D2:
+            ks = torch.cat([ks, k2[k0[i] : k0[i] + n].double()[:, None].expand(n, H, D2)], -1)
+        vs = v[k0[i] : k0[i] + n].double().view(n, G, -1)[..., :DV]
+        vs = vs.expand(n, H, DV) if shared else vs.repeat_interleave(rep, 1)
+        qs = q[rows].double().view(new[i], H, D1 + D2)
+        s = (qs[:, None] * ks[None]).sum(-1).permute(0, 2, 1) * scale  # [new, H, n]
+        mag = ((qs[:, None] * ks[None]).abs().sum(-1).permute(0, 2, 1) * scale).amax()
+        at = past[i] + torch.arange(new[i], device="cuda")[:, None]
+        j = torch.arange(n, device="cuda")[None]
+        lo = torch.zeros_like(at)
+        if window:
+            lo = torch.maximum(lo, at - window + 1)
+        if chunk:
+            lo = torch.maximum(lo, at // chunk * chunk)
+        see = (j <= at) & ((j >= lo) | (j < keep))
+        if cap:
+            s = cap * torch.tanh(s / cap)
+        if slope is not None:
+            s = s - slope.double()[None, :, None] * (at - j)[:, None]
+        if sig is not None:
+            p = torch.sigmoid(s + sig.double()[None, :, None]) * see[:, None]
+        else:
+            s = s.masked_fill(~see[:, None], float("-inf"))
+            if sink is not None:
+                s = torch.cat([s, sink.double()[None, :, None].expand(new[i], H, 1)], -1)
+            p = torch.softmax(s, -1)[..., :n]
+        want = (p.permute(0, 2, 1)[..., None] * vs[None]).sum(1)
+        size = (p.permute(0, 2, 1)[..., None] * vs[None].abs()).sum(1)
+        if gate is not None:
+            f = torch.sigmoid(gate[rows].double().view(new[i], H, DV))
+            want, size = want * f, size * f
+        err = 2 * EPS * (n + mag * (D1 + D2 + 4) + 64) * size
+        assert bool(((got[rows].double().view(new[i], H, DV) - want).abs() <= err + 1e-30).all())
+
+
+def _fp32_path(S, q, k1, k2, v, out, H, hm, D1, D2, DV, shared, desc, max_new, scale, rep, window, keep, cap, sink, chunk, sig, slope, gate):
+    """The fp32 products for either type of the keys (the launcher takes the matrix pipe for bf16 ones)."""
+    L = S.L
+    L.call("mi355_latent_attn", desc[0].numel(), max_new, H, hm, D1, D2, DV, L.ptr(q), q.stride(0), D1 + D2, L.ptr(k1), k1.stride(0), 0 if shared else D1, L.ptr(k2), 0 if k2 is None else k2.stride(0),
+           L.ptr(v), v.stride(0), 0 if shared else (D1 if v is k1 else DV), L.ptr(out), out.stride(0), DV, S._dt(v), *[L.ptr(t) for t in desc], float(scale), 0, 1, None, 0, rep, window, keep, cap, L.ptr(sink),
+           0, None, None, 0, None, chunk, L.ptr(sig), S._dt(out), L.ptr(slope), L.ptr(gate), 0 if gate is None else gate.stride(0))
+    return out
