@@ -7,6 +7,7 @@
 // decays, recurrent state and router arithmetic are fp32 in both modes.  A "row" is a token of the packed batch; sequences are described
 // by int32 device arrays.  One wave works on one row unless stated.
 #include "common.h"
+#include "lane_sums.h"
 
 #define ST(s) ((hipStream_t)(s))
 
@@ -367,22 +368,66 @@ extern "C" int mi355_gated_headnorm(int64_t tokens, int H, int D, const float* o
 // a_t = sigmoid(z_t + zbias)^(inv_tau) = exp(inv_tau * logsigmoid(.)) in fp32 -- or, with head_decay, the constant head_decay[h] for every key channel
 // of head h (retention: z / zbias are then unused).  k_t is multiplied by kscale.
 // Block: 64 value columns x RC row chunks of GLA_R key channels; a thread keeps GLA_R state entries of one column in registers.
-// Tokens go through in groups of GLA_TB: the group's q / k / decay rows are staged in LDS once, partial outputs of the row chunks meet in LDS.
+// Tokens go through in groups of TB (16; 8 where 16 do not fit LDS): the group's q / k / decay rows are staged in LDS once, partial outputs of the row chunks meet in LDS.  A wave's 16 channels of a token are
+// one LDS word a lane for each of q, k and the decay, dealt out over the lanes by the operand modifiers of the products (48 words a lane were 0.8 us of LDS traffic a token); three
+// products with a sum each per state entry.  Three sequences of 150 tokens, 16 heads of 128 channels, 128 columns, three layers and four steps each: 604 -> 413 us; one token a sequence 16 -> 8.9 us a launch.
 #define GLA_R 16
-#define GLA_TB 8
 __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
-__global__ void gla_kernel(const int* __restrict__ seq_off, const int* __restrict__ slot, int H, int dk, int dv, const void* __restrict__ q, const void* __restrict__ k,
+// st[r] <- a[r] st[r] + k[r] v, acc += q[r] st[r] for the 16 channels that the lanes of a row of 16 hold one of: row_newbcast:r is lane r's operand for all of them.  (hipcc moves the
+// broadcast operand of a sum of products to a register first; s_nop: operands that a vector instruction may just have written.)
+__device__ __forceinline__ void gla_rows(float (&st)[GLA_R], float& acc, float q, float k, float a, float v) {
+    static_assert(GLA_R == 16, "one channel a lane of a row");
+    asm("s_nop 1\n\t"
+                 "v_mul_f32_dpp %0, %19, %0 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %0, %18, %20 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %1, %19, %1 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %1, %18, %20 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %2, %19, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %2, %18, %20 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %3, %19, %3 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %3, %18, %20 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %4, %19, %4 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %4, %18, %20 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %5, %19, %5 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %5, %18, %20 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %6, %19, %6 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %6, %18, %20 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %7, %19, %7 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %7, %18, %20 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %8, %19, %8 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %8, %18, %20 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %9, %19, %9 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %9, %18, %20 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %10, %19, %10 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %10, %18, %20 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %11, %19, %11 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %11, %18, %20 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %12, %19, %12 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %12, %18, %20 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %13, %19, %13 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %13, %18, %20 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %14, %19, %14 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %14, %18, %20 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_mul_f32_dpp %15, %19, %15 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\tv_fmac_f32_dpp %15, %18, %20 row_newbcast:15 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %0 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %1 row_newbcast:1 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %2 row_newbcast:2 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %3 row_newbcast:3 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %4 row_newbcast:4 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %5 row_newbcast:5 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %6 row_newbcast:6 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %7 row_newbcast:7 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %8 row_newbcast:8 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %9 row_newbcast:9 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %10 row_newbcast:10 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %11 row_newbcast:11 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %12 row_newbcast:12 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %13 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %14 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
+                 "v_fmac_f32_dpp %16, %17, %15 row_newbcast:15 row_mask:0xf bank_mask:0xf"
+        : "+v"(st[0]), "+v"(st[1]), "+v"(st[2]), "+v"(st[3]), "+v"(st[4]), "+v"(st[5]), "+v"(st[6]), "+v"(st[7]), "+v"(st[8]), "+v"(st[9]), "+v"(st[10]), "+v"(st[11]), "+v"(st[12]),
+          "+v"(st[13]), "+v"(st[14]), "+v"(st[15]), "+v"(acc)
+        : "v"(q), "v"(k), "v"(a), "v"(v));
+}
+
+template <int TB>
+__global__ __launch_bounds__(TB == 16 ? 512 : 1024) void gla_kernel(const int* __restrict__ seq_off, const int* __restrict__ slot, int H, int dk, int dv, const void* __restrict__ q, const void* __restrict__ k,
                            const void* __restrict__ v, const void* __restrict__ z, int dt, int z_dt, int v_dt, int64_t ldq, int64_t ldk, int64_t ldv_, int64_t ldz,
                            const float* __restrict__ zbias, float inv_tau, float qscale, const float* __restrict__ head_decay, float kscale,
                            float* __restrict__ state, float* __restrict__ o, int below) {
     extern __shared__ __attribute__((aligned(16))) float smem[];
     const int RC = blockDim.x >> 6;
     float* sq = smem;                       // [TB][dk]
-    float* sk = sq + GLA_TB * dk;           // [TB][dk]
-    float* sa = sk + GLA_TB * dk;           // [TB][dk]
-    float* sv = sa + GLA_TB * dk;           // [TB][64]
-    float* sp = sv + GLA_TB * 64;           // [TB][RC][64]
+    float* sk = sq + TB * dk;           // [TB][dk]
+    float* sa = sk + TB * dk;           // [TB][dk]
+    float* sv = sa + TB * dk;           // [TB][64]
+    float* sp = sv + TB * 64;           // [TB][RC][64]
     const int s = blockIdx.x, h = blockIdx.y, col = blockIdx.z * 64 + (threadIdx.x & 63), chunk = threadIdx.x >> 6;
     const int t0 = seq_off[s], t1 = seq_off[s + 1];
     if (below && t1 - t0 >= below) return;  // (the same for the whole workgroup)
@@ -395,79 +440,84 @@ __global__ void gla_kernel(const int* __restrict__ seq_off, const int* __restric
         st[r] = (col_ok && i < dk) ? S[(int64_t)i * dv + col] : 0.f;
     }
     // the next group's rows travel from memory into registers while the current group is worked on (a group's loads would otherwise cost a full
-    // memory round trip between every eight tokens); dk <= 16 RC, so a thread carries at most 2 entries of q / k / z and 8 of v
-    float rq[2], rk[2], rz[2], rv[8];
+    // memory round trip between every group).  A thread carries one channel of every P-th token of q / k / z (blockDim >= 4 dk, so P >= 4), and one value column of every RC-th.
+    const int P = (int)blockDim.x / dk, j0 = threadIdx.x / dk, i0 = threadIdx.x - j0 * dk, vc = blockIdx.z * 64 + (threadIdx.x & 63);
+    const bool mine = j0 < P;
+    const float zb = head_decay || !mine ? 0.f : zbias[h * dk + i0], hd = head_decay ? head_decay[h] : 0.f;
+    float rq[TB / 4], rk[TB / 4], rz[TB / 4], rv[TB];
     auto fetch = [&](int tb) {
-        const int nt = min(GLA_TB, t1 - tb);
+        const int nt = min(TB, t1 - tb);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = threadIdx.x + u * blockDim.x;
-            rq[u] = rk[u] = rz[u] = 0.f;
-            if (e < nt * dk) {
-                const int j = e / dk, i = e % dk;
-                const int64_t t = tb + j;
-                rq[u] = ld_dt(q, dt, t * ldq + (int64_t)h * dk + i);
-                rk[u] = ld_dt(k, dt, t * ldk + (int64_t)h * dk + i);
-                if (!head_decay) rz[u] = ld_dt(z, z_dt, t * ldz + (int64_t)h * dk + i) + zbias[h * dk + i];
+        for (int u = 0; u < TB / 4; ++u) {
+            if (u * P >= nt) break;
+            const int j = j0 + u * P;
+            if (mine && j < nt) {
+                const int64_t t = tb + j, at = (int64_t)h * dk + i0;
+                rq[u] = ld_dt(q, dt, t * ldq + at);
+                rk[u] = ld_dt(k, dt, t * ldk + at);
+                if (!head_decay) rz[u] = ld_dt(z, z_dt, t * ldz + at);
             }
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int e = threadIdx.x + u * blockDim.x;
-            rv[u] = 0.f;
-            if (e < nt * 64) {
-                const int j = e >> 6, c = blockIdx.z * 64 + (e & 63);
-                if (c < dv) rv[u] = ld_dt(v, v_dt, (int64_t)(tb + j) * ldv_ + (int64_t)h * dv + c);
-            }
+        for (int u = 0; u < TB; ++u) {
+            if (u * RC >= nt) break;
+            const int j = chunk + u * RC;
+            rv[u] = j < nt && vc < dv ? ld_dt(v, v_dt, (int64_t)(tb + j) * ldv_ + (int64_t)h * dv + vc) : 0.f;
         }
     };
     if (t0 < t1) fetch(t0);
-    for (int tb = t0; tb < t1; tb += GLA_TB) {
-        const int nt = min(GLA_TB, t1 - tb);
+    for (int tb = t0; tb < t1; tb += TB) {
+        const int nt = min(TB, t1 - tb);
         __syncthreads();  // the previous group's rows and partial sums are consumed
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int e = threadIdx.x + u * blockDim.x;
-            if (e < nt * dk) {
+        for (int u = 0; u < TB / 4; ++u) {
+            if (u * P >= nt) break;
+            const int j = j0 + u * P;
+            if (mine && j < nt) {
+                const int e = j * dk + i0;
                 sq[e] = rq[u] * qscale;
                 sk[e] = rk[u] * kscale;
-                sa[e] = head_decay ? head_decay[h] : expf(inv_tau * log_sigmoid(rz[u]));
+                sa[e] = head_decay ? hd : expf(inv_tau * log_sigmoid(rz[u] + zb));
             }
         }
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int e = threadIdx.x + u * blockDim.x;
-            if (e < nt * 64) sv[e] = rv[u];
+        for (int u = 0; u < TB; ++u) {
+            if (u * RC >= nt) break;
+            const int j = chunk + u * RC;
+            if (j < nt) sv[j * 64 + (threadIdx.x & 63)] = rv[u];
         }
         __syncthreads();
-        if (tb + GLA_TB < t1) fetch(tb + GLA_TB);
-        const bool full = chunk * GLA_R + GLA_R <= dk && dk % 4 == 0;
-        for (int j = 0; j < nt; ++j) {
-            const float vv = sv[j * 64 + (threadIdx.x & 63)];
-            const float* qa = sq + j * dk + chunk * GLA_R;
-            const float* ka = sk + j * dk + chunk * GLA_R;
-            const float* aa = sa + j * dk + chunk * GLA_R;
-            float acc = 0.f;
-            if (full) {
-#pragma unroll
-                for (int r4 = 0; r4 < GLA_R / 4; ++r4) {
-                    const f32x4 q4 = *(const f32x4*)(qa + 4 * r4), k4 = *(const f32x4*)(ka + 4 * r4), a4 = *(const f32x4*)(aa + 4 * r4);
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        st[4 * r4 + i] = a4[i] * st[4 * r4 + i] + k4[i] * vv;
-                        acc += st[4 * r4 + i] * q4[i];
-                    }
+        if (tb + TB < t1) fetch(tb + TB);
+        const bool full = chunk * GLA_R + GLA_R <= dk;
+        if (full) {  // a lane holds one of the 16 channels' operands, and the next token's are on their way
+            const int at = chunk * GLA_R + (threadIdx.x & 15), lane = threadIdx.x & 63;
+            float qn = sq[at], kn = sk[at], an = sa[at], vn = sv[lane];
+            for (int j = 0; j < nt; ++j) {
+                const float qr = qn, kr = kn, ar = an, vv = vn;
+                if (j + 1 < nt) {
+                    const int e = (j + 1) * dk + at;
+                    qn = sq[e], kn = sk[e], an = sa[e], vn = sv[(j + 1) * 64 + lane];
                 }
-            } else {
+                float acc = 0.f;
+                gla_rows(st, acc, qr, kr, ar, vv);
+                sp[(j * RC + chunk) * 64 + lane] = acc;
+            }
+        } else {
+            for (int j = 0; j < nt; ++j) {
+                const float vv = sv[j * 64 + (threadIdx.x & 63)];
+                const float* qa = sq + j * dk + chunk * GLA_R;
+                const float* ka = sk + j * dk + chunk * GLA_R;
+                const float* aa = sa + j * dk + chunk * GLA_R;
+                float acc = 0.f;
 #pragma unroll
                 for (int r = 0; r < GLA_R; ++r) {
                     if (chunk * GLA_R + r < dk) {
-                        st[r] = aa[r] * st[r] + ka[r] * vv;
-                        acc += st[r] * qa[r];
+                        st[r] = fmaf(ka[r], vv, aa[r] * st[r]);
+                        acc = fmaf(qa[r], st[r], acc);
                     }
                 }
+                sp[(j * RC + chunk) * 64 + (threadIdx.x & 63)] = acc;
             }
-            sp[(j * RC + chunk) * 64 + (threadIdx.x & 63)] = acc;
         }
         __syncthreads();
         for (int e = threadIdx.x; e < nt * 64; e += blockDim.x) {
@@ -494,10 +544,13 @@ extern "C" int mi355_gla_fwd_below(int n_seq, const int* seq_off, const int* slo
     MI355_REQUIRE(head_decay || (z && zbias && dt_ok(z_dt) && ldz >= (int64_t)H * dk), "gla_fwd: the decay needs its rows and bias, or a constant per head");
     MI355_REQUIRE(ldq >= (int64_t)H * dk && ldk >= (int64_t)H * dk && ldv >= (int64_t)H * dv, "gla_fwd: rows too short");
     const int RC = (dk + GLA_R - 1) / GLA_R;
-    const size_t lds_bytes = sizeof(float) * ((size_t)3 * GLA_TB * dk + (size_t)GLA_TB * 64 + (size_t)GLA_TB * RC * 64);
+    const size_t lds_bytes = sizeof(float) * ((size_t)3 * 8 * dk + (size_t)8 * 64 + (size_t)8 * RC * 64);
     MI355_REQUIRE(lds_bytes <= 64 * 1024, "gla_fwd: LDS budget exceeded");
-    gla_kernel<<<dim3(n_seq, H, (dv + 63) / 64), 64 * RC, lds_bytes, ST(stream)>>>(seq_off, slot, H, dk, dv, q, k, v, z, dt, z_dt, v_dt, ldq, ldk, ldv, ldz, zbias, inv_tau, qscale,
-                                                                                   head_decay, kscale, state, o, below);
+    const dim3 grid(n_seq, H, (dv + 63) / 64);
+    if (2 * lds_bytes <= 64 * 1024 && RC <= 8)
+        gla_kernel<16><<<grid, 64 * RC, 2 * lds_bytes, ST(stream)>>>(seq_off, slot, H, dk, dv, q, k, v, z, dt, z_dt, v_dt, ldq, ldk, ldv, ldz, zbias, inv_tau, qscale, head_decay, kscale, state, o, below);
+    else
+        gla_kernel<8><<<grid, 64 * RC, lds_bytes, ST(stream)>>>(seq_off, slot, H, dk, dv, q, k, v, z, dt, z_dt, v_dt, ldq, ldk, ldv, ldz, zbias, inv_tau, qscale, head_decay, kscale, state, o, below);
     MI355_LAUNCH_CHECK("gla_fwd");
     return 0;
 }

@@ -149,3 +149,36 @@ def _fp32_path(S, q, k1, k2, v, out, H, hm, D1, D2, DV, shared, desc, max_new, s
            L.ptr(v), v.stride(0), 0 if shared else (D1 if v is k1 else DV), L.ptr(out), out.stride(0), DV, S._dt(v), *[L.ptr(t) for t in desc], float(scale), 0, 1, None, 0, rep, window, keep, cap, L.ptr(sink),
            0, None, None, 0, None, chunk, L.ptr(sig), S._dt(out), L.ptr(slope), L.ptr(gate), 0 if gate is None else gate.stride(0))
     return out
+
+
+@pytest.mark.parametrize("H,dk,dv,fixed,dt", [(1, 1, 5, False, F32), (2, 16, 64, False, BF16), (2, 17, 65, True, F32), (1, 64, 64, False, F32), (2, 96, 100, False, BF16), (1, 112, 64, True, F32), (1, 128, 130, False, F32), (1, 144, 64, True, BF16),
+                                              (1, 256, 70, False, F32)])
+def test_gla_in_groups_of_16_and_of_8_tokens(H, dk, dv, fixed, dt):
+    """Key channels that fill the rows of 16 lanes and that do not, groups of 16 tokens and (where those exceed LDS or half the threads) of 8, sequences that end around a group.  The state
+    rounds twice a token, the output dk + RC times: 64 bits within 2^-24 (2 T + dk + 40) of the sums of sizes (decays: a few roundings each, which the 16 T term holds)."""
+    from llm_quest_amd import kernels_seq as S
+
+    n = [1, 7, 8, 9, 0, 15, 16, 17, 33]
+    T = sum(n)
+    g = torch.Generator().manual_seed(dk + dv)
+    q, k, v = (torch.randn(T, H * w, generator=g).to(dt).cuda() for w in (dk, dk, dv))
+    z, bias, dec = torch.randn(T, H * dk, generator=g).cuda() + 2, 0.3 * torch.randn(H * dk, generator=g).cuda(), (0.5 + 0.5 * torch.rand(H, generator=g)).cuda()
+    st0 = torch.randn(len(n) + 1, H, dk, dv, generator=g).cuda()
+    slots = torch.arange(len(n), 0, -1)
+    st = st0.clone()
+    offs = [sum(n[:i]) for i in range(len(n) + 1)]
+    if fixed:
+        got = S.gla(q, k, v, None, None, 1.0, dk**-0.5, i32(offs), i32(slots.tolist()), st, H, dk, dv, head_decay=dec, kscale=0.5)
+    else:
+        got = S.gla(q, k, v, z, bias, 0.25, dk**-0.5, i32(offs), i32(slots.tolist()), st, H, dk, dv)
+    a = dec.double()[None, :, None].expand(T, H, dk) if fixed else torch.sigmoid((z.double() + bias.double()).view(T, H, dk)) ** 0.25
+    assert torch.equal(st[0], st0[0])
+    for i, sl in enumerate(slots.tolist()):
+        s, m = st0[sl].double(), st0[sl].double().abs()
+        for t in range(offs[i], offs[i + 1]):
+            kv = (k[t].double().view(H, dk, 1) * (0.5 if fixed else 1.0)) * v[t].double().view(H, 1, dv)
+            s, m = a[t][..., None] * s + kv, a[t][..., None] * m + kv.abs()
+            qt = q[t].double().view(H, dk) * dk**-0.5
+            want, size = torch.einsum("hk,hkv->hv", qt, s), torch.einsum("hk,hkv->hv", qt.abs(), m)
+            assert bool(((got[t].double().view(H, dv) - want).abs() <= EPS * (16 * (t - offs[i] + 1) + dk + 40) * size).all())
+        assert bool(((st[sl].double() - s).abs() <= EPS * (16 * n[i] + 4) * m).all())
