@@ -42,6 +42,26 @@ __device__ __forceinline__ double cumulated_log(const float* alpha, int64_t idx,
 // a token's beta; zero counts as 1e-30 (as the decays' floor: nothing that is kept changes, and u / beta is v minus what the state already holds)
 __device__ __forceinline__ float beta_of(const float* beta, int64_t idx, bool in) { return in ? decay_at_least(beta[idx]) : 0.f; }
 
+// four consecutive bf16 of row `r`, or of the last row where `r` lies beyond the sequence (its reader puts zeros there): a load without a branch, which can be under way
+__device__ __forceinline__ u32x2 held4(const bf16_t* p, int64_t ld, int r, int cnt, int c) { return *reinterpret_cast<const u32x2*>(p + min(r, cnt - 1) * ld + c); }
+__device__ __forceinline__ u32x4 held8(const bf16_t* p, int64_t ld, int r, int cnt, int c) { return *reinterpret_cast<const u32x4*>(p + min(r, cnt - 1) * ld + c); }
+// requests stay in front of the products that hide them (short of registers, the compiler moves them down to where they are used)
+__device__ __forceinline__ void in_order() { __builtin_amdgcn_sched_barrier(0); }
+// a lane's 16 features of a row (transposed accumulators: c_row(4 c, hf) on); wide: the rows lie on 8-byte words
+__device__ __forceinline__ void put16(bf16_t* p, const f32x4 (&v)[4], int hf, bool wide) {
+    if (wide) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) *reinterpret_cast<u32x2*>(p + c_row(4 * c, hf)) = u32x2{pack_bf2(v[c][0], v[c][1]), pack_bf2(v[c][2], v[c][3])};
+    } else {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) p[c_row(e, hf)] = f2bf(v[e >> 2][e & 3]);
+    }
+}
+__device__ __forceinline__ float both_halves(float v) {  // the sum over a lane and its other half's
+    const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return __uint_as_float(r[0]) + __uint_as_float(r[1]);
+}
+
 // The scans' workgroups: the four value ranges of a head read the same Kw / P / Q / K, so they go to one XCD (workgroups are dealt to the eight XCDs in turn), side by side.
 __device__ __forceinline__ bool scan_place(int heads, int& head, int& v0) {
     const int id = blockIdx.x;
@@ -480,17 +500,26 @@ __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, in
 }
 
 // ------------------------------------------------------------------------------------------- the rest of the backward: one workgroup per chunk and head
+// Bound: the fp32 matrix pipe (130 us of 8 x 708 tokens x 16 heads) and the chunk's blocks from memory (0.5 GB, 105 us), with eight waves a CU to overlap them; so
+// nothing may stand between the products.  542 -> 287 us (96 chunks, one a CU: 110 -> 50): sums over a token's features meet in a lane, since results are taken transposed (half-wave
+// sums, one row after the other, were a quarter of the time); loads carry no condition (rows beyond the sequence are its last, and what they give is dropped) and stand two stages
+// ahead, held there by in_order(); the first product's operands are requested all at once; the pairs' decay sums go by 256 threads and scans instead of 64 chains (25 000 clocks -> 5 000).
+// Requests three stages ahead: 293 us (registers spill); the two workgroups of a CU set off apart: 370 against 366 at that time.
 __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const bf16_t* __restrict__ v,
                                                           int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha, const float* __restrict__ saved,
                                                           const float* __restrict__ ws, const bf16_t* __restrict__ d_o, bf16_t* __restrict__ dq, bf16_t* __restrict__ dk,
                                                           bf16_t* __restrict__ dv, int64_t lddv, float* __restrict__ dbeta, float* __restrict__ dalpha, float* __restrict__ pdq,
-                                                          float* __restrict__ pdk, float qscale) {
+                                                          float* __restrict__ pdk, float qscale, int wide) {
     constexpr int LM = GC + 4, LZ = GC + 2;
     __shared__ __attribute__((aligned(16))) float Z[GC][GD + 4];   // -dU S0; later Y, then d(Q K^T) (first half), and the pairs' decay terms (second half)
-    __shared__ __attribute__((aligned(16))) float M1[GC][LM];      // dR; later d(K K^T) + its transpose
-    __shared__ __attribute__((aligned(16))) float M2[GC][LM];      // R
+    __shared__ __attribute__((aligned(16))) float M12[2 * GC * LM];  // dU; later the next two
+    float(*M1)[LM] = reinterpret_cast<float(*)[LM]>(M12);            // dR; later d(K K^T) + its transpose
+    float(*M2)[LM] = reinterpret_cast<float(*)[LM]>(M12 + GC * LM);  // R
+    float(*Ud)[GD + 4] = reinterpret_cast<float(*)[GD + 4]>(M12);
+    static_assert(GC * (GD + 4) <= 2 * GC * LM, "dU fits the space of the two matrices");
     __shared__ double gd[GC];
     __shared__ float be[GC], al[GC], gam[GC], gp[GC], redG[4][GC], redP[4][GC], redB[4][GC], dss[4];
+    __shared__ double pairs[4][GC];
     float(*M3)[LZ] = reinterpret_cast<float(*)[LZ]>(&Z[0][0]);
     float(*ME)[LZ] = reinterpret_cast<float(*)[LZ]>(&Z[0][0] + GC * LZ);
     static_assert(2 * GC * LZ <= GC * (GD + 4), "both late matrices fit the early one's space");
@@ -501,123 +530,180 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
     const float* blk = saved + (head * NC + n) * G_BLOCK;
     const float *dS = ws + (head * NC + n) * W_BLOCK, *dU = dS + W_DU, *Up = blk + G_U;
     const int col = 32 * wave + ln;
+    // Everything of the first product is requested at once: dU, which the next phase reads too, goes to LDS, a lane's share of the first state stays in registers.
+    f32x4 ud[8];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 4;
-        *reinterpret_cast<f32x4*>(&M2[r][c]) = *reinterpret_cast<const f32x4*>(blk + G_R + r * GC + c);
-    }
-    if (wave == 0) {
-        float a;
-        gd[lane] = cumulated_log(alpha, (tok0 + lane) * Hv + h, lane < cnt, a);
-        al[lane] = a;
-        be[lane] = beta_of(beta, (tok0 + lane) * Hv + h, lane < cnt);
-        gam[lane] = blk[G_GAM + lane];
-        gp[lane] = blk[G_GAM + GC + lane];
-    }
-    {  // Z = -dU S0: wave = 32 columns, both row halves, contraction over the value rows straight from memory (a state row's 32 columns are one line)
+    for (int i = 0; i < 8; ++i) ud[i] = *reinterpret_cast<const f32x4*>(dU + 4 * (tid + 256 * i));
+    float st[GD / 2];
+#pragma unroll
+    for (int j = 0; j < GD / 2; ++j) st[j] = blk[(8 * (j >> 2) + 4 * hf + (j & 3)) * GD + col];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) *reinterpret_cast<f32x4*>(&Ud[(tid + 256 * i) >> 5][((tid + 256 * i) & 31) * 4]) = ud[i];
+    __syncthreads();
+    {  // Z = -dU S0: wave = 32 columns, both row halves
         f32x16 z[2] = {zero16(), zero16()};
-        f32x4 du[2];
-        float s0[4];
-        auto request = [&](int kb) {
 #pragma unroll
-            for (int r = 0; r < 2; ++r) du[r] = *reinterpret_cast<const f32x4*>(dU + (32 * r + ln) * GD + kb + 4 * hf);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s0[j] = blk[(kb + 4 * hf + j) * GD + col];
-        };
-        request(0);
-#pragma unroll 2
         for (int kb = 0; kb < GD; kb += 8) {
-            const f32x4 c0 = -du[0], c1 = -du[1], cs = {s0[0], s0[1], s0[2], s0[3]};
-            if (kb + 8 < GD) request(kb + 8);
+            const f32x4 d0 = *reinterpret_cast<const f32x4*>(&Ud[ln][kb + 4 * hf]), d1 = *reinterpret_cast<const f32x4*>(&Ud[32 + ln][kb + 4 * hf]);
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                z[0] = mfma2(c0[j], cs[j], z[0]);
-                z[1] = mfma2(c1[j], cs[j], z[1]);
+                z[0] = mfma2(st[kb / 2 + j], -d0[j], z[0]);
+                z[1] = mfma2(st[kb / 2 + j], -d1[j], z[1]);
             }
         }
 #pragma unroll
         for (int r = 0; r < 2; ++r)
 #pragma unroll
-            for (int e = 0; e < 16; ++e) Z[32 * r + c_row(e, hf)][col] = z[r][e];
+            for (int e = 0; e < 16; e += 4) *reinterpret_cast<f32x4*>(&Z[32 * r + ln][32 * wave + c_row(e, hf)]) = f32x4{z[r][e], z[r][e + 1], z[r][e + 2], z[r][e + 3]};
     }
     __syncthreads();
     // the 64 x 64 matrices: wave = tile (ti, tj)
     const int ti = wave >> 1, tj = wave & 1, j0 = 32 * tj + ln;
     f32x16 lkk, e1, dqk;
+    f32x4 rr[4];
+    float un[32];  // dU once more, by columns
     {
         f32x16 kk = zero16(), qk = zero16(), dP = zero16(), dT = zero16(), tz = zero16(), dPt = zero16();
         if (wave != 1) {
             const int ri = 32 * ti + ln, rj = 32 * tj + ln;
+            const float* ur = Up + rj * GD + 8 * hf;
+            struct Stage {  // 16 features, a half wave's eight of them together
+                u32x4 o, v, k, qi, ki;
+                f32x4 u[2];
+            };
+            auto request = [&](Stage& t, int kb) {
+                t.o = held8(op, ldo, ri, cnt, kb + 8 * hf), t.v = held8(vp, ldv, rj, cnt, kb + 8 * hf), t.k = held8(kp, ldqk, rj, cnt, kb + 8 * hf);
+                t.qi = held8(qp, ldqk, ri, cnt, kb + 8 * hf), t.ki = held8(kp, ldqk, ri, cnt, kb + 8 * hf);
 #pragma unroll
-            for (int c = 0; c < GD; c += 16) {
-                const u32x4 z4 = {0u, 0u, 0u, 0u};
-                const u32x4 qi = ri < cnt ? *reinterpret_cast<const u32x4*>(qp + ri * ldqk + c + 8 * hf) : z4, ki = ri < cnt ? *reinterpret_cast<const u32x4*>(kp + ri * ldqk + c + 8 * hf) : z4,
-                            kj = rj < cnt ? *reinterpret_cast<const u32x4*>(kp + rj * ldqk + c + 8 * hf) : z4;
-                kk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, ki), __builtin_bit_cast(bf16x8, kj), kk, 0, 0, 0);
-                qk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, qi), __builtin_bit_cast(bf16x8, kj), qk, 0, 0, 0);
-            }
-#pragma unroll 2
-            for (int kb = 0; kb < GD; kb += 8) {
-                const f32x4 oi = widen4(row4(op, ldo, ri, cnt, kb + 4 * hf)), uj = *reinterpret_cast<const f32x4*>(Up + rj * GD + kb + 4 * hf);
-                const f32x4 di = *reinterpret_cast<const f32x4*>(dU + ri * GD + kb + 4 * hf), vj = widen4(row4(vp, ldv, rj, cnt, kb + 4 * hf));
-                const f32x4 zi = *reinterpret_cast<const f32x4*>(&Z[ri][kb + 4 * hf]), kj = widen4(row4(kp, ldqk, rj, cnt, kb + 4 * hf));
+                for (int c = 0; c < 2; ++c) t.u[c] = *reinterpret_cast<const f32x4*>(ur + kb + 4 * c);
+                in_order();
+            };
+            auto work = [&](const Stage& t, int kb) {
+                const u32x4 &o = t.o, &v8 = t.v, &k8 = t.k;
 #pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    dP = mfma2(oi[j], uj[j], dP);
-                    dT = mfma2(di[j], vj[j], dT);
-                    tz = mfma2(zi[j], kj[j], tz);
+                for (int c = 0; c < 2; ++c) {
+                    const f32x4 of = widen4(u32x2{o[2 * c], o[2 * c + 1]}), vf = widen4(u32x2{v8[2 * c], v8[2 * c + 1]}), kf = widen4(u32x2{k8[2 * c], k8[2 * c + 1]});
+                    const f32x4 zi = *reinterpret_cast<const f32x4*>(&Z[ri][kb + 8 * hf + 4 * c]), di = *reinterpret_cast<const f32x4*>(&Ud[ri][kb + 8 * hf + 4 * c]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        dP = mfma2(of[j], t.u[c][j], dP);
+                        dT = mfma2(di[j], vf[j], dT);
+                        tz = mfma2(zi[j], kf[j], tz);
+                    }
                 }
-                if ((kb & 24) == 24) add16(dPt, dP);
+                kk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.ki), __builtin_bit_cast(bf16x8, k8), kk, 0, 0, 0);
+                qk = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, t.qi), __builtin_bit_cast(bf16x8, k8), qk, 0, 0, 0);
+            };
+            Stage x, y;
+            request(x, 0);
+            for (int kb = 0; kb < GD - 32; kb += 32) {
+                request(y, kb + 16);
+                work(x, kb);
+                request(x, kb + 32);
+                work(y, kb + 16);
+                add16(dPt, dP);
             }
+            request(y, GD - 16);
+            work(x, GD - 32);
+            work(y, GD - 16);
+            add16(dPt, dP);
             add16(dP, dPt);
+        } else {  // (the upper right tiles are empty)
+            float a;
+            gd[lane] = cumulated_log(alpha, (tok0 + lane) * Hv + h, lane < cnt, a);
+            al[lane] = a;
+            be[lane] = beta_of(beta, (tok0 + lane) * Hv + h, lane < cnt);
+            gam[lane] = blk[G_GAM + lane];
+            gp[lane] = blk[G_GAM + GC + lane];
         }
-        const double gj = gd[j0];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
+        for (int i = 0; i < 4; ++i) rr[i] = *reinterpret_cast<const f32x4*>(blk + G_R + 4 * (tid + 256 * i));
+#pragma unroll
+        for (int j = 0; j < 32; ++j) un[j] = dU[(8 * (j >> 2) + 4 * hf + (j & 3)) * GD + col];
+        __syncthreads();  // dU's place is free
+        const double gj = gd[j0];
+        const float gaj = gam[j0], bj = be[j0];
+#pragma unroll
+        for (int e = 0; e < 16; ++e) {  // (no branch: what lies above the diagonal is computed and dropped)
             const int i = 32 * ti + c_row(e, hf);
-            const bool in = i >= j0;
-            const float D = in ? exp_of(gd[i] - gj) : 0.f, t = in ? dT[e] + gam[j0] * tz[e] : 0.f, p = in ? qscale * dP[e] : 0.f;
-            lkk[e] = i > j0 ? kk[e] * D : 0.f;
-            e1[e] = p * (qk[e] * D);
+            const bool in = i >= j0 && i < cnt;  // (the operands' rows beyond the sequence are its last)
+            const float x = exp_of(gd[i] - gj), D = in ? x : 0.f, t = in ? dT[e] + gaj * tz[e] : 0.f, p = in ? qscale * dP[e] : 0.f;
+            lkk[e] = in && i > j0 ? kk[e] * D : 0.f;
+            e1[e] = in ? p * (qk[e] * D) : 0.f;
             dqk[e] = p * D;
-            M1[i][j0] = t * be[j0];
+            M1[i][j0] = t * bj;
+            if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);  // (four at a time: the registers)
         }
+        asm volatile("" : "+v"(lkk), "+v"(e1), "+v"(dqk));  // (here and not where they are first used: three products' sums would stay instead)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) *reinterpret_cast<f32x4*>(&M2[(tid + 256 * i) >> 4][((tid + 256 * i) & 15) * 4]) = rr[i];
     }
     __syncthreads();
+    // From here on results are taken transposed (the operands change places, the products and their order stay): a lane holds 16 features of one token, four neighbours at a time, so
+    // what a token sums over its features meets in the lane and its other half, and rows are read and written four features at a time.
     f32x16 w[2];  // dK, from here on
     {  // dV = T^T dU, d(gam K) = T^T Z: wave = 32 columns
-        f32x16 a[2] = {zero16(), zero16()}, g[2] = {zero16(), zero16()}, at = zero16(), gt = zero16();
-#pragma unroll 2
-        for (int kb = 0; kb < GC; kb += 8) {
+        f32x16 a[2] = {zero16(), zero16()}, g[2] = {zero16(), zero16()};
+#pragma unroll
+        for (int kb = 0; kb < 32; kb += 8)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = kb + 4 * hf + j;
-                const float bu = dU[i * GD + col], bz = Z[i][col], r0 = M2[i][ln], r1 = M2[i][32 + ln];
-                a[0] = mfma2(r0, bu, a[0]);
-                g[0] = mfma2(r0, bz, g[0]);
-                if (kb >= 32) {  // R is lower triangular
-                    a[1] = mfma2(r1, bu, a[1]);
-                    g[1] = mfma2(r1, bz, g[1]);
-                }
+                const float r0 = M2[i][ln];
+                a[0] = mfma2(un[kb / 2 + j], r0, a[0]);
+                g[0] = mfma2(Z[i][col], r0, g[0]);
             }
-            if (kb == 24) add16(at, a[0]), add16(gt, g[0]);
-        }
+        f32x16 at = zero16(), gt = zero16();
+        add16(at, a[0]), add16(gt, g[0]);
+#pragma unroll
+        for (int kb = 32; kb < GC; kb += 8)  // R is lower triangular
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = kb + 4 * hf + j;
+                const float bz = Z[i][col], r0 = M2[i][ln], r1 = M2[i][32 + ln];
+                a[0] = mfma2(un[kb / 2 + j], r0, a[0]);
+                g[0] = mfma2(bz, r0, g[0]);
+                a[1] = mfma2(un[kb / 2 + j], r1, a[1]);
+                g[1] = mfma2(bz, r1, g[1]);
+            }
         add16(a[0], at);
         add16(g[0], gt);
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < 2; ++r) {
+            const int i = 32 * r + ln;
+            const bool in = i < cnt;
+            const float bi = be[i], ga = gam[i];
+            bf16_t* out = dv + (tok0 + i) * lddv + (int64_t)h * GD + 32 * wave;
+            f32x4 u4[4];
+            u32x2 k4[4];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int i = 32 * r + c_row(e, hf);
-                // d(beta): what reaches u = beta (v - the state's answer to k) times that difference, which is u / beta
-                const float sb = half_sum(a[r][e] * Up[i * GD + col]);
-                if (ln == 0) redB[wave][i] = sb;
-                if (i < cnt) dv[(tok0 + i) * lddv + (int64_t)h * GD + col] = f2bf(be[i] * a[r][e]);
-                const float d = be[i] * g[r][e];
-                w[r][e] = gam[i] * d;
-                const float sg = half_sum(d * one(kp, ldqk, i, cnt, col));
-                if (ln == 0) redG[wave][i] = sg;
+            for (int c = 0; c < 4; ++c) {
+                u4[c] = *reinterpret_cast<const f32x4*>(Up + i * GD + 32 * wave + c_row(4 * c, hf));
+                k4[c] = held4(kp, ldqk, i, cnt, 32 * wave + c_row(4 * c, hf));
             }
+            float sb[4], sg[4];
+            f32x4 ov[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const f32x4 kf = widen4(k4[c]);
+                float o[4], pb[4], pg[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float av = a[r][4 * c + j], d = bi * g[r][4 * c + j];
+                    // d(beta): what reaches u = beta (v - the state's answer to k) times that difference, which is u / beta
+                    pb[j] = av * u4[c][j];
+                    o[j] = bi * av;
+                    w[r][4 * c + j] = ga * d;
+                    pg[j] = d * kf[j];
+                }
+                sb[c] = (pb[0] + pb[1]) + (pb[2] + pb[3]);
+                sg[c] = (pg[0] + pg[1]) + (pg[2] + pg[3]);
+                ov[c] = {o[0], o[1], o[2], o[3]};
+            }
+            const float b1 = both_halves((sb[0] + sb[1]) + (sb[2] + sb[3])), g1 = both_halves((sg[0] + sg[1]) + (sg[2] + sg[3]));
+            if (hf == 0) redB[wave][i] = b1, redG[wave][i] = in ? g1 : 0.f;
+            if (in) put16(out, ov, hf, wide);
+        }
     }
     __syncthreads();  // Z is done with
     {  // Y = dR R^T
@@ -633,27 +719,37 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
     }
     __syncthreads();
     f32x16 dn = zero16();
-    if (wave != 1) {  // dN = -R^T Y
-        for (int kb = 32 * ti; kb < GC; kb += 8)
+    auto dn_rows = [&](int k0) {
+#pragma unroll
+        for (int kb = k0; kb < k0 + 32; kb += 8)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = kb + 4 * hf + j;
                 dn = mfma2(M2[i][32 * ti + ln], M3[i][32 * tj + ln], dn);
             }
+    };
+    if (wave != 1) {  // dN = -R^T Y
+        if (ti == 0) dn_rows(0);
+        dn_rows(32);
     }
     __syncthreads();  // dR and Y are done with
     if (wave != 1) {
+        double gj = gd[j0];
+        asm volatile("" : "+v"(gj));  // (once more, and not kept in registers from above)
+        float* spare = &M1[ln][GC];  // (the rows' padding takes what is not below the diagonal)
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int i = 32 * ti + c_row(e, hf);
-            const float d = i > j0 ? -dn[e] : 0.f;
-            const float dl = be[i] * d, D = i > j0 ? exp_of(gd[i] - gd[j0]) : 0.f;
-            if (i > j0) M1[i][j0] = M1[j0][i] = dl * D;
-            else if (i == j0) M1[i][i] = 0.f;
+            const bool in = i > j0;
+            const float x = exp_of(gd[i] - gj), D = in ? x : 0.f, dl = be[i] * (in ? -dn[e] : 0.f), m = dl * D;
+            *(in ? &M1[i][j0] : spare) = m;
+            *(in ? &M1[j0][i] : spare) = m;
             M3[i][j0] = dqk[e];
             ME[i][j0] = fmaf(dl, lkk[e], e1[e]);
+            if (e % 4 == 3) __builtin_amdgcn_sched_barrier(0);
         }
     } else {
+        M1[lane][lane] = 0.f;
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
             const int i = c_row(e, hf);
@@ -661,113 +757,205 @@ __global__ __launch_bounds__(256, 2) void gdrc_bwd_kernel(int S, int NC, int Hqk
             ME[i][j0] = 0.f;
         }
     }
+    // the last large products' first operands, under way from here on
+    struct Late {
+        u32x4 o[2];
+        f32x4 u[2][2];
+        float s0[8], s1[8];
+    };
+    auto request_late = [&](Late& t, int kb) {
+#pragma unroll
+        for (int r = 0; r < 2; ++r) {
+            t.o[r] = held8(op, ldo, 32 * r + ln, cnt, kb + 8 * hf);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) t.u[r][c] = *reinterpret_cast<const f32x4*>(Up + (32 * r + ln) * GD + kb + 8 * hf + 4 * c);
+        }
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            t.s0[j] = blk[(kb + 8 * hf + j) * GD + col];
+            t.s1[j] = dS[(kb + 8 * hf + j) * GD + col];
+        }
+        in_order();
+    };
+    Late now, next;
+    request_late(now, 0);
     __syncthreads();
     // dQ = scale gam (dO S0), dK += Gp (U dS): contraction over the value rows, straight from memory as above
     f32x16 x[2] = {zero16(), zero16()};
     {
         f32x16 y[2] = {zero16(), zero16()};
         float sds = 0.f;
-        u32x2 ox[2];
-        f32x4 ur[2];
-        float s0[4], s1[4];
-        auto request = [&](int kb) {
+        auto work = [&](const Late& t) {
+            const u32x4 &o0 = t.o[0], &o1 = t.o[1];
 #pragma unroll
-            for (int r = 0; r < 2; ++r) {
-                ox[r] = row4(op, ldo, 32 * r + ln, cnt, kb + 4 * hf);
-                ur[r] = *reinterpret_cast<const f32x4*>(Up + (32 * r + ln) * GD + kb + 4 * hf);
-            }
+            for (int c = 0; c < 2; ++c) {
+                const f32x4 a0 = widen4(u32x2{o0[2 * c], o0[2 * c + 1]}), a1 = widen4(u32x2{o1[2 * c], o1[2 * c + 1]});
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                s0[j] = blk[(kb + 4 * hf + j) * GD + col];
-                s1[j] = dS[(kb + 4 * hf + j) * GD + col];
+                for (int j = 0; j < 4; ++j) {
+                    const float c0 = t.s0[4 * c + j], c1 = t.s1[4 * c + j];
+                    sds = fmaf(c0, c1, sds);
+                    x[0] = mfma2(c0, a0[j], x[0]);
+                    x[1] = mfma2(c0, a1[j], x[1]);
+                    y[0] = mfma2(c1, t.u[0][c][j], y[0]);
+                    y[1] = mfma2(c1, t.u[1][c][j], y[1]);
+                }
             }
         };
-        request(0);
-#pragma unroll 2
-        for (int kb = 0; kb < GD; kb += 8) {
-            const f32x4 a0 = widen4(ox[0]), a1 = widen4(ox[1]), u0 = ur[0], u1 = ur[1], c0 = {s0[0], s0[1], s0[2], s0[3]}, c1 = {s1[0], s1[1], s1[2], s1[3]};
-            if (kb + 8 < GD) request(kb + 8);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                sds = fmaf(c0[j], c1[j], sds);
-                x[0] = mfma2(a0[j], c0[j], x[0]);
-                x[1] = mfma2(a1[j], c0[j], x[1]);
-                y[0] = mfma2(u0[j], c1[j], y[0]);
-                y[1] = mfma2(u1[j], c1[j], y[1]);
-            }
+        for (int kb = 0; kb < GD - 32; kb += 32) {  // (no request behind a condition: where the paths meet, a wait is for either's)
+            request_late(next, kb + 16);
+            work(now);
+            request_late(now, kb + 32);
+            work(next);
         }
+        request_late(next, GD - 16);
+        work(now);
+        work(next);
 #pragma unroll
-        for (int r = 0; r < 2; ++r)
+        for (int r = 0; r < 2; ++r) {
+            const int i = 32 * r + ln;
+            const bool in = i < cnt;
+            const float ga = gam[i], gi = gp[i];
+            u32x2 q4[4], k4[4];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int i = 32 * r + c_row(e, hf);
-                const float qx = qscale * x[r][e];
-                const float sg = half_sum(qx * one(qp, ldqk, i, cnt, col)), sp = half_sum(y[r][e] * one(kp, ldqk, i, cnt, col));
-                if (ln == 0) {
-                    redG[wave][i] += sg;
-                    redP[wave][i] = sp;
-                }
-                x[r][e] = gam[i] * qx;
-                w[r][e] = fmaf(gp[i], y[r][e], w[r][e]);
+            for (int c = 0; c < 4; ++c) {
+                q4[c] = held4(qp, ldqk, i, cnt, 32 * wave + c_row(4 * c, hf));
+                k4[c] = held4(kp, ldqk, i, cnt, 32 * wave + c_row(4 * c, hf));
             }
+            float sg[4], sp[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const f32x4 qf = widen4(q4[c]), kf = widen4(k4[c]);
+                float pg[4], pp[4];
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const float qx = qscale * x[r][4 * c + j], yv = y[r][4 * c + j];
+                    pg[j] = qx * qf[j];
+                    pp[j] = yv * kf[j];
+                    x[r][4 * c + j] = ga * qx;
+                    w[r][4 * c + j] = fmaf(gi, yv, w[r][4 * c + j]);
+                }
+                sg[c] = (pg[0] + pg[1]) + (pg[2] + pg[3]);
+                sp[c] = (pp[0] + pp[1]) + (pp[2] + pp[3]);
+            }
+            const float g1 = both_halves((sg[0] + sg[1]) + (sg[2] + sg[3])), p1 = both_halves((sp[0] + sp[1]) + (sp[2] + sp[3]));
+            if (hf == 0) redG[wave][i] += in ? g1 : 0.f, redP[wave][i] = in ? p1 : 0.f;
+        }
         sds = half_sum(sds);
         sds += __shfl_xor(sds, 32, 64);
         if (lane == 0) dss[wave] = sds;
     }
     // dK += (dKK + dKK^T) K + dQK^T Q, dQ += dQK K
-#pragma unroll 2
-    for (int kb = 0; kb < GC; kb += 8) {
-        const f32x4 s0 = *reinterpret_cast<const f32x4*>(&M1[ln][kb + 4 * hf]), s1 = *reinterpret_cast<const f32x4*>(&M1[32 + ln][kb + 4 * hf]);
+    {
+        bf16_t kn[2][8], qn[2][8];
+        const int ld = (int)ldqk, first = 8 * hf * ld, last = (cnt - 1) * ld;
+        auto request = [&](int b16) {
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int t = kb + 4 * hf + j;
-            const float kf = one(kp, ldqk, t, cnt, col), qf = one(qp, ldqk, t, cnt, col);
-            w[0] = mfma2(s0[j], kf, w[0]);
-            w[1] = mfma2(s1[j], kf, w[1]);
-            w[0] = mfma2(M3[t][ln], qf, w[0]);
-            x[1] = mfma2(M3[32 + ln][t], kf, x[1]);
-            if (kb >= 32) w[1] = mfma2(M3[t][32 + ln], qf, w[1]);
-            else x[0] = mfma2(M3[ln][t], kf, x[0]);
+            for (int j = 0; j < 8; ++j) {
+                const unsigned at = 2u * (unsigned)(min(first + (16 * b16 + j) * ld, last) + col);
+                kn[b16 & 1][j] = *reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(kp) + at);
+                qn[b16 & 1][j] = *reinterpret_cast<const bf16_t*>(reinterpret_cast<const char*>(qp) + at);
+            }
+            in_order();
+        };
+        request(0);
+#pragma unroll
+        for (int b16 = 0; b16 < 4; ++b16) {
+            if (b16 < 3) request(b16 + 1);
+#pragma unroll
+            for (int c = 0; c < 2; ++c) {
+                const int k0 = 16 * b16 + 8 * hf + 4 * c;
+                const f32x4 s0 = *reinterpret_cast<const f32x4*>(&M1[ln][k0]), s1 = *reinterpret_cast<const f32x4*>(&M1[32 + ln][k0]);
+                const f32x2 x1a = *reinterpret_cast<const f32x2*>(&M3[32 + ln][k0]), x1b = *reinterpret_cast<const f32x2*>(&M3[32 + ln][k0 + 2]);
+                const f32x2 x0a = *reinterpret_cast<const f32x2*>(&M3[ln][k0]), x0b = *reinterpret_cast<const f32x2*>(&M3[ln][k0 + 2]);
+                const float x1[4] = {x1a[0], x1a[1], x1b[0], x1b[1]}, x0[4] = {x0a[0], x0a[1], x0b[0], x0b[1]};
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const bool in = k0 + j < cnt;
+                    const float kf = bf2f(in ? kn[b16 & 1][4 * c + j] : (bf16_t)0), qf = bf2f(in ? qn[b16 & 1][4 * c + j] : (bf16_t)0);
+                    w[0] = mfma2(kf, s0[j], w[0]);
+                    w[1] = mfma2(kf, s1[j], w[1]);
+                    w[0] = mfma2(qf, M3[k0 + j][ln], w[0]);
+                    x[1] = mfma2(kf, x1[j], x[1]);
+                    if (b16 >= 2) w[1] = mfma2(qf, M3[k0 + j][32 + ln], w[1]);
+                    else x[0] = mfma2(kf, x0[j], x[0]);
+                }
+            }
         }
     }
 #pragma unroll
-    for (int r = 0; r < 2; ++r)
+    for (int r = 0; r < 2; ++r) {
+        const int i = 32 * r + ln;
+        if (i >= cnt) continue;
+        f32x4 dx[4], dw[4];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) {
-            const int i = 32 * r + c_row(e, hf);
-            if (i >= cnt) continue;
-            if (pdq) {  // several value heads share a q / k head: per value head, summed afterwards
-                const int64_t at = (head * S + t0 + i) * GD + col;
-                pdq[at] = x[r][e];
-                pdk[at] = w[r][e];
-            } else {
-                dq[(tok0 + i) * ldqk + hq * GD + col] = f2bf(x[r][e]);
-                dk[(tok0 + i) * ldqk + hq * GD + col] = f2bf(w[r][e]);
-            }
+        for (int c = 0; c < 4; ++c) {
+            dx[c] = f32x4{x[r][4 * c], x[r][4 * c + 1], x[r][4 * c + 2], x[r][4 * c + 3]};
+            dw[c] = f32x4{w[r][4 * c], w[r][4 * c + 1], w[r][4 * c + 2], w[r][4 * c + 3]};
         }
-    // d(log alpha_t): every pair (i, j) with j < t <= i, what reaches token i >= t from the chunk's first state, what token j < t leaves in its last, and the state passing through
-    if (tid < GC) {
+        if (pdq) {  // several value heads share a q / k head: per value head, summed afterwards
+            const int64_t at = (head * S + t0 + i) * GD + 32 * wave;
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                *reinterpret_cast<f32x4*>(pdq + at + c_row(4 * c, hf)) = dx[c];
+                *reinterpret_cast<f32x4*>(pdk + at + c_row(4 * c, hf)) = dw[c];
+            }
+        } else {
+            put16(dq + (tok0 + i) * ldqk + hq * GD + 32 * wave, dx, hf, wide);
+            put16(dk + (tok0 + i) * ldqk + hq * GD + 32 * wave, dw, hf, wide);
+        }
+    }
+    // d(log alpha_t): every pair (i, j) with j < t <= i, what reaches token i >= t from the chunk's first state, what token j < t leaves in its last, and the state passing through.
+    // Row i's sums over the columns before each t by four lanes, then column t's over the rows from t on by one lane of each wave; all in fp64.
+    {
+        const int i = tid >> 2, c = 16 * (tid & 3);
+        float row[16];
+        double mine = 0.;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+            row[j] = ME[i][c + j];
+            mine += row[j];
+        }
         double run = 0.;
-        float row[GC];
 #pragma unroll
-        for (int j = 0; j < GC; ++j) row[j] = ME[tid][j];
+        for (int o = 1; o < 4; ++o) {
+            const double v = __shfl_up(mine, o, 4);
+            if ((tid & 3) >= o) run += v;
+        }
 #pragma unroll
-        for (int j = 0; j < GC; ++j) {
-            const float c = row[j];
-            ME[tid][j] = (float)run;  // sum over the columns before j
-            run += c;
+        for (int j = 0; j < 16; ++j) {
+            ME[i][c + j] = (float)run;
+            run += row[j];
         }
     }
     __syncthreads();
-    if (tid < cnt) {
-        const int t = tid;
-        double s = gam[GC - 1] * ((dss[0] + dss[1]) + (dss[2] + dss[3]));
-        for (int i = 0; i < GC; ++i) {
-            if (i >= t) s += ME[i][t] + gam[i] * ((redG[0][i] + redG[1][i]) + (redG[2][i] + redG[3][i]));
-            else s += gp[i] * ((redP[0][i] + redP[1][i]) + (redP[2][i] + redP[3][i]));
+    {
+        double s = 0.;
+#pragma unroll
+        for (int o = 0; o < 16; ++o) {
+            const int i = 16 * wave + o;
+            const float m = ME[i][lane];
+            s += i >= lane ? m : 0.f;
         }
-        dalpha[(tok0 + t) * Hv + h] = (float)s / al[t];
-        dbeta[(tok0 + t) * Hv + h] = ((redB[0][t] + redB[1][t]) + (redB[2][t] + redB[3][t])) / be[t];
+        pairs[wave][lane] = s;
+    }
+    __syncthreads();
+    if (wave == 0) {
+        const int t = lane;
+        double from = gam[t] * ((redG[0][t] + redG[1][t]) + (redG[2][t] + redG[3][t]));  // summed over the tokens from t on
+        const double leaves = gp[t] * ((redP[0][t] + redP[1][t]) + (redP[2][t] + redP[3][t]));
+        double left = leaves;  // summed over the tokens up to t
+#pragma unroll
+        for (int o = 1; o < GC; o <<= 1) {
+            const double f = __shfl_down(from, o, 64), l = __shfl_up(left, o, 64);
+            if (t + o < GC) from += f;
+            if (t >= o) left += l;
+        }
+        const double before = __shfl_up(left, 1, 64);
+        const double s = (double)(gam[GC - 1] * ((dss[0] + dss[1]) + (dss[2] + dss[3]))) + ((pairs[0][t] + pairs[1][t]) + (pairs[2][t] + pairs[3][t])) + from + (t ? before : 0.);
+        if (t < cnt) {
+            dalpha[(tok0 + t) * Hv + h] = (float)s / al[t];
+            dbeta[(tok0 + t) * Hv + h] = ((redB[0][t] + redB[1][t]) + (redB[2][t] + redB[3][t])) / be[t];
+        }
     }
 }
 
@@ -853,7 +1041,7 @@ extern "C" int mi355_gdr_chunked_bwd(int B, int S, int Hqk, int Hv, const void* 
     gdrc_rscan_kernel<<<(B * Hv + 7) / 8 * 32, 256, 0, ST(stream)>>>(B * Hv, S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, saved, (const bf16_t*)d_o, ws, d_final_state, d_initial_state, qs);
     MI355_LAUNCH_CHECK("gdr_chunked_bwd(scan)");
     gdrc_bwd_kernel<<<dim3(NC, Hv, B), 256, 0, ST(stream)>>>(S, NC, Hqk, Hv, (const bf16_t*)q, (const bf16_t*)k, (const bf16_t*)v, ldv, beta, alpha, saved, ws, (const bf16_t*)d_o, (bf16_t*)dq,
-                                                             (bf16_t*)dk, (bf16_t*)dv, lddv, dbeta, dalpha, pdq, pdk, qs);
+                                                             (bf16_t*)dk, (bf16_t*)dv, lddv, dbeta, dalpha, pdq, pdk, qs, (((uintptr_t)dq | (uintptr_t)dk | (uintptr_t)dv) & 7) == 0 && lddv % 4 == 0);
     MI355_LAUNCH_CHECK("gdr_chunked_bwd");
     if (pdq) {
         const int64_t total = (int64_t)B * S * Hqk * GD;
