@@ -2090,6 +2090,15 @@ int choose_ksplit(int64_t tiles, int64_t slots, int64_t K, int64_t M, int64_t N,
     return ks < 2 ? 1 : (int)ks;
 }
 
+void launch_splitk_reduce(const GemmParams& p, int out_dtype, hipStream_t s) {
+    const int64_t work = p.M * (p.N >> 2);
+    const int rgrid = (int)((work + 255) / 256 > 2048 ? 2048 : (work + 255) / 256);
+    if (out_dtype == MI355_DT_BF16)
+        hipLaunchKernelGGL(splitk_reduce_kernel<MI355_DT_BF16>, dim3(rgrid), dim3(256), 0, s, p.M, p.N, p.ksplit, p.ws, p.C, p.ldc, p.R, p.ldr);
+    else
+        hipLaunchKernelGGL(splitk_reduce_kernel<MI355_DT_F32>, dim3(rgrid), dim3(256), 0, s, p.M, p.N, p.ksplit, p.ws, p.C, p.ldc, p.R, p.ldr);
+}
+
 template <class T, bool A_TR, bool B_TR>
 int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes, hipStream_t s) {
     p.tiles_m = (int)((p.M + T::BM - 1) / T::BM);
@@ -2103,12 +2112,7 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
     const int grid = (int)(tiles * p.ksplit);
     if (p.ksplit > 1) {
         hipLaunchKernelGGL((gemm_bf16_kernel<T, A_TR, B_TR, MI355_DT_F32>), dim3(grid), dim3(T::NTHREADS), 0, s, p);
-        const int64_t work = p.M * (p.N >> 2);
-        const int rgrid = (int)((work + 255) / 256 > 2048 ? 2048 : (work + 255) / 256);
-        if (out_dtype == MI355_DT_BF16)
-            hipLaunchKernelGGL(splitk_reduce_kernel<MI355_DT_BF16>, dim3(rgrid), dim3(256), 0, s, p.M, p.N, p.ksplit, p.ws, p.C, p.ldc, p.R, p.ldr);
-        else
-            hipLaunchKernelGGL(splitk_reduce_kernel<MI355_DT_F32>, dim3(rgrid), dim3(256), 0, s, p.M, p.N, p.ksplit, p.ws, p.C, p.ldc, p.R, p.ldr);
+        launch_splitk_reduce(p, out_dtype, s);
         MI355_LAUNCH_CHECK("mi355_gemm_bf16(split-K)");
         return 0;
     }
@@ -2117,6 +2121,181 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
     else
         hipLaunchKernelGGL((gemm_bf16_kernel<T, A_TR, B_TR, MI355_DT_F32>), dim3(grid), dim3(T::NTHREADS), 0, s, p);
     MI355_LAUNCH_CHECK("mi355_gemm_bf16");
+    return 0;
+}
+
+// ---------------------------------------------------------------------------------------------- mid-size NT products: one workgroup per CU, a ring of four K-tiles
+// Products of too few 256x256 tiles (under half of the CUs) used to run on Cfg128, whose workgroups only reach the matrix pipe's rate in pairs: alone on a CU a K-tile of 64 took
+// 0.75 us, in pairs 1.05 us for both -- each wave waits for its own LDS reads and its own DMA, one K-tile ahead.  Here ONE workgroup of four waves has the CU and all of its LDS: four
+// K-tiles of the BM x 128 output tile, three in flight while one is multiplied, one barrier a K-tile; the fragments of the next half K-tile are read between the products of this one
+// (two register sets), the requests issued there too.  BM = 192 (96 x 64 a wave): 5 664 x 1 024 is 240 tiles, one round of the 256 CUs, where 128 x 128 gave 360 for 2 x 256 places, and LDS and L2 carry a sixth fewer
+// bytes a flop.  What bounds it: the panels' way from L2 to LDS, 13 TB/s over the chip at 0.64 us (BM 128) and 0.76 us (BM 192) a K-tile with
+// every CU at work; alone on the chip a workgroup takes 0.44 and 0.6, its LDS reads and writes 0.4.
+// (The ring is dynamic LDS: told its size, the compiler gives the one wave per SIMD all 512 registers, half of them accumulation registers, and moves the sums back and forth -- 1.4 times
+// the time.)
+// NT form, plain epilogue (bias and residual allowed).  The same bits as gemm_bf16_kernel: every output is summed over K in the same order.
+template <int BM, int OUT_DT>
+__global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
+    constexpr int BN = 128, NS = 4, FM = BM / 32, FN = 4;
+    constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, A_PPW = A_BYTES / 4096, B_PPW = 4, PPW = A_PPW + B_PPW, STG_LD = 68;
+    static_assert(A_BYTES % 4096 == 0 && (NS - 1) * PPW <= 63 && FM >= 4, "pieces divide over four waves; the vmcnt field is 6 bits; reads are dealt over four rows of products");
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int nwg = p.tiles_m * p.tiles_n;
+    const int split = blockIdx.x / nwg;
+    const int pid = xcd_chunked(blockIdx.x - split * nwg, nwg);
+    const int in_group = 6 * p.tiles_n, first_m = (pid / in_group) * 6, gsz = min(p.tiles_m - first_m, 6);  // six row panels under every column panel, as in gemm_tile
+    const int64_t m0 = (int64_t)(first_m + (pid % in_group) % gsz) * BM, n0 = (int64_t)((pid % in_group) / gsz) * BN;
+    const int nt = (int)((p.K + 63) / 64);
+    const int t0 = (int)((int64_t)nt * split / p.ksplit), n = (int)((int64_t)nt * (split + 1) / p.ksplit) - t0;
+    const int kend = (int)min(p.K, (int64_t)(t0 + n) * 64);  // K < 2^30: lda >= K, and 256 rows span < 2 GiB
+
+    unsigned voffA[A_PPW], voffB[B_PPW];
+    int kneedA[A_PPW], kneedB[B_PPW];
+    piece_offsets<false, BM, 64, A_PPW>(wave, lane, p.lda, p.M - m0, voffA, kneedA);
+    piece_offsets<false, BN, 64, B_PPW>(wave, lane, p.ldb, p.N - n0, voffB, kneedB);
+    const bf16_t* baseA = uniform_ptr(p.A + m0 * p.lda);
+    const bf16_t* baseB = uniform_ptr(p.B + n0 * p.ldb);
+    auto issue = [&](int t, int from, int to) {  // this wave's pieces [from, to) of K-tile t; past the end out of range: zeros, and the counts of the waits below hold
+        const int k0 = t < n ? (t0 + t) * 64 : 0, krem = t < n ? kend - k0 : 0;
+        char* dA = smem + (t & (NS - 1)) * STAGE + wave * A_PPW * 1024;
+        char* dB = smem + (t & (NS - 1)) * STAGE + A_BYTES + wave * B_PPW * 1024;
+#pragma unroll
+        for (int j = 0; j < PPW; ++j) {
+            if (j < from || j >= to) continue;
+            if (j < A_PPW) dma_piece(baseA + k0, kneedA[j < A_PPW ? j : 0] < krem ? voffA[j < A_PPW ? j : 0] : OOB, dA + j * 1024);
+            else dma_piece(baseB + k0, kneedB[j < A_PPW ? 0 : j - A_PPW] < krem ? voffB[j < A_PPW ? 0 : j - A_PPW] : OOB, dB + (j - A_PPW) * 1024);
+        }
+    };
+    const int wr0 = (wave >> 1) * (BM / 2), wc0 = (wave & 1) * 64;
+    // the swizzle of a row goes by its last four bits: one lane offset serves every fragment of a half (frag_rowk)
+    const int off0 = (lane & 15) * 128 + (swz_rowk<64>(lane >> 4, lane & 15) << 4), off1 = (lane & 15) * 128 + (swz_rowk<64>(4 + (lane >> 4), lane & 15) << 4);
+    auto frag_a = [&](int t, int off, int i) { return *reinterpret_cast<const bf16x8*>(smem + (t & (NS - 1)) * STAGE + wr0 * 128 + off + i * 2048); };
+    auto frag_b = [&](int t, int off, int j) { return *reinterpret_cast<const bf16x8*>(smem + (t & (NS - 1)) * STAGE + A_BYTES + wc0 * 128 + off + j * 2048); };
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; ++i)
+#pragma unroll
+        for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    // products of one half K-tile; the reads of the next half (of K-tile t) and the requests for K-tile `next` stand between their rows, in this order: left to itself the compiler puts
+    // the reads behind all products, where nothing covers them, and ten requests in a row hold the one wave of a SIMD up (the second half's requests in front of its products: 5 % more)
+    auto half = [&](const bf16x8 (&a)[FM], const bf16x8 (&b)[FN], int t, int off, bf16x8 (&an)[FM], bf16x8 (&bn)[FN], int next) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            if (i < 2) bn[2 * i] = frag_b(t, off, 2 * i), bn[2 * i + 1] = frag_b(t, off, 2 * i + 1);
+            else if (2 * i - 4 < FM) an[2 * i - 4] = frag_a(t, off, 2 * i - 4), an[2 * i - 3] = frag_a(t, off, 2 * i - 3);
+            if (i == FM - 1 && 2 * i - 2 < FM) an[FM - 2] = frag_a(t, off, FM - 2), an[FM - 1] = frag_a(t, off, FM - 1);
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);  // lane: four columns of row lane & 15
+            if (next >= 0) issue(next, i * PPW / FM, (i + 1) * PPW / FM);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    bf16x8 a0[FM], b0[FN], a1[FM], b1[FN];
+#pragma unroll
+    for (int t = 0; t < NS; ++t) issue(t, 0, PPW);
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * PPW) : "memory");
+    __builtin_amdgcn_s_barrier();
+#pragma unroll
+    for (int j = 0; j < FN; ++j) b0[j] = frag_b(0, off0, j);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) a0[i] = frag_a(0, off0, i);
+    for (int t = 0; t < n; ++t) {
+        __builtin_amdgcn_sched_barrier(0);
+        half(a0, b0, t, off1, a1, b1, -1);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                    // this wave's reads of K-tile t are complete
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * PPW) : "memory");  // its pieces of t + 1 have landed
+        __builtin_amdgcn_s_barrier();                                         // ... and every wave's
+        __builtin_amdgcn_sched_barrier(0);
+        half(a1, b1, t + 1, off0, a0, b0, t + NS);                            // t + NS goes into the stage that t has left
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
+
+    // ---- 16 rows of the wave's 64 columns at a time through LDS, to leave as whole row segments
+    float* stg = reinterpret_cast<float*>(smem) + wave * 16 * STG_LD;
+    constexpr int VEC = OUT_DT == MI355_DT_BF16 ? 7 : 3;  // elements - 1 of 16 bytes
+    const bool vec_c = (p.ldc & VEC) == 0 && ((uintptr_t)p.C & 15) == 0, vec_r = p.R && (p.ldr & VEC) == 0 && ((uintptr_t)p.R & 15) == 0;
+    const int64_t gn = n0 + wc0 + (lane & 7) * 8, gm0 = m0 + wr0 + (lane >> 3);
+    const int cols = (int)min((int64_t)8, p.N - gn);
+#pragma unroll
+    for (int i = 0; i < FM; ++i) {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) *reinterpret_cast<f32x4*>(stg + (lane & 15) * STG_LD + j * 16 + (lane >> 4) * 4) = acc[i][j];
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const int64_t gm = gm0 + i * 16 + half * 8;
+            const f32x4 v0 = *reinterpret_cast<const f32x4*>(stg + ((lane >> 3) + half * 8) * STG_LD + (lane & 7) * 8);
+            const f32x4 v1 = *reinterpret_cast<const f32x4*>(stg + ((lane >> 3) + half * 8) * STG_LD + (lane & 7) * 8 + 4);
+            if (gm >= p.M || cols <= 0) continue;
+            if (OUT_DT == MI355_DT_F32 && p.ksplit > 1) {  // N % 8 == 0; residual and conversion: splitk_reduce_kernel
+                float* slab = p.ws + ((int64_t)split * p.M + gm) * p.N + gn;
+                *reinterpret_cast<f32x4*>(slab) = v0;
+                *reinterpret_cast<f32x4*>(slab + 4) = v1;
+                continue;
+            }
+            float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
+            if (p.bias) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e)
+                    if (e < cols) v[e] += p.bias[gn + e];
+            }
+            if constexpr (OUT_DT == MI355_DT_BF16) {
+                bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + gm * p.ldc + gn;
+                const bf16_t* r = reinterpret_cast<const bf16_t*>(p.R) + gm * p.ldr + gn;
+                if (vec_r && cols == 8) {
+                    const u32x4 rv = *reinterpret_cast<const u32x4*>(r);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) v[2 * e] += __uint_as_float(rv[e] << 16), v[2 * e + 1] += __uint_as_float(rv[e] & 0xffff0000u);
+                } else if (p.R) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e < cols) v[e] += bf2f(r[e]);
+                }
+                if (vec_c && cols == 8) {
+                    *reinterpret_cast<u32x4*>(c) = (u32x4){pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7])};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e < cols) c[e] = f2bf(v[e]);
+                }
+            } else {
+                float* c = reinterpret_cast<float*>(p.C) + gm * p.ldc + gn;
+                const float* r = reinterpret_cast<const float*>(p.R) + gm * p.ldr + gn;
+                if (p.R) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e < cols) v[e] += r[e];
+                }
+                if (vec_c && cols == 8) {
+                    *reinterpret_cast<f32x4*>(c) = (f32x4){v[0], v[1], v[2], v[3]};
+                    *reinterpret_cast<f32x4*>(c + 4) = (f32x4){v[4], v[5], v[6], v[7]};
+                } else {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e)
+                        if (e < cols) c[e] = v[e];
+                }
+            }
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <int BM>
+int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStream_t s) {
+    p.tiles_m = (int)((p.M + BM - 1) / BM);
+    p.tiles_n = (int)((p.N + 127) / 128);
+    p.ksplit = ksplit;
+    p.ws = (float*)workspace;
+    const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * ksplit));
+    constexpr int lds = 4 * (BM + 128) * 128;  // gemm_ring_kernel's NS stages
+    if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16>), grid, dim3(256), lds, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32>), grid, dim3(256), lds, s, p);
+    if (ksplit > 1) launch_splitk_reduce(p, out_dtype, s);
+    MI355_LAUNCH_CHECK("mi355_gemm_bf16(ring)");
     return 0;
 }
 
@@ -2245,6 +2424,13 @@ __global__ __launch_bounds__(256) void colsum_kernel(int64_t M, int64_t N, const
 GEMM_BRIDGE_DECL(1) GEMM_BRIDGE_DECL(2) GEMM_BRIDGE_DECL(3) GEMM_BRIDGE_DECL(4) GEMM_BRIDGE_DECL(5)
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_persist_part2(const void* params, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_pp_part6(const void* params, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_ring_part7(const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream);
+#if GEMM_PART == 7 || GEMM_PART == -1
+extern "C" int mi355_gemm_ring_part7(const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream) {
+    const GemmParams& p = *static_cast<const GemmParams*>(params);
+    return rows == 192 ? launch_ring<192>(p, out_dtype, ksplit, ws, (hipStream_t)stream) : launch_ring<128>(p, out_dtype, ksplit, ws, (hipStream_t)stream);
+}
+#endif
 #if GEMM_PART == 6 || GEMM_PART == -1
 extern "C" int mi355_gemm_pp_part6(const void* params, void* stream) { return launch_pp(*static_cast<const GemmParams*>(params), (hipStream_t)stream); }
 #endif
@@ -2315,6 +2501,28 @@ static int pp_mask() {
     return e && *e ? atoi(e) : MI355_GEMM_PP_DEFAULT;
 }
 
+// Tile rows (128 or 192; 0: none fits) and K shares of gemm_ring_kernel for a product of too few 256x256 tiles.  Only in ONE round of the 256 CUs: with more tiles Cfg128's two
+// workgroups per CU are the better filling (996 x 6144, K = 1024: 21 us, this kernel in two rounds 25).  The least of: the launch (3.5 us, 4.5 with 192 rows), its K-tiles (0.44 us each
+// where up to a quarter of the CUs work, 0.62 from half of them on; 192 rows 0.6 / 0.76), and for K shares -- from 32 K-tiles on, as in choose_ksplit -- the reduction's launch and bytes.
+// us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
+// 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
+// 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
+static int choose_ring(int64_t M, int64_t N, int64_t K, bool may_split, int64_t ws_bytes, int& ksplit) {
+    const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
+    if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
+    int rows = 0;
+    double least = 0;
+    for (int r = 128; r <= 192; r += 64) {
+        const int64_t tiles = (M + r - 1) / r * tn;
+        for (int64_t ks = 1; ks * tiles <= 256 && ks <= 16 && (ks == 1 || (may_split && nt >= 32 && ks * M * N * 4 <= ws_bytes)); ++ks) {
+            const double wgs = (double)(ks * tiles), busy = wgs <= 64 ? 0 : wgs >= 128 ? 1 : (wgs - 64) / 64;
+            const double t = (r == 192 ? 4.5 : 3.5) + (double)((nt + ks - 1) / ks) * (r == 192 ? 0.6 + 0.16 * busy : 0.44 + 0.18 * busy) + (ks > 1 ? 2.5 + (double)(ks * M * N) * 8 / 4.5e6 : 0);
+            if (!rows || t < least) least = t, rows = r, ksplit = (int)ks;
+        }
+    }
+    return rows;
+}
+
 extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* B,
                                int64_t ldb, void* C, int64_t ldc, int out_dtype, const float* bias,
                                const void* residual, int64_t ldr, int epilogue, void* workspace, int64_t workspace_bytes,
@@ -2376,7 +2584,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
                                 workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
         if (M < 256 || N < 256) cfg = 1;
         else if (long_split && tiles256 < 128) cfg = 3;
-        else if (form != MI355_GEMM_TN && tiles256 < 128) cfg = 1;  // measured: 92 tiles -> 128x128 wins (+2.8 % on the config-5 step), 180 tiles -> 256x256 wins
+        else if (form != MI355_GEMM_TN && tiles256 < 128 + (form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE)) cfg = 1;  // measured: 92 tiles -> 128x128 wins (+2.8 % on the config-5 step), 180 tiles -> 256x256 wins; 128 tiles, plain NT (2 000 x 4 096, K = 1024): 33 -> 15 us (gemm_ring_kernel)
         // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Round 4, batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)
         // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,
@@ -2408,7 +2616,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
             const int64_t esz = out_dtype == MI355_DT_F32 ? 4 : 2, rsz = epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_GELU_ERF ? esz : 2;
             if (int rc = mi355_gemm_bf16(form, m_main, N, K, A, lda, B, ldb, C, ldc, out_dtype, bias, residual, ldr, epilogue, workspace, workspace_bytes, 0, stream)) return rc;
             return mi355_gemm_bf16(form, M - m_main, N, K, (const bf16_t*)A + m_main * lda, lda, B, ldb, (char*)C + m_main * ldc * esz, ldc, out_dtype, bias,
-                                   residual ? (const char*)residual + m_main * ldr * rsz : nullptr, ldr, epilogue, workspace, workspace_bytes, 1, stream);
+                                   residual ? (const char*)residual + m_main * ldr * rsz : nullptr, ldr, epilogue, workspace, workspace_bytes, form == MI355_GEMM_NT ? 0 : 1, stream);
         }
     }
     if (cfg == 8) {  // ping-pong form: needs at least as many K-tiles as write-out slots
@@ -2419,6 +2627,11 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         const bool ok = persist_ok;
         if (ok) return mi355_gemm_persist_part2(&p, s);
         cfg = 2;
+    }
+    if (cfg == 1 && tile_hint == 0 && form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE && !split3 && ablate == 0) {
+        int ksplit = 1;
+        const bool may_split = workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
+        if (const int rows = choose_ring(M, N, K, may_split, workspace_bytes, ksplit)) return mi355_gemm_ring_part7(&p, out_dtype, rows, ksplit, workspace, s);
     }
     switch (cfg) {
         case 2: return mi355_gemm_part2(form, &p, out_dtype, workspace, workspace_bytes, s);

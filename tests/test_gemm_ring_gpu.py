@@ -1,0 +1,82 @@
+"""NT products of too few 256x256 tiles (one workgroup per CU, a ring of four K-tiles, row panels of 128 or 192): against 64 bits, and the bits of the 128x128 kernel (tile hint 1)."""
+
+import pytest
+import torch
+
+from llm_quest_amd import _lib as L
+
+pytestmark = pytest.mark.gpu
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+def product(A, B, odt, bias=None, residual=None, hint=0, ldc=None, ws=True):
+    M, N = A.shape[0], B.shape[0]
+    C = torch.full((M, ldc or N), 7.0, dtype=odt, device="cuda")
+    R = residual
+    buf = torch.empty(32 << 20, dtype=F32, device="cuda") if ws else None
+    L.require_gpu(A, B, C, bias, R, buf)
+    L.call("mi355_gemm_bf16", L.GEMM_NT, M, N, A.shape[1], A.data_ptr(), A.stride(0), B.data_ptr(), B.stride(0), C.data_ptr(), C.stride(0), L.dt_code(odt), L.ptr(bias), L.ptr(R),
+           R.stride(0) if R is not None else 0, 0, L.ptr(buf), buf.numel() * 4 if ws else 0, hint)
+    if ldc:
+        assert torch.equal(C[:, N:], torch.full_like(C[:, N:], 7.0))  # nothing beyond the matrix
+    return C[:, :N]
+
+
+def error_bound(A, B, extra):
+    """Largest error of one fp32 sum of K exact bf16 products: K rounding steps of the sum of magnitudes (any order), and of what is added to it."""
+    mag = A.double().abs() @ B.double().abs().t() + extra
+    return (A.shape[1] + 4) * 2.0 ** -24 * mag
+
+
+# one tile and parts of it; row panels of 128 and of 192 (5 100 x 1 024: 216 tiles of 192 rows, 320 of 128); the ring filled once, odd and even counts of K-tiles, a remainder in the last; K shares
+# (long K, few tiles); 192: the longest K that keeps to the 128x128 kernel
+SIZES = [(1, 8, 256), (9, 16, 200), (127, 128, 320), (129, 136, 192), (191, 264, 264), (300, 1000, 1016), (61, 1024, 3072), (333, 1024, 3584), (5100, 1024, 328), (2000, 4096, 256), (996, 768, 1992)]
+
+
+@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("odt", [BF16, F32])
+@pytest.mark.parametrize("bias,residual", [(False, False), (True, True), (False, True)])
+def test_against_64_bits(M, N, K, odt, bias, residual):
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K, generator=g, device="cuda").to(BF16)
+    B = torch.randn(N, K, generator=g, device="cuda").to(BF16)
+    b = torch.randn(N, generator=g, device="cuda") if bias else None
+    r = torch.randn(M, N, generator=g, device="cuda").to(odt) if residual else None
+    got = product(A, B, odt, b, r)
+    extra = (b.double() if bias else 0) + (r.double() if residual else 0)
+    exact = A.double() @ B.double().t() + extra
+    bound = error_bound(A, B, extra.abs() if bias or residual else 0)
+    if odt == BF16:
+        bound = bound + 2.0 ** -8 * exact.abs()  # one rounding to eight bits
+    assert ((got.double() - exact).abs() <= bound).all()
+    if K < 2048:  # without K shares: every sum in the same order
+        assert torch.equal(product(A, B, odt, b, r, hint=1), got)
+
+
+@pytest.mark.parametrize("odt", [BF16, F32])
+@pytest.mark.parametrize("N,ldc,lda,skip", [(130, 133, 0, 0), (136, 140, 8, 0), (100, 100, 24, 3), (1024, 1025, 8, 1)])
+def test_rows_that_are_not_aligned(N, ldc, lda, skip, odt):
+    """Output and residual rows at any element, operands with longer rows, columns that end inside eight; nothing is written outside."""
+    M, K = 150, 648
+    g = torch.Generator(device="cuda").manual_seed(N)
+    A = torch.randn(M, K + lda, generator=g, device="cuda").to(BF16)[:, :K]
+    B = torch.randn(N, K + lda, generator=g, device="cuda").to(BF16)[:, :K]
+    r = torch.randn(M, N + skip, generator=g, device="cuda").to(odt)[:, skip:]
+    got, exact = product(A, B, odt, residual=r, ldc=ldc), A.double() @ B.double().t() + r.double()
+    bound = error_bound(A, B, r.double().abs()) + (2.0 ** -8 * exact.abs() if odt == BF16 else 0)
+    assert ((got.double() - exact).abs() <= bound).all()
+
+
+@pytest.mark.parametrize("ws", [True, False])
+def test_values_that_are_not_finite_stay_in_their_row(ws):
+    A, B = torch.ones(200, 2048, device="cuda", dtype=BF16), torch.ones(256, 2048, device="cuda", dtype=BF16)
+    A[3, 5], A[150, 2047], B[100, 64] = float("nan"), float("inf"), float("inf")
+    got, want = product(A, B, F32, ws=ws), A.double() @ B.double().t()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isfinite(got)], want[torch.isfinite(want)].float())
+
+
+def test_same_bits_every_time():
+    A, B = torch.randn(700, 3072, device="cuda").to(BF16), torch.randn(1024, 3072, device="cuda").to(BF16)
+    first = product(A, B, BF16)
+    assert all(torch.equal(first, product(A, B, BF16)) for _ in range(3))
