@@ -470,6 +470,11 @@ int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, const void* 
                        const float* cos, const float* sin, const int32_t* pos, void* k_cache, void* v_cache, int64_t batch_stride, int64_t ld, int capacity,
                        const int32_t* write_pos, const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, const void* w_out, const void* norm2_w,
                        const void* w_gate_up, const void* w_down, float scale, float eps, int splits, void* scratch, int64_t scratch_bytes, void* out, void* stream);
+/* `layers` mi355_decode_block calls in a row, each on the rows that the one before it left: layer i's operands are table[13 i ..]: norm1_w, w_qkv, q_norm_w, k_norm_w, k_cache, v_cache, w_out,
+ * norm2_w, w_gate_up, w_down (addresses), batch_stride, ld, capacity; its result goes to rows_a (i even) or rows_b (odd).  rows_a is neither rows_b nor h (h may be rows_b); one scratch serves all. */
+int mi355_decode_blocks(int layers, const int64_t* table, int B, int d, int F, int Hq, int Hkv, int D, const void* h, const float* cos, const float* sin, const int32_t* pos,
+                        const int32_t* write_pos, const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, float scale, float eps, int splits, void* scratch, int64_t scratch_bytes,
+                        void* rows_a, void* rows_b, void* stream);
 /* The tail of a greedy step under hipGraph replay: tok[b] = next_ids[b], rope_pos[b] += 1, *write_pos += 1, *length += 1 (generate.py:139-148's
  * bookkeeping, kept on the device). */
 int mi355_decode_advance(int B, const int64_t* next_ids, int64_t* tok, int32_t* rope_pos, int32_t* write_pos, int32_t* length, void* stream);

@@ -888,6 +888,21 @@ extern "C" int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, c
     return mi355_gemv_bf16(B, d, F, act, la, w_down, F, out, d, h1, l1, stream);
 }
 
+extern "C" int mi355_decode_blocks(int layers, const int64_t* table, int B, int d, int F, int Hq, int Hkv, int D, const void* h, const float* cos, const float* sin, const int32_t* pos,
+                                   const int32_t* write_pos, const int32_t* len_dev, const uint8_t* key_mask, int64_t ldm, float scale, float eps, int splits, void* scratch,
+                                   int64_t scratch_bytes, void* rows_a, void* rows_b, void* stream) {
+    MI355_REQUIRE(layers >= 1 && table && rows_a && rows_b && rows_a != rows_b && h != rows_a, "decode_blocks: bad arguments");
+    for (int i = 0; i < layers; ++i, table += 13) {
+        void* out = i & 1 ? rows_b : rows_a;
+        const auto at = [&](int j) { return reinterpret_cast<void*>(static_cast<uintptr_t>(table[j])); };
+        MI355_REQUIRE(table[12] > 0 && table[12] <= 0x7fffffff, "decode_blocks: bad capacity");
+        if (int rc = mi355_decode_block(B, d, F, Hq, Hkv, D, h, at(0), at(1), at(2), at(3), cos, sin, pos, at(4), at(5), table[10], table[11], (int)table[12], write_pos, len_dev, key_mask, ldm,
+                                        at(6), at(7), at(8), at(9), scale, eps, splits, scratch, scratch_bytes, out, stream)) return rc;
+        h = out;
+    }
+    return 0;
+}
+
 extern "C" int mi355_decode_advance(int B, const int64_t* next_ids, int64_t* tok, int32_t* rope_pos, int32_t* write_pos, int32_t* length, void* stream) {
     MI355_REQUIRE(B > 0 && next_ids && tok && rope_pos && write_pos && length, "decode_advance: bad arguments");
     decode_advance_kernel<<<(B + 63) / 64, 64, 0, ST(stream)>>>(B, next_ids, tok, rope_pos, write_pos, length);

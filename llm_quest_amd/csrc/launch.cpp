@@ -21,7 +21,7 @@
     E(merge_patches) E(scatter_rows) E(zc_weight) E(mrope_table) E(rowmask) E(headnorm_rope_fwd) E(headnorm_rope_bwd) E(sigmoid_gate_fwd) E(sigmoid_gate_bwd) \
     E(attn_generic_fwd) E(attn_generic_bwd) E(gdn_gates_fwd) E(gdn_gates_bwd) E(causal_conv_silu_fwd) E(causal_conv_silu_bwd) E(l2norm_fwd) E(l2norm_bwd) \
     E(gated_delta_rule_fwd) E(causal_conv_silu_step) E(gated_delta_rule_bwd) E(gdr_chunked_fwd) E(gdr_chunked_bwd) E(gated_rmsnorm_fwd) E(gated_rmsnorm_bwd) \
-    E(resize_h_u8) E(resize_v_normalize) E(pad_tokens) E(gemv_bf16) E(gemv_bf16_f32out) E(gemv_bf16_pro) E(decode_block) E(attn_decode_qkv) E(decode_advance) \
+    E(resize_h_u8) E(resize_v_normalize) E(pad_tokens) E(gemv_bf16) E(gemv_bf16_f32out) E(gemv_bf16_pro) E(decode_block) E(decode_blocks) E(attn_decode_qkv) E(decode_advance) \
     E(attn_decode) E(kv_append_rows) E(kv_append) E(argmax_rows) E(argmax_rows_f32) E(embed_hash_fwd) E(add_layernorm_fwd) E(rmsnorm_rows) E(delta_rule_tokens) \
     E(delta_chunked) E(latent_kv_append) E(rope_heads) E(gated_headnorm) E(gla_fwd) E(gla_fwd_below) E(router_logits) E(moe_route) E(moe_dispatch) E(moe_table_dispatch) \
     E(bgemm) E(latent_attn) E(group_rmsnorm_sum) E(ragged_conv) E(qkv_rows_append) E(delta_rule_ragged) E(glu_rows) E(sandwich_rmsnorm) E(pool_rows_update) E(act_rows) \

@@ -8,6 +8,8 @@ Two shapes of call, both without autograd:
     batches fall back to the GEMM), attention is one query row per head over the cache (``mi355_attn_decode``).
 """
 
+from array import array
+
 import torch
 
 from . import _lib as L
@@ -291,6 +293,65 @@ def block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state=None, coun
 
 
 
+STEP_LAYERS = 4  # layers behind one native call: the device starts on a step when the first four's operands are gathered
+
+
+def _layer_operands(blk, i, like, d, F, B, kv_cache):
+    """The addresses of layer i in the order of ``mi355_decode_blocks`` (the caches': filled in when their rows are claimed); None where the layer is unlike ``like`` (heads, head dim,
+    scale) or one that ``_block_step`` leaves to the separate calls or has an error for."""
+    arena, m = blk.__dict__.get("_arena"), blk._modules
+    att = m.get("att")
+    if arena is None or att is None or (att.num_heads, att.num_kv_groups, att.head_dim, att.att_scaling, att.layer_idx) != (*like, i):
+        return None
+    arena.ensure()
+    try:  # the modules' own tables: attribute look-up through nn.Module costs a third of a microsecond each
+        a, f = att._modules, m["ffn"]._modules
+        weights = [x._parameters["weight"] for x in (m["norm1"], a["w_queries"], a["w_values"], a["q_norm"], a["k_norm"], a["out_proj"], m["norm2"], f["lin1"], f["lin_gate"], f["lin2"])]
+        n1, wq, wv, qn, kn, wo, n2, w1, wg, wd = weights
+        qkv, gu = arena.fused_ptr(wq, wv), arena.fused_ptr(w1, wg)
+    except (KeyError, AttributeError):  # parameters that are not plain ones of this block's arena
+        return None
+    kc, vc, (Hq, Hkv, D, _) = kv_cache.keys_cache[i], kv_cache.values_cache[i], like
+    if (arena.data.dtype != BF16 or wo.shape != (d, Hq * D) or wd.shape != (d, F) or w1.shape[0] != F or kc.dtype != BF16 or kc.shape != vc.shape or kc.shape[0] != B
+            or kc.shape[2] != Hkv * D or kc.stride() != vc.stride() or kc.stride(2) != 1):
+        return None
+    L.require_gpu(arena.data, kc, vc)
+    return [n1.data_ptr(), qkv, qn.data_ptr(), kn.data_ptr(), 0, 0, wo.data_ptr(), n2.data_ptr(), gu, wd.data_ptr(), 0, 0, 0]
+
+
+def _step_layers(blocks, h, B, cos, sin, pos, km, kv_cache, dev_state, counters, scratch):
+    """The layers of a one-token step, up to ``STEP_LAYERS`` to a native call (``mi355_decode_blocks``): ``_block_step``'s launches in its order, the same bits; layers that it does not take go
+    through ``block_cached``.  A layer cost the host 38 us in a call of its own -- 18 the five launches, the rest 13 modules and parameters looked up and checked -- where one row's kernels take 26.
+    580-token prompt and 16 tokens 20.1 -> 16.1 ms, six 61-token prompts and 24 tokens 29.2 -> 25.0."""
+    att, d, F = blocks[0].att, h.shape[1], blocks[0].ffn.lin1.weight.shape[0]
+    like = Hq, Hkv, D, scale = att.num_heads, att.num_kv_groups, att.head_dim, att.att_scaling
+    start = kv_cache.start_pos
+    write_pos, len_dev, *more = counters if dev_state is None else dev_state[1:]
+    splits = step_splits(start + 1, B, Hq) if dev_state is None else more[0] if more else 1
+    ok = ((D == 64 or D == 128) and len(kv_cache.keys_cache) == len(blocks) and fused_rows(B, max(d, F)) and h.dtype == BF16 and h.is_contiguous() and cos.dtype == sin.dtype == torch.float32
+          and pos.dtype == write_pos.dtype == len_dev.dtype == torch.int32 and pos.numel() == B and (km is None or (km.dtype == torch.uint8 and km.shape[0] == B and km.stride(1) == 1)))
+    rows, table, n = [torch.empty_like(h), torch.empty_like(h)], array("q"), 0  # a call starts on rows[0]; its input is rows[1] or the caller's
+    for i, blk in enumerate(blocks):
+        layer = _layer_operands(blk, i, like, d, F, B, kv_cache) if ok else None
+        if layer is not None and km is not None and km.shape[1] < (start + 1 if dev_state is None else kv_cache.keys_cache[i].shape[1]):
+            layer = None
+        if layer is not None:
+            kc, vc, end = kv_cache.claim_rows(i, 1) if dev_state is None else (kv_cache.keys_cache[i], kv_cache.values_cache[i], kv_cache.keys_cache[i].shape[1])
+            layer[4], layer[5], (layer[10], layer[11], _), layer[12] = kc.data_ptr(), vc.data_ptr(), kc.stride(), end
+            table.extend(layer)
+            n += 1
+        if n and (layer is None or n == STEP_LAYERS or i + 1 == len(blocks)):
+            L.require_gpu(h, cos, sin, pos, write_pos, len_dev, km)
+            L.call("mi355_decode_blocks", n, table.buffer_info()[0], B, d, F, Hq, Hkv, D, h.data_ptr(), cos.data_ptr(), sin.data_ptr(), pos.data_ptr(), write_pos.data_ptr(), len_dev.data_ptr(),
+                   L.ptr(km), 0 if km is None else km.stride(0), scale, 1e-6, splits, scratch.data_ptr(), scratch.numel(), rows[0].data_ptr(), rows[1].data_ptr())
+            if n & 1:
+                rows.reverse()
+            h, table, n = rows[1], array("q"), 0
+        if layer is None:
+            h = block_cached(blk, h, B, 1, cos, sin, pos, km, kv_cache, dev_state, counters, scratch)
+    return h
+
+
 @torch.no_grad()
 def qwen3_forward_cached(model, x, kv_cache, attn_mask=None, position_ids=None, input_embedded=False, dev_state=None):
     """Logits (b, s, vocab) of ``Qwen3Model`` with ``kv_cache`` updated in place (reference: qwen3_model.py:60-94).
@@ -329,8 +390,11 @@ def qwen3_forward_cached(model, x, kv_cache, attn_mask=None, position_ids=None, 
     if decode and len(blocks) and B <= 8:
         heads = blocks[0].att.num_heads
         scratch = block_scratch(blocks[0], B, step_splits(start + 1, B, heads) if dev_state is None else dev_state[3] if len(dev_state) > 3 else 1, h.device)
-    for blk in blocks:
-        h = block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state, counters, scratch)
+    if scratch is not None:
+        h = _step_layers(blocks, h, B, cos, sin, pos, km, kv_cache, dev_state, counters, scratch)
+    else:
+        for blk in blocks:
+            h = block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state, counters, scratch)
     if decode and fused_rows(B * S, h.shape[1]):
         return gemv_pro(h, model.out_head.weight, "rmsnorm", model.final_norm.weight).view(B, S, -1)
     lin = _lin(decode)

@@ -72,3 +72,37 @@ def test_weight_streams_of_every_shape_of_launch(M, N, K):
     got = ops_decode.gemv(x, w, residual=r)
     # fp32 sums of K exact products, then one bf16 rounding: half a step of 2^-8, the sums' own error far below
     assert bool(((got.double() - ref).abs() <= ref.abs() * 2**-8 + K**0.5 * 1e-5).all())
+
+
+@pytest.mark.parametrize("B,layers,masked,device_side", [(1, 1, False, False), (1, 4, True, False), (3, 5, False, False), (8, 7, True, False), (9, 3, False, False), (2, 6, False, True), (1, 5, True, True)])
+def test_layers_behind_one_call_are_the_layers_one_by_one(monkeypatch, B, layers, masked, device_side):
+    """Even and odd counts of layers to a call, a cache that grows in the step, a layer in the middle that takes the separate calls; logits and caches the same bits."""
+    from llm_quest_amd import ops_decode as OD
+    from llm_quest_amd.qwen.qwen3.qwen3_model import Qwen3Model
+    from llm_quest_amd.utils import KVCache
+
+    torch.manual_seed(B + layers)
+    past = 5
+    with torch.device("cuda"):
+        m = Qwen3Model(dict(vocab_size=300, emb_dim=64, n_layers=layers, n_heads=4, num_kv_groups=2, hidden_dim=136, head_dim=64, rope_base=10_000, context_length=64, dtype=BF16, tie_embeddings=True,
+                            model_type="dense")).eval()
+    ids = torch.randint(0, 300, (B, past + 3), device="cuda")
+    km = (torch.rand(B, 1024, device="cuda") < 0.7) if masked else None
+    operands, outs = OD._layer_operands, []
+    for how in ("all", "all but the third", "none"):
+        monkeypatch.setattr(OD, "_layer_operands", lambda blk, i, *a: None if how == "none" or (how != "all" and i == 2) else operands(blk, i, *a))
+        c = KVCache(num_layers=layers, prompt_len=past, context_len=64)
+        with torch.inference_mode():
+            seen = [m(ids[:, :past], kv_cache=c, attn_mask=None if km is None else km[:, :past])]
+            if device_side:
+                c.reserve(past + 3)
+            for t in range(3):
+                at = lambda v: torch.tensor([v], dtype=torch.int32, device="cuda")
+                state = (at(past + t).repeat(B), at(past + t), at(past + t + 1), 1) if device_side else None
+                seen.append(OD.qwen3_forward_cached(m, ids[:, past + t : past + t + 1], c, attn_mask=km, dev_state=state))
+                if device_side:
+                    c.start_pos += 1
+        assert c.start_pos == past + 3
+        outs.append(seen + [x[:, : past + 3].clone() for x in c.keys_cache + c.values_cache])
+    for got in outs[:-1]:
+        assert all(torch.equal(a, b) for a, b in zip(got, outs[-1]))
