@@ -565,6 +565,16 @@ __device__ __forceinline__ void split_pair(float x0, float x1, unsigned& hi, uns
     mid = (m0 >> 16) | m1;
     lo = (__float_as_uint(s0) >> 16) | (__float_as_uint(s1) & 0xffff0000u);
 }
+// the same parts of finite numbers in 11 instructions instead of 25; a part of an infinity or NaN is NaN, and so is every sum it reaches: for kernels that sum those again (`settled`)
+__device__ __forceinline__ void split_finite(float x0, float x1, unsigned& hi, unsigned& mid, unsigned& lo) {
+    const unsigned u0 = __float_as_uint(x0), u1 = __float_as_uint(x1);
+    const float r0 = x0 - __uint_as_float(u0 & 0xffff0000u), r1 = x1 - __uint_as_float(u1 & 0xffff0000u);
+    const unsigned m0 = __float_as_uint(r0), m1 = __float_as_uint(r1);
+    const float s0 = r0 - __uint_as_float(m0 & 0xffff0000u), s1 = r1 - __uint_as_float(m1 & 0xffff0000u);
+    hi = __builtin_amdgcn_perm(u1, u0, 0x07060302u);  // the upper halves side by side
+    mid = __builtin_amdgcn_perm(m1, m0, 0x07060302u);
+    lo = __builtin_amdgcn_perm(__float_as_uint(s1), __float_as_uint(s0), 0x07060302u);
+}
 __device__ __forceinline__ Split8 split8(const f32x4 a, const f32x4 b) {
     Split8 r;
     unsigned h, m, l;
@@ -584,14 +594,18 @@ __device__ __forceinline__ float settled(const BgemmArgs& p, float v, int b, int
     return v;
 }
 
-// Tile of 64 WM rows x 128 columns, four waves of 32 WM x 64 (2 x 2): k in steps of 32 through one LDS stage (A as three bf16 planes, split once per tile), the next
-// step's operands on their way in registers.  VALU (the split) and matrix pipe are level at WM = 1; WM = 2 halves the split's and B's share where there are rows for it.
+// Tile of 64 WM rows x 128 columns, four waves of 32 WM x 64 (2 x 2): k in steps of 32 through two LDS stages that take turns (A as three bf16 planes, split once per tile), one barrier a
+// step, operands requested DEPTH steps ahead into registers.  VALU (the split) and matrix pipe are level at WM = 1; WM = 2 halves the split's and B's share where there are rows for it.
+// With one stage and requests one step ahead a step was the weights' way from memory: 1.1 - 1.5 us, its products 0.16.  450 fp32 rows, us, before -> now: 2048 -> 1024 74 -> 49, 1024 -> 8256 86 -> 49; 3 000 rows
+// 1024 -> 4096 218 -> 115; 900 rows over 16 experts 1792 -> 1024 83 -> 62.  The split in front of the last step's products instead of behind them: experts 42 / 57, but 204 registers leave two
+// workgroups to a CU (1024 -> 8256: 60); interleaved with the products it spills; eight steps ahead too.
 #define FK 32
 template <int WM>
-__global__ __launch_bounds__(256) void bgemm_f32_tile_kernel(BgemmArgs p) {
+__global__ __launch_bounds__(256, 2) void bgemm_f32_tile_kernel(BgemmArgs p) {
     constexpr int R = 64 * WM, AP = R / 32;  // A: 8 threads per row of 32 fp32, 32 rows per pass; B: 4 threads per row of 32 bf16, 64 rows per pass
-    __shared__ __attribute__((aligned(16))) bf16_t As[3][R][FK + MPAD];
-    __shared__ __attribute__((aligned(16))) bf16_t Bs[128][FK + MPAD];
+    constexpr int DEPTH = WM == 1 ? 4 : 2;   // (sums and running sums of WM = 2 take 128 registers)
+    __shared__ __attribute__((aligned(16))) bf16_t As[2][3][R][FK + MPAD];
+    __shared__ __attribute__((aligned(16))) bf16_t Bs[2][128][FK + MPAD];
     const int b = blockIdx.z;
     int row0 = 0, rows = p.M;
     if (p.grp_offs) {
@@ -601,26 +615,25 @@ __global__ __launch_bounds__(256) void bgemm_f32_tile_kernel(BgemmArgs p) {
     const int m0 = blockIdx.y * R, n0 = blockIdx.x * 128;
     if (m0 >= rows) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
-    const float* a_row[AP];
+    const float* a_row[AP];  // rows and columns beyond the end: the last one again, their results are not stored
     const int ar = tid >> 3, ak = (tid & 7) * 4, br = tid >> 2, bk = (tid & 3) * 8;
 #pragma unroll
     for (int i = 0; i < AP; ++i) {
-        a_row[i] = nullptr;
-        if (m0 + ar + 32 * i < rows) {
-            const int r = row0 + m0 + ar + 32 * i;
-            a_row[i] = (const float*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
-        }
+        const int r = row0 + min(m0 + ar + 32 * i, rows - 1);
+        a_row[i] = (const float*)p.A + (int64_t)b * p.a_bs + (int64_t)(p.a_rows ? p.a_rows[r] / p.a_div : r) * p.lda;
     }
     const bf16_t* b_row[2];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) b_row[i] = n0 + br + 64 * i < p.N ? (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)(n0 + br + 64 * i) * p.sbn : nullptr;
-    f32x4 ra[AP];
-    u32x4 rb[2];
-    auto fetch = [&](int k0) {  // K is a multiple of 8: a 16-byte word lies inside or outside as a whole
+    for (int i = 0; i < 2; ++i) b_row[i] = (const bf16_t*)p.B + (int64_t)b * p.b_bs + (int64_t)min(n0 + br + 64 * i, p.N - 1) * p.sbn;
+    f32x4 ra[DEPTH][AP];
+    u32x4 rb[DEPTH][2];
+    auto fetch = [&](f32x4 (&x)[AP], u32x4 (&w)[2], int k0) {  // K is a multiple of 8: a 16-byte word lies inside or outside as a whole; outside: the row's first one, replaced by zeros below
+        int ka = k0 + ak, kb = k0 + bk;
+        if (k0 + FK > p.K) ka = ka < p.K ? ka : 0, kb = kb < p.K ? kb : 0;
 #pragma unroll
-        for (int i = 0; i < AP; ++i) ra[i] = a_row[i] && k0 + ak < p.K ? *(const f32x4*)(a_row[i] + k0 + ak) : (f32x4){0.f, 0.f, 0.f, 0.f};
+        for (int i = 0; i < AP; ++i) x[i] = *(const f32x4*)(a_row[i] + ka);
 #pragma unroll
-        for (int i = 0; i < 2; ++i) rb[i] = b_row[i] && k0 + bk < p.K ? *(const u32x4*)(b_row[i] + k0 + bk) : (u32x4){0u, 0u, 0u, 0u};
+        for (int i = 0; i < 2; ++i) w[i] = *(const u32x4*)(b_row[i] + kb);
     };
     f32x16 acc[WM][2], tot[WM][2];
 #pragma unroll
@@ -632,51 +645,69 @@ __global__ __launch_bounds__(256) void bgemm_f32_tile_kernel(BgemmArgs p) {
     const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW;
     int left = per;
     const int wm = (wave >> 1) * 32 * WM, wn = (wave & 1) * 64;
-    fetch(0);
-    for (int k0 = 0; k0 < p.K; k0 += FK) {
-        __syncthreads();  // the previous step's fragments are read
+    auto stage = [&](f32x4 (&x)[AP], u32x4 (&w)[2], int k0, int st) {
+        if (k0 + FK > p.K) {
+            if (k0 + ak >= p.K)
+#pragma unroll
+                for (int i = 0; i < AP; ++i) x[i] = (f32x4){0.f, 0.f, 0.f, 0.f};
+            if (k0 + bk >= p.K) w[0] = w[1] = (u32x4){0u, 0u, 0u, 0u};
+        }
 #pragma unroll
         for (int i = 0; i < AP; ++i) {
             u32x2 h, m, l;
-            unsigned x, y, z;
-            split_pair(ra[i][0], ra[i][1], x, y, z); h[0] = x; m[0] = y; l[0] = z;
-            split_pair(ra[i][2], ra[i][3], x, y, z); h[1] = x; m[1] = y; l[1] = z;
-            *(u32x2*)&As[0][ar + 32 * i][ak] = h;
-            *(u32x2*)&As[1][ar + 32 * i][ak] = m;
-            *(u32x2*)&As[2][ar + 32 * i][ak] = l;
+            unsigned hi, mid, lo;
+            split_finite(x[i][0], x[i][1], hi, mid, lo); h[0] = hi; m[0] = mid; l[0] = lo;
+            split_finite(x[i][2], x[i][3], hi, mid, lo); h[1] = hi; m[1] = mid; l[1] = lo;
+            *(u32x2*)&As[st][0][ar + 32 * i][ak] = h;
+            *(u32x2*)&As[st][1][ar + 32 * i][ak] = m;
+            *(u32x2*)&As[st][2][ar + 32 * i][ak] = l;
         }
 #pragma unroll
-        for (int i = 0; i < 2; ++i) *(u32x4*)&Bs[br + 64 * i][bk] = rb[i];
-        __syncthreads();
-        if (k0 + FK < p.K) fetch(k0 + FK);
+        for (int i = 0; i < 2; ++i) *(u32x4*)&Bs[st][br + 64 * i][bk] = w[i];
+    };
+    auto step = [&](f32x4 (&x)[AP], u32x4 (&w)[2], int k0, int st) {
+        stage(x, w, k0, st);
+        __builtin_amdgcn_sched_barrier(0);
+        fetch(x, w, k0 + DEPTH * FK);
+        // this wave's rows of the step are written, and its reads of the stage (two steps ago) are done -- behind the barrier everyone's; requests stay under way
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int kk = 0; kk < FK; kk += 16) {
-            if (k0 + kk >= p.K) break;
-            bf16x8 bf[2];
+            if (k0 + kk < p.K) {
+                bf16x8 bf[2];
 #pragma unroll
-            for (int j = 0; j < 2; ++j) bf[j] = *(const bf16x8*)&Bs[wn + 32 * j + ln][kk + 8 * hf];
+                for (int j = 0; j < 2; ++j) bf[j] = *(const bf16x8*)&Bs[st][wn + 32 * j + ln][kk + 8 * hf];
 #pragma unroll
-            for (int s = 2; s >= 0; --s)
+                for (int s = 2; s >= 0; --s)
 #pragma unroll
-                for (int i = 0; i < WM; ++i) {
-                    const bf16x8 af = *(const bf16x8*)&As[s][wm + 32 * i + ln][kk + 8 * hf];
+                    for (int i = 0; i < WM; ++i) {
+                        const bf16x8 af = *(const bf16x8*)&As[st][s][wm + 32 * i + ln][kk + 8 * hf];
 #pragma unroll
-                    for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf[j], acc[i][j], 0, 0, 0);
+                        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf[j], acc[i][j], 0, 0, 0);
+                    }
+                if (--left == 0) {
+                    left = per;
+#pragma unroll
+                    for (int i = 0; i < WM; ++i)
+#pragma unroll
+                        for (int j = 0; j < 2; ++j)
+#pragma unroll
+                            for (int e = 0; e < 16; ++e) {
+                                tot[i][j][e] += acc[i][j][e];
+                                acc[i][j][e] = 0.f;
+                            }
                 }
-            if (--left == 0) {
-                left = per;
-#pragma unroll
-                for (int i = 0; i < WM; ++i)
-#pragma unroll
-                    for (int j = 0; j < 2; ++j)
-#pragma unroll
-                        for (int e = 0; e < 16; ++e) {
-                            tot[i][j][e] += acc[i][j][e];
-                            acc[i][j][e] = 0.f;
-                        }
             }
         }
-    }
+    };
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) fetch(ra[d], rb[d], d * FK);
+    for (int k0 = 0; k0 < p.K; k0 += DEPTH * FK)  // (steps past K: zeros written, nothing multiplied)
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) step(ra[d], rb[d], k0 + d * FK, d & 1);
     if (left != per) {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
