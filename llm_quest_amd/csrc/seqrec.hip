@@ -282,6 +282,62 @@ __global__ __launch_bounds__(256) void ragged_conv_vec_kernel(int C, int taps, c
     st4_dt(y, y_dt, t * ldy + c, acc);
 }
 
+// The same for long steps: eight packed rows and four channels to a thread.  A row at a time every thread fetched its 16 x TAPS bytes of weights and each row came TAPS times: 1.9 TB/s.  Here the
+// weights come once, the rows all at once, and the window slides in registers; where a sequence ends inside the eight, the next one's window comes from its state.  The sums are
+// ragged_conv_vec_kernel's, in its order.  5 400 fp32 rows, four taps, us with the state's launch, before -> now: 6 144 channels 92 -> 55, 1 024 24 -> 18.
+constexpr int CONV_ROWS = 8;
+template <int TAPS>
+__global__ __launch_bounds__(256) void ragged_conv_rows_kernel(int tokens, int C, const void* __restrict__ x, int x_dt, int64_t ldx, const float* __restrict__ w,
+                                                               const int* __restrict__ row_seq, const int* __restrict__ seq_off, const int* __restrict__ slot,
+                                                               const float* __restrict__ state, int act, int residual, void* __restrict__ y, int y_dt, int64_t ldy,
+                                                               const float* __restrict__ bias) {
+    const int t0 = blockIdx.x * CONV_ROWS, c = 4 * (blockIdx.y * 256 + threadIdx.x);
+    if (c >= C) return;
+    f32x4 in[CONV_ROWS], window[TAPS - 1], b4 = {0.f, 0.f, 0.f, 0.f};
+    float wf[4 * TAPS];
+#pragma unroll
+    for (int r = 0; r < CONV_ROWS; ++r) in[r] = ld4_dt(x, x_dt, (int64_t)min(t0 + r, tokens - 1) * ldx + c);
+#pragma unroll
+    for (int i = 0; i < TAPS; ++i) {
+        const f32x4 wv = *(const f32x4*)(w + (int64_t)c * TAPS + 4 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) wf[4 * i + e] = wv[e];
+    }
+    if (bias) b4 = *(const f32x4*)(bias + c);
+    int end = t0;  // where the sequence of the row ends (t0: none yet)
+#pragma unroll
+    for (int r = 0; r < CONV_ROWS; ++r) {
+        const int t = t0 + r;
+        if (t >= tokens) return;
+        if (t == end) {  // another sequence (or the thread's first row): what came before the row
+            const int s = row_seq[t], start = seq_off[s];
+            const float* st = state + (int64_t)slot[s] * (TAPS - 1) * C;
+            end = seq_off[s + 1];
+#pragma unroll
+            for (int j = 0; j < TAPS - 1; ++j) {
+                const int sl = t - start - (TAPS - 1) + j;
+                window[j] = sl >= 0 ? ld4_dt(x, x_dt, (int64_t)(start + sl) * ldx + c) : *(const f32x4*)(st + (int64_t)(TAPS - 1 + sl) * C + c);
+            }
+        }
+        f32x4 acc = b4;
+#pragma unroll
+        for (int j = 0; j < TAPS; ++j) {
+            const f32x4 v = j < TAPS - 1 ? window[j < TAPS - 1 ? j : 0] : in[r];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = fmaf(wf[e * TAPS + j], v[e], acc[e]);
+        }
+        if (act == 1) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) acc[e] = acc[e] / (1.0f + expf(-acc[e]));
+        }
+        if (residual) acc += in[r];
+        st4_dt(y, y_dt, (int64_t)t * ldy + c, acc);
+#pragma unroll
+        for (int j = 0; j + 1 < TAPS - 1; ++j) window[j] = window[j + 1];
+        window[TAPS - 2] = in[r];
+    }
+}
+
 __global__ __launch_bounds__(256) void ragged_conv_state_kernel(int n_seq, int C, int taps, const void* __restrict__ x, int x_dt, int64_t ldx, const int* __restrict__ seq_off,
                                                                 const int* __restrict__ slot, float* __restrict__ state) {
     const int64_t total = (int64_t)n_seq * C;
@@ -311,10 +367,13 @@ extern "C" int mi355_ragged_conv(int64_t tokens, int n_seq, int C, int taps, con
     MI355_REQUIRE(rec_dt_ok(x_dt) && rec_dt_ok(y_dt) && ldx >= C && ldy >= C && (act == 0 || act == 1), "ragged_conv: bad operands");
     const int64_t total = tokens * C;
     if (C % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && al16(x) && al16(y) && al16(state) && al16(bias) && tokens < ((int64_t)1 << 31)) {
-        const dim3 grid((unsigned)tokens, (C / 4 + 255) / 256);
+        const dim3 grid((unsigned)tokens, (C / 4 + 255) / 256), rows_grid((unsigned)((tokens + CONV_ROWS - 1) / CONV_ROWS), grid.y);
+        // eight rows to a thread once that leaves two workgroups to a CU (700 x 6 144, 528 workgroups: 18.4 -> 15.9 us; 700 x 1 024, 88: level)
+        const bool rows = (int64_t)rows_grid.x * rows_grid.y >= 512;
 #define CONV_CASE(TP)                                                                                                                                          \
     case TP:                                                                                                                                                   \
-        ragged_conv_vec_kernel<TP><<<grid, 256, 0, ST(stream)>>>(C, taps, x, x_dt, ldx, w, row_seq, seq_off, slot, state, act, residual, y, y_dt, ldy, bias);      \
+        if (rows) ragged_conv_rows_kernel<TP><<<rows_grid, 256, 0, ST(stream)>>>((int)tokens, C, x, x_dt, ldx, w, row_seq, seq_off, slot, state, act, residual, y, y_dt, ldy, bias); \
+        else ragged_conv_vec_kernel<TP><<<grid, 256, 0, ST(stream)>>>(C, taps, x, x_dt, ldx, w, row_seq, seq_off, slot, state, act, residual, y, y_dt, ldy, bias);      \
         break;
         switch (al16(w) ? taps : 0) {
             CONV_CASE(2) CONV_CASE(3) CONV_CASE(4) CONV_CASE(5) CONV_CASE(6) CONV_CASE(7) CONV_CASE(8)
