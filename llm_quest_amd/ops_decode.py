@@ -296,7 +296,7 @@ def block_cached(blk, h, B, S, cos, sin, pos, km, kv_cache, dev_state=None, coun
 STEP_LAYERS = 4  # layers behind one native call: the device starts on a step when the first four's operands are gathered
 
 
-def _layer_operands(blk, i, like, d, F, B, kv_cache):
+def _layer_operands(blk, i, like, h, F, B, kv_cache):
     """The addresses of layer i in the order of ``mi355_decode_blocks`` (the caches': filled in when their rows are claimed); None where the layer is unlike ``like`` (heads, head dim,
     scale) or one that ``_block_step`` leaves to the separate calls or has an error for."""
     arena, m = blk.__dict__.get("_arena"), blk._modules
@@ -311,11 +311,11 @@ def _layer_operands(blk, i, like, d, F, B, kv_cache):
         qkv, gu = arena.fused_ptr(wq, wv), arena.fused_ptr(w1, wg)
     except (KeyError, AttributeError):  # parameters that are not plain ones of this block's arena
         return None
-    kc, vc, (Hq, Hkv, D, _) = kv_cache.keys_cache[i], kv_cache.values_cache[i], like
+    kc, vc, d, (Hq, Hkv, D, _) = kv_cache.keys_cache[i], kv_cache.values_cache[i], h.shape[1], like
     if (arena.data.dtype != BF16 or wo.shape != (d, Hq * D) or wd.shape != (d, F) or w1.shape[0] != F or kc.dtype != BF16 or kc.shape != vc.shape or kc.shape[0] != B
             or kc.shape[2] != Hkv * D or kc.stride() != vc.stride() or kc.stride(2) != 1):
         return None
-    L.require_gpu(arena.data, kc, vc)
+    L.require_gpu(h, arena.data, kc, vc)
     return [n1.data_ptr(), qkv, qn.data_ptr(), kn.data_ptr(), 0, 0, wo.data_ptr(), n2.data_ptr(), gu, wd.data_ptr(), 0, 0, 0]
 
 
@@ -332,7 +332,7 @@ def _step_layers(blocks, h, B, cos, sin, pos, km, kv_cache, dev_state, counters,
           and pos.dtype == write_pos.dtype == len_dev.dtype == torch.int32 and pos.numel() == B and (km is None or (km.dtype == torch.uint8 and km.shape[0] == B and km.stride(1) == 1)))
     rows, table, n = [torch.empty_like(h), torch.empty_like(h)], array("q"), 0  # a call starts on rows[0]; its input is rows[1] or the caller's
     for i, blk in enumerate(blocks):
-        layer = _layer_operands(blk, i, like, d, F, B, kv_cache) if ok else None
+        layer = _layer_operands(blk, i, like, h, F, B, kv_cache) if ok else None
         if layer is not None and km is not None and km.shape[1] < (start + 1 if dev_state is None else kv_cache.keys_cache[i].shape[1]):
             layer = None
         if layer is not None:
