@@ -682,9 +682,13 @@ def transpose(x, out=None):
 def dgrad(dy, w, out=None):
     """dX = dY W for a Linear with weight W [N_out, N_in].  Above ``DGRAD_NT_MIN_ROWS`` token rows W is transposed first (one pass over the
     weight, 63 MB per transformer block) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads;
-    same-box A/B in DESIGN.md.  The result is the same sum in the same order per K-tile, bit-identical to the NN form."""
-    M = dy.shape[0]
-    if DGRAD_NT and M >= DGRAD_NT_MIN_ROWS and (w.shape[0] & 7) == 0 and (w.shape[1] & 7) == 0:
+    same-box A/B in DESIGN.md.  The result is the same sum in the same order per K-tile, bit-identical to the NN form where neither is split over K."""
+    M, (Kd, N) = dy.shape[0], w.shape
+    # From 1 280 rows also where a long sum meets few output tiles (one round of the NT form's ring of K-tiles): by 1 024 columns, us, NN / transpose + NT, K = 4 096: 1 416 rows 41 / 34, 2 836 65 / 44,
+    # 3 545 75 / 47; K = 7 168: 64 / 46, 95 / 64, 115 / 79.  Not below (996 rows, K = 4 096 27 / 29, and a launch more for a step that waits for its launches), not for wide outputs of short sums
+    # (3 072 x 1 024, 2 000 rows 25 / 28), not behind a vocabulary (its K is split over the chip, and the transpose is 0.2 ms).
+    long_sum = M >= 1280 and 2 * N <= Kd and 2048 <= Kd <= 16384
+    if DGRAD_NT and (M >= DGRAD_NT_MIN_ROWS or long_sum) and (Kd & 7) == 0 and (N & 7) == 0:
         return gemm(L.GEMM_NT, dy, transpose(w), out=out)
     return gemm(L.GEMM_NN, dy, w, out=out)
 

@@ -80,3 +80,17 @@ def test_same_bits_every_time():
     A, B = torch.randn(700, 3072, device="cuda").to(BF16), torch.randn(1024, 3072, device="cuda").to(BF16)
     first = product(A, B, BF16)
     assert all(torch.equal(first, product(A, B, BF16)) for _ in range(3))
+
+
+@pytest.mark.parametrize("M,N,K", [(1279, 1024, 2048), (1280, 1024, 2048), (1280, 1024, 2040), (1500, 328, 3000), (4095, 1024, 4096), (1300, 64, 16392)])
+def test_input_gradients_on_both_sides_of_the_rule(M, N, K):
+    """dX = dY W by the NN form or on the transposed weight: the same product."""
+    from llm_quest_amd import kernels as KK
+
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    dy, w = torch.randn(M, K, generator=g, device="cuda").to(BF16), torch.randn(K, N, generator=g, device="cuda").to(BF16)
+    exact = dy.double() @ w.double()
+    bound = error_bound(dy, w.t(), 0) + 2.0 ** -8 * exact.abs()
+    assert ((KK.dgrad(dy, w).double() - exact).abs() <= bound).all()
+    out = torch.empty(M, N, dtype=BF16, device="cuda")
+    assert torch.equal(KK.dgrad(dy, w, out=out), KK.dgrad(dy, w))
