@@ -383,12 +383,17 @@ __global__ __launch_bounds__(256) void ga_bwd_dq_kernel(int B, int S, int Hq, in
     const unsigned drow = (unsigned)(((int64_t)it.b * Hq + it.h) * S + query);
     put(0);
     if (it.ntiles > 1) request(1);
-    for (int kt = 0; kt < it.ntiles; ++kt) {
-        const int key0 = kt * 32;
+    auto next_tile = [&](int kt) {
         __syncthreads();
         if (kt + 1 < it.ntiles) put(kt + 1);
         if (kt + 2 < it.ntiles) request(kt + 2);
-        // (a wave without an item, or above its diagonal, works on tiles that it sees nothing of: a branch around the products costs every trip 256 register copies)
+    };
+    // A wave without an item, or above its diagonal, multiplies nothing: a weight of zero times a later token that is not finite would be NaN.  Those tiles are its last ones, so they
+    // have a loop of their own (a branch around the products costs every trip 256 register copies).
+    const int seen = !it.on ? 0 : all_keys ? it.ntiles : it.q0 / 32 + 1;
+    for (int kt = 0; kt < seen; ++kt) {
+        const int key0 = kt * 32;
+        next_tile(kt);
         const char* kimg = smem + (kt & 1) * 2 * C::IMG;
         const char* vimg = kimg + C::IMG;
         f32x16 s = dot_rows<D>(kimg, qf, lane), dp = dot_rows<D>(vimg, gf, lane);
@@ -415,6 +420,7 @@ __global__ __launch_bounds__(256) void ga_bwd_dq_kernel(int B, int S, int Hq, in
         add_cols<D, D == 256 ? 'a' : 0>(acc, kimg, co, pack_frag(s, 0), pack_frag(s, 1));
     }
     settle<D == 256 ? 'a' : 0>(acc);
+    for (int kt = seen; kt < it.ntiles; ++kt) next_tile(kt);
     store_t_tiles<C::DT>(acc, 1.f, dq + (tok0 + query) * lddq + (int64_t)it.h * D, qvalid, lane);
 }
 

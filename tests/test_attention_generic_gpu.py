@@ -41,3 +41,45 @@ def test_edges_of_tiles_against_64_bits(B, S, Hq, Hkv, D, masked):
     assert bool((grads[:, (Hq + 2 * Hkv) * D :] == 7.0).all())  # nothing beside the gradients was written
     o2, _ = Q.attn_generic_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=km)
     assert torch.equal(o, o2)
+
+
+@pytest.mark.parametrize("entry", ["generic", "generic_dropout", "causal_dropout"])
+@pytest.mark.parametrize("S,Hq,Hkv,D", [(160, 1, 1, 256), (161, 3, 1, 128), (127, 2, 2, 64), (97, 6, 2, 256), (130, 1, 1, 32)])
+def test_a_token_that_is_not_finite_stays_where_it_is_seen(entry, S, Hq, Hkv, D):
+    """Without padding a token is seen by itself and later ones: in whole tiles of 32 before it outputs and query gradients keep their bits, in tiles behind a bad query those of the keys
+    and values do.  Groups of one, two and three query heads: the four waves of a query-major workgroup stand at different query tiles."""
+    from llm_quest_amd import kernels as K, kernels_q35 as Q
+
+    B, bad = 2, S - 20
+    g = torch.Generator().manual_seed(S + D)
+    q, k, v, do = (torch.randn(B * S, H * D, generator=g).to(BF16).cuda() for H in (Hq, Hkv, Hkv, Hq))
+
+    def run(q, k, v, do):
+        grads = [torch.empty_like(t) for t in (q, k, v)]
+        if entry == "generic":
+            o, lse = Q.attn_generic_fwd(q, k, v, B, S, Hq, Hkv, D)
+            Q.attn_generic_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, *grads)
+        elif entry == "generic_dropout":
+            o, lse = K.attn_generic_dropout_fwd(q, k, v, B, S, Hq, Hkv, D, 0.2, 3, 5)
+            K.attn_generic_dropout_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, *grads, 0.2, 3, 5)
+        else:
+            o, lse = K.attn_dropout_fwd(q, k, v, B, S, Hq, Hkv, D, 0.2, 3, 5, causal=True)
+            K.attn_dropout_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, *grads, 0.2, 3, 5, causal=True)
+        return [t.view(B, S, -1) for t in (o, *grads)]
+
+    o, dq, dk, dv = run(q, k, v, do)
+    before, behind = slice(0, bad // 32 * 32), slice((bad // 32 + 1) * 32, S)
+    for value in (float("nan"), float("inf")):
+        for which in (1, 2):  # a key, a value
+            rows = [q, k, v, do]
+            rows[which] = rows[which].clone()
+            rows[which].view(B, S, -1)[:, bad] = value
+            o1, dq1, _, _ = run(*rows)
+            assert torch.equal(o1[:, before], o[:, before]) and torch.equal(dq1[:, before], dq[:, before])
+        for which in (0, 3):  # a query, an output gradient
+            rows = [q, k, v, do]
+            rows[which] = rows[which].clone()
+            rows[which].view(B, S, -1)[:, bad] = value
+            o1, dq1, dk1, dv1 = run(*rows)
+            assert torch.equal(o1[:, before], o[:, before]) and torch.equal(dq1[:, before], dq[:, before])
+            assert torch.equal(dk1[:, behind], dk[:, behind]) and torch.equal(dv1[:, behind], dv[:, behind])
