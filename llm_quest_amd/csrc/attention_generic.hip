@@ -42,6 +42,26 @@ __device__ __forceinline__ void drop4(const DropArgs& da, unsigned row, int key4
     for (int e = 0; e < 4; ++e) mul[e] = bits[e] >= da.thresh ? da.inv_keep : 0.f;
 }
 
+// the same bits where a lane holds one key and 16 queries (x = 4 g + e: row(x)): a draw is four keys of one query, and four neighbouring lanes hold those keys, so each of them draws
+// for one query of every four and the bits go round by DPP -- 4 draws for 16.  Drawn per element, by both waves of a pair, they were more than the products: 128 x 197, 12 heads of 64, all keys seen, backward
+// 552 -> 430 us (one draw per element by one wave for both, before the pair: 480); 8 x 708, 8 heads of 256 over 2, causal 340 -> 246.
+template <class Row>
+__device__ __forceinline__ void drop_bits(const DropArgs& da, int key, Row row, unsigned (&kept)[4]) {
+    const int j = key & 3;
+    unsigned mine = 0;
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+        unsigned bits[4];
+        philox4x32_10((unsigned)key >> 2, row(4 * g + j), da.o0, da.o1, da.k0, da.k1, bits);
+#pragma unroll
+        for (int w = 0; w < 4; ++w) mine |= (unsigned)(bits[w] >= da.thresh) << (4 * g + w);
+    }
+    kept[0] = (unsigned)__builtin_amdgcn_mov_dpp((int)mine, 0x00, 0xf, 0xf, true) >> j;  // quad_perm: lane e of the four
+    kept[1] = (unsigned)__builtin_amdgcn_mov_dpp((int)mine, 0x55, 0xf, 0xf, true) >> j;
+    kept[2] = (unsigned)__builtin_amdgcn_mov_dpp((int)mine, 0xaa, 0xf, 0xf, true) >> j;
+    kept[3] = (unsigned)__builtin_amdgcn_mov_dpp((int)mine, 0xff, 0xf, 0xf, true) >> j;
+}
+
 template <int D>
 struct GA {
     static constexpr int ROWB = D * 2;       // bytes per LDS row
@@ -505,19 +525,16 @@ __global__ __launch_bounds__(256) void ga_bwd_dkv_kernel(int B, int S, int Hq, i
             for (int g = 0; g < 4; ++g) probs[stream][g][lane] = f32x4{s[4 * g], s[4 * g + 1], s[4 * g + 2], s[4 * g + 3]};
         }
         __syncthreads();
+        unsigned kept[4] = {~0u, ~0u, ~0u, ~0u};  // per query of a group of four: bit 4 g, this lane's key
+        // (DROP is a template parameter: the p = 0 kernels of the Qwen3.5 training path carry no Philox code)
+        if (DROP && da.thresh) drop_bits(da, key, [&](int x) { return (unsigned)(((int64_t)b * Hq + h) * S + qs + 8 * (x >> 2) + 4 * (lane >> 5) + (x & 3)); }, kept);
 #pragma unroll
         for (int g = 0; g < 4; ++g) {
             const f32x4 dl = *reinterpret_cast<const f32x4*>(&stats[r & 1][wave][8 * g + 4 * (lane >> 5)]), p = probs[stream][g][lane];
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int qi = qs + 8 * g + 4 * (lane >> 5) + e, x = 4 * g + e;
-                float keep = 1.f;
-                if (DROP && da.thresh) {  // (DROP is a template parameter: the p = 0 kernels of the Qwen3.5 training path carry no Philox code)  // this lane's key inside its group of four, for attention row (b, h, qi)
-                    unsigned bits[4];
-                    philox4x32_10((unsigned)key >> 2, (unsigned)(((int64_t)b * Hq + h) * S + qi), da.o0, da.o1, da.k0, da.k1, bits);
-                    const unsigned bsel = (key & 3) == 0 ? bits[0] : (key & 3) == 1 ? bits[1] : (key & 3) == 2 ? bits[2] : bits[3];
-                    keep = bsel >= da.thresh ? da.inv_keep : 0.f;
-                }
+                const int x = 4 * g + e;
+                const float keep = DROP && da.thresh ? (kept[e] >> 4 * g & 1u ? da.inv_keep : 0.f) : 1.f;
                 if (second) s[x] = p[e] * (s[x] * keep - dl[e]) * scale;
                 else s[x] *= keep;
             }

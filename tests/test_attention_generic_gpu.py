@@ -83,3 +83,26 @@ def test_a_token_that_is_not_finite_stays_where_it_is_seen(entry, S, Hq, Hkv, D)
             o1, dq1, dk1, dv1 = run(*rows)
             assert torch.equal(o1[:, before], o[:, before]) and torch.equal(dq1[:, before], dq[:, before])
             assert torch.equal(dk1[:, behind], dk[:, behind]) and torch.equal(dv1[:, behind], dv[:, behind])
+
+
+@pytest.mark.parametrize("S,Hq,Hkv,D,causal", [(33, 1, 1, 256, True), (97, 4, 2, 256, False), (70, 3, 1, 128, True), (197, 2, 2, 64, False), (5, 2, 1, 32, False)])
+def test_the_backward_draws_the_forwards_mask(S, Hq, Hkv, D, causal):
+    """dO . O and dV . V are one sum over the kept weights, sum_ij w_ij dO_i . V_j, in every head group: level to the roundings of w, O and dV to bf16 (2^-9 of each, of no fixed sign: 16 times
+    that of the terms' 2-norm).  A mask that differs would leave about half that norm."""
+    from llm_quest_amd import kernels as K
+
+    B, p = 2, 0.3
+    g = torch.Generator().manual_seed(S * D)
+    q, k, v, do = (torch.randn(B * S, H * D, generator=g).to(BF16).cuda() for H in (Hq, Hkv, Hkv, Hq))
+    grads = [torch.empty_like(t) for t in (q, k, v)]
+    o, lse = K.attn_dropout_fwd(q, k, v, B, S, Hq, Hkv, D, p, 11, 13, causal=causal)
+    K.attn_dropout_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, *grads, p, 11, 13, causal=causal)
+    heads = lambda t, H: t.double().view(B, S, H, D).transpose(1, 2)
+    per_group = lambda t: t.reshape(B, Hkv, -1).sum(-1)
+    left, right = per_group(heads(o, Hq) * heads(do, Hq)), per_group(heads(v, Hkv) * heads(grads[2], Hkv))
+    qd, kd, vd = heads(q, Hq), heads(k, Hkv).repeat_interleave(Hq // Hkv, 1), heads(v, Hkv).repeat_interleave(Hq // Hkv, 1)
+    scores = (qd @ kd.mT.contiguous()) * D**-0.5
+    if causal:
+        scores = scores.masked_fill(torch.ones(S, S, dtype=torch.bool, device="cuda").triu(1), float("-inf"))
+    terms = torch.softmax(scores, -1) / (1 - p) * (heads(do, Hq) @ vd.mT.contiguous())
+    assert bool(((left - right).abs() <= 16 * 2**-9 * per_group(terms**2).sqrt()).all())
