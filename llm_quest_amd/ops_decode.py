@@ -64,11 +64,13 @@ def decode_splits(n_keys, B, Hq):
 
 
 def step_splits(n_keys, B, Hq):
-    """``decode_splits`` of a whole layer's step: the splits of ONE sequence are folded where the output projection reads them, without a launch, so they are 128 keys each -- what
-    the attention's eight waves stream in one round (580-token prompt: 6.7 us in three splits, 5.8 in five)."""
+    """``decode_splits`` of a whole layer's step: the splits of ONE sequence are folded where the output projection reads them, without a launch, so they start at 128 keys each -- what
+    the attention's eight waves stream in one round (580-token prompt: 6.7 us in three splits, 5.8 in five) -- but every workgroup of the projection reads all of them, eight at a time:
+    past eight a split costs more than the keys that it takes off the others, until those are 1 024 each.  Captured steps (sized for the longest cache, us a token of 16 heads, 8 / 12 / 16 splits):
+    90 keys in room for 4 064 778 / 866 / 951; 710 785 / 850 / 928; 2 000 834 / 897 / 965; 4 000 909 / 967 / 1 030; 8 000 1 091 / 1 106 / 1 150; 14 000 1 342 / 1 311 / 1 358; 32 000 2 065 / 1 908 / 1 962."""
     if B > 1 or n_keys <= 256:
         return decode_splits(n_keys, B, Hq)
-    return max(1, min((n_keys + 127) // 128, 16, max(1, 256 // Hq)))
+    return max(1, min(max(min((n_keys + 127) // 128, 8), min(n_keys // 1024, 12)), 256 // Hq))
 
 
 def _split_ws(splits, B, Hq, D, device):
