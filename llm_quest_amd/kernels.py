@@ -679,16 +679,24 @@ def transpose(x, out=None):
     return out
 
 
+def dgrad_transposes(M, N, Kd):
+    """Whether dX [M, N] = dY [M, Kd] W is taken from a transposed copy of W by the NT form: from ``DGRAD_NT_MIN_ROWS`` rows always.
+
+    From 1 280 rows for long sums that are enough work to pay for the copy, whichever NT kernel they meet (one round of ``gemm_ring_kernel`` or, wider, 128 x 128 tiles).  us, NN / copy + NT, from 4.2e9
+    products on: K = 4 096, N = 1 024, 1 416 rows 41 / 34, 2 836 66 / 45; K = 8 192, N = 512, 1 280 rows 44 / 32; N = 4 096 168 / 122 (4 000 rows 277 / 227); K = 2 048, N = 1 024, 2 836 rows
+    39 / 25; K = 12 288, N = 6 144, 1 340 rows 397 / 299, 4 000 704 / 631.  Wider, the copy is
+    not paid back by few rows (K = 14 336, N = 7 168, 1 280 rows 411 / 435).  Below the line: K = 2 048, N = 64 15 / 18, N = 1 024, 1 280 rows 23 / 24; K = 4 096, N = 512, 1 700 rows 25.5 / 26;
+    996 rows, N = 1 024 27 / 29.  Up to 255 K-tiles of 64: beyond, the NN form divides K over the chip (K = 16 376, N = 1 024, 1 280 rows 82 / 101; 16 384, N = 4 096 206 / 243).
+    Wide outputs of short sums stay as they are (3 072 x 1 024, 2 000 rows 25 / 28)."""
+    return M >= DGRAD_NT_MIN_ROWS or (M >= 1280 and 2 * N <= Kd and N <= 6144 and 2048 <= Kd <= 16320 and M * N * Kd >= 4.2e9)
+
+
 def dgrad(dy, w, out=None):
-    """dX = dY W for a Linear with weight W [N_out, N_in].  Above ``DGRAD_NT_MIN_ROWS`` token rows W is transposed first (one pass over the
-    weight, 63 MB per transformer block) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads;
-    same-box A/B in DESIGN.md.  The result is the same sum in the same order per K-tile, bit-identical to the NN form where neither is split over K."""
+    """dX = dY W for a Linear with weight W [N_out, N_in].  Where ``dgrad_transposes`` says so W is transposed first (one pass over the
+    weight, 63 MB per transformer block) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads.
+    The result is the same sum in the same order per K-tile, bit-identical to the NN form where neither is split over K."""
     M, (Kd, N) = dy.shape[0], w.shape
-    # From 1 280 rows also where a long sum meets few output tiles (one round of the NT form's ring of K-tiles): by 1 024 columns, us, NN / transpose + NT, K = 4 096: 1 416 rows 41 / 34, 2 836 65 / 44,
-    # 3 545 75 / 47; K = 7 168: 64 / 46, 95 / 64, 115 / 79.  Not below (996 rows, K = 4 096 27 / 29, and a launch more for a step that waits for its launches), not for wide outputs of short sums
-    # (3 072 x 1 024, 2 000 rows 25 / 28), not behind a vocabulary (its K is split over the chip, and the transpose is 0.2 ms).
-    long_sum = M >= 1280 and 2 * N <= Kd and 2048 <= Kd <= 16384
-    if DGRAD_NT and (M >= DGRAD_NT_MIN_ROWS or long_sum) and (Kd & 7) == 0 and (N & 7) == 0:
+    if DGRAD_NT and dgrad_transposes(M, N, Kd) and (Kd & 7) == 0 and (N & 7) == 0:
         return gemm(L.GEMM_NT, dy, transpose(w), out=out)
     return gemm(L.GEMM_NN, dy, w, out=out)
 

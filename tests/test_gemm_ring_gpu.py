@@ -82,7 +82,7 @@ def test_same_bits_every_time():
     assert all(torch.equal(first, product(A, B, BF16)) for _ in range(3))
 
 
-@pytest.mark.parametrize("M,N,K", [(1279, 1024, 2048), (1280, 1024, 2048), (1280, 1024, 2040), (1500, 328, 3000), (4095, 1024, 4096), (1300, 64, 16392)])
+@pytest.mark.parametrize("M,N,K", [(1279, 1024, 2048), (1280, 1024, 2048), (1280, 1024, 2040), (1500, 328, 3000), (4095, 1024, 4096), (1300, 64, 16392), (1300, 2048, 4096), (2000, 3072, 6144), (1300, 1024, 16328), (1300, 1024, 16320)])
 def test_input_gradients_on_both_sides_of_the_rule(M, N, K):
     """dX = dY W by the NN form or on the transposed weight: the same product."""
     from llm_quest_amd import kernels as KK
