@@ -2501,6 +2501,14 @@ static int pp_mask() {
     return e && *e ? atoi(e) : MI355_GEMM_PP_DEFAULT;
 }
 
+// Forward products and input gradients of fewer 256x256 tiles than half of the CUs: measured 92 tiles -> 128x128 wins (+2.8 % on the hybrid step), 180 tiles -> 256x256 wins.  At 128 tiles, plain
+// NT, nine shapes from 512 x 16 384 to 32 700 x 256, K = 512 / 1 024 / 3 584 / 7 168, us: 256x256 19 - 20 / 29 - 34 / 106 - 120 / 159 - 194, 128x128 15 / 22 - 24 / 63 - 67 / 115 - 155 (300 x 16 384,
+// which fits gemm_ring_kernel: 16 / 20 / 47 / 79).
+static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
+    const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
+    return M < 256 || N < 256 || (form != MI355_GEMM_TN && tiles256 < 128 + (form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE));
+}
+
 // Tile rows (128 or 192; 0: none fits) and K shares of gemm_ring_kernel for a product of too few 256x256 tiles.  Only in ONE round of the 256 CUs: with more tiles Cfg128's two
 // workgroups per CU are the better filling (996 x 6144, K = 1024: 21 us, this kernel in two rounds 25).  The least of: the launch (3.5 us, 4.5 with 192 rows), its K-tiles (0.44 us each
 // where up to a quarter of the CUs work, 0.62 from half of them on; 192 rows 0.6 / 0.76), and for K shares -- from 32 K-tiles on, as in choose_ksplit -- the reduction's launch and bytes.
@@ -2521,6 +2529,12 @@ static int choose_ring(int64_t M, int64_t N, int64_t K, bool may_split, int64_t 
         }
     }
     return rows;
+}
+
+extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int may_split, int64_t workspace_bytes) {
+    int ksplit = 1;
+    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(MI355_GEMM_NT, M, N, MI355_EPI_NONE) ? choose_ring(M, N, K, may_split != 0, workspace_bytes, ksplit) : 0;
+    return rows ? rows | ksplit << 8 : 0;
 }
 
 extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* B,
@@ -2584,7 +2598,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
                                 workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
         if (M < 256 || N < 256) cfg = 1;
         else if (long_split && tiles256 < 128) cfg = 3;
-        else if (form != MI355_GEMM_TN && tiles256 < 128 + (form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE)) cfg = 1;  // measured: 92 tiles -> 128x128 wins (+2.8 % on the config-5 step), 180 tiles -> 256x256 wins; 128 tiles, plain NT (2 000 x 4 096, K = 1024): 33 -> 15 us (gemm_ring_kernel)
+        else if (small_tiles(form, M, N, epilogue)) cfg = 1;
         // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Round 4, batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)
         // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,

@@ -29,14 +29,16 @@ def error_bound(A, B, extra):
 
 
 # one tile and parts of it; row panels of 128 and of 192 (5 100 x 1 024: 216 tiles of 192 rows, 320 of 128); the ring filled once, odd and even counts of K-tiles, a remainder in the last; K shares
-# (long K, few tiles); 192: the longest K that keeps to the 128x128 kernel
-SIZES = [(1, 8, 256), (9, 16, 200), (127, 128, 320), (129, 136, 192), (191, 264, 264), (300, 1000, 1016), (61, 1024, 3072), (333, 1024, 3584), (5100, 1024, 328), (2000, 4096, 256), (996, 768, 1992)]
+# (long K, few tiles); 256 tiles of 192 rows where there are 128 of 256 x 256; without the ring (rows 0): more tiles than the one round, fewer K-tiles than the ring
+SIZES = [(1, 8, 256, 128), (9, 16, 200, 128), (127, 128, 320, 128), (129, 136, 192, 0), (191, 264, 264, 128), (300, 1000, 1016, 128), (61, 1024, 3072, 128), (333, 1024, 3584, 128), (5100, 1024, 328, 192),
+         (300, 16384, 256, 192), (2000, 4096, 256, 0), (300, 16392, 256, 0), (996, 768, 1992, 128)]
 
 
-@pytest.mark.parametrize("M,N,K", SIZES)
+@pytest.mark.parametrize("M,N,K,rows", SIZES)
 @pytest.mark.parametrize("odt", [BF16, F32])
 @pytest.mark.parametrize("bias,residual", [(False, False), (True, True), (False, True)])
-def test_against_64_bits(M, N, K, odt, bias, residual):
+def test_against_64_bits(M, N, K, rows, odt, bias, residual):
+    assert (L.load().mi355_gemm_nt_ring(M, N, K, not bias and N % 8 == 0, 128 << 20) & 255) == rows
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     A = torch.randn(M, K, generator=g, device="cuda").to(BF16)
     B = torch.randn(N, K, generator=g, device="cuda").to(BF16)
@@ -49,7 +51,7 @@ def test_against_64_bits(M, N, K, odt, bias, residual):
     if odt == BF16:
         bound = bound + 2.0 ** -8 * exact.abs()  # one rounding to eight bits
     assert ((got.double() - exact).abs() <= bound).all()
-    if K < 2048:  # without K shares: every sum in the same order
+    if K < 2048:  # no K shares, or the same: every sum in the same order
         assert torch.equal(product(A, B, odt, b, r, hint=1), got)
 
 
