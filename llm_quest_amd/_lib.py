@@ -5,9 +5,11 @@ fallback.  ``build()`` compiles it in-tree with hipcc for gfx950 (cross-compiles
 """
 
 import ctypes
+import importlib.machinery
 import os
 import subprocess
 import sys
+import warnings
 
 import torch
 
@@ -188,13 +190,19 @@ def build(verbose=False, force=False):
         raise RuntimeError("building libmi355vlm.so failed:\n" + res.stdout[-4000:] + res.stderr[-4000:])
     if verbose:
         print(res.stdout[-2000:])
+    if not os.path.exists(LAUNCH_PATH):
+        warnings.warn("llm_quest_amd: the native launch path was not built, launches go through ctypes, about 6 us each slower:\n" + res.stderr[-2000:])
     return LIB_PATH
 
 
-try:
-    from . import _launch  # built beside the library (csrc/Makefile); without it the launches below go through ctypes, with the same results
-except ImportError:
-    _launch = None
+# The native launch path, built beside the library for this interpreter (csrc/Makefile); without it launches go through ctypes, with the same results.
+LAUNCH_PATH = os.path.join(_HERE, "_launch" + importlib.machinery.EXTENSION_SUFFIXES[0])
+_launch = None
+if os.path.exists(LAUNCH_PATH):
+    try:
+        from . import _launch
+    except ImportError as e:
+        warnings.warn(f"llm_quest_amd: {LAUNCH_PATH} does not load ({e}): launches go through ctypes, about 6 us each slower")
 if not hasattr(torch._C, "_cuda_getDevice"):
     _launch = None
 

@@ -1,5 +1,11 @@
 """The native launch path (csrc/launch.cpp) does what the Python functions of _lib.py do, and hands them what it does not take.  No GPU: device and stream are stood in for, the entry
 points are asked for what they refuse on the host."""
+import importlib.machinery
+import os
+import shutil
+import subprocess
+import sys
+import sysconfig
 import threading
 
 import pytest
@@ -7,7 +13,9 @@ import torch
 
 from llm_quest_amd import _lib
 
-launch = pytest.importorskip("llm_quest_amd._launch")
+launch = _lib._launch
+if launch is None and not (shutil.which("g++") and os.path.exists(os.path.join(sysconfig.get_paths()["include"], "Python.h"))):
+    pytest.skip("no compiler or headers to build the extension with", allow_module_level=True)  # (with them a missing or broken extension fails below)
 BAD_FORM = (7, 1, 1, 8, None, 8, None, 8, None, 8, 0, None, None, 0, 0, None, 0, 0)
 
 
@@ -89,3 +97,35 @@ def test_the_device_belongs_to_the_thread(slow):
     t.start()
     t.join()
     assert seen == [-1] and launch.device() == 0
+
+
+def _sources(tmp_path):
+    """The extension's part of the source tree, built nowhere yet."""
+    root = os.path.dirname(os.path.dirname(os.path.abspath(_lib.__file__)))
+    for f in ("llm_quest_amd/csrc/launch.cpp", "llm_quest_amd/csrc/Makefile", "llm_quest_amd/_lib.py", "include/mi355_vlm.h"):
+        (tmp_path / f).parent.mkdir(parents=True, exist_ok=True)
+        shutil.copy(os.path.join(root, f), tmp_path / f)
+    (tmp_path / "llm_quest_amd" / "__init__.py").touch()
+    return tmp_path / "llm_quest_amd"
+
+
+@pytest.mark.parametrize("target", ["all", "serve"])
+@pytest.mark.parametrize("compiler", ["g++", "false"])
+def test_the_library_builds_without_the_extension(tmp_path, target, compiler):
+    """A host compiler that fails costs the extension, not the build; one that works leaves a file that no other interpreter takes, and none that any would take."""
+    package = _sources(tmp_path)
+    (package / "_launch.so").touch()
+    have = ["-o", "../libmi355vlm.so", "-o", "../libmi355serve.so"]  # the libraries count as built
+    for lib in have[1::2]:
+        (package / "csrc" / lib).touch()
+    done = subprocess.run(["make", "-C", str(package / "csrc"), "PYTHON=" + sys.executable, "CXX=" + compiler, *have, target], capture_output=True, text=True)
+    assert done.returncode == 0, done.stderr
+    built = sorted(p.name for p in package.glob("_launch*"))
+    assert built == (["_launch" + importlib.machinery.EXTENSION_SUFFIXES[0]] if compiler == "g++" else [])
+
+
+def test_an_extension_that_does_not_load_is_said(tmp_path):
+    package = _sources(tmp_path)
+    (package / ("_launch" + importlib.machinery.EXTENSION_SUFFIXES[0])).write_bytes(b"not a library")
+    done = subprocess.run([sys.executable, "-c", "from llm_quest_amd import _lib; assert _lib._launch is None and _lib.call is _lib._python_call"], cwd=tmp_path, capture_output=True, text=True)
+    assert done.returncode == 0 and "does not load" in done.stderr, done.stderr
