@@ -375,7 +375,8 @@ extern "C" int mi355_gated_headnorm(int64_t tokens, int H, int D, const float* o
 __device__ __forceinline__ float log_sigmoid(float z) { return fminf(z, 0.f) - log1pf(expf(-fabsf(z))); }
 
 // st[r] <- a[r] st[r] + k[r] v, acc += q[r] st[r] for the 16 channels that the lanes of a row of 16 hold one of: row_newbcast:r is lane r's operand for all of them.  (hipcc moves the
-// broadcast operand of a sum of products to a register first; s_nop: operands that a vector instruction may just have written.)
+// broadcast operand of a sum of products to a register first; s_nop: operands that a vector instruction may just have written; &: results are written before the last use of the four
+// operands, and must not share a register with one that happens to hold the same value.)
 __device__ __forceinline__ void gla_rows(float (&st)[GLA_R], float& acc, float q, float k, float a, float v) {
     static_assert(GLA_R == 16, "one channel a lane of a row");
     asm("s_nop 1\n\t"
@@ -411,8 +412,8 @@ __device__ __forceinline__ void gla_rows(float (&st)[GLA_R], float& acc, float q
                  "v_fmac_f32_dpp %16, %17, %13 row_newbcast:13 row_mask:0xf bank_mask:0xf\n\t"
                  "v_fmac_f32_dpp %16, %17, %14 row_newbcast:14 row_mask:0xf bank_mask:0xf\n\t"
                  "v_fmac_f32_dpp %16, %17, %15 row_newbcast:15 row_mask:0xf bank_mask:0xf"
-        : "+v"(st[0]), "+v"(st[1]), "+v"(st[2]), "+v"(st[3]), "+v"(st[4]), "+v"(st[5]), "+v"(st[6]), "+v"(st[7]), "+v"(st[8]), "+v"(st[9]), "+v"(st[10]), "+v"(st[11]), "+v"(st[12]),
-          "+v"(st[13]), "+v"(st[14]), "+v"(st[15]), "+v"(acc)
+        : "+&v"(st[0]), "+&v"(st[1]), "+&v"(st[2]), "+&v"(st[3]), "+&v"(st[4]), "+&v"(st[5]), "+&v"(st[6]), "+&v"(st[7]), "+&v"(st[8]), "+&v"(st[9]), "+&v"(st[10]), "+&v"(st[11]), "+&v"(st[12]),
+          "+&v"(st[13]), "+&v"(st[14]), "+&v"(st[15]), "+&v"(acc)
         : "v"(q), "v"(k), "v"(a), "v"(v));
 }
 
