@@ -33,7 +33,6 @@ constexpr int W_DU = GD * GD, W_BLOCK = W_DU + GC * GD;  // backward workspace o
 __device__ __forceinline__ u32x2 row4(const bf16_t* p, int64_t ld, int r, int cnt, int c) {
     return r < cnt ? *reinterpret_cast<const u32x2*>(p + r * ld + c) : u32x2{0u, 0u};
 }
-__device__ __forceinline__ float one(const bf16_t* p, int64_t ld, int r, int cnt, int c) { return r < cnt ? bf2f(p[r * ld + c]) : 0.f; }
 
 __device__ __forceinline__ double cumulated_log(const float* alpha, int64_t idx, bool in, float& a_out) {
     a_out = decay_at_least(in ? alpha[idx] : 1.f);
