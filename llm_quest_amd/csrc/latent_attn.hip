@@ -242,6 +242,8 @@ __global__ __launch_bounds__(256) void latent_attn_fma_kernel(LatAttnArgs p, int
 // barrier in the loop): the four heads' partial scores of a key fold into one register -- heads by rows of 16 lanes -- in six swaps and adds, and the weights come back to all lanes
 // as scalars.  Which of the two a sequence takes depends on its own new tokens alone, so a row's bits do not depend on the rest of the step.  118 -> 20.7 us
 // (keys dealt to 8 waves; what is left is two rounds of a wave's keys from memory, the exchange and the launch).
+// STEP_NEW is what steps of a token (or a token and one more) need, not where the other kernel gets better.  us at 3 / 8 new tokens, the tile -> this kernel, 8 heads, 256 + 64 | 256 shared: three sequences of 150
+// keys 99 / 100 -> 17 / 18, of 2 000 1 055 / 1 059 -> 135 / 136; 32 sequences of 150 100 / 102 -> 19 / 34; 8 heads of 128 + 64 | 128 of their own, 32 sequences of 2 000: 826 / 825 -> 373 / 975.
 constexpr int STEP_NEW = 2, STEP_WAVES = 8, STEP_KB = 4;
 __device__ __forceinline__ float fold32(float a, float b) {  // lanes 0 .. 31: a folded over the halves, 32 .. 63: b
     const auto r = __builtin_amdgcn_permlane32_swap(__float_as_uint(a), __float_as_uint(b), false, false);

@@ -63,6 +63,9 @@ def test_experts_of_few_rows(counts, K, N, epi, dt):
 CASES = [dict(), dict(shared=True, D2=8), dict(shared=True, values_are_keys=True, D1=256, D2=64, DV=256, H=8), dict(H=6, rep=3, DV=70), dict(H=8, rep=4, window=37, keep=5), dict(H=4, rep=2, chunk=48),
          dict(H=3, window=20, chunk=64, softcap=3.0), dict(H=5, shared=True, sink=True, slope=True), dict(H=2, sig=True, window=33), dict(H=4, gate=True, softcap=2.0, D1=130, DV=257),
          dict(H=9, shared=True, D1=512, D2=128, DV=512, values_are_keys=True), dict(H=2, D1=100, DV=129, window=1), dict(H=4, rep=4, sink=True, window=16, keep=64)]
+# values that are the first features of the keys and come by the keys' row table itself (the served models' call): read once, in every size of the kernel
+CASES += [dict(opt, values_are_keys=True, one_table=True) for opt in (dict(shared=True, D1=72, D2=8, DV=48, H=5), dict(shared=True, D1=200, DV=150, H=4, sink=True), dict(shared=True, D1=256, D2=64, DV=256, H=8, window=37),
+                                                                      dict(shared=True, D1=512, D2=128, DV=512, H=9), dict(H=6, rep=3, D1=64, DV=64), dict(H=8, rep=4, D1=130, DV=129, sig=True))]
 
 
 @pytest.mark.parametrize("opt", CASES, ids=lambda o: "-".join(f"{k}{int(v)}" for k, v in o.items()) or "plain")
@@ -93,7 +96,8 @@ def test_attention_of_one_or_two_new_tokens(opt, dt):
     def run(seqs):
         out = torch.full((R, H * DV), float("nan"), device="cuda")
         pick = lambda a: i32([a[i] for i in seqs])
-        desc = (pick(q0), pick(new), pick(past), pick(k0), pick(k0), pick(k0))
+        table = pick(k0)
+        desc = (pick(q0), pick(new), pick(past), table, pick(k0), table if opt.get("one_table") else pick(k0))
         hm = 1
         while hm * 2 <= 8 and (shared or rep % (hm * 2) == 0):
             hm *= 2
