@@ -3,9 +3,9 @@
  * LLM-quest VLM forward/backward hot path.
  *
  * The reference (casinca/LLM-quest) has NO native/FFI layer: every op is a stock torch call inside an
- * nn.Module.forward (SURVEY.md section 8b).  Each entry point below therefore cites the reference *call site*
+ * nn.Module.forward.  Each entry point below therefore cites the reference *call site*
  * it replaces (file:line relative to the reference checkout); the binding a maintainer adds on the reference
- * side is a ctypes stub, shown in INTEGRATION.md.
+ * side is a ctypes stub.
  *
  * Conventions
  *   - plain pointers are DEVICE pointers (HBM) unless stated; sizes are element counts unless "_bytes"
@@ -81,7 +81,7 @@ int mi355_abi_version(void);
  *                    SwiGLU-backward epilogues; other calls fall back to 2.  0 takes it by itself from 512 tiles upward (environment variable
  *                    MI355_GEMM_PERSIST_MIN_TILES, read per call, moves that threshold: its 256 workgroups assume they all start together, so a caller that runs
  *                    collectives or another stream's kernels beside its GEMMs raises it for that time -- llm_quest_amd/ddp.py does)
- * Requirements: K-contiguous dims multiple of 8 elements (16-byte rows); see DESIGN.md.            */
+ * Requirements: K-contiguous dims multiple of 8 elements (16-byte rows).            */
 int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* B,
                     int64_t ldb, void* C, int64_t ldc, int out_dtype, const float* bias, const void* residual,
                     int64_t ldr, int epilogue, void* workspace, int64_t workspace_bytes, int tile_hint, void* stream);
@@ -305,7 +305,7 @@ int mi355_adamw(int64_t n, void* param, int p_dtype, const void* grad, int g_dty
 int mi355_add_f32_to_bf16(int64_t n, const float* a, const void* b_bf16, void* dst_bf16, void* stream);
 
 /* ---------------------------------------------------------------------------------------------------------------------
- * Qwen3.5 hybrid text stack (BASELINE config 5, SURVEY.md section 8 row a24): csrc/qwen35.hip, csrc/attention_generic.hip.
+ * Qwen3.5 hybrid text stack: csrc/qwen35.hip, csrc/attention_generic.hip.
  * "proj" below is the token-major output of ONE fused projection GEMM; column blocks of it are passed as pointer + ld.
  * ------------------------------------------------------------------------------------------------------------------- */
 
@@ -412,7 +412,7 @@ int mi355_gated_rmsnorm_bwd(int64_t tokens, int H, int D, const void* o, const f
                             const void* dout, void* d_o, void* dgate, int64_t lddg, float* dw_partial, int parts, void* stream);
 
 /* ---------------------------------------------------------------------------------------------------------------------
- * Input pipeline on the step's left edge (SURVEY.md section 8 row f3): MultimodalDataset's per-sample work, dataset.py:295-383.
+ * Input pipeline on the step's left edge: MultimodalDataset's per-sample work, dataset.py:295-383.
  * ------------------------------------------------------------------------------------------------------------------- */
 
 /* transforms.Resize((s, s)) on a PIL image = Pillow's fixed-point two-pass bilinear resampler (Resample.c), bit-exact.  bounds
@@ -431,7 +431,7 @@ int mi355_pad_tokens(int B, int L, const int64_t* flat_ids, const int64_t* offse
                      void* stream);
 
 /* ---------------------------------------------------------------------------------------------------------------------
- * KV-cache decoding on the step's right edge (SURVEY.md section 8 row f4): generate_loop_kv_cache (generate.py:97-151) with
+ * KV-cache decoding on the step's right edge: generate_loop_kv_cache (generate.py:97-151) with
  * utils.KVCache (utils.py:409-531).  csrc/decode.hip.
  * ------------------------------------------------------------------------------------------------------------------- */
 

@@ -5,7 +5,7 @@ built under ``with torch.device("cuda")`` inherits CPU tables that no ``.to()`` 
 force at the call) is part of the key.
 
 The HIP attention kernels never read the (ctx, ctx) mask -- causality is computed from indices -- but the buffer is
-still produced so ``state_dict()`` / attribute access match the reference (long-context row).
+still produced so ``state_dict()`` / attribute access match the reference.
 """
 
 import torch

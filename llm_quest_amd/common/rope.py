@@ -6,7 +6,7 @@ init.  Applying a rotation has two implementations behind one signature:
   * device tensors: the HIP kernel ``mi355_rope_apply`` (csrc/rope_dropout.hip) with the reference's rounding points, wrapped
     in an autograd node whose backward is the kernel's adjoint mode; MRoPE-I first gathers its interleaved per-token coefficient
     rows with ``mi355_mrope_table`` (an exact gather), so 1-D RoPE, partial rotation, 2-D axial RoPE and MRoPE are one kernel;
-  * host tensors (table checks, the GPT-2 CPU plumbing of BASELINE config 1): the same arithmetic in torch ops.
+  * host tensors (table checks, the GPT-2 CPU model): the same arithmetic in torch ops.
 
 Inside the training step the rotation never runs on its own: it is fused with the QK-norm (``mi355_qknorm_rope_fwd``,
 ``mi355_headnorm_rope_fwd``).  These entry points are the drop-in boundary for callers that use ``RoPE`` directly.

@@ -1,5 +1,5 @@
 """Model configuration dicts (the constructor-dict keys are part of the API) -- subset of the reference's ``config.py``
-covering the hot path: GPT-2 (config 1), ViT-Base (config 2/4) and dense Qwen3 (config 3/4)."""
+covering the hot path: GPT-2, ViT-Base and dense Qwen3."""
 
 import torch
 

@@ -218,7 +218,7 @@ __global__ __launch_bounds__(256, 2) void attn_fwd_kernel(int B, int S, int Hq, 
 //     batch rows walk every tile.
 // (An experiment with ONE wave per SIMD, both heads of a kv pair per wave and a hand-placed schedule lives outside the product library in
 // tools/experimental/attention_fwd2.hip: its MFMAs hide completely, but a lone wave pays ~10 cycles for every dependent vector instruction and
-// nothing covers its per-block prologue / epilogue: 322 us against this kernel's time at the headline shape)
+// nothing covers its per-block prologue / epilogue: 322 us against this kernel's time at the headline shape.)
 constexpr float LEAN_THR = 8.0f;
 constexpr unsigned LEAN_FILL = __builtin_bit_cast(unsigned, MASK_T);
 __device__ __forceinline__ float lean_max3(float m, float x, float y) {
@@ -797,7 +797,7 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_kernel(int B, int S, int H
 // LEAN: the row constants are INITIAL ACCUMULATORS (`lse` / `delta` then point at -lse * log2(e) and -delta, written by the delta kernel) and the
 // scale log2(e) / sqrt(d) is folded into this wave's K rows once per key block (bf16(k * c): one more rounding of a bf16 operand), so the S chain
 // delivers the exponent of P and the dP chain dP - delta: the B phase shrinks from six vector instructions per score (scale the constant, fma, exp2,
-// subtract, multiply, pack) to three (exp2, multiply, pack) -- the pass is bound by what its lone wave has to issue (DESIGN.md section 5).
+// subtract, multiply, pack) to three (exp2, multiply, pack) -- the pass is bound by what its lone wave has to issue.
 template <int D, bool LEAN>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dkv_kernel(int B, int S, int Hq, int Hkv, const bf16_t* __restrict__ q, int64_t ldq,
                                                               const bf16_t* __restrict__ k, int64_t ldk, const bf16_t* __restrict__ v,

@@ -2,7 +2,7 @@
 // 32 for the tiny fixtures), with the mask semantics of F.scaled_dot_product_attention as the reference calls it
 // (qwen3_next_attention.py:238-254, qwen3_5_text_model.py:244-259): boolean mask, True = attend, everything else -inf.
 //   allowed(i, j) = j <= i  OR  key j is padding        <- upstream ORs the inverted padding mask into the ALLOW mask,
-//                                                           which un-masks padded keys for every query (SURVEY 9.6); reproduced.
+//                                                           which un-masks padded keys for every query; reproduced.
 // Same data flow as the tuned forward: S^T = K Q^T with the query on the MFMA lane (mfma_f32_32x32x16_bf16, A = K rows from
 // LDS, B = Q rows in registers), lane-local online softmax, P^T packed from the accumulators as the B operand of
 // O^T += V^T P^T, V consumed K-strided through ds_read_b64_tr_b16.

@@ -1,4 +1,4 @@
-// KV-cache decoding on the step's right edge (SURVEY.md section 8 row f4): the per-token path of generate_loop_kv_cache
+// KV-cache decoding on the step's right edge: the per-token path of generate_loop_kv_cache
 // (llm_quest/generate.py:97-151) through Qwen3 with utils.KVCache (utils.py:409-531).  One new token per sequence makes every
 // linear layer a matrix-VECTOR product and attention one query row against the cache: both are HBM-bound byte streams (weights,
 // resp. cached K/V read exactly once per token), so the kernels here are bandwidth kernels, not MFMA kernels.

@@ -397,7 +397,7 @@ __global__ __launch_bounds__(1024) void ce_rows_regs_kernel(int64_t rows, int64_
     }
 }
 
-// One block of 1024 threads, four independent row loads in flight per thread (round 6: 256 threads walking 320 dependent iterations took 233 us -- on the step's critical
+// One block of 1024 threads, four independent row loads in flight per thread (256 threads walking 320 dependent iterations took 233 us -- on the step's critical
 // path between the loss rows and the backward -- this form ~30); a fixed summation order: per thread, per wave, then the sixteen waves in order.
 __global__ __launch_bounds__(1024) void ce_finalize_kernel(int64_t rows, const float* __restrict__ loss_rows,
                                                            const int64_t* __restrict__ targets, float* __restrict__ out3) {

@@ -257,7 +257,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int pid, co
     // super-group height by in-step A/B on the VLM step (ms/step, two runs each): 2: 245.9 / 246.2, 3: 243.8 / 243.8, 4: 245.3 / 245.3, 6: 243.8 / 244.3,
     // 8: 245.2 / 245.6, 16: 249.7 / 248.0.  Profiling bits 5-7 of the tile hint select another height.
     const int gsel = (p.ablate >> 5) & 7;
-    // Round 3, NT gate-up shape alone (profiles/r03_tile_walk.json): fabric reads 1 383 / 1 116 / 996 / 946 / 1 010 / 1 390 MB at heights 2 / 3 / 4 / 6 / 8 / 16, time
+    // NT gate-up shape alone (profiles/r03_tile_walk.json): fabric reads 1 383 / 1 116 / 996 / 946 / 1 010 / 1 390 MB at heights 2 / 3 / 4 / 6 / 8 / 16, time
     // 602 / 595 / 582 / 584 / 583 / 585 us -- the walk moves the re-fetch by 1.5x and the time by 2 %; in the step, all NT launches at 6 against 3: 194.5 / 194.6 against
     // 194.9 / 195.2 ms.  NT launches therefore walk 6-row groups, the K-strided forms stay at 3 (selector 6 = 3 rows for A/B runs).
     const int GROUP_M = gsel == 1 ? 4 : gsel == 2 ? 16 : gsel == 3 ? 2 : gsel == 4 ? 6 : gsel == 5 ? 8 : gsel == 6 ? 3 : (!A_TR && !B_TR) ? 6 : 3;
@@ -818,7 +818,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int pid, co
     if (extra_barrier) __builtin_amdgcn_s_barrier();
     TL_STAMP(2);
 #ifdef GEMM_EPI_ABL  // profiling builds only (tools/build_variant.sh epi1 gemm_p2 "-DGEMM_EPI_ABL=1", tools/time_nt_shapes.py): no write-out at all -- what is left is
-    // prologue + main loop.  Round 4, batch 160: QKV 907 -> 767 us, gate-up + SwiGLU 1 490 -> 1 100, down dgrad + SwiGLU backward 975 -> 575, dctx 455 -> 368.
+    // prologue + main loop.  Batch 160: QKV 907 -> 767 us, gate-up + SwiGLU 1 490 -> 1 100, down dgrad + SwiGLU backward 975 -> 575, dctx 455 -> 368.
     if (GEMM_EPI_ABL & 1) {
         float keep = 0.f;
 #pragma unroll
@@ -1167,7 +1167,7 @@ __global__ __launch_bounds__(T::NTHREADS, T::MIN_WAVES) void gemm_bf16_kernel(Ge
 }
 
 // ---------------------------------------------------------------------------------------------- persistent NT kernel (tile hint 7)
-// tools/gemm_timeline.py (per-workgroup wall-clock stamps, round 4) on the QKV projection of the step, 256x256 tile, K = 1024: of a tile's 31.0 us turn on its CU the
+// tools/gemm_timeline.py (per-workgroup wall-clock stamps) on the QKV projection of the step, 256x256 tile, K = 1024: of a tile's 31.0 us turn on its CU the
 // main loop is 24.8; the rest is prologue 1.9 (entry -> first K-tile landed), barrier 0.6, write-out 2.45 (LDS-bandwidth: 512 KiB of fp32 staging traffic per tile),
 // stores retiring 0.5 and 0.8 between a workgroup's end and its successor's entry.  This kernel keeps ONE workgroup per CU alive over its share of the tiles:
 //   * the K-tile stream runs across tile boundaries (the last two barriers of a tile request the next tile's first two K-tiles), so there is no prologue, no
@@ -1200,7 +1200,7 @@ __global__ __launch_bounds__(512, 2) void gemm_nt_persist_kernel(GemmParams p, i
     // streams, stream r takes the run's pairs r, r + 8, ...; at K = 1 024 an XCD's four weight panels (2 MB) stay in its L2 for the whole launch.  A column group's
     // missing panels (N / 256 not a multiple of 4) are walked as empty tiles (everything beyond the matrix: zero operands, no stores).  Needs the full grid of 256.
     constexpr bool walk = WALK;
-    // cache policy of the output stores (0 default, 2 = nt, 16 = sc1, 18 = both).  Round 6, same-box bench.py pairs with the walk by shape: base 435.7 / 436.4 ms, nt on the
+    // cache policy of the output stores (0 default, 2 = nt, 16 = sc1, 18 = both).  Same-box bench.py pairs with the walk by shape: base 435.7 / 436.4 ms, nt on the
     // weight-stationary launches 434.3 / 435.1, sc1 436.1 / 435.3, sc1 nt 434.5 / 434.8: nt there (the tile is written once and next read by another kernel; the L2 keeps the
     // weight panels instead)
     constexpr int CAUX = WALK ? GEMM_C_AUX_WALK : GEMM_C_AUX_OLD;
@@ -1582,7 +1582,7 @@ int launch_persist(GemmParams p, hipStream_t s) {
 // ---------------------------------------------------------------------------------------------- ping-pong persistent NT kernel (tile hint 8)
 // gemm_nt_persist_kernel's two waves per SIMD (w and w + 4: the upper and the lower 128 rows of the 256 x 256 tile) reach their write-out together, so the
 // matrix pipe of every SIMD idles for the whole write-out: 2.45 of a tile's 27.5 us with the plain epilogue at K = 1 024, a quarter of the tile with the SwiGLU
-// forms (round 5: 1.26 PF plain, 1.11 / 0.84 PF fused).  VALU / LDS / store issue and the matrix pipe are separate resources of a SIMD; what keeps them from
+// forms (1.26 PF plain, 1.11 / 0.84 PF fused).  VALU / LDS / store issue and the matrix pipe are separate resources of a SIMD; what keeps them from
 // overlapping is only that both waves are in the same phase.  This kernel runs the two wave groups E K-tiles apart:
 //   * time is counted in SLOTS (one K-tile of the stream, one workgroup barrier each).  A group's tile takes NT = K / 64 multiplying slots and E write-out
 //     slots (the write-out cut into E chunks, one per slot); the lower group (waves 4-7) starts E slots late.  So whenever one group writes out, the other
@@ -1595,7 +1595,7 @@ int launch_persist(GemmParams p, hipStream_t s) {
 //     panel; waves 0-3 right behind the barrier that frees the stage, waves 4-7 half a slot later (the CU has one address unit: see gemm_nt_persist_kernel).
 // NT form, bf16 output, K % 64 == 0, K / 64 >= E, N % 8 == 0, no bias.
 //
-// STATUS (round 6): correct on every epilogue kind (tools/experimental/pp_check.py: bit-identical to tile 2 on integer operands, fp32-summation noise on random ones), and
+// STATUS: correct on every epilogue kind (tools/experimental/pp_check.py: bit-identical to tile 2 on integer operands, fp32-summation noise on random ones), and
 // SLOWER than gemm_nt_persist_kernel wherever the write-out matters, so the library does not choose it (MI355_GEMM_PP_DEFAULT 0; tile hint 8 / MI355_GEMM_PP select it).
 // Batch 160, isolated, us (hint 7 -> hint 8): QKV 771 -> 881, out-proj + residual 424 -> 453, gate-up + SwiGLU 1 310 -> 1 451, down dgrad + SwiGLU backward 905 -> 1 063,
 // LM head forward 21.8 -> 22.6 ms; long-K shapes level (dqkv 733 -> 752, LM head dgrad 19.3 -> 18.6 ms: the walk).  In the step: +1.5 ... +7 ms per kind.  Why:
@@ -2353,7 +2353,7 @@ int check_operands(const char* who, int form, int64_t M, int64_t N, int64_t K, c
 // ---------------------------------------------------------------------------------------------- colsum
 // Column sums (bias gradients): a workgroup owns 512 columns x `rows_per_block` rows; a thread keeps 8 adjacent columns, a wave reads one kilobyte
 // of a row per instruction (16-byte loads, whole lines), the four waves take rows r, r+1, r+2, r+3; partial sums meet in LDS and leave as one
-// fp32 atomic per column and workgroup.  (Round 4: the first version read one 2-byte element per thread -- 128-byte row segments -- and ran at
+// fp32 atomic per column and workgroup.  (A first version read one 2-byte element per thread -- 128-byte row segments -- and ran at
 // 1.8 TB/s: 4.7 ms of the 53-ms ViT-B/16 training step.)
 template <int DT>
 __global__ __launch_bounds__(256) void colsum_kernel(int64_t M, int64_t N, const void* Xv, int64_t ldx, float* out, int rows_per_block) {
@@ -2484,7 +2484,7 @@ static int64_t persist_min_tiles() {
 // 8 SwiGLU backward, 16 attention delta (MI355_GEMM_PP; read per call: A/B runs and tests change it inside one process)
 static bool walk_on(int64_t N, int64_t K) {
     // MI355_GEMM_WALK: the persistent NT kernel's weight-stationary walk (gemm_nt_persist_kernel<.., WALK>) for launches the library chooses by itself: 0 never, 1 always,
-    // 2 (default) by shape: few column panels under a long K (the dgrads into d = 1024, the out / down projections), or very many column panels (the LM head).  Round 6,
+    // 2 (default) by shape: few column panels under a long K (the dgrads into d = 1024, the out / down projections), or very many column panels (the LM head).
     // batch 160, same-box bench.py runs: never 443.3 / 443.6 / 444.7 / 445.9 ms, by shape 438.5 / 438.6 / 441.4-441.8, always 441.6 / 440.6; per shape class (16 + mask):
     // N <= 1024 with K >= 3072 -3.7 ms, + K = 2048 -0.2, the LM head 0 to -1.2, N = 2048 0, N = 3072 / 4096 / 6144 (K = 1024) +1.0 to +1.9 ms each.  Read per call.
     const char* e = getenv("MI355_GEMM_WALK");
@@ -2589,7 +2589,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         // per form, 246.2 ms/step with tile 3 everywhere vs +0.9 (NT) / +4.3 (NN) / +0.5 (TN) ms with tile 4.  The step decides.
         // The same A/B puts the forward projections (NT) on tile 2 (BK 64, two stages, fragments prefetched one phase ahead):
         // 239.3 vs 243.8-246 ms/step with NT on tile 3, although tile 3 is 10-20 % faster on every isolated NT shape.
-        // 256x256 tiles need at least half of the 256 CUs' worth of tiles; below that (small token counts: config 5 at B = 8 has 92 tiles for
+        // 256x256 tiles need at least half of the 256 CUs' worth of tiles; below that (small token counts: the hybrid model at B = 8 has 92 tiles for
         // its N = 1024 outputs) four times as many 128x128 tiles, two workgroups per CU, fill the chip instead
         const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
         // input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
@@ -2599,7 +2599,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         if (M < 256 || N < 256) cfg = 1;
         else if (long_split && tiles256 < 128) cfg = 3;
         else if (small_tiles(form, M, N, epilogue)) cfg = 1;
-        // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Round 4, batch 160:
+        // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)
         // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,
         // which the four waves have no partner to hide (151 936 x 1 024, tile 5 / 3 / 1: 61 tokens 117 / 96 / 100, 333 196 / 174 / 200, 602 259 / 248 / 275, 1 024 367 / 374 / 398;
@@ -2608,7 +2608,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         else if (form == MI355_GEMM_NT) cfg = 2;
         else cfg = 3;
     }
-    // the persistent form of tile 2 (hint 7): same bits, no prologue / barrier / workgroup turnover per tile and a quarter of the staging traffic.  Round 4, batch 160, isolated:
+    // the persistent form of tile 2 (hint 7): same bits, no prologue / barrier / workgroup turnover per tile and a quarter of the staging traffic.  Batch 160, isolated:
     // QKV 890-917 -> 818-825 us, gate-up + SwiGLU 1 489-1 494 -> 1 418-1 422, down dgrad + SwiGLU backward 959-986 -> 920, dqkv dgrad 788-818 -> 756-764.  Chosen by itself from two
     // rounds of tiles upward (below that every workgroup has one tile and split-K may pay instead)
     const bool persist_ok = form == MI355_GEMM_NT && out_dtype == MI355_DT_BF16 && (epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_SWIGLU_FWD || epilogue == MI355_EPI_SWIGLU_BWD) &&

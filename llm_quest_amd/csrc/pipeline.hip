@@ -1,4 +1,4 @@
-// Input pipeline on the step's left edge (SURVEY.md section 8 row f3): the per-sample work of MultimodalDataset
+// Input pipeline on the step's left edge: the per-sample work of MultimodalDataset
 // (llm_quest/dataset.py:295-383) as HBM-bound byte kernels -- Pillow's two-pass fixed-point bilinear resize
 // (transforms.Resize on a PIL image), ToTensor + Normalize, and the pad / truncate / mask of the tokenised caption.
 // Integer arithmetic end to end up to the final float conversion: bit-exact against Pillow 12.2 (tests/test_pipeline_*.py).

@@ -1,6 +1,6 @@
 // Measurement aid, not part of the training path: what the matrix pipe ALONE sustains on this board -- v_mfma_f32_32x32x16_bf16 on every SIMD of the launch's workgroups, random bf16
 // operands held in registers, no memory traffic.  On random data the board's power cap, not the 2.4-GHz slot count behind the 2.5-PFLOP/s dense peak, sets this rate
-// (DESIGN.md section 5; tools/microbench/mfma_power.hip is the stand-alone form with the all-zero and LDS-fed variants).  bench.py times it beside the step so that the
+// (tools/microbench/mfma_power.hip is the stand-alone form with the all-zero and LDS-fed variants).  bench.py times it beside the step so that the
 // bench line carries the ceiling of the box it ran on.
 #include "common.h"
 
@@ -43,7 +43,7 @@ __global__ __launch_bounds__(256, 1) void mfma_pipe_kernel(float* __restrict__ o
 }
 
 // The shape the GEMMs issue (gemm.hip: v_mfma_f32_16x16x32_bf16 on a 128 x 64 wave tile): one K step = 32 products on eight + four fragments, 32 independent
-// accumulators of four registers.  Round 5's attempt at this loop came out issue-bound as compiled (63 % of the slots: 64 accumulators, the fragments re-materialised);
+// accumulators of four registers.  An earlier attempt at this loop came out issue-bound as compiled (63 % of the slots: 64 accumulators, the fragments re-materialised);
 // here the twelve fragments stay pinned across the loop and a repetition is exactly 32 back-to-back MFMAs.
 __global__ __launch_bounds__(256, 1) void mfma_pipe16_kernel(float* __restrict__ out, int reps) {
     u32x4 fr[12];

@@ -1,4 +1,4 @@
-// Qwen3.5 hybrid text stack (BASELINE config 5, SURVEY.md section 8 row a24): the row / elementwise / recurrence kernels of
+// Qwen3.5 hybrid text stack: the row / elementwise / recurrence kernels of
 // FusedGatedDeltaNet and MRoPEGatedAttention.  All HBM- or latency-bound; the dense contractions of these layers run on
 // gemm.hip and attention_generic.hip.
 //

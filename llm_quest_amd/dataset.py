@@ -1,4 +1,4 @@
-"""Input pipeline on the step's left edge (SURVEY.md section 8 row f3) -- batch contract of ``MultimodalDataset``
+"""Input pipeline on the step's left edge -- batch contract of ``MultimodalDataset``
 (llm_quest/dataset.py:295-383) with the per-sample arithmetic on HIP kernels.
 
 Upstream does, per sample on the host: PIL resize to (image_size, image_size) (bilinear), ``ToTensor``, ImageNet ``Normalize``,

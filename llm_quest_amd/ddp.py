@@ -1,6 +1,6 @@
 """Data-parallel gradient exchange: one process per GPU, RCCL all-reduce over xGMI overlapped with backward.
 
-The reference has no distributed code at all; BASELINE's north star adds exactly one strategy:
+The reference has no distributed code at all; this package adds exactly one strategy:
 pure data parallelism over one 8 x MI355X node.  Design:
 
   * every rank holds a full replica and an independent micro-batch shard (weak scaling);
@@ -33,7 +33,7 @@ and 160 x 512 it is 0.17 GB against 0.31 GB (split).  Without a token count (``b
 with one 16-byte all-reduce (MIN / MAX of T, on a control stream of its own) and raises on EVERY rank instead of hanging in ``all_gather_into_tensor``.
 All ranks must either pass a count or pass none.
 
-Bucket groups and GEMM windows (round 5).  The compute stream's large NT GEMMs run on a persistent kernel -- one workgroup per CU for the launch's whole length,
+Bucket groups and GEMM windows.  The compute stream's large NT GEMMs run on a persistent kernel -- one workgroup per CU for the launch's whole length,
 all 256 starting together -- and a collective's channels are workgroups that hold CUs: a persistent launch beside a collective lasts up to twice as long, the per-tile
 form of the same kernel loses 17-27 % (tools/contention.py).  So the block buckets go out in GROUPS of ``MI355_DDP_BUCKET_BLOCKS`` (default 7: four groups for the 28
 blocks; the collectives of a group run back to back on the communication stream from the moment its last block is complete), and behind each group the compute stream
@@ -41,7 +41,7 @@ runs a WINDOW: its next ``MI355_DDP_WINDOW_LAUNCHES`` (default 2) persistent-siz
 dgrad GEMMs of the following block, ~2.2 ms against ~1.3 ms of ring all-reduce for 7 x 31.5 MB on eight ranks -- then the compute stream waits for the group's
 completion event (a bound on the worst case, not a stall in the normal one) and the persistent kernel is back.  Five windows per step instead of a whole backward on
 the slower kernel; ``kernels._WINDOW.stats`` counts both kinds of launch and ``bench.py`` prints them for N > 1.
-The window's length is MEASURED, not assumed (round 6): every group's collectives are bracketed by two events on the communication stream, every window by two on the
+The window's length is MEASURED, not assumed: every group's collectives are bracketed by two events on the communication stream, every window by two on the
 compute stream; ``begin_step`` reads the pairs that have completed and sets ``window_launches = ceil(slowest group's all-reduce / one windowed launch)`` (1..16), so on
 a slower fabric, more ranks or another node count the windows grow with the collectives instead of the compute stream stalling at their end (``window_for``;
 ``MI355_DDP_WINDOW_LAUNCHES`` pins the length, ``MI355_DDP_WINDOW_WAIT=0`` drops the bound at a window's end altogether).
@@ -73,7 +73,7 @@ def init_from_env(backend=None):
     local = int(os.environ.get("LOCAL_RANK", "0"))
     if world > 1 and not dist.is_initialized():
         # RCCL's collectives are kernels: each channel is one workgroup on one CU, taken from the compute stream's GEMMs (whose 256x256 tiles run one
-        # 8-wave workgroup per CU and size their grids for 256 free CUs: DESIGN.md section 6).  MI355_RCCL_CHANNELS caps / pins that number for A/B
+        # 8-wave workgroup per CU and size their grids for 256 free CUs).  MI355_RCCL_CHANNELS caps / pins that number for A/B
         # runs on an 8-GPU node (it sets NCCL_MIN_NCHANNELS / NCCL_MAX_NCHANNELS, which RCCL reads at communicator creation); unset = RCCL's own choice.
         ch = os.environ.get("MI355_RCCL_CHANNELS")
         if ch:
@@ -320,7 +320,7 @@ class GradSync:
         """all_gather_into_tensor needs the same count on every rank.  One 16-byte MAX all-reduce of (T, -T), EVERY step that passes a token count (whatever this
         rank's byte rule says: the check itself must be collective).  With RCCL it runs on a control stream of its own and the host does NOT wait for it here: the
         result stays on the device until ``_verify_tokens`` reads it -- in front of the step's first bucket hand-off, i.e. before any collective whose shape depends
-        on the split decision, and by then long complete -- so a step has no host synchronisation in ``begin_step`` (round 5 read it back at once)."""
+        on the split decision, and by then long complete -- so a step has no host synchronisation in ``begin_step``."""
         if self.backend == "nccl":
             dev = self._device()
             if self._ctl_stream is None:
@@ -468,7 +468,7 @@ def sync_for_vlm(vlm_model, adapter):
 
 
 def sync_for_qwen35(vlm):
-    """GradSync for ``Qwen3_5VLM`` / ``Qwen3_5TextModel`` (BASELINE config 5): the text blocks' bf16 arenas fire last -> first during
+    """GradSync for ``Qwen3_5VLM`` / ``Qwen3_5TextModel``: the text blocks' bf16 arenas fire last -> first during
     backward, the embedding / head arena and every parameter outside an arena (fp32 GDN parameters, the fp32 vision tower) follow in
     ``finish_step``."""
     lm = getattr(vlm, "language_model", vlm)

@@ -1,7 +1,7 @@
 """Train / eval engine -- API of ``llm_quest/engine.py`` (same function names, arguments and return values).
 
 Host-side control flow only; everything per-batch on the device goes through the HIP kernels.  Models that are plain
-PyTorch modules on the CPU (BASELINE config 1: GPT-2 plumbing) run through the same loops unchanged.
+PyTorch modules on the CPU (GPT-2 plumbing) run through the same loops unchanged.
 """
 
 import math
@@ -276,7 +276,7 @@ def profile_training_eval_loop(train_loader, val_loader, model, optimizer, num_e
     """A short training run under ``torch.profiler`` (reference: engine.py:499-640): inline linear warm-up / cosine schedule
     over ``len(train_loader) * num_epoch`` steps, one optimizer step per batch with clip 1.0, eval every ``eval_freq`` steps,
     and an early stop once ``wait + warmup + active`` steps were traced.  Kernel-level numbers for the HIP path come from
-    rocprofv3 (DESIGN.md); this entry gives the host-side timeline the reference's users expect."""
+    rocprofv3; this entry gives the host-side timeline the reference's users expect."""
     import os
 
     from torch.profiler import ProfilerActivity, profile

@@ -1,6 +1,6 @@
 """Fingerprint of the kernel sources the headline step runs: the csrc/*.hip files the step launches, their shared headers, and the compile
 flags those files are built with (the ``CXXFLAGS`` / ``FLAGS_<file>`` lines of csrc/Makefile -- NOT the Makefile as a whole: adding an
-unrelated source to ``SRCS`` must not invalidate the counters of kernels that did not change, which is what cost round 3 its ``traffic``).
+unrelated source to ``SRCS`` must not invalidate the counters of kernels that did not change).
 
 Counter files under ``profiles/`` are taken in separate ``rocprofv3 --pmc`` passes and committed; each carries the fingerprint of the
 sources it was measured on, written ON THE GPU BOX AT COLLECTION TIME (``tools/collect_evidence.sh`` -> ``stamp.json`` beside the raw

@@ -1,4 +1,4 @@
-"""Text generation loops -- API of ``llm_quest/generate.py`` for the paths on SURVEY.md section 8 row f4: ``generate_loop``
+"""Text generation loops -- API of ``llm_quest/generate.py`` for the paths below: ``generate_loop``
 (full re-forward per token), ``generate_loop_kv_cache`` (prefill + one-token decode steps through ``KVCache``) and ``sampling``.
 
 Greedy sampling (``temp == 0``, the default) is a HIP kernel (first index of the row maximum).  Stochastic sampling (temperature /

@@ -1,4 +1,4 @@
-"""GPT-2 plumbing model for BASELINE config 1 (CPU forward, batch 4 x seq 128) -- API of ``llm_quest/gpt/gpt_model.py``.
+"""GPT-2 on the CPU (forward, batch 4 x seq 128) -- API of ``llm_quest/gpt/gpt_model.py``.
 
 Config 1 is explicitly a host-side smoke test of the boundary ("plumbing, no GPU"), so this model is plain PyTorch and
 is NOT part of the HIP hot path; it exists so the engine / VLM loops can be exercised end to end without a GPU (the

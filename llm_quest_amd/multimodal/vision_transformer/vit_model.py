@@ -81,8 +81,8 @@ def tower_precision(vit):
     """Arithmetic of the FROZEN tower's hidden states (``ViTModel(images, output_hidden_states=True)`` without grad: the vision half of the early-fusion
     step).  "fp32": what the reference computes there (multimodal/vlm_engine.py:99-104 calls the ViT outside autocast) -- split-bf16 GEMMs + exact-fp32
     attention, hidden states within 1e-4 of the fp32 reference; "bf16": bf16 MFMA operands with an fp32 residual stream (the dtype flow of the
-    reference's ViT TRAINING path under autocast, SURVEY 9.17), hidden states within ~1e-2.  Per model (``vit.tower_precision = ...``) or
-    ``MI355_VIT_TOWER``; DESIGN.md section 4 has the measured price of each."""
+    reference's ViT TRAINING path under autocast), hidden states within ~1e-2.  Per model (``vit.tower_precision = ...``) or
+    ``MI355_VIT_TOWER``."""
     import os
 
     val = getattr(vit, "tower_precision", None) or os.environ.get("MI355_VIT_TOWER", DEFAULT_TOWER_PRECISION)
@@ -111,7 +111,7 @@ class ViTModel(nn.Module):
         from llm_quest_amd.multimodal.vision_transformer import vit_train
 
         if vit_train.needs_training_path(self):
-            # trainable ViT (BASELINE config 2): one autograd node, bf16 logits as under the reference's autocast
+            # trainable ViT: one autograd node, bf16 logits as under the reference's autocast
             return vit_train.run_train(self, x, output_hidden_states)
         b = x.shape[0]
         pe = self.patch_embedding

@@ -1,6 +1,6 @@
-"""ViT forward+backward on HIP kernels (BASELINE config 2: ViT-Base/16 fwd+bwd in bf16).
+"""ViT forward+backward on HIP kernels (ViT-Base/16 fwd+bwd in bf16).
 
-Dtype flow = the reference under ``torch.autocast(bf16)`` (SURVEY.md section 9.17): fp32 master parameters and fp32 residual
+Dtype flow = the reference under ``torch.autocast(bf16)``: fp32 master parameters and fp32 residual
 stream, bf16 MFMA operands (weights cast once per step, LayerNorm outputs written as bf16), bf16 logits.  The whole
 encoder is ONE autograd node: forward keeps what backward needs (28 KB per token per layer), backward runs the dgrad /
 wgrad GEMMs, flash-attention backward (non-causal, D=64), exact-GELU and LayerNorm(sigma+eps) backward kernels and writes

@@ -142,7 +142,7 @@ class ViTTransformerBlock(nn.Module):
         if self.training and (self.dropout.p > 0 or self.att.dropout.p > 0):
             raise RuntimeError("ViTTransformerBlock.run_f32 is the frozen tower's inference path: call .eval() (dropout is active)")
         att, ffn = self.att, self.ffn
-        # (round 6: the LayerNorms and the GELU projection write their fp32 results as split operands themselves -- K.split3 of an fp32 tensor reads 4 and writes
+        # (the LayerNorms and the GELU projection write their fp32 results as split operands themselves -- K.split3 of an fp32 tensor reads 4 and writes
         # 6 bytes per element, 20 GB per step at the bench's batch; only the attention's context still takes the separate pass)
         ctx = att.context_f32(self.ln_1.normalize(x2d, "split3"), B, S)
         x2 = K.gemm(L.GEMM_NT, K.split3(ctx), split3_cached(att, "wo3", [att.out_proj.weight]), bias=att.out_proj.bias.detach(), residual=x2d, out_dtype=F32)

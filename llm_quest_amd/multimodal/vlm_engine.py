@@ -1,7 +1,7 @@
 """Early-fusion VLM train / eval step -- API of ``llm_quest/multimodal/vlm_engine.py``.
 
-The reference wires ViT -> adapter -> GPT-2 (vlm_engine.py:44-164); BASELINE config 4 composes the same step with
-Qwen3-0.6B as the language model (SURVEY.md section 8c).  Both work here:
+The reference wires ViT -> adapter -> GPT-2 (vlm_engine.py:44-164); the vision-language configuration composes the same step with
+Qwen3-0.6B as the language model.  Both work here:
   * an LLM exposing ``forward_hidden`` / ``lm_loss`` (llm_quest_amd Qwen3Model) takes the FAST path: fused embeddings
     are assembled by strided HIP copies, the decoder runs on the fused sequence with causal | ~key_mask, and the tied LM
     head + cross entropy run only on the rows that feed the loss (positions n_vision-1 .. S-2);

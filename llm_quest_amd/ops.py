@@ -1,6 +1,6 @@
 """Autograd layer over the HIP kernels.
 
-Design (MI355X-first, see DESIGN.md):
+Design (MI355X-first):
   * activations are token-major 2-D bf16 tensors [B*S, width]; heads are never transposed in HBM;
   * one ``torch.autograd.Function`` per transformer block (not per op): forward enqueues ~10 kernels, backward ~20,
     so the autograd graph has ~30 nodes per step and Python overhead stays far below the GPU time;

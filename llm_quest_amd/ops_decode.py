@@ -1,4 +1,4 @@
-"""Inference with a KV cache through Qwen3 (SURVEY.md section 8 row f4): ``Qwen3Model.forward(x, kv_cache=...)`` as
+"""Inference with a KV cache through Qwen3: ``Qwen3Model.forward(x, kv_cache=...)`` as
 ``generate_loop_kv_cache`` drives it (llm_quest/generate.py:97-151, qwen3_attention.py:117-146).
 
 Two shapes of call, both without autograd:
@@ -551,7 +551,7 @@ def q35_mixer_cached(att, arena, h1, st, i):
     v = proj[:, QG + KV :]
     had_rows = cache.kv_cache.start_pos > 0
     kc, vc, end = cache.append_kv_rows(k, v, i, B, S)
-    if decode:  # every cached key is visible: causal for the newest query, and upstream un-masks padded keys (SURVEY 9.6)
+    if decode:  # every cached key is visible: causal for the newest query, and upstream un-masks padded keys
         ctx = attn_decode(q, kc, vc, end, H, G, D)
     else:
         if had_rows:

@@ -1,4 +1,4 @@
-"""Autograd layer of the Qwen3.5 hybrid text stack (BASELINE config 5, SURVEY.md section 8 row a24) over the HIP kernels.
+"""Autograd layer of the Qwen3.5 hybrid text stack over the HIP kernels.
 
 Same design as ``ops.py``: token-major 2-D bf16 activations, ONE autograd node per transformer block, every linear layer of a
 half-block fused into a single projection GEMM whose column blocks the row kernels address in place (no splits, no head

@@ -1,4 +1,4 @@
-"""AdamW on parameter arenas (SURVEY.md section 8 row f1: optimizer / clip on device).
+"""AdamW on parameter arenas (optimizer / clip on device).
 
 The reference's step is ``clip_grad_norm_(params, 1.0)`` followed by ``torch.optim.AdamW.step()`` (engine.py:441-450): a
 foreach chain over ~310 tensors.  Here the parameters of a transformer block are one flat buffer (llm_quest_amd/arena.py), so

@@ -1,6 +1,6 @@
 """Dense Qwen3 model on HIP kernels -- API of ``llm_quest/qwen/qwen3/qwen3_model.py`` (Qwen3Model).
 
-Extensions over the reference signature (both needed by BASELINE config 4):
+Extensions over the reference signature (both needed by the vision-language model):
   * ``forward(..., input_embedded=False)``: ``x`` may already be embeddings (b, s, emb) -- the early-fusion entry that
     upstream only has on GPTModel (gpt_model.py:43-51);
   * ``forward_hidden`` / ``lm_loss``: the engine's fast path -- final-normed hidden states, then the tied LM head and
@@ -109,7 +109,7 @@ class Qwen3Model(nn.Module):
 
     def forward(self, x, attn_mask=None, kv_cache=None, position_ids=None, input_embedded=False):
         """Logits (b, s, vocab) in the model dtype (reference: qwen3_model.py:60-94)."""
-        if kv_cache is not None:  # inference: prefill / one-token decode through utils.KVCache (SURVEY.md section 8 row f4)
+        if kv_cache is not None:  # inference: prefill / one-token decode through utils.KVCache
             from llm_quest_amd import ops_decode
 
             return ops_decode.qwen3_forward_cached(self, x, kv_cache, attn_mask, position_ids, input_embedded)

@@ -1,4 +1,4 @@
-"""Hugging Face -> this package's parameter names for Qwen3 (SURVEY.md section 8 row f2; API of
+"""Hugging Face -> this package's parameter names for Qwen3 (API of
 ``llm_quest/qwen/qwen3/qwen3_weight_loading.py``; the shared helpers live in ``llm_quest_amd/utils.py`` as upstream's do in ``utils.py``).
 
 There is no network on the build / GPU boxes, so the download step is replaced by a local source: a dict of tensors or a
@@ -30,7 +30,7 @@ def get_remapping_rules(model_cfg):
     if not model_cfg["tie_embeddings"]:
         rules.append(("lm_head.weight", "out_head.weight"))
     if model_cfg.get("model_type", "dense") == "moe":
-        raise NotImplementedError("MoE checkpoints are outside this package's scope (DESIGN.md section 7)")
+        raise NotImplementedError("MoE checkpoints are outside this package's scope")
     rules += [
         (".mlp.gate_proj.weight", ".ffn.lin_gate.weight"),
         (".mlp.up_proj.weight", ".ffn.lin1.weight"),

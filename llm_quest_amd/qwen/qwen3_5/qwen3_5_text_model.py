@@ -1,8 +1,8 @@
-"""Qwen3.5 hybrid text model on HIP kernels -- API of ``llm_quest/qwen/qwen3_5/qwen3_5_text_model.py`` (
-SURVEY.md section 8 row a24): ``FusedGatedDeltaNet``, ``MRoPEGatedAttention``, ``Qwen3_5TransformerBlock``, ``Qwen3_5TextModel``
+"""Qwen3.5 hybrid text model on HIP kernels -- API of ``llm_quest/qwen/qwen3_5/qwen3_5_text_model.py``:
+``FusedGatedDeltaNet``, ``MRoPEGatedAttention``, ``Qwen3_5TransformerBlock``, ``Qwen3_5TextModel``
 with the reference's constructor keys, forward signatures and ``state_dict`` keys.
 
-One autograd node per block (llm_quest_amd/ops_q35.py).  ``cache=Qwen3_5Cache`` decodes through ``ops_decode`` (SURVEY.md section 8 f4) at every level
+One autograd node per block (llm_quest_amd/ops_q35.py).  ``cache=Qwen3_5Cache`` decodes through ``ops_decode`` at every level
 the reference takes it: the model (``qwen35_forward_cached``), a block, or a token mixer called on its own (``q35_block_cached`` / ``q35_mixer_cached``:
 the same kernels, so the layers composed by hand equal the model bit for bit).  Extensions as on Qwen3Model: ``forward_hidden`` / ``lm_loss`` (LM head + cross entropy on
 just the rows that feed the loss).

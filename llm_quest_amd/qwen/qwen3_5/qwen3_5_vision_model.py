@@ -1,4 +1,4 @@
-"""Qwen3.5 vision tower on HIP kernels -- API of ``llm_quest/qwen/qwen3_5/qwen3_5_vision_model.py`` (BASELINE config 5).
+"""Qwen3.5 vision tower on HIP kernels -- API of ``llm_quest/qwen/qwen3_5/qwen3_5_vision_model.py``.
 
 Same class names, constructor-dict keys, ``forward`` signatures and state_dict keys as the reference (``patch_embed.conv_proj``,
 ``pos_embed``, ``blocks.N.{norm1,norm2,att.qkv,att.proj,ffn.lin1,ffn.lin2}``, ``merge_adapter.{norm,lin1,lin2}``).  Dtype flow as for

@@ -1,6 +1,6 @@
 """Qwen3.5 multimodal wrapper pieces on HIP kernels -- API of ``llm_quest/qwen/qwen3_5/qwen3_5_vlm_model.py``.
 
-the vision tower, the masked-scatter early fusion, the 3-D MRoPE position
+The vision tower, the masked-scatter early fusion, the 3-D MRoPE position
 ids and the hybrid text stack (``Qwen3_5TextModel``: gated delta net + gated attention) all run on HIP kernels.  ``language_model``
 may still be passed in (anything with ``emb_dict`` and the reference's ``forward(inputs_embs=..., position_ids=..., attn_mask=...)``).
 """

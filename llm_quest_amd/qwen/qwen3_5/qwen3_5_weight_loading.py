@@ -1,4 +1,4 @@
-"""Hugging Face -> this package's parameter names for Qwen3.5, text stack and vision tower (SURVEY.md section 8 row f2; API of
+"""Hugging Face -> this package's parameter names for Qwen3.5, text stack and vision tower (API of
 ``llm_quest/qwen/qwen3_5/qwen3_5_weight_loading.py:22-178``).
 
 As for Qwen3 (``qwen3_weight_loading.py`` next door) the hub download is replaced by a local source: a dict of tensors, a

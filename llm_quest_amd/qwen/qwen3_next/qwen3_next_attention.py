@@ -1,5 +1,5 @@
 """Qwen3-Next attention pieces on HIP kernels -- API of ``llm_quest/qwen/qwen3_next/qwen3_next_attention.py`` as far as the
-Qwen3.5 text stack uses it (BASELINE config 5, SURVEY.md section 8 row a24): ``ZeroCenteredRMSNorm``, ``l2_norm``,
+Qwen3.5 text stack uses it: ``ZeroCenteredRMSNorm``, ``l2_norm``,
 ``compute_alpha_factor``, ``gated_delta_rule`` and ``GatedAttention``.  Same constructor keys, attribute names and
 ``state_dict`` keys as upstream; GPU tensors only (no CPU fallback)."""
 
