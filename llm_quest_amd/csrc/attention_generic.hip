@@ -244,19 +244,19 @@ __device__ __forceinline__ void heavy_first(int& blk, int& hkv, int& b) {
     hkv = bh % (int)gridDim.y, b = bh / (int)gridDim.y;
 }
 
-// Query-major passes: an item is (query head of the group, 32 queries), heads fastest; a wave takes an item, a workgroup four neighbours -- the four heads of a group at one
-// query tile, where a group has four -- that share every key / value tile.  Two stages of tiles, and a third tile on its way in registers under the products.
+// Query-major passes: an item is (query head of the group, 32 queries), heads fastest; a wave takes an item, a workgroup `per` neighbours, four as a rule -- the four heads of a group at
+// one query tile, where a group has four -- that share every key / value tile.  Two stages of tiles, and a third tile on its way in registers under the products.
 struct QItem {
     int h, q0, ntiles, b, hkv;
     bool on;
 };
-__device__ __forceinline__ QItem query_item(int S, int rep, bool all_keys, int wave) {
+__device__ __forceinline__ QItem query_item(int S, int rep, bool all_keys, int wave, int per = 4) {  // per: items of a workgroup
     QItem it;
     int blk;
     heavy_first(blk, it.hkv, it.b);
     blk = (int)gridDim.x - 1 - blk;
-    const int nqt = (S + 31) / 32, items = rep * nqt, i = blk * 4 + wave, last = min(blk * 4 + 3, items - 1);
-    it.on = i < items;
+    const int nqt = (S + 31) / 32, items = rep * nqt, i = blk * per + wave, last = min(blk * per + per - 1, items - 1);
+    it.on = wave < per && i < items;
     const int c = it.on ? i : items - 1;
     it.h = it.hkv * rep + c % rep, it.q0 = c / rep * 32;
     it.ntiles = all_keys ? nqt : last / rep + 1;
@@ -267,12 +267,12 @@ template <int D, bool PLAIN, bool DROP>
 __global__ __launch_bounds__(256) void ga_fwd_kernel(int B, int S, int Hq, int Hkv, const bf16_t* __restrict__ q, int64_t ldq,
                                                      const bf16_t* __restrict__ k, int64_t ldk, const bf16_t* __restrict__ v, int64_t ldv,
                                                      bf16_t* __restrict__ o, int64_t ldo, float* __restrict__ lse,
-                                                     const uint8_t* __restrict__ key_mask, float scale_log2, DropArgs da) {
+                                                     const uint8_t* __restrict__ key_mask, float scale_log2, DropArgs da, int per) {
     using C = GA<D>;
     __shared__ __attribute__((aligned(1024))) char smem[4 * C::IMG];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const bool all_keys = PLAIN ? !da.causal : key_mask != nullptr;  // every key tile is walked
-    const QItem it = query_item(S, Hq / Hkv, all_keys, wave);
+    const QItem it = query_item(S, Hq / Hkv, all_keys, wave, per);
     const int query = it.q0 + (lane & 31);
     const bool qvalid = it.on && query < S;
     const int64_t tok0 = (int64_t)it.b * S;
@@ -563,7 +563,14 @@ __global__ __launch_bounds__(256) void ga_bwd_dkv_kernel(int B, int S, int Hq, i
     store_t_tiles<C::DT>(acc, 1.f, second ? dk + (tok0 + key) * lddk + (int64_t)hkv * D : dv + (tok0 + key) * lddv + (int64_t)hkv * D, kvalid, lane);
 }
 
-dim3 query_grid(int B, int S, int Hq, int Hkv) { return dim3((Hq / Hkv * ((S + 31) / 32) + 3) / 4, Hkv, B); }
+dim3 query_grid(int B, int S, int Hq, int Hkv, int per = 4) { return dim3((Hq / Hkv * ((S + 31) / 32) + per - 1) / per, Hkv, B); }
+// Items of a workgroup in the forward pass: four waves on a CU share its LDS, so while CUs are without a workgroup an item has one of its own (its other three waves fetch), or two have.  us with 1 / 2 / 4,
+// head dim 256, 8 heads over 2: 20 tokens 6.9 / 7.9 / 9.8, 333 23 / 24 / 26, 2 000 (504 items) 119 / 108 / 111, 3 x 708 (552) 58 / 45 / 47; 8 x 708 (1 472) 137 / 81 / 51.  Heads of 32 and 64
+// gain nothing from two (2 000 tokens, 8 heads of 32 over 2: 47 / 50 / 48).
+int items_per_workgroup(int B, int S, int Hq, int Hkv, int D) {
+    const int64_t items = (int64_t)Hq / Hkv * ((S + 31) / 32), groups = (int64_t)Hkv * B;
+    return items * groups <= 256 ? 1 : D >= 128 && (items + 1) / 2 * groups <= 256 ? 2 : 4;
+}
 
 int check_ga(int B, int S, int Hq, int Hkv, int D, int64_t ldq, int64_t ldk, int64_t ldv, int64_t ldo) {
     MI355_REQUIRE(B > 0 && S > 0 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0, "attn_generic: query heads (%d) must be a multiple of kv heads (%d)", Hq, Hkv);
@@ -583,9 +590,10 @@ extern "C" int mi355_attn_generic_fwd(int B, int S, int Hq, int Hkv, int D, cons
 #define GA_DROP false
     if (check_ga(B, S, Hq, Hkv, D, ldq, ldk, ldv, ldo)) return 1;
     MI355_REQUIRE(q && k && v && o && lse, "attn_generic_fwd: null pointer");
-    const dim3 grid = query_grid(B, S, Hq, Hkv);
+    const int per = items_per_workgroup(B, S, Hq, Hkv, D);
+    const dim3 grid = query_grid(B, S, Hq, Hkv, per);
     const DropArgs da = {};
-#define LAUNCH(DD) ga_fwd_kernel<DD, false, GA_DROP><<<grid, 256, 0, ST(stream)>>>(B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (bf16_t*)o, ldo, lse, key_mask, scale * LOG2E, da)
+#define LAUNCH(DD) ga_fwd_kernel<DD, false, GA_DROP><<<grid, 256, 0, ST(stream)>>>(B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (bf16_t*)o, ldo, lse, key_mask, scale * LOG2E, da, per)
     switch (D) {
         case 32: LAUNCH(32); break;
         case 64: LAUNCH(64); break;
@@ -641,8 +649,9 @@ extern "C" int mi355_attn_dropout_fwd(int B, int S, int Hq, int Hkv, int D, cons
     MI355_REQUIRE(q && k && v && o && lse, "attn_dropout_fwd: null pointer");
     DropArgs da;
     if (make_drop_args("attn_dropout_fwd", B, S, Hq, causal, p, seed, offset, &da)) return 1;
-    const dim3 grid = query_grid(B, S, Hq, Hkv);
-#define LAUNCH(DD) ga_fwd_kernel<DD, true, true><<<grid, 256, 0, ST(stream)>>>(B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (bf16_t*)o, ldo, lse, nullptr, scale * LOG2E, da)
+    const int per = items_per_workgroup(B, S, Hq, Hkv, D);
+    const dim3 grid = query_grid(B, S, Hq, Hkv, per);
+#define LAUNCH(DD) ga_fwd_kernel<DD, true, true><<<grid, 256, 0, ST(stream)>>>(B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (bf16_t*)o, ldo, lse, nullptr, scale * LOG2E, da, per)
     switch (D) {
         case 32: LAUNCH(32); break;
         case 64: LAUNCH(64); break;
@@ -688,8 +697,9 @@ extern "C" int mi355_attn_generic_dropout_fwd(int B, int S, int Hq, int Hkv, int
     MI355_REQUIRE(q && k && v && o && lse, "attn_generic_dropout_fwd: null pointer");
     DropArgs da;
     if (make_drop_args("attn_generic_dropout_fwd", B, S, Hq, 1, p, seed, offset, &da)) return 1;
-    const dim3 grid = query_grid(B, S, Hq, Hkv);
-#define LAUNCH(DD) ga_fwd_kernel<DD, false, GA_DROP><<<grid, 256, 0, ST(stream)>>>(B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (bf16_t*)o, ldo, lse, key_mask, scale * LOG2E, da)
+    const int per = items_per_workgroup(B, S, Hq, Hkv, D);
+    const dim3 grid = query_grid(B, S, Hq, Hkv, per);
+#define LAUNCH(DD) ga_fwd_kernel<DD, false, GA_DROP><<<grid, 256, 0, ST(stream)>>>(B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (bf16_t*)o, ldo, lse, key_mask, scale * LOG2E, da, per)
     switch (D) {
         case 32: LAUNCH(32); break;
         case 64: LAUNCH(64); break;

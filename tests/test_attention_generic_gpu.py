@@ -8,7 +8,9 @@ BF16 = torch.bfloat16
 
 @pytest.mark.parametrize("B,S,Hq,Hkv,D,masked", [
     (1, 1, 1, 1, 256, False), (2, 31, 3, 3, 256, False), (1, 32, 4, 1, 256, False), (3, 33, 8, 2, 256, False), (1, 97, 5, 1, 256, True), (2, 160, 8, 2, 256, False),
-    (1, 333, 8, 2, 256, False), (2, 65, 4, 4, 256, True), (2, 129, 6, 2, 128, False), (1, 64, 3, 1, 64, True), (2, 95, 2, 2, 32, False)])
+    (1, 333, 8, 2, 256, False), (2, 65, 4, 4, 256, True), (2, 129, 6, 2, 128, False), (1, 64, 3, 1, 64, True), (2, 95, 2, 2, 32, False),
+    # two and four (head, query tile) pairs to a workgroup in the forward pass: from 257 pairs, and from 513 or at small heads
+    (4, 130, 16, 2, 256, False), (5, 101, 9, 3, 128, True), (20, 97, 8, 2, 256, False), (21, 70, 6, 2, 128, True), (6, 97, 12, 12, 64, False), (9, 65, 10, 2, 32, True)])
 def test_edges_of_tiles_against_64_bits(B, S, Hq, Hkv, D, masked):
     from llm_quest_amd import kernels_q35 as Q
 
