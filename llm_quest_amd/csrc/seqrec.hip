@@ -368,8 +368,11 @@ extern "C" int mi355_ragged_conv(int64_t tokens, int n_seq, int C, int taps, con
     const int64_t total = tokens * C;
     if (C % 4 == 0 && ldx % 4 == 0 && ldy % 4 == 0 && al16(x) && al16(y) && al16(state) && al16(bias) && tokens < ((int64_t)1 << 31)) {
         const dim3 grid((unsigned)tokens, (C / 4 + 255) / 256), rows_grid((unsigned)((tokens + CONV_ROWS - 1) / CONV_ROWS), grid.y);
-        // eight rows to a thread once that leaves two workgroups to a CU (700 x 6 144, 528 workgroups: 18.4 -> 15.9 us; 700 x 1 024, 88: level)
-        const bool rows = (int64_t)rows_grid.x * rows_grid.y >= 512;
+        // Eight rows to a thread once that leaves two workgroups to a CU (700 x 6 144, 528 workgroups: 18.4 -> 15.9 us; 700 x 1 024, 88: level) and what it saves -- a thread's reads of older
+        // rows and weights, seven times of eight -- is more than its longer way through them: threads x (taps - 1) from 192 000 in fp32, 288 000 in bf16.  us, a row / eight rows a thread: 5 400 x 256,
+        // 3 taps 7.8 / 9.7, 4 taps 8.7 / 10.3 (bf16 9.0 / 11.0), 8 taps 20.2 / 12.2 (15.6 / 13.7); 8 192 x 256, 4 taps 13.1 / 10.8 (10.4 / 11.1); 8 192 x 384 16.4 / 12.9 (15.3 / 12.8).
+        const int64_t threads = (int64_t)rows_grid.x * (C / 4);
+        const bool rows = (int64_t)rows_grid.x * rows_grid.y >= 512 && threads * (taps - 1) * (x_dt == MI355_DT_F32 ? 3 : 2) >= 576000;
 #define CONV_CASE(TP)                                                                                                                                          \
     case TP:                                                                                                                                                   \
         if (rows) ragged_conv_rows_kernel<TP><<<rows_grid, 256, 0, ST(stream)>>>((int)tokens, C, x, x_dt, ldx, w, row_seq, seq_off, slot, state, act, residual, y, y_dt, ldy, bias); \

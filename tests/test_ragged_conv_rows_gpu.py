@@ -6,13 +6,13 @@ pytestmark = pytest.mark.gpu
 F32 = torch.float32
 
 
-@pytest.mark.parametrize("taps", [2, 3, 4, 8])
+@pytest.mark.parametrize("C,taps", [(1028, 2), (1028, 3), (1028, 4), (1028, 8), (4100, 2), (4100, 3), (300, 4), (768, 4)])  # (4 200 x 1 028 rows of two taps, and of three in bf16, stay with a row a thread)
 @pytest.mark.parametrize("sizes", [(4097,), (1, 1, 1, 4200), (2049, 3, 8, 5, 1, 2100), (7,) * 600])
 @pytest.mark.parametrize("dtype,act,residual", [(torch.bfloat16, True, False), (F32, False, True)])
-def test_packed_rows_are_the_sequences_one_by_one(taps, sizes, dtype, act, residual):
+def test_packed_rows_are_the_sequences_one_by_one(C, taps, sizes, dtype, act, residual):
     from llm_quest_amd import kernels_seq as S
 
-    C, n = 1028, len(sizes)
+    n = len(sizes)
     T = sum(sizes)
     g = torch.Generator(device="cuda").manual_seed(T + taps)
     i32 = lambda v: torch.tensor(v, dtype=torch.int32, device="cuda")
