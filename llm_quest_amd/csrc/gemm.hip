@@ -2211,17 +2211,37 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
         __builtin_amdgcn_sched_barrier(0);
         half(a1, b1, t + 1, off0, a0, b0, t + NS);                            // t + NS goes into the stage that t has left
     }
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
-    __syncthreads();
-
     // ---- 16 rows of the wave's 64 columns at a time through LDS, to leave as whole row segments
     float* stg = reinterpret_cast<float*>(smem) + wave * 16 * STG_LD;
-    constexpr int VEC = OUT_DT == MI355_DT_BF16 ? 7 : 3;  // elements - 1 of 16 bytes
+    constexpr bool B16 = OUT_DT == MI355_DT_BF16;
+    constexpr int VEC = B16 ? 7 : 3;  // elements - 1 of 16 bytes
+    const bool slabs = !B16 && p.ksplit > 1;
     const bool vec_c = (p.ldc & VEC) == 0 && ((uintptr_t)p.C & 15) == 0, vec_r = p.R && (p.ldr & VEC) == 0 && ((uintptr_t)p.R & 15) == 0;
     const int64_t gn = n0 + wc0 + (lane & 7) * 8, gm0 = m0 + wr0 + (lane >> 3);
     const int cols = (int)min((int64_t)8, p.N - gn);
+    // What is added to the sums is requested in front: the bias once, whole residual rows 32 ahead.  Where they are used the loads stood one after the other with nothing beside the SIMD's one wave to hide
+    // them: K = 768, us, plain | bias and residual, so -> here (gemm_bf16_kernel): 1 416 x 3 072 fp32 17.7 | 36.1 -> 18.7 (22.0), bf16 15.6 | 30.8 -> 17.1 (18.6); 5 664 x 768 fp32 17.8 | 36.2 -> 18.9 (22.3).
+    const bool whole_r = vec_r && cols == 8 && !slabs;
+    u32x4 rv[3][2][B16 ? 1 : 2];
+    auto request_r = [&](int i) {
+        if (!whole_r || i >= FM) return;
+#pragma unroll
+        for (int half = 0; half < 2; ++half) {
+            const char* r = reinterpret_cast<const char*>(p.R) + (min(gm0 + i * 16 + half * 8, p.M - 1) * p.ldr + gn) * (B16 ? 2 : 4);  // (rows past the end: the last one, not stored)
+#pragma unroll
+            for (int w = 0; w < (B16 ? 1 : 2); ++w) rv[i % 3][half][w] = *reinterpret_cast<const u32x4*>(r + 16 * w);
+        }
+    };
+    float bias[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) bias[e] = p.bias && !slabs && e < cols ? p.bias[gn + e] : 0.f;
+    request_r(0);
+    request_r(1);
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __syncthreads();
 #pragma unroll
     for (int i = 0; i < FM; ++i) {
+        request_r(i + 2);
 #pragma unroll
         for (int j = 0; j < FN; ++j) *reinterpret_cast<f32x4*>(stg + (lane & 15) * STG_LD + j * 16 + (lane >> 4) * 4) = acc[i][j];
         __builtin_amdgcn_wave_barrier();
@@ -2231,7 +2251,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
             const f32x4 v0 = *reinterpret_cast<const f32x4*>(stg + ((lane >> 3) + half * 8) * STG_LD + (lane & 7) * 8);
             const f32x4 v1 = *reinterpret_cast<const f32x4*>(stg + ((lane >> 3) + half * 8) * STG_LD + (lane & 7) * 8 + 4);
             if (gm >= p.M || cols <= 0) continue;
-            if (OUT_DT == MI355_DT_F32 && p.ksplit > 1) {  // N % 8 == 0; residual and conversion: splitk_reduce_kernel
+            if (slabs) {  // N % 8 == 0; residual and conversion: splitk_reduce_kernel
                 float* slab = p.ws + ((int64_t)split * p.M + gm) * p.N + gn;
                 *reinterpret_cast<f32x4*>(slab) = v0;
                 *reinterpret_cast<f32x4*>(slab + 4) = v1;
@@ -2240,16 +2260,15 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
             float v[8] = {v0[0], v0[1], v0[2], v0[3], v1[0], v1[1], v1[2], v1[3]};
             if (p.bias) {
 #pragma unroll
-                for (int e = 0; e < 8; ++e)
-                    if (e < cols) v[e] += p.bias[gn + e];
+                for (int e = 0; e < 8; ++e) v[e] += bias[e];
             }
-            if constexpr (OUT_DT == MI355_DT_BF16) {
+            if constexpr (B16) {
                 bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + gm * p.ldc + gn;
                 const bf16_t* r = reinterpret_cast<const bf16_t*>(p.R) + gm * p.ldr + gn;
-                if (vec_r && cols == 8) {
-                    const u32x4 rv = *reinterpret_cast<const u32x4*>(r);
+                if (whole_r) {
+                    const u32x4 x = rv[i % 3][half][0];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[2 * e] += __uint_as_float(rv[e] << 16), v[2 * e + 1] += __uint_as_float(rv[e] & 0xffff0000u);
+                    for (int e = 0; e < 4; ++e) v[2 * e] += __uint_as_float(x[e] << 16), v[2 * e + 1] += __uint_as_float(x[e] & 0xffff0000u);
                 } else if (p.R) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
@@ -2265,7 +2284,10 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
             } else {
                 float* c = reinterpret_cast<float*>(p.C) + gm * p.ldc + gn;
                 const float* r = reinterpret_cast<const float*>(p.R) + gm * p.ldr + gn;
-                if (p.R) {
+                if (whole_r) {
+#pragma unroll
+                    for (int e = 0; e < 8; ++e) v[e] += __uint_as_float(rv[i % 3][half][B16 ? 0 : e >> 2][e & 3]);
+                } else if (p.R) {
 #pragma unroll
                     for (int e = 0; e < 8; ++e)
                         if (e < cols) v[e] += r[e];

@@ -96,3 +96,16 @@ def test_input_gradients_on_both_sides_of_the_rule(M, N, K):
     assert ((KK.dgrad(dy, w).double() - exact).abs() <= bound).all()
     out = torch.empty(M, N, dtype=BF16, device="cuda")
     assert torch.equal(KK.dgrad(dy, w, out=out), KK.dgrad(dy, w))
+
+
+@pytest.mark.parametrize("M,N,K,odt", [(300, 200, 320, BF16), (5100, 1000, 328, BF16), (5100, 1000, 328, F32), (129, 136, 256, F32)])
+def test_a_residual_that_the_result_overwrites(M, N, K, odt):
+    """Residual rows are read ahead of the rows that are written: the same result in place."""
+    assert L.load().mi355_gemm_nt_ring(M, N, K, 1, 0)
+    g = torch.Generator(device="cuda").manual_seed(M)
+    A, B = (torch.randn(n, K, generator=g, device="cuda").to(BF16) for n in (M, N))
+    r = torch.randn(M, N, generator=g, device="cuda").to(odt)
+    apart = product(A, B, odt, residual=r)
+    L.require_gpu(A, B, r)
+    L.call("mi355_gemm_bf16", L.GEMM_NT, M, N, K, A.data_ptr(), K, B.data_ptr(), K, r.data_ptr(), N, L.dt_code(odt), None, r.data_ptr(), N, 0, None, 0, 0)
+    assert torch.equal(r, apart)
