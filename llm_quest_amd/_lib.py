@@ -166,7 +166,7 @@ SIGNATURES = {
 # size / constant queries: no stream argument, the return value is the answer (name -> (argtypes, restype))
 QUERIES = {
     "mi355_gated_delta_rule_chunk": ([], _I),
-    "mi355_gemm_nt_ring": ([_L, _L, _L, _I, _L], _I),
+    "mi355_gemm_nt_ring": ([_L, _L, _L, _I, _I, _L], _I),
     "mi355_gated_delta_rule_bwd_workspace_bytes": ([_I, _I, _I, _I, _I], _L),
     "mi355_delta_chunked_workspace_bytes": ([_L, _I, _I, _I], _L),
     "mi355_gdr_chunked_saved_bytes": ([_I, _I, _I], _L),

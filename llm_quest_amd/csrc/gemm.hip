@@ -2539,14 +2539,16 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
-static int choose_ring(int64_t M, int64_t N, int64_t K, bool may_split, int64_t ws_bytes, int& ksplit) {
+static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
     if (nt < 6) return 0;  // the launch and the ring's filling are most of the time: K = 256 / 320 / 384 / 448 / 512, 82 shapes from 16 x 64 to 8 000 x 1 024, mean of here over Cfg128 1.04 / 1.01 / 0.99 / 0.96 / 0.94
+    // fp32 results show the length of their sums: no fewer shares than Cfg128 would take (2 000 x 1 024, K = 4 096: off by 1.7e-7 in four shares, 2.7e-7 in one)
+    const int shares = out_dtype == MI355_DT_F32 && may_split ? choose_ksplit((M + 127) / 128 * tn, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes) : 1;
     int rows = 0;
     double least = 0;
     for (int r = 128; r <= 192; r += 64) {
         const int64_t tiles = (M + r - 1) / r * tn;
-        for (int64_t ks = 1; ks * tiles <= 256 && ks <= 16 && (ks == 1 || (may_split && nt >= 32 && ks * M * N * 4 <= ws_bytes)); ++ks) {
+        for (int64_t ks = shares; ks * tiles <= 256 && ks <= 16 && (ks == 1 || (may_split && nt >= 32 && ks * M * N * 4 <= ws_bytes)); ++ks) {
             const double wgs = (double)(ks * tiles), busy = wgs <= 64 ? 0 : wgs >= 128 ? 1 : (wgs - 64) / 64;
             const double t = (r == 192 ? 4.5 : 3.5) + (double)((nt + ks - 1) / ks) * (r == 192 ? 0.6 + 0.16 * busy : 0.44 + 0.18 * busy) + (ks > 1 ? 2.5 + (double)(ks * M * N) * 8 / 4.5e6 : 0);
             if (!rows || t < least) least = t, rows = r, ksplit = (int)ks;
@@ -2555,9 +2557,9 @@ static int choose_ring(int64_t M, int64_t N, int64_t K, bool may_split, int64_t 
     return (ksplit > 1 && nt < 6 * ksplit) || (rows == 192 && ksplit > 3 && nt >= 256) ? 0 : rows;
 }
 
-extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int may_split, int64_t workspace_bytes) {
+extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {
     int ksplit = 1;
-    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(MI355_GEMM_NT, M, N, MI355_EPI_NONE) ? choose_ring(M, N, K, may_split != 0, workspace_bytes, ksplit) : 0;
+    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(MI355_GEMM_NT, M, N, MI355_EPI_NONE) ? choose_ring(M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit) : 0;
     return rows ? rows | ksplit << 8 : 0;
 }
 
@@ -2669,7 +2671,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     if (cfg == 1 && tile_hint == 0 && form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE && !split3 && ablate == 0) {
         int ksplit = 1;
         const bool may_split = workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
-        if (const int rows = choose_ring(M, N, K, may_split, workspace_bytes, ksplit)) return mi355_gemm_ring_part7(&p, out_dtype, rows, ksplit, workspace, s);
+        if (const int rows = choose_ring(M, N, K, out_dtype, may_split, workspace_bytes, ksplit)) return mi355_gemm_ring_part7(&p, out_dtype, rows, ksplit, workspace, s);
     }
     switch (cfg) {
         case 2: return mi355_gemm_part2(form, &p, out_dtype, workspace, workspace_bytes, s);
