@@ -2534,14 +2534,14 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // Tile rows (128 or 192; 0: none fits) and K shares of gemm_ring_kernel for a product of too few 256x256 tiles.  Only in ONE round of the 256 CUs: with more tiles Cfg128's two
 // workgroups per CU are the better filling (996 x 6144, K = 1024: 21 us, this kernel in two rounds 25).  The least of: the launch (3.5 us, 4.5 with 192 rows), its K-tiles (0.44 us each
 // where up to a quarter of the CUs work, 0.62 from half of them on; 192 rows 0.6 / 0.76), and for K shares -- from 32 K-tiles on, as in choose_ksplit -- the reduction's launch and bytes.
-// Not where the least is shares of fewer than six K-tiles: filling and emptying the ring is then most of it (32 rows, 2 048 x 2 048, 16 shares of two: Cfg128 12.1, here 13.8; 160 rows, eight of four 15.6 / 17.6).
-// Nor four and more shares of 256 K-tiles and more on 192 rows, whose K-tiles take 0.95 us (996 x 768, seven shares, K = 16 384 49 / 53, 32 768 78 / 88; 1 300 x 1 024, four, K = 16 384 65 / 69).
+// Both edges with weights that come from memory, as a step's do (2 500 products of 9 - 333 rows; mean of here over Cfg128): K = 256 / 320 / 384 / 512 0.95 / 0.93 / 0.88 / 0.83, shares of two to five
+// K-tiles 0.88.  (Weights that an earlier call left in the caches turn that over: K = 256 1.04, shares of two 1.01.)
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
 static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
-    if (nt < 6) return 0;  // the launch and the ring's filling are most of the time: K = 256 / 320 / 384 / 448 / 512, 82 shapes from 16 x 64 to 8 000 x 1 024, mean of here over Cfg128 1.04 / 1.01 / 0.99 / 0.96 / 0.94
+    if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
     // fp32 results show the length of their sums: no fewer shares than Cfg128 would take (2 000 x 1 024, K = 4 096: off by 1.7e-7 in four shares, 2.7e-7 in one)
     const int shares = out_dtype == MI355_DT_F32 && may_split ? choose_ksplit((M + 127) / 128 * tn, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes) : 1;
     int rows = 0;
@@ -2554,7 +2554,7 @@ static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_
             if (!rows || t < least) least = t, rows = r, ksplit = (int)ks;
         }
     }
-    return (ksplit > 1 && nt < 6 * ksplit) || (rows == 192 && ksplit > 3 && nt >= 256) ? 0 : rows;
+    return rows;
 }
 
 extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {

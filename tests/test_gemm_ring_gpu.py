@@ -29,9 +29,9 @@ def error_bound(A, B, extra):
 
 
 # one tile and parts of it; row panels of 128 and of 192 (5 100 x 1 024: 216 tiles of 192 rows, 320 of 128); the ring filled once, odd and even counts of K-tiles, a remainder in the last; K shares
-# (long K, few tiles; None: 12 shares of four K-tiles are not the ring's, one of 48, for a bias, is); 256 tiles of 192 rows where there are 128 of 256 x 256; without the ring (rows 0): more tiles than the one round, fewer K-tiles than the ring
-SIZES = [(1, 8, 328, 128), (9, 16, 400, 128), (127, 128, 448, 128), (129, 136, 320, 0), (191, 264, 392, 128), (300, 1000, 1016, 128), (61, 1024, 3072, None), (300, 1000, 3072, 128), (333, 1024, 3584, 128),
-         (5100, 1024, 328, 192), (300, 16384, 336, 192), (2000, 4096, 336, 0), (300, 16392, 336, 0), (996, 768, 1992, 128)]
+# (long K, few tiles); 256 tiles of 192 rows where there are 128 of 256 x 256; without the ring (rows 0): more tiles than the one round, fewer K-tiles than the ring
+SIZES = [(1, 8, 256, 128), (9, 16, 200, 128), (127, 128, 320, 128), (129, 136, 192, 0), (191, 264, 264, 128), (300, 1000, 1016, 128), (61, 1024, 3072, 128), (333, 1024, 3584, 128), (5100, 1024, 328, 192),
+         (300, 16384, 256, 192), (2000, 4096, 256, 0), (300, 16392, 256, 0), (996, 768, 1992, 128)]
 
 
 @pytest.mark.parametrize("M,N,K,rows", SIZES)
@@ -39,7 +39,7 @@ SIZES = [(1, 8, 328, 128), (9, 16, 400, 128), (127, 128, 448, 128), (129, 136, 3
 @pytest.mark.parametrize("bias,residual", [(False, False), (True, True), (False, True)])
 def test_against_64_bits(M, N, K, rows, odt, bias, residual):
     may_split = not bias and N % 8 == 0
-    assert (L.load().mi355_gemm_nt_ring(M, N, K, L.dt_code(odt), may_split, 128 << 20) & 255) == ((0 if may_split else 128) if rows is None else rows)
+    assert (L.load().mi355_gemm_nt_ring(M, N, K, L.dt_code(odt), may_split, 128 << 20) & 255) == rows
     g = torch.Generator(device="cuda").manual_seed(M + N + K)
     A = torch.randn(M, K, generator=g, device="cuda").to(BF16)
     B = torch.randn(N, K, generator=g, device="cuda").to(BF16)
@@ -72,8 +72,8 @@ def test_rows_that_are_not_aligned(N, ldc, lda, skip, odt):
 
 @pytest.mark.parametrize("ws", [True, False])
 def test_values_that_are_not_finite_stay_in_their_row(ws):
-    assert L.load().mi355_gemm_nt_ring(200, 256, 6144, L.dt_code(F32), ws, 128 << 20) >> 8 == (16 if ws else 1)
-    A, B = torch.ones(200, 6144, device="cuda", dtype=BF16), torch.ones(256, 6144, device="cuda", dtype=BF16)
+    assert (L.load().mi355_gemm_nt_ring(200, 256, 2048, L.dt_code(F32), ws, 128 << 20) >> 8 > 1) is ws
+    A, B = torch.ones(200, 2048, device="cuda", dtype=BF16), torch.ones(256, 2048, device="cuda", dtype=BF16)
     A[3, 5], A[150, 2047], B[100, 64] = float("nan"), float("inf"), float("inf")
     got, want = product(A, B, F32, ws=ws), A.double() @ B.double().t()
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
@@ -100,7 +100,7 @@ def test_input_gradients_on_both_sides_of_the_rule(M, N, K):
     assert torch.equal(KK.dgrad(dy, w, out=out), KK.dgrad(dy, w))
 
 
-@pytest.mark.parametrize("M,N,K,odt", [(300, 200, 400, BF16), (5100, 1000, 328, BF16), (5100, 1000, 328, F32), (129, 136, 336, F32)])
+@pytest.mark.parametrize("M,N,K,odt", [(300, 200, 320, BF16), (5100, 1000, 328, BF16), (5100, 1000, 328, F32), (129, 136, 256, F32)])
 def test_a_residual_that_the_result_overwrites(M, N, K, odt):
     """Residual rows are read ahead of the rows that are written: the same result in place."""
     assert L.load().mi355_gemm_nt_ring(M, N, K, L.dt_code(odt), 1, 0)
