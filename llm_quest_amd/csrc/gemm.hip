@@ -119,6 +119,7 @@ struct GemmParams {
     float* ad_ndl;
     int ad_S, ad_Hq;
     int split3;  // fp32 output kernels only: C is bf16 [M, 3N], the value as [hi | lo | hi] (MI355_DT_SPLIT3)
+    int fold;    // gemm_ring_kernel: K-tiles of a running sum (0: one sum over all of them)
 };
 
 __device__ __forceinline__ float gelu_erf(float x) { return x * 0.5f * (1.0f + erff(x * 0.70710678118654752440f)); }
@@ -2134,7 +2135,9 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
 // (The ring is dynamic LDS: told its size, the compiler gives the one wave per SIMD all 512 registers, half of them accumulation registers, and moves the sums back and forth -- 1.4 times
 // the time.)
 // NT form, plain epilogue (bias and residual allowed).  The same bits as gemm_bf16_kernel: every output is summed over K in the same order.
-template <int BM, int OUT_DT>
+// FOLD: the sum over K is cut every p.fold K-tiles and the cuts are added in order -- as near to 64 bits as that many shares of K, without their slabs (2 000 x 1 024, K = 4 096, fp32: 2.7e-7
+// uncut, 1.7e-7 in four).
+template <int BM, int OUT_DT, bool FOLD>
 __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     constexpr int BN = 128, NS = 4, FM = BM / 32, FN = 4;
     constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, A_PPW = A_BYTES / 4096, B_PPW = 4, PPW = A_PPW + B_PPW, STG_LD = 68;
@@ -2178,6 +2181,21 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    f32x4 tot[FOLD ? FM : 1][FOLD ? FN : 1];
+    int left = p.fold;
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < (FOLD ? FM : 0); ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) tot[i][j] += acc[i][j], acc[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+        left = p.fold;
+    };
+    if constexpr (FOLD) {
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) tot[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
+    }
     // products of one half K-tile; the reads of the next half (of K-tile t) and the requests for K-tile `next` stand between their rows, in this order: left to itself the compiler puts
     // the reads behind all products, where nothing covers them, and ten requests in a row hold the one wave of a SIMD up (the second half's requests in front of its products: 5 % more)
     auto half = [&](const bf16x8 (&a)[FM], const bf16x8 (&b)[FN], int t, int off, bf16x8 (&an)[FM], bf16x8 (&bn)[FN], int next) {
@@ -2210,6 +2228,16 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
         __builtin_amdgcn_s_barrier();                                         // ... and every wave's
         __builtin_amdgcn_sched_barrier(0);
         half(a1, b1, t + 1, off0, a0, b0, t + NS);                            // t + NS goes into the stage that t has left
+        if constexpr (FOLD) {
+            if (--left == 0) fold();
+        }
+    }
+    if constexpr (FOLD) {
+        fold();
+#pragma unroll
+        for (int i = 0; i < FM; ++i)
+#pragma unroll
+            for (int j = 0; j < FN; ++j) acc[i][j] = tot[i][j];
     }
     // ---- 16 rows of the wave's 64 columns at a time through LDS, to leave as whole row segments
     float* stg = reinterpret_cast<float*>(smem) + wave * 16 * STG_LD;
@@ -2314,8 +2342,9 @@ int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStr
     p.ws = (float*)workspace;
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * ksplit));
     constexpr int lds = 4 * (BM + 128) * 128;  // gemm_ring_kernel's NS stages
-    if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16>), grid, dim3(256), lds, s, p);
-    else hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32>), grid, dim3(256), lds, s, p);
+    if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false>), grid, dim3(256), lds, s, p);
+    else if (BM == 192 || !p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false>), grid, dim3(256), lds, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<128, MI355_DT_F32, true>), grid, dim3(256), lds, s, p);  // (192 rows: running sums do not fit the registers)
     if (ksplit > 1) launch_splitk_reduce(p, out_dtype, s);
     MI355_LAUNCH_CHECK("mi355_gemm_bf16(ring)");
     return 0;
@@ -2539,27 +2568,30 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
-static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit) {
+static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
     if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
-    // fp32 results show the length of their sums: no fewer shares than Cfg128 would take (2 000 x 1 024, K = 4 096: off by 1.7e-7 in four shares, 2.7e-7 in one)
+    // fp32 results show the length of their sums: those are no longer than Cfg128's, whose shares the workgroups of 128 rows may also take one after the other (FOLD)
     const int shares = out_dtype == MI355_DT_F32 && may_split ? choose_ksplit((M + 127) / 128 * tn, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes) : 1;
     int rows = 0;
     double least = 0;
     for (int r = 128; r <= 192; r += 64) {
         const int64_t tiles = (M + r - 1) / r * tn;
-        for (int64_t ks = shares; ks * tiles <= 256 && ks <= 16 && (ks == 1 || (may_split && nt >= 32 && ks * M * N * 4 <= ws_bytes)); ++ks) {
+        for (int64_t ks = r == 192 ? shares : 1; ks * tiles <= 256 && ks <= 16 && (ks == 1 || (may_split && nt >= 32 && ks * M * N * 4 <= ws_bytes)); ++ks) {
             const double wgs = (double)(ks * tiles), busy = wgs <= 64 ? 0 : wgs >= 128 ? 1 : (wgs - 64) / 64;
             const double t = (r == 192 ? 4.5 : 3.5) + (double)((nt + ks - 1) / ks) * (r == 192 ? 0.6 + 0.16 * busy : 0.44 + 0.18 * busy) + (ks > 1 ? 2.5 + (double)(ks * M * N) * 8 / 4.5e6 : 0);
             if (!rows || t < least) least = t, rows = r, ksplit = (int)ks;
         }
     }
+    if (rows == 192 && ksplit > 3 && nt >= 256) return 0;  // (their K-tiles take 0.95 us: 996 x 768, seven shares, K = 16 384 Cfg128 46, here 51; 1 300 x 768, six 51 / 58; 1 300 x 1 024, four 64 / 68)
+    const int64_t cuts = rows ? (shares + ksplit - 1) / ksplit : 1;
+    fold = cuts > 1 ? (int)(((nt + ksplit - 1) / ksplit + cuts - 1) / cuts) : 0;
     return rows;
 }
 
 extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {
-    int ksplit = 1;
-    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(MI355_GEMM_NT, M, N, MI355_EPI_NONE) ? choose_ring(M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit) : 0;
+    int ksplit = 1, fold;
+    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(MI355_GEMM_NT, M, N, MI355_EPI_NONE) ? choose_ring(M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit, fold) : 0;
     return rows ? rows | ksplit << 8 : 0;
 }
 
@@ -2603,7 +2635,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     p.M = M; p.N = N; p.K = K; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.ldr = ldr;
     p.epilogue = epilogue; p.tiles_m = p.tiles_n = 0; p.ksplit = 1; p.ws = nullptr; p.ablate = ablate;
     p.ad_lse = nullptr; p.ad_delta = p.ad_nl2 = p.ad_ndl = nullptr; p.ad_S = p.ad_Hq = 0;
-    p.split3 = split3;
+    p.split3 = split3, p.fold = 0;
     hipStream_t s = (hipStream_t)stream;
     int cfg = tile_hint;
     if (cfg == 0) {
@@ -2671,7 +2703,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     if (cfg == 1 && tile_hint == 0 && form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE && !split3 && ablate == 0) {
         int ksplit = 1;
         const bool may_split = workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
-        if (const int rows = choose_ring(M, N, K, out_dtype, may_split, workspace_bytes, ksplit)) return mi355_gemm_ring_part7(&p, out_dtype, rows, ksplit, workspace, s);
+        if (const int rows = choose_ring(M, N, K, out_dtype, may_split, workspace_bytes, ksplit, p.fold)) return mi355_gemm_ring_part7(&p, out_dtype, rows, ksplit, workspace, s);
     }
     switch (cfg) {
         case 2: return mi355_gemm_part2(form, &p, out_dtype, workspace, workspace_bytes, s);

@@ -113,12 +113,16 @@ def test_a_residual_that_the_result_overwrites(M, N, K, odt):
     assert torch.equal(r, apart)
 
 
-@pytest.mark.parametrize("M,N,K", [(2000, 1024, 4096), (996, 1024, 4096), (333, 1024, 3584), (700, 512, 8192), (1300, 1536, 6144), (5664, 1024, 3584)])
-def test_fp32_results_are_no_further_from_64_bits(M, N, K):
-    """A sum in fewer shares is longer and rounds more; fp32 results would show it.  The 128 x 128 kernel with its own shares (hint 1) is the measure: one per cent for the spread of a norm over half a
-    million results and more."""
+@pytest.mark.parametrize("M,N,K,shares", [(2000, 1024, 4096, 1), (996, 1024, 4096, 2), (333, 1024, 3584, 8), (700, 512, 8192, 8), (1300, 1536, 6144, 1), (5664, 1024, 3584, 1), (12, 32000, 2048, 1), (1000, 3000, 2056, 1)])
+@pytest.mark.parametrize("residual", [False, True])
+def test_fp32_results_are_no_further_from_64_bits(M, N, K, shares, residual):
+    """A sum in fewer shares is longer and rounds more; fp32 results would show it: where the ring takes fewer it cuts them in its workgroups.  The 128 x 128 kernel with its own shares (hint 1) is the
+    measure: one per cent for the spread of a norm over a third of a million results and more (a residual of their size, once added, rounds both alike)."""
+    rows = L.load().mi355_gemm_nt_ring(M, N, K, L.dt_code(F32), 1, 128 << 20)
+    assert rows >> 8 >= shares
     g = torch.Generator(device="cuda").manual_seed(M + K)
     A, B = (torch.randn(n, K, generator=g, device="cuda").to(BF16) for n in (M, N))
-    exact = A.double() @ B.double().t()
-    err = [float((product(A, B, F32, hint=h).double() - exact).norm()) for h in (0, 1)]
+    r = torch.randn(M, N, generator=g, device="cuda") if residual else None
+    exact = A.double() @ B.double().t() + (r.double() if residual else 0)
+    err = [float((product(A, B, F32, residual=r, hint=h).double() - exact).norm()) for h in (0, 1)]
     assert err[0] <= 1.01 * err[1]
