@@ -10,10 +10,10 @@
 // What bounds them: the products alone take 7 us of a forward at 8 sequences of 708 tokens, 8 heads of 256 over 2 key heads (17 700 pairs of 32 queries and 32 keys, 32 products
 // of 32 clocks each), so a pair is a chain of LDS reads, products and softmax arithmetic of one wave, and its workgroup's tiles must already be there: tiles arrive through
 // registers two ahead into two stages of swizzled LDS images, one barrier a tile, fragments four ahead of their products, masks as bits that tiles seen whole skip.
-// Workgroups are four neighbouring (head, query tile) pairs of one kv head, or 32 keys, the long ones first: at 128 queries / keys each, a key-major grid was 96 workgroups.
+// Workgroups are up to four neighbouring (head, query tile) pairs of one kv head, or 32 keys, the long ones first: at 128 queries / keys each, a key-major grid was 96 workgroups.
 // us, one tile per pair of barriers, loads exposed -> now (key-major: 1.5 times the products, to fit its accumulators -> a pair of waves, one product each):
-//     8 x 708, 8 heads of 256 over 2: forward 207 -> 52, backward 740 -> 191;  1 x 333: 45 -> 25, 231 -> 92;  2 x 1 024 with a key mask (all keys walked): 210 -> 69, 906 -> 260;
-//     3 x 100, 6 heads of 128 over 2: 17 -> 13, 65 -> 28;  2 x 77, 4 heads of 64: 12 -> 12, 22 -> 18 (the launches).
+//     8 x 708, 8 heads of 256 over 2: forward 195 -> 52, backward 729 -> 184;  1 x 333: 46 -> 22, 231 -> 91;  2 x 1 024 with a key mask (all keys walked): 193 -> 65, 858 -> 257;
+//     3 x 100, 6 heads of 128 over 2: 13 -> 8.5, 59 -> 25;  2 x 77, 4 heads of 64: 8.5 -> 6.0, 22 -> 13 (the launches).
 //
 // PLAIN = true is the second semantics built on the same kernels (mi355_attn_dropout_fwd / _bwd): softmax over all keys or
 // plain causal (no key mask, no quirk), with nn.Dropout(p) on the NORMALISED weights as ViTMultiHeadAttention applies it

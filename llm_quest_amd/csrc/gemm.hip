@@ -2134,7 +2134,7 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
 // every CU at work; alone on the chip a workgroup takes 0.44 and 0.6, its LDS reads and writes 0.4.
 // (The ring is dynamic LDS: told its size, the compiler gives the one wave per SIMD all 512 registers, half of them accumulation registers, and moves the sums back and forth -- 1.4 times
 // the time.)
-// NT form, plain epilogue (bias and residual allowed).  The same bits as gemm_bf16_kernel: every output is summed over K in the same order.
+// NT form, plain epilogue (bias and residual allowed).  The bits of gemm_bf16_kernel in as many shares of K: every output is summed over K in the same order.
 // FOLD: the sum over K is cut every p.fold K-tiles and the cuts are added in order -- as near to 64 bits as that many shares of K, without their slabs (2 000 x 1 024, K = 4 096, fp32: 2.7e-7
 // uncut, 1.7e-7 in four).
 template <int BM, int OUT_DT, bool FOLD>
