@@ -682,13 +682,12 @@ def transpose(x, out=None):
 def dgrad_transposes(M, N, Kd):
     """Whether dX [M, N] = dY [M, Kd] W is taken from a transposed copy of W by the NT form: from ``DGRAD_NT_MIN_ROWS`` rows always.
 
-    From 1 280 rows for long sums that are enough work to pay for the copy, whichever NT kernel they meet (one round of ``gemm_ring_kernel`` or, wider, 128 x 128 tiles).  us, NN / copy + NT, from 4.2e9
-    products on: K = 4 096, N = 1 024, 1 416 rows 41 / 34, 2 836 66 / 45; K = 8 192, N = 512, 1 280 rows 44 / 32; N = 4 096 168 / 122 (4 000 rows 277 / 227); K = 2 048, N = 1 024, 2 836 rows
-    39 / 25; K = 12 288, N = 6 144, 1 340 rows 397 / 299, 4 000 704 / 631.  Wider, the copy is
-    not paid back by few rows (K = 14 336, N = 7 168, 1 280 rows 411 / 435).  Below the line: K = 2 048, N = 64 15 / 18, N = 1 024, 1 280 rows 23 / 24; K = 4 096, N = 512, 1 700 rows 25.5 / 26;
-    996 rows, N = 1 024 27 / 29.  Up to 255 K-tiles of 64: beyond, the NN form divides K over the chip (K = 16 376, N = 1 024, 1 280 rows 82 / 101; 16 384, N = 4 096 206 / 243).
-    Wide outputs of short sums stay as they are (3 072 x 1 024, 2 000 rows 25 / 28)."""
-    return M >= DGRAD_NT_MIN_ROWS or (M >= 1280 and 2 * N <= Kd and N <= 6144 and 2048 <= Kd <= 16320 and M * N * Kd >= 4.2e9)
+    From 1 280 rows for long sums that are enough work to pay for the copy, whichever NT kernel they meet (one round of ``gemm_ring_kernel`` or, wider, 128 x 128 tiles).  us with the weight in memory, NN / copy
+    + NT, from 4e9 products on: K = 4 096, N = 1 024, 1 280 rows 42 / 29, 2 836 63 / 42; K = 8 192, N = 512, 1 280 rows 44 / 33; N = 4 096 165 / 116 (4 000 rows 272 / 225); K = 2 048, N = 1 024, 2 000
+    rows 28 / 26, 2 836 44 / 25; K = 14 336, N = 7 168, 1 280 rows 472 / 433, 4 000 954 / 813 (a copy of 0.2 GB).  Below that line the two are level (0.93 - 1.07), and a launch more is not: K = 2 048, N = 768,
+    1 280 rows 23 / 24; 996 rows, K = 4 096 28 / 27.  From 256 K-tiles of 64 on the NN form divides K over the chip, and few rows are its own: K = 16 384, N = 4 096, 1 280 rows 205 / 245, 2 836 520 / 402;
+    N = 1 024 72 / 73, 130 / 112.  Wide outputs of short sums stay as they are (3 072 x 1 024, 2 000 rows 25 / 28)."""
+    return M >= DGRAD_NT_MIN_ROWS or (M >= (1280 if Kd <= 16320 else 2000) and 2 * N <= Kd and 2048 <= Kd <= 16384 and M * N * Kd >= 4e9)
 
 
 def dgrad(dy, w, out=None):
