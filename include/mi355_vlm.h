@@ -88,6 +88,8 @@ int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, in
 /* Which kernel mi355_gemm_bf16 takes by itself (tile_hint 0) for the NT form with a plain epilogue: rows | K shares << 8 of the one-round ring of K-tiles (128- or 192-row tiles), 0: another one.
  * may_split: a workspace, no bias, N % 8 == 0, ldc and ldr multiples of 4. */
 int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes);
+/* The same for the NN form. */
+int mi355_gemm_nn_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes);
 
 /* Several independent GEMMs of ONE operand form in one launch, no bias / epilogue / K split.  Replaces the weight-gradient
  * half of autograd's backward for the Linear layers of one transformer block (qwen3_transformer_block.py:48-53,84-99,

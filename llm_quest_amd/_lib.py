@@ -167,6 +167,7 @@ SIGNATURES = {
 QUERIES = {
     "mi355_gated_delta_rule_chunk": ([], _I),
     "mi355_gemm_nt_ring": ([_L, _L, _L, _I, _I, _L], _I),
+    "mi355_gemm_nn_ring": ([_L, _L, _L, _I, _I, _L], _I),
     "mi355_gated_delta_rule_bwd_workspace_bytes": ([_I, _I, _I, _I, _I], _L),
     "mi355_delta_chunked_workspace_bytes": ([_L, _I, _I, _I], _L),
     "mi355_gdr_chunked_saved_bytes": ([_I, _I, _I], _L),

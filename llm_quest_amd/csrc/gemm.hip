@@ -2134,10 +2134,13 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
 // every CU at work; alone on the chip a workgroup takes 0.44 and 0.6, its LDS reads and writes 0.4.
 // (The ring is dynamic LDS: told its size, the compiler gives the one wave per SIMD all 512 registers, half of them accumulation registers, and moves the sums back and forth -- 1.4 times
 // the time.)
-// NT form, plain epilogue (bias and residual allowed).  The bits of gemm_bf16_kernel in as many shares of K: every output is summed over K in the same order.
+// NT and NN forms, plain epilogue (bias and residual allowed).  The bits of gemm_bf16_kernel in as many shares of K: every output is summed over K in the same order.
+// B_TR (NN): the column fragments come by transposing reads issued from asm, the whole half's in front of its first row of products, and each half ends with a wait for them.  gemm_bf16_kernel's NN
+// form waits for its one K-tile in flight; us with weights from memory, gemm_bf16_kernel -> here: 333 x 1 024, K = 1 024 20.3 -> 13.3, 3 584 21.5 -> 17.6; 996 x 1 024, K = 4 096 27.6 -> 22.4,
+// 6 144 46.5 -> 26.7; 996 x 4 096, K = 1 024 25.2 -> 16.0; 2 000 x 2 048, K = 2 048 52.0 -> 23.6.  With every CU at work a K-tile of 128 rows takes 0.07 us longer than in the NT form.
 // FOLD: the sum over K is cut every p.fold K-tiles and the cuts are added in order -- as near to 64 bits as that many shares of K, without their slabs (2 000 x 1 024, K = 4 096, fp32: 2.7e-7
 // uncut, 1.7e-7 in four).
-template <int BM, int OUT_DT, bool FOLD>
+template <int BM, int OUT_DT, bool FOLD, bool B_TR>
 __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     constexpr int BN = 128, NS = 4, FM = BM / 32, FN = 4;
     constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, A_PPW = A_BYTES / 4096, B_PPW = 4, PPW = A_PPW + B_PPW, STG_LD = 68;
@@ -2157,9 +2160,10 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     unsigned voffA[A_PPW], voffB[B_PPW];
     int kneedA[A_PPW], kneedB[B_PPW];
     piece_offsets<false, BM, 64, A_PPW>(wave, lane, p.lda, p.M - m0, voffA, kneedA);
-    piece_offsets<false, BN, 64, B_PPW>(wave, lane, p.ldb, p.N - n0, voffB, kneedB);
+    piece_offsets<B_TR, BN, 64, B_PPW>(wave, lane, p.ldb, p.N - n0, voffB, kneedB);
     const bf16_t* baseA = uniform_ptr(p.A + m0 * p.lda);
-    const bf16_t* baseB = uniform_ptr(p.B + n0 * p.ldb);
+    const bf16_t* baseB = uniform_ptr(B_TR ? p.B + n0 : p.B + n0 * p.ldb);
+    const int64_t stepB = B_TR ? p.ldb : 1;
     auto issue = [&](int t, int from, int to) {  // this wave's pieces [from, to) of K-tile t; past the end out of range: zeros, and the counts of the waits below hold
         const int k0 = t < n ? (t0 + t) * 64 : 0, krem = t < n ? kend - k0 : 0;
         char* dA = smem + (t & (NS - 1)) * STAGE + wave * A_PPW * 1024;
@@ -2168,7 +2172,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
         for (int j = 0; j < PPW; ++j) {
             if (j < from || j >= to) continue;
             if (j < A_PPW) dma_piece(baseA + k0, kneedA[j < A_PPW ? j : 0] < krem ? voffA[j < A_PPW ? j : 0] : OOB, dA + j * 1024);
-            else dma_piece(baseB + k0, kneedB[j < A_PPW ? 0 : j - A_PPW] < krem ? voffB[j < A_PPW ? 0 : j - A_PPW] : OOB, dB + (j - A_PPW) * 1024);
+            else dma_piece(baseB + k0 * stepB, kneedB[j < A_PPW ? 0 : j - A_PPW] < krem ? voffB[j < A_PPW ? 0 : j - A_PPW] : OOB, dB + (j - A_PPW) * 1024);
         }
     };
     const int wr0 = (wave >> 1) * (BM / 2), wc0 = (wave & 1) * 64;
@@ -2176,6 +2180,19 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     const int off0 = (lane & 15) * 128 + (swz_rowk<64>(lane >> 4, lane & 15) << 4), off1 = (lane & 15) * 128 + (swz_rowk<64>(4 + (lane >> 4), lane & 15) << 4);
     auto frag_a = [&](int t, int off, int i) { return *reinterpret_cast<const bf16x8*>(smem + (t & (NS - 1)) * STAGE + wr0 * 128 + off + i * 2048); };
     auto frag_b = [&](int t, int off, int j) { return *reinterpret_cast<const bf16x8*>(smem + (t & (NS - 1)) * STAGE + A_BYTES + wc0 * 128 + off + j * 2048); };
+    // B_TR: [64 k][128 columns]; the XOR of a lane's row reaches into the column bits, so each of the wave's four column tiles has a lane offset of its own (frag_tr)
+    unsigned offt[FN];
+#pragma unroll
+    for (int j = 0; j < FN; ++j) {
+        const int g = lane >> 4, q = (lane >> 2) & 3, chunk = ((wc0 >> 3) + 2 * j + ((lane & 3) >> 1)) ^ ((q | ((g & 1) << 2)) << 1);
+        offt[j] = (unsigned)(uintptr_t)LDS_PTR(smem) + A_BYTES + (8 * g + q) * 256 + (chunk << 4) + (lane & 1) * 8;
+    }
+    auto issue_bt = [&](TrHalves& f, int t, auto kk, int j) {  // the first (kk 0) or second half of K-tile t; read asynchronously: tr_wait_join stands at the end of the same half
+        const unsigned addr = offt[j] + (t & (NS - 1)) * STAGE;
+        asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%c3\n\tds_read_b64_tr_b16 %1, %2 offset:%c4"
+                     : "=&v"(f.lo), "=&v"(f.hi)
+                     : "v"(addr), "i"(decltype(kk)::value * 8192), "i"(decltype(kk)::value * 8192 + 1024));
+    };
     f32x4 acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
@@ -2198,17 +2215,28 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     }
     // products of one half K-tile; the reads of the next half (of K-tile t) and the requests for K-tile `next` stand between their rows, in this order: left to itself the compiler puts
     // the reads behind all products, where nothing covers them, and ten requests in a row hold the one wave of a SIMD up (the second half's requests in front of its products: 5 % more)
-    auto half = [&](const bf16x8 (&a)[FM], const bf16x8 (&b)[FN], int t, int off, bf16x8 (&an)[FM], bf16x8 (&bn)[FN], int next) {
+    auto half = [&](const bf16x8 (&a)[FM], const bf16x8 (&b)[FN], int t, auto kk, bf16x8 (&an)[FM], bf16x8 (&bn)[FN], int next) {
+        const int off = decltype(kk)::value ? off1 : off0;
+        TrHalves h[FN];
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-            if (i < 2) bn[2 * i] = frag_b(t, off, 2 * i), bn[2 * i + 1] = frag_b(t, off, 2 * i + 1);
+            if constexpr (B_TR) {  // column fragments first, and nothing requested in front of the last row of products: it covers the wait at the end
+                if (i == 0) {
+#pragma unroll
+                    for (int j = 0; j < FN; ++j) issue_bt(h[j], t, kk, j);
+                } else if (2 * i - 2 < FM) an[2 * i - 2] = frag_a(t, off, 2 * i - 2), an[2 * i - 1] = frag_a(t, off, 2 * i - 1);
+            } else if (i < 2) bn[2 * i] = frag_b(t, off, 2 * i), bn[2 * i + 1] = frag_b(t, off, 2 * i + 1);
             else if (2 * i - 4 < FM) an[2 * i - 4] = frag_a(t, off, 2 * i - 4), an[2 * i - 3] = frag_a(t, off, 2 * i - 3);
-            if (i == FM - 1 && 2 * i - 2 < FM) an[FM - 2] = frag_a(t, off, FM - 2), an[FM - 1] = frag_a(t, off, FM - 1);
+            if (!B_TR && i == FM - 1 && 2 * i - 2 < FM) an[FM - 2] = frag_a(t, off, FM - 2), an[FM - 1] = frag_a(t, off, FM - 1);
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
             for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);  // lane: four columns of row lane & 15
             if (next >= 0) issue(next, i * PPW / FM, (i + 1) * PPW / FM);
             __builtin_amdgcn_sched_barrier(0);
+        }
+        if constexpr (B_TR) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0) that the compiler sees: it knows the reads of `an` only, and would wait for them in the next half, by a count that the reads issued there have passed
+            tr_wait_join<0>(h, bn);
         }
     };
     bf16x8 a0[FM], b0[FN], a1[FM], b1[FN];
@@ -2216,18 +2244,26 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     for (int t = 0; t < NS; ++t) issue(t, 0, PPW);
     asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * PPW) : "memory");
     __builtin_amdgcn_s_barrier();
+    if constexpr (B_TR) {
+        TrHalves h[FN];
 #pragma unroll
-    for (int j = 0; j < FN; ++j) b0[j] = frag_b(0, off0, j);
+        for (int j = 0; j < FN; ++j) issue_bt(h[j], 0, std::integral_constant<int, 0>{}, j);
+        tr_wait_join<0>(h, b0);
+    } else {
+#pragma unroll
+        for (int j = 0; j < FN; ++j) b0[j] = frag_b(0, off0, j);
+    }
 #pragma unroll
     for (int i = 0; i < FM; ++i) a0[i] = frag_a(0, off0, i);
+    if constexpr (B_TR) __builtin_amdgcn_s_waitcnt(0xc07f);  // (as at the end of `half`, whose state the loop's top shares)
     for (int t = 0; t < n; ++t) {
         __builtin_amdgcn_sched_barrier(0);
-        half(a0, b0, t, off1, a1, b1, -1);
+        half(a0, b0, t, std::integral_constant<int, 1>{}, a1, b1, -1);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                    // this wave's reads of K-tile t are complete
         asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * PPW) : "memory");  // its pieces of t + 1 have landed
         __builtin_amdgcn_s_barrier();                                         // ... and every wave's
         __builtin_amdgcn_sched_barrier(0);
-        half(a1, b1, t + 1, off0, a0, b0, t + NS);                            // t + NS goes into the stage that t has left
+        half(a1, b1, t + 1, std::integral_constant<int, 0>{}, a0, b0, t + NS);                            // t + NS goes into the stage that t has left
         if constexpr (FOLD) {
             if (--left == 0) fold();
         }
@@ -2334,7 +2370,7 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     }
 }
 
-template <int BM>
+template <int BM, bool B_TR>
 int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStream_t s) {
     p.tiles_m = (int)((p.M + BM - 1) / BM);
     p.tiles_n = (int)((p.N + 127) / 128);
@@ -2342,9 +2378,9 @@ int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStr
     p.ws = (float*)workspace;
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * ksplit));
     constexpr int lds = 4 * (BM + 128) * 128;  // gemm_ring_kernel's NS stages
-    if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false>), grid, dim3(256), lds, s, p);
-    else if (BM == 192 || !p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false>), grid, dim3(256), lds, s, p);
-    else hipLaunchKernelGGL((gemm_ring_kernel<128, MI355_DT_F32, true>), grid, dim3(256), lds, s, p);  // (192 rows: running sums do not fit the registers)
+    if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR>), grid, dim3(256), lds, s, p);
+    else if (BM == 192 || !p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR>), grid, dim3(256), lds, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<128, MI355_DT_F32, true, B_TR>), grid, dim3(256), lds, s, p);  // (192 rows: running sums do not fit the registers)
     if (ksplit > 1) launch_splitk_reduce(p, out_dtype, s);
     MI355_LAUNCH_CHECK("mi355_gemm_bf16(ring)");
     return 0;
@@ -2475,11 +2511,13 @@ __global__ __launch_bounds__(256) void colsum_kernel(int64_t M, int64_t N, const
 GEMM_BRIDGE_DECL(1) GEMM_BRIDGE_DECL(2) GEMM_BRIDGE_DECL(3) GEMM_BRIDGE_DECL(4) GEMM_BRIDGE_DECL(5)
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_persist_part2(const void* params, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_pp_part6(const void* params, void* stream);
-extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_ring_part7(const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_ring_part7(int form, const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream);
 #if GEMM_PART == 7 || GEMM_PART == -1
-extern "C" int mi355_gemm_ring_part7(const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream) {
+extern "C" int mi355_gemm_ring_part7(int form, const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream) {
     const GemmParams& p = *static_cast<const GemmParams*>(params);
-    return rows == 192 ? launch_ring<192>(p, out_dtype, ksplit, ws, (hipStream_t)stream) : launch_ring<128>(p, out_dtype, ksplit, ws, (hipStream_t)stream);
+    hipStream_t s = (hipStream_t)stream;
+    if (form == MI355_GEMM_NN) return rows == 192 ? launch_ring<192, true>(p, out_dtype, ksplit, ws, s) : launch_ring<128, true>(p, out_dtype, ksplit, ws, s);
+    return rows == 192 ? launch_ring<192, false>(p, out_dtype, ksplit, ws, s) : launch_ring<128, false>(p, out_dtype, ksplit, ws, s);
 }
 #endif
 #if GEMM_PART == 6 || GEMM_PART == -1
@@ -2554,10 +2592,10 @@ static int pp_mask() {
 
 // Forward products and input gradients of fewer 256x256 tiles than half of the CUs: measured 92 tiles -> 128x128 wins (+2.8 % on the hybrid step), 180 tiles -> 256x256 wins.  At 128 tiles, plain
 // NT, nine shapes from 512 x 16 384 to 32 700 x 256, K = 512 / 1 024 / 3 584 / 7 168, us: 256x256 19 - 20 / 29 - 34 / 106 - 120 / 159 - 194, 128x128 15 / 22 - 24 / 63 - 67 / 115 - 155 (300 x 16 384,
-// which fits gemm_ring_kernel: 16 / 20 / 47 / 79).
+// which fits gemm_ring_kernel: 16 / 20 / 47 / 79).  NN at 128 tiles: 3 900 x 2 048, K = 1 024 37 / 25, 2 048 83 / 47; 2 000 x 4 096, K = 1 024 41.5 / 28; at 152 and 192 tiles 38 / 35.5 and 42 / 45.
 static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
-    return M < 256 || N < 256 || (form != MI355_GEMM_TN && tiles256 < 128 + (form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE));
+    return M < 256 || N < 256 || (form != MI355_GEMM_TN && tiles256 < 128 + (epilogue == MI355_EPI_NONE));
 }
 
 // Tile rows (128 or 192; 0: none fits) and K shares of gemm_ring_kernel for a product of too few 256x256 tiles.  Only in ONE round of the 256 CUs: with more tiles Cfg128's two
@@ -2568,7 +2606,7 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
-static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold) {
+static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
     if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
     // fp32 results show the length of their sums: those are no longer than Cfg128's, whose shares the workgroups of 128 rows may also take one after the other (FOLD)
@@ -2583,16 +2621,27 @@ static int choose_ring(int64_t M, int64_t N, int64_t K, int out_dtype, bool may_
             if (!rows || t < least) least = t, rows = r, ksplit = (int)ks;
         }
     }
+    if (form == MI355_GEMM_NN && M > 128 && nt >= 1024) return 0;  // a vocabulary-wide layer's: Cfg128 / here 197 x 1 024, K = 151 936 133 / 162, 248 320 205 / 246 (one row panel: 61 rows 184 / 147)
     if (rows == 192 && ksplit > 3 && nt >= 256) return 0;  // (their K-tiles take 0.95 us: 996 x 768, seven shares, K = 16 384 Cfg128 46, here 51; 1 300 x 768, six 51 / 58; 1 300 x 1 024, four 64 / 68)
     const int64_t cuts = rows ? (shares + ksplit - 1) / ksplit : 1;
     fold = cuts > 1 ? (int)(((nt + ksplit - 1) / ksplit + cuts - 1) / cuts) : 0;
     return rows;
 }
 
-extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {
+// input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
+// 128x128 / 256x256: K = 248 320, 333 rows 294 / 304, 602 585 / 446, 2 048 1 298 / 1 092; K = 20 000, 708 rows 54 / 57, 1 300 88 / 82; by 768, K = 50 256, 602 rows 83 / 81
+static bool long_split_nn(int64_t M, int64_t N, int64_t K, bool may_split, int64_t workspace_bytes) {
+    return may_split && !(N & 7) && workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
+}
+
+static int ring_query(int form, int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {
     int ksplit = 1, fold;
-    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(MI355_GEMM_NT, M, N, MI355_EPI_NONE) ? choose_ring(M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit, fold) : 0;
+    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(form, M, N, MI355_EPI_NONE) ? choose_ring(form, M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit, fold) : 0;
     return rows ? rows | ksplit << 8 : 0;
+}
+extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) { return ring_query(MI355_GEMM_NT, M, N, K, out_dtype, may_split, workspace_bytes); }
+extern "C" int mi355_gemm_nn_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {
+    return long_split_nn(M, N, K, may_split != 0, workspace_bytes) && ((M + 255) / 256) * ((N + 255) / 256) < 128 ? 0 : ring_query(MI355_GEMM_NN, M, N, K, out_dtype, may_split, workspace_bytes);
 }
 
 extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* B,
@@ -2650,10 +2699,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         // 256x256 tiles need at least half of the 256 CUs' worth of tiles; below that (small token counts: the hybrid model at B = 8 has 92 tiles for
         // its N = 1024 outputs) four times as many 128x128 tiles, two workgroups per CU, fill the chip instead
         const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
-        // input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
-        // 128x128 / 256x256: K = 248 320, 333 rows 294 / 304, 602 585 / 446, 2 048 1 298 / 1 092; K = 20 000, 708 rows 54 / 57, 1 300 88 / 82; by 768, K = 50 256, 602 rows 83 / 81
-        const bool long_split = form == MI355_GEMM_NN && workspace && !bias && epilogue == MI355_EPI_NONE && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3)) &&
-                                workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
+        const bool long_split = form == MI355_GEMM_NN && epilogue == MI355_EPI_NONE && long_split_nn(M, N, K, workspace && !bias && !(ldc & 3) && (!residual || !(ldr & 3)), workspace_bytes);
         if (M < 256 || N < 256) cfg = 1;
         else if (long_split && tiles256 < 128) cfg = 3;
         else if (small_tiles(form, M, N, epilogue)) cfg = 1;
@@ -2700,10 +2746,10 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         if (ok) return mi355_gemm_persist_part2(&p, s);
         cfg = 2;
     }
-    if (cfg == 1 && tile_hint == 0 && form == MI355_GEMM_NT && epilogue == MI355_EPI_NONE && !split3 && ablate == 0) {
+    if (cfg == 1 && tile_hint == 0 && form != MI355_GEMM_TN && epilogue == MI355_EPI_NONE && !split3 && ablate == 0) {
         int ksplit = 1;
         const bool may_split = workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
-        if (const int rows = choose_ring(M, N, K, out_dtype, may_split, workspace_bytes, ksplit, p.fold)) return mi355_gemm_ring_part7(&p, out_dtype, rows, ksplit, workspace, s);
+        if (const int rows = choose_ring(form, M, N, K, out_dtype, may_split, workspace_bytes, ksplit, p.fold)) return mi355_gemm_ring_part7(form, &p, out_dtype, rows, ksplit, workspace, s);
     }
     switch (cfg) {
         case 2: return mi355_gemm_part2(form, &p, out_dtype, workspace, workspace_bytes, s);

@@ -680,22 +680,33 @@ def transpose(x, out=None):
 
 
 def dgrad_transposes(M, N, Kd):
-    """Whether dX [M, N] = dY [M, Kd] W is taken from a transposed copy of W by the NT form: from ``DGRAD_NT_MIN_ROWS`` rows always.
+    """Whether dX [M, N] = dY [M, Kd] W, where the NN form does not run on the one-round ring (``dgrad_on_ring``), is taken from a transposed copy of W by the NT form: from ``DGRAD_NT_MIN_ROWS`` rows always.
 
-    From 1 280 rows for long sums that are enough work to pay for the copy, whichever NT kernel they meet (one round of ``gemm_ring_kernel`` or, wider, 128 x 128 tiles).  us with the weight in memory, NN / copy
-    + NT, from 4e9 products on: K = 4 096, N = 1 024, 1 280 rows 42 / 29, 2 836 63 / 42; K = 8 192, N = 512, 1 280 rows 44 / 33; N = 4 096 165 / 116 (4 000 rows 272 / 225); K = 2 048, N = 1 024, 2 000
+    From 1 280 rows for long sums that are enough work to pay for the copy, whichever NT kernel they meet (one round of ``gemm_ring_kernel`` or, wider, 128 x 128 tiles).  us with the weight in memory, NN (128 x 128
+    tiles) / copy + NT, from 4e9 products on: K = 4 096, N = 1 024, 1 280 rows 42 / 29, 2 836 63 / 42; K = 8 192, N = 512, 1 280 rows 44 / 33; N = 4 096 165 / 116 (4 000 rows 272 / 225); K = 2 048, N = 1 024, 2 000
     rows 28 / 26, 2 836 44 / 25; K = 14 336, N = 7 168, 1 280 rows 472 / 433, 4 000 954 / 813 (a copy of 0.2 GB).  Below that line the two are level (0.93 - 1.07), and a launch more is not: K = 2 048, N = 768,
     1 280 rows 23 / 24; 996 rows, K = 4 096 28 / 27.  From 256 K-tiles of 64 on the NN form divides K over the chip, and few rows are its own: K = 16 384, N = 4 096, 1 280 rows 205 / 245, 2 836 520 / 402;
     N = 1 024 72 / 73, 130 / 112.  Wide outputs of short sums stay as they are (3 072 x 1 024, 2 000 rows 25 / 28)."""
     return M >= DGRAD_NT_MIN_ROWS or (M >= (1280 if Kd <= 16320 else 2000) and 2 * N <= Kd and 2048 <= Kd <= 16384 and M * N * Kd >= 4e9)
 
 
+def dgrad_on_ring(M, N, Kd, dtype=BF16):
+    """Whether dX [M, N] = dY [M, Kd] W of fewer than ``DGRAD_NT_MIN_ROWS`` rows runs in the NN form on the one-round ring of K-tiles, where a copy of W no longer pays.  us with the weight in memory,
+    NN / copy + NT, N = 1 024: K = 2 048, 2 836 rows 21.5 / 24.9; K = 3 584, 1 416 rows 26.7 / 32.0; K = 8 192, 2 000 rows 46.7 / 51.1.  Its K-tiles of 128 rows are the slower ones: over long sums
+    that are not divided the copy is paid back (K = 6 144, 3 900 rows 56.2 / 56.3, 8 192 72.5 / 70.7).  Above the line it is level where it counts: 5 664 rows alone 44.8 / 48.2 (K = 3 584), in a training
+    step, at the clocks that its power leaves, the step takes as long."""
+    if M >= DGRAD_NT_MIN_ROWS or _TILE_BY_FORM[L.GEMM_NN] or _TILE_OVERRIDE:
+        return False
+    r = L.load().mi355_gemm_nn_ring(M, N, Kd, L.dt_code(dtype), 1, WS_BYTES)
+    return r != 0 and (r != (128 | 1 << 8) or Kd < 6144)
+
+
 def dgrad(dy, w, out=None):
-    """dX = dY W for a Linear with weight W [N_out, N_in].  Where ``dgrad_transposes`` says so W is transposed first (one pass over the
+    """dX = dY W for a Linear with weight W [N_out, N_in].  Where ``dgrad_transposes`` says so and ``dgrad_on_ring`` does not, W is transposed first (one pass over the
     weight, 63 MB per transformer block) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads.
     The result is the same sum in the same order per K-tile, bit-identical to the NN form where neither is split over K."""
     M, (Kd, N) = dy.shape[0], w.shape
-    if DGRAD_NT and dgrad_transposes(M, N, Kd) and (Kd & 7) == 0 and (N & 7) == 0:
+    if DGRAD_NT and dgrad_transposes(M, N, Kd) and (Kd & 7) == 0 and (N & 7) == 0 and not dgrad_on_ring(M, N, Kd, BF16 if out is None else out.dtype):
         return gemm(L.GEMM_NT, dy, transpose(w), out=out)
     return gemm(L.GEMM_NN, dy, w, out=out)
 

@@ -126,3 +126,63 @@ def test_fp32_results_are_no_further_from_64_bits(M, N, K, shares, residual):
     exact = A.double() @ B.double().t() + (r.double() if residual else 0)
     err = [float((product(A, B, F32, residual=r, hint=h).double() - exact).norm()) for h in (0, 1)]
     assert err[0] <= 1.01 * err[1]
+
+
+# ---- the NN form: one tile and parts of it, panels of 128 and of 192 rows, the ring filled once, odd and even counts of K-tiles, a remainder in the last, K shares
+NN_SIZES = [(1, 8, 256, 128), (9, 16, 200, 128), (127, 128, 320, 128), (129, 136, 192, 0), (191, 264, 264, 128), (300, 1000, 1016, 128), (61, 1024, 3072, 128), (333, 1024, 3584, 128), (5100, 1024, 328, 192),
+            (300, 16384, 256, 192), (2000, 4096, 256, 0), (996, 768, 1992, 128), (4096, 1024, 448, 128), (61, 256, 66000, 128), (197, 256, 66000, 0), (602, 128, 33000, 0)]
+
+
+@pytest.mark.parametrize("M,N,K,rows", NN_SIZES)
+@pytest.mark.parametrize("odt", [BF16, F32])
+@pytest.mark.parametrize("bias,residual", [(False, False), (True, True)])
+def test_nn_against_64_bits(M, N, K, rows, odt, bias, residual):
+    if not bias:
+        assert (L.load().mi355_gemm_nn_ring(M, N, K, L.dt_code(odt), 1, 128 << 20) & 255) == rows
+    g = torch.Generator(device="cuda").manual_seed(M + N + K)
+    A = torch.randn(M, K + 8, generator=g, device="cuda").to(BF16)[:, :K]
+    W = torch.randn(K, N + 16, generator=g, device="cuda").to(BF16)[:, 8 : N + 8]  # rows longer than the operand: nothing beside it is read into a sum
+    b = torch.randn(N, generator=g, device="cuda") if bias else None
+    r = torch.randn(M, N, generator=g, device="cuda").to(odt) if residual else None
+
+    def take(hint):
+        C, buf = torch.full((M, N + 4), 7.0, dtype=odt, device="cuda"), torch.empty(32 << 20, dtype=F32, device="cuda")
+        L.require_gpu(A, W, C, b, r, buf)
+        L.call("mi355_gemm_bf16", L.GEMM_NN, M, N, K, A.data_ptr(), A.stride(0), W.data_ptr(), W.stride(0), C.data_ptr(), C.stride(0), L.dt_code(odt), L.ptr(b), L.ptr(r), N if residual else 0, 0, buf.data_ptr(),
+               buf.numel() * 4, hint)
+        assert torch.equal(C[:, N:], torch.full_like(C[:, N:], 7.0))
+        return C[:, :N]
+
+    got, extra = take(0), (b.double() if bias else 0) + (r.double() if residual else 0)
+    exact = A.double() @ W.double() + extra
+    bound = error_bound(A, W.t(), extra.abs() if bias or residual else 0)
+    if odt == BF16:
+        bound = bound + 2.0 ** -8 * exact.abs()  # one rounding to eight bits
+    assert ((got.double() - exact).abs() <= bound).all()
+    if K < 2048:  # no K shares, or the same: every sum in the same order
+        assert torch.equal(take(1), got)
+
+
+@pytest.mark.parametrize("M,N,K", [(333, 1024, 3584), (996, 1024, 6144), (2000, 1024, 4096), (197, 768, 2304)])
+def test_nn_fp32_results_are_no_further_from_64_bits(M, N, K):
+    """As for the NT form: the 128 x 128 kernel with its own shares of K (hint 1) is the measure."""
+    assert L.load().mi355_gemm_nn_ring(M, N, K, L.dt_code(F32), 1, 128 << 20)
+    g = torch.Generator(device="cuda").manual_seed(M + K)
+    A, W = torch.randn(M, K, generator=g, device="cuda").to(BF16), torch.randn(K, N, generator=g, device="cuda").to(BF16)
+    exact, buf, err = A.double() @ W.double(), torch.empty(32 << 20, dtype=F32, device="cuda"), []
+    for hint in (0, 1):
+        C = torch.empty(M, N, device="cuda")
+        L.require_gpu(A, W, C, buf)
+        L.call("mi355_gemm_bf16", L.GEMM_NN, M, N, K, A.data_ptr(), K, W.data_ptr(), N, C.data_ptr(), N, L.dt_code(F32), None, None, 0, 0, buf.data_ptr(), buf.numel() * 4, hint)
+        err.append(float((C.double() - exact).norm()))
+    assert err[0] <= 1.01 * err[1]
+
+
+def test_nn_values_that_are_not_finite_stay_in_their_row_and_column():
+    A, W = torch.ones(200, 2048, device="cuda", dtype=BF16), torch.ones(2048, 256, device="cuda", dtype=BF16)
+    A[3, 5], A[150, 2047], W[64, 100] = float("nan"), float("inf"), float("inf")
+    from llm_quest_amd import kernels as KK
+
+    got, want = KK.gemm(L.GEMM_NN, A, W, out_dtype=F32), A.double() @ W.double()
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
+    assert torch.equal(got[torch.isfinite(got)], want[torch.isfinite(want)].float())
