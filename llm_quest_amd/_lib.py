@@ -5,6 +5,7 @@ fallback.  ``build()`` compiles it in-tree with hipcc for gfx950 (cross-compiles
 """
 
 import ctypes
+import functools
 import importlib.machinery
 import os
 import subprocess
@@ -207,6 +208,25 @@ if os.path.exists(LAUNCH_PATH):
 if not hasattr(torch._C, "_cuda_getDevice"):
     _launch = None
 
+# Native forms of the launchers that steps of few rows call by the hundred (csrc/wrap.cpp), built for this interpreter and this torch; without them every call takes its Python form.
+WRAP_PATH = os.path.join(_HERE, "_wrap" + importlib.machinery.EXTENSION_SUFFIXES[0])
+_wrap = None
+if _launch is not None and os.path.exists(WRAP_PATH):
+    try:
+        from . import _wrap
+
+        if _wrap.torch_version != torch.__version__.split("+")[0]:
+            raise ImportError(f"built for torch {_wrap.torch_version}")
+    except ImportError as e:
+        _wrap = None
+        warnings.warn(f"llm_quest_amd: {WRAP_PATH} does not load ({e}): launchers stay in Python, about 10 us a launch slower")
+
+
+def native(fn):
+    """The launcher ``fn``, its calls taken by the operator of the same name in csrc/wrap.cpp where everything is as ``fn`` wants it, by ``fn`` itself otherwise."""
+    op = None if _wrap is None else _wrap.operator_for(fn.__name__, fn)
+    return fn if op is None else functools.update_wrapper(op, fn)
+
 
 def load():
     """Load the shared library (no GPU needed) and bind every declared symbol."""
@@ -236,6 +256,8 @@ def load():
         fn.restype = ctypes.c_int
         if _launch is not None:
             _launch.bind(name, ctypes.cast(fn, _P).value)
+        if _wrap is not None:
+            _wrap.bind(name, ctypes.cast(fn, _P).value)
     for name, (argtypes, restype) in QUERIES.items():
         try:
             fn = getattr(lib, name)
@@ -245,6 +267,8 @@ def load():
             raise
         fn.argtypes = argtypes
         fn.restype = restype
+        if _wrap is not None:
+            _wrap.bind(name, ctypes.cast(fn, _P).value)
     _lib = lib
     return lib
 
@@ -323,6 +347,8 @@ _python_call, _python_require_gpu = call, require_gpu
 if _launch is not None:
     _launch.setup(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, _python_call, _python_require_gpu, _fail)
     call, require_gpu, ptr = _launch.call, _launch.require_gpu, _launch.ptr
+if _wrap is not None:
+    _wrap.setup(torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream, _launch.set_device, _fail)
 
 
 def dt_code(dtype):

@@ -128,6 +128,7 @@ def _nt_tick(M, N, eligible=True, device=None):
     w.stats["persistent_eligible"] += 1
 
 
+@L.native
 def gemm(form, a, b, out=None, out_dtype=BF16, bias=None, residual=None, gelu=False, allow_split_k=True, tile=0, split3_out=False):
     """C = epi(op(A) op(B) + bias) + residual.  form NT: A[M,K] B[N,K]; NN: A[M,K] B[K,N]; TN: A[K,M] B[K,N].
     ``split3_out`` (NT, no residual): the fp32 result leaves the epilogue as bf16 [M, 3N] = [hi | lo | hi] -- the activation operand of the next fp32-grade
@@ -184,6 +185,7 @@ def gemm(form, a, b, out=None, out_dtype=BF16, bias=None, residual=None, gelu=Fa
     return out
 
 
+@L.native
 def gemm_grouped(form, problems, tile=0):
     """One launch for several independent GEMMs of one form: problems = [(a, b, out, residual_or_None), ...] (<= 8, same
     output dtype, outputs preallocated).  Used for the weight gradients of a transformer block."""
@@ -266,6 +268,7 @@ def gemm_dgrad_gelu_bwd(dy, w, y1, tanh=False, tile=0):
     return out
 
 
+@L.native
 def gemm_gateup_swiglu(x, w_fused, tile=0):
     """(gu [M, 2F], a [M, F]) of a SwiGLU FFN in ONE launch: gu = x @ [lin1 | lin_gate]^T as usual, a = u * silu(g) from the epilogue
     (replaces gemm + swiglu_fwd)."""
@@ -284,6 +287,7 @@ def gemm_gateup_swiglu(x, w_fused, tile=0):
     return gu, a
 
 
+@L.native
 def gemm_dgrad_swiglu_bwd(dy, w, gu, tile=0):
     """d(gate-up) [M, 2F] of a SwiGLU FFN in ONE launch: d(act) = dy @ w (NN, w = lin2.weight [N_out, F]) stays in the accumulators and the
     activation's backward runs in the epilogue against ``gu`` = the forward's [lin1 | lin_gate] output (replaces gemm + swiglu_bwd)."""
@@ -306,6 +310,7 @@ def gemm_dgrad_swiglu_bwd(dy, w, gu, tile=0):
     return out
 
 
+@L.native
 def colsum(x, out=None, accumulate=False):
     """out[n] (+)= sum_m x[m, n]; x bf16 or fp32 (row-strided views allowed), out fp32."""
     L.require_gpu(x, out)
@@ -318,6 +323,7 @@ def colsum(x, out=None, accumulate=False):
     return out
 
 
+@L.native
 def rmsnorm_fwd(x2d, w, eps=1e-6, want_rstd=True):
     L.require_gpu(x2d, w)
     if x2d.dtype != BF16 or w.dtype != BF16 or not x2d.is_contiguous() or w.numel() != x2d.shape[1]:
@@ -328,6 +334,7 @@ def rmsnorm_fwd(x2d, w, eps=1e-6, want_rstd=True):
     return y, rstd
 
 
+@L.native
 def rmsnorm_bwd(x2d, w, rstd, dy, dres=None, dw_out=None, dw_accumulate=False):
     """Returns (dx [+ dres], dw).  dw goes to ``dw_out`` (bf16/fp32, optionally accumulated) or a new fp32 tensor."""
     L.require_gpu(x2d, w, rstd, dy, dres)
@@ -345,6 +352,7 @@ def rmsnorm_bwd(x2d, w, rstd, dy, dres=None, dw_out=None, dw_accumulate=False):
     return dx, dw
 
 
+@L.native
 def qknorm_rope_fwd(qkv, qw, kw, cos, sin, pos, Hq, Hkv, D, eps=1e-6):
     """qw = kw = None: RoPE only (no per-head normalisation); rstd is then None."""
     L.require_gpu(qkv, qw, kw, cos, sin, pos)
@@ -362,6 +370,7 @@ def qknorm_rope_fwd(qkv, qw, kw, cos, sin, pos, Hq, Hkv, D, eps=1e-6):
     return q, k, rstd
 
 
+@L.native
 def qknorm_rope_bwd(qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, Hq, Hkv, D):
     """Writes d(qkv)[:, :(Hq+Hkv)*D] into dqkv (the V third is left to the caller); returns (dqw_f32, dkw_f32).
     dq=None: the key heads only (the query heads' share ran inside attn_bwd_qnorm); dqw_f32 is then zeros."""
@@ -384,6 +393,7 @@ def qknorm_rope_bwd(qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, Hq, Hkv, D):
     return dw[:D], dw[D:]
 
 
+@L.native
 def swiglu_fwd(gu, F):
     L.require_gpu(gu)
     if not (gu.is_contiguous() and gu.dtype == BF16 and gu.shape[1] == 2 * F):
@@ -393,6 +403,7 @@ def swiglu_fwd(gu, F):
     return a
 
 
+@L.native
 def swiglu_bwd(gu, da, F):
     L.require_gpu(gu, da)
     if not (da.is_contiguous() and da.dtype == BF16 and tuple(da.shape) == (gu.shape[0], F)):
@@ -450,6 +461,7 @@ def _attn_scratch(device, nbytes):
     return ws
 
 
+@L.native
 def attn_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=None, causal=True, scale=None):
     """q [B*S,Hq*D], k/v [B*S,Hkv*D] (row-strided views allowed).  Returns (o [B*S,Hq*D], lse fp32 [B,Hq,S])."""
     L.require_gpu(q, k, v, key_mask)
@@ -465,6 +477,7 @@ def attn_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=None, causal=True, scale=None):
     return o, lse
 
 
+@L.native
 def attn_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dq, dk, dv, key_mask=None, causal=True, scale=None):
     """dq/dk/dv are caller-provided (possibly row-strided) destinations."""
     L.require_gpu(q, k, v, o, do, lse, dq, dk, dv)
@@ -547,6 +560,7 @@ def dgrad_attn_delta(dy, w, ctx, lse, B, S, Hq, D):
     return out, delta
 
 
+@L.native
 def attn_bwd_qnorm(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dk, dv, qkv, qw, cos, sin, pos, rstd, dqkv, key_mask=None, causal=True, scale=None, delta=None):
     """attn_bwd whose dQ pass ends in the backward of the QK-norm + RoPE of the query heads: writes d(qkv)[:, :Hq*D] into ``dqkv`` (dQ never exists
     as a matrix) and returns the fp32 [D] gradient of the query norm weight -- or None when this form does not apply (head_dim != 128, no scratch
@@ -701,6 +715,7 @@ def dgrad_on_ring(M, N, Kd, dtype=BF16):
     return r != 0 and (r != (128 | 1 << 8) or Kd < 6144)
 
 
+@L.native
 def dgrad(dy, w, out=None):
     """dX = dY W for a Linear with weight W [N_out, N_in].  Where ``dgrad_transposes`` says so and ``dgrad_on_ring`` does not, W is transposed first (one pass over the
     weight, 63 MB per transformer block) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads.
@@ -711,6 +726,7 @@ def dgrad(dy, w, out=None):
     return gemm(L.GEMM_NN, dy, w, out=out)
 
 
+@L.native
 def copy2d(src, dst):
     """dst[r,:] = src[r,:] for 2-D views with unit inner stride (bit-exact)."""
     L.require_gpu(src, dst)
@@ -733,6 +749,7 @@ def patchify(img, patch, out_dtype=BF16):
     return rows
 
 
+@L.native
 def layernorm_fwd(x2d, scale, shift, out_dtype=BF16, eps=1e-5, want_stats=False, mode=0):
     L.require_gpu(x2d, scale, shift)
     if x2d.dtype != F32 or not x2d.is_contiguous() or scale.dtype != F32 or shift.dtype != F32:
@@ -828,6 +845,7 @@ def adamw_(param_flat, grad_flat, exp_avg, exp_avg_sq, step, lr, betas=(0.9, 0.9
            L.ptr(exp_avg_sq), float(lr), float(betas[0]), float(betas[1]), float(eps), float(weight_decay), int(step), L.ptr(sumsq), float(max_norm))
 
 
+@L.native
 def add_f32_to_bf16(a_f32, b_bf16, dst_bf16):
     L.require_gpu(a_f32, dst_bf16)
     L.call("mi355_add_f32_to_bf16", a_f32.numel(), L.ptr(a_f32), L.ptr(b_bf16), L.ptr(dst_bf16))
@@ -843,6 +861,7 @@ def scale_bf16(x, scale_f32, out=None):
     return out
 
 
+@L.native
 def gelu_fwd(x, tanh=False):
     L.require_gpu(x)
     if x.dtype != BF16 or not x.is_contiguous() or x.numel() % 8:
@@ -861,6 +880,7 @@ def gelu_bwd(x, dy, tanh=False):
     return dx
 
 
+@L.native
 def gelu_bwd_colsum(x, dy, dest, tanh=False):
     """``gelu_bwd`` of [rows, width], width % 8 == 0, with the result's column sums into ``dest`` (see ``reduce_rows_into``)."""
     L.require_gpu(x, dy)
@@ -906,6 +926,7 @@ def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=No
     return dx, outs[0], outs[1]
 
 
+@L.native
 def reduce_rows_into(partial, parts, width, dests):
     """``dests`` = one (fp32 tensor of ``width`` elements, accumulate) or None per segment of partial [parts, len(dests) * width]: the segments' column sums in one launch -- and one
     more for each time that a destination comes again (a parameter in two places: the workgroups of one launch are in no order)."""
@@ -930,6 +951,7 @@ def layernorm_bwd_bf16_fits(x2d, scale, dy, dres):
     return x2d.shape[1] in (768, 1024) and not (x2d.data_ptr() | dy.data_ptr() | scale.data_ptr() | (0 if dres is None else dres.data_ptr())) % 16
 
 
+@L.native
 def layernorm_bwd_bf16(x2d, scale, mean, rsig, dy, dres, dests, eps=1e-5, mode=0):
     """``layernorm_bwd`` -> (dx fp32, dx bf16); ``dests`` = destinations (see ``reduce_rows_into``) of the gradients of scale, shift and of the bias whose output dx is the gradient of."""
     L.require_gpu(x2d, dy, dres)
@@ -1129,3 +1151,7 @@ def mfma_pipe_rate(seconds=2.0, blocks=256, shape="32x32x16"):
     run(n)  # first half: the clock settles
     per = run(n)
     return flop / (per * 1e-3) / 1e12
+
+
+if L._wrap is not None:
+    L._wrap.set_kernels(globals())  # (its scratch and its switches, for the native forms)

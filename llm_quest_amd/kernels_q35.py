@@ -30,6 +30,7 @@ def _reduce_parts(part, out=None, accumulate=False):
     return out
 
 
+@L.native
 def zc_weight(scale):
     """bf16(1 + scale) of ZeroCenteredRMSNorm."""
     L.require_gpu(scale)
@@ -73,6 +74,7 @@ def _check_heads(src, H, D, head_stride, name):
         raise ValueError(f"{name}: view of width {src.shape[1]} does not cover {H} heads of {D} at stride {head_stride}")
 
 
+@L.native
 def headnorm_rope_fwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, eps=1e-6):
     """src: 2-D view whose column 0 is head 0 (heads every ``head_stride`` columns).  Returns (out [tokens, H*D], rstd)."""
     L.require_gpu(src, w_eff, cos_t, sin_t, pos)
@@ -92,6 +94,7 @@ def headnorm_rope_fwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, eps=1e-6
     return out, rstd
 
 
+@L.native
 def headnorm_rope_bwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, rstd, dout, dsrc, dhead_stride):
     """Writes d(src) into the strided view ``dsrc``; returns d(w_eff) fp32 [D]."""
     L.require_gpu(src, dout, dsrc)
@@ -108,6 +111,7 @@ def headnorm_rope_bwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, rstd, do
     return _reduce_parts(part)
 
 
+@L.native
 def sigmoid_gate_fwd(ctx, gate, H, D, gate_head_stride):
     L.require_gpu(ctx, gate)
     _check_heads(gate, H, D, gate_head_stride, "sigmoid_gate_fwd")
@@ -118,6 +122,7 @@ def sigmoid_gate_fwd(ctx, gate, H, D, gate_head_stride):
     return out
 
 
+@L.native
 def sigmoid_gate_bwd(ctx, gate, H, D, gate_head_stride, dout, dgate, dgate_head_stride):
     L.require_gpu(ctx, gate, dout, dgate)
     _check_heads(gate, H, D, gate_head_stride, "sigmoid_gate_bwd")
@@ -129,6 +134,7 @@ def sigmoid_gate_bwd(ctx, gate, H, D, gate_head_stride, dout, dgate, dgate_head_
     return dctx
 
 
+@L.native
 def attn_generic_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=None, scale=None):
     L.require_gpu(q, k, v, key_mask)
     _check_attn_operand(q, "q", B * S, Hq * D)
@@ -143,6 +149,7 @@ def attn_generic_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=None, scale=None):
     return o, lse
 
 
+@L.native
 def attn_generic_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dq, dk, dv, key_mask=None, scale=None):
     L.require_gpu(q, k, v, o, do, lse, dq, dk, dv)
     for t, n, w in ((q, "q", Hq), (k, "k", Hkv), (v, "v", Hkv), (o, "o", Hq), (do, "do", Hq), (dq, "dq", Hq), (dk, "dk", Hkv), (dv, "dv", Hkv)):
@@ -155,6 +162,7 @@ def attn_generic_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dq, dk, dv, key_mask
            L.ptr(do), do.stride(0), L.ptr(lse), L.ptr(delta), L.ptr(dq), dq.stride(0), L.ptr(dk), dk.stride(0), L.ptr(dv), dv.stride(0), L.ptr(key_mask), scale)
 
 
+@L.native
 def gdn_gates_fwd(b_lin, a_lin, log_A, dt_bias):
     L.require_gpu(b_lin, a_lin, log_A, dt_bias)
     _cols(b_lin, "gdn_gates_fwd(b_lin)")
@@ -168,6 +176,7 @@ def gdn_gates_fwd(b_lin, a_lin, log_A, dt_bias):
     return beta, alpha
 
 
+@L.native
 def gdn_gates_bwd(b_lin, a_lin, log_A, dt_bias, dbeta, dalpha, db_lin, da_lin):
     """Writes d(b_lin), d(a_lin) into the given column views; returns (dlog_A fp32 [Hv], ddt_bias fp32 [Hv])."""
     L.require_gpu(b_lin, a_lin, dbeta, dalpha, db_lin, da_lin)
@@ -187,6 +196,7 @@ def gdn_gates_bwd(b_lin, a_lin, log_A, dt_bias, dbeta, dalpha, db_lin, da_lin):
     return both[:Hv], both[Hv:]
 
 
+@L.native
 def causal_conv_silu_fwd(x, w, B, S):
     """x: [B*S, C] view (row pitch = projection width); w: conv1d.weight (C, 1, k) bf16 contiguous."""
     L.require_gpu(x, w)
@@ -214,6 +224,7 @@ def causal_conv_silu_step(x_new, conv_state, w):
 CONV_TOKEN_CHUNK = 32
 
 
+@L.native
 def causal_conv_silu_bwd(x, w, dy, dx, B, S):
     """Writes d(x) into the column view ``dx``; returns d(weight) fp32 flat [C*k]."""
     L.require_gpu(x, w, dy, dx)
@@ -230,6 +241,7 @@ def causal_conv_silu_bwd(x, w, dy, dx, B, S):
     return _reduce_parts(part)
 
 
+@L.native
 def l2norm_fwd(x, H, D):
     L.require_gpu(x)
     _cols(x, "l2norm_fwd")
@@ -240,6 +252,7 @@ def l2norm_fwd(x, H, D):
     return y
 
 
+@L.native
 def l2norm_bwd(x, dy, dx, H, D):
     L.require_gpu(x, dy, dx)
     _cols(x, "l2norm_bwd")
@@ -338,6 +351,7 @@ def gated_delta_rule_bwd(q, k, v, beta, alpha, ck, do, dv, B, S, Hqk, Hv, Dk, Dv
     return (dq, dk, dbeta, dalpha, d_init) if want_d_initial else (dq, dk, dbeta, dalpha)
 
 
+@L.native
 def gated_rmsnorm_fwd(o, w_f32, gate, H, D, eps=1e-6):
     L.require_gpu(o, w_f32, gate)
     _cols(gate, "gated_rmsnorm_fwd(gate)")
@@ -349,6 +363,7 @@ def gated_rmsnorm_fwd(o, w_f32, gate, H, D, eps=1e-6):
     return out, rstd
 
 
+@L.native
 def gated_rmsnorm_bwd(o, w_f32, gate, rstd, dout, dgate, H, D):
     """Writes d(gate) into the column view ``dgate``; returns (d_o bf16, dw fp32 [D])."""
     L.require_gpu(o, gate, rstd, dout, dgate)

@@ -33,6 +33,7 @@ def _i32(t, name, n=None):
         raise ValueError(f"{name}: contiguous int32 tensor{'' if n is None else f' of at least {n} entries'} required")
 
 
+@L.native
 def embed_hash(tok, prev, table, scale, bigram=None, buckets=0, mul_prev=0, mul_cur=0, out=None):
     """fp32 [tokens, width] = table[tok] * scale (+ bigram row hashed from (prev, tok); prev < 0 selects row ``buckets``); into ``out`` if given."""
     L.require_gpu(tok, prev, table, bigram)
@@ -53,6 +54,7 @@ def embed_hash(tok, prev, table, scale, bigram=None, buckets=0, mul_prev=0, mul_
     return out
 
 
+@L.native
 def add_layernorm(x, w, b, eps, alpha=1.0, y=None, parts=1, cast_dtype=None):
     """LayerNorm(alpha * x + sum of y's ``parts`` rows per token) on fp32 rows -> (fp32 rows, the same rows in ``cast_dtype`` or None)."""
     L.require_gpu(x, w, b, y)
@@ -71,6 +73,7 @@ def add_layernorm(x, w, b, eps, alpha=1.0, y=None, parts=1, cast_dtype=None):
     return out, (out if cast_dtype == F32 else cast)
 
 
+@L.native
 def rmsnorm_rows(x, w, eps, out_dtype=None):
     L.require_gpu(x, w)
     _rows(x, "rmsnorm_rows(x)")
@@ -87,6 +90,7 @@ def rope_frequencies(dims, base, device):
     return torch.pow(torch.tensor(float(base), dtype=torch.float64), -2.0 * i / dims).to(F32).to(device)
 
 
+@L.native
 def latent_kv_append(src, rank, rot, w, eps, pos, dst_row, freq, dims, cache2d, layout=0):
     """src [tokens, rank + rot] -> rows ``dst_row`` of ``cache2d`` [rows, rank + rot]: RMSNorm on the latent, rotary on the shared key part (``layout`` 0:
     neighbouring entries form a pair; 1: entry i pairs with entry i + dims / 2)."""
@@ -102,6 +106,7 @@ def latent_kv_append(src, rank, rot, w, eps, pos, dst_row, freq, dims, cache2d, 
            int(layout), L.ptr(cache2d), _dt(cache2d), cache2d.stride(0))
 
 
+@L.native
 def rope_heads(src, H, n, src_hs, src_off, dst, dst_hs, dst_off, rot_start, dims, freq, pos, layout=0):
     """dst (fp32) <- n entries per head of src, the pairs of [rot_start, rot_start + dims) rotated by the token's position.  ``layout`` 0: neighbouring
     entries form a pair; 1: entry i pairs with entry i + dims / 2."""
@@ -118,6 +123,7 @@ def rope_heads(src, H, n, src_hs, src_off, dst, dst_hs, dst_off, rot_start, dims
     return dst
 
 
+@L.native
 def gated_headnorm(o, w, gate, H, D, eps, out_dtype):
     L.require_gpu(o, w, gate)
     _rows(gate, "gated_headnorm(gate)")
@@ -148,6 +154,7 @@ def _run_chunked(q, k, v, tok, head_decay, qscale, kscale, seq_off, slot, state,
     return o
 
 
+@L.native
 def gla(q, k, v, z, zbias, inv_tau, qscale, seq_off, slot, state, H, dk, dv, head_decay=None, kscale=1.0, max_new=0, min_new=0):
     """Gated linear attention over a ragged batch; ``state`` fp32 [slots, H, dk, dv] is read and written at ``slot``.  Returns fp32 [tokens, H * dv].
     ``head_decay`` (fp32 [H]): a fixed decay per head instead of the per-channel one from ``z`` (``z`` / ``zbias`` may then be None); keys are multiplied
@@ -193,6 +200,7 @@ def _gla_fixed(q, k, v, head_decay, qscale, kscale, seq_off, slot, state, H, dk,
     return o
 
 
+@L.native
 def router_logits(x32, w):
     """fp32 [tokens, experts] = x32 (fp32 rows) times w[experts, width]^T (bf16), fp32 FMA."""
     L.require_gpu(x32, w)
@@ -204,6 +212,7 @@ def router_logits(x32, w):
     return out
 
 
+@L.native
 def moe_route(logits, correction, top, groups, keep, scale, softmax=False):
     """(ids int32 [tokens, top], weights fp32 [tokens, top]).  ``softmax`` True: scores are the softmax over all experts, the winners' scores times ``scale``
     are the weights (not renormalised; of several groups the ``keep`` with the largest members stay eligible); ``softmax`` "chosen": ``correction`` is a bias on the logits, the ``top`` largest win and their weights are the
@@ -218,6 +227,7 @@ def moe_route(logits, correction, top, groups, keep, scale, softmax=False):
     return ids, wts
 
 
+@L.native
 def moe_dispatch(ids, E):
     L.require_gpu(ids)
     _i32(ids, "moe_dispatch(ids)")
@@ -243,6 +253,7 @@ def moe_table_dispatch(tok, vocab, tables, meta, specs):
     return [(offs[i, : e + 1], perm[i, : T * top]) for i, (top, e) in enumerate(specs)]
 
 
+@L.native
 def bgemm(a, b, c, M, N, Kd, batch=1, lda=None, a_bs=0, sbn=None, sbk=1, b_bs=0, ldc=None, c_bs=0, grp_offs=None, a_rows=None, a_div=1, c_rows=None,
           row_scale=None, epi=0, mfma=None, bias=None, limit=0.0, n_out=0):
     """The general strided product (see include/mi355_vlm.h).  Strides default to a's / c's row pitch and b stored [N, K]; the caller vouches that the
@@ -257,6 +268,7 @@ def bgemm(a, b, c, M, N, Kd, batch=1, lda=None, a_bs=0, sbn=None, sbk=1, b_bs=0,
     return c
 
 
+@L.native
 def linear(x, w, out_dtype=None, bias=None):
     """x [M, K] (bf16 or fp32) times w[N, K]^T (bf16) (+ bias fp32 [N]).  bf16 rows go through the MFMA GEMMs (weight stream for <= 8 rows), fp32 rows through
     the fp32 product (``bgemm``: exact products, fp32 sums in an order that does not depend on M)."""
@@ -292,6 +304,7 @@ def attn_key_splits(n_seq, head_tiles, max_new, hm, max_keys, per_split=256):
     return max(1, min(-(-max_keys // per_split), 32, 256 // tiles))
 
 
+@L.native
 def latent_attn(q, k1, k2, v, out, H, hm, D1, D2, DV, q_hs, k1_hs, v_hs, o_hs, desc, max_new, scale, max_keys=0, kv_rep=1, window=0, keep_first=0, softcap=0.0,
                 sink=None, pool=0, pooled=None, pool_row0=None, chunk=0, sig_bias=None, slope=None, gate=None):
     """Two-part-key causal attention over a ragged batch.  ``desc`` = (q_row0, n_new, past, k1_row0, k2_row0, v_row0) int32 [n_seq] each.  ``max_keys``
@@ -352,6 +365,7 @@ def latent_attn(q, k1, k2, v, out, H, hm, D1, D2, DV, q_hs, k1_hs, v_hs, o_hs, d
     return out
 
 
+@L.native
 def group_rmsnorm_sum(x, groups, eps, y1=None, y2=None, parts=1, x_out=None, norm_a=None, norm_b=None):
     """v = x + y1 + (sum of y2's ``parts`` rows per token) on fp32 rows; ``x_out`` (True: a new tensor, or a tensor, or None) receives v.  ``norm_a`` /
     ``norm_b`` = (weight fp32 [width], dtype or None, want_fp32_copy): RMS norm of v in ``groups`` equal consecutive groups times the weight.
@@ -386,6 +400,7 @@ def group_rmsnorm_sum(x, groups, eps, y1=None, y2=None, parts=1, x_out=None, nor
     return x_out, outs[0], outs[1]
 
 
+@L.native
 def ragged_conv(x, w, state, row_seq, seq_off, slot, act=False, residual=False, out_dtype=None, bias=None):
     """Causal convolution over time on every channel of the packed rows ``x`` [tokens, C], w fp32 [C, taps]; ``state`` fp32 [slots, taps - 1, C] carries a
     sequence's last inputs from step to step (read, then updated).  y = (x if residual) + (silu if act)(conv + bias)."""
@@ -409,6 +424,7 @@ def ragged_conv(x, w, state, row_seq, seq_off, slot, act=False, residual=False, 
     return y
 
 
+@L.native
 def qkv_rows_append(src, H, G, d, dv, bias, qw, kw, eps, qscale, dims, layout, freq, pos, dst_row, cache2d, q_temp=None, vmix=None, lam=0.0, v_heads=None, unit_norm=False,
                     rot_amp=1.0, tie_v=False):
     """Rows [H x d | G x d | G x dv] -> fp32 queries [tokens, H * d] (bias, head norm, rotation, per-head scale) and key / value rows of ``cache2d``.
@@ -491,6 +507,7 @@ def pack_gate_up(gate, up):
     return out.reshape(nb * 64, Kd)
 
 
+@L.native
 def glu_rows(x, kind, limit=0.0, out_dtype=None):
     """Rows [gate | up] -> act(gate) * up: ``GLU_GELU_TANH``, ``GLU_SILU``, or ``GLU_CLAMPED_SWISH`` (g = min(gate, limit), u = clamp(up, +-limit),
     g sigmoid(1.702 g) (u + 1))."""
@@ -721,6 +738,7 @@ def gated_groupnorm(o, w, gate, groups, eps, out_dtype, gate_first=False):
 UNARY_RELU2, UNARY_TANH, UNARY_HEAD_GATE, UNARY_SOFTCAP = 0, 1, 2, 3
 
 
+@L.native
 def unary_rows(x, kind, gate=None, group=1, out_dtype=None, limit=0.0):
     """``UNARY_RELU2``: relu(x)^2; ``UNARY_TANH``; ``UNARY_HEAD_GATE``: x[r, i] * sigmoid(gate[r, i // group]) (gate [rows, n / group]);
     ``UNARY_SOFTCAP``: limit * tanh(x / limit)."""
@@ -845,6 +863,7 @@ def yarn_rope_frequencies(dims, base, scaling, device):
     return (f / fac * ramp + f * (1.0 - ramp)).to(F32).to(device), 0.1 * math.log(fac) + 1.0
 
 
+@L.native
 def hyper_mix(x, S, y=None, parts=1, y_scale=1.0, mix=None, put=None, read=None, rows=None, x_out=None, want_u=False, norm=None, eps=0.0, out_dtype=None):
     """What lies between two sublayers of a decoder with ``S`` residual streams.  ``x`` fp32 [tokens, S, width], or [tokens, width]: all streams alike.  With a
     pending sublayer output ``y`` ([tokens * parts, width], bf16 or fp32) every stream becomes sum_s mix[s, t] x_s + put[t] * y_scale * (sum of y's parts), all from

@@ -19,6 +19,7 @@ from . import ops
 BF16 = torch.bfloat16
 
 
+@L.native
 def gemv(x2d, w, residual=None):
     """x [M <= 8, K] @ w[N, K]^T (+ residual); larger M goes through the MFMA GEMM."""
     M = x2d.shape[0]
