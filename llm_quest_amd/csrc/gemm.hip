@@ -2138,9 +2138,11 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
 // B_TR (NN): the column fragments come by transposing reads issued from asm, the whole half's in front of its first row of products, and each half ends with a wait for them.  gemm_bf16_kernel's NN
 // form waits for its one K-tile in flight; us with weights from memory, gemm_bf16_kernel -> here: 333 x 1 024, K = 1 024 20.3 -> 13.3, 3 584 21.5 -> 17.6; 996 x 1 024, K = 4 096 27.6 -> 22.4,
 // 6 144 46.5 -> 26.7; 996 x 4 096, K = 1 024 25.2 -> 16.0; 2 000 x 2 048, K = 2 048 52.0 -> 23.6.  With every CU at work a K-tile of 128 rows takes 0.07 us longer than in the NT form.
+// KIND: a fused epilogue in the write-out, the same bits: SwiGLU's backward behind the NN form (its [u | g] rows requested as a residual's are) and GELU behind the NT form; us, gemm_bf16_kernel -> here:
+// 333 x 3 072, K = 1 024, SwiGLU backward 24.8 -> 16.5, 996 rows 28.9 -> 18.6, 1 416 rows 32.1 -> 23.4; K = 768, GELU, 333 rows 23.3 -> 18.7, 1 200 24.0 -> 19.9.
 // FOLD: the sum over K is cut every p.fold K-tiles and the cuts are added in order -- as near to 64 bits as that many shares of K, without their slabs (2 000 x 1 024, K = 4 096, fp32: 2.7e-7
 // uncut, 1.7e-7 in four).
-template <int BM, int OUT_DT, bool FOLD, bool B_TR>
+template <int BM, int OUT_DT, bool FOLD, bool B_TR, int KIND>
 __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     constexpr int BN = 128, NS = 4, FM = BM / 32, FN = 4;
     constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, A_PPW = A_BYTES / 4096, B_PPW = 4, PPW = A_PPW + B_PPW, STG_LD = 68;
@@ -2286,14 +2288,18 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     // What is added to the sums is requested in front: the bias once, whole residual rows 32 ahead.  Where they are used the loads stood one after the other with nothing beside the SIMD's one wave to hide
     // them: K = 768, us, plain | bias and residual, so -> here (gemm_bf16_kernel): 1 416 x 3 072 fp32 17.7 | 36.1 -> 18.7 (22.0), bf16 15.6 | 30.8 -> 17.1 (18.6); 5 664 x 768 fp32 17.8 | 36.2 -> 18.9 (22.3).
     const bool whole_r = vec_r && cols == 8 && !slabs;
-    u32x4 rv[3][2][B16 ? 1 : 2];
+    constexpr bool SWIGLU = KIND == MI355_EPI_SWIGLU_BWD;  // R: the forward's [u | g], whose eight u and eight g take the residual's place (whole and aligned: the entry point's condition)
+    constexpr int WORDS = B16 && !SWIGLU ? 1 : 2;
+    static_assert(B16 || KIND == MI355_EPI_NONE, "fused epilogues write bf16");
+    u32x4 rv[3][2][WORDS];
     auto request_r = [&](int i) {
         if (!whole_r || i >= FM) return;
 #pragma unroll
         for (int half = 0; half < 2; ++half) {
             const char* r = reinterpret_cast<const char*>(p.R) + (min(gm0 + i * 16 + half * 8, p.M - 1) * p.ldr + gn) * (B16 ? 2 : 4);  // (rows past the end: the last one, not stored)
+            const int64_t step = SWIGLU ? 2 * p.N : 16;
 #pragma unroll
-            for (int w = 0; w < (B16 ? 1 : 2); ++w) rv[i % 3][half][w] = *reinterpret_cast<const u32x4*>(r + 16 * w);
+            for (int w = 0; w < WORDS; ++w) rv[i % 3][half][w] = *reinterpret_cast<const u32x4*>(r + step * w);
         }
     };
     float bias[8];
@@ -2326,7 +2332,24 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
 #pragma unroll
                 for (int e = 0; e < 8; ++e) v[e] += bias[e];
             }
-            if constexpr (B16) {
+            if constexpr (KIND == MI355_EPI_GELU_ERF) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) v[e] = gelu_erf(v[e]);
+            }
+            if constexpr (SWIGLU) {  // as in gemm_tile: d(act) rounded to bf16 first
+                const u32x4 uv = rv[i % 3][half][0], gv = rv[i % 3][half][WORDS - 1];
+                u32x4 o0, o1;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float du[2], dg[2];
+                    swiglu_grads(bf2f(f2bf(v[2 * e])), __uint_as_float(uv[e] << 16), __uint_as_float(gv[e] << 16), du[0], dg[0]);
+                    swiglu_grads(bf2f(f2bf(v[2 * e + 1])), __uint_as_float(uv[e] & 0xffff0000u), __uint_as_float(gv[e] & 0xffff0000u), du[1], dg[1]);
+                    o0[e] = pack_bf2(du[0], du[1]), o1[e] = pack_bf2(dg[0], dg[1]);
+                }
+                bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + gm * p.ldc + gn;
+                *reinterpret_cast<u32x4*>(c) = o0;
+                *reinterpret_cast<u32x4*>(c + p.N) = o1;
+            } else if constexpr (B16) {
                 bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + gm * p.ldc + gn;
                 const bf16_t* r = reinterpret_cast<const bf16_t*>(p.R) + gm * p.ldr + gn;
                 if (whole_r) {
@@ -2378,9 +2401,11 @@ int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStr
     p.ws = (float*)workspace;
     const dim3 grid((unsigned)(p.tiles_m * p.tiles_n * ksplit));
     constexpr int lds = 4 * (BM + 128) * 128;  // gemm_ring_kernel's NS stages
-    if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR>), grid, dim3(256), lds, s, p);
-    else if (BM == 192 || !p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR>), grid, dim3(256), lds, s, p);
-    else hipLaunchKernelGGL((gemm_ring_kernel<128, MI355_DT_F32, true, B_TR>), grid, dim3(256), lds, s, p);  // (192 rows: running sums do not fit the registers)
+    constexpr int FUSED = B_TR ? MI355_EPI_SWIGLU_BWD : MI355_EPI_GELU_ERF;
+    if (p.epilogue == FUSED) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, FUSED>), grid, dim3(256), lds, s, p);
+    else if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
+    else if (BM == 192 || !p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<128, MI355_DT_F32, true, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);  // (192 rows: running sums do not fit the registers)
     if (ksplit > 1) launch_splitk_reduce(p, out_dtype, s);
     MI355_LAUNCH_CHECK("mi355_gemm_bf16(ring)");
     return 0;
@@ -2746,9 +2771,10 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         if (ok) return mi355_gemm_persist_part2(&p, s);
         cfg = 2;
     }
-    if (cfg == 1 && tile_hint == 0 && form != MI355_GEMM_TN && epilogue == MI355_EPI_NONE && !split3 && ablate == 0) {
+    const bool ring_epilogue = epilogue == MI355_EPI_NONE || (out_dtype == MI355_DT_BF16 && epilogue == (form == MI355_GEMM_NT ? MI355_EPI_GELU_ERF : MI355_EPI_SWIGLU_BWD));
+    if (cfg == 1 && tile_hint == 0 && form != MI355_GEMM_TN && ring_epilogue && !split3 && ablate == 0) {
         int ksplit = 1;
-        const bool may_split = workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
+        const bool may_split = epilogue == MI355_EPI_NONE && workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
         if (const int rows = choose_ring(form, M, N, K, out_dtype, may_split, workspace_bytes, ksplit, p.fold)) return mi355_gemm_ring_part7(form, &p, out_dtype, rows, ksplit, workspace, s);
     }
     switch (cfg) {

@@ -186,3 +186,24 @@ def test_nn_values_that_are_not_finite_stay_in_their_row_and_column():
     got, want = KK.gemm(L.GEMM_NN, A, W, out_dtype=F32), A.double() @ W.double()
     assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isinf(got), torch.isinf(want))
     assert torch.equal(got[torch.isfinite(got)], want[torch.isfinite(want)].float())
+
+
+@pytest.mark.parametrize("M,N,K,rows", [(1, 8, 256, 128), (127, 128, 320, 128), (333, 3072, 1024, 128), (5100, 1000, 328, 192), (129, 136, 192, 0), (2000, 3072, 256, 0)])
+def test_fused_epilogues_are_the_128_x_128_kernels(M, N, K, rows):
+    """SwiGLU's backward behind the NN form, GELU (with and without a residual) behind the NT form: the bits of hint 1, rows and columns that end inside a tile, nothing written beside them."""
+    lib, g = L.load(), torch.Generator(device="cuda").manual_seed(M + N)
+    assert lib.mi355_gemm_nn_ring(M, N, K, 0, 0, 0) & 255 == rows
+    A, W = torch.randn(M, K, generator=g, device="cuda").to(BF16), (torch.randn(K, N, generator=g, device="cuda") * 0.1).to(BF16)
+    gu, Wt = torch.randn(M, 2 * N + 16, generator=g, device="cuda").to(BF16)[:, 8 : 2 * N + 8], W.t().contiguous()
+    r, bias = torch.randn(M, N, generator=g, device="cuda").to(BF16), torch.randn(N, generator=g, device="cuda")
+
+    def take(form, b, width, residual, epi, hint, bias=None):
+        C = torch.full((M, width + 8), 7.0, dtype=BF16, device="cuda")
+        L.require_gpu(A, b, C, residual, bias)
+        L.call("mi355_gemm_bf16", form, M, N, K, A.data_ptr(), K, b.data_ptr(), b.stride(0), C.data_ptr(), C.stride(0), L.DT_BF16, L.ptr(bias), L.ptr(residual), 0 if residual is None else residual.stride(0), epi, None, 0, hint)
+        assert torch.equal(C[:, width:], torch.full_like(C[:, width:], 7.0))
+        return C[:, :width]
+
+    assert torch.equal(take(L.GEMM_NN, W, 2 * N, gu, L.EPI_SWIGLU_BWD, 0), take(L.GEMM_NN, W, 2 * N, gu, L.EPI_SWIGLU_BWD, 1))
+    for residual in (None, r):
+        assert torch.equal(take(L.GEMM_NT, Wt, N, residual, L.EPI_GELU, 0, bias), take(L.GEMM_NT, Wt, N, residual, L.EPI_GELU, 1, bias))
