@@ -1254,3 +1254,25 @@ def test_layernorm_backward_with_bf16_result_and_column_sums(rows, width, dt, re
     assert torch.equal(KK.layernorm_bwd(x, scale, mean, rsig, dy, dres=dres, dests=(None, (dsh, False))), want_dx) and torch.equal(dsh, want_sh)
     with pytest.raises(RuntimeError, match="width"):
         KK.L.call("mi355_layernorm_bwd_bf16", 1, 512, *([x.data_ptr()] * 5), 1, None, *([dx.data_ptr()] * 3), 1, 1e-5, 0)
+
+
+@pytest.mark.parametrize("lengths", [[1], [31, 1], [32], [33], [1, 32, 31], [31, 33, 64, 65, 1, 1, 2, 97], [1] * 70, [5, 60, 5, 3, 29, 1]])
+@pytest.mark.parametrize("accumulate", [False, True])
+def test_embedding_gradient_of_runs_on_block_edges(K, lengths, accumulate):
+    """Runs of equal ids that begin, end and lie anywhere in the blocks of 32 sorted positions, ids outside the table at either end: every row's sum once, nothing else touched.  The bound is fp32
+    addition's (one rounding a row added) and one rounding to eight bits."""
+    ids = torch.cat([torch.full((n,), 3 * i - 1) for i, n in enumerate(lengths)] + [torch.full((3,), 3 * len(lengths) + 2)])  # the first run's and the last one's ids lie outside
+    g = torch.Generator().manual_seed(len(ids))
+    ids = ids[torch.randperm(len(ids), generator=g)]
+    dout, table = torch.randn(len(ids), 520, generator=g).to(BF16), torch.randn(3 * len(lengths) + 2, 528, generator=g).to(BF16)
+    want, mag = table.double()[:, :520].clone(), table.double()[:, :520].abs()
+    for row in range(table.shape[0]):
+        at = ids == row
+        if at.any():
+            want[row] = (want[row] if accumulate else 0) + dout[at].double().sum(0)
+            mag[row] = (mag[row] if accumulate else 0) + dout[at].double().abs().sum(0)
+    out = dev(table)
+    K.embedding_bwd_sorted(dev(ids), dev(dout), out[:, :520], accumulate, 1.0)
+    got = out.cpu()
+    bound = max(lengths) * 2.0 ** -24 * mag + 2.0 ** -8 * want.abs()
+    assert ((got[:, :520].double() - want).abs() <= bound).all() and torch.equal(got[:, 520:], table[:, 520:])
