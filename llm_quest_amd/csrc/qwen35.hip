@@ -321,91 +321,91 @@ __global__ __launch_bounds__(256) void gdn_gates_bwd_kernel(int64_t tokens, int 
 
 // ------------------------------------------------------------------------------------------- causal depthwise conv + SiLU
 // y[t, c] = bf16(silu(bf16(sum_j w[c, j] x[t - (k-1) + j, c])))  within each sequence (qwen3_5_text_model.py:81-90, 138-140).
-// A thread owns 8 adjacent channels (16-byte loads) of one token.
-template <int KS>
+// A thread owns 8 adjacent channels (16-byte loads) of TOK tokens of one sequence.  Bound: a token read four times and its channels' taps, 64 bytes a thread, from the caches: two tokens read
+// five rows for two and the taps once; 5 664 tokens x 6 144 channels 57.7 -> 45.1 us (four 46.1, eight 50.7: fewer threads under way), 1 416 17.9 -> 16.3; below half a million threads level or
+// worse (333 tokens 7.3 / 7.3, 33 3.8 / 4.7).
+template <int KS, int TOK>
 __global__ __launch_bounds__(256) void conv_silu_fwd_kernel(int B, int S, int C, const bf16_t* __restrict__ x, int64_t ldx,
                                                             const bf16_t* __restrict__ w, bf16_t* __restrict__ y) {
-    const int cvec = C >> 3;
+    static_assert(KS == 4, "rings of four slots");
+    const int cvec = C >> 3, runs = (S + TOK - 1) / TOK;
     const int64_t idx = (int64_t)blockIdx.x * 256 + threadIdx.x;
-    if (idx >= (int64_t)B * S * cvec) return;
-    const int64_t tok = idx / cvec;
-    const int c0 = (int)(idx % cvec) * 8;
-    const int s = (int)(tok % S);
-    float wv[8][KS];
-    {
-        float tmp[8 * KS];
+    if (idx >= (int64_t)B * runs * cvec) return;
+    const int64_t run = idx / cvec;
+    const int c0 = (int)(idx % cvec) * 8, s0 = (int)(run % runs) * TOK;
+    const bf16_t* xp = x + (run / runs) * S * ldx + c0;
+    bf16_t* yp = y + (run / runs) * S * C + c0;
+    const auto at = [](const u32x4& v, int c) { return __uint_as_float(c & 1 ? v[c >> 1] & 0xffff0000u : v[c >> 1] << 16); };
+    u32x4 xr[TOK + KS - 1], wr[KS];  // rows s0 - 3 on; taps [8 channels][KS]
 #pragma unroll
-        for (int i = 0; i < KS; ++i) unpack8(*reinterpret_cast<const u32x4*>(w + (int64_t)c0 * KS + i * 8), *reinterpret_cast<float(*)[8]>(tmp + 8 * i));
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-            for (int j = 0; j < KS; ++j) wv[c][j] = tmp[c * KS + j];
+    for (int i = 0; i < TOK + KS - 1; ++i) {
+        const int s = s0 + i - (KS - 1);
+        xr[i] = s >= 0 && s < S ? *reinterpret_cast<const u32x4*>(xp + (int64_t)s * ldx) : u32x4{0u, 0u, 0u, 0u};
     }
-    float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
 #pragma unroll
-    for (int j = 0; j < KS; ++j) {
-        const int sj = s - (KS - 1) + j;
-        if (sj >= 0) {
-            float xv[8];
-            unpack8(*reinterpret_cast<const u32x4*>(x + (tok - (KS - 1) + j) * ldx + c0), xv);
+    for (int i = 0; i < KS; ++i) wr[i] = *reinterpret_cast<const u32x4*>(w + (int64_t)c0 * KS + i * 8);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) acc[c] = fmaf(wv[c][j], xv[c], acc[c]);
+    for (int t = 0; t < TOK; ++t) {
+        if (s0 + t >= S) break;
+        float o[8];
+#pragma unroll
+        for (int c = 0; c < 8; ++c) {
+            float acc = 0.f;
+#pragma unroll
+            for (int j = 0; j < KS; ++j)
+                if (s0 + t + j >= KS - 1) acc = fmaf(at(wr[c * KS / 8], c * KS % 8 + j), at(xr[t + j], c), acc);
+            o[c] = silu_f(rbf(acc));
         }
+        *reinterpret_cast<u32x4*>(yp + (int64_t)(s0 + t) * C) = pack8(o);
     }
-    float o[8];
-#pragma unroll
-    for (int c = 0; c < 8; ++c) o[c] = silu_f(rbf(acc[c]));
-    *reinterpret_cast<u32x4*>(y + tok * C + c0) = pack8(o);
 }
 
-// A thread owns 8 channels and walks a chunk of TCH tokens of one sequence and the KS - 1 tokens behind it: dc = bf16(dy * silu'(c)) stays in registers, dx[t, c] =
+// A thread owns two channels and walks a chunk of TCH tokens of one sequence and the KS - 1 tokens behind it: dc = bf16(dy * silu'(c)) stays in registers, dx[t, c] =
 // sum_j w[c, j] dc[t + (k-1) - j, c] leaves as soon as its last dc is known, and the filter gradient of the chunk's own tokens goes to dw_partial[chunk][C*KS].
 // Bound: bytes (x, dy, dx once each, 3 / TCH of x and dy again); four tokens are requested while four are worked on, and the windows are rings of KS = 4 slots that
-// four unrolled tokens turn once around.  5 664 tokens x 6 144 channels, in two passes with dc in memory and a token's operands fetched when it was its turn: 137 us -> 94 (2.2 TB/s);
-// 333 tokens: 50 for the first pass alone -> 43.
+// four unrolled tokens turn once around.  Two channels and not eight: their windows take a quarter of the registers, and four times the threads hide the loads, the exponentials and the chain over
+// the chunk's tokens; with the sum of the chunks' parts, eight / four / two channels, us: 5 664 tokens x 6 144 channels 103 / 81 / 71, 1 416 48 / 39 / 30, 333 45 / 28 / 19, 33 42 / 26 / 17.
 template <int KS>
 __global__ __launch_bounds__(256) void conv_silu_bwd_kernel(int B, int S, int C, int TCH, int chunks_per_seq, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ w,
                                                             const bf16_t* __restrict__ dy, bf16_t* __restrict__ dx, int64_t lddx, float* __restrict__ dw_partial) {
     static_assert(KS == 4, "rings of four slots");
-    const int cvec = C >> 3;
-    const int cv = blockIdx.x * 256 + threadIdx.x;
-    if (cv >= cvec) return;
-    const int c0 = cv * 8;
+    constexpr int CH = 2;
+    const int c0 = (blockIdx.x * 256 + threadIdx.x) * CH;
+    if (c0 >= C) return;
     const int chunk = blockIdx.y;  // over B * chunks_per_seq
     const int b = chunk / chunks_per_seq, s0 = (chunk % chunks_per_seq) * TCH;
     const int s1 = s0 + TCH < S ? s0 + TCH : S;
-    const u32x4 z4 = {0u, 0u, 0u, 0u};
+    const auto at = [](unsigned v, int c) { return __uint_as_float(c ? v & 0xffff0000u : v << 16); };
     const bf16_t *xp = x + (int64_t)b * S * ldx + c0, *gp = dy + (int64_t)b * S * C + c0;
-    u32x4 xn[4], gn[4];
+    unsigned xn[4], gn[4];
     auto request = [&](int s) {
 #pragma unroll
         for (int u = 0; u < 4; ++u) {
-            xn[u] = s + u < S ? *reinterpret_cast<const u32x4*>(xp + (int64_t)(s + u) * ldx) : z4;
-            gn[u] = s + u < S ? *reinterpret_cast<const u32x4*>(gp + (int64_t)(s + u) * C) : z4;
+            xn[u] = s + u < S ? *reinterpret_cast<const unsigned*>(xp + (int64_t)(s + u) * ldx) : 0u;
+            gn[u] = s + u < S ? *reinterpret_cast<const unsigned*>(gp + (int64_t)(s + u) * C) : 0u;
         }
     };
     request(s0);
-    float wv[8][KS], dw[8][KS];
+    float wv[CH][KS], dw[CH][KS];
     {
-        float tmp[8 * KS];
+        float taps[8];
+        unpack8(*reinterpret_cast<const u32x4*>(w + (int64_t)c0 * KS), taps);
 #pragma unroll
-        for (int i = 0; i < KS; ++i) unpack8(*reinterpret_cast<const u32x4*>(w + (int64_t)c0 * KS + i * 8), *reinterpret_cast<float(*)[8]>(tmp + 8 * i));
-#pragma unroll
-        for (int c = 0; c < 8; ++c)
-#pragma unroll
-            for (int j = 0; j < KS; ++j) {
-                wv[c][j] = tmp[c * KS + j];
-                dw[c][j] = 0.f;
-            }
+        for (int j = 0; j < CH * KS; ++j) {
+            wv[j / KS][j % KS] = taps[j];
+            dw[j / KS][j % KS] = 0.f;
+        }
     }
-    float win[KS][8], dcs[KS][8];  // slot (s - s0) & 3: x and dc of token s
+    float win[KS][CH], dcs[KS][CH];  // slot (s - s0) & 3: x and dc of token s
 #pragma unroll
     for (int j = 1; j < KS; ++j) {
         const int sj = s0 - KS + j;
-        unpack8(sj >= 0 ? *reinterpret_cast<const u32x4*>(xp + (int64_t)sj * ldx) : z4, win[j]);
+        const unsigned r = sj >= 0 ? *reinterpret_cast<const unsigned*>(xp + (int64_t)sj * ldx) : 0u;
+#pragma unroll
+        for (int c = 0; c < CH; ++c) win[j][c] = at(r, c);
     }
     for (int sg = s0; sg < s1 + KS - 1; sg += 4) {
-        u32x4 xc[4], gc[4];
+        unsigned xc[4], gc[4];
 #pragma unroll
         for (int u = 0; u < 4; ++u) xc[u] = xn[u], gc[u] = gn[u];
         if (sg + 4 < s1 + KS - 1) request(sg + 4);
@@ -413,15 +413,13 @@ __global__ __launch_bounds__(256) void conv_silu_bwd_kernel(int B, int S, int C,
         for (int u = 0; u < 4; ++u) {
             const int s = sg + u;
             if (s >= s1 + KS - 1) break;
-            float g[8];
-            unpack8(xc[u], win[u]);
-            unpack8(gc[u], g);
 #pragma unroll
-            for (int c = 0; c < 8; ++c) {
+            for (int c = 0; c < CH; ++c) {
+                win[u][c] = at(xc[u], c);
                 float acc = 0.f;
 #pragma unroll
                 for (int j = 0; j < KS; ++j) acc = fmaf(wv[c][j], win[(u + 1 + j) & 3][c], acc);
-                dcs[u][c] = s < S ? rbf(g[c] * dsilu_f(rbf(acc))) : 0.f;
+                dcs[u][c] = s < S ? rbf(at(gc[u], c) * dsilu_f(rbf(acc))) : 0.f;
                 if (s < s1) {
 #pragma unroll
                     for (int j = 0; j < KS; ++j) dw[c][j] = fmaf(dcs[u][c], win[(u + 1 + j) & 3][c], dw[c][j]);
@@ -429,20 +427,22 @@ __global__ __launch_bounds__(256) void conv_silu_bwd_kernel(int B, int S, int C,
             }
             const int t = s - (KS - 1);
             if (t >= s0) {
-                float acc[8] = {0, 0, 0, 0, 0, 0, 0, 0};
+                float acc[CH];
+#pragma unroll
+                for (int c = 0; c < CH; ++c) acc[c] = 0.f;
 #pragma unroll
                 for (int j = 0; j < KS; ++j)
                     if (s - j < S) {
 #pragma unroll
-                        for (int c = 0; c < 8; ++c) acc[c] = fmaf(wv[c][j], dcs[(u - j) & 3][c], acc[c]);
+                        for (int c = 0; c < CH; ++c) acc[c] = fmaf(wv[c][j], dcs[(u - j) & 3][c], acc[c]);
                     }
-                *reinterpret_cast<u32x4*>(dx + ((int64_t)b * S + t) * lddx + c0) = pack8(acc);
+                *reinterpret_cast<unsigned*>(dx + ((int64_t)b * S + t) * lddx + c0) = pack_bf2(acc[0], acc[1]);
             }
         }
     }
     float* dst = dw_partial + (int64_t)chunk * C * KS + (int64_t)c0 * KS;
 #pragma unroll
-    for (int c = 0; c < 8; ++c)
+    for (int c = 0; c < CH; ++c)
 #pragma unroll
         for (int j = 0; j < KS; ++j) dst[c * KS + j] = dw[c][j];
 }
@@ -1447,7 +1447,8 @@ extern "C" int mi355_causal_conv_silu_fwd(int B, int S, int C, int ksize, const 
     MI355_REQUIRE(B > 0 && S > 0 && C > 0 && C % 8 == 0 && ldx % 8 == 0 && ldx >= C, "causal_conv_silu: channels and ld must be multiples of 8");
     MI355_REQUIRE(ksize == 4, "causal_conv_silu: kernel size %d not built (4 only: linear_conv_kernel_size of every Qwen3.5 config)", ksize);
     MI355_REQUIRE(x && w && y, "causal_conv_silu_fwd: null pointer");
-    conv_silu_fwd_kernel<4><<<grid1d((int64_t)B * S * (C / 8)), 256, 0, ST(stream)>>>(B, S, C, (const bf16_t*)x, ldx, (const bf16_t*)w, (bf16_t*)y);
+    if ((int64_t)B * S * (C / 8) >= 1 << 19) conv_silu_fwd_kernel<4, 2><<<grid1d((int64_t)B * ((S + 1) / 2) * (C / 8)), 256, 0, ST(stream)>>>(B, S, C, (const bf16_t*)x, ldx, (const bf16_t*)w, (bf16_t*)y);
+    else conv_silu_fwd_kernel<4, 1><<<grid1d((int64_t)B * S * (C / 8)), 256, 0, ST(stream)>>>(B, S, C, (const bf16_t*)x, ldx, (const bf16_t*)w, (bf16_t*)y);
     MI355_LAUNCH_CHECK("causal_conv_silu_fwd");
     return 0;
 }
@@ -1468,7 +1469,7 @@ extern "C" int mi355_causal_conv_silu_bwd(int B, int S, int C, int ksize, const 
         return mi355_copy2d(rows, (int64_t)C * 2, dc_ws, (int64_t)C * 2, dx, lddx * 2, stream);
     }
     const int cps = (S + token_chunk - 1) / token_chunk;
-    dim3 g1((C / 8 + 255) / 256, B * cps);
+    dim3 g1((C / 2 + 255) / 256, B * cps);
     conv_silu_bwd_kernel<4><<<g1, 256, 0, ST(stream)>>>(B, S, C, token_chunk, cps, (const bf16_t*)x, ldx, (const bf16_t*)w, (const bf16_t*)dy, (bf16_t*)dx, lddx, dw_partial);
     MI355_LAUNCH_CHECK("causal_conv_silu_bwd");
     return 0;

@@ -1034,3 +1034,18 @@ def test_chunked_gated_delta_rule_refuses_what_it_cannot_read():
     L.require_gpu(x)
     with pytest.raises(RuntimeError, match="too small"):
         L.call("mi355_gdr_chunked_fwd", 1, 64, 1, 1, L.ptr(x), L.ptr(x), L.ptr(x), 128, L.ptr(f), L.ptr(f), L.ptr(x), L.ptr(f), 16, 0, None, None)
+
+
+@pytest.mark.parametrize("B,S,C", [(2, 701, 3000), (3, 1, 1398104), (1, 700, 6000)])
+def test_causal_conv_of_two_tokens_a_thread(B, S, C):
+    """From half a million threads a thread takes two tokens: the same bits as each sequence's channels by themselves, an odd last token, one token alone."""
+    from llm_quest_amd import kernels_q35 as Q
+
+    assert B * S * (C // 8) >= 1 << 19
+    g = torch.Generator(device="cuda").manual_seed(S)
+    x, w = torch.randn(B * S, C + 8, generator=g, device="cuda").to(torch.bfloat16)[:, :C], torch.randn(C, 1, 4, generator=g, device="cuda").to(torch.bfloat16)
+    y = Q.causal_conv_silu_fwd(x, w, B, S)
+    for b in range(B):
+        for c in range(0, C, C // 8 // 3 * 8):
+            part = slice(c, min(C, c + C // 8 // 3 * 8))
+            assert torch.equal(y[b * S : (b + 1) * S, part], Q.causal_conv_silu_fwd(x[b * S : (b + 1) * S, part], w[part].contiguous(), 1, S))
