@@ -49,6 +49,55 @@ __device__ __forceinline__ void add16(f32x16& to, f32x16& from) {  // a chain's 
     }
 }
 
+// ---- fp32 products on the bf16 matrix pipe: a number is the sum of three bf16 parts (24 bits: 8 and 8 and the rest, exactly), a product the sum of the parts' products, exact in fp32.  Of two split
+// operands the six largest are taken -- what is left out is 2^-26 of the product -- the first parts' by themselves in one accumulator, the others in a second: a sum over 128 rounds eight times at its
+// own size where a chain of fp32 products rounds 64 times.  32 clocks for 32 x 32 x 16 and 16 of a part against 512 on the fp32 pipe.  An infinity or a NaN makes the sum a NaN.
+struct Parts8 { bf16x8 p[3]; };  // eight consecutive k of a fragment's row
+__device__ __forceinline__ void parts_of(float a, float b, unsigned (&w)[3]) {
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+        w[i] = pack_bf2(a, b);
+        a -= __uint_as_float(w[i] << 16);
+        b -= __uint_as_float(w[i] & 0xffff0000u);
+    }
+}
+__device__ __forceinline__ Parts8 parts8(const f32x4& a, const f32x4& b) {
+    unsigned w[4][3];
+    parts_of(a[0], a[1], w[0]), parts_of(a[2], a[3], w[1]), parts_of(b[0], b[1], w[2]), parts_of(b[2], b[3], w[3]);
+    Parts8 r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) r.p[i] = __builtin_bit_cast(bf16x8, u32x4{w[0][i], w[1][i], w[2][i], w[3][i]});
+    return r;
+}
+__device__ __forceinline__ f32x16 mfma16(const bf16x8& a, const bf16x8& b, const f32x16& c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
+__device__ __forceinline__ void mfma_parts(const Parts8& a, const Parts8& b, f32x16& hi, f32x16& lo) {
+    lo = mfma16(a.p[2], b.p[0], lo);
+    lo = mfma16(a.p[0], b.p[2], lo);
+    lo = mfma16(a.p[1], b.p[1], lo);
+    lo = mfma16(a.p[1], b.p[0], lo);
+    lo = mfma16(a.p[0], b.p[1], lo);
+    hi = mfma16(a.p[0], b.p[0], hi);
+}
+__device__ __forceinline__ void mfma_parts(const bf16x8& a, const Parts8& b, f32x16& hi, f32x16& lo) {  // a: a bf16 operand
+    lo = mfma16(a, b.p[2], lo);
+    lo = mfma16(a, b.p[1], lo);
+    hi = mfma16(a, b.p[0], hi);
+}
+// the three parts of [rows][ld] in LDS, a plane each: the fragment at `at` (elements), and four values of it written
+template <int PLANE>
+__device__ __forceinline__ Parts8 parts_at(const bf16_t* planes, int at) {
+    Parts8 r;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) r.p[i] = *reinterpret_cast<const bf16x8*>(planes + i * PLANE + at);
+    return r;
+}
+template <int PLANE>
+__device__ __forceinline__ void put_parts(bf16_t* planes, int at, float a, float b, float c, float d) {
+    unsigned w0[3], w1[3];
+    parts_of(a, b, w0), parts_of(c, d, w1);
+#pragma unroll
+    for (int i = 0; i < 3; ++i) *reinterpret_cast<u32x2*>(planes + i * PLANE + at) = u32x2{w0[i], w1[i]};
+}
 // whether any of 16 values is infinite or NaN
 __device__ __forceinline__ bool lost16(const f32x16& v) {
     float z = 0.f;

@@ -7,12 +7,13 @@
 //     U = Uv - Kw S^T,  O = scale gam (Q S^T) + P U,  S <- gam_63 S + (Gp U)^T K                                                    -- the chain: one step per chunk
 // and the adjoint splits the same way: only dS crosses chunks (dU = P^T dO + Gp (K dS^T), dS <- gam_63 dS + (scale gam dO)^T Q - dU^T Kw), everything else is one
 // workgroup per chunk afterwards.  Four kernels: prep, scan, reverse scan (both per 32 value rows of the state: a row never meets another), and the rest.
-// All sums are fp32 FMAs on v_mfma_f32_32x32x2_f32 (the two products of bf16 operands alone, K K^T and Q K^T, on the bf16 shape: exact); the log decays are cumulated
+// All sums are fp32 FMAs on v_mfma_f32_32x32x2_f32 (the two products of bf16 operands alone, K K^T and Q K^T, on the bf16 shape: exact; the scan's Kw S^T, Q S^T and P U of three bf16 parts to an
+// fp32 number, which is all of it); the log decays are cumulated
 // in fp64, so a difference of two large ones keeps its digits.  d(alpha) is taken from sums over the pairs that span a token -- never as a difference of
 // larger sums, so it keeps its digits where alpha is tiny (below 1e-30 alpha counts as 1e-30); d(beta) as what reaches u times u / beta.
 // A matrix pipe's chain of 128 products rounds 128 times at its size where lanes sum 16 and meet in a tree; so the chains that show are cut (add16) and the state's gradient
 // gathers its terms from the last token to the first.  Distance to 64 bits, token-by-token kernels | here, 256 tokens, geometric mean of four draws: outputs, d(q), d(k), d(v)
-// 1.65e-3 | 1.65e-3 (their bf16); fp32: state 7.4e-8 | 8.6e-8, d(state) 9.0e-8 | 9.5e-8 (2.9e-7 from the first token on), d(beta) 1.5e-7 | 1.8e-7 (2.6e-7 with whole chains), d(alpha)
+// 1.65e-3 | 1.65e-3 (their bf16); fp32: state 7.4e-8 | 8.4e-8, d(state) 9.0e-8 | 9.5e-8 (2.9e-7 from the first token on), d(beta) 1.5e-7 | 1.8e-7 (2.6e-7 with whole chains), d(alpha)
 // 1.7e-7 | 2.1e-7 (2.5e-7); decays near one 4.4e-7 | 3.6e-7, 5.0e-7 | 4.9e-7; nearly parallel keys 1.5e-7 | 2.3e-7, 2.1e-7 | 4.4e-7.  Cutting d(q)'s and d(k)'s chains as well:
 // d(alpha) 1.9e-7 for 50 us of a backward of 680 (registers spill).
 // Bound: the fp32 matrix pipe (256 FLOP a clock and CU).  The products of one 64-token chunk of one head: 37 MFLOP forward and backward together.
@@ -174,17 +175,23 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int n0, int ke
 }
 
 // ------------------------------------------------------------------------------------------- scan: the state chunk by chunk, 32 value rows per workgroup
-// Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave.  Bound: the chain
-// of chunks -- reads in flight, then two products behind two barriers.  Everything a chunk reads first is requested at its top, all at once: 172 us at 8 x 708 tokens x 16
-// heads (167 before its chains were cut, and so measured: requested a chunk ahead 189, the registers spill; in two halves 187; the value ranges of a head on different XCDs 177).
+// Waves 0, 1 take Kw S^T (row halves), waves 2, 3 Q S^T and then P U; the state's four 32-column tiles go one to a wave, which holds its tile in registers (lane = value row) and leaves
+// its three bf16 parts in LDS for the next chunk's products; so does U, for P U.  The state's own sum, S <- gam_63 S + (Gp U)^T K, stays on the fp32 pipe: on the bf16 pipe a chain's
+// roundings differ, and where decays are strong the state is one such rounding from exact (4.4e-8 against 5.2e-8 from 64 bits; as it is 4.3e-8), for no time gained.  Bound: the chain of chunks
+// and the bytes (8 x 708 tokens x 16 heads: 344 MB, 70 us): two products behind two barriers, every operand of the next chunk requested under this one's second half.
+// 172 -> 148 us at 8 x 708 tokens x 16 heads, 58 -> 45 at 333 tokens (the state in fp32 in LDS, read by both sides' fp32 products, a chunk's operands requested at its own top).
+constexpr int SP = GV * (GD + 8), UP = GV * (GC + 8);  // planes of S [32 v][128 k] and U^T [32 v][64 t]
 __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int n0, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                            const bf16_t* __restrict__ v, int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha, float* __restrict__ saved,
                                                            bf16_t* __restrict__ o, const float* initial_state, float* final_state, int keep, float qscale) {
-    __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];
-    __shared__ __attribute__((aligned(16))) float Us[GC][GV + 8];
+    __shared__ __attribute__((aligned(16))) bf16_t Sp[3 * SP];
+    __shared__ __attribute__((aligned(16))) bf16_t Ut[3 * UP];
+    __shared__ __attribute__((aligned(16))) float Ug[GV][GC + 4];  // Gp U
     __shared__ __attribute__((aligned(16))) bf16_t Ks[GC][GD + 8];
-    __shared__ float gg[2 * GC];
+    __shared__ __attribute__((aligned(16))) float gg[2][2 * GC];
     __shared__ int lost[2];  // a chunk's flag: set by its U, cleared a chunk later
+    static_assert(GV * (GD + 4) * 4 <= 3 * SP * 2, "the recurrence's state lies where the planes were");
+    float(*Ss)[GD + 4] = reinterpret_cast<float(*)[GD + 4]>(Sp);
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
     int at, v0;
     if (!scan_place(heads, at, v0)) return;
@@ -194,124 +201,143 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
     const bf16_t *qp = q + (int64_t)b * S * ldqk + hq * GD, *kp = k + (int64_t)b * S * ldqk + hq * GD;
     const int64_t block = keep ? G_BLOCK : G_SMALL;
     float* base = saved + head * NC * block + (keep ? G_KW : 0);
+    const int row = 32 * rh + ln, col = 32 * wave + 4 * hf;  // the lane's row of a fragment; its first column of the state
+    // (a chunk's addresses: a scalar base and 32 bits a lane, or they take more registers than there are)
+    const unsigned kw_at = row * GD + 8 * hf, p_at = row * GC + 8 * hf, q_at = row * (unsigned)ldqk + 8 * hf, u_at = (32 * rh + 4 * hf) * GD + ln, s_at = ln * GD + col, k_at = (tid >> 4) * (unsigned)ldqk + (tid & 15) * 8,
+                   k_step = 16 * (unsigned)ldqk, o_at = (32 * rh + 4 * hf) * (unsigned)(Hv * GD) + ln, o_step = Hv * GD;
+    // what a chunk reads: a Kw row (waves 0, 1) or a Q row and a P row (waves 2, 3) in fragment form; K; U before the state's part; its decays
+    f32x4 fr[16];
+    u32x4 kr[4];
+    float uv[16], gr = 0.f;
+    auto request = [&](int n) {
+        const float* blk = base + n * block;
+        const int t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
+        if (!qside) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
-        if (initial_state) s = *reinterpret_cast<const f32x4*>(initial_state + (head * GD + v0 + r) * GD + c);
-        *reinterpret_cast<f32x4*>(&Ss[r][c]) = s;
+            for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(blk + kw_at + 16 * (i >> 1) + 4 * (i & 1));
+            const float* ub = blk + C_U + v0;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) uv[e] = ub[u_at + c_row(e, 0) * GD];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) fr[i] = row < cnt ? *reinterpret_cast<const f32x4*>(qp + t0 * ldqk + q_at + 16 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) kr[i] = (tid >> 4) + 16 * i < cnt ? *reinterpret_cast<const u32x4*>(kp + t0 * ldqk + (k_at + i * k_step)) : u32x4{0u, 0u, 0u, 0u};
+        if (tid < 2 * GC) gr = blk[C_GAM + tid];
+    };
+    auto request_p = [&](int n) {
+        if (qside) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) fr[8 + i] = *reinterpret_cast<const f32x4*>(base + n * block + C_P + p_at + 16 * (i >> 1) + 4 * (i & 1));
+        }
+    };
+    f32x16 s;  // S[v0 + ln][32 wave + c_row(e, hf)]
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+        if (initial_state) x = *reinterpret_cast<const f32x4*>(initial_state + (head * GD + v0 + ln) * GD + col + 8 * c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[4 * c + e] = x[e];
     }
+    auto put_state = [&]() {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) put_parts<SP>(Sp, ln * (GD + 8) + col + 8 * c, s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]);
+    };
+    put_state();
+    request(0);
+    request_p(0);
     if (tid < 2) lost[tid] = 0;
+    if (tid < 2 * GC) gg[0][tid] = gr;
     int n = 0;
     for (; n < NC; ++n) {
         float* blk = base + n * block;
         const int t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
-        // a Kw row (waves 0, 1) or, in half the words, a Q row (waves 2, 3) in fragment form, all of it in flight at once
-        const int row = 32 * rh + ln;
-        const float* kw = blk + row * GD + 4 * hf;
-        f32x4 fr[16];
-        if (!qside) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(kw + 8 * i);
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const u32x2 w0 = row4(qp + t0 * ldqk, ldqk, row, cnt, 16 * i + 4 * hf), w1 = row4(qp + t0 * ldqk, ldqk, row, cnt, 16 * i + 8 + 4 * hf);
-                fr[i] = f32x4{__uint_as_float(w0[0]), __uint_as_float(w0[1]), __uint_as_float(w1[0]), __uint_as_float(w1[1])};
-            }
-        }
-        u32x4 kr[4];
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
-            kr[i] = r < cnt ? *reinterpret_cast<const u32x4*>(kp + (t0 + r) * ldqk + c) : u32x4{0u, 0u, 0u, 0u};
-        }
-        const float gr = tid < 2 * GC ? blk[C_GAM + tid] : 0.f;
+        const float* g = gg[n & 1];
         __syncthreads();  // the state is whole, the last chunk's K and U are read
-        if (tid < 2 * GC) gg[tid] = gr;
         if (tid == 0) lost[(n + 1) & 1] = 0;
         if (keep) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-                *reinterpret_cast<f32x4*>(blk - G_KW + (v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
-            }
-        }
-        f32x16 uv = zero16(), acc = zero16();
-        if (!qside) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) uv[e] = blk[C_U + (32 * rh + c_row(e, hf)) * GD + v0 + ln];
-        }
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-            const f32x4 s = *reinterpret_cast<const f32x4*>(&Ss[ln][8 * i + 4 * hf]);
-            f32x4 a;
-            if (!qside) a = fr[i];
-            else a = widen4(i & 1 ? u32x2{__float_as_uint(fr[i >> 1][2]), __float_as_uint(fr[i >> 1][3])} : u32x2{__float_as_uint(fr[i >> 1][0]), __float_as_uint(fr[i >> 1][1])});
-#pragma unroll
-            for (int j = 0; j < 4; ++j) acc = mfma2(a[j], s[j], acc);
-            if (i == 7) {
-#pragma unroll
-                for (int e = 0; e < 16; ++e) {
-                    uv[e] -= acc[e];
-                    acc[e] = 0.f;
-                }
-            }
-            if (i % 4 == 3) asm volatile("" ::: "memory");  // keep the state reads of later steps where they are: all sixteen at once cost more registers than there are
+            for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(blk - G_KW + v0 * GD + s_at + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
         }
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
             *reinterpret_cast<u32x4*>(&Ks[r][c]) = kr[i];
         }
-        f32x4 pr[8];
-#pragma unroll
-        for (int i = 0; i < 8; ++i) pr[i] = qside ? *reinterpret_cast<const f32x4*>(blk + C_P + (32 * rh + ln) * GC + 8 * i + 4 * hf) : f32x4{0.f, 0.f, 0.f, 0.f};
+        f32x16 hi = zero16(), lo = zero16();
         if (!qside) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int r = 32 * rh + c_row(e, hf);
-                acc[e] = uv[e] - acc[e];
-                Us[r][ln] = acc[e];
-                blk[C_U + r * GD + v0 + ln] = acc[e];
+            for (int i = 0; i < 8; ++i) {
+                mfma_parts(parts8(fr[2 * i], fr[2 * i + 1]), parts_at<SP>(Sp, ln * (GD + 8) + 16 * i + 8 * hf), hi, lo);
+                if (i & 1) asm volatile("" ::: "memory");  // keep the reads of later steps where they are: all at once cost more registers than there are
             }
-            if (__any(lost16(acc)) && lane == 0) lost[n & 1] = 1;
+            f32x16 u;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) u[e] = uv[e] - (hi[e] + lo[e]);
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                const int t = 32 * rh + 8 * c + 4 * hf;
+                const f32x4 G = *reinterpret_cast<const f32x4*>(g + GC + t);
+                put_parts<UP>(Ut, ln * (GC + 8) + t, u[4 * c], u[4 * c + 1], u[4 * c + 2], u[4 * c + 3]);
+                *reinterpret_cast<f32x4*>(&Ug[ln][t]) = f32x4{u[4 * c] * G[0], u[4 * c + 1] * G[1], u[4 * c + 2] * G[2], u[4 * c + 3] * G[3]};
+            }
+            if (__any(lost16(u)) && lane == 0) lost[n & 1] = 1;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) (blk + C_U + v0)[u_at + c_row(e, 0) * GD] = u[e];
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                mfma_parts(__builtin_bit_cast(bf16x8, fr[i]), parts_at<SP>(Sp, ln * (GD + 8) + 16 * i + 8 * hf), hi, lo);
+                if (i & 1) asm volatile("" ::: "memory");
+            }
         }
         __syncthreads();
         const int gone = lost[n & 1];
+        if (n + 1 < NC) request(n + 1);
         if (qside) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] = (acc[e] - uv[e]) * (gg[32 * rh + c_row(e, hf)] * qscale);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                if (rh == 0 && i >= 4) break;  // P is lower triangular
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc = mfma2(pr[i][j], Us[8 * i + 4 * hf + j][ln], acc);
+            for (int e = 0; e < 16; ++e) {
+                const float f = g[32 * rh + c_row(e, hf)] * qscale;
+                hi[e] *= f;
+                lo[e] *= f;
             }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                if (rh == 0 && i >= 2) break;  // P is lower triangular
+                mfma_parts(parts8(fr[8 + 2 * i], fr[9 + 2 * i]), parts_at<UP>(Ut, ln * (GC + 8) + 16 * i + 8 * hf), hi, lo);
+                asm volatile("" ::: "memory");
+            }
+            if (n + 1 < NC) request_p(n + 1);
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = 32 * rh + c_row(e, hf);
-                if (r < cnt) o[((int64_t)b * S + t0 + r) * Hv * GD + (int64_t)h * GD + v0 + ln] = f2bf(acc[e]);
+                if (r < cnt) (o + (((int64_t)b * S + t0) * Hv + h) * GD + v0)[o_at + c_row(e, 0) * o_step] = f2bf(hi[e] + lo[e]);
             }
         }
         if (gone) break;  // (the same for the whole workgroup)
-        f32x16 s;
-        const float gC = gg[GC - 1];
+        const float gC = g[GC - 1];
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
-#pragma unroll 2
-        for (int kb = 0; kb < GC; kb += 8)
+        for (int e = 0; e < 16; ++e) s[e] *= gC;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int t = kb + 4 * hf + j;
-                s = mfma2(Us[t][ln] * gg[GC + t], bf2f(Ks[t][32 * wave + ln]), s);
-            }
+        for (int i = 0; i < 8; ++i) {
+            const f32x4 d = *reinterpret_cast<const f32x4*>(&Ug[ln][8 * i + 4 * hf]);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = s[e];  // read by this wave alone since the last barrier
+            for (int j = 0; j < 4; ++j) s = mfma2(bf2f(Ks[8 * i + 4 * hf + j][32 * wave + ln]), d[j], s);
+            if (i & 1) asm volatile("" ::: "memory");
+        }
+        put_state();
+        if (tid < 2 * GC) gg[(n + 1) & 1][tid] = gr;
+    }
+    if (n == NC && final_state) {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(final_state + (head * GD + v0 + ln) * GD + col + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
     }
     // A chunk whose U is not finite, and all behind it: the recurrence itself, eight lanes to a value row.  (In a chunk the triangles' zeros are multiplied, not skipped: a token's key,
     // value, decay or beta that is not finite reaches U and with it the rows before it.  A query reaches its own row alone.)
     if (n < NC) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) Ss[ln][32 * wave + c_row(e, hf)] = s[e];  // (the planes are read no more)
         __threadfence();
         __syncthreads();  // what the chunk wrote of its outputs and U lies below what comes
         const int r = tid >> 3, c = (tid & 7) * 16;
@@ -345,15 +371,8 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
             }
         }
 #pragma unroll
-        for (int i = 0; i < 16; ++i) Ss[r][c + i] = st[i];
-    }
-    if (final_state) {
-        __syncthreads();
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-            *reinterpret_cast<f32x4*>(final_state + (head * GD + v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
-        }
+        for (int i = 0; i < 16; ++i)
+            if (final_state) final_state[(head * GD + v0 + r) * GD + c + i] = st[i];
     }
 }
 

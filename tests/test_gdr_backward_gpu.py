@@ -54,3 +54,28 @@ def test_last_chunks_and_views(S, Hqk, Hv):
         t[S:] = float("nan")
     lost = (*_backward(q, k, v, beta, alpha, do, dv, B, S, Hqk, Hv), dv)
     assert all(torch.equal(a[:S], b[:S]) for a, b in zip(got[:4], lost)) and bool(torch.isfinite(lost[4][:S].float()).all())
+
+
+@pytest.mark.parametrize("S,decay,size", [(64, 0.3, 1.0), (65, 8.0, 1e30), (96, 0.0, 1e-30), (127, 0.01, 1.0), (129, 8.0, 1.0), (192, 0.001, 1e30), (321, 0.3, 1e-3)])
+def test_state_from_a_state(S, decay, size):
+    """The final state and the outputs of chunks that start from a state, against 64 bits, over whole and last chunks, decays from none to strong, and sizes where the parts of a split number come
+    near either end of fp32.  The state is a sum over 64 tokens a chunk of fp32 products, each rounding 2^-24 of it at most, of U that summed 128 the same way; outputs are bf16."""
+    from llm_quest_amd import kernels_q35 as K
+
+    B, Hqk, Hv = 2, 1, 2
+    q, k, v, beta, _, _ = _operands(B, S, Hqk, Hv, S)
+    g = torch.Generator().manual_seed(S + 1)
+    v, alpha = (v.float() * size).to(BF16), torch.exp(-decay * torch.rand(B * S, Hv, generator=g)).cuda()
+    st = (torch.randn(B, Hv, 128, 128, generator=g) * size).cuda()
+    hd = lambda t: t.double().view(B, S, -1, 128)
+    qd, kd, vd, bd, ad, want, out = hd(q).repeat_interleave(Hv, 2), hd(k).repeat_interleave(Hv, 2), hd(v), beta.double().view(B, S, Hv), alpha.double().view(B, S, Hv), st.double(), []
+    for t in range(S):
+        want = want * ad[:, t, :, None, None]
+        u = bd[:, t, :, None] * (vd[:, t] - (want * kd[:, t, :, None]).sum(-1))
+        want = want + u[..., None] * kd[:, t, :, None]
+        out.append((want * qd[:, t, :, None]).sum(-1) * 128**-0.5)
+    out = torch.stack(out, 1).reshape(B * S, -1)
+    for keep in (True, False):
+        o, _, fin = K.gated_delta_rule_fwd(q, k, v, beta, alpha, B, S, Hqk, Hv, 128, 128, keep=keep, want_state=True, state=st.clone(), chunked=True)
+        assert float((fin.double() - want).norm()) < 64 * 2**-24 * float(want.norm())
+        assert float((o.double() - out).norm()) < 2**-8 * float(out.norm())
