@@ -178,6 +178,9 @@ int mi355_attn_bwd(int B, int S, int Hq, int Hkv, int D, const void* q, int64_t 
  * shape has no such form and workspace may be NULL): the dK/dV pass leaves dS there in bf16 and dQ = scale * dS K is one product over
  * it, instead of a pass that recomputes the scores.  Same results contract as mi355_attn_bwd; the scratch holds nothing afterwards. */
 int64_t mi355_attn_bwd_workspace_bytes(int B, int S, int Hq, int D);
+/* Bytes that a call gains from behind that workspace (0: none): with workspace_bytes of both together, the key blocks of a call too small for the chip are split and their fp32 parts lie there.
+ * Never needed, and not used with MI355_ATTN_DELTA_READY. */
+int64_t mi355_attn_bwd_split_bytes(int B, int S, int Hq, int Hkv, int D, int causal);
 /* byte offset, inside that workspace, of the fp32 [B, Hq, S] array -lse * log2(e) (which = 0) or -delta (which = 1); -1 = no workspace form */
 int64_t mi355_attn_bwd_workspace_rowconst_offset(int B, int S, int Hq, int D, int which);
 /* OR into `causal` of mi355_attn_bwd_ws / mi355_attn_bwd_qnorm: delta and both row-constant arrays are already filled (mi355_gemm_bf16_attn_delta) */

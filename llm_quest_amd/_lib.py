@@ -176,6 +176,7 @@ QUERIES = {
     "mi355_gdr_chunked_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
     "mi355_decode_block_scratch_bytes": ([_I, _I, _I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
+    "mi355_attn_bwd_split_bytes": ([_I, _I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_rowconst_offset": ([_I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_qnorm_partials": ([_I, _I, _I], _L),
     "mi355_embedding_bwd_sorted_workspace_bytes": ([_L, _I], _L),

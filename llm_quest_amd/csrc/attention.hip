@@ -798,14 +798,24 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dq_kernel(int B, int S, int H
 // scale log2(e) / sqrt(d) is folded into this wave's K rows once per key block (bf16(k * c): one more rounding of a bf16 operand), so the S chain
 // delivers the exponent of P and the dP chain dP - delta: the B phase shrinks from six vector instructions per score (scale the constant, fma, exp2,
 // subtract, multiply, pack) to three (exp2, multiply, pack) -- the pass is bound by what its lone wave has to issue.
-template <int D, bool LEAN>
+// `most` != 0: a key block's stream of (head, query tile) pairs is cut into parts of at most `most` tiles, a workgroup each (dkv_blocks: how many parts a block has); a part leaves its fp32
+// dK^T, dV^T in `parts`, as the registers hold them, and the dQ pass's launch adds them up beside its own work (dkv_fold).  A workgroup's time is its longest chain of tiles, 2.3 us each, whatever else
+// the chip could do: two samples of 498 tokens, 8 key / value heads, are 64 blocks of 4 to 16 tiles.  The whole
+// backward, 16 heads over 8: 2 x 498 tokens 56 -> 36 us, 1 x 709 74 -> 38, 1 x 1 500 130 -> 70, 3 x 560 64 -> 47, 1 x 300 39 -> 27.
+__host__ __device__ __forceinline__ int dkv_tiles(int S, int rep, int causal, int kb) { return ((S + 63) / 64 - (causal ? 2 * kb : 0)) * rep; }
+__host__ __device__ __forceinline__ int dkv_blocks(int S, int rep, int causal, int most, int kb) {  // parts of all key blocks in front of kb
+    int n = 0;
+    for (int i = 0; i < kb; ++i) n += (dkv_tiles(S, rep, causal, i) + most - 1) / most;
+    return n;
+}
+template <int D, bool LEAN, bool SPLIT = false>
 __global__ __launch_bounds__(256, 1) void attn_bwd_dkv_kernel(int B, int S, int Hq, int Hkv, const bf16_t* __restrict__ q, int64_t ldq,
                                                               const bf16_t* __restrict__ k, int64_t ldk, const bf16_t* __restrict__ v,
                                                               int64_t ldv, const bf16_t* __restrict__ d_o, int64_t lddo,
                                                               const float* __restrict__ lse, const float* __restrict__ delta,
                                                               bf16_t* __restrict__ dk, int64_t lddk, bf16_t* __restrict__ dv, int64_t lddv,
                                                               const uint8_t* __restrict__ key_mask, int causal, float scale, float scale_log2,
-                                                              int bpw, bf16_t* __restrict__ ds_out) {
+                                                              int bpw, bf16_t* __restrict__ ds_out, int most, float* __restrict__ parts) {
     // ds_out != nullptr: this pass also leaves dS / scale (bf16, the values its own dK^T product consumes) in a scratch buffer, so that
     // dQ = scale * dS K becomes ONE product (attn_bwd_dq_spill_kernel) instead of the dQ pass's three (it recomputes S and dP):
     // 5 products for the whole backward instead of 7.
@@ -827,20 +837,37 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkv_kernel(int B, int S, int 
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     // one workgroup = `bpw` consecutive 128-key blocks of one (batch, kv head)
     const int nkb = (S + 127) / 128, nchunk = (nkb + bpw - 1) / bpw;
-    const int chunk = blockIdx.x % nchunk, bh = blockIdx.x / nchunk;
-    const int hkv = bh % Hkv, b = bh / Hkv;
     const int rep = Hq / Hkv;
-    const int kb_lo = chunk * bpw, kb_hi = min(nkb, kb_lo + bpw);
+    int bh = blockIdx.x / nchunk, kb_lo = blockIdx.x % nchunk * bpw, kb_hi = min(nkb, kb_lo + bpw);
+    int first = 0, left = 0x7fffffff;  // of the block's stream: the first tile, and how many
+    bool whole = true;
+    if constexpr (SPLIT) {
+        const int per = dkv_blocks(S, rep, causal, most, nkb);
+        int j = blockIdx.x % per;
+        bh = blockIdx.x / per;
+        for (kb_lo = 0;; ++kb_lo) {
+            const int tiles = dkv_tiles(S, rep, causal, kb_lo), n = (tiles + most - 1) / most;
+            if (j < n) {
+                first = tiles * j / n, left = tiles * (j + 1) / n - first, whole = n == 1;
+                break;
+            }
+            j -= n;
+        }
+        kb_hi = kb_lo + 1;
+    }
+    const int hkv = bh % Hkv, b = bh / Hkv;
     const int nqt_all = (S + 63) / 64;
     auto qt0_of = [&](int kb) { return causal ? kb * 2 : 0; };  // first query tile that can see any key of the block
+    const int ch0 = first / (nqt_all - qt0_of(kb_lo)), cq0 = first % (nqt_all - qt0_of(kb_lo)), share = left;
 
     // ---- Q / dO tile stream over (key block, head, query tile), NST-deep
     // (head and query tile advance as counters: a scalar division per tile was a tenth of the tile's time)
-    int ikb = kb_lo, ih = 0, iq = 0, istage = 0;  // next tile to request: key block, query head within the kv group, query tile counted from the block's first
+    int ikb = kb_lo, ih = ch0, iq = cq0, istage = 0;  // next tile to request: key block, query head within the kv group, query tile counted from the block's first
     auto issue_next = [&]() -> bool {
         if (ikb < kb_hi && iq >= nqt_all - qt0_of(ikb)) { iq = 0; ++ih; }
         if (ikb < kb_hi && ih >= rep) { ih = 0; ++ikb; }
-        if (ikb >= kb_hi) return false;
+        if (ikb >= kb_hi || left == 0) return false;
+        --left;
         const int hq = hkv * rep + ih;
         const int qt = qt0_of(ikb) + iq;
         char* st_ = smem + istage * STAGE;
@@ -906,9 +933,9 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkv_kernel(int B, int S, int 
         static_for<KS>([&](auto ks) { owned_write4<OWNED, VF0 + 4 * ks.value>(tv[ks.value]); });
         const int qt0 = qt0_of(kb);
         const int per_head = nqt_all - qt0;
-        const int nit = per_head * rep;
+        const int nit = min(per_head * rep, share);
         PROF_ADD(3, t_pro);
-        int ch = 0, cq = -1;  // the tile consumed: query head within the kv group, query tile counted from qt0
+        int ch = ch0, cq = cq0 - 1;  // the tile consumed: query head within the kv group, query tile counted from qt0
         for (int it = 0; it < nit; ++it) {
             if (++cq == per_head) { cq = 0; ++ch; }
             // this wave's pieces of the tile have landed (a younger tile may stay in flight), then everybody's
@@ -1124,6 +1151,14 @@ __global__ __launch_bounds__(256, 1) void attn_bwd_dkv_kernel(int B, int S, int 
         [[maybe_unused]] const unsigned long long t_epi = PROF_T();
         owned_settle<OWNED>();
         if (kb + 1 < kb_hi) request_kv(kb + 1);
+        if (SPLIT && !whole) {
+            float* at = parts + ((int64_t)blockIdx.x * 4 + wave) * (8 * DT) * 256 + lane * 4;
+            static_for<8 * DT>([&](auto i) {
+                constexpr int r = 4 * i.value;
+                *reinterpret_cast<f32x4*>(at + i.value * 256) = f32x4{owned_read<OWNED, r>(), owned_read<OWNED, r + 1>(), owned_read<OWNED, r + 2>(), owned_read<OWNED, r + 3>()};
+            });
+            continue;
+        }
         // 16-byte stores: the two half-waves hold adjacent 8-byte pieces of a key's row (d = 8 g4 + 4 (lane >> 5) + 0..3); one v_permlane32_swap per word
         // gives the lower half-wave both pieces of an even g4 and the upper half-wave both pieces of the odd one -- 8 stores per tensor instead of 16
         // (the write-out is bound by what it costs to issue a store)
@@ -1198,10 +1233,55 @@ __device__ unsigned long long g_dq_prof[32];
 #define DQ_T() 0ull
 #define DQ_MARK(i) do { } while (0)
 #endif
+// the parts of the dK/dV pass's split key blocks (its write-out, on sums over the parts in their order): FOLD_WG workgroups a block behind the grid's own
+constexpr int FOLD_WG = 4;
+struct DkvFold {
+    const float* parts;
+    int most;  // 0: nothing was split
+    bf16_t *dk, *dv;
+    int64_t lddk, lddv;
+};
+template <int D>
+__device__ void dkv_fold(const DkvFold& f, int idx, int S, int Hq, int Hkv, int causal, float scale) {
+    constexpr int DT = Cfg<D>::DT, PER = 2 * DT / FOLD_WG;
+    static_assert(2 * DT % FOLD_WG == 0, "whole pieces to a workgroup");
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, rep = Hq / Hkv, nkb = (S + 127) / 128;
+    const int piece = idx % FOLD_WG, kb = idx / FOLD_WG % nkb, bh = idx / FOLD_WG / nkb, hkv = bh % Hkv, b = bh / Hkv;
+    const int n = (dkv_tiles(S, rep, causal, kb) + f.most - 1) / f.most, key = kb * 128 + wave * 32 + (lane & 31);
+    if (n == 1) return;
+    const int64_t slot = (int64_t)bh * dkv_blocks(S, rep, causal, f.most, nkb) + dkv_blocks(S, rep, causal, f.most, kb);
+    const float* at = f.parts + (slot * 4 + wave) * (8 * DT) * 256 + lane * 4;
+    f32x4 sum[PER][4];  // dV (two quads of a piece), dK
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) sum[i][c] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int j = 0; j < n; ++j) {
+        f32x4 x[PER][4];
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) x[i][c] = *reinterpret_cast<const f32x4*>(at + (int64_t)j * 4 * (8 * DT) * 256 + ((c >> 1) * 4 * DT + 2 * (PER * piece + i) + (c & 1)) * 256);
+#pragma unroll
+        for (int i = 0; i < PER; ++i)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) sum[i][c] += x[i][c];
+    }
+#pragma unroll
+    for (int i = 0; i < PER; ++i)
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const f32x4 a = t ? sum[i][2] * scale : sum[i][0], c = t ? sum[i][3] * scale : sum[i][1];
+            const auto s0 = __builtin_amdgcn_permlane32_swap(pack_bf2(a[0], a[1]), pack_bf2(c[0], c[1]), false, false), s1 = __builtin_amdgcn_permlane32_swap(pack_bf2(a[2], a[3]), pack_bf2(c[2], c[3]), false, false);
+            bf16_t* out = (t ? f.dk + ((int64_t)b * S + key) * f.lddk : f.dv + ((int64_t)b * S + key) * f.lddv) + (int64_t)hkv * D + 16 * (PER * piece + i) + 8 * (lane >> 5);
+            if (key < S) *reinterpret_cast<u32x4*>(out) = u32x4{s0[0], s1[0], s0[1], s1[1]};
+        }
+}
+
 template <int D, bool FUSE>
 __global__ __launch_bounds__(256, 2) void attn_bwd_dq_spill_kernel(int B, int S, int Hq, int Hkv, const bf16_t* __restrict__ k, int64_t ldk,
                                                                    const bf16_t* __restrict__ ds, bf16_t* __restrict__ dq, int64_t lddq,
-                                                                   int causal, float scale, QkFuse f) {
+                                                                   int causal, float scale, QkFuse f, DkvFold fold) {
     using C = Cfg<D>;
     constexpr int DT = C::DT, DSW = 4096;  // a wave's dS bytes per 64-key tile: 2 key groups x 2 KiB
     // Two workgroups per CU (one's LDS-DMA issue and write-out run under the other's tiles) and TWO rings: the K tiles (shared by the four waves, served
@@ -1215,7 +1295,12 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_spill_kernel(int B, int S,
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int nqb = (S + 127) / 128;
-    const int vid = xcd_chunked((int)blockIdx.x, (int)gridDim.x);
+    const int own = B * Hq * nqb;
+    if ((int)blockIdx.x >= own) {
+        dkv_fold<D>(fold, (int)blockIdx.x - own, S, Hq, Hkv, causal, scale);
+        return;
+    }
+    const int vid = xcd_chunked((int)blockIdx.x, own);
     int qb, bh;
     heavy_first(vid, nqb, B * Hq, ATTN_HEAD_GROUP, qb, bh);
     const int hq = bh % Hq, b = bh / Hq;
@@ -1650,6 +1735,27 @@ extern "C" int mi355_attn_fwd(int B, int S, int Hq, int Hkv, int D, const void* 
     return 0;
 }
 
+// Tiles to a part of the dK/dV pass (0: key blocks stay whole): the fewest, from SPLIT_TILES on, with which all parts are on the chip at once (one a CU).  From
+// 2 tiles on: 2 x 130 tokens, 16 heads over 16, 23 -> 26 us (a part's start and its 128 KB cost more than a tile); from 4 on: 1 x 128, 16 over 8, 24 against 19.  From 4 096 rows on the delta pass is
+// another product's epilogue, whose caller knows nothing of parts, and what it leaves is to give the same bits.
+constexpr int SPLIT_TILES = 3, SPLIT_CUS = 256;
+static int dkv_split(int B, int S, int Hq, int Hkv, int D, int causal) {
+    const int nblk = (S + 127) / 128, rep = Hq / Hkv;
+    const int64_t pairs = (int64_t)B * Hkv;
+    if (D != 128 || (int64_t)B * S >= 4096 || pairs * nblk >= SPLIT_CUS) return 0;
+    int64_t all = 0;
+    for (int kb = 0; kb < nblk; ++kb) all += dkv_tiles(S, rep, causal, kb);
+    const int longest = dkv_tiles(S, rep, causal, 0);
+    for (int64_t most = all * pairs / SPLIT_CUS > SPLIT_TILES ? all * pairs / SPLIT_CUS : SPLIT_TILES; most < longest; ++most)
+        if (pairs * dkv_blocks(S, rep, causal, (int)most, nblk) <= SPLIT_CUS) return (int)most;
+    return 0;
+}
+extern "C" int64_t mi355_attn_bwd_split_bytes(int B, int S, int Hq, int Hkv, int D, int causal) {
+    if (B <= 0 || S <= 0 || Hq <= 0 || Hkv <= 0 || Hq % Hkv || S > 64 * ATTN_MAX_TILES || (causal & MI355_ATTN_DELTA_READY)) return 0;
+    const int most = dkv_split(B, S, Hq, Hkv, D, causal & 0xff);
+    return most ? (int64_t)B * Hkv * dkv_blocks(S, Hq / Hkv, causal & 0xff, most, (S + 127) / 128) * 128 * 128 * 2 * 4 : 0;
+}
+
 // the dS scratch: one bf16 per (query, key) of the padded square
 static int64_t attn_bwd_ds_bytes(int B, int S, int Hq) {
     const int64_t nqb = (S + 127) / 128;
@@ -1702,7 +1808,8 @@ static int attn_bwd_impl(int B, int S, int Hq, int Hkv, int D, const void* q, in
     const int nblk = (S + 127) / 128;
     const int bpw_q = (int64_t)B * Hq >= 512 ? nblk : 1;
     const int bpw_k = (int64_t)B * Hkv >= 512 ? nblk : 1;
-    const int64_t gq = (int64_t)B * Hq * ((nblk + bpw_q - 1) / bpw_q), gk = (int64_t)B * Hkv * ((nblk + bpw_k - 1) / bpw_k);
+    const int64_t gq = (int64_t)B * Hq * ((nblk + bpw_q - 1) / bpw_q);
+    int64_t gk = (int64_t)B * Hkv * ((nblk + bpw_k - 1) / bpw_k);
     MI355_REQUIRE(S <= 64 * ATTN_MAX_TILES, "mi355_attn_bwd: S must be <= %d", 64 * ATTN_MAX_TILES);
     MI355_REQUIRE(gq < 0x7fffffffLL, "mi355_attn_bwd: grid too large");
     // workspace given (head_dim 128): the dK/dV pass spills dS and dQ is one product over it; otherwise the dQ pass recomputes S and dP
@@ -1717,26 +1824,38 @@ static int attn_bwd_impl(int B, int S, int Hq, int Hkv, int D, const void* q, in
     bf16_t* ds_ws = spill ? (bf16_t*)workspace : nullptr;
     float* nl2 = spill ? (float*)((char*)workspace + attn_bwd_ds_bytes(B, S, Hq)) : nullptr;
     float* ndl = spill ? (float*)((char*)nl2 + (((int64_t)B * Hq * S * 4 + 15) & ~(int64_t)15)) : nullptr;
+    // a caller whose workspace has room for them gets the key blocks of a call of few split
+    const int64_t split = spill && !delta_ready ? mi355_attn_bwd_split_bytes(B, S, Hq, Hkv, D, causal) : 0;
+    DkvFold fold{};
+    if (split && workspace_bytes >= mi355_attn_bwd_workspace_bytes(B, S, Hq, D) + split) {
+        fold = DkvFold{(const float*)((char*)workspace + mi355_attn_bwd_workspace_bytes(B, S, Hq, D)), dkv_split(B, S, Hq, Hkv, D, causal & 0xff), (bf16_t*)dk, (bf16_t*)dv, lddk, lddv};
+        gk = split / (128 * 128 * 2 * 4);
+    }
+    const int64_t gs = (int64_t)B * Hq * nblk + (fold.most ? (int64_t)B * Hkv * nblk * FOLD_WG : 0);
+    MI355_REQUIRE(gs < 0x7fffffffLL, "mi355_attn_bwd: grid too large");
 #define BWD_LAUNCH(DD)                                                                                                              \
     if (!delta_ready)                                                                                                               \
         hipLaunchKernelGGL(attn_delta_kernel<DD>, dim3(dgrid), dim3(256), 0, s, B, S, Hq, (const bf16_t*)o, ldo, (const bf16_t*)d_o, lddo, delta, lse, nl2, ndl); \
-    if (spill && DD == 128)                                                                                                         \
+    if (fold.most)                                                                                                                  \
+        hipLaunchKernelGGL((attn_bwd_dkv_kernel<128, true, true>), dim3((unsigned)gk), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, \
+                           (const bf16_t*)v, ldv, (const bf16_t*)d_o, lddo, nl2, ndl, (bf16_t*)dk, lddk, (bf16_t*)dv, lddv, key_mask, causal, scale, sl2, 1, ds_ws, fold.most, const_cast<float*>(fold.parts)); \
+    else if (spill && DD == 128)                                                                                                    \
         hipLaunchKernelGGL((attn_bwd_dkv_kernel<128, true>), dim3((unsigned)gk), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, \
-                           (const bf16_t*)v, ldv, (const bf16_t*)d_o, lddo, nl2, ndl, (bf16_t*)dk, lddk, (bf16_t*)dv, lddv, key_mask, causal, scale, sl2, bpw_k, ds_ws); \
+                           (const bf16_t*)v, ldv, (const bf16_t*)d_o, lddo, nl2, ndl, (bf16_t*)dk, lddk, (bf16_t*)dv, lddv, key_mask, causal, scale, sl2, bpw_k, ds_ws, 0, (float*)nullptr); \
     else                                                                                                                             \
         hipLaunchKernelGGL((attn_bwd_dkv_kernel<DD, false>), dim3((unsigned)gk), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, \
-                           (const bf16_t*)v, ldv, (const bf16_t*)d_o, lddo, lse, delta, (bf16_t*)dk, lddk, (bf16_t*)dv, lddv, key_mask, causal, scale, sl2, bpw_k, ds_ws); \
+                           (const bf16_t*)v, ldv, (const bf16_t*)d_o, lddo, lse, delta, (bf16_t*)dk, lddk, (bf16_t*)dv, lddv, key_mask, causal, scale, sl2, bpw_k, ds_ws, 0, (float*)nullptr); \
     if (!spill)                                                                                                                      \
         hipLaunchKernelGGL(attn_bwd_dq_kernel<DD>, dim3((unsigned)gq), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk,  \
                            (const bf16_t*)v, ldv, (const bf16_t*)d_o, lddo, lse, delta, (bf16_t*)dq, lddq, key_mask, causal, scale, sl2, bpw_q);
     if (D == 128) {
         BWD_LAUNCH(128)
         if (spill && fuse)
-            hipLaunchKernelGGL((attn_bwd_dq_spill_kernel<128, true>), dim3((unsigned)((int64_t)B * Hq * nblk)), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)k, ldk,
-                               (const bf16_t*)ds_ws, (bf16_t*)nullptr, (int64_t)0, causal & 0xff, scale, *fuse);
+            hipLaunchKernelGGL((attn_bwd_dq_spill_kernel<128, true>), dim3((unsigned)gs), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)k, ldk,
+                               (const bf16_t*)ds_ws, (bf16_t*)nullptr, (int64_t)0, causal & 0xff, scale, *fuse, fold);
         else if (spill)
-            hipLaunchKernelGGL((attn_bwd_dq_spill_kernel<128, false>), dim3((unsigned)((int64_t)B * Hq * nblk)), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)k, ldk,
-                               (const bf16_t*)ds_ws, (bf16_t*)dq, lddq, causal & 0xff, scale, QkFuse{});
+            hipLaunchKernelGGL((attn_bwd_dq_spill_kernel<128, false>), dim3((unsigned)gs), dim3(256), 0, s, B, S, Hq, Hkv, (const bf16_t*)k, ldk,
+                               (const bf16_t*)ds_ws, (bf16_t*)dq, lddq, causal & 0xff, scale, QkFuse{}, fold);
     } else {
         BWD_LAUNCH(64)
     }

@@ -59,6 +59,8 @@ Slot* const slots[] = {
 using WorkspaceBytes = int64_t (*)(int, int, int, int);
 using Partials = int64_t (*)(int, int, int);
 WorkspaceBytes attn_bwd_workspace_bytes;
+using SplitBytes = int64_t (*)(int, int, int, int, int, int);
+SplitBytes attn_bwd_split_bytes;
 Partials attn_bwd_qnorm_partials;
 
 void need(bool holds) {
@@ -470,6 +472,15 @@ T attn_scratch(Call& c, const T& beside, int64_t bytes) {
     Py_DECREF(got);
     return t;
 }
+// kernels._attn_split_scratch: `bytes` and room for the parts of split key blocks, or `bytes` alone
+T attn_split_scratch(Call& c, const T& beside, int64_t& bytes, int B, int S, int Hq, int Hkv, int D, int causal) {
+    if (const int64_t more = attn_bwd_split_bytes(B, S, Hq, Hkv, D, causal))
+        if (T t = attn_scratch(c, beside, bytes + more)) {
+            bytes += more;
+            return t;
+        }
+    return attn_scratch(c, beside, bytes);
+}
 void count_form(const char* form) {  // kernels.attn_bwd_form[form] += 1
     PyObject* all = kernels_item("attn_bwd_form");
     PyObject* n = PyDict_GetItemString(all, form);
@@ -483,7 +494,7 @@ OP(attn_bwd, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", "dq", 
     need(D > 0);
     for (const T* t : {&q, &o, &dO, &dq}) need(attn_operand(*t, B * S, Hq * D));
     for (const T* t : {&k, &v, &dk, &dv}) need(attn_operand(*t, B * S, Hkv * D));
-    need(lse.is(F32) && lse.contiguous() && lse.shape({B, Hq, S}) && attn_bwd_workspace_bytes && (dry || slot::attn_bwd_ws.address));
+    need(lse.is(F32) && lse.contiguous() && lse.shape({B, Hq, S}) && attn_bwd_workspace_bytes && attn_bwd_split_bytes && (dry || slot::attn_bwd_ws.address));
     const double scale = c.given(16) ? c.real(16) : std::pow((double)D, -0.5);
     const int flags = (int)c.truth(15, true) | (int)kernels_int("_ATTN_ABLATE");
     const T delta = c.empty_like(lse);
@@ -491,7 +502,7 @@ OP(attn_bwd, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", "dq", 
     T ws;
     if (!dry) c.get_ready();
     if (bytes) {
-        ws = attn_scratch(c, q, bytes);
+        ws = attn_split_scratch(c, q, bytes, B, S, Hq, Hkv, D, c.truth(15, true));
         if (!ws) bytes = 0;  // (over the cap, or no memory: the recompute form)
     }
     count_form(bytes ? "spill" : "recompute");
@@ -511,12 +522,12 @@ OP(attn_bwd_qnorm, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", 
     need(rstd.is(F32) && rstd.dim() == 2 && rstd.contiguous() && rstd.size(0) == B * S && rstd.size(1) >= Hq && qw.is(BF16) && qw.numel() == D);
     need(cos.is(F32) && sin.is(F32) && cos.contiguous() && sin.contiguous() && cos.dim() >= 1 && cos.size(cos.dim() - 1) == D && pos.is(I32) && pos.numel() == B * S);
     need(!delta || (delta.is(F32) && delta.contiguous() && delta.like(lse)));
-    need(attn_bwd_workspace_bytes && attn_bwd_qnorm_partials && (dry || (slot::attn_bwd_qnorm.address && slot::reduce_rows_f32.address)));
+    need(attn_bwd_workspace_bytes && attn_bwd_split_bytes && attn_bwd_qnorm_partials && (dry || (slot::attn_bwd_qnorm.address && slot::reduce_rows_f32.address)));
     const double scale = c.given(22) ? c.real(22) : std::pow((double)D, -0.5);
     int flags = (int)c.truth(21, true) | (int)kernels_int("_ATTN_ABLATE");
     if (!dry) c.get_ready();
-    const int64_t bytes = attn_bwd_workspace_bytes(B, S, Hq, D);
-    const T ws = bytes ? attn_scratch(c, q, bytes) : T{};
+    int64_t bytes = attn_bwd_workspace_bytes(B, S, Hq, D);
+    const T ws = !bytes ? T{} : delta ? attn_scratch(c, q, bytes) : attn_split_scratch(c, q, bytes, B, S, Hq, Hkv, D, c.truth(21, true));
     need(bool(ws));
     PyObject* cs = PyObject_CallFunctionObjArgs(kernels_item("rope_cs16"), c.v[15], c.v[16], nullptr);
     if (!cs) throw Raised();
@@ -1250,6 +1261,7 @@ PyObject* bind(PyObject*, PyObject* args) {
     if (!PyArg_ParseTuple(args, "sK", &name, &address)) return nullptr;
     void* at = reinterpret_cast<void*>(address);
     if (!strcmp(name, "mi355_attn_bwd_workspace_bytes")) attn_bwd_workspace_bytes = reinterpret_cast<WorkspaceBytes>(at);
+    if (!strcmp(name, "mi355_attn_bwd_split_bytes")) attn_bwd_split_bytes = reinterpret_cast<SplitBytes>(at);
     if (!strcmp(name, "mi355_attn_bwd_qnorm_partials")) attn_bwd_qnorm_partials = reinterpret_cast<Partials>(at);
     for (Slot* s : slots)
         if (!strcmp(s->name, name)) s->address = at;

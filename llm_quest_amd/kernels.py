@@ -461,6 +461,15 @@ def _attn_scratch(device, nbytes):
     return ws
 
 
+def _attn_split_scratch(device, need, B, S, Hq, Hkv, D, causal):
+    """The dS scratch with room for the parts of split key blocks behind it where a call has them: (scratch or None, bytes)."""
+    more = L.load().mi355_attn_bwd_split_bytes(B, S, Hq, Hkv, D, int(causal))
+    ws = _attn_scratch(device, need + more) if more else None
+    if ws is not None:
+        return ws, need + more
+    return _attn_scratch(device, need), need
+
+
 @L.native
 def attn_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=None, causal=True, scale=None):
     """q [B*S,Hq*D], k/v [B*S,Hkv*D] (row-strided views allowed).  Returns (o [B*S,Hq*D], lse fp32 [B,Hq,S])."""
@@ -489,7 +498,7 @@ def attn_bwd(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dq, dk, dv, key_mask=None, c
     scale = D ** -0.5 if scale is None else scale
     ws, need = None, L.load().mi355_attn_bwd_workspace_bytes(B, S, Hq, D) if _ATTN_DS_SPILL else 0
     if need:
-        ws = _attn_scratch(q.device, need)
+        ws, need = _attn_split_scratch(q.device, need, B, S, Hq, Hkv, D, causal)
         if ws is None:
             need = 0  # over the cap / no memory: the recompute form (mi355_attn_bwd_ws with a NULL workspace)
     attn_bwd_form["spill" if need else "recompute"] += 1
@@ -578,7 +587,10 @@ def attn_bwd_qnorm(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dk, dv, qkv, qw, cos, 
             and cos.dtype == F32 and sin.dtype == F32 and cos.is_contiguous() and sin.is_contiguous() and cos.shape[-1] == D and pos.dtype == torch.int32 and pos.numel() == B * S):
         raise ValueError("attn_bwd_qnorm: qkv / dqkv bf16 [B*S, >=Hq*D], rstd fp32 [B*S, heads], q weight bf16 [D], cos / sin fp32 [positions, D], pos int32 [B*S]")
     need = L.load().mi355_attn_bwd_workspace_bytes(B, S, Hq, D)
-    ws = _attn_scratch(q.device, need) if need else None
+    if delta is None:
+        ws, need = _attn_split_scratch(q.device, need, B, S, Hq, Hkv, D, causal) if need else (None, 0)
+    else:  # (dgrad_attn_delta left the row constants in the scratch of this size)
+        ws = _attn_scratch(q.device, need) if need else None
     if ws is None:
         return None
     attn_bwd_form["spill"] += 1

@@ -479,6 +479,44 @@ def test_attention_backward_scratch_form_equals_recompute_form(K, B, S, Hq, Hkv,
                L.ptr(lse), L.ptr(delta), L.ptr(dq), dq.stride(0), L.ptr(dk), dk.stride(0), L.ptr(dv), dv.stride(0), L.ptr(km), int(causal), D ** -0.5, L.ptr(ws), need - 16)
 
 
+@pytest.mark.parametrize(
+    "B,S,Hq,Hkv,causal,ragged",
+    [(1, 1, 2, 1, True, False), (1, 128, 16, 8, True, False), (1, 129, 3, 1, True, False), (2, 498, 16, 8, True, True), (1, 709, 4, 1, True, False), (1, 2000, 4, 2, False, True), (7, 584, 4, 4, True, False),
+     (1, 4095, 2, 2, True, False), (8, 512, 2, 1, True, False)],
+)
+def test_attention_backward_of_split_key_blocks(K, B, S, Hq, Hkv, causal, ragged):
+    """Key blocks cut into parts (where the workspace has room for them) against whole ones: dQ the same bits, dK and dV the same fp32 products in sums of parts, so one bf16 rounding apart (2^-8 of
+    a value at most where both fall to either side), the same bits twice, nothing written beyond a row's heads; and which calls are cut."""
+    from llm_quest_amd import _lib as L
+
+    D = 128
+    g = torch.Generator().manual_seed(S)
+    q, k, v, do = (dev(torch.randn(B * S, w * D, generator=g).to(BF16)) for w in (Hq, Hkv, Hkv, Hq))
+    km = None
+    if ragged:
+        km = torch.ones(B, S, dtype=torch.uint8)
+        km[0, S - S // 3 :] = 0
+        km = dev(km)
+    o, lse = K.attn_fwd(q, k, v, B, S, Hq, Hkv, D, key_mask=km, causal=causal)
+    base, more = L.load().mi355_attn_bwd_workspace_bytes(B, S, Hq, D), L.load().mi355_attn_bwd_split_bytes(B, S, Hq, Hkv, D, int(causal))
+    assert more % (128 * 128 * 8) == 0 and more <= 256 * 128 * 128 * 8 and (more > 0) == (B * S < 4096 and S > 1) and L.load().mi355_attn_bwd_split_bytes(B, S, Hq, Hkv, 64, 1) == 0
+    delta = torch.empty_like(lse)
+    outs = []
+    for room in (base, base + more, base + more):
+        ws = torch.full((room,), 255, dtype=torch.uint8, device="cuda")  # (NaNs: nothing may be read that the call did not write)
+        dq = torch.empty_like(q)
+        dk, dv = (torch.full((B * S, Hkv * D + 8), 7.0, dtype=BF16, device="cuda") for _ in range(2))
+        L.require_gpu(q, ws)
+        L.call("mi355_attn_bwd_ws", B, S, Hq, Hkv, D, L.ptr(q), q.stride(0), L.ptr(k), k.stride(0), L.ptr(v), v.stride(0), L.ptr(o), o.stride(0), L.ptr(do), do.stride(0),
+               L.ptr(lse), L.ptr(delta), L.ptr(dq), dq.stride(0), L.ptr(dk), dk.stride(0), L.ptr(dv), dv.stride(0), L.ptr(km), int(causal), D ** -0.5, L.ptr(ws), room)
+        assert bool((dk[:, Hkv * D :] == 7).all()) and bool((dv[:, Hkv * D :] == 7).all())
+        outs.append((dq, dk, dv))
+    assert torch.equal(outs[0][0], outs[1][0]) and all(torch.equal(a, b) for a, b in zip(outs[1], outs[2]))
+    for a, b in zip(outs[0][1:], outs[1][1:]):
+        a, b = a.float(), b.float()
+        assert float(((a - b).abs() - 2**-7 * a.abs()).max()) < 1e-5 * float(a.abs().max()) and rel_l2(b, a) < 2**-9
+
+
 def test_attention_backward_scratch_is_capped_and_falls_back_to_the_recompute_form(K, monkeypatch):
     """The dS scratch grows with S^2; above the cap (MI355_ATTN_DS_SPILL_MAX_MB) -- or without memory for it -- ``attn_bwd`` must take the
     O(S)-memory recompute form instead of allocating: S = 4096, B = 4 with the cap lowered under the 1 GiB this shape asks for.  Checked against
