@@ -6,8 +6,8 @@
 // Which sequences of a step go this way is their own number of new tokens' affair (`from`): beside a long prompt, a short one and a single token
 // get the bits that they get alone -- of the delta rule inside the scan's launch, whose long chains hide them; of retention by mi355_gla_fwd_below.
 // A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
-// the chip could multiply; the chunks take 359 us and 188 us.  Bound: the scan's chain of chunks (two products behind two barriers each), not the
-// pipe.  In the scan the first product's rows are requested in two halves: all at once 286 us and a chunk ahead 262 (the registers spill).
+// the chip could multiply; the chunks take 354 us and 183 us.  Bound: the scan's chain of chunks (two products behind two barriers each), not the
+// pipe.
 // Chains of 128 products on the matrix pipe are cut (add16): outputs' distance to 64 bits, token by token | here with whole chains | here: 1.29e-7 | 2.32e-7 | 1.73e-7, decays near zero
 // 1.19e-7 | 2.27e-7 | 1.45e-7, nearly parallel keys 1.29e-7 | 2.67e-7 | 1.90e-7, decays near one 4.7e-7 | 5.0e-7 | 4.7e-7, retention 3.1e-7 | 3.0e-7 | 2.6e-7; 6 of the 363 us that the six prompts took.
 // A chunk whose U is not finite and all behind it go token by token inside the scan: the triangles' zeros are multiplied, not skipped, and a token's key, value, decay or beta that
@@ -147,20 +147,20 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
 }
 
 // One workgroup per sequence, head and 32 value columns, chunk by chunk.  Waves 0, 1 take Kw S (row halves), waves 2, 3 q S and then P U; the state's four tiles of 32 key
-// channels go one to a wave.
+// channels go one to a wave.  Every operand of a chunk is requested a chunk ahead, by each side for itself: six prompts of 900 tokens, 16 heads, 219 -> 184 us (retention 180 -> 158), one of 2 000
+// 266 -> 236 with its prep; in one loop for both sides 230 (registers spill, and waits count every store).
 template <bool DELTA>
 __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
     __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];  // [value column][key channel]
     __shared__ __attribute__((aligned(16))) float Us[GC][GV + 8];
     __shared__ __attribute__((aligned(16))) float Ks[GC][GD + 4];
-    __shared__ float gg[2 * GC], gC;
+    __shared__ float gg[2][256];  // gam, Gp and the chunk's decay (a word a thread: a condition would take the request with it, to where it is used)
     __shared__ int lost[2];  // a chunk's flag: set by its U, cleared a chunk later
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5, rh = wave & 1;
     // the four value ranges of a head read the same rows: to one XCD (workgroups are dealt to the eight XCDs in turn), side by side
     const int id = blockIdx.x, at = (id >> 5) * 8 + (id & 7), v0 = ((id >> 3) & 3) * GV;
     if (at >= p.heads) return;
     const int h = at % p.H, s = at / p.H, hq = h / (p.H / p.G), s0 = p.seq_off[s], len = p.seq_off[s + 1] - s0, NC = (len + GC - 1) / GC;
-    const bool qside = wave >= 2;
     const float *qp = p.q + (int64_t)s0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)s0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)s0 * p.ldv + (int64_t)h * GD + v0;
     float* state = p.state + ((int64_t)p.slot[s] * p.H + h) * GD * GD + v0;
     if (NC <= 0) return;
@@ -177,106 +177,127 @@ __global__ __launch_bounds__(256, 2) void dchunk_scan_kernel(DChunkArgs p) {
         if (DELTA) by_token(s0, s0 + len, state, GD, 1);
         return;
     }
+    const int row = 32 * rh + ln;
+    const float* first = chunk_block(p, s, h, 0);
+    const int64_t block = (int64_t)p.H * D_BLOCK;
     if (tid < 2) lost[tid] = 0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;
-        Ss[c][r] = state[(int64_t)r * GD + c];
-    }
     int n = 0;
-    for (; n < NC; ++n) {
-        const float* blk = chunk_block(p, s, h, n);
-        const int t0 = n * GC, cnt = min(GC, len - t0);
-        // a Kw row (waves 0, 1) or a q row (waves 2, 3) in fragment form, eight words in flight
-        const int row = 32 * rh + ln;
-        const float* src = qside ? qp + (t0 + row) * p.ldq + 4 * hf : DELTA ? blk + D_KW + row * GD + 4 * hf : nullptr;
-        if (qside && row >= cnt) src = nullptr;
-        f32x4 fr[8];
+    // The two sides' waves run loops of their own (the barriers are counted by wave, not by place): in one loop a wait for a chunk's operands cannot be counted over the other side's
+    // requests and stores and becomes a wait for all of them, and both sides' registers are live at once.
+    auto chunks = [&](auto side) {
+        constexpr bool Q = decltype(side)::value;
+        // what a chunk reads: a Kw row, or a q row and a P row, in fragment form; keys; U before the state's part; its decays.  (Loads carry no condition: rows beyond the sequence are its
+        // last; of queries they give rows that are not written, keys and values are dropped where they are used.)
+        f32x4 fr[16], kr[8], pr[8];
+        float uv[16], gr;
+        auto request = [&](int n) {
+            const float* blk = first + n * block;
+            const int t0 = n * GC, last = min(GC, len - t0) - 1;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) fr[i] = src ? *reinterpret_cast<const f32x4*>(src + 8 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
-        __syncthreads();  // the state is whole, the last chunk's keys and U are read
-        f32x4 kr[8], pr[8];
-        f32x16 uv = zero16();
+            for (int i = 0; i < 8; ++i) kr[i] = *reinterpret_cast<const f32x4*>(kp + t0 * p.ldk + min((tid >> 5) + 8 * i, last) * p.ldk + (tid & 31) * 4);
+            gr = blk[D_G + min(tid, 2 * GC)];
+            if (Q || DELTA) {
+                const float* src = Q ? qp + t0 * p.ldq + min(row, last) * p.ldq + 4 * hf : blk + D_KW + row * GD + 4 * hf;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-            kr[i] = r < cnt ? *reinterpret_cast<const f32x4*>(kp + (t0 + r) * p.ldk + c) : f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-        if (!qside) {
+                for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(src + 8 * i);
+            }
+            if (!Q) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const int r = 32 * rh + c_row(e, hf);
+                    uv[e] = DELTA ? (blk + D_U + v0)[r * GD + ln] : (vp + t0 * p.ldv)[min(r, last) * p.ldv + ln];
+                }
+            }
+        };
+        auto request_p = [&](int n) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) pr[i] = *reinterpret_cast<const f32x4*>(first + n * block + D_P + row * GC + 4 * hf + 8 * i);
+        };
+        auto put_out = [&](int t0, int cnt, const f32x16& x) {  // rows beyond the sequence: beyond the buffer, dropped
+            auto rs = __builtin_amdgcn_make_buffer_rsrc(p.o + ((int64_t)s0 + t0) * p.H * GD + (int64_t)h * GD + v0, 0, 0x7fffffff, 0x00020000);
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = 32 * rh + c_row(e, hf);
-                if (DELTA) uv[e] = blk[D_U + r * GD + v0 + ln];
-                else uv[e] = r < cnt ? vp[(t0 + r) * p.ldv + ln] : 0.f;
+                __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(x[e]), rs, r < cnt ? (r * p.H * GD + ln) * 4 : -1, 0, 0);
             }
+        };
+        request(0);
+        if (Q) request_p(0);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {  // (behind the first chunk's requests: one latency for both)
+            const int idx = tid + 256 * i, r = idx >> 5, c = idx & 31;
+            Ss[c][r] = state[(int64_t)r * GD + c];
         }
-        if (tid < 2 * GC) gg[tid] = blk[D_G + tid];
-        if (tid == 0) gC = blk[D_G + 2 * GC], lost[(n + 1) & 1] = 0;
-        f32x16 acc = zero16();
-        if (DELTA || qside) {
+        if (Q) {
 #pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                const f32x4 c = *reinterpret_cast<const f32x4*>(&Ss[ln][8 * i + 4 * hf]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc = mfma2(fr[i % 8][j], c[j], acc);
-                if (i == 7) {  // (as add16: what is left of U, or minus the first half of q S)
-#pragma unroll
-                    for (int e = 0; e < 16; ++e) {
-                        uv[e] -= acc[e];
-                        acc[e] = 0.f;
-                    }
-                }
-                if (i < 8) fr[i] = src ? *reinterpret_cast<const f32x4*>(src + 8 * (i + 8)) : f32x4{0.f, 0.f, 0.f, 0.f};
-                if (i % 4 == 3) asm volatile("" ::: "memory");  // keep the state reads of later steps where they are: all sixteen at once cost more registers than there are
-            }
+            for (int i = 0; i < 16; ++i) asm volatile("" : "+v"(fr[i])::"memory");  // (landed before the loop, where only its own requests are then waited for)
+            put_out(0, 0, zero16());  // (dropped whole: sixteen stores behind P's request from either way in)
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-            *reinterpret_cast<f32x4*>(&Ks[r][c]) = kr[i];
-        }
-        if (qside) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) pr[i] = *reinterpret_cast<const f32x4*>(blk + D_P + (32 * rh + ln) * GC + 8 * i + 4 * hf);
-        } else {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                acc[e] = uv[e] - acc[e];
-                Us[32 * rh + c_row(e, hf)][ln] = acc[e];
-            }
-            if (__any(lost16(acc)) && lane == 0) lost[n & 1] = 1;
-        }
-        __syncthreads();
-        const int gone = lost[n & 1];
-        if (qside) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) acc[e] = (acc[e] - uv[e]) * gg[32 * rh + c_row(e, hf)];
+        gg[0][tid] = gr;
+        for (; n < NC; ++n) {
+            const int t0 = n * GC, cnt = min(GC, len - t0);
+            const float* g = gg[n & 1];
+            __syncthreads();  // the state is whole, the last chunk's keys and U are read
+            if (tid == 0) lost[(n + 1) & 1] = 0;
 #pragma unroll
             for (int i = 0; i < 8; ++i) {
-                if (rh == 0 && i >= 4) break;  // P is lower triangular
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc = mfma2(pr[i][j], Us[8 * i + 4 * hf + j][ln], acc);
+                const int r = (tid >> 5) + 8 * i;
+                *reinterpret_cast<f32x4*>(&Ks[r][(tid & 31) * 4]) = r < cnt ? kr[i] : f32x4{0.f, 0.f, 0.f, 0.f};
             }
+            f32x16 acc = zero16(), half = zero16();
+            if (DELTA || Q) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int r = 32 * rh + c_row(e, hf);
-                if (r < cnt) p.o[((int64_t)s0 + t0 + r) * p.H * GD + (int64_t)h * GD + v0 + ln] = acc[e];
+                for (int i = 0; i < 16; ++i) {
+                    const f32x4 c = *reinterpret_cast<const f32x4*>(&Ss[ln][8 * i + 4 * hf]);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc = mfma2(fr[i][j], c[j], acc);
+                    if (i == 7) add16(half, acc);
+                }
             }
+            if (!Q) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float v = DELTA || 32 * rh + c_row(e, hf) < cnt ? uv[e] : 0.f;
+                    acc[e] = (v - half[e]) - acc[e];
+                    Us[32 * rh + c_row(e, hf)][ln] = acc[e];
+                }
+                if (__any(lost16(acc)) && lane == 0) lost[n & 1] = 1;
+            }
+            __syncthreads();
+            const int gone = lost[n & 1];
+            request(min(n + 1, NC - 1));  // (the last chunk's own once more: nothing here hangs on a condition)
+            if (Q) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) acc[e] = (acc[e] + half[e]) * g[32 * rh + c_row(e, hf)];
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    if (rh == 0 && i >= 4) break;  // P is lower triangular
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) acc = mfma2(pr[i][j], Us[8 * i + 4 * hf + j][ln], acc);
+                }
+                request_p(min(n + 1, NC - 1));
+                asm volatile("" ::: "memory");  // (the stores behind the requests: waits for those then leave the stores alone)
+                put_out(t0, cnt, acc);
+            }
+            if (gone) break;  // (the same for the whole workgroup)
+            f32x16 c;
+            const float gC = g[2 * GC];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) c[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
+#pragma unroll
+            for (int kb = 0; kb < GC; kb += 8)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    const int t = kb + 4 * hf + j;
+                    c = mfma2(Us[t][ln] * g[GC + t], Ks[t][32 * wave + ln], c);
+                }
+#pragma unroll
+            for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = c[e];  // read by this wave alone since the last barrier
+            gg[(n + 1) & 1][tid] = gr;
         }
-        if (gone) break;  // (the same for the whole workgroup)
-        f32x16 c;
-#pragma unroll
-        for (int e = 0; e < 16; ++e) c[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
-#pragma unroll 2
-        for (int kb = 0; kb < GC; kb += 8)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                const int t = kb + 4 * hf + j;
-                c = mfma2(Us[t][ln] * gg[GC + t], Ks[t][32 * wave + ln], c);
-            }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = c[e];  // read by this wave alone since the last barrier
-    }
+    };
+    if (wave >= 2) chunks(std::true_type{});
+    else chunks(std::false_type{});
     if (n < NC) {
         __threadfence();
         __syncthreads();  // what the chunk wrote of its outputs lies below what comes

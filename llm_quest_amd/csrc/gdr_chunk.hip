@@ -179,7 +179,8 @@ __global__ __launch_bounds__(256, 2) void gdrc_prep_kernel(int S, int n0, int ke
 // its three bf16 parts in LDS for the next chunk's products; so does U, for P U.  The state's own sum, S <- gam_63 S + (Gp U)^T K, stays on the fp32 pipe: on the bf16 pipe a chain's
 // roundings differ, and where decays are strong the state is one such rounding from exact (4.4e-8 against 5.2e-8 from 64 bits; as it is 4.3e-8), for no time gained.  Bound: the chain of chunks
 // and the bytes (8 x 708 tokens x 16 heads: 344 MB, 70 us): two products behind two barriers, every operand of the next chunk requested under this one's second half.
-// 172 -> 148 us at 8 x 708 tokens x 16 heads, 58 -> 45 at 333 tokens (the state in fp32 in LDS, read by both sides' fp32 products, a chunk's operands requested at its own top).
+// 172 -> 148 us at 8 x 708 tokens x 16 heads, 58 -> 45 at 333 tokens (the state in fp32 in LDS, read by both sides' fp32 products, a chunk's operands requested at its own top) -> 136 and 37 with a
+// loop for each side.
 constexpr int SP = GV * (GD + 8), UP = GV * (GC + 8);  // planes of S [32 v][128 k] and U^T [32 v][64 t]
 __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int n0, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k,
                                                            const bf16_t* __restrict__ v, int64_t ldv, const float* __restrict__ beta, const float* __restrict__ alpha, float* __restrict__ saved,
@@ -188,147 +189,153 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
     __shared__ __attribute__((aligned(16))) bf16_t Ut[3 * UP];
     __shared__ __attribute__((aligned(16))) float Ug[GV][GC + 4];  // Gp U
     __shared__ __attribute__((aligned(16))) bf16_t Ks[GC][GD + 8];
-    __shared__ __attribute__((aligned(16))) float gg[2][2 * GC];
+    __shared__ __attribute__((aligned(16))) float gg[2][256];  // gam and Gp (a word a thread: a condition would take the request with it, to where it is used)
     __shared__ int lost[2];  // a chunk's flag: set by its U, cleared a chunk later
     static_assert(GV * (GD + 4) * 4 <= 3 * SP * 2, "the recurrence's state lies where the planes were");
     float(*Ss)[GD + 4] = reinterpret_cast<float(*)[GD + 4]>(Sp);
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5, rh = wave & 1;
     int at, v0;
     if (!scan_place(heads, at, v0)) return;
     const int h = at % Hv, b = at / Hv, hq = h / (Hv / Hqk);
-    const bool qside = wave >= 2;
     const int64_t ldqk = (int64_t)Hqk * GD, head = at;
     const bf16_t *qp = q + (int64_t)b * S * ldqk + hq * GD, *kp = k + (int64_t)b * S * ldqk + hq * GD;
     const int64_t block = keep ? G_BLOCK : G_SMALL;
     float* base = saved + head * NC * block + (keep ? G_KW : 0);
     const int row = 32 * rh + ln, col = 32 * wave + 4 * hf;  // the lane's row of a fragment; its first column of the state
-    // (a chunk's addresses: a scalar base and 32 bits a lane, or they take more registers than there are)
-    const unsigned kw_at = row * GD + 8 * hf, p_at = row * GC + 8 * hf, q_at = row * (unsigned)ldqk + 8 * hf, u_at = (32 * rh + 4 * hf) * GD + ln, s_at = ln * GD + col, k_at = (tid >> 4) * (unsigned)ldqk + (tid & 15) * 8,
-                   k_step = 16 * (unsigned)ldqk, o_at = (32 * rh + 4 * hf) * (unsigned)(Hv * GD) + ln, o_step = Hv * GD;
-    // what a chunk reads: a Kw row (waves 0, 1) or a Q row and a P row (waves 2, 3) in fragment form; K; U before the state's part; its decays
-    f32x4 fr[16];
-    u32x4 kr[4];
-    float uv[16], gr = 0.f;
-    auto request = [&](int n) {
-        const float* blk = base + n * block;
-        const int t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
-        if (!qside) {
-#pragma unroll
-            for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(blk + kw_at + 16 * (i >> 1) + 4 * (i & 1));
-            const float* ub = blk + C_U + v0;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) uv[e] = ub[u_at + c_row(e, 0) * GD];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) fr[i] = row < cnt ? *reinterpret_cast<const f32x4*>(qp + t0 * ldqk + q_at + 16 * i) : f32x4{0.f, 0.f, 0.f, 0.f};
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) kr[i] = (tid >> 4) + 16 * i < cnt ? *reinterpret_cast<const u32x4*>(kp + t0 * ldqk + (k_at + i * k_step)) : u32x4{0u, 0u, 0u, 0u};
-        if (tid < 2 * GC) gr = blk[C_GAM + tid];
-    };
-    auto request_p = [&](int n) {
-        if (qside) {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) fr[8 + i] = *reinterpret_cast<const f32x4*>(base + n * block + C_P + p_at + 16 * (i >> 1) + 4 * (i & 1));
-        }
-    };
     f32x16 s;  // S[v0 + ln][32 wave + c_row(e, hf)]
-#pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        f32x4 x = {0.f, 0.f, 0.f, 0.f};
-        if (initial_state) x = *reinterpret_cast<const f32x4*>(initial_state + (head * GD + v0 + ln) * GD + col + 8 * c);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) s[4 * c + e] = x[e];
-    }
     auto put_state = [&]() {
 #pragma unroll
         for (int c = 0; c < 4; ++c) put_parts<SP>(Sp, ln * (GD + 8) + col + 8 * c, s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]);
     };
-    put_state();
-    request(0);
-    request_p(0);
     if (tid < 2) lost[tid] = 0;
-    if (tid < 2 * GC) gg[0][tid] = gr;
     int n = 0;
-    for (; n < NC; ++n) {
-        float* blk = base + n * block;
-        const int t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
-        const float* g = gg[n & 1];
-        __syncthreads();  // the state is whole, the last chunk's K and U are read
-        if (tid == 0) lost[(n + 1) & 1] = 0;
-        if (keep) {
+    // The two sides' waves run loops of their own (the barriers are counted by wave, not by place): in one loop a wait for a chunk's operands cannot be counted over the other side's
+    // requests and stores and becomes a wait for every store before it.
+    auto chunks = [&](auto side) {
+        constexpr bool Q = decltype(side)::value;
+        // what a chunk reads: a Kw row, or a Q row and a P row, in fragment form; K; U before the state's part; its decays.  (Loads carry no condition: rows beyond the sequence are its
+        // last; of queries they give rows that are not written, keys are dropped where they are used.)
+        f32x4 fr[16];
+        u32x4 kr[4];
+        float uv[16], gr;
+        auto request = [&](int n) {
+            const float* blk = base + n * block;
+            const int t0 = (n0 + n) * GC, last = min(GC, S - t0) - 1;
 #pragma unroll
-            for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(blk - G_KW + v0 * GD + s_at + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
-        }
+            for (int i = 0; i < 4; ++i) kr[i] = *reinterpret_cast<const u32x4*>(kp + t0 * ldqk + (min((tid >> 4) + 16 * i, last) * (unsigned)ldqk + (tid & 15) * 8));
+            gr = blk[C_GAM + min(tid, 2 * GC - 1)];
+            if (Q) {
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
-            *reinterpret_cast<u32x4*>(&Ks[r][c]) = kr[i];
-        }
-        f32x16 hi = zero16(), lo = zero16();
-        if (!qside) {
+                for (int i = 0; i < 8; ++i) fr[i] = *reinterpret_cast<const f32x4*>(qp + t0 * ldqk + (min(row, last) * (unsigned)ldqk + 8 * hf) + 16 * i);
+            } else {
 #pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                mfma_parts(parts8(fr[2 * i], fr[2 * i + 1]), parts_at<SP>(Sp, ln * (GD + 8) + 16 * i + 8 * hf), hi, lo);
-                if (i & 1) asm volatile("" ::: "memory");  // keep the reads of later steps where they are: all at once cost more registers than there are
+                for (int i = 0; i < 16; ++i) fr[i] = *reinterpret_cast<const f32x4*>(blk + row * GD + 8 * hf + 16 * (i >> 1) + 4 * (i & 1));
+#pragma unroll
+                for (int e = 0; e < 16; ++e) uv[e] = (blk + C_U + v0)[(32 * rh + c_row(e, hf)) * GD + ln];
             }
-            f32x16 u;
+        };
+        auto request_p = [&](int n) {
 #pragma unroll
-            for (int e = 0; e < 16; ++e) u[e] = uv[e] - (hi[e] + lo[e]);
-#pragma unroll
-            for (int c = 0; c < 4; ++c) {
-                const int t = 32 * rh + 8 * c + 4 * hf;
-                const f32x4 G = *reinterpret_cast<const f32x4*>(g + GC + t);
-                put_parts<UP>(Ut, ln * (GC + 8) + t, u[4 * c], u[4 * c + 1], u[4 * c + 2], u[4 * c + 3]);
-                *reinterpret_cast<f32x4*>(&Ug[ln][t]) = f32x4{u[4 * c] * G[0], u[4 * c + 1] * G[1], u[4 * c + 2] * G[2], u[4 * c + 3] * G[3]};
-            }
-            if (__any(lost16(u)) && lane == 0) lost[n & 1] = 1;
-#pragma unroll
-            for (int e = 0; e < 16; ++e) (blk + C_U + v0)[u_at + c_row(e, 0) * GD] = u[e];
-        } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                mfma_parts(__builtin_bit_cast(bf16x8, fr[i]), parts_at<SP>(Sp, ln * (GD + 8) + 16 * i + 8 * hf), hi, lo);
-                if (i & 1) asm volatile("" ::: "memory");
-            }
-        }
-        __syncthreads();
-        const int gone = lost[n & 1];
-        if (n + 1 < NC) request(n + 1);
-        if (qside) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const float f = g[32 * rh + c_row(e, hf)] * qscale;
-                hi[e] *= f;
-                lo[e] *= f;
-            }
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (rh == 0 && i >= 2) break;  // P is lower triangular
-                mfma_parts(parts8(fr[8 + 2 * i], fr[9 + 2 * i]), parts_at<UP>(Ut, ln * (GC + 8) + 16 * i + 8 * hf), hi, lo);
-                asm volatile("" ::: "memory");
-            }
-            if (n + 1 < NC) request_p(n + 1);
+            for (int i = 0; i < 8; ++i) fr[8 + i] = *reinterpret_cast<const f32x4*>(base + n * block + C_P + row * GC + 8 * hf + 16 * (i >> 1) + 4 * (i & 1));
+        };
+        auto put_out = [&](int t0, int cnt, const f32x16& x) {  // rows beyond the sequence: beyond the buffer, dropped
+            auto rs = __builtin_amdgcn_make_buffer_rsrc(o + (((int64_t)b * S + t0) * Hv + h) * GD + v0, 0, 0x7fffffff, 0x00020000);
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
                 const int r = 32 * rh + c_row(e, hf);
-                if (r < cnt) (o + (((int64_t)b * S + t0) * Hv + h) * GD + v0)[o_at + c_row(e, 0) * o_step] = f2bf(hi[e] + lo[e]);
+                __builtin_amdgcn_raw_buffer_store_b16(f2bf(x[e]), rs, r < cnt ? (r * Hv * GD + ln) * 2 : -1, 0, 0);
             }
-        }
-        if (gone) break;  // (the same for the whole workgroup)
-        const float gC = g[GC - 1];
+        };
+        request(0);
+        if (Q) request_p(0);
 #pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] *= gC;
+        for (int c = 0; c < 4; ++c) {  // (behind the first chunk's requests: one latency for both)
+            f32x4 x = {0.f, 0.f, 0.f, 0.f};
+            if (initial_state) x = *reinterpret_cast<const f32x4*>(initial_state + (head * GD + v0 + ln) * GD + col + 8 * c);
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const f32x4 d = *reinterpret_cast<const f32x4*>(&Ug[ln][8 * i + 4 * hf]);
-#pragma unroll
-            for (int j = 0; j < 4; ++j) s = mfma2(bf2f(Ks[8 * i + 4 * hf + j][32 * wave + ln]), d[j], s);
-            if (i & 1) asm volatile("" ::: "memory");
+            for (int e = 0; e < 4; ++e) s[4 * c + e] = x[e];
         }
         put_state();
-        if (tid < 2 * GC) gg[(n + 1) & 1][tid] = gr;
-    }
+        if (Q) {
+#pragma unroll
+            for (int i = 0; i < 8; ++i) asm volatile("" : "+v"(fr[i])::"memory");  // (landed before the loop, where only its own requests are then waited for)
+            put_out(n0 * GC, 0, s);  // (dropped whole: sixteen stores behind P's request from either way in)
+        }
+        gg[0][tid] = gr;
+        for (; n < NC; ++n) {
+            float* blk = base + n * block;
+            const int t0 = (n0 + n) * GC, cnt = min(GC, S - t0);
+            const float* g = gg[n & 1];
+            __syncthreads();  // the state is whole, the last chunk's K and U are read
+            if (tid == 0) lost[(n + 1) & 1] = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int r = (tid >> 4) + 16 * i;
+                *reinterpret_cast<u32x4*>(&Ks[r][(tid & 15) * 8]) = r < cnt ? kr[i] : u32x4{0u, 0u, 0u, 0u};
+            }
+            f32x16 hi = zero16(), lo = zero16();
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const Parts8 sp = parts_at<SP>(Sp, ln * (GD + 8) + 16 * i + 8 * hf);
+                if (Q) mfma_parts(__builtin_bit_cast(bf16x8, fr[i]), sp, hi, lo);
+                else mfma_parts(parts8(fr[2 * i], fr[2 * i + 1]), sp, hi, lo);
+            }
+            if (!Q) {
+                f32x16 u;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) u[e] = uv[e] - (hi[e] + lo[e]);
+#pragma unroll
+                for (int c = 0; c < 4; ++c) {
+                    const int t = 32 * rh + 8 * c + 4 * hf;
+                    const f32x4 G = *reinterpret_cast<const f32x4*>(g + GC + t);
+                    put_parts<UP>(Ut, ln * (GC + 8) + t, u[4 * c], u[4 * c + 1], u[4 * c + 2], u[4 * c + 3]);
+                    *reinterpret_cast<f32x4*>(&Ug[ln][t]) = f32x4{u[4 * c] * G[0], u[4 * c + 1] * G[1], u[4 * c + 2] * G[2], u[4 * c + 3] * G[3]};
+                }
+                if (__any(lost16(u)) && lane == 0) lost[n & 1] = 1;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) (blk + C_U + v0)[(32 * rh + c_row(e, hf)) * GD + ln] = u[e];
+            }
+            if (keep) {
+#pragma unroll
+                for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(blk - G_KW + v0 * GD + ln * GD + col + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
+            }
+            __syncthreads();
+            const int gone = lost[n & 1];
+            request(min(n + 1, NC - 1));  // (the last chunk's own once more: nothing here hangs on a condition)
+            if (Q) {
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    const float f = g[32 * rh + c_row(e, hf)] * qscale;
+                    hi[e] *= f;
+                    lo[e] *= f;
+                }
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    if (rh == 0 && i >= 2) break;  // P is lower triangular
+                    mfma_parts(parts8(fr[8 + 2 * i], fr[9 + 2 * i]), parts_at<UP>(Ut, ln * (GC + 8) + 16 * i + 8 * hf), hi, lo);
+                }
+                request_p(min(n + 1, NC - 1));
+                asm volatile("" ::: "memory");  // (the stores behind the requests: waits for those then leave the stores alone)
+#pragma unroll
+                for (int e = 0; e < 16; ++e) hi[e] += lo[e];
+                put_out(t0, cnt, hi);
+            }
+            if (gone) break;  // (the same for the whole workgroup)
+            const float gC = g[GC - 1];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] *= gC;
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const f32x4 d = *reinterpret_cast<const f32x4*>(&Ug[ln][8 * i + 4 * hf]);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) s = mfma2(bf2f(Ks[8 * i + 4 * hf + j][32 * wave + ln]), d[j], s);
+            }
+            put_state();
+            gg[(n + 1) & 1][tid] = gr;
+        }
+    };
+    if (wave >= 2) chunks(std::true_type{});
+    else chunks(std::false_type{});
     if (n == NC && final_state) {
 #pragma unroll
         for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(final_state + (head * GD + v0 + ln) * GD + col + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
