@@ -6,7 +6,7 @@
 // Which sequences of a step go this way is their own number of new tokens' affair (`from`): beside a long prompt, a short one and a single token
 // get the bits that they get alone -- of the delta rule inside the scan's launch, whose long chains hide them; of retention by mi355_gla_fwd_below.
 // A prompt's tokens through the token-by-token kernels are one dependent chain: six prompts of 900 tokens, 16 heads, 921 us a delta layer and 504 us of retention whatever
-// the chip could multiply; the chunks take 354 us and 183 us.  Bound: the scan's chain of chunks (two products behind two barriers each), not the
+// the chip could multiply; the chunks take 318 us and 179 us.  Bound: the scan's chain of chunks (two products behind two barriers each), not the
 // pipe.
 // Chains of 128 products on the matrix pipe are cut (add16): outputs' distance to 64 bits, token by token | here with whole chains | here: 1.29e-7 | 2.32e-7 | 1.73e-7, decays near zero
 // 1.19e-7 | 2.27e-7 | 1.45e-7, nearly parallel keys 1.29e-7 | 2.67e-7 | 1.90e-7, decays near one 4.7e-7 | 5.0e-7 | 4.7e-7, retention 3.1e-7 | 3.0e-7 | 2.6e-7; 6 of the 363 us that the six prompts took.
@@ -54,6 +54,19 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
     if (cnt <= 0 || p.seq_off[s + 1] - p.seq_off[s] < p.from) return;
     const float *qp = p.q + (int64_t)t0 * p.ldq + (int64_t)hq * GD, *kp = p.k + (int64_t)t0 * p.ldk + (int64_t)hq * GD, *vp = p.v + (int64_t)t0 * p.ldv + (int64_t)h * GD;
     float* blk = chunk_block(p, s, h, n);
+    // Everything is requested before it is needed, one latency for each: keys and their factors, queries in fragment form (tile (ti, tj) of Q K^T), and, once those are used, a column of
+    // values: six prompts of 900 tokens, 16 heads, 135 -> 105 us (retention 38 -> 35).  (No conditions: rows beyond the sequence are its last, dropped where they are used.)
+    const int ti = wave >> 1, tj = wave & 1, last = cnt - 1;
+    f32x4 kr[8], qr[16];
+    float kf[8];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        const int r = min((tid >> 5) + 8 * i, last);
+        kr[i] = *reinterpret_cast<const f32x4*>(kp + r * p.ldk + (tid & 31) * 4);
+        kf[i] = DELTA ? p.tok[((int64_t)t0 + r) * p.H + h][2] : p.kscale;
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) qr[i] = *reinterpret_cast<const f32x4*>(qp + min(32 * ti + ln, last) * p.ldq + 8 * i + 4 * hf);
     if (wave == 0) {
         f32x4 c = {1.f, 0.f, 0.f, 0.f};
         if (lane < cnt) {
@@ -71,20 +84,17 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
     }
 #pragma unroll
     for (int i = 0; i < 8; ++i) {  // keys, made unit vectors (resp. scaled) on the way
-        const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-        f32x4 kv = {0.f, 0.f, 0.f, 0.f};
-        if (r < cnt) kv = *reinterpret_cast<const f32x4*>(kp + r * p.ldk + c) * (DELTA ? p.tok[((int64_t)t0 + r) * p.H + h][2] : p.kscale);
-        *reinterpret_cast<f32x4*>(&Ks[r][c]) = kv;
+        const int r = (tid >> 5) + 8 * i;
+        *reinterpret_cast<f32x4*>(&Ks[r][(tid & 31) * 4]) = r < cnt ? kr[i] * kf[i] : f32x4{0.f, 0.f, 0.f, 0.f};
     }
     __syncthreads();
+    [[maybe_unused]] float vr[32];
     {  // K K^T and Q K^T: wave = tile (ti, tj); the tile above the diagonal is zero
-        const int ti = wave >> 1, tj = wave & 1;
         f32x16 kk = zero16(), qk = zero16(), kkt = zero16(), qkt = zero16();
         if (wave != 1) {
-            const int qr = 32 * ti + ln;
-#pragma unroll 4
+#pragma unroll
             for (int c = 0; c < GD; c += 8) {
-                const f32x4 qv = qr < cnt ? *reinterpret_cast<const f32x4*>(qp + qr * p.ldq + c + 4 * hf) : f32x4{0.f, 0.f, 0.f, 0.f};
+                const f32x4 qv = 32 * ti + ln < cnt ? qr[c / 8] : f32x4{0.f, 0.f, 0.f, 0.f};
                 const f32x4 bv = *reinterpret_cast<const f32x4*>(&Ks[32 * tj + ln][c + 4 * hf]);
                 const f32x4 av = *reinterpret_cast<const f32x4*>(&Ks[32 * ti + ln][c + 4 * hf]);
 #pragma unroll
@@ -98,6 +108,10 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
                 }
             }
             qk = qkt, kk = kkt;
+        }
+        if (DELTA) {
+#pragma unroll
+            for (int i = 0; i < 32; ++i) vr[i] = vp[min(8 * (i >> 2) + 4 * hf + (i & 3), last) * p.ldv + 32 * wave + ln];
         }
         const int j = 32 * tj + ln;
         const double gj = gd[j];
@@ -115,7 +129,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
         // Uv = R (b V), Kw = R (b gam K): wave = 32 columns, both row halves (the upper one ends at token 32)
         f32x16 u0 = zero16(), u1 = zero16(), w0 = zero16(), w1 = zero16(), ut = zero16(), wt = zero16();
         const int col = 32 * wave + ln;
-#pragma unroll 2
+#pragma unroll
         for (int kb = 0; kb < GC; kb += 8) {
             const f32x4 a1 = *reinterpret_cast<const f32x4*>(&T[32 + ln][kb + 4 * hf]);
             f32x4 a0 = {0.f, 0.f, 0.f, 0.f};
@@ -123,7 +137,7 @@ __global__ __launch_bounds__(256, 2) void dchunk_prep_kernel(DChunkArgs p) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int t = kb + 4 * hf + j;
-                const float bv = t < cnt ? vp[t * p.ldv + col] * be[t] : 0.f, bk = Ks[t][col] * (be[t] * gam[t]);
+                const float bv = t < cnt ? vr[kb / 2 + j] * be[t] : 0.f, bk = Ks[t][col] * (be[t] * gam[t]);
                 u1 = mfma2(a1[j], bv, u1);
                 w1 = mfma2(a1[j], bk, w1);
                 if (kb < 32) {
