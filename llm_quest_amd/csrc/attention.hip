@@ -12,6 +12,7 @@
 // whose visible keys are all masked degenerates to uniform attention over all S keys exactly as upstream; keys
 // beyond S do not exist and get -inf.  Scores stay in fp32 (the reference rounds them to bf16 twice).
 #include "attn_common.h"
+#include "lane_sums.h"
 
 namespace {
 
@@ -1676,6 +1677,148 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_spill_kernel(int B, int S,
     }
 }
 
+// ---- the whole backward of a short sequence (at most 256 tokens, head_dim 64, as many key / value heads as heads) in one pass: a workgroup of eight waves per (sequence, head).  A wave owns 32 keys
+// -- their K and V rows as operands, dK^T and dV^T as accumulators -- and the workgroup sweeps 64-query tiles:
+//   S = Q K^T, dP = dO V^T, P = exp2(S c - lse'), dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS   (key on the lane; P and dS are the B operands as the accumulators hold them)
+//   dS [key][query] to LDS, and behind a barrier dQ^T = K^T dS^T, 16 x 16 tiles, two a wave, over all keys.
+// delta = rowsum(dO O) is summed where dO is read.  Three passes (delta, dK / dV, dQ) read the operands three times and formed S and dP twice: 128 x 197 tokens, 12 heads, 260 -> 138 us, 5 x 197 26 -> 20,
+// 128 x 50 71 -> 36, 64 x 17 32 -> 12; the bytes of the first, 311 MB, take 64.  Bound: one workgroup a CU (93 KB), whose two waves a SIMD run products, exponentials and LDS reads (2.5, 3 and 4.7
+// thousand clocks of a tile's 10.5) one after the other; dQ of a tile beside the keys' side of the next, one barrier a tile, 143; a SIMD's two waves in opposite order 160 (registers spill).
+constexpr int SHORT_KEYS = 256;
+// eight k of a column from LDS rows of bf16, by two transposing reads of four rows each (a 16-lane group: four rows of 16 columns): `at` is this lane's address in the first
+__device__ __forceinline__ bf16x8 read_down(const bf16_t* at, int second) {
+    const bf16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)(at));
+    const bf16x4 hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)(at + second));
+    return __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7);
+}
+__global__ __launch_bounds__(512) void attn_bwd_short_kernel(int S, int H, const bf16_t* __restrict__ q, int64_t ldq, const bf16_t* __restrict__ k, int64_t ldk, const bf16_t* __restrict__ v, int64_t ldv,
+                                                             const bf16_t* __restrict__ o, int64_t ldo, const bf16_t* __restrict__ d_o, int64_t lddo, const float* __restrict__ lse, bf16_t* __restrict__ dq,
+                                                             int64_t lddq, bf16_t* __restrict__ dk, int64_t lddk, bf16_t* __restrict__ dv, int64_t lddv, const uint8_t* __restrict__ key_mask, int causal,
+                                                             float scale, float scale_log2) {
+    constexpr int D = 64, QT = 64, LD = D + 8, KS = D / 16, DT = D / 32;
+    __shared__ __attribute__((aligned(16))) bf16_t Ks[SHORT_KEYS][LD], Ds[SHORT_KEYS][QT + 8], Qs[QT][LD], Os[QT][LD];
+    __shared__ __attribute__((aligned(16))) float nlse[QT], delta[QT];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5;
+    const int grp = lane >> 4, q4 = (lane >> 2) & 3, p4 = lane & 3;
+    const int h = blockIdx.x % H, b = blockIdx.x / H, groups = (S + 31) / 32, key = 32 * wave + ln;
+    const int64_t tok = (int64_t)b * S;
+    const bool live = wave < groups, kin = key < S, kreal = kin && (key_mask == nullptr || key_mask[tok + key] != 0);
+    const int row = tid >> 3, c8 = (tid & 7) * 8;
+    u32x4 rq, rg, ro;
+    float rl;
+    auto request = [&](int q0) {
+        const int64_t r = tok + min(q0 + row, S - 1);
+        rq = *reinterpret_cast<const u32x4*>(q + r * ldq + h * D + c8);
+        rg = *reinterpret_cast<const u32x4*>(d_o + r * lddo + h * D + c8);
+        ro = *reinterpret_cast<const u32x4*>(o + r * ldo + h * D + c8);
+        rl = lse[((int64_t)b * H + h) * S + min(q0 + row, S - 1)];
+    };
+    request(0);
+    const u32x4 none = {0u, 0u, 0u, 0u};
+    bf16x8 kf[KS], vf[KS];
+    if (live) {
+        const int64_t r = tok + min(key, S - 1);
+#pragma unroll
+        for (int i = 0; i < KS; ++i) {
+            const u32x4 kw = *reinterpret_cast<const u32x4*>(k + r * ldk + h * D + 16 * i + 8 * hf), vw = *reinterpret_cast<const u32x4*>(v + r * ldv + h * D + 16 * i + 8 * hf);
+            kf[i] = __builtin_bit_cast(bf16x8, kin ? kw : none);
+            vf[i] = __builtin_bit_cast(bf16x8, kin ? vw : none);
+            *reinterpret_cast<bf16x8*>(&Ks[key][16 * i + 8 * hf]) = kf[i];
+        }
+    }
+    f32x16 dvt[DT], dkt[DT];
+#pragma unroll
+    for (int i = 0; i < DT; ++i)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) dvt[i][e] = dkt[i][e] = 0.f;
+    const bool open = 32 * wave + 32 <= S && key_mask == nullptr && !causal;  // no score of the wave's is hidden
+    for (int q0 = 0; q0 < S; q0 += QT) {
+        {   // (the last tile's readers are past the barrier in front of its dQ)
+            const bool in = q0 + row < S;
+            *reinterpret_cast<u32x4*>(&Qs[row][c8]) = in ? rq : none;
+            *reinterpret_cast<u32x4*>(&Os[row][c8]) = in ? rg : none;
+            float x = 0.f;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                x = fmaf(__uint_as_float(rg[e] << 16), __uint_as_float(ro[e] << 16), x);
+                x = fmaf(__uint_as_float(rg[e] & 0xffff0000u), __uint_as_float(ro[e] & 0xffff0000u), x);
+            }
+            x = lanes_sum<8>(x);
+            if ((tid & 7) == 0) nlse[row] = in ? -rl * LOG2E : 0.f, delta[row] = in ? x : 0.f;
+        }
+        __syncthreads();
+        if (q0 + QT < S) request(q0 + QT);
+        auto keys = [&](int st, auto masked) {  // 32 queries against the wave's keys
+            f32x16 s, dp;
+#pragma unroll
+            for (int e = 0; e < 16; ++e) s[e] = dp[e] = 0.f;
+#pragma unroll
+            for (int i = 0; i < KS; ++i) {
+                s = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&Qs[32 * st + ln][16 * i + 8 * hf]), kf[i], s, 0, 0, 0);
+                dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(*reinterpret_cast<const bf16x8*>(&Os[32 * st + ln][16 * i + 8 * hf]), vf[i], dp, 0, 0, 0);
+            }
+            unsigned pw[8], dw[8];
+#pragma unroll
+            for (int g4 = 0; g4 < 4; ++g4) {
+                const f32x4 nl = *reinterpret_cast<const f32x4*>(&nlse[32 * st + 8 * g4 + 4 * hf]), de = *reinterpret_cast<const f32x4*>(&delta[32 * st + 8 * g4 + 4 * hf]);
+                float pv[4], dsv[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    float t = fmaf(s[4 * g4 + e], scale_log2, nl[e]);
+                    if (decltype(masked)::value) t = !kreal || (causal && key > q0 + 32 * st + 8 * g4 + 4 * hf + e) ? -INFINITY : t;
+                    pv[e] = __builtin_amdgcn_exp2f(t);
+                    dsv[e] = pv[e] * (dp[4 * g4 + e] - de[e]);
+                }
+                pw[2 * g4] = pack_bf2(pv[0], pv[1]), pw[2 * g4 + 1] = pack_bf2(pv[2], pv[3]);
+                dw[2 * g4] = pack_bf2(dsv[0], dsv[1]), dw[2 * g4 + 1] = pack_bf2(dsv[2], dsv[3]);
+                *reinterpret_cast<u32x2*>(&Ds[key][32 * st + 8 * g4 + 4 * hf]) = u32x2{dw[2 * g4], dw[2 * g4 + 1]};
+            }
+#pragma unroll
+            for (int sd = 0; sd < 2; ++sd) {  // k: queries 16 sd + 4 hf + 0 .. 3 and + 8, in both operands
+                const bf16x8 pb = __builtin_bit_cast(bf16x8, u32x4{pw[4 * sd], pw[4 * sd + 1], pw[4 * sd + 2], pw[4 * sd + 3]}), db = __builtin_bit_cast(bf16x8, u32x4{dw[4 * sd], dw[4 * sd + 1], dw[4 * sd + 2], dw[4 * sd + 3]});
+#pragma unroll
+                for (int dt = 0; dt < DT; ++dt) {
+                    const int r = 32 * st + 16 * sd + 4 * hf + q4, c = 32 * dt + 16 * (grp & 1) + 4 * p4;
+                    dvt[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_down(&Os[r][c], 8 * LD), pb, dvt[dt], 0, 0, 0);
+                    dkt[dt] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(read_down(&Qs[r][c], 8 * LD), db, dkt[dt], 0, 0, 0);
+                }
+            }
+        };
+        if (open && q0 + 32 < S) {
+            keys(0, std::false_type{});
+            keys(1, std::false_type{});
+        } else if (live) {
+            for (int st = 0; st < 2 && q0 + 32 * st < S; ++st) keys(st, std::true_type{});
+        }
+        __syncthreads();
+        const int qt = wave >> 1, dh = wave & 1;  // 16 queries, 32 features of dQ
+        f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+        for (int g = 0; g < groups && q0 + 16 * qt < S; ++g) {
+            const int r = 32 * g + 8 * grp + q4;
+            const bf16x8 db = read_down(&Ds[r][16 * qt + 4 * p4], 4 * (QT + 8));
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(read_down(&Ks[r][32 * dh + 16 * j + 4 * p4], 4 * LD), db, acc[j], 0, 0, 0);
+        }
+        const int qq = q0 + 16 * qt + (lane & 15);
+        if (qq < S) {
+#pragma unroll
+            for (int j = 0; j < 2; ++j)
+                *reinterpret_cast<u32x2*>(dq + (tok + qq) * lddq + h * D + 32 * dh + 16 * j + 4 * grp) = u32x2{pack_bf2(acc[j][0] * scale, acc[j][1] * scale), pack_bf2(acc[j][2] * scale, acc[j][3] * scale)};
+        }
+    }
+    if (live) {
+#pragma unroll
+        for (int i = 0; i < 2 * DT; ++i) {  // as the long kernel's write-out: the two half-waves' 8-byte pieces of a row swapped into 16
+            const int dt = i / 2, e = 8 * (i % 2), col = 32 * dt + 2 * e + 8 * hf;
+#pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const f32x16 a = t ? dkt[dt] * scale : dvt[dt];
+                const auto x = __builtin_amdgcn_permlane32_swap(pack_bf2(a[e], a[e + 1]), pack_bf2(a[e + 4], a[e + 5]), false, false), y = __builtin_amdgcn_permlane32_swap(pack_bf2(a[e + 2], a[e + 3]), pack_bf2(a[e + 6], a[e + 7]), false, false);
+                if (kin) *reinterpret_cast<u32x4*>((t ? dk + (tok + key) * lddk : dv + (tok + key) * lddv) + h * D + col) = u32x4{x[0], y[0], x[1], y[1]};
+            }
+        }
+    }
+}
 
 int check_common(const char* name, int B, int S, int Hq, int Hkv, int D) {
     MI355_REQUIRE(D == 64 || D == 128, "%s: head_dim must be 64 or 128 (got %d)", name, D);
@@ -1803,6 +1946,13 @@ static int attn_bwd_impl(int B, int S, int Hq, int Hkv, int D, const void* q, in
     const float sl2 = scale * LOG2E;
     const int64_t items = (int64_t)B * S * ((Hq + 512 / D - 1) / (512 / D));
     const int dgrid = (int)((items + 3) / 4 > 8192 ? 8192 : (items + 3) / 4);
+    if (D == 64 && Hq == Hkv && S <= SHORT_KEYS && !((causal >> 8) & 1024)) {  // (at every size measured the faster one: from 2 x 1 to 300 x 33 and 128 x 256 tokens)
+        MI355_REQUIRE((int64_t)B * Hq < 0x7fffffffLL, "mi355_attn_bwd: grid too large");
+        attn_bwd_short_kernel<<<(unsigned)(B * Hq), 512, 0, s>>>(S, Hq, (const bf16_t*)q, ldq, (const bf16_t*)k, ldk, (const bf16_t*)v, ldv, (const bf16_t*)o, ldo, (const bf16_t*)d_o, lddo, lse, (bf16_t*)dq, lddq,
+                                                                 (bf16_t*)dk, lddk, (bf16_t*)dv, lddv, key_mask, causal & 0xff, scale, sl2);
+        MI355_LAUNCH_CHECK("mi355_attn_bwd");
+        return 0;
+    }
     // enough (batch, head) pairs to fill the chip twice over: one workgroup walks all blocks of its pair (no per-block launch,
     // prologue and first-tile latency); otherwise one block per workgroup for parallelism
     const int nblk = (S + 127) / 128;

@@ -480,6 +480,53 @@ def test_attention_backward_scratch_form_equals_recompute_form(K, B, S, Hq, Hkv,
 
 
 @pytest.mark.parametrize(
+    "B,S,H,causal,mask",
+    [(2, 1, 2, False, None), (3, 31, 1, True, None), (2, 32, 3, False, "pad"), (1, 33, 2, True, "holes"), (2, 64, 1, True, None), (2, 65, 2, False, "holes"), (5, 197, 3, False, None), (2, 224, 2, True, "pad"),
+     (2, 225, 2, False, None), (1, 255, 2, True, "holes"), (1, 256, 4, False, "pad"), (1, 256, 1, True, None)],
+)
+def test_attention_backward_of_short_sequences(K, B, S, H, causal, mask):
+    """One pass for head_dim 64 and up to 256 tokens, over the edges of its 32-key waves and 64-query tiles: against fp64 (bf16 P and dS: 2^-9 of a value, as the passes of longer sequences), on operands
+    and into gradients that are columns of wider rows; nothing beside them is written; keys that a mask hides get zeros, and what stands in their rows, or in the next sequence, reaches no other."""
+    D, w = 64, 8
+    g = torch.Generator().manual_seed(S)
+    x = torch.randn(B * S, 3 * H * D, generator=g).to(BF16)
+    qkv = dev(x)
+    q, k, v = (qkv[:, i * H * D : (i + 1) * H * D] for i in range(3))
+    do = dev(torch.randn(B * S, H * D, generator=g).to(BF16))
+    km = None
+    if mask:
+        km = torch.ones(B, S, dtype=torch.uint8)
+        if mask == "holes":
+            km[:, 2::5] = 0
+        else:
+            km[0, S - S // 3 :] = 0
+        km = dev(km)
+    o, lse = K.attn_fwd(q, k, v, B, S, H, H, D, key_mask=km, causal=causal)
+
+    def run(do):
+        wide = torch.full((B * S, 3 * H * D + w), 7.0, dtype=BF16, device="cuda")
+        out = [wide[:, i * H * D : (i + 1) * H * D] for i in range(3)]
+        K.attn_bwd(q, k, v, o, do, lse, B, S, H, H, D, *out, key_mask=km, causal=causal)
+        assert bool((wide[:, 3 * H * D :] == 7).all())
+        return out
+
+    got = run(do)
+    assert all(torch.equal(a, b) for a, b in zip(got, run(do)))
+    qr, kr, vr = (t.double().requires_grad_(True) for t in (q, k, v))
+    o_ref, _ = _attn_ref(qr, kr, vr, B, S, H, H, D, km, causal)
+    o_ref.backward(do.double())
+    for name, a, r in zip(("dq", "dk", "dv"), got, (qr.grad, kr.grad, vr.grad)):
+        if S > 1 or name == "dv":  # (one token: P is one, dS zero but for rounding)
+            assert rel_l2(a, r) < 8e-3, name
+    if mask:
+        assert not any(bool(t[km.view(-1) == 0].any()) for t in got[1:])
+    if B > 1:
+        do2 = do.clone()
+        do2[S:] = float("nan")
+        assert all(torch.equal(a[:S], b[:S]) for a, b in zip(got, run(do2)))
+
+
+@pytest.mark.parametrize(
     "B,S,Hq,Hkv,causal,ragged",
     [(1, 1, 2, 1, True, False), (1, 128, 16, 8, True, False), (1, 129, 3, 1, True, False), (2, 498, 16, 8, True, True), (1, 709, 4, 1, True, False), (1, 2000, 4, 2, False, True), (7, 584, 4, 4, True, False),
      (1, 4095, 2, 2, True, False), (8, 512, 2, 1, True, False)],
