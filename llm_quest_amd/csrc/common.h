@@ -32,16 +32,27 @@ __device__ __forceinline__ unsigned pack_bf2(float lo, float hi) {
     return __builtin_bit_cast(unsigned, r);
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+// All-reduce over a wave on the VALU: each step adds (resp. takes the larger of) a lane and the one whose number differs in bit 5, 4, 3, 2, 1, 0 -- the order, and so the bits, of a butterfly of
+// __shfl_xor, which goes through the LDS crossbar at some 120 clocks a step.  From bit 2 on a lane equals the one eight further, so a rotation by four reaches what differs in bit 2.  (All 64 lanes
+// active, as there.)  A short row's norm is its loads' latency and this chain: 8 x 1 024, LayerNorm forward
+// 2.50 -> 2.18 us, residual sum and norm 2.70 -> 2.37; 600 x 1 024 RMSNorm 2.28 -> 2.12, router logits 3.41 -> 3.07; 17 000 x 1 024 29.7 -> 27.5.
+template <int CTRL>
+__device__ __forceinline__ float wave_dpp(float v) {
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), CTRL, 0xf, 0xf, true));
 }
-__device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+template <typename Op>
+__device__ __forceinline__ float wave_fold(float v, Op op) {
+    const auto a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(a[0]), __uint_as_float(a[1]));
+    const auto b = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = op(__uint_as_float(b[0]), __uint_as_float(b[1]));
+    v = op(v, wave_dpp<0x128>(v));  // row_ror:8
+    v = op(v, wave_dpp<0x124>(v));  // row_ror:4
+    v = op(v, wave_dpp<0x4E>(v));   // quad_perm:[2,3,0,1]
+    return op(v, wave_dpp<0xB1>(v));  // quad_perm:[1,0,3,2]
 }
+__device__ __forceinline__ float wave_sum(float v) { return wave_fold(v, [](float x, float y) { return x + y; }); }
+__device__ __forceinline__ float wave_max(float v) { return wave_fold(v, [](float x, float y) { return fmaxf(x, y); }); }
 
 // ---- SwiGLU: one definition for the elementwise kernels and the GEMM epilogues, so fused == separate bit for bit.  sigmoid through v_exp + v_rcp
 // (1 ulp each; an IEEE division costs ten instructions per element, and the epilogues are bound by what their lanes issue); operands and results
