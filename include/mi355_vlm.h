@@ -601,6 +601,10 @@ int mi355_moe_route(int64_t tokens, int E, int top, int groups, int keep, const 
                     float* wts, void* stream);
 /* Dispatch lists of `entries` = tokens * top choices: offs int32 [E + 1], perm int32 [entries] = the entries sorted by expert (token order inside one). */
 int mi355_moe_dispatch(int64_t entries, int E, const int* ids, int* offs, int* perm, void* stream);
+/* The three calls above in one launch, the same bits, for the few tokens and experts of which mi355_moe_choose_takes is 1 (others are refused). */
+int mi355_moe_choose_takes(int64_t tokens, int E, int K, int top);
+int mi355_moe_choose(int64_t tokens, int E, int K, int top, int groups, int keep, const float* x, int64_t ldx, const void* W, int64_t ldw, const float* correction, float scale, int mode,
+                     int* ids, float* wts, int* offs, int* perm, void* stream);
 /* The dispatch lists of all `layers` of a step whose experts a table of the token ids picks (no router), in one launch: layer l's table int32 [vocab, top] starts
  * at tables + meta[4 l], its top <= max_top and expert count <= max_E (<= 4096) are meta[4 l + 1] and meta[4 l + 2]; entry (t, c) belongs to expert
  * table[tok[t], c].  Layer l's lists: offs + l * (max_E + 1) (E + 1 entries) and perm + l * tokens * max_top (tokens * top entries), as mi355_moe_dispatch writes them. */

@@ -127,6 +127,7 @@ SIGNATURES = {
     "mi355_router_logits": [_L, _I, _I, _P, _L, _P, _L, _P, _P],
     "mi355_moe_route": [_L, _I, _I, _I, _I, _P, _P, _F, _I, _P, _P, _P],
     "mi355_moe_dispatch": [_L, _I, _P, _P, _P, _P],
+    "mi355_moe_choose": [_L, _I, _I, _I, _I, _I, _P, _L, _P, _L, _P, _F, _I, _P, _P, _P, _P, _P],
     "mi355_moe_table_dispatch": [_I, _L, _I, _I, _I, _P, _P, _P, _P, _P, _P],
     "mi355_bgemm": [_I, _I, _I, _I, _P, _I, _L, _L, _P, _I, _L, _L, _L, _P, _I, _L, _L, _P, _P, _I, _P, _P, _I, _I, _P, _F, _I, _P],
     "mi355_latent_attn": [_I, _I, _I, _I, _I, _I, _I, _P, _L, _I, _P, _L, _I, _P, _L, _P, _L, _I, _P, _L, _I, _I, _P, _P, _P, _P, _P, _P, _F, _I, _I, _P, _L, _I, _I, _I, _F, _P, _I, _P, _P, _L, _P, _I, _P, _I, _P, _P, _L, _P],
@@ -176,6 +177,7 @@ QUERIES = {
     "mi355_gdr_chunked_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
     "mi355_decode_block_scratch_bytes": ([_I, _I, _I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_bytes": ([_I, _I, _I, _I], _L),
+    "mi355_moe_choose_takes": ([_L, _I, _I, _I], _I),
     "mi355_attn_bwd_split_bytes": ([_I, _I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_workspace_rowconst_offset": ([_I, _I, _I, _I, _I], _L),
     "mi355_attn_bwd_qnorm_partials": ([_I, _I, _I], _L),

@@ -278,17 +278,15 @@ class GroupedSigmoidMoE(_Frozen):
             self.correction32 = _f32(self.correction)
             self._ready = device
 
-    def route(self, logits):
-        return S.moe_route(logits, self.correction32, self.top, self.groups, self.keep, self.scale)
+    def route(self, x32):
+        return S.moe_choose(x32, self.w_router, self.correction32, self.top, self.groups, self.keep, self.scale)
 
     @torch.no_grad()
     def step(self, x32, h):
         """x32: the fp32 residual rows (the router reads them), h: the same rows in the activation dtype -> fp32 [T * top, width]."""
         self.prepare(h.device)
         T, E, top = h.shape[0], self.experts, self.top
-        logits = S.router_logits(x32, self.w_router)
-        ids, wts = self.route(logits)
-        offs, perm = S.moe_dispatch(ids.view(-1), E)
+        ids, wts, offs, perm = self.route(x32)
         act = torch.empty((T * top, self.ff), dtype=h.dtype, device=h.device)
         S.bgemm(h, self.w_up, act, T * top, self.ff, self.width, batch=E, sbn=self.width, b_bs=self.ff * self.width, grp_offs=offs, a_rows=perm, a_div=top, epi=1)
         out = torch.empty((T * top, self.width), dtype=F32, device=h.device)
@@ -303,8 +301,8 @@ class GroupedSoftmaxMoE(GroupedSigmoidMoE):
     def __init__(self, width, ff, experts, top, groups=1, keep=1, scale=1.0):
         super().__init__(width, ff, experts, top, groups, keep, scale, correction=False)
 
-    def route(self, logits):
-        return S.moe_route(logits, None, self.top, self.groups, self.keep, self.scale, softmax=True)
+    def route(self, x32):
+        return S.moe_choose(x32, self.w_router, None, self.top, self.groups, self.keep, self.scale, True)
 
 
 # ----------------------------------------------------------------------------------------------- mechanisms of parallel-sublayer hybrid decoders
@@ -634,18 +632,16 @@ class SoftmaxTopkMoE(GatedExperts):
     @torch.no_grad()
     def step(self, h32, h):
         """h32: the normed fp32 rows (the router reads them), h: the same rows in the activation dtype -> fp32 [T * top, width]."""
-        E, top = self.experts, self.top
+        top = self.top
         if self._ready != h.device:
             self.b_router32 = _f32(self.b_router)
             self._ready = h.device
-        logits = S.router_logits(h32, self.w_router)
         if self.chosen_softmax:
-            ids, wts = S.moe_route(logits, self.b_router32, top, 1, 1, 1.0, softmax="chosen")
+            ids, wts, offs, perm = S.moe_choose(h32, self.w_router, self.b_router32, top, 1, 1, 1.0, "chosen")
         else:
             if self.b_router32 is not None:
                 raise ValueError("SoftmaxTopkMoE: a router bias comes with weights over the winners")
-            ids, wts = S.moe_route(logits, None, top, 1, 1, 1.0, softmax=True)
-        offs, perm = S.moe_dispatch(ids.view(-1), E)
+            ids, wts, offs, perm = S.moe_choose(h32, self.w_router, None, top, 1, 1, 1.0, True)
         out = self.run_experts(h, offs, perm, wts)
         if self.shared is not None:
             return out, self.shared.step(h32, h, out_dtype=F32)

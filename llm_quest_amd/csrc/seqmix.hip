@@ -565,6 +565,40 @@ extern "C" int mi355_gla_fwd(int n_seq, const int* seq_off, const int* slot, int
 // ------------------------------------------------------------------------------------------- router logits
 // logits[t, e] = sum_k x[t, k] * W[e, k]: fp32 rows against a small bf16 matrix, fp32 FMA.  One workgroup per token keeps the row in LDS; wave w takes
 // experts w, w + 4, ...; a lane reads 8 weights (16 bytes) at a time when the rows allow it.
+// an expert's logits of N rows by a wave, the rows in LDS
+template <int N>
+__device__ __forceinline__ void router_logits_of(const float* const (&xs)[N], const bf16_t* wr, int Kd, int vec, int lane, float (&out)[N]) {
+#pragma unroll
+    for (int n = 0; n < N; ++n) out[n] = 0.f;
+    if (vec) {
+#pragma unroll 2
+        for (int k = lane * 8; k < Kd; k += 512) {
+            const u32x4 r = *(const u32x4*)(wr + k);
+#pragma unroll
+            for (int n = 0; n < N; ++n) {
+                const f32x4 a = *(const f32x4*)(xs[n] + k), c = *(const f32x4*)(xs[n] + k + 4);
+                float acc = out[n];
+                acc = fmaf(a[0], __uint_as_float(r[0] << 16), acc);
+                acc = fmaf(a[1], __uint_as_float(r[0] & 0xffff0000u), acc);
+                acc = fmaf(a[2], __uint_as_float(r[1] << 16), acc);
+                acc = fmaf(a[3], __uint_as_float(r[1] & 0xffff0000u), acc);
+                acc = fmaf(c[0], __uint_as_float(r[2] << 16), acc);
+                acc = fmaf(c[1], __uint_as_float(r[2] & 0xffff0000u), acc);
+                acc = fmaf(c[2], __uint_as_float(r[3] << 16), acc);
+                out[n] = fmaf(c[3], __uint_as_float(r[3] & 0xffff0000u), acc);
+            }
+        }
+    } else {
+        for (int k = lane; k < Kd; k += 64) {
+            const float w = bf2f(wr[k]);
+#pragma unroll
+            for (int n = 0; n < N; ++n) out[n] = fmaf(xs[n][k], w, out[n]);
+        }
+    }
+#pragma unroll
+    for (int n = 0; n < N; ++n) out[n] = wave_sum(out[n]);
+}
+
 __global__ __launch_bounds__(256) void router_logits_kernel(int64_t T, int E, int Kd, const float* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ W, int64_t ldw,
                                                             float* __restrict__ out, int vec) {
     extern __shared__ __attribute__((aligned(16))) float xs[];
@@ -574,26 +608,9 @@ __global__ __launch_bounds__(256) void router_logits_kernel(int64_t T, int E, in
         for (int k = tid; k < Kd; k += 256) xs[k] = x[t * ldx + k];
         __syncthreads();
         for (int e = wave; e < E; e += 4) {
-            const bf16_t* wr = W + (int64_t)e * ldw;
-            float acc = 0.f;
-            if (vec) {
-                for (int k = lane * 8; k < Kd; k += 512) {
-                    const u32x4 r = *(const u32x4*)(wr + k);
-                    const f32x4 a = *(const f32x4*)(xs + k), c = *(const f32x4*)(xs + k + 4);
-                    acc = fmaf(a[0], __uint_as_float(r[0] << 16), acc);
-                    acc = fmaf(a[1], __uint_as_float(r[0] & 0xffff0000u), acc);
-                    acc = fmaf(a[2], __uint_as_float(r[1] << 16), acc);
-                    acc = fmaf(a[3], __uint_as_float(r[1] & 0xffff0000u), acc);
-                    acc = fmaf(c[0], __uint_as_float(r[2] << 16), acc);
-                    acc = fmaf(c[1], __uint_as_float(r[2] & 0xffff0000u), acc);
-                    acc = fmaf(c[2], __uint_as_float(r[3] << 16), acc);
-                    acc = fmaf(c[3], __uint_as_float(r[3] & 0xffff0000u), acc);
-                }
-            } else {
-                for (int k = lane; k < Kd; k += 64) acc = fmaf(xs[k], bf2f(wr[k]), acc);
-            }
-            acc = wave_sum(acc);
-            if (lane == 0) out[t * E + e] = acc;
+            float z[1];
+            router_logits_of<1>({xs}, W + (int64_t)e * ldw, Kd, vec, lane, z);
+            if (lane == 0) out[t * E + e] = z[0];
         }
     }
 }
@@ -615,142 +632,144 @@ extern "C" int mi355_router_logits(int64_t tokens, int E, int K, const float* x,
 // winners * scale, not renormalised.
 // mode 2 (softmax over the winners): as mode 1 on logits + correction (a bias that counts for choice and weight), the winners' s divided by their sum --
 // the softmax over the chosen logits alone -- times scale.
+// the number of the largest value over a wave (element lane + 64 j in register j), the lowest of equals, -1 if none is above -inf; `best`: that value
+template <int EPL>
+__device__ __forceinline__ int wave_argmax(const float (&c)[EPL], float& best) {
+    best = -__builtin_huge_valf();
+#pragma unroll
+    for (int j = 0; j < EPL; ++j) best = c[j] > best ? c[j] : best;
+    best = wave_max(best);
+    if (!(best > -__builtin_huge_valf())) return -1;
+    int at = -1;
+#pragma unroll
+    for (int j = EPL - 1; j >= 0; --j) {
+        const unsigned long long has = __ballot(c[j] == best);
+        at = has ? 64 * j + __builtin_ctzll(has) : at;
+    }
+    return at;
+}
+template <int EPL>
+__device__ __forceinline__ void route_token(int E, int top, int groups, int keep, const float* logits, const float* __restrict__ corr, float scale, int mode, int* ids, float* wts) {
+    const int lane = threadIdx.x & 63;
+    const float NEG = -__builtin_huge_valf();
+    float s[EPL], c[EPL];
+    if (mode >= 1) {
+        float mx = NEG;
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            const int e = lane + 64 * j;
+            s[j] = e < E ? logits[e] + (mode == 2 && corr ? corr[e] : 0.f) : NEG;
+            mx = fmaxf(mx, s[j]);
+        }
+        mx = wave_max(mx);
+        float den = 0.f;
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            s[j] = lane + 64 * j < E ? expf(s[j] - mx) : 0.f;
+            den += s[j];
+        }
+        den = wave_sum(den);
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            s[j] = s[j] / den;
+            c[j] = lane + 64 * j < E ? s[j] : NEG;
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            const int e = lane + 64 * j;
+            if (e < E) {
+                const float zz = logits[e];
+                s[j] = 1.0f / (1.0f + expf(-zz));
+                c[j] = s[j] + (corr ? corr[e] : 0.f);
+            } else {
+                s[j] = 0.f;
+                c[j] = NEG;
+            }
+        }
+    }
+    if (mode <= 1 && groups > 1) {
+        const int per = E / groups;
+        // group scores: lane g keeps the score of group g (+ 64 * register)
+        float gs[EPL];
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) gs[j] = NEG;
+        for (int g = 0; g < groups; ++g) {
+            float best, second, of[EPL];
+#pragma unroll
+            for (int j = 0; j < EPL; ++j) {
+                const int e = lane + 64 * j;
+                of[j] = e < E && e / per == g ? c[j] : NEG;
+            }
+            const int bi = wave_argmax<EPL>(of, best);
+#pragma unroll
+            for (int j = 0; j < EPL; ++j)
+                if (lane + 64 * j == bi) of[j] = NEG;
+            wave_argmax<EPL>(of, second);
+            const float score = mode == 0 && per > 1 ? best + second : best;
+#pragma unroll
+            for (int j = 0; j < EPL; ++j)
+                if (lane + 64 * j == g) gs[j] = score;
+        }
+        // the `keep` best groups stay; mark them in a bit per (lane, register)
+        unsigned kept = 0;
+        for (int n = 0; n < keep; ++n) {
+            float best, of[EPL];
+            int low = -1;  // the lowest group that is left: where none scores above -inf
+#pragma unroll
+            for (int j = EPL - 1; j >= 0; --j) {
+                const bool left = lane + 64 * j < groups && !(kept >> j & 1);
+                const unsigned long long has = __ballot(left);
+                low = has ? 64 * j + __builtin_ctzll(has) : low;
+                of[j] = left ? gs[j] : NEG;
+            }
+            int bi = wave_argmax<EPL>(of, best);
+            if (bi < 0) bi = low;
+#pragma unroll
+            for (int j = 0; j < EPL; ++j)
+                if (lane + 64 * j == bi) kept |= 1u << j;
+        }
+        // an expert is allowed iff its group was kept: ask the lane that holds the group's bit
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            const int e = lane + 64 * j;
+            const int g = e < E ? e / per : 0;
+            const unsigned kb = __shfl(kept, g & 63, 64);
+            if (e < E && !(kb >> (g >> 6) & 1)) c[j] = NEG;
+        }
+    }
+    float wsum = 0.f, mine = 0.f;
+    int my_id = 0;
+    for (int n = 0; n < top; ++n) {
+        float best;
+        const int bi = wave_argmax<EPL>(c, best);
+        float sv = 0.f;  // (0 if no expert was left)
+#pragma unroll
+        for (int j = 0; j < EPL; ++j) {
+            if (bi >= 64 * j && bi < 64 * j + 64) sv = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(s[j]), bi - 64 * j));
+            if (lane + 64 * j == bi) c[j] = NEG;
+        }
+        wsum += sv;
+        if (lane == n % 64 && n < 64) mine = sv, my_id = bi < 0 ? 0 : bi;
+        else if (n >= 64 && lane == 0) {  // more than 64 winners per token: written one by one
+            ids[n] = bi < 0 ? 0 : bi;
+            wts[n] = sv;
+        }
+    }
+    const float inv = mode == 1 ? scale : scale / (wsum + 1e-20f);
+    if (lane < top && lane < 64) {
+        ids[lane] = my_id;
+        wts[lane] = mine * inv;
+    }
+    if (top > 64 && lane == 0)
+        for (int n = 64; n < top; ++n) wts[n] *= inv;
+}
+
 template <int EPL>
 __global__ __launch_bounds__(256) void moe_route_kernel(int64_t T, int E, int top, int groups, int keep, const float* __restrict__ logits, const float* __restrict__ corr,
                                                         float scale, int mode, int* __restrict__ ids, float* __restrict__ wts) {
-    const int lane = threadIdx.x & 63;
-    const float NEG = -__builtin_huge_valf();
-    for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < T; t += (int64_t)gridDim.x * 4) {
-        float s[EPL], c[EPL];
-        if (mode >= 1) {
-            float mx = NEG;
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) {
-                const int e = lane + 64 * j;
-                s[j] = e < E ? logits[t * E + e] + (mode == 2 && corr ? corr[e] : 0.f) : NEG;
-                mx = fmaxf(mx, s[j]);
-            }
-            mx = wave_max(mx);
-            float den = 0.f;
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) {
-                s[j] = lane + 64 * j < E ? expf(s[j] - mx) : 0.f;
-                den += s[j];
-            }
-            den = wave_sum(den);
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) {
-                s[j] = s[j] / den;
-                c[j] = lane + 64 * j < E ? s[j] : NEG;
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) {
-                const int e = lane + 64 * j;
-                if (e < E) {
-                    const float zz = logits[t * E + e];
-                    s[j] = 1.0f / (1.0f + expf(-zz));
-                    c[j] = s[j] + (corr ? corr[e] : 0.f);
-                } else {
-                    s[j] = 0.f;
-                    c[j] = NEG;
-                }
-            }
-        }
-        if (mode <= 1 && groups > 1) {
-            const int per = E / groups;
-            // group scores: lane g keeps the score of group g (+ 64 * register)
-            float gs[EPL];
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) gs[j] = NEG;
-            for (int g = 0; g < groups; ++g) {
-                float best = NEG, second = NEG;
-                int bi = -1;
-#pragma unroll
-                for (int j = 0; j < EPL; ++j) {
-                    const int e = lane + 64 * j;
-                    if (e < E && e / per == g && c[j] > best) best = c[j], bi = e;
-                }
-                // wave argmax (value, lowest index)
-                for (int o = 32; o > 0; o >>= 1) {
-                    const float ob = __shfl_xor(best, o, 64);
-                    const int oi = __shfl_xor(bi, o, 64);
-                    if (ob > best || (ob == best && oi >= 0 && (bi < 0 || oi < bi))) best = ob, bi = oi;
-                }
-#pragma unroll
-                for (int j = 0; j < EPL; ++j) {
-                    const int e = lane + 64 * j;
-                    if (e < E && e / per == g && e != bi && c[j] > second) second = c[j];
-                }
-                second = wave_max(second);
-                const float score = mode == 0 && per > 1 ? best + second : best;
-#pragma unroll
-                for (int j = 0; j < EPL; ++j)
-                    if (lane + 64 * j == g) gs[j] = score;
-            }
-            // the `keep` best groups stay; mark them in a bit per (lane, register)
-            unsigned kept = 0;
-            for (int n = 0; n < keep; ++n) {
-                float best = NEG;
-                int bi = -1;
-#pragma unroll
-                for (int j = 0; j < EPL; ++j) {
-                    const int g = lane + 64 * j;
-                    if (g < groups && !(kept >> j & 1) && (gs[j] > best || bi < 0)) best = gs[j], bi = g;
-                }
-                for (int o = 32; o > 0; o >>= 1) {
-                    const float ob = __shfl_xor(best, o, 64);
-                    const int oi = __shfl_xor(bi, o, 64);
-                    if (oi >= 0 && (bi < 0 || ob > best || (ob == best && oi < bi))) best = ob, bi = oi;
-                }
-#pragma unroll
-                for (int j = 0; j < EPL; ++j)
-                    if (lane + 64 * j == bi) kept |= 1u << j;
-            }
-            // an expert is allowed iff its group was kept: ask the lane that holds the group's bit
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) {
-                const int e = lane + 64 * j;
-                const int g = e < E ? e / per : 0;
-                const unsigned kb = __shfl(kept, g & 63, 64);
-                if (e < E && !(kb >> (g >> 6) & 1)) c[j] = NEG;
-            }
-        }
-        float wsum = 0.f, mine = 0.f;
-        int my_id = 0;
-        for (int n = 0; n < top; ++n) {
-            float best = NEG;
-            int bi = -1;
-#pragma unroll
-            for (int j = 0; j < EPL; ++j) {
-                const int e = lane + 64 * j;
-                if (e < E && c[j] > best) best = c[j], bi = e;
-            }
-            for (int o = 32; o > 0; o >>= 1) {
-                const float ob = __shfl_xor(best, o, 64);
-                const int oi = __shfl_xor(bi, o, 64);
-                if (oi >= 0 && (bi < 0 || ob > best || (ob == best && oi < bi))) best = ob, bi = oi;
-            }
-            float sv = 0.f;
-#pragma unroll
-            for (int j = 0; j < EPL; ++j)
-                if (lane + 64 * j == bi) sv = s[j], c[j] = NEG;
-            sv = wave_sum(sv);  // exactly one lane holds it (0 if no expert was left)
-            wsum += sv;
-            if (lane == n % 64 && n < 64) mine = sv, my_id = bi < 0 ? 0 : bi;
-            else if (n >= 64 && lane == 0) {  // more than 64 winners per token: written one by one
-                ids[t * top + n] = bi < 0 ? 0 : bi;
-                wts[t * top + n] = sv;
-            }
-        }
-        const float inv = mode == 1 ? scale : scale / (wsum + 1e-20f);
-        if (lane < top && lane < 64) {
-            ids[t * top + lane] = my_id;
-            wts[t * top + lane] = mine * inv;
-        }
-        if (top > 64 && lane == 0)
-            for (int n = 64; n < top; ++n) wts[t * top + n] *= inv;
-    }
+    for (int64_t t = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); t < T; t += (int64_t)gridDim.x * 4)
+        route_token<EPL>(E, top, groups, keep, logits + t * E, corr, scale, mode, ids + t * top, wts + t * top);
 }
 
 extern "C" int mi355_moe_route(int64_t tokens, int E, int top, int groups, int keep, const float* logits, const float* correction, float scale, int mode, int* ids,
@@ -855,6 +874,58 @@ extern "C" int mi355_moe_dispatch(int64_t entries, int E, const int* ids, int* o
     const int nw = disp_waves(E);
     moe_dispatch_kernel<<<1, 1024, sizeof(int) * (nw * E + 16), ST(stream)>>>(entries, E, nw, ids, offs, perm);
     MI355_LAUNCH_CHECK("moe_dispatch");
+    return 0;
+}
+
+// Router logits, choice and dispatch lists of a few tokens by one workgroup: three launches of 7, 8.7 and 5.3 us, each mostly its start, its loads' latency and its drain (5, 4.7 and 5.3
+// since the choice takes its maxima on the VALU).  The same arithmetic in the same order (router_logits_of, route_token, dispatch_lists).  16 experts of 1 024 channels in 4 groups, three tokens:
+// 17.3 -> 11.8 (the choice) -> 8.1 us; 128 experts, 8 of them chosen, 35 -> 23 -> 17.
+template <int EPL>
+__global__ __launch_bounds__(1024) void moe_choose_kernel(int T, int E, int Kd, int top, int groups, int keep, const float* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ W, int64_t ldw, int vec,
+                                                          const float* __restrict__ corr, float scale, int mode, int* __restrict__ ids, float* __restrict__ wts, int* __restrict__ offs, int* __restrict__ perm) {
+    extern __shared__ __attribute__((aligned(16))) float choose_lds[];
+    float *xs = choose_lds, *logits = xs + T * Kd;  // [T][K], [T][E]
+    int *chosen = reinterpret_cast<int*>(logits + T * E), *lists = chosen + T * top;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    for (int t = 0; t < T; ++t)
+        for (int k = tid; k < Kd; k += 1024) xs[t * Kd + k] = x[t * ldx + k];
+    __syncthreads();
+    for (int e = wave; e < E; e += 16)
+        for (int t = 0; t < T; t += 4) {
+            const float* const rows[4] = {xs + t * Kd, xs + min(t + 1, T - 1) * Kd, xs + min(t + 2, T - 1) * Kd, xs + min(t + 3, T - 1) * Kd};
+            float z[4];
+            router_logits_of<4>(rows, W + (int64_t)e * ldw, Kd, vec, lane, z);
+            if (lane < 4 && t + lane < T) logits[(t + lane) * E + e] = lane == 0 ? z[0] : lane == 1 ? z[1] : lane == 2 ? z[2] : z[3];
+        }
+    __syncthreads();
+    if (wave < T) {
+        route_token<EPL>(E, top, groups, keep, logits + wave * E, corr, scale, mode, chosen + wave * top, wts + wave * top);
+        for (int n = lane; n < top; n += 64) ids[wave * top + n] = chosen[wave * top + n];  // (a wave's LDS works in order)
+    }
+    __syncthreads();
+    dispatch_lists(T * top, E, 1, [=](int64_t i) { return chosen[i]; }, offs, perm, lists);
+}
+
+static size_t choose_lds_bytes(int64_t T, int E, int K, int top) { return sizeof(float) * (size_t)(T * ((int64_t)K + E + top) + E + 16); }
+extern "C" int mi355_moe_choose_takes(int64_t tokens, int E, int K, int top) {
+    // one launch | three, us: 64 experts of 1 024 channels, 3 tokens 12.7 | 17.5, 8 tokens 18.7 | 17.9; 256 of 512 22 | 33 and 35 | 33.5; 16 of 1 024, 8 tokens 10.2 | 12.0.  One CU reads all the
+    // weights and, from five tokens on, twice; rows and lists lie in 64 KB of LDS.
+    return tokens > 0 && (tokens <= 4 || (tokens <= 8 && E <= 32)) && E > 0 && E <= 512 && top > 0 && top <= E && K > 0 && K <= 16384 && K % 4 == 0 && (int64_t)E * K <= (1 << 17) && choose_lds_bytes(tokens, E, K, top) <= 64 * 1024;
+}
+
+extern "C" int mi355_moe_choose(int64_t tokens, int E, int K, int top, int groups, int keep, const float* x, int64_t ldx, const void* W, int64_t ldw, const float* correction, float scale, int mode,
+                                int* ids, float* wts, int* offs, int* perm, void* stream) {
+    MI355_REQUIRE(x && W && ids && wts && offs && perm && ldx >= K && ldw >= K && mode >= 0 && mode <= 2 && mi355_moe_choose_takes(tokens, E, K, top), "moe_choose: bad arguments, or not so few tokens and experts");
+    MI355_REQUIRE(groups >= 1 && E % groups == 0 && keep >= 1 && keep <= groups && (int64_t)keep * (E / groups) >= top, "moe_choose: the kept groups must hold the experts to choose");
+    const int vec = K % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)W & 15) == 0, T = (int)tokens;
+    const size_t lds = choose_lds_bytes(tokens, E, K, top);
+#define CHOOSE(EPL) moe_choose_kernel<EPL><<<1, 1024, lds, ST(stream)>>>(T, E, K, top, groups, keep, x, ldx, (const bf16_t*)W, ldw, vec, correction, scale, mode, ids, wts, offs, perm)
+    if (E <= 64) CHOOSE(1);
+    else if (E <= 128) CHOOSE(2);
+    else if (E <= 256) CHOOSE(4);
+    else CHOOSE(8);
+#undef CHOOSE
+    MI355_LAUNCH_CHECK("moe_choose");
     return 0;
 }
 

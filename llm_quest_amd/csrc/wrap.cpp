@@ -29,7 +29,7 @@
     E(attn_bwd_qnorm) E(add_f32_to_bf16) E(layernorm_fwd) E(layernorm_bwd_bf16) E(reduce_rows_into) E(gelu_fwd) E(gelu_bwd_colsum) E(copy2d) E(zc_weight) E(headnorm_rope_fwd) E(headnorm_rope_bwd) \
     E(sigmoid_gate_fwd) E(sigmoid_gate_bwd) E(attn_generic_fwd) E(attn_generic_bwd) E(gdn_gates_fwd) E(gdn_gates_bwd) E(causal_conv_silu_fwd) E(causal_conv_silu_bwd) E(l2norm_fwd) E(l2norm_bwd) \
     E(gated_rmsnorm_fwd) E(gated_rmsnorm_bwd) E(gemv_bf16) E(gemv_bf16_f32out) E(hyper_mix) E(bgemm) E(latent_attn) E(qkv_rows_append) E(group_rmsnorm_sum) E(ragged_conv) E(gated_headnorm) E(glu_rows) \
-    E(add_layernorm_fwd) E(rmsnorm_rows) E(latent_kv_append) E(rope_heads) E(gla_fwd) E(router_logits) E(moe_route) E(moe_dispatch) E(unary_rows) E(embed_hash_fwd)
+    E(add_layernorm_fwd) E(rmsnorm_rows) E(latent_kv_append) E(rope_heads) E(gla_fwd) E(router_logits) E(moe_route) E(moe_dispatch) E(moe_choose) E(unary_rows) E(embed_hash_fwd)
 
 namespace {
 
@@ -59,6 +59,8 @@ Slot* const slots[] = {
 using WorkspaceBytes = int64_t (*)(int, int, int, int);
 using Partials = int64_t (*)(int, int, int);
 WorkspaceBytes attn_bwd_workspace_bytes;
+using ChooseTakes = int (*)(int64_t, int, int, int);
+ChooseTakes moe_choose_takes;
 using SplitBytes = int64_t (*)(int, int, int, int, int, int);
 SplitBytes attn_bwd_split_bytes;
 Partials attn_bwd_qnorm_partials;
@@ -1145,6 +1147,23 @@ OP(moe_dispatch, "ids", "E") {
     return tuple(offs, perm);
 }
 
+OP(moe_choose, "x32", "w", "correction", "top", "groups", "keep", "scale", "softmax") {
+    const T x = c.tensor(0), w = c.tensor(1), corr = c.maybe(2);
+    need(x.rows() && x.is(F32) && w.is(BF16) && w.rows() && w.size(1) == x.size(1) && (!corr || (corr.is(F32) && corr.numel() == w.size(0))) && (!c.v[7] || PyBool_Check(c.v[7])) && moe_choose_takes);
+    const int64_t tokens = x.size(0), E = w.size(0), K = w.size(1), top = c.integer(3);
+    need(tokens > 0 && E > 0 && top > 0 && top <= E && E <= 512 && K <= 16384 && (dry || (slot::moe_choose.address && slot::router_logits.address && slot::moe_route.address && slot::moe_dispatch.address)));
+    const bool one = moe_choose_takes(tokens, E, K, top);
+    const T logits = one ? T{} : c.empty(x, {tokens, E}, F32), ids = c.empty(x, {tokens, top}, I32), wts = c.empty(x, {tokens, top}, F32), offs = c.empty(x, {E + 1}, I32), perm = c.empty(x, {tokens * top}, I32);
+    if (one) {
+        LAUNCH(moe_choose, tokens, E, K, top, c.integer(4), c.integer(5), x, x.ld(), w, w.ld(), corr, c.real(6), (int)c.truth(7, false), ids, wts, offs, perm);
+    } else {
+        LAUNCH(router_logits, tokens, E, K, x, x.ld(), w, w.ld(), logits);
+        LAUNCH(moe_route, tokens, E, top, c.integer(4), c.integer(5), logits, corr, c.real(6), (int)c.truth(7, false), ids, wts);
+        LAUNCH(moe_dispatch, tokens * top, E, ids, offs, perm);
+    }
+    return tuple(ids, wts, offs, perm);
+}
+
 OP(unary_rows, "x", "kind", "gate", "group", "out_dtype", "limit") {
     const T x = c.tensor(0), gate = c.maybe(2);
     const int64_t kind = c.integer(1), group = c.integer(3, 1);
@@ -1261,6 +1280,7 @@ PyObject* bind(PyObject*, PyObject* args) {
     if (!PyArg_ParseTuple(args, "sK", &name, &address)) return nullptr;
     void* at = reinterpret_cast<void*>(address);
     if (!strcmp(name, "mi355_attn_bwd_workspace_bytes")) attn_bwd_workspace_bytes = reinterpret_cast<WorkspaceBytes>(at);
+    if (!strcmp(name, "mi355_moe_choose_takes")) moe_choose_takes = reinterpret_cast<ChooseTakes>(at);
     if (!strcmp(name, "mi355_attn_bwd_split_bytes")) attn_bwd_split_bytes = reinterpret_cast<SplitBytes>(at);
     if (!strcmp(name, "mi355_attn_bwd_qnorm_partials")) attn_bwd_qnorm_partials = reinterpret_cast<Partials>(at);
     for (Slot* s : slots)

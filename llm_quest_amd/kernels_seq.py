@@ -237,6 +237,27 @@ def moe_dispatch(ids, E):
     return offs, perm
 
 
+@L.native
+def moe_choose(x32, w, correction, top, groups, keep, scale, softmax=False):
+    """``router_logits``, ``moe_route`` and ``moe_dispatch`` of one step: (ids, weights, offs, perm); few tokens in one launch, the same bits."""
+    T, E, K = x32.shape[0], w.shape[0], x32.shape[1]
+    if not L.load().mi355_moe_choose_takes(T, E, K, top):
+        logits = router_logits(x32, w)
+        ids, wts = moe_route(logits, correction, top, groups, keep, scale, softmax)
+        return (ids, wts, *moe_dispatch(ids.view(-1), E))
+    L.require_gpu(x32, w, correction)
+    _rows(x32, "moe_choose(x)")
+    if x32.dtype != F32 or w.dtype != BF16 or w.dim() != 2 or w.stride(1) != 1 or w.shape[1] != K:
+        raise ValueError("moe_choose: x fp32 [tokens, width], w bf16 [experts, width]")
+    if correction is not None and (correction.dtype != F32 or correction.numel() != E):
+        raise ValueError("moe_choose: correction fp32 [experts]")
+    ids, perm = (torch.empty(shape, dtype=I32, device=x32.device) for shape in ((T, top), (T * top,)))
+    wts, offs = torch.empty((T, top), dtype=F32, device=x32.device), torch.empty((E + 1,), dtype=I32, device=x32.device)
+    L.call("mi355_moe_choose", T, E, K, top, groups, keep, L.ptr(x32), x32.stride(0), L.ptr(w), w.stride(0), L.ptr(correction), float(scale), 2 if softmax == "chosen" else 1 if softmax else 0,
+           L.ptr(ids), L.ptr(wts), L.ptr(offs), L.ptr(perm))
+    return ids, wts, offs, perm
+
+
 def moe_table_dispatch(tok, vocab, tables, meta, specs):
     """The dispatch lists of every layer of a step whose experts a table of the token ids picks, in one launch.  ``tables`` int32: the layers' tables [vocab, top]
     one after the other; ``specs`` = [(top, experts)] per layer, ``meta`` int32 [layers, 4] = (start of the table, top, experts, 0) on the device.  Returns per

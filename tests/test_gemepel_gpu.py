@@ -584,3 +584,56 @@ def test_bf16_product_on_wide_tiles(rows, n, K, epi, out):
         bad = max(bad, float((c[r, :n_out].double() - y).norm() / y.norm()))
     assert bad < (2e-6 if out == F32 else 2.5e-3)
     assert bool((c[:, n_out:] == 7.0).all())  # nothing beside the columns
+
+
+@pytest.mark.parametrize("T,E,K,top,groups,keep", [(1, 1, 4, 1, 1, 1), (1, 16, 1024, 2, 4, 2), (4, 64, 1024, 6, 8, 3), (3, 65, 100, 4, 5, 2), (4, 128, 520, 8, 1, 1), (3, 240, 512, 70, 4, 4), (2, 512, 256, 3, 16, 5),
+                                                   (8, 8, 1744, 8, 2, 2), (5, 32, 512, 3, 8, 2), (7, 24, 64, 5, 2, 1), (9, 16, 1024, 2, 1, 1), (5, 33, 64, 2, 1, 1), (4, 64, 4096, 2, 1, 1), (4, 16, 102, 2, 2, 1)])
+def test_choice_of_few_tokens_in_one_launch(T, E, K, top, groups, keep):
+    """One launch against the three it stands for: the same ids, weights and lists bit for bit, in every mode, over rows of any pitch and weights of any alignment; what it does not take goes
+    the old way."""
+    from llm_quest_amd import _lib as L
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(T * E + K)
+    lds = 4 * (T * (K + E + top) + E + 16)
+    assert bool(L.load().mi355_moe_choose_takes(T, E, K, top)) == (T <= (8 if E <= 32 else 4) and K % 4 == 0 and E * K <= 1 << 17 and lds <= 65536)
+    x = torch.randn(T, K + 3, generator=g).to(DEV)[:, :K]
+    for off in (0, 1):
+        w = torch.randn(E * K + off, generator=g).to(torch.bfloat16).to(DEV)[off:].view(E, K)
+        corr = torch.randn(E, generator=g).to(DEV)
+        x[:, 0] = 0.0 if off else x[:, 0]
+        for softmax, c in ((False, corr), (False, None), (True, None), ("chosen", corr)):
+            if softmax == "chosen" and groups > 1:
+                continue
+            got = S.moe_choose(x, w, c, top, groups, keep, 1.7, softmax)
+            ids, wts = S.moe_route(S.router_logits(x, w), c, top, groups, keep, 1.7, softmax)
+            want = (ids, wts, *S.moe_dispatch(ids.view(-1), E))
+            assert all(a.shape == b.shape and torch.equal(a, b) for a, b in zip(got, want))
+
+
+@pytest.mark.parametrize("E,top,groups,keep", [(4, 2, 1, 1), (65, 5, 5, 2), (130, 9, 10, 3), (300, 66, 1, 1), (512, 4, 128, 3)])
+def test_choice_of_experts_among_equals_and_none(E, top, groups, keep):
+    """The order of the choice: the larger score first, of equals the lower number; -inf and NaN scores are chosen last, as expert 0 with weight 0 once nothing else is left."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(E)
+    z = torch.randint(-2, 3, (6, E), generator=g).float()
+    corr = torch.zeros(E)
+    corr[1::3] = float("-inf")
+    z[1, ::2], z[2], z[3, E // 2 :] = float("nan"), float("nan"), -200.0
+    for c in (None, corr):
+        ids, wts = (t.cpu() for t in S.moe_route(z.to(DEV), None if c is None else c.to(DEV), top, groups, keep, 1.0))
+        s = torch.sigmoid(z)
+        for t in range(6):
+            score = [(float(s[t, e]) + (0.0 if c is None else float(c[e])), e) for e in range(E)]
+            ok = [(v, e) for v, e in score if v > float("-inf")]  # (NaN is not)
+            if groups > 1:
+                per, gs = E // groups, []
+                for n in range(groups):
+                    two = sorted((v for v, e in ok if e // per == n), reverse=True)[:2] + [float("-inf")] * 2
+                    gs.append((-(two[0] + two[1] if per > 1 else two[0]), n))
+                kept = {n for _, n in sorted(gs)[:keep]}
+                ok = [(v, e) for v, e in ok if e // per in kept]
+            want = [e for _, e in sorted(ok, key=lambda x: (-x[0], x[1]))][:top]
+            assert ids[t].tolist() == want + [0] * (top - len(want))
+            assert not wts[t, len(want) :].any()

@@ -286,6 +286,9 @@ def test_served_rows(both):
     assert not both("embed_hash", ints(T).long(), None, tab, 1.0) and not both("embed_hash", ints(T), ints(T), tab, 1.0, torch.randn(8, W).to(B), 9)
     lg = torch.randn(T, 8)
     assert both("router_logits", x2, rows(8, W)) and both("moe_route", lg, None, 2, 1, 1, 1.0, softmax=True) and both("moe_route", lg, torch.randn(8), 2, 4, 2, 2.5) and not both("moe_route", lg, torch.randn(8), 2, 1, 1, 1.0, softmax="chosen")
+    for n, corr in itertools.product((3, 8, 9), (None, torch.randn(8))):  # (from nine tokens on three launches)
+        assert both("moe_choose", torch.randn(n, W), rows(8, W), corr, 2, 4, 2, 2.5) and both("moe_choose", torch.randn(n, W), rows(8, W), corr, 2, 1, 1, 1.0, True)
+    assert not both("moe_choose", x2, rows(8, W), None, 2, 1, 1, 1.0, "chosen") and not both("moe_choose", x2, rows(8, W + 8), None, 2, 1, 1, 1.0)
     assert both("moe_dispatch", ints(10), 8) and not both("moe_dispatch", ints(10).long(), 8)
     out = torch.empty(T, 24)
     assert both("bgemm", x2, rows(24, W), out, T, 24, W) and both("bgemm", rows(T, W), rows(24, W), out, T, 24, W, batch=2, lda=W, a_bs=1, sbn=W, sbk=1, b_bs=3, ldc=24, c_bs=2, mfma=False, bias=torch.randn(24), limit=3, n_out=12)
