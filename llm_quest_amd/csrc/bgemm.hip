@@ -38,6 +38,7 @@ struct BgemmArgs {
     float limit;
     int n_out;
     int a_dt, b_dt, c_dt;
+    bool rows_last;          // row tiles are the grid's slowest index (see row_tile_of)
 };
 
 // Gated activations of a feed-forward's [gate | up] product.  2: g = min(gate, limit), u = clamp(up, -limit, limit), g sigmoid(1.702 g) (u + 1).
@@ -58,16 +59,22 @@ __device__ __forceinline__ float ldx(const void* p, int dt, int64_t i) { return 
 #define BN 64
 #define BK 16
 
+// A workgroup's matrix (or group) and row tile.  With groups M counts all groups' rows, so most of a group's row tiles are empty, and between the groups' first ones they hold those up: row tiles are
+// then the slowest index (450 fp32 tokens on 2 of 16 experts, 1 024 -> 1 792, 56 rows an expert in 15 tiles of 64: 46 -> 34 us; on 4 of 64 45 -> 33).  Not where groups have several tiles and the
+// weights are more than the caches hold, which every row tile would then read again (3 000 tokens on 16 experts of 2 048 -> 7 168: 643 -> 693 us); nor without groups.
+__device__ __forceinline__ int batch_of(const BgemmArgs& p) { return p.rows_last ? blockIdx.y : blockIdx.z; }
+__device__ __forceinline__ int row_tile_of(const BgemmArgs& p) { return p.rows_last ? blockIdx.z : blockIdx.y; }
+static dim3 tile_grid(const BgemmArgs& p, int64_t cols, int64_t rows, int batch) { return p.rows_last ? dim3((unsigned)cols, (unsigned)batch, (unsigned)rows) : dim3((unsigned)cols, (unsigned)rows, (unsigned)batch); }
 __global__ __launch_bounds__(256) void bgemm_fma_kernel(BgemmArgs p) {
     __shared__ float As[BK][BM + 4];
     __shared__ float Bs[BK][BN + 4];
-    const int b = blockIdx.z;
+    const int b = batch_of(p);
     int row0 = 0, rows = p.M;
     if (p.grp_offs) {
         row0 = p.grp_offs[b];
         rows = p.grp_offs[b + 1] - row0;
     }
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int m0 = row_tile_of(p) * BM, n0 = blockIdx.x * BN;
     if (m0 >= rows) return;
     const int tid = threadIdx.x, tx = tid & 15, ty = tid >> 4;
     // loader roles: A element (m = tid / 4 + {0}, k = (tid % 4) * 4 .. +4): 64 rows x 16 k
@@ -155,13 +162,13 @@ __global__ __launch_bounds__(256) void bgemm_fma_kernel(BgemmArgs p) {
 __global__ __launch_bounds__(256) void bgemm_mfma_kernel(BgemmArgs p) {
     __shared__ bf16_t As[BM][MK + MPAD];
     __shared__ bf16_t Bs[BN][MK + MPAD];
-    const int b = blockIdx.z;
+    const int b = batch_of(p);
     int row0 = 0, rows = p.M;
     if (p.grp_offs) {
         row0 = p.grp_offs[b];
         rows = p.grp_offs[b + 1] - row0;
     }
-    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int m0 = row_tile_of(p) * BM, n0 = blockIdx.x * BN;
     if (m0 >= rows) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const bf16_t* A = (const bf16_t*)p.A;
@@ -243,13 +250,13 @@ template <bool VEC>
 __global__ __launch_bounds__(256) void bgemm_mfma128_kernel(BgemmArgs p) {
     __shared__ __attribute__((aligned(16))) bf16_t As[TM][TK + MPAD];
     __shared__ __attribute__((aligned(16))) bf16_t Bs[TM][TK + MPAD];
-    const int b = blockIdx.z;
+    const int b = batch_of(p);
     int row0 = 0, rows = p.M;
     if (p.grp_offs) {
         row0 = p.grp_offs[b];
         rows = p.grp_offs[b + 1] - row0;
     }
-    const int m0 = blockIdx.y * TM, n0 = blockIdx.x * TM;
+    const int m0 = row_tile_of(p) * TM, n0 = blockIdx.x * TM;
     if (m0 >= rows) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
     const bf16_t* A = (const bf16_t*)p.A;
@@ -597,24 +604,29 @@ __device__ __forceinline__ float settled(const BgemmArgs& p, float v, int b, int
 // Tile of 64 WM rows x 128 columns, four waves of 32 WM x 64 (2 x 2): k in steps of 32 through two LDS stages that take turns (A as three bf16 planes, split once per tile), one barrier a
 // step, operands requested DEPTH steps ahead into registers.  VALU (the split) and matrix pipe are level at WM = 1; WM = 2 halves the split's and B's share where there are rows for it.
 // With one stage and requests one step ahead a step was the weights' way from memory: 1.1 - 1.5 us, its products 0.16.  450 fp32 rows, us, before -> now: 2048 -> 1024 74 -> 49, 1024 -> 8256 86 -> 49; 3 000 rows
-// 1024 -> 4096 218 -> 115; 900 rows over 16 experts 1792 -> 1024 83 -> 62.  The split in front of the last step's products instead of behind them: experts 42 / 57, but 204 registers leave two
+// 1024 -> 4096 218 -> 115; 900 rows over 16 experts 1792 -> 1024 83 -> 62 (now 40).  The split in front of the last step's products instead of behind them: experts 42 / 57, but 204 registers leave two
 // workgroups to a CU (1024 -> 8256: 60); interleaved with the products it spills; eight steps ahead too.
+// HALVES = 2: eight waves, for products whose tiles leave CUs idle -- one workgroup then fills a CU where two would have.  The shares of a sum (SW of them, added in order) go to the two groups of four
+// waves in turn; the second group hands its share over in LDS, and the first adds both in their order: the same bits.  450 rows, 2048 -> 1024: 47.6 -> 39.9 us.
 #define FK 32
-template <int WM>
-__global__ __launch_bounds__(256, 2) void bgemm_f32_tile_kernel(BgemmArgs p) {
+template <int WM, int HALVES>
+__global__ __launch_bounds__(256 * HALVES, 2 / HALVES) void bgemm_f32_tile_kernel(BgemmArgs p) {
     constexpr int R = 64 * WM, AP = R / 32;  // A: 8 threads per row of 32 fp32, 32 rows per pass; B: 4 threads per row of 32 bf16, 64 rows per pass
     constexpr int DEPTH = WM == 1 ? 4 : 2;   // (sums and running sums of WM = 2 take 128 registers)
-    __shared__ __attribute__((aligned(16))) bf16_t As[2][3][R][FK + MPAD];
-    __shared__ __attribute__((aligned(16))) bf16_t Bs[2][128][FK + MPAD];
-    const int b = blockIdx.z;
+    __shared__ __attribute__((aligned(16))) bf16_t Asm[HALVES][2][3][R][FK + MPAD];
+    __shared__ __attribute__((aligned(16))) bf16_t Bsm[HALVES][2][128][FK + MPAD];
+    __shared__ __attribute__((aligned(16))) f32x4 swap[HALVES > 1 ? 256 * WM * 8 : 1];
+    const int b = batch_of(p);
     int row0 = 0, rows = p.M;
     if (p.grp_offs) {
         row0 = p.grp_offs[b];
         rows = p.grp_offs[b + 1] - row0;
     }
-    const int m0 = blockIdx.y * R, n0 = blockIdx.x * 128;
+    const int m0 = row_tile_of(p) * R, n0 = blockIdx.x * 128;
     if (m0 >= rows) return;
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
+    const int half = HALVES > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 8) : 0, tid = threadIdx.x & 255, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5;
+    bf16_t(&As)[2][3][R][FK + MPAD] = Asm[half];
+    bf16_t(&Bs)[2][128][FK + MPAD] = Bsm[half];
     const float* a_row[AP];  // rows and columns beyond the end: the last one again, their results are not stored
     const int ar = tid >> 3, ak = (tid & 7) * 4, br = tid >> 2, bk = (tid & 3) * 8;
 #pragma unroll
@@ -665,10 +677,10 @@ __global__ __launch_bounds__(256, 2) void bgemm_f32_tile_kernel(BgemmArgs p) {
 #pragma unroll
         for (int i = 0; i < 2; ++i) *(u32x4*)&Bs[st][br + 64 * i][bk] = w[i];
     };
-    auto step = [&](f32x4 (&x)[AP], u32x4 (&w)[2], int k0, int st) {
+    auto step = [&](f32x4 (&x)[AP], u32x4 (&w)[2], int k0, int st, int next, int end) {
         stage(x, w, k0, st);
         __builtin_amdgcn_sched_barrier(0);
-        fetch(x, w, k0 + DEPTH * FK);
+        fetch(x, w, next);
         // this wave's rows of the step are written, and its reads of the stage (two steps ago) are done -- behind the barrier everyone's; requests stay under way
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
@@ -676,7 +688,7 @@ __global__ __launch_bounds__(256, 2) void bgemm_f32_tile_kernel(BgemmArgs p) {
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int kk = 0; kk < FK; kk += 16) {
-            if (k0 + kk < p.K) {
+            if (k0 + kk < end) {
                 bf16x8 bf[2];
 #pragma unroll
                 for (int j = 0; j < 2; ++j) bf[j] = *(const bf16x8*)&Bs[st][wn + 32 * j + ln][kk + 8 * hf];
@@ -688,7 +700,7 @@ __global__ __launch_bounds__(256, 2) void bgemm_f32_tile_kernel(BgemmArgs p) {
 #pragma unroll
                         for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af, bf[j], acc[i][j], 0, 0, 0);
                     }
-                if (--left == 0) {
+                if (HALVES == 1 && --left == 0) {
                     left = per;
 #pragma unroll
                     for (int i = 0; i < WM; ++i)
@@ -703,12 +715,62 @@ __global__ __launch_bounds__(256, 2) void bgemm_f32_tile_kernel(BgemmArgs p) {
             }
         }
     };
+    if constexpr (HALVES == 1) {
 #pragma unroll
-    for (int d = 0; d < DEPTH; ++d) fetch(ra[d], rb[d], d * FK);
-    for (int k0 = 0; k0 < p.K; k0 += DEPTH * FK)  // (steps past K: zeros written, nothing multiplied)
+        for (int d = 0; d < DEPTH; ++d) fetch(ra[d], rb[d], d * FK);
+        for (int k0 = 0; k0 < p.K; k0 += DEPTH * FK)  // (steps past K: zeros written, nothing multiplied)
 #pragma unroll
-        for (int d = 0; d < DEPTH; ++d) step(ra[d], rb[d], k0 + d * FK, d & 1);
-    if (left != per) {
+            for (int d = 0; d < DEPTH; ++d) step(ra[d], rb[d], k0 + d * FK, d & 1, k0 + (d + DEPTH) * FK, p.K);
+    } else {
+        const int in_share = (per + 1) / 2, all = SW / 2 * in_share;  // steps of FK; a share that is no whole number of them ends within its last
+        auto share_at = [&](int share) { return (2 * share + half) * per * 16; };
+        int fs = 0, fp = 0;  // the next step to request: share, place in it
+        auto requested = [&]() {
+            const int at = share_at(fs) + fp * FK;
+            if (++fp == in_share) fp = 0, ++fs;
+            return min(at, p.K);  // (from K on: nothing is read beyond the rows' first words)
+        };
+#pragma unroll
+        for (int d = 0; d < DEPTH; ++d) fetch(ra[d], rb[d], requested());
+        int share = 0, place = 0;
+        for (int t = 0; t < all; t += DEPTH)
+#pragma unroll
+            for (int d = 0; d < DEPTH; ++d) {
+                if (t + d >= all) break;  // (the same for the whole workgroup)
+                const int begin = share_at(share);
+                step(ra[d], rb[d], min(begin + place * FK, p.K), d & 1, requested(), min(p.K, begin + per * 16));
+                if (++place < in_share) continue;
+                if (half == 1) {
+#pragma unroll
+                    for (int i = 0; i < WM * 8; ++i) swap[i * 256 + tid] = f32x4{acc[i / 8][i / 4 % 2][4 * (i % 4)], acc[i / 8][i / 4 % 2][4 * (i % 4) + 1], acc[i / 8][i / 4 % 2][4 * (i % 4) + 2], acc[i / 8][i / 4 % 2][4 * (i % 4) + 3]};
+                }
+                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // (as in a step: requests stay under way)
+                __builtin_amdgcn_s_barrier();
+                asm volatile("" ::: "memory");
+                const bool first = 2 * share * per * 16 < p.K, second = (2 * share + 1) * per * 16 < p.K;  // a share beyond K is none
+#pragma unroll
+                for (int i = 0; i < WM; ++i)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int g = 0; g < 4; ++g) {
+                            if (half == 0) {
+                                const f32x4 x = swap[((i * 2 + j) * 4 + g) * 256 + tid];
+#pragma unroll
+                                for (int e = 0; e < 4; ++e) {
+                                    float v = tot[i][j][4 * g + e];
+                                    v = first ? v + acc[i][j][4 * g + e] : v;
+                                    tot[i][j][4 * g + e] = second ? v + x[e] : v;
+                                }
+                            }
+#pragma unroll
+                            for (int e = 0; e < 4; ++e) acc[i][j][4 * g + e] = 0.f;
+                        }
+                place = 0, ++share;
+            }
+        if (half == 1) return;
+    }
+    if (HALVES == 1 && left != per) {
 #pragma unroll
         for (int i = 0; i < WM; ++i)
 #pragma unroll
@@ -785,8 +847,8 @@ __global__ __launch_bounds__(64 * SW) void bgemm_stream_kernel(BgemmArgs p) {
     using elem_t = std::conditional_t<F32, float, bf16_t>;
     using frag_t = std::conditional_t<F32, FragF32, u32x4>;
     __shared__ float red[SW][NB][16][64];
-    const int b = blockIdx.z, row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? p.grp_offs[b + 1] - row0 : p.M;
-    const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32 * NB;
+    const int b = batch_of(p), row0 = p.grp_offs ? p.grp_offs[b] : 0, rows = p.grp_offs ? p.grp_offs[b + 1] - row0 : p.M;
+    const int m0 = row_tile_of(p) * 32, n0 = blockIdx.x * 32 * NB;
     if (m0 >= rows) return;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5;
     const int steps = (p.K + 15) / 16, per = (steps + SW - 1) / SW, s0 = min(wave * per, steps), s1 = min(s0 + per, steps);
@@ -1038,9 +1100,10 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
     p.bias = bias;
     p.limit = limit, p.n_out = n_out;
     p.epi = epi, p.a_dt = a_dt, p.b_dt = b_dt, p.c_dt = c_dt;
+    p.rows_last = grp_offs && (M <= 64 * (int64_t)batch || (int64_t)batch * N * K <= 64 << 20);
     const bool vec = sbk == 1 && K % 8 == 0 && lda % 8 == 0 && a_bs % 8 == 0 && sbn % 8 == 0 && b_bs % 8 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0;
     if (use_mfma && grp_offs && M <= STREAM_ROWS && K >= 256 && vec) {
-        const dim3 grid((N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
+        const dim3 grid = tile_grid(p, (N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
         if (epi >= 2) bgemm_stream_kernel<true, false><<<grid, 64 * SW, 0, ST(stream)>>>(p);
         else bgemm_stream_kernel<false, false><<<grid, 64 * SW, 0, ST(stream)>>>(p);
         MI355_LAUNCH_CHECK("bgemm(stream)");
@@ -1057,7 +1120,7 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
         }
         const int64_t my128 = ((int64_t)M + TM - 1) / TM;
         MI355_REQUIRE(my128 <= 65535, "bgemm: too many row tiles");
-        const dim3 grid((N + TM - 1) / TM, (unsigned)my128, batch);
+        const dim3 grid = tile_grid(p, (N + TM - 1) / TM, my128, batch);
         if (vec) bgemm_mfma128_kernel<true><<<grid, 256, 0, ST(stream)>>>(p);
         else bgemm_mfma128_kernel<false><<<grid, 256, 0, ST(stream)>>>(p);
         MI355_LAUNCH_CHECK("bgemm");
@@ -1071,7 +1134,7 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
         const int64_t ty = ((int64_t)M + 63) / 64;
         MI355_REQUIRE(ty <= 65535, "bgemm: too many row tiles");
         if (M <= F32_STREAM_ROWS) {
-            const dim3 grid((N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
+            const dim3 grid = tile_grid(p, (N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
             const int64_t pitch = f32_rows_pitch(K), planes = 6 * (M + 1) * pitch, sums = SW * 16 * 64 * 4;
             if (epi < 2 && M <= 32 && planes <= F32_ROWS_LDS) {  // (M bounds the rows of every group)
                 const unsigned lds = (unsigned)(planes > sums ? planes : sums);
@@ -1084,15 +1147,19 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
             else bgemm_stream_kernel<false, true><<<grid, 64 * SW, 0, ST(stream)>>>(p);
         } else {
             const int64_t tn = (N + 127) / 128, tiles = (grp_offs ? 1 : batch) * tn * ((M + 127) / 128);
-            if (tiles >= 512) bgemm_f32_tile_kernel<2><<<dim3((unsigned)tn, (unsigned)((M + 127) / 128), batch), 256, 0, ST(stream)>>>(p);
-            else bgemm_f32_tile_kernel<1><<<dim3((unsigned)tn, (unsigned)ty, batch), 256, 0, ST(stream)>>>(p);
+            // Eight waves to a tile while every tile has a CU: 450 rows 2048 -> 1024 (64 tiles) 47.6 -> 39.9 us, 1024 -> 1536 29.5 -> 26.8; 304 tiles 38.5 | 53, 376 67 | 84; at K = 512 level.  Of groups a
+            // tile for half of them is counted beside the full ones.
+            const int64_t few = tn * (grp_offs ? ty + batch / 2 : ty * batch);
+            if (tiles >= 512) bgemm_f32_tile_kernel<2, 1><<<tile_grid(p, tn, (M + 127) / 128, batch), 256, 0, ST(stream)>>>(p);
+            else if (few <= 256 && K >= 1024) bgemm_f32_tile_kernel<1, 2><<<tile_grid(p, tn, ty, batch), 512, 0, ST(stream)>>>(p);
+            else bgemm_f32_tile_kernel<1, 1><<<tile_grid(p, tn, ty, batch), 256, 0, ST(stream)>>>(p);
         }
         MI355_LAUNCH_CHECK("bgemm(f32)");
         return 0;
     }
     const int64_t my = ((int64_t)M + BM - 1) / BM;
     MI355_REQUIRE(my <= 65535, "bgemm: too many row tiles");
-    const dim3 grid((N + BN - 1) / BN, (unsigned)my, batch);
+    const dim3 grid = tile_grid(p, (N + BN - 1) / BN, my, batch);
     if (use_mfma) bgemm_mfma_kernel<<<grid, 256, 0, ST(stream)>>>(p);
     else bgemm_fma_kernel<<<grid, 256, 0, ST(stream)>>>(p);
     MI355_LAUNCH_CHECK("bgemm");

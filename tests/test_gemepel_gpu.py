@@ -637,3 +637,41 @@ def test_choice_of_experts_among_equals_and_none(E, top, groups, keep):
             want = [e for _, e in sorted(ok, key=lambda x: (-x[0], x[1]))][:top]
             assert ids[t].tolist() == want + [0] * (top - len(want))
             assert not wts[t, len(want) :].any()
+
+
+@pytest.mark.parametrize("M,N,K", [(129, 128, 1024), (192, 130, 1032), (193, 1, 1096), (450, 1024, 2048), (300, 260, 1992), (1000, 384, 1024), (130, 512, 4096), (450, 1024, 1016)])
+def test_tiles_of_eight_waves(M, N, K):
+    """Few tiles of a long sum go to eight waves, which divide its shares: the bits of four (the same rows among enough others to fill the chip) over sums that are no whole number of shares or
+    steps, in groups, gated and scattered, and an infinity's row by FMA as ever."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(M + K)
+    many = 16384 // ((N + 127) // 128)
+    a, w = torch.randn(many, K, generator=g).to(DEV), (torch.randn(N, K, generator=g) * K**-0.5).to(torch.bfloat16).to(DEV)
+    a[1, 3], a[M - 1, K - 1] = float("inf"), float("nan")
+    few, all_ = torch.empty(M, N, device=DEV), torch.empty(many, N, device=DEV)
+    S.bgemm(a[:M], w, few, M, N, K)
+    S.bgemm(a, w, all_, many, N, K)
+    assert torch.equal(few.view(torch.int32), all_[:M].view(torch.int32))
+    want = a[2 : M - 1].double() @ w.double().mT
+    assert float((few[2 : M - 1].double() - want).norm()) < 2**-21 * float(want.norm())  # (sums of K products in eight shares, each product 2^-24)
+
+
+@pytest.mark.parametrize("lens,N,K", [([0, 70, 1, 0, 64, 130], 256, 1024), ([65, 0, 0, 200], 128, 2048), ([3] * 60, 64, 1024), ([400, 0, 500], 192, 512)])
+@pytest.mark.parametrize("dt", ["fp32", "bf16"])
+def test_groups_of_any_length(lens, N, K, dt):
+    """Rows of groups, empty ones among them, whichever index of the grid counts row tiles: each group's product is the one it has alone."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(N + K)
+    T, E, dtype = sum(lens), len(lens), torch.float32 if dt == "fp32" else torch.bfloat16
+    a, w = torch.randn(T, K, generator=g).to(dtype).to(DEV), (torch.randn(E, N, K, generator=g) * K**-0.5).to(torch.bfloat16).to(DEV)
+    offs = torch.tensor([0] + [sum(lens[: i + 1]) for i in range(E)], dtype=torch.int32, device=DEV)
+    perm = torch.randperm(T, generator=g).to(torch.int32).to(DEV)
+    out = torch.full((T, N), 7.0, device=DEV)
+    S.bgemm(a, w, out, T, N, K, batch=E, sbn=K, b_bs=N * K, grp_offs=offs, a_rows=perm, a_div=1, c_rows=perm)
+    want = torch.empty(T, N, dtype=torch.float64, device=DEV)
+    for e in range(E):
+        rows = perm[int(offs[e]) : int(offs[e + 1])].long()
+        want[rows] = a[rows].double() @ w[e].double().mT
+    assert float((out.double() - want).norm()) < 2**-20 * float(want.norm())
