@@ -7,15 +7,16 @@
 //     U = Uv - Kw S^T,  O = scale gam (Q S^T) + P U,  S <- gam_63 S + (Gp U)^T K                                                    -- the chain: one step per chunk
 // and the adjoint splits the same way: only dS crosses chunks (dU = P^T dO + Gp (K dS^T), dS <- gam_63 dS + (scale gam dO)^T Q - dU^T Kw), everything else is one
 // workgroup per chunk afterwards.  Four kernels: prep, scan, reverse scan (both per 32 value rows of the state: a row never meets another), and the rest.
-// All sums are fp32 FMAs on v_mfma_f32_32x32x2_f32 (the two products of bf16 operands alone, K K^T and Q K^T, on the bf16 shape: exact; the scan's Kw S^T, Q S^T and P U of three bf16 parts to an
+// All sums are fp32 FMAs on v_mfma_f32_32x32x2_f32 (the two products of bf16 operands alone, K K^T and Q K^T, on the bf16 shape: exact; the scans' products with the state, U, dO of three bf16 parts to an
 // fp32 number, which is all of it); the log decays are cumulated
 // in fp64, so a difference of two large ones keeps its digits.  d(alpha) is taken from sums over the pairs that span a token -- never as a difference of
 // larger sums, so it keeps its digits where alpha is tiny (below 1e-30 alpha counts as 1e-30); d(beta) as what reaches u times u / beta.
 // A matrix pipe's chain of 128 products rounds 128 times at its size where lanes sum 16 and meet in a tree; so the chains that show are cut (add16) and the state's gradient
 // gathers its terms from the last token to the first.  Distance to 64 bits, token-by-token kernels | here, 256 tokens, geometric mean of four draws: outputs, d(q), d(k), d(v)
-// 1.65e-3 | 1.65e-3 (their bf16); fp32: state 7.4e-8 | 8.4e-8, d(state) 9.0e-8 | 9.5e-8 (2.9e-7 from the first token on), d(beta) 1.5e-7 | 1.8e-7 (2.6e-7 with whole chains), d(alpha)
+// 1.65e-3 | 1.65e-3 (their bf16); fp32: state 7.4e-8 | 8.6e-8, d(state) 9.0e-8 | 9.5e-8 (2.9e-7 from the first token on), d(beta) 1.5e-7 | 1.8e-7 (2.6e-7 with whole chains), d(alpha)
 // 1.7e-7 | 2.1e-7 (2.5e-7); decays near one 4.4e-7 | 3.6e-7, 5.0e-7 | 4.9e-7; nearly parallel keys 1.5e-7 | 2.3e-7, 2.1e-7 | 4.4e-7.  Cutting d(q)'s and d(k)'s chains as well:
 // d(alpha) 1.9e-7 for 50 us of a backward of 680 (registers spill).
+// Three-part products in the scans against fp32 ones there, 64 draws of gates: state 1.41e-7 -> 1.37e-7, d(state) 2.44e-7 -> 2.43e-7, d(beta) 2.67e-7 -> 2.28e-7, d(alpha) 4.82e-7 -> 4.69e-7.
 // Bound: the fp32 matrix pipe (256 FLOP a clock and CU).  The products of one 64-token chunk of one head: 37 MFLOP forward and backward together.
 #include "gdr_chunk.h"
 
@@ -384,143 +385,143 @@ __global__ __launch_bounds__(256, 2) void gdrc_scan_kernel(int heads, int S, int
 }
 
 // ------------------------------------------------------------------------------------------- reverse scan: the state's gradient, 32 value rows per workgroup
+// dU = P^T dO + Gp (K dS^T): a wave takes 16 tokens, both products over their whole sums, of three bf16 parts to dS and P (two tiles of 16 x 16).  dS <- gam_63 dS + (scale gam dO)^T Q - dU^T Kw stays on the
+// fp32 pipe, as the scan's: the state's four tiles of 32 key channels go one to a wave, in registers (lane = value row), their three parts in LDS for the next chunk.  Bound: the chain of chunks and the
+// bytes; every operand is requested a chunk ahead, without conditions (rows beyond the sequence are its last, made zero where they are used).  8 x 708 tokens x 16
+// heads 159 -> 120 us, 333 tokens 57 -> 40 (fp32 products of halves of a sum that met in LDS, K and P requested where they were used).
 __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, int NC, int Hqk, int Hv, const bf16_t* __restrict__ q, const bf16_t* __restrict__ k, const float* __restrict__ saved,
                                                             const bf16_t* __restrict__ d_o, float* __restrict__ ws, const float* d_final, float* d_initial, float qscale) {
-    __shared__ __attribute__((aligned(16))) float Ss[GV][GD + 4];
-    __shared__ float Us[GC][GV + 4];
-    __shared__ __attribute__((aligned(16))) float Ws[GC][GD + 4];
+    __shared__ __attribute__((aligned(16))) bf16_t Sp[3 * SP];
     __shared__ __attribute__((aligned(16))) bf16_t Qs[GC][GD + 8];
-    __shared__ __attribute__((aligned(16))) bf16_t Os[GC][GV];  // (unpadded: two workgroups of this kernel fill a CU's LDS to the byte)
-    __shared__ float gg[2 * GC];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ln = lane & 31, hf = lane >> 5, rh = wave & 1, kh = wave >> 1;
+    __shared__ __attribute__((aligned(16))) bf16_t Os[GC][GV + 8];
+    __shared__ __attribute__((aligned(16))) float Og[GV][GC + 4], Ug[GV][GC + 4];  // scale gam dO and dU, [value row][token]
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), ln = lane & 31, hf = lane >> 5;
+    const int l16 = lane & 15, g = lane >> 4, q4 = (lane >> 2) & 3, p4 = lane & 3;
     int at, v0;
     if (!scan_place(heads, at, v0)) return;
-    const int h = at % Hv, b = at / Hv, hq = h / (Hv / Hqk);
+    const int h = at % Hv, b = at / Hv, hq = h / (Hv / Hqk), col = 32 * wave + 4 * hf, orow = tid >> 2, ocol = (tid & 3) * 8;
     const int64_t ldqk = (int64_t)Hqk * GD, ldo = (int64_t)Hv * GD, head = at;
     const bf16_t *qp = q + (int64_t)b * S * ldqk + hq * GD, *kp = k + (int64_t)b * S * ldqk + hq * GD, *gp = d_o + (int64_t)b * S * ldo + (int64_t)h * GD + v0;
     const float* base = saved + head * NC * G_BLOCK;
     float* wbase = ws + head * NC * W_BLOCK;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-        f32x4 s = {0.f, 0.f, 0.f, 0.f};
-        if (d_final) s = *reinterpret_cast<const f32x4*>(d_final + (head * GD + v0 + r) * GD + c);
-        *reinterpret_cast<f32x4*>(&Ss[r][c]) = s;
-    }
-    f32x4 wr[8];
-    u32x4 qr[4], gr;
-    float gv = 0.f;
+    // what a chunk reads: 16 rows of K and 16 columns of P in fragment form; the wave's 32 columns of Kw; Q; dO; decays
+    u32x4 kr[4], qr[4], gr;
+    float pr[16], wr[32], gam, last;
+    f32x4 Gp;
     auto request = [&](int n) {
         const float* blk = base + (int64_t)n * G_BLOCK;
-        const int t0 = n * GC, cnt = min(GC, S - t0);
+        const int t0 = n * GC, end = min(GC, S - t0) - 1;
+        gr = *reinterpret_cast<const u32x4*>(gp + t0 * ldo + min(orow, end) * ldo + ocol);
+        gam = blk[G_GAM + orow];
 #pragma unroll
-        for (int i = 0; i < 8; ++i) wr[i] = *reinterpret_cast<const f32x4*>(blk + G_KW + (tid + 256 * i) * 4);
+        for (int i = 0; i < 4; ++i) qr[i] = *reinterpret_cast<const u32x4*>(qp + t0 * ldqk + (min((tid >> 4) + 16 * i, end) * (unsigned)ldqk + (tid & 15) * 8));
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
-            qr[i] = r < cnt ? *reinterpret_cast<const u32x4*>(qp + (t0 + r) * ldqk + c) : u32x4{0u, 0u, 0u, 0u};
-        }
-        const int r = tid >> 2, c = (tid & 3) * 8;
-        gr = r < cnt ? *reinterpret_cast<const u32x4*>(gp + (t0 + r) * ldo + c) : u32x4{0u, 0u, 0u, 0u};
-        if (tid < 2 * GC) gv = blk[G_GAM + tid];
+        for (int i = 0; i < 4; ++i) kr[i] = *reinterpret_cast<const u32x4*>(kp + t0 * ldqk + (min(16 * wave + l16, end) * (unsigned)ldqk + 8 * g) + 32 * i);
+#pragma unroll
+        for (int i = 0; i < 16; ++i) pr[i] = (blk + G_P)[(32 * (i >> 3) + 8 * g + (i & 7)) * GC + 16 * wave + l16];
+        Gp = *reinterpret_cast<const f32x4*>(blk + G_GAM + GC + 16 * wave + 4 * g);
+        last = blk[G_GAM + GC - 1];
+    };
+    auto request_w = [&](int n) {
+#pragma unroll
+        for (int i = 0; i < 32; ++i) wr[i] = (base + (int64_t)n * G_BLOCK + G_KW)[(8 * (i >> 2) + 4 * hf + (i & 3)) * GD + 32 * wave + ln];
+    };
+    f32x16 s;  // dS[v0 + ln][32 wave + c_row(e, hf)]
+    auto put_state = [&]() {
+#pragma unroll
+        for (int c = 0; c < 4; ++c) put_parts<SP>(Sp, ln * (GD + 8) + col + 8 * c, s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]);
     };
     request(NC - 1);
+    request_w(NC - 1);
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        f32x4 x = {0.f, 0.f, 0.f, 0.f};
+        if (d_final) x = *reinterpret_cast<const f32x4*>(d_final + (head * GD + v0 + ln) * GD + col + 8 * c);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) s[4 * c + e] = x[e];
+    }
+    put_state();
     for (int n = NC - 1; n >= 0; --n) {
-        const float* blk = base + (int64_t)n * G_BLOCK;
         float* wblk = wbase + (int64_t)n * W_BLOCK;
-        const int t0 = n * GC, cnt = min(GC, S - t0);
+        const int cnt = min(GC, S - n * GC);
+        const float gC = last;
         __syncthreads();  // dS is whole, the last chunk's operands are read
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-            *reinterpret_cast<f32x4*>(&Ws[r][c]) = wr[i];
-        }
-#pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 4, c = (idx & 15) * 8;
-            *reinterpret_cast<u32x4*>(&Qs[r][c]) = qr[i];
+            const int r = (tid >> 4) + 16 * i;
+            *reinterpret_cast<u32x4*>(&Qs[r][(tid & 15) * 8]) = r < cnt ? qr[i] : u32x4{0u, 0u, 0u, 0u};
         }
         {
-            const int r = tid >> 2, c = (tid & 3) * 8;
-            *reinterpret_cast<u32x4*>(&Os[r][c]) = gr;
+            const u32x4 x = orow < cnt ? gr : u32x4{0u, 0u, 0u, 0u};
+            const float f = gam * qscale;
+            *reinterpret_cast<u32x4*>(&Os[orow][ocol]) = x;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                Og[ocol + 2 * e][orow] = __uint_as_float(x[e] << 16) * f;
+                Og[ocol + 2 * e + 1][orow] = __uint_as_float(x[e] & 0xffff0000u) * f;
+            }
         }
-        if (tid < 2 * GC) gg[tid] = gv;
+        f32x4 hi[2], lo[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) hi[j] = lo[j] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-            *reinterpret_cast<f32x4*>(wblk + (v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
+            const bf16x8 kf = __builtin_bit_cast(bf16x8, kr[i]);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                const Parts8 sp = parts_at<SP>(Sp, (16 * j + l16) * (GD + 8) + 32 * i + 8 * g);
+                lo[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, sp.p[2], lo[j], 0, 0, 0);
+                lo[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, sp.p[1], lo[j], 0, 0, 0);
+                hi[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, sp.p[0], hi[j], 0, 0, 0);
+            }
+        }
+#pragma unroll
+        for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(wblk + v0 * GD + ln * GD + col + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
+        Parts8 pp[2];
+#pragma unroll
+        for (int i = 0; i < 2; ++i) pp[i] = parts8(f32x4{pr[8 * i], pr[8 * i + 1], pr[8 * i + 2], pr[8 * i + 3]}, f32x4{pr[8 * i + 4], pr[8 * i + 5], pr[8 * i + 6], pr[8 * i + 7]});
+        __syncthreads();  // dO lies
+        f32x4 u[2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            f32x4 ph = {0.f, 0.f, 0.f, 0.f}, pl = ph;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const bf16_t* o = &Os[32 * i + 8 * g + q4][16 * j + 4 * p4];
+                const bf16x4 o0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)(o)), o1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)(o + 4 * (GV + 8)));
+                const bf16x8 of = __builtin_shufflevector(o0, o1, 0, 1, 2, 3, 4, 5, 6, 7);
+                pl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pp[i].p[2], of, pl, 0, 0, 0);
+                pl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pp[i].p[1], of, pl, 0, 0, 0);
+                ph = __builtin_amdgcn_mfma_f32_16x16x32_bf16(pp[i].p[0], of, ph, 0, 0, 0);
+            }
+#pragma unroll
+            for (int e = 0; e < 4; ++e) u[j][e] = 16 * wave + 4 * g + e < cnt ? fmaf(Gp[e], hi[j][e] + lo[j][e], ph[e] + pl[e]) : 0.f;
+            *reinterpret_cast<f32x4*>(&Ug[16 * j + l16][16 * wave + 4 * g]) = u[j];
         }
         __syncthreads();
-        // dU = P^T dO + Gp (K dS^T): wave = (row half, half of the contraction); the two halves of a contraction meet in LDS
-        f32x16 u = zero16(), ut = zero16(), pt = zero16();
-        {
-            f32x4 kf[8];
+        request(n > 0 ? n - 1 : 0);  // (the first chunk's own once more: nothing here hangs on a condition)
 #pragma unroll
-            for (int i = 0; i < 8; ++i) kf[i] = widen4(row4(kp + t0 * ldqk, ldqk, 32 * rh + ln, cnt, 64 * kh + 8 * i + 4 * hf));
-            float pf[16];
-            const bool some = !(rh == 1 && kh == 0);  // P[i][j] with i < 32 <= j is zero
-            if (some) {
+        for (int j = 0; j < 2; ++j)
 #pragma unroll
-                for (int i = 0; i < 4; ++i)
+            for (int e = 0; e < 4; ++e) (wblk + W_DU + v0)[(16 * wave + 4 * g + e) * GD + 16 * j + l16] = u[j][e];
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) pf[4 * i + j] = blk[G_P + (32 * kh + 8 * i + 4 * hf + j) * GC + 32 * rh + ln];
-            }
-            if (n > 0) request(n - 1);
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                const f32x4 s = *reinterpret_cast<const f32x4*>(&Ss[ln][64 * kh + 8 * i + 4 * hf]);
-#pragma unroll
-                for (int j = 0; j < 4; ++j) u = mfma2(kf[i][j], s[j], u);
-                if (i == 3) add16(ut, u);
-            }
-            add16(u, ut);
-            if (some) {
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) pt = mfma2(pf[4 * i + j], bf2f(Os[32 * kh + 8 * i + 4 * hf + j][ln]), pt);
-            }
-        }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) u[e] = fmaf(gg[GC + 32 * rh + c_row(e, hf)], u[e], pt[e]);
-        if (kh == 1) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) Us[32 * rh + c_row(e, hf)][ln] = u[e];
-        }
-        __syncthreads();
-        if (kh == 0) {
-#pragma unroll
-            for (int e = 0; e < 16; ++e) {
-                const int r = 32 * rh + c_row(e, hf);
-                const float d = u[e] + Us[r][ln];
-                Us[r][ln] = d;
-                wblk[W_DU + r * GD + v0 + ln] = d;
-            }
-        }
-        __syncthreads();
-        f32x16 s;
-        const float gC = gg[GC - 1];
-#pragma unroll
-        for (int e = 0; e < 16; ++e) s[e] = gC * Ss[c_row(e, hf)][32 * wave + ln];
+        for (int e = 0; e < 16; ++e) s[e] *= gC;
         // from the last token to the first: what reaches the chunk's start grows that way (the other way around the large terms come first and every later sum rounds at their size)
-#pragma unroll 2
-        for (int kb = GC - 8; kb >= 0; kb -= 8)
+#pragma unroll
+        for (int i = 7; i >= 0; --i) {
+            const f32x4 o4 = *reinterpret_cast<const f32x4*>(&Og[ln][8 * i + 4 * hf]), u4 = *reinterpret_cast<const f32x4*>(&Ug[ln][8 * i + 4 * hf]);
 #pragma unroll
             for (int j = 3; j >= 0; --j) {
-                const int t = kb + 4 * hf + j;
-                s = mfma2(bf2f(Os[t][ln]) * (gg[t] * qscale), bf2f(Qs[t][32 * wave + ln]), s);
-                s = mfma2(-Us[t][ln], Ws[t][32 * wave + ln], s);
+                s = mfma2(bf2f(Qs[8 * i + 4 * hf + j][32 * wave + ln]), o4[j], s);
+                s = mfma2(wr[4 * i + j], -u4[j], s);
             }
-#pragma unroll
-        for (int e = 0; e < 16; ++e) Ss[c_row(e, hf)][32 * wave + ln] = s[e];  // read by this wave alone since the barrier behind dU
+        }
+        request_w(n > 0 ? n - 1 : 0);
+        put_state();
     }
     if (d_initial) {
-        __syncthreads();
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-            const int idx = tid + 256 * i, r = idx >> 5, c = (idx & 31) * 4;
-            *reinterpret_cast<f32x4*>(d_initial + (head * GD + v0 + r) * GD + c) = *reinterpret_cast<const f32x4*>(&Ss[r][c]);
-        }
+        for (int c = 0; c < 4; ++c) *reinterpret_cast<f32x4*>(d_initial + (head * GD + v0 + ln) * GD + col + 8 * c) = f32x4{s[4 * c], s[4 * c + 1], s[4 * c + 2], s[4 * c + 3]};
     }
 }
 
