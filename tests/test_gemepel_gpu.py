@@ -675,3 +675,47 @@ def test_groups_of_any_length(lens, N, K, dt):
         rows = perm[int(offs[e]) : int(offs[e + 1])].long()
         want[rows] = a[rows].double() @ w[e].double().mT
     assert float((out.double() - want).norm()) < 2**-20 * float(want.norm())
+
+
+@pytest.mark.parametrize("T,H,D", [(1, 1, 1), (3, 5, 63), (7, 3, 64), (5, 2, 65), (2, 4, 128), (3, 2, 129), (2, 1, 256), (2, 2, 257), (1024, 12, 64), (4097, 3, 128), (1537, 8, 200), (2000, 16, 96)])
+def test_heads_of_a_wave(T, H, D):
+    """Kernels whose waves take several heads from some 12 000 on: one head to a wave or many, the rows' bits are those of the same rows in a short call; sizes around 64 values a lane's word."""
+    from llm_quest_amd import _lib as L
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(T + D)
+    few = min(T, 5)
+    o, gate = torch.randn(T, H * D, generator=g).to(DEV), torch.randn(T, H * D + 3, generator=g).to(torch.bfloat16).to(DEV)[:, 1 : H * D + 1]
+    w, freq, pos = torch.randn(D, generator=g).to(DEV), torch.rand(max(D // 2, 1), generator=g).to(DEV), torch.arange(T, dtype=torch.int32, device=DEV)
+    big, small = S.gated_headnorm(o, w, gate, H, D, 1e-6, torch.float32), S.gated_headnorm(o[:few].contiguous(), w, gate[:few], H, D, 1e-6, torch.float32)
+    assert torch.equal(big[:few], small)
+    x, z = o.double().view(T, H, D), gate.double().view(T, H, D)
+    want = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-6) * w.double() * z * torch.sigmoid(z)
+    assert float((big.double().view(T, H, D) - want).norm()) < 1e-6 * float(want.norm())
+    for dims in {0, D // 2, D // 4 * 2}:
+        dims -= dims % 2
+        for layout in (0, 1):
+            outs = []
+            for n in (T, few):
+                dst = torch.full((n, H * D), 7.0, device=DEV)
+                S.rope_heads(o[:n], H, D, D, 0, dst, D, 0, D - dims, dims, freq, pos[:n], layout)
+                outs.append(dst)
+            assert torch.equal(outs[0][:few], outs[1]) and not bool((outs[0] == 7).all())
+            i = torch.arange(dims // 2, device=DEV)
+            a, b = (i, i + dims // 2) if layout else (2 * i, 2 * i + 1)
+            ang = (pos.float()[:, None, None] * freq[: dims // 2]).double()
+            want = x.clone()
+            u, v = x[..., D - dims + a], x[..., D - dims + b]
+            want[..., D - dims + a], want[..., D - dims + b] = u * ang.cos() - v * ang.sin(), v * ang.cos() + u * ang.sin()
+            assert float((outs[0].double().view(T, H, D) - want).norm()) < 1e-6 * float(want.norm())
+    if D <= 256:
+        q, k, b, a = (torch.randn(T, n, generator=g).to(DEV) for n in (H * D, H * D, H, H))
+        A, dt, ws = torch.randn(H, generator=g).to(DEV), torch.randn(H, generator=g).to(DEV), []
+        L.require_gpu(q, k)
+        for n in (T, few):
+            ws.append(torch.empty(n, H, 4, device=DEV))
+            L.call("mi355_delta_rule_tokens", n, H, H, D, L.ptr(q), L.ptr(k), L.DT_F32, q.stride(0), k.stride(0), L.ptr(b), L.ptr(a), L.DT_F32, H, H, L.ptr(A), L.ptr(dt), 0.5, L.ptr(ws[-1]))
+        assert torch.equal(ws[0][:few], ws[1])
+        kd, qd = k.double().view(T, H, D), q.double().view(T, H, D)
+        want = torch.stack([torch.exp(-A.double().exp() * torch.nn.functional.softplus(a.double() + dt.double())), torch.sigmoid(b.double()), ((kd * kd).sum(-1) + 1e-6).rsqrt(), 0.5 * ((qd * qd).sum(-1) + 1e-6).rsqrt()], -1)
+        assert float((ws[0].double() - want).norm()) < 1e-6 * float(want.norm())
