@@ -2733,7 +2733,9 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,
         // which the four waves have no partner to hide (151 936 x 1 024, tile 5 / 3 / 1: 61 tokens 117 / 96 / 100, 333 196 / 174 / 200, 602 259 / 248 / 275, 1 024 367 / 374 / 398;
         // 50 256 x 768 (591 tiles): 61 tokens 36 / 28 / 25, 602 74 / 74 / 69, 1 500 136 / 147 / 144)
-        else if (form == MI355_GEMM_TN) cfg = M * N <= 5 * 1024 * 1024 || tiles256 < 160 ? 1 : K >= 1024 ? 5 : tiles256 >= 1024 ? 3 : 1;
+        // Of the two 256 x 256 tiles of eight waves the one with 64-token steps, where the last of them is more than half full (248 320 x 1 024, us, tile 3 / 2: 61 tokens 157 / 144, 128 185 / 172, 197
+        // 217 / 223, 333 281 / 276, 500 363 / 336, 700 437 / 421; 151 936 x 1 024 97 / 89, 113 / 110, 139 / 143, 175 / 178, 226 / 213, 272 / 263)
+        else if (form == MI355_GEMM_TN) cfg = M * N <= 5 * 1024 * 1024 || tiles256 < 160 ? 1 : K >= 1024 ? 5 : tiles256 >= 1024 ? ((K - 1) % 64 >= 32 ? 2 : 3) : 1;
         else if (form == MI355_GEMM_NT) cfg = 2;
         else cfg = 3;
     }

@@ -207,3 +207,22 @@ def test_fused_epilogues_are_the_128_x_128_kernels(M, N, K, rows):
     assert torch.equal(take(L.GEMM_NN, W, 2 * N, gu, L.EPI_SWIGLU_BWD, 0), take(L.GEMM_NN, W, 2 * N, gu, L.EPI_SWIGLU_BWD, 1))
     for residual in (None, r):
         assert torch.equal(take(L.GEMM_NT, Wt, N, residual, L.EPI_GELU, 0, bias), take(L.GEMM_NT, Wt, N, residual, L.EPI_GELU, 1, bias))
+
+
+@pytest.mark.parametrize("tokens", [32, 33, 64, 96, 97, 500, 1000])
+def test_wide_weight_gradients_of_few_tokens(tokens):
+    """Gradients of a thousand 256 x 256 tiles: the two tiles that a short sum may take give the same bits, which are the fp32 sum rounded once."""
+    from llm_quest_amd import _lib as L
+
+    V, D = 65536 + 40, 1024
+    g = torch.Generator().manual_seed(tokens)
+    dy, x = torch.randn(tokens, V, generator=g).to(torch.bfloat16).cuda(), torch.randn(tokens, D, generator=g).to(torch.bfloat16).cuda()
+    outs = []
+    for hint in (0, 2, 3):
+        out = torch.empty(V, D, dtype=torch.bfloat16, device="cuda")
+        L.require_gpu(dy, x, out)
+        L.call("mi355_gemm_bf16", 2, V, D, tokens, L.ptr(dy), V, L.ptr(x), D, L.ptr(out), D, L.DT_BF16, None, None, 0, 0, None, 0, hint)
+        outs.append(out)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+    want = dy[:, -300:].float().T.contiguous() @ x.float()
+    assert float((outs[0][-300:].float() - want).norm()) < 2**-8 * float(want.norm())
