@@ -278,7 +278,11 @@ class GroupedSigmoidMoE(_Frozen):
             self.correction32 = _f32(self.correction)
             self._ready = device
 
-    def route(self, x32):
+    def route(self, logits):
+        return S.moe_route(logits, self.correction32, self.top, self.groups, self.keep, self.scale)
+
+    def choose(self, x32):
+        """The rows' experts, weights and dispatch lists: ``route`` of the router's logits, and the lists."""
         return S.moe_choose(x32, self.w_router, self.correction32, self.top, self.groups, self.keep, self.scale)
 
     @torch.no_grad()
@@ -286,7 +290,7 @@ class GroupedSigmoidMoE(_Frozen):
         """x32: the fp32 residual rows (the router reads them), h: the same rows in the activation dtype -> fp32 [T * top, width]."""
         self.prepare(h.device)
         T, E, top = h.shape[0], self.experts, self.top
-        ids, wts, offs, perm = self.route(x32)
+        ids, wts, offs, perm = self.choose(x32)
         act = torch.empty((T * top, self.ff), dtype=h.dtype, device=h.device)
         S.bgemm(h, self.w_up, act, T * top, self.ff, self.width, batch=E, sbn=self.width, b_bs=self.ff * self.width, grp_offs=offs, a_rows=perm, a_div=top, epi=1)
         out = torch.empty((T * top, self.width), dtype=F32, device=h.device)
@@ -301,7 +305,10 @@ class GroupedSoftmaxMoE(GroupedSigmoidMoE):
     def __init__(self, width, ff, experts, top, groups=1, keep=1, scale=1.0):
         super().__init__(width, ff, experts, top, groups, keep, scale, correction=False)
 
-    def route(self, x32):
+    def route(self, logits):
+        return S.moe_route(logits, None, self.top, self.groups, self.keep, self.scale, softmax=True)
+
+    def choose(self, x32):
         return S.moe_choose(x32, self.w_router, None, self.top, self.groups, self.keep, self.scale, True)
 
 

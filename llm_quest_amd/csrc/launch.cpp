@@ -23,7 +23,7 @@
     E(gated_delta_rule_fwd) E(causal_conv_silu_step) E(gated_delta_rule_bwd) E(gdr_chunked_fwd) E(gdr_chunked_bwd) E(gated_rmsnorm_fwd) E(gated_rmsnorm_bwd) \
     E(resize_h_u8) E(resize_v_normalize) E(pad_tokens) E(gemv_bf16) E(gemv_bf16_f32out) E(gemv_bf16_pro) E(decode_block) E(decode_blocks) E(attn_decode_qkv) E(decode_advance) \
     E(attn_decode) E(kv_append_rows) E(kv_append) E(argmax_rows) E(argmax_rows_f32) E(embed_hash_fwd) E(add_layernorm_fwd) E(rmsnorm_rows) E(delta_rule_tokens) \
-    E(delta_chunked) E(latent_kv_append) E(rope_heads) E(gated_headnorm) E(gla_fwd) E(gla_fwd_below) E(router_logits) E(moe_route) E(moe_dispatch) E(moe_table_dispatch) \
+    E(delta_chunked) E(latent_kv_append) E(rope_heads) E(gated_headnorm) E(gla_fwd) E(gla_fwd_below) E(router_logits) E(moe_route) E(moe_dispatch) E(moe_choose) E(moe_table_dispatch) \
     E(bgemm) E(latent_attn) E(group_rmsnorm_sum) E(ragged_conv) E(qkv_rows_append) E(delta_rule_ragged) E(glu_rows) E(sandwich_rmsnorm) E(pool_rows_update) E(act_rows) \
     E(dyt_sum) E(token_shift) E(linrec_ragged) E(rglru_ragged) E(gated_groupnorm) E(unary_rows) E(mingru_ragged) E(depth_sum) E(diff_attn) E(diff_join) E(hyper_mix) \
     E(mfma_pipe_probe) E(rope_apply) E(dropout) E(attn_dropout_fwd) E(attn_generic_dropout_fwd) E(attn_generic_dropout_bwd) E(attn_dropout_bwd)
