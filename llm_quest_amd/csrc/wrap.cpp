@@ -1189,11 +1189,14 @@ OP(embed_hash, "tok", "prev", "table", "scale", "bigram", "buckets", "mul_prev",
 }
 
 // ---------------------------------------------------------------------------------------------- the operators as callables
+// What a function can do besides being called an operator can too: it is pickled and copied by its module and name, weakly referenced, bound where it is a class's attribute, and asked for whatever else
+// its Python form has (__code__, __defaults__, ...).
 struct Callable {
     PyObject_HEAD
     vectorcallfunc vectorcall;
     PyObject* slow;
     PyObject* dict;
+    PyObject* weak;
     Op* op;
 };
 
@@ -1239,6 +1242,7 @@ PyObject* op_vectorcall(PyObject* self, PyObject* const* args, size_t nargsf, Py
 void op_dealloc(PyObject* self) {
     PyObject_GC_UnTrack(self);
     Callable* f = reinterpret_cast<Callable*>(self);
+    if (f->weak) PyObject_ClearWeakRefs(self);
     Py_CLEAR(f->slow);
     Py_CLEAR(f->dict);
     PyObject_GC_Del(self);
@@ -1256,6 +1260,15 @@ int op_clear(PyObject* self) {
     return 0;
 }
 PyObject* op_repr(PyObject* self) { return PyUnicode_FromFormat("<native form of %R>", reinterpret_cast<Callable*>(self)->slow); }
+PyObject* op_reduce(PyObject* self, PyObject*) { return PyObject_GetAttrString(self, "__qualname__"); }
+PyObject* op_descr_get(PyObject* self, PyObject* of, PyObject*) { return of && of != Py_None ? PyMethod_New(self, of) : Py_NewRef(self); }
+PyObject* op_getattro(PyObject* self, PyObject* name) {
+    PyObject* own = PyObject_GenericGetAttr(self, name);
+    if (own || !PyErr_ExceptionMatches(PyExc_AttributeError)) return own;
+    PyErr_Clear();
+    return PyObject_GetAttr(reinterpret_cast<Callable*>(self)->slow, name);
+}
+PyMethodDef op_methods[] = {{"__reduce__", op_reduce, METH_NOARGS, "by module and name, as a function"}, {}};
 PyGetSetDef op_getset[] = {{"__dict__", PyObject_GenericGetDict, PyObject_GenericSetDict, nullptr, nullptr}, {}};
 PyTypeObject op_type = {PyVarObject_HEAD_INIT(nullptr, 0)};
 
@@ -1267,7 +1280,7 @@ PyObject* operator_for(PyObject*, PyObject* args) {  // (name, Python form) -> t
         if (!strcmp(ops[i].name, name)) {
             Callable* f = PyObject_GC_New(Callable, &op_type);
             if (!f) return nullptr;
-            f->vectorcall = op_vectorcall, f->slow = Py_NewRef(slow), f->dict = nullptr, f->op = &ops[i];
+            f->vectorcall = op_vectorcall, f->slow = Py_NewRef(slow), f->dict = nullptr, f->weak = nullptr, f->op = &ops[i];
             PyObject_GC_Track(reinterpret_cast<PyObject*>(f));
             return reinterpret_cast<PyObject*>(f);
         }
@@ -1350,7 +1363,10 @@ PyMODINIT_FUNC PyInit__wrap() {
     op_type.tp_repr = op_repr;
     op_type.tp_getset = op_getset;
     op_type.tp_dictoffset = offsetof(Callable, dict);
-    op_type.tp_getattro = PyObject_GenericGetAttr;
+    op_type.tp_weaklistoffset = offsetof(Callable, weak);
+    op_type.tp_methods = op_methods;
+    op_type.tp_descr_get = op_descr_get;
+    op_type.tp_getattro = op_getattro;
     op_type.tp_setattro = PyObject_GenericSetAttr;
     if (PyType_Ready(&op_type) < 0) return nullptr;
     for (int i = 0; i < n_ops; ++i)

@@ -1,7 +1,11 @@
 """The native forms of the launchers (csrc/wrap.cpp) against their Python forms, without a GPU: what each would hand to the library, and what it returns, over the forms that a call may have -- strides,
 optional operands, types, odd sizes -- and over calls that the Python form refuses, which the native one must leave to it."""
+import copy
+import functools
 import inspect
 import itertools
+import pickle
+import weakref
 
 import pytest
 import torch
@@ -118,6 +122,23 @@ def rows(r, c, dtype=B, pad=0):
 
 def ints(n):
     return torch.arange(n, dtype=I)
+
+
+def test_operators_are_what_functions_are_besides_being_called():
+    class Holder:
+        product = K.gemm
+
+    for name, _ in L._wrap.names():
+        f, slow = form(name), form(name).__wrapped__
+        assert pickle.loads(pickle.dumps(f)) is f and copy.deepcopy(f) is f and copy.copy(f) is f and weakref.ref(f)() is f
+        assert f.__name__ == name and f.__code__ is slow.__code__ and f.__defaults__ == slow.__defaults__ and f.__globals__ is slow.__globals__ and inspect.signature(f) == inspect.signature(slow)
+        assert not hasattr(f, "nothing") and f.__doc__ == slow.__doc__
+    module = torch.nn.Module()
+    module.product, module.half = K.gemm, functools.partial(K.gemm, L.GEMM_NT)
+    copied = copy.deepcopy(module)
+    assert copied.product is K.gemm and copied.half.func is K.gemm and copied.half.args == (L.GEMM_NT,) and pickle.loads(pickle.dumps(copied.half)).func is K.gemm
+    h = Holder()
+    assert Holder.product is K.gemm and inspect.ismethod(h.product) and h.product.__self__ is h and h.product.__func__ is K.gemm
 
 
 def test_arguments_are_named_as_in_python():
