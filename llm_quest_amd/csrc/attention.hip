@@ -1681,6 +1681,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dq_spill_kernel(int B, int S,
 // -- their K and V rows as operands, dK^T and dV^T as accumulators -- and the workgroup sweeps 64-query tiles:
 //   S = Q K^T, dP = dO V^T, P = exp2(S c - lse'), dS = P (dP - delta), dV^T += dO^T P, dK^T += Q^T dS   (key on the lane; P and dS are the B operands as the accumulators hold them)
 //   dS [key][query] to LDS, and behind a barrier dQ^T = K^T dS^T, 16 x 16 tiles, two a wave, over all keys.
+// Under a causal mask 32 keys and 32 queries that lie wholly in front of them are not multiplied: a token whose numbers are not finite spoils no gradient that does not hang on it, but for those of its own 32.
 // delta = rowsum(dO O) is summed where dO is read.  Three passes (delta, dK / dV, dQ) read the operands three times and formed S and dP twice: 128 x 197 tokens, 12 heads, 260 -> 138 us, 5 x 197 26 -> 20,
 // 128 x 50 71 -> 36, 64 x 17 32 -> 12; the bytes of the first, 311 MB, take 64.  Bound: one workgroup a CU (93 KB), whose two waves a SIMD run products, exponentials and LDS reads (2.5, 3 and 4.7
 // thousand clocks of a tile's 10.5) one after the other; dQ of a tile beside the keys' side of the next, one barrier a tile, 143; a SIMD's two waves in opposite order 160 (registers spill).
@@ -1788,12 +1789,14 @@ __global__ __launch_bounds__(512) void attn_bwd_short_kernel(int S, int H, const
             keys(0, std::false_type{});
             keys(1, std::false_type{});
         } else if (live) {
-            for (int st = 0; st < 2 && q0 + 32 * st < S; ++st) keys(st, std::true_type{});
+            for (int st = 0; st < 2 && q0 + 32 * st < S; ++st)
+                if (!causal || 32 * wave < q0 + 32 * st + 32) keys(st, std::true_type{});  // (all keys behind all queries: a zero P would still be multiplied, and 0 x NaN is no zero)
         }
         __syncthreads();
         const int qt = wave >> 1, dh = wave & 1;  // 16 queries, 32 features of dQ
         f32x4 acc[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
-        for (int g = 0; g < groups && q0 + 16 * qt < S; ++g) {
+        const int seen = causal ? min(groups, (q0 + 16 * qt) / 32 + 1) : groups;  // (the others left no dS)
+        for (int g = 0; g < seen && q0 + 16 * qt < S; ++g) {
             const int r = 32 * g + 8 * grp + q4;
             const bf16x8 db = read_down(&Ds[r][16 * qt + 4 * p4], 4 * (QT + 8));
 #pragma unroll

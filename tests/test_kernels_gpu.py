@@ -486,7 +486,7 @@ def test_attention_backward_scratch_form_equals_recompute_form(K, B, S, Hq, Hkv,
 )
 def test_attention_backward_of_short_sequences(K, B, S, H, causal, mask):
     """One pass for head_dim 64 and up to 256 tokens, over the edges of its 32-key waves and 64-query tiles: against fp64 (bf16 P and dS: 2^-9 of a value, as the passes of longer sequences), on operands
-    and into gradients that are columns of wider rows; nothing beside them is written; keys that a mask hides get zeros, and what stands in their rows, or in the next sequence, reaches no other."""
+    and into gradients that are columns of wider rows; nothing beside them is written; keys that a mask hides get zeros, and what stands in the next sequence reaches no other."""
     D, w = 64, 8
     g = torch.Generator().manual_seed(S)
     x = torch.randn(B * S, 3 * H * D, generator=g).to(BF16)
@@ -524,6 +524,36 @@ def test_attention_backward_of_short_sequences(K, B, S, H, causal, mask):
         do2 = do.clone()
         do2[S:] = float("nan")
         assert all(torch.equal(a[:S], b[:S]) for a, b in zip(got, run(do2)))
+
+
+@pytest.mark.parametrize("S", [33, 65, 197, 256])
+def test_attention_backward_of_short_causal_sequences_keeps_tokens_apart(K, S):
+    """Under the causal mask the queries' gradients of the first 32 n tokens hang on nothing behind them, and the keys' and values' gradients of the others on no query before them: the same bits
+    where those are NaN."""
+    B, H, D = 2, 3, 64
+    g = torch.Generator().manual_seed(S)
+    q, k, v, do = (dev(torch.randn(B, S, H * D, generator=g).to(BF16)) for _ in range(4))
+    rows = lambda t: t.view(B * S, H * D)
+    o, lse = K.attn_fwd(rows(q), rows(k), rows(v), B, S, H, H, D, causal=True)
+    o = o.view(B, S, H * D)
+
+    def run(q, k, v, o, do, lse):
+        out = [torch.empty(B * S, H * D, dtype=BF16, device="cuda") for _ in range(3)]
+        K.attn_bwd(rows(q), rows(k), rows(v), rows(o), rows(do), lse, B, S, H, H, D, *out, causal=True)
+        return [t.view(B, S, H * D) for t in out]
+
+    def lost(t, part):
+        t = t.clone()
+        (t[:, part] if t.dim() == 3 and t.shape[1] == S else t[:, :, part]).fill_(float("nan"))
+        return t
+
+    dq, dk, dv = run(q, k, v, o, do, lse)
+    for cut in range(32, S, 32):
+        late, early = slice(cut, S), slice(0, cut)
+        got = run(*(lost(t, late) for t in (q, k, v, o, do, lse)))
+        assert torch.equal(got[0][:, early], dq[:, early])
+        got = run(lost(q, early), k, v, lost(o, early), lost(do, early), lost(lse, early))
+        assert torch.equal(got[1][:, late], dk[:, late]) and torch.equal(got[2][:, late], dv[:, late])
 
 
 @pytest.mark.parametrize(
