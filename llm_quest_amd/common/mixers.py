@@ -278,12 +278,19 @@ class GroupedSigmoidMoE(_Frozen):
             self.correction32 = _f32(self.correction)
             self._ready = device
 
+    def _rule(self):
+        return self.correction32, self.top, self.groups, self.keep, self.scale
+
     def route(self, logits):
-        return S.moe_route(logits, self.correction32, self.top, self.groups, self.keep, self.scale)
+        """The router's logits' (ids int32 [tokens, top], weights fp32 [tokens, top]).  One that takes this one's place, in a subclass or on an instance, decides."""
+        return S.moe_route(logits, *self._rule())
 
     def choose(self, x32):
-        """The rows' experts, weights and dispatch lists: ``route`` of the router's logits, and the lists."""
-        return S.moe_choose(x32, self.w_router, self.correction32, self.top, self.groups, self.keep, self.scale)
+        """The rows' experts, weights and dispatch lists: ``route`` of the router's logits, and the lists; the classes' own ``route`` of few tokens in one launch with the rest."""
+        if getattr(self.route, "__func__", None) is GroupedSigmoidMoE.route:
+            return S.moe_choose(x32, self.w_router, *self._rule())
+        ids, wts = self.route(S.router_logits(x32, self.w_router))
+        return (ids, wts, *S.moe_dispatch(ids.view(-1), self.experts))
 
     @torch.no_grad()
     def step(self, x32, h):
@@ -305,11 +312,8 @@ class GroupedSoftmaxMoE(GroupedSigmoidMoE):
     def __init__(self, width, ff, experts, top, groups=1, keep=1, scale=1.0):
         super().__init__(width, ff, experts, top, groups, keep, scale, correction=False)
 
-    def route(self, logits):
-        return S.moe_route(logits, None, self.top, self.groups, self.keep, self.scale, softmax=True)
-
-    def choose(self, x32):
-        return S.moe_choose(x32, self.w_router, None, self.top, self.groups, self.keep, self.scale, True)
+    def _rule(self):
+        return None, self.top, self.groups, self.keep, self.scale, True
 
 
 # ----------------------------------------------------------------------------------------------- mechanisms of parallel-sublayer hybrid decoders

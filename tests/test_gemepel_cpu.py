@@ -111,3 +111,33 @@ def test_registry_and_loader_checks(tmp_path):
         from llm_quest_amd import kernels_seq as S
 
         S.rmsnorm_rows(torch.zeros(2, 8), torch.ones(8), 1e-6)
+
+
+def test_a_router_of_ones_own_decides_the_experts(monkeypatch):
+    """``route`` in a subclass or on an instance is asked for the choice; the classes' own goes with logits and lists in one call, with the same rule."""
+    import types
+
+    from llm_quest_amd.common import mixers as M
+
+    asked = []
+    monkeypatch.setattr(M.S, "router_logits", lambda x, w: ("logits", x, w))
+    monkeypatch.setattr(M.S, "moe_dispatch", lambda ids, E: (("offs", ids.tolist(), E), "perm"))
+    monkeypatch.setattr(M.S, "moe_choose", lambda *a: asked.append(("choose", a)) or ("ids", "wts", "offs", "perm"))
+    monkeypatch.setattr(M.S, "moe_route", lambda *a, **k: asked.append(("route", (*a, *k.values()))) or ("ids", "wts"))
+    sigmoid, softmax = M.GroupedSigmoidMoE(8, 4, 6, 2, 3, 2, 2.5), M.GroupedSoftmaxMoE(8, 4, 6, 2)
+    sigmoid.correction32 = softmax.correction32 = None
+    for moe, rule in ((sigmoid, (None, 2, 3, 2, 2.5)), (softmax, (None, 2, 1, 1, 1.0, True))):
+        asked.clear()
+        assert moe.choose("x") == ("ids", "wts", "offs", "perm") and moe.route("z") == ("ids", "wts")
+        assert asked == [("choose", ("x", moe.w_router, *rule)), ("route", ("z", *rule))]
+
+    def own(self, logits):
+        assert logits == ("logits", "x", self.w_router)
+        return torch.tensor([[5, 1]], dtype=torch.int32), "weights"
+
+    on_instance = M.GroupedSigmoidMoE(8, 4, 6, 2, 3, 2, 2.5)
+    on_instance.route = types.MethodType(own, on_instance)
+    asked.clear()
+    for moe in (type("A", (M.GroupedSigmoidMoE,), {"route": own})(8, 4, 6, 2, 3, 2, 2.5), type("B", (M.GroupedSoftmaxMoE,), {"route": own})(8, 4, 6, 2), on_instance):
+        ids, wts, offs, perm = moe.choose("x")
+        assert ids.tolist() == [[5, 1]] and wts == "weights" and offs == ("offs", [5, 1], 6) and perm == "perm" and not asked
