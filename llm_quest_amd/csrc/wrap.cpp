@@ -112,27 +112,30 @@ PyObject* tuple(const A&... a) {  // steals nothing; tensors, none
     return out;
 }
 
-PyObject* kernels_item(const char* name) {  // borrowed
-    PyObject* o = kernels ? PyDict_GetItemString(kernels, name) : nullptr;
+PyObject* item(PyObject* space, const char* name) {  // borrowed
+    PyObject* o = space ? PyDict_GetItemString(space, name) : nullptr;
     need(o != nullptr);
     return o;
 }
-long kernels_int(const char* name) {
-    const long v = PyLong_AsLong(kernels_item(name));
+long number(PyObject* o) {
+    const long v = PyLong_AsLong(o);
     if (v == -1 && PyErr_Occurred()) PyErr_Clear(), throw Decline();
     return v;
 }
+PyObject* kernels_item(const char* name) { return item(kernels, name); }
+long kernels_int(const char* name) { return number(kernels_item(name)); }
 bool kernels_true(const char* name) { return PyObject_IsTrue(kernels_item(name)) == 1; }
 
 constexpr int MAX_ARGS = 34;
 
 struct Call {
     PyObject* v[MAX_ARGS] = {};
-    PyObject* self = nullptr;  // (the slow form, for names in errors)
+    PyObject* home = nullptr;  // the namespace of the Python form, whose constants hold here too
     int device = -1;
     bool ready = false;
     void* stream = nullptr;
 
+    long constant(const char* name) const { return number(item(home, name)); }
     bool given(int i) const { return v[i] && v[i] != Py_None; }
     T tensor(int i) {
         T t = maybe(i);
@@ -337,7 +340,7 @@ OP(gemm, "form", "a", "b", "out", "out_dtype", "bias", "residual", "gelu", "allo
 
 OP(dgrad, "dy", "w", "out") {
     const T dy = c.tensor(0), w = c.tensor(1), out = c.maybe(2);
-    need(dy.rows() && dy.size(0) < 1280);  // (kernels.dgrad_transposes says no to fewer rows than that)
+    need(dy.rows() && dy.size(0) < std::min(c.constant("DGRAD_NT_MIN_ROWS"), 1280L));  // (kernels.dgrad_transposes says no to fewer rows than both)
     return wrapped(product(c, MI355_GEMM_NN, dy, w, out, BF16, T{}, T{}, MI355_EPI_NONE, true));
 }
 
@@ -393,7 +396,7 @@ OP(rmsnorm_bwd, "x2d", "w", "rstd", "dy", "dres", "dw_out", "dw_accumulate") {
     const T x = c.tensor(0), w = c.tensor(1), rstd = c.tensor(2), dy = c.tensor(3), dres = c.maybe(4);
     T dw = c.maybe(5);
     need(x.dim() == 2 && dy.contiguous() && dy.like(x) && dy.is(BF16) && (!dres || (dres.contiguous() && dres.like(x) && dres.is(BF16))));
-    const int64_t rows = x.size(0), width = x.size(1), parts = std::min<int64_t>(kernels_int("NORM_PARTS"), (rows + 3) / 4);
+    const int64_t rows = x.size(0), width = x.size(1), parts = std::min<int64_t>(c.constant("NORM_PARTS"), (rows + 3) / 4);
     const bool accumulate = c.truth(6, false) && dw;
     const int dw_code = dw ? dw.code() : MI355_DT_F32;
     const T dx = c.empty_like(x), part = c.empty(x, {parts, width}, F32);
@@ -422,7 +425,7 @@ OP(qknorm_rope_bwd, "qkv", "qw", "kw", "cos", "sin", "pos", "rstd", "dq", "dk", 
     const int64_t tokens = qkv.size(0), hpw = D == 128 ? 4 : 8;
     need(!dq || (dq.contiguous() && dq.is(BF16) && dq.shape({tokens, Hq * D})));
     need(dk.contiguous() && dk.is(BF16) && dk.shape({tokens, Hkv * D}) && dqkv.contiguous() && dqkv.like(qkv) && dqkv.is(BF16));
-    const int64_t parts = std::min<int64_t>(kernels_int("QK_PARTS"), (tokens * ((Hq + Hkv + hpw - 1) / hpw) + 3) / 4);
+    const int64_t parts = std::min<int64_t>(c.constant("QK_PARTS"), (tokens * ((Hq + Hkv + hpw - 1) / hpw) + 3) / 4);
     const T part = c.empty(qkv, {parts, 2 * D}, F32);
     need(dry || slot::reduce_rows_f32.address);
     LAUNCH(qknorm_rope_bwd, tokens, Hq, Hkv, D, qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, part, parts);
@@ -720,7 +723,7 @@ OP(headnorm_rope_bwd, "src", "H", "D", "head_stride", "w_eff", "cos_t", "sin_t",
     const T src = c.tensor(0), w = c.maybe(4), cos = c.maybe(5), sin = c.maybe(6), pos = c.maybe(7), rstd = c.maybe(8), dout = c.tensor(9), dsrc = c.tensor(10);
     const int64_t H = c.integer(1), D = c.integer(2), hs = c.integer(3), dhs = c.integer(11);
     need(heads(src, H, D, hs) && heads(dsrc, H, D, dhs) && (!cos || cos.dim() == 2));
-    const int64_t tokens = src.size(0), R = cos ? cos.size(1) : 0, parts = std::max<int64_t>(1, std::min<int64_t>(kernels_int("NORM_PARTS"), (tokens * H + 3) / 4));
+    const int64_t tokens = src.size(0), R = cos ? cos.size(1) : 0, parts = std::max<int64_t>(1, std::min<int64_t>(c.constant("NORM_PARTS"), (tokens * H + 3) / 4));
     need(dout.is(BF16) && dout.contiguous() && dout.shape({tokens, H * D}) && (dry || slot::reduce_rows_f32.address));
     const T part = c.empty(src, {parts, D}, F32);
     LAUNCH(headnorm_rope_bwd, tokens, H, D, R, src, src.ld(), hs, w, cos, sin, pos, rstd, dout, dsrc, dsrc.ld(), dhs, part, parts);
@@ -802,8 +805,8 @@ OP(causal_conv_silu_fwd, "x", "w", "B", "S") {
 
 OP(causal_conv_silu_bwd, "x", "w", "dy", "dx", "B", "S") {
     const T x = c.tensor(0), w = c.tensor(1), dy = c.tensor(2), dx = c.tensor(3);
-    const int64_t B = c.integer(4), S = c.integer(5), chunk = 32;  // kernels_q35.CONV_TOKEN_CHUNK
-    need(cols(x) && cols(dx) && w.dim() >= 1 && dy.is(BF16) && dy.contiguous() && dy.shape({B * S, x.size(1)}) && dx.shape({B * S, x.size(1)}) && (dry || slot::reduce_rows_f32.address));
+    const int64_t B = c.integer(4), S = c.integer(5), chunk = c.constant("CONV_TOKEN_CHUNK");
+    need(chunk > 0 && cols(x) && cols(dx) && w.dim() >= 1 && dy.is(BF16) && dy.contiguous() && dy.shape({B * S, x.size(1)}) && dx.shape({B * S, x.size(1)}) && (dry || slot::reduce_rows_f32.address));
     const int64_t C = x.size(1), ks = w.size(w.dim() - 1);
     const void* mine = dx.t.storage().data();  // only a gradient that overwrites its operands needs scratch
     const T ws = mine == x.t.storage().data() || mine == dy.t.storage().data() ? c.empty(x, {B * S, C}, BF16) : T{};
@@ -842,7 +845,7 @@ OP(gated_rmsnorm_bwd, "o", "w_f32", "gate", "rstd", "dout", "dgate", "H", "D") {
     const T o = c.tensor(0), w = c.tensor(1), gate = c.tensor(2), rstd = c.tensor(3), dout = c.tensor(4), dgate = c.tensor(5);
     const int64_t H = c.integer(6), D = c.integer(7);
     need(cols(dgate) && o.dim() == 2 && gate.dim() >= 1 && dout.is(BF16) && dout.contiguous() && dout.like(o) && dgate.like(o) && (dry || slot::reduce_rows_f32.address));
-    const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(kernels_int("NORM_PARTS"), (o.size(0) * H + 3) / 4));
+    const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(c.constant("NORM_PARTS"), (o.size(0) * H + 3) / 4));
     const T d_o = c.empty_like(o), part = c.empty(o, {parts, D}, F32);
     LAUNCH(gated_rmsnorm_bwd, o.size(0), H, D, o, w, gate, gate.ld(), rstd, dout, d_o, dgate, dgate.ld(), part, parts);
     return tuple(d_o, reduce_parts(c, part));
@@ -1222,6 +1225,7 @@ PyObject* op_vectorcall(PyObject* self, PyObject* const* args, size_t nargsf, Py
     HANDLE_TH_ERRORS
     if (fn_device && at::impl::PythonTorchFunctionTLS::stack_len() == 0 && !c10::impl::TorchDispatchModeTLS::any_modes_set()) {
         Call c;
+        c.home = PyFunction_Check(f->slow) ? PyFunction_GET_GLOBALS(f->slow) : nullptr;
         if (bound(*f->op, c, args, PyVectorcall_NARGS(nargsf), kwnames)) {
             try {
                 return f->op->body(c);

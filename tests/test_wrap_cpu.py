@@ -183,6 +183,31 @@ def test_products_that_the_persistent_kernel_may_take_are_counted_in_python(both
     assert not both("gemm", L.GEMM_TN, a, a) and both("gemm", L.GEMM_NT, a[:256], b)
 
 
+def test_constants_are_read_where_the_python_form_reads_them(both, monkeypatch):
+    """One that is changed in its module holds for both forms: the same calls, or none natively."""
+    monkeypatch.setattr(K, "transpose", lambda w: w.t().contiguous())
+    dy, w = rows(600, 64), rows(64, 40)
+    assert both("dgrad", dy, w) and both("dgrad", torch.empty(1279, 4096, dtype=B), torch.empty(4096, 1024, dtype=B))  # (a row more is transposed)
+    with monkeypatch.context() as m:
+        m.setattr(K, "DGRAD_NT_MIN_ROWS", 512)
+        assert not both("dgrad", dy, w) and both("dgrad", dy[:511], w)
+        m.setattr(K, "DGRAD_NT_MIN_ROWS", 1 << 20)
+        assert not both("dgrad", rows(1280, 64), w) and both("dgrad", rows(1279, 64), w)
+    x, g = rows(40, 16), rows(40, 16)
+    for parts in (3, 512):
+        monkeypatch.setattr(K, "NORM_PARTS", parts)
+        monkeypatch.setattr(K, "QK_PARTS", parts)
+        monkeypatch.setattr(Q, "NORM_PARTS", 8 * parts)
+        monkeypatch.setattr(Q, "CONV_TOKEN_CHUNK", parts + 4)
+        assert both("rmsnorm_bwd", x, torch.randn(16).to(B), torch.randn(40), g)
+        assert both("gated_rmsnorm_bwd", x, torch.randn(8), x, torch.randn(40, 2), g, rows(40, 16), 2, 8)
+        assert both("headnorm_rope_bwd", x, 2, 8, 8, torch.randn(8).to(B), None, None, None, torch.randn(40, 2), g, rows(40, 16), 8)
+        assert both("qknorm_rope_bwd", rows(40, 6 * 64), None, None, None, None, None, None, None, rows(40, 64), rows(40, 6 * 64), 4, 1, 64)
+        assert both("causal_conv_silu_bwd", x, torch.randn(16, 1, 4).to(B), g, rows(40, 16), 2, 20)
+    monkeypatch.setattr(Q, "CONV_TOKEN_CHUNK", "thirty")
+    assert not both("causal_conv_silu_bwd", x, torch.randn(16, 1, 4).to(B), g, rows(40, 16), 2, 20)
+
+
 def test_training_rows(both):
     for M, W in ((1, 8), (37, 256)):
         x, w, g = rows(M, W), torch.randn(W).to(B), rows(M, W)
