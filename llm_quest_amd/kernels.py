@@ -439,18 +439,21 @@ def release_attention_scratch():
 def _attn_scratch(device, nbytes):
     """dS scratch of the attention backward, one per (device, stream): every layer of a model reuses it (a backward pass fills it and
     empties it again before the next one starts on the same stream).  Returns None when the request is over the cap or cannot be
-    allocated -- the caller then runs the recompute form.  A buffer more than 4x the request is replaced by a fitting one."""
+    allocated -- the caller then runs the recompute form.  A buffer more than 4x the request is replaced by a fitting one; one that is too small
+    for a request that is not granted stays for those it serves."""
     if nbytes > _ATTN_DS_SPILL_MAX:
         return None
     key = (device, L.stream(device))
-    ws = _ATTN_WS.pop(key, None)
-    if ws is not None and (ws.numel() < nbytes or ws.numel() > 4 * nbytes):
-        ws = None
+    held = _ATTN_WS.pop(key, None)
+    ws = held if held is not None and nbytes <= held.numel() <= 4 * nbytes else None
     if ws is None:
         free, _ = torch.cuda.mem_get_info(device)
-        cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device)
+        cached = torch.cuda.memory_reserved(device) - torch.cuda.memory_allocated(device) + (0 if held is None else held.numel())
         if nbytes > (free + cached) // 4:
+            if held is not None:
+                _ATTN_WS[key] = held
             return None
+        held = None  # its memory may serve
         try:
             ws = torch.empty(nbytes, dtype=torch.uint8, device=device)
         except torch.OutOfMemoryError:
