@@ -642,11 +642,12 @@ def test_choice_of_experts_among_equals_and_none(E, top, groups, keep):
 @pytest.mark.parametrize("M,N,K", [(129, 128, 1024), (192, 130, 1032), (193, 1, 1096), (450, 1024, 2048), (300, 260, 1992), (1000, 384, 1024), (130, 512, 4096), (450, 1024, 1016)])
 def test_tiles_of_eight_waves(M, N, K):
     """Few tiles of a long sum go to eight waves, which divide its shares: the bits of four (the same rows among enough others to fill the chip) over sums that are no whole number of shares or
-    steps, in groups, gated and scattered, and an infinity's row by FMA as ever."""
+    steps, and an infinity's row by FMA as ever."""
     from llm_quest_amd import kernels_seq as S
 
-    g = torch.Generator().manual_seed(M + K)
-    many = 16384 // ((N + 127) // 128)
+    g, tn = torch.Generator().manual_seed(M + K), (N + 127) // 128
+    many = 24576 // tn
+    assert tn * ((M + 63) // 64) <= 256 < tn * ((many + 63) // 64) and tn * ((many + 127) // 128) < 512  # 64-row tiles of eight waves (from K = 1 024 on) and of four
     a, w = torch.randn(many, K, generator=g).to(DEV), (torch.randn(N, K, generator=g) * K**-0.5).to(torch.bfloat16).to(DEV)
     a[1, 3], a[M - 1, K - 1] = float("inf"), float("nan")
     few, all_ = torch.empty(M, N, device=DEV), torch.empty(many, N, device=DEV)
@@ -655,6 +656,37 @@ def test_tiles_of_eight_waves(M, N, K):
     assert torch.equal(few.view(torch.int32), all_[:M].view(torch.int32))
     want = a[2 : M - 1].double() @ w.double().mT
     assert float((few[2 : M - 1].double() - want).norm()) < 2**-21 * float(want.norm())  # (sums of K products in eight shares, each product 2^-24)
+
+
+@pytest.mark.parametrize("lens,N,K", [([0, 70, 1, 0, 64, 130], 256, 1024), ([129], 128, 1032), ([3, 200, 0, 65], 192, 1096), ([64, 64, 64], 128, 2048)])
+@pytest.mark.parametrize("epi", [0, 1, 2, 4])
+def test_tiles_of_eight_waves_in_groups(lens, N, K, epi):
+    """The same of gathered and scattered rows in groups, with the row's factor, squared ReLU and the gated epilogues: the bits of four waves, which take the call once a last group makes it a large one."""
+    from llm_quest_amd import kernels_seq as S
+
+    g, tn, T, E = torch.Generator().manual_seed(N + K), (N + 127) // 128, sum(lens), len(lens)
+    more = 24576 // tn - T
+    assert T > 128 and tn * ((T + 63) // 64 + E // 2) <= 256 < tn * ((T + more + 63) // 64) and tn * ((T + more + 127) // 128) < 512
+    a, w = torch.randn(T + more, K, generator=g).to(DEV), (torch.randn(E + 1, N, K, generator=g) * K**-0.5).to(torch.bfloat16).to(DEV)
+    offs = torch.tensor([0] + [sum(lens[: i + 1]) for i in range(E)] + [T + more], dtype=torch.int32, device=DEV)
+    to, scale = torch.randperm(T, generator=g), torch.rand(T + more, generator=g).to(DEV)
+    rows = torch.cat([to, torch.arange(T, T + more)]).to(torch.int32).to(DEV)
+    width, outs = N // 2 if epi >= 2 else N, []
+    for n, groups in ((T, E), (T + more, E + 1)):
+        out = torch.full((n, width + 2), 7.0, device=DEV)
+        S.bgemm(a, w, out, n, N, K, batch=groups, sbn=K, b_bs=N * K, grp_offs=offs, a_rows=rows, c_rows=rows, row_scale=scale, epi=epi, limit=2.5, n_out=width if epi >= 2 else 0)
+        assert bool((out[:, width:] == 7).all())
+        outs.append(out[:T, :width])
+    assert torch.equal(outs[0], outs[1]) and not bool((outs[0] == 7).any())
+    e = max(range(E), key=lambda i: lens[i])
+    r = rows[int(offs[e]) : int(offs[e + 1])].long()
+    y = a[r].double() @ w[e].double().mT
+    if epi >= 2:
+        v = y.view(len(r), -1, 2, 32)
+        gt, up = (v[:, :, i].flatten(1) for i in (0, 1))
+        y = gt.clamp(max=2.5) * torch.sigmoid(1.702 * gt.clamp(max=2.5)) * (up.clamp(-2.5, 2.5) + 1) if epi == 2 else torch.nn.functional.silu(gt) * up
+    y = (torch.relu(y) ** 2 if epi == 1 else y) * scale[r].double()[:, None]
+    assert float((outs[0][r].double() - y).norm()) < 2**-19 * float(y.norm())  # (the sum's 2^-21, squared or through a gate, and the epilogue's roundings)
 
 
 @pytest.mark.parametrize("lens,N,K", [([0, 70, 1, 0, 64, 130], 256, 1024), ([65, 0, 0, 200], 128, 2048), ([3] * 60, 64, 1024), ([400, 0, 500], 192, 512)])
@@ -677,9 +709,11 @@ def test_groups_of_any_length(lens, N, K, dt):
     assert float((out.double() - want).norm()) < 2**-20 * float(want.norm())
 
 
-@pytest.mark.parametrize("T,H,D", [(1, 1, 1), (3, 5, 63), (7, 3, 64), (5, 2, 65), (2, 4, 128), (3, 2, 129), (2, 1, 256), (2, 2, 257), (1024, 12, 64), (4097, 3, 128), (1537, 8, 200), (2000, 16, 96)])
+@pytest.mark.parametrize("T,H,D", [(1, 1, 1), (3, 5, 63), (7, 3, 64), (5, 2, 65), (2, 4, 128), (3, 2, 129), (2, 1, 256), (2, 2, 257), (1024, 12, 64), (4097, 3, 128), (1537, 8, 200), (2000, 16, 96),
+                                   (2100, 16, 128), (4099, 16, 64), (8193, 16, 128)])
 def test_heads_of_a_wave(T, H, D):
-    """Kernels whose waves take several heads from some 12 000 on: one head to a wave or many, the rows' bits are those of the same rows in a short call; sizes around 64 values a lane's word."""
+    """Kernels whose waves take several heads from some 12 000 on: one head to a wave or many (of rotations two
+    from 1 024 tokens of 16 heads on, four from 2 048, eight from 4 096, all from 8 192), the rows' bits are those of the same rows in a short call; sizes around 64 values a lane's word, rotations of every lane's pair."""
     from llm_quest_amd import _lib as L
     from llm_quest_amd import kernels_seq as S
 
@@ -692,7 +726,7 @@ def test_heads_of_a_wave(T, H, D):
     x, z = o.double().view(T, H, D), gate.double().view(T, H, D)
     want = x * torch.rsqrt((x * x).mean(-1, keepdim=True) + 1e-6) * w.double() * z * torch.sigmoid(z)
     assert float((big.double().view(T, H, D) - want).norm()) < 1e-6 * float(want.norm())
-    for dims in {0, D // 2, D // 4 * 2}:
+    for dims in {0, D // 2, D // 4 * 2, D if D <= 128 else 128}:
         dims -= dims % 2
         for layout in (0, 1):
             outs = []
