@@ -1884,7 +1884,10 @@ extern "C" int mi355_attn_fwd(int B, int S, int Hq, int Hkv, int D, const void* 
 // Tiles to a part of the dK/dV pass (0: key blocks stay whole): the fewest, from SPLIT_TILES on, with which all parts are on the chip at once (one a CU).  From
 // 2 tiles on: 2 x 130 tokens, 16 heads over 16, 23 -> 26 us (a part's start and its 128 KB cost more than a tile); from 4 on: 1 x 128, 16 over 8, 24 against 19.  From 4 096 rows on the delta pass is
 // another product's epilogue, whose caller knows nothing of parts, and what it leaves is to give the same bits.
-constexpr int SPLIT_TILES = 3, SPLIT_CUS = 256;
+// Not where the parts, written and read again (0.05 us each with the chip full of them), cost what the longest chain becomes shorter by (2.3 us a tile): us, whole blocks / parts, 128 sequences of one
+// token, 4 heads over 1 (256 parts for two tiles) 23 / 36, 8 x 65, 16 over 8 (128) 25 / 28, 3 x 256 full, 16 over 16 (192) 30.3 / 32.0, 8 x 256 full, 16 over 8 (256 for four) 43 / 44; on the other
+// side 2 x 257, 16 over 16 (64 for two) 31.3 / 29.2, 8 x 256, 16 over 8 (128 for four) 42 / 40, 2 x 498, 16 over 16 (224 for five) 41.4 / 39.7.
+constexpr int SPLIT_TILES = 3, SPLIT_CUS = 256, SPLIT_PARTS_A_TILE = 48;
 static int dkv_split(int B, int S, int Hq, int Hkv, int D, int causal) {
     const int nblk = (S + 127) / 128, rep = Hq / Hkv;
     const int64_t pairs = (int64_t)B * Hkv;
@@ -1892,8 +1895,16 @@ static int dkv_split(int B, int S, int Hq, int Hkv, int D, int causal) {
     int64_t all = 0;
     for (int kb = 0; kb < nblk; ++kb) all += dkv_tiles(S, rep, causal, kb);
     const int longest = dkv_tiles(S, rep, causal, 0);
-    for (int64_t most = all * pairs / SPLIT_CUS > SPLIT_TILES ? all * pairs / SPLIT_CUS : SPLIT_TILES; most < longest; ++most)
-        if (pairs * dkv_blocks(S, rep, causal, (int)most, nblk) <= SPLIT_CUS) return (int)most;
+    for (int64_t most = all * pairs / SPLIT_CUS > SPLIT_TILES ? all * pairs / SPLIT_CUS : SPLIT_TILES; most < longest; ++most) {
+        if (pairs * dkv_blocks(S, rep, causal, (int)most, nblk) > SPLIT_CUS) continue;
+        int64_t written = 0;
+        for (int kb = 0; kb < nblk; ++kb) {
+            const int64_t n = (dkv_tiles(S, rep, causal, kb) + most - 1) / most;
+            written += n > 1 ? pairs * n : 0;
+        }
+        const int64_t n = (longest + most - 1) / most, chain = (longest + n - 1) / n;
+        return written <= SPLIT_PARTS_A_TILE * (longest - chain) ? (int)most : 0;
+    }
     return 0;
 }
 extern "C" int64_t mi355_attn_bwd_split_bytes(int B, int S, int Hq, int Hkv, int D, int causal) {

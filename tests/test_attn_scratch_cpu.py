@@ -54,3 +54,12 @@ def test_what_is_not_granted_takes_nothing_away(memory):
     assert K._attn_scratch(dev, 900).numel() == 900
     memory["free"] = 0
     assert K._attn_scratch(dev, 5000) is None and K._attn_scratch(dev, 900).numel() == 900 and memory["made"] == [900]
+
+
+@pytest.mark.parametrize("B,S,Hq,Hkv,causal,cut", [
+    (128, 1, 4, 1, True, False), (128, 17, 4, 1, False, False), (8, 65, 16, 8, True, False), (2, 197, 16, 16, False, False), (3, 256, 16, 16, False, False), (8, 257, 4, 4, False, False),
+    (8, 256, 16, 8, False, False), (8, 129, 16, 8, False, False), (1, 128, 16, 8, True, True), (1, 300, 16, 8, True, True), (2, 498, 16, 8, True, True), (1, 709, 16, 8, True, True), (3, 560, 16, 8, True, True),
+    (1, 1500, 16, 8, True, True), (1, 2000, 16, 8, False, True), (2, 257, 16, 16, True, True), (8, 256, 16, 8, True, True), (32, 64, 4, 1, True, True), (2, 498, 16, 16, True, True), (7, 584, 4, 4, True, True)])
+def test_which_key_blocks_are_split(B, S, Hq, Hkv, causal, cut):
+    """Split where the longest chain of tiles becomes shorter by more than the parts cost to write and add up, whole where it does not (both sides measured)."""
+    assert (K.L.load().mi355_attn_bwd_split_bytes(B, S, Hq, Hkv, 128, int(causal)) > 0) is cut
