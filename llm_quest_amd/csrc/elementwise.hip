@@ -466,7 +466,8 @@ __global__ __launch_bounds__(256) void embedding_bwd_kernel(int64_t tokens, int 
 // whatever the ids repeat, and only the touched rows move (the atomic form walks a dense fp32 copy of the table).
 // A run of equal ids can be long (padding or placeholder tokens: thousands of positions), so the sum is a fixed two-level tree over blocks of
 // EMB_BLK sorted positions, whatever the launch geometry: pass 1, a wave to each run's part inside a block, sums it in position order (one wave to a whole block: 32 different ids
-// were 32 memory round trips after another, 70 us and more for any number of tokens; now 6 us for 333 tokens, 17 016 25) --
+// were 32 memory round trips after another, 70 us and more for any number of tokens; now 6 us for 333 tokens, 17 016 22).  Neighbouring workgroups take the same position of neighbouring blocks: long
+// runs' parts all begin at their blocks' first positions, and with neighbouring positions to neighbouring workgroups every eighth had all the work, those of one XCD --
 // a run that lies inside one block is finished there; a part that began before the block goes to scratch slot 0 of the block, a part that goes on
 // past it to slot 1 -- and pass 2, one wave per block whose slot 1 is in use (the block that holds the run's first position), adds the slot-0
 // parts of the following blocks in block order and writes the row.  scale: 1 / world under data parallelism.
@@ -489,8 +490,10 @@ __global__ __launch_bounds__(256) void embedding_bwd_sorted_kernel(int64_t token
                                                                    float scale, bf16_t* __restrict__ table, int64_t ldt, int accumulate,
                                                                    float* __restrict__ part) {
     const int lane = threadIdx.x & 63;
-    for (int64_t j = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); j < tokens; j += (int64_t)gridDim.x * 4) {  // a wave to each position; where a run's part of its block begins, it sums that part
-        const int64_t blk = j / EMB_BLK, lo = blk * EMB_BLK, hi = min(tokens, lo + EMB_BLK);
+    const int64_t nblk = (tokens + EMB_BLK - 1) / EMB_BLK;
+    for (int64_t blk = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6); blk < nblk; blk += (int64_t)gridDim.x * 4) {  // a wave to each position; where a run's part of its block begins, it sums that part
+        const int64_t lo = blk * EMB_BLK, hi = min(tokens, lo + EMB_BLK), j = lo + blockIdx.y;
+        if (j >= tokens) continue;
         const int64_t id = sid[j];
         static_assert(EMB_BLK + 2 <= 64, "a wave looks at a block's positions and one on either side");
         const bool same = lane < EMB_BLK + 2 && lo - 1 + lane >= 0 && lo - 1 + lane < tokens && sid[lo - 1 + lane] == id;  // positions lo - 1 .. hi
@@ -878,7 +881,7 @@ extern "C" int mi355_embedding_bwd_sorted(int64_t tokens, int width, int64_t voc
                   "mi355_embedding_bwd_sorted: a 16-byte aligned workspace of %lld bytes is needed (mi355_embedding_bwd_sorted_workspace_bytes)",
                   (long long)mi355_embedding_bwd_sorted_workspace_bytes(tokens, width));
     const int64_t nblk = (tokens + EMB_BLK - 1) / EMB_BLK;
-    hipLaunchKernelGGL(embedding_bwd_sorted_kernel, dim3(grid_for(tokens, 4)), dim3(256), 0, STREAM, tokens, width, vocab, sorted_ids, perm, (const bf16_t*)dout, ldd,
+    hipLaunchKernelGGL(embedding_bwd_sorted_kernel, dim3((unsigned)((nblk + 3) / 4 < 1 << 20 ? (nblk + 3) / 4 : 1 << 20), (unsigned)(tokens < EMB_BLK ? tokens : EMB_BLK)), dim3(256), 0, STREAM, tokens, width, vocab, sorted_ids, perm, (const bf16_t*)dout, ldd,
                        scale, (bf16_t*)table, ldt, accumulate, workspace);
     if (nblk > 1)
         hipLaunchKernelGGL(embedding_bwd_join_kernel, dim3(grid_for(nblk - 1, 4)), dim3(256), 0, STREAM, tokens, width, vocab, sorted_ids, scale, (bf16_t*)table, ldt,
