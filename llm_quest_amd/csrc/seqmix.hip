@@ -298,11 +298,12 @@ extern "C" int mi355_latent_kv_append(int64_t tokens, int rank, int rot, const v
 // Copy n entries per head from src to dst (fp32) and turn the pairs of [rot_start, rot_start + dims) -- layout 0: neighbours (2i, 2i+1); layout 1: the
 // two halves of the range, (i, i + dims/2):
 // dst[t, h * dst_hs + dst_off + i] = src[t, h * src_hs + src_off + i]
+template <bool MANY>
 __global__ __launch_bounds__(256) void rope_heads_kernel(int64_t T, int H, int n, const void* __restrict__ src, int src_dt, int64_t lds_, int src_hs, int src_off,
                                                          float* __restrict__ dst, int64_t ldd, int dst_hs, int dst_off, int rot_start, int dims, int layout,
                                                          const float* __restrict__ freq, const int* __restrict__ pos, int own) {
     const int lane = threadIdx.x & 63;
-    if (own > 1) {  // a lane's pair has one angle for all heads of its token, `own` of which are a wave's
+    if constexpr (MANY) {  // a lane's pair has one angle for all heads of its token, `own` of which are a wave's
         const int parts = H / own;
         const int64_t items = T * parts;
         const int ia = rot_start + (layout ? lane : 2 * lane), ib = rot_start + (layout ? lane + dims / 2 : 2 * lane + 1);
@@ -352,10 +353,14 @@ extern "C" int mi355_rope_heads(int64_t tokens, int H, int n, const void* src, i
     MI355_REQUIRE(rot_start >= 0 && dims >= 0 && dims % 2 == 0 && rot_start + dims <= n && (dims == 0 || freq), "rope_heads: the rotated range must lie inside the head");
     MI355_REQUIRE(src_off >= 0 && dst_off >= 0 && ld_src >= (int64_t)(H - 1) * src_hs + src_off + n && ld_dst >= (int64_t)(H - 1) * dst_hs + dst_off + n, "rope_heads: rows too short");
     int own = 1;  // as many heads to a wave as leave eight waves for every SIMD: an angle costs as much as some ten heads.  5 400 tokens x 16 heads of
-    // 128: half of a head turned 27 -> 21 us, all of it 25 -> 18.
-    while (dims <= 128 && own < 16 && H % (2 * own) == 0 && tokens * (H / (2 * own)) >= 8192) own *= 2;
-    rope_heads_kernel<<<rows_grid(tokens * (H / own), 4), 256, 0, ST(stream)>>>(tokens, H, n, src, src_dt, ld_src, src_hs, src_off, dst, ld_dst, dst_hs, dst_off, rot_start, dims,
-                                                                                                layout, freq, pos, own);
+    // 128: half of a head turned 27 -> 21 us, all of it 25 -> 18.  (Of longer heads the rows are the time: 9 000 x 8 heads of 256, 16 of them turned 33 | 38, 128 28 | 30; a kernel of its own, or one head
+    // to a wave pays for its registers: 17 000 x 7 of 128, 16 turned 37 | 40.)
+    while (dims <= 128 && n <= 128 && own < 16 && H % (2 * own) == 0 && tokens * (H / (2 * own)) >= 8192) own *= 2;
+#define ROPE(MANY) rope_heads_kernel<MANY><<<rows_grid(tokens * (H / own), 4), 256, 0, ST(stream)>>>(tokens, H, n, src, src_dt, ld_src, src_hs, src_off, dst, ld_dst, dst_hs, dst_off, rot_start, dims, \
+                                                                                                     layout, freq, pos, own)
+    if (own > 1) ROPE(true);
+    else ROPE(false);
+#undef ROPE
     MI355_LAUNCH_CHECK("rope_heads");
     return 0;
 }
