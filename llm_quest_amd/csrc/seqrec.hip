@@ -636,6 +636,8 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(int64_t T, DeltaArgs p)
                 }
             }
         }
+        float bb = 0.f, aa = 0.f, dt = 0.f, al = 0.f;  // (one head: its numbers are on their way while its rows are summed)
+        if (U == 1 && V > 0 && lane == 0) bb = ldr_dt(p.b, p.ba_dt, t * p.ldb + h), aa = ldr_dt(p.a, p.ba_dt, t * p.lda + h), dt = p.dt_bias[h], al = p.A_log[h];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             float a = 0.f, c = 0.f;
@@ -658,10 +660,10 @@ __global__ __launch_bounds__(256) void delta_prep_kernel(int64_t T, DeltaArgs p)
         }
         const int64_t it = it0 + lane;
         if (lane < U && it < items) {
-            if (U > 1) t = it / p.H, h = (int)(it - t * p.H);
-            const float bb = ldr_dt(p.b, p.ba_dt, t * p.ldb + h), aa = ldr_dt(p.a, p.ba_dt, t * p.lda + h) + p.dt_bias[h];
+            if (U > 1 || V == 0) t = it / p.H, h = (int)(it - t * p.H), bb = ldr_dt(p.b, p.ba_dt, t * p.ldb + h), aa = ldr_dt(p.a, p.ba_dt, t * p.lda + h), dt = p.dt_bias[h], al = p.A_log[h];
+            aa += dt;
             const float sp = aa > 20.f ? aa : log1pf(expf(aa));
-            p.ws[it] = f32x4{expf(-expf(p.A_log[h]) * sp), 1.0f / (1.0f + expf(-bb)), 1.0f / sqrtf(sk + 1e-6f), p.qscale / sqrtf(sq + 1e-6f)};
+            p.ws[it] = f32x4{expf(-expf(al) * sp), 1.0f / (1.0f + expf(-bb)), 1.0f / sqrtf(sk + 1e-6f), p.qscale / sqrtf(sq + 1e-6f)};
         }
     }
 }
