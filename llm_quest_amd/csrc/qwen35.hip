@@ -347,15 +347,15 @@ __global__ __launch_bounds__(256) void conv_silu_fwd_kernel(int B, int S, int C,
 #pragma unroll
     for (int t = 0; t < TOK; ++t) {
         if (s0 + t >= S) break;
-        float o[8];
+        float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int c = 0; c < 8; ++c) {
-            float acc = 0.f;
+        for (int j = 0; j < KS; ++j)
+            if (s0 + t + j >= KS - 1) {  // (one condition a tap: one a channel and tap cost short sequences 0.4 us of 2.5)
 #pragma unroll
-            for (int j = 0; j < KS; ++j)
-                if (s0 + t + j >= KS - 1) acc = fmaf(at(wr[c * KS / 8], c * KS % 8 + j), at(xr[t + j], c), acc);
-            o[c] = silu_f(rbf(acc));
-        }
+                for (int c = 0; c < 8; ++c) o[c] = fmaf(at(wr[c * KS / 8], c * KS % 8 + j), at(xr[t + j], c), o[c]);
+            }
+#pragma unroll
+        for (int c = 0; c < 8; ++c) o[c] = silu_f(rbf(o[c]));
         *reinterpret_cast<u32x4*>(yp + (int64_t)(s0 + t) * C) = pack8(o);
     }
 }
