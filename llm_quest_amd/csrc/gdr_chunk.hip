@@ -487,6 +487,7 @@ __global__ __launch_bounds__(256, 2) void gdrc_rscan_kernel(int heads, int S, in
             f32x4 ph = {0.f, 0.f, 0.f, 0.f}, pl = ph;
 #pragma unroll
             for (int i = 0; i < 2; ++i) {
+                if (i == 0 && wave >= 2) continue;  // P is lower triangular, and its zeros are not multiplied: a dO that is not finite reaches no later token but those of its own 32
                 const bf16_t* o = &Os[32 * i + 8 * g + q4][16 * j + 4 * p4];
                 const bf16x4 o0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)(o)), o1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((__attribute__((address_space(3))) bf16x4*)(o + 4 * (GV + 8)));
                 const bf16x8 of = __builtin_shufflevector(o0, o1, 0, 1, 2, 3, 4, 5, 6, 7);

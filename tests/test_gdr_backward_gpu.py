@@ -56,6 +56,22 @@ def test_last_chunks_and_views(S, Hqk, Hv):
     assert all(torch.equal(a[:S], b[:S]) for a, b in zip(got[:4], lost)) and bool(torch.isfinite(lost[4][:S].float()).all())
 
 
+@pytest.mark.parametrize("S", [64, 65, 96, 130])
+def test_output_gradients_reach_no_later_token(S):
+    """A dO that is not finite reaches the tokens up to its own; of those behind it, its own 32 at most (in which zeros are multiplied)."""
+    B, Hqk, Hv = 1, 1, 2
+    q, k, v, beta, alpha, do = _operands(B, S, Hqk, Hv, S)
+    dv = torch.empty_like(v)
+    want = (*_backward(q, k, v, beta, alpha, do, dv, B, S, Hqk, Hv), dv)
+    for t in [t for t in (0, 17, 31, 32, 40, 63, 64, 97, 128) if t < S]:
+        for x in (float("inf"), float("nan")):
+            bad, dv = do.clone(), torch.empty_like(v)
+            bad[t, 130] = x
+            got = (*_backward(q, k, v, beta, alpha, bad, dv, B, S, Hqk, Hv), dv)
+            later = t // 32 * 32 + 32
+            assert all(torch.equal(a[later:], b[later:]) for a, b in zip(got, want)) and not bool(torch.isfinite(got[0][t].float()).all())
+
+
 @pytest.mark.parametrize("S,decay,size", [(64, 0.3, 1.0), (65, 8.0, 1e30), (96, 0.0, 1e-30), (127, 0.01, 1.0), (129, 8.0, 1.0), (192, 0.001, 1e30), (321, 0.3, 1e-3)])
 def test_state_from_a_state(S, decay, size):
     """The final state and the outputs of chunks that start from a state, against 64 bits, over whole and last chunks, decays from none to strong, and sizes where the parts of a split number come
