@@ -1735,8 +1735,8 @@ __global__ __launch_bounds__(512) void attn_bwd_short_kernel(int S, int H, const
     const bool open = 32 * wave + 32 <= S && key_mask == nullptr && !causal;  // no score of the wave's is hidden
     for (int q0 = 0; q0 < S; q0 += QT) {
         {   // (the last tile's readers are past the barrier in front of its dQ)
-            const bool in = q0 + row < S;
-            *reinterpret_cast<u32x4*>(&Qs[row][c8]) = in ? rq : none;
+            const bool in = q0 + row < S;  // (queries beyond the sequence: the last one's scores and no dO -- of a zero row 0 x inf would be a score that is none)
+            *reinterpret_cast<u32x4*>(&Qs[row][c8]) = rq;
             *reinterpret_cast<u32x4*>(&Os[row][c8]) = in ? rg : none;
             float x = 0.f;
 #pragma unroll
@@ -1745,7 +1745,7 @@ __global__ __launch_bounds__(512) void attn_bwd_short_kernel(int S, int H, const
                 x = fmaf(__uint_as_float(rg[e] & 0xffff0000u), __uint_as_float(ro[e] & 0xffff0000u), x);
             }
             x = lanes_sum<8>(x);
-            if ((tid & 7) == 0) nlse[row] = in ? -rl * LOG2E : 0.f, delta[row] = in ? x : 0.f;
+            if ((tid & 7) == 0) nlse[row] = -rl * LOG2E, delta[row] = in ? x : 0.f;
         }
         __syncthreads();
         if (q0 + QT < S) request(q0 + QT);

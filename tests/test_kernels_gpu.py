@@ -526,6 +526,22 @@ def test_attention_backward_of_short_sequences(K, B, S, H, causal, mask):
         assert all(torch.equal(a[:S], b[:S]) for a, b in zip(got, run(do2)))
 
 
+@pytest.mark.parametrize("S", [2, 33, 63, 65, 197, 255])
+@pytest.mark.parametrize("causal", [False, True])
+def test_attention_backward_of_short_sequences_with_a_key_that_is_never_chosen(K, S, causal):
+    """A key whose scores are all -inf has no weight: its gradients are zero, not the NaN of a query beyond the sequence's end."""
+    H, D, at = 2, 64, S // 2
+    g = torch.Generator().manual_seed(S)
+    q, k, v, do = (dev(torch.randn(S, H * D, generator=g).to(BF16)) for _ in range(4))
+    q[:, 5::D] = q[:, 5::D].abs() + 1
+    k[at, 5::D] = float("-inf")
+    o, lse = K.attn_fwd(q, k, v, 1, S, H, H, D, causal=causal)
+    dq, dk, dv = (torch.empty_like(q) for _ in range(3))
+    K.attn_bwd(q, k, v, o, do, lse, 1, S, H, H, D, dq, dk, dv, causal=causal)
+    for t in (dk, dv):
+        assert bool(torch.isfinite(t.float()).all()) and not bool(t[at].any())
+
+
 @pytest.mark.parametrize("S", [33, 65, 197, 256])
 def test_attention_backward_of_short_causal_sequences_keeps_tokens_apart(K, S):
     """Under the causal mask the queries' gradients of the first 32 n tokens hang on nothing behind them, and the keys' and values' gradients of the others on no query before them: the same bits
