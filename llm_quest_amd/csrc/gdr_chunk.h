@@ -52,6 +52,8 @@ __device__ __forceinline__ void add16(f32x16& to, f32x16& from) {  // a chain's 
 // ---- fp32 products on the bf16 matrix pipe: a number is the sum of three bf16 parts (24 bits: 8 and 8 and the rest, exactly), a product the sum of the parts' products, exact in fp32.  Of two split
 // operands the six largest are taken -- what is left out is 2^-26 of the product -- the first parts' by themselves in one accumulator, the others in a second: a sum over 128 rounds eight times at its
 // own size where a chain of fp32 products rounds 64 times.  32 clocks for 32 x 32 x 16 and 16 of a part against 512 on the fp32 pipe.  An infinity or a NaN makes the sum a NaN.
+// Not all 24 bits near the ends of the range: below some 2^-110 the third part is subnormal, or nothing; and what lies within half a step of bf16 of the largest number has an infinite first part, so
+// its sums are NaN (the forward's scan then takes the recurrence).
 struct Parts8 { bf16x8 p[3]; };  // eight consecutive k of a fragment's row
 __device__ __forceinline__ void parts_of(float a, float b, unsigned (&w)[3]) {
 #pragma unroll

@@ -31,11 +31,6 @@ constexpr int C_U = GC * GD, C_P = C_U + GC * GD, C_GAM = C_P + GC * GC, C_R = C
 constexpr int64_t SPAN_BYTES = 256 << 20;  // of a forward that keeps nothing: what one span of chunks takes at most, if that holds four (a prompt of any length, bounded scratch)
 constexpr int W_DU = GD * GD, W_BLOCK = W_DU + GC * GD;  // backward workspace of a chunk: dS at its end, dU
 
-// four consecutive bf16 of row `r` of a [tokens, ld] operand, zeros beyond the sequence
-__device__ __forceinline__ u32x2 row4(const bf16_t* p, int64_t ld, int r, int cnt, int c) {
-    return r < cnt ? *reinterpret_cast<const u32x2*>(p + r * ld + c) : u32x2{0u, 0u};
-}
-
 __device__ __forceinline__ double cumulated_log(const float* alpha, int64_t idx, bool in, float& a_out) {
     a_out = decay_at_least(in ? alpha[idx] : 1.f);
     return cumulated_log64(a_out);

@@ -322,8 +322,8 @@ __global__ __launch_bounds__(256) void gdn_gates_bwd_kernel(int64_t tokens, int 
 // ------------------------------------------------------------------------------------------- causal depthwise conv + SiLU
 // y[t, c] = bf16(silu(bf16(sum_j w[c, j] x[t - (k-1) + j, c])))  within each sequence (qwen3_5_text_model.py:81-90, 138-140).
 // A thread owns 8 adjacent channels (16-byte loads) of TOK tokens of one sequence.  Bound: a token read four times and its channels' taps, 64 bytes a thread, from the caches: two tokens read
-// five rows for two and the taps once; 5 664 tokens x 6 144 channels 57.7 -> 45.1 us (four 46.1, eight 50.7: fewer threads under way), 1 416 17.9 -> 16.3; below half a million threads level or
-// worse (333 tokens 7.3 / 7.3, 33 3.8 / 4.7).
+// five rows for two and the taps once; 5 664 tokens x 6 144 channels 57.7 -> 45.1 us (four 46.1, eight 50.7: fewer threads under way), 1 416 17.9 -> 14.9; below half a million threads worse
+// (one | two, 500 tokens 6.5 | 6.8, 333 5.2 | 5.5, 33 3.2 | 3.8).
 template <int KS, int TOK>
 __global__ __launch_bounds__(256) void conv_silu_fwd_kernel(int B, int S, int C, const bf16_t* __restrict__ x, int64_t ldx,
                                                             const bf16_t* __restrict__ w, bf16_t* __restrict__ y) {

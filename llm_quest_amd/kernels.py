@@ -424,7 +424,7 @@ _ATTN_ABLATE = int(os.environ.get("MI355_ATTN_ABLATE", "0")) << 8  # profiling s
 _ATTN_DS_SPILL = os.environ.get("MI355_ATTN_DS_SPILL", "1") != "0"  # 0: the dQ pass recomputes S and dP (no scratch)
 # The dS scratch grows with S^2 (2 bytes per (query, key) of the padded square per head): 1.2 GB at the headline shape, 17 GB at S = 8192, B = 8.
 # Above this cap -- or a quarter of the device's free memory, or when the allocation fails -- the backward takes the recompute form (three
-# products in the dQ pass, O(S) memory, bit-identical gradients): long-context training keeps working, only slower per layer.
+# products in the dQ pass, O(S) memory; gradients 3.5e-3 of their norm apart, the rounding of bf16 operands): long-context training keeps working, only slower per layer.
 _ATTN_DS_SPILL_MAX = int(float(os.environ.get("MI355_ATTN_DS_SPILL_MAX_MB", "4096")) * (1 << 20))
 _ATTN_WS = {}  # (device, stream handle) -> uint8 buffer; at most _ATTN_WS_SLOTS entries (least recently used dropped: dead streams do not pin memory)
 _ATTN_WS_SLOTS = 4
@@ -465,7 +465,8 @@ def _attn_scratch(device, nbytes):
 
 
 def _attn_split_scratch(device, need, B, S, Hq, Hkv, D, causal):
-    """The dS scratch with room for the parts of split key blocks behind it where a call has them: (scratch or None, bytes)."""
+    """The dS scratch with room for the parts of split key blocks behind it where a call has them: (scratch or None, bytes).  Where the cap or the memory that is free grants the scratch alone,
+    the call's key blocks stay whole: dK and dV are then one sum each instead of a few parts' added, the same fp32 products, one bf16 rounding apart at most, 1e-5 to 1e-4 of their norm (dQ has the same bits)."""
     more = L.load().mi355_attn_bwd_split_bytes(B, S, Hq, Hkv, D, int(causal))
     ws = _attn_scratch(device, need + more) if more else None
     if ws is not None:

@@ -439,7 +439,7 @@ def test_attention_fwd_bwd(K, B, S, Hq, Hkv, D, causal, ragged):
                                                       (2, 200, 4, 2, True, "holes")])
 def test_attention_backward_scratch_form_equals_recompute_form(K, B, S, Hq, Hkv, causal, ragged):
     """mi355_attn_bwd_ws (the dK/dV pass leaves dS in a scratch buffer, dQ = scale * dS K is one product over it) against the form
-    without a workspace (the dQ pass recomputes S and dP).  The two were bit-identical while they shared their arithmetic; since round 3 the
+    without a workspace (the dQ pass recomputes S and dP).  The
     scratch form's dK/dV pass folds the scale into its bf16 K rows and starts its chains from -lse / -delta (one more operand rounding, ~1e-3
     of a score), so they agree to the bf16 level of a gradient, and each is checked against fp64 elsewhere; a scratch buffer that is too small
     is refused."""
