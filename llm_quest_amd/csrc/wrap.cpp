@@ -40,7 +40,7 @@ struct Raised {};   // thrown: a Python exception is set
 
 PyObject *fn_device, *fn_stream, *fn_set_device, *fn_fail;  // current device, raw handle of its stream, what launches that follow run on, raises (name, rc)
 PyObject* kernels;                                          // kernels.py's namespace: its scratch and its switches
-PyObject* dry;                                              // a list: calls are written there instead of made, and tensors may be anywhere (tests)
+thread_local PyObject* dry;                                 // a list: this thread's calls are written there instead of made, and tensors may be anywhere (tests)
 
 struct Slot {
     const char* name;
@@ -1347,7 +1347,7 @@ PyMethodDef methods[] = {
     {"bind", bind, METH_VARARGS, "bind(name, address): where an entry point of the loaded library is"},
     {"setup", setup, METH_VARARGS, "setup(getDevice, getCurrentRawStream, set_device, fail)"},
     {"set_kernels", set_kernels, METH_O, "set_kernels(namespace of kernels.py)"},
-    {"dry", set_dry, METH_O, "dry(list): calls are appended to it as (entry point, arguments) instead of made, on tensors of any device; dry(None) ends that"},
+    {"dry", set_dry, METH_O, "dry(list): this thread's calls are appended to it as (entry point, arguments) instead of made, on tensors of any device; dry(None) ends that"},
     {"names", names, METH_NOARGS, "[(operator, number of arguments)]"},
     {"arguments", arguments, METH_O, "the names of an operator's arguments"},
     {nullptr, nullptr, 0, nullptr}};

@@ -141,6 +141,28 @@ def test_operators_are_what_functions_are_besides_being_called():
     assert Holder.product is K.gemm and inspect.ismethod(h.product) and h.product.__self__ is h and h.product.__func__ is K.gemm
 
 
+def test_a_dry_run_is_one_threads_own():
+    import threading
+
+    calls, seen = [], []
+
+    def other():
+        try:
+            K.gelu_fwd(torch.randn(8).to(B))
+        except Exception as e:  # (no GPU tensor)
+            seen.append(type(e))
+
+    L._wrap.dry(calls)
+    try:
+        t = threading.Thread(target=other)
+        t.start()
+        t.join()
+        K.copy2d(rows(2, 8), rows(2, 8))
+    finally:
+        L._wrap.dry(None)
+    assert seen and [c[0] for c in calls] == ["mi355_copy2d"]
+
+
 def test_arguments_are_named_as_in_python():
     for name, _ in L._wrap.names():
         assert list(inspect.signature(form(name)).parameters) == L._wrap.arguments(name), name
