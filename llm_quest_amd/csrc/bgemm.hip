@@ -61,7 +61,8 @@ __device__ __forceinline__ float ldx(const void* p, int dt, int64_t i) { return 
 
 // A workgroup's matrix (or group) and row tile.  With groups M counts all groups' rows, so most of a group's row tiles are empty, and between the groups' first ones they hold those up: row tiles are
 // then the slowest index (450 fp32 tokens on 2 of 16 experts, 1 024 -> 1 792, 56 rows an expert in 15 tiles of 64: 46 -> 34 us; on 4 of 64 45 -> 33).  Not where groups have several tiles and the
-// weights are more than the caches hold, which every row tile would then read again (3 000 tokens on 16 experts of 2 048 -> 7 168: 643 -> 693 us); nor without groups.
+// weights are more than the caches hold, which every row tile would then read again (3 000 tokens on 16 experts of 2 048 -> 7 168: 643 -> 693 us); nor without groups.  (Of 128 groups of 190 - 400 fp32
+// rows, whose empty tiles are most of the launch either way, it is 2 048 -> 256 913 -> 300 us, 1 024 -> 512 600 -> 352, but 512 -> 1 024 471 -> 516.)
 __device__ __forceinline__ int batch_of(const BgemmArgs& p) { return p.rows_last ? blockIdx.y : blockIdx.z; }
 __device__ __forceinline__ int row_tile_of(const BgemmArgs& p) { return p.rows_last ? blockIdx.z : blockIdx.y; }
 static dim3 tile_grid(const BgemmArgs& p, int64_t cols, int64_t rows, int batch) { return p.rows_last ? dim3((unsigned)cols, (unsigned)batch, (unsigned)rows) : dim3((unsigned)cols, (unsigned)rows, (unsigned)batch); }

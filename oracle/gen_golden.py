@@ -247,7 +247,7 @@ def gen_vlm(out):
     ids = torch.randint(0, 512, (2, 20))
     tm = torch.ones(2, 20, dtype=torch.bool)
     tm[0, 13:] = False
-    # composition harness of SURVEY.md section 8c over the reference's public attributes
+    # composition harness over the reference's public attributes
     h = vit(img, output_hidden_states=True)
     ve = ad(h.to(torch.bfloat16))
     te = llm.emb_dict(ids)
@@ -374,7 +374,7 @@ TINY_Q35_TEXT = dict(
 
 
 def gen_qwen35_text(out):
-    """BASELINE config 5 text stack: per-op vectors + a tiny hybrid model, bf16 and fp32."""
+    """The Qwen3.5 text stack: per-op vectors + a tiny hybrid model, bf16 and fp32."""
     from llm_quest.common.rope import RoPE
     from llm_quest.qwen.qwen3_5.qwen3_5_text_model import Qwen3_5TextModel
     from llm_quest.qwen.qwen3_next.qwen3_next_attention import ZeroCenteredRMSNorm, compute_alpha_factor, gated_delta_rule, l2_norm
@@ -447,7 +447,7 @@ def gen_qwen35_text(out):
 
 
 def gen_qwen35_vlm(out):
-    """BASELINE config 5 at the wrapper level: the reference's ``Qwen3_5VLM.forward``
+    """The Qwen3.5 VLM at the wrapper level: the reference's ``Qwen3_5VLM.forward``
     (qwen3_5_vlm_model.py:178-227) on a tiny model -- fp32 vision tower, bf16 hybrid text stack, two samples with 8 image placeholders each
     (2 frame pairs x 2x2 merged rows), a padding mask -- logits and EVERY parameter gradient; plus the same step with the text stack in fp32
     (the bf16 model's weights upcast: a true weight twin, the floor of the 1.5x rule)."""
@@ -493,7 +493,7 @@ def gen_qwen35_vlm(out):
 
 
 def gen_decode(out):
-    """KV-cache decoding (SURVEY.md section 8 row f4): the reference's tiny Qwen3 (weights of qwen3_tiny.safetensors) driven exactly
+    """KV-cache decoding: the reference's tiny Qwen3 (weights of qwen3_tiny.safetensors) driven exactly
     as generate_loop_kv_cache does -- prefill with a KVCache, then one-token steps with position_ids -- teacher-forced with seeded
     tokens so every step's logits are comparable, plus the greedy loop itself."""
     from safetensors.torch import load_file
@@ -524,7 +524,7 @@ def gen_decode(out):
 
 
 def gen_decode35(out):
-    """Qwen3_5Cache decoding (second half): the reference's tiny hybrid text model (bf16 weights of
+    """Qwen3_5Cache decoding: the reference's tiny hybrid text model (bf16 weights of
     qwen35_text_tiny.safetensors; fp32 twin = the same weights upcast) driven as qwen3_5_generate_text_only.py does -- prefill with
     MRoPE position ids + cache, then teacher-forced one-token steps."""
     from safetensors.torch import load_file
@@ -555,7 +555,7 @@ def gen_decode35(out):
 
 
 def gen_pipeline(out):
-    """Input pipeline (SURVEY.md section 8 row f3): Pillow's bilinear resize -- the third-party arithmetic behind
+    """Input pipeline: Pillow's bilinear resize -- the third-party arithmetic behind
     transforms.Resize in MultimodalDataset (dataset.py:341-349) -- on seeded random RGB images."""
     import numpy as np
     import PIL
@@ -574,7 +574,7 @@ def gen_pipeline(out):
 
 
 def gen_signatures(out):
-    """Names + argument lists of every symbol on the drop-in boundary (SURVEY.md section 8b), read from the reference's source
+    """Names + argument lists of every symbol on the drop-in boundary, read from the reference's source
     with ast (oracle/signatures.py): data only, no source text."""
     import json
 

@@ -1,5 +1,5 @@
 """Model-level CPU restatements, functional over a state_dict.  TEST INFRASTRUCTURE ONLY
-(see oracle/__init__.py).  State-dict key names are the reference's (SURVEY.md section 8b), so the same
+(see oracle/__init__.py).  State-dict key names are the reference's, so the same
 dict loads into the reference modules, into ``llm_quest_amd`` modules and into these functions.
 """
 
@@ -37,7 +37,7 @@ def qwen3_block(sd, pfx, x, cfg, cos, sin, key_mask=None, position_ids=None):
 
 def qwen3_forward(sd, cfg, tokens=None, key_mask=None, position_ids=None, inputs_embeds=None):
     """Qwen3Model.forward (qwen/qwen3/qwen3_model.py:60-94).  ``inputs_embeds`` is the embedded-input entry the
-    composed VLM needs (SURVEY.md section 8c harness: blocks -> final_norm -> tied out_head)."""
+    composed VLM needs (blocks -> final_norm -> tied out_head)."""
     cos, sin = ops.rope_tables(cfg["rope_base"], cfg["head_dim"], cfg["context_length"])
     x = F.embedding(tokens, sd["emb_dict.weight"]) if inputs_embeds is None else inputs_embeds
     for i in range(cfg["n_layers"]):
@@ -111,7 +111,7 @@ def adapter_forward(sd, x):
 
 
 def vlm_forward_loss(vit_sd, vit_cfg, ad_sd, llm_sd, llm_cfg, image, input_ids, text_mask):
-    """Composed early-fusion train-step forward for BASELINE config 4 (SURVEY.md section 8c harness, built from
+    """Composed early-fusion train-step forward (built from
     multimodal/vlm_engine.py:94-128 with Qwen3 in place of GPT-2): frozen ViT hidden states -> adapter (bf16) ->
     cat([vision, tok_emb]) -> Qwen3 blocks with causal | ~key_mask -> final_norm -> tied head -> vlm_loss.
     Returns (loss, logits, fused_embeddings)."""

@@ -1,4 +1,4 @@
-"""CPU restatement of the input pipeline on the step's left edge (SURVEY.md section 8 row f3): the batch contract of
+"""CPU restatement of the input pipeline on the step's left edge: the batch contract of
 ``MultimodalDataset`` (llm_quest/dataset.py:295-383).  TEST INFRASTRUCTURE ONLY (see oracle/__init__.py).
 
 The arithmetic of that path lives in third-party code that is NOT under /root/reference:

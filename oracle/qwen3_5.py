@@ -1,6 +1,6 @@
-"""CPU restatement of the Qwen3.5 multimodal pieces (BASELINE config 5): vision tower, merge adapter, wrapper index ops.
-TEST INFRASTRUCTURE ONLY (see oracle/__init__.py).  The hybrid text stack (gated delta net, gated attention) is not
-restated yet -- DESIGN.md lists it under "next"."""
+"""CPU restatement of the Qwen3.5 multimodal pieces: vision tower, merge adapter, wrapper index ops.
+TEST INFRASTRUCTURE ONLY (see oracle/__init__.py).  The hybrid text stack (gated delta net, gated attention) is in
+oracle/qwen3_5_text.py."""
 
 import numpy as np
 import torch

@@ -1,4 +1,4 @@
-"""CPU restatement of the Qwen3.5 text stack (BASELINE config 5, SURVEY.md section 8 row a24).  TEST INFRASTRUCTURE ONLY
+"""CPU restatement of the Qwen3.5 text stack.  TEST INFRASTRUCTURE ONLY
 (see oracle/__init__.py): functional, state-dict in / tensors out, every function cites the reference lines it follows.
 Pinned by tests/golden/qwen35_text_tiny.safetensors (generated from the reference by oracle/gen_golden.py::gen_qwen35_text).
 """

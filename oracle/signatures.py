@@ -1,13 +1,13 @@
 """Public call signatures of a Python source tree, read with ``ast`` (nothing is imported or executed).
 
 TEST INFRASTRUCTURE ONLY (see oracle/__init__.py).  ``oracle/gen_golden.py`` runs ``collect`` over the reference's modules on
-the hot path (SURVEY.md section 8b) and commits the result as ``tests/golden/signatures.json`` -- names and argument lists,
+the hot path and commits the result as ``tests/golden/signatures.json`` -- names and argument lists,
 data only; ``tests/test_signatures_cpu.py`` runs the same function over ``llm_quest_amd`` and compares.
 """
 
 import ast
 
-# reference modules (relative to the package root) that make up the drop-in boundary of SURVEY.md section 8(b)
+# reference modules (relative to the package root) that make up the drop-in boundary
 MODULES = [
     "common/rope.py", "common/buffers.py", "engine.py", "generate.py", "utils.py", "dataset.py",
     "multimodal/vlm_engine.py", "multimodal/vlm_generation.py",
@@ -20,7 +20,7 @@ MODULES = [
     "gpt/gpt_model.py",
 ]
 
-# symbols of those modules that SURVEY.md section 2 / 8 mark OUT OF SCOPE (not on the hot path): left out of the fixture, with the reason
+# symbols of those modules that are OUT OF SCOPE (not on the hot path): left out of the fixture, with the reason
 OUT_OF_SCOPE = {
     "common/buffers.py": {"GlobalBuffers.get_swa_buffers": "sliding-window attention (Gemma family)", "GlobalBuffers.get_swa_mask": "sliding-window attention"},
     "qwen/qwen3/qwen3_model.py": {"Qwen3MoEModel": "MoE variant"},

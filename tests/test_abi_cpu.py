@@ -62,7 +62,7 @@ def test_host_side_validation_rejects_bad_calls_without_touching_the_gpu():
 
 
 def test_host_side_of_every_entry_point_is_clean_under_address_sanitizer():
-    """SURVEY.md section 5 (sanitizers, CPU build only): the AddressSanitizer build of the library (`make asan`: host code instrumented,
+    """Sanitizers, CPU build only: the AddressSanitizer build of the library (`make asan`: host code instrumented,
     device code untouched) takes degenerate calls of EVERY entry point -- null pointers, zero / negative / huge sizes, odd enums -- in a
     child process with the ASAN runtime preloaded (tools/asan_abi_probe.py).  Each call must return a code; ASAN must report nothing."""
     import glob
@@ -117,8 +117,8 @@ def test_attention_backward_owned_agprs_are_untouched_by_the_compiler(tmp_path):
 
 
 def test_integration_md_stubs_match_the_binding_table():
-    """Every `_lib.<name>.argtypes = [...]` line of INTEGRATION.md (the stubs a reference maintainer would copy) must list exactly the
-    argument types of `_lib.SIGNATURES` -- the doc cannot drift from the header again (round 2: a 16-argument stub of a 17-argument call)."""
+    """Every `_lib.<name>.argtypes = [...]` line of the integration guide (the stubs a reference maintainer would copy) must list exactly the
+    argument types of `_lib.SIGNATURES`: a stub of one argument less reads rubbish."""
     import ctypes
 
     from llm_quest_amd import _lib

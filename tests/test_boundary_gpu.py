@@ -1,4 +1,4 @@
-"""Drop-in boundary entry points that run on their own: ``RoPE.apply`` / ``apply_mrope`` / ``VisionRoPE.apply`` on
+"""Drop-in boundary entry points that run on their own (the reference's public symbols): ``RoPE.apply`` / ``apply_mrope`` / ``VisionRoPE.apply`` on
 device tensors (``mi355_rope_apply``) and the ``forward`` of every Qwen3.5 vision sub-module, against fixtures the reference produced
 (``tests/golden/rope_extra.safetensors``, ``per_op``, ``qwen35_text_tiny``, ``qwen35_vision_tiny``)."""
 

@@ -282,7 +282,7 @@ def test_tied_head_embedding_bucket_is_exchanged_in_two_parts_gloo():
 
 
 def _world8_worker(rank, world, port, out):
-    """The headline step's hand-offs at EIGHT ranks (the 8-rank arithmetic had only ever run with two): 28 block buckets last -> first in groups of
+    """The headline step's hand-offs at EIGHT ranks: 28 block buckets last -> first in groups of
     7, the tied head / embedding bucket in two parts (64 x 512 tokens: the byte rule says split at 8 ranks) and whole (160 x 512: dense), the adapter's bucket and the
     rest in finish_step -- every gradient the 8-rank mean."""
     os.environ.update(MASTER_ADDR="127.0.0.1", MASTER_PORT=str(port), RANK=str(rank), WORLD_SIZE=str(world), LOCAL_RANK=str(rank))
@@ -428,7 +428,7 @@ def test_gemm_window_bounds_the_per_tile_stretch_behind_a_bucket_group(monkeypat
 
 
 def test_gemm_window_counts_only_persistent_eligible_launches_and_sizes_itself(monkeypatch):
-    """a launch the library would NOT put on the persistent kernel (bias, fp32 output, a tile hint ...: ``eligible=False``) does not use the window up; the
+    """A launch the library would NOT put on the persistent kernel (bias, fp32 output, a tile hint ...: ``eligible=False``) does not use the window up; the
     user's own MI355_GEMM_PERSIST_MIN_TILES is the threshold; GradSync.window_for sizes a window from the measured all-reduce and launch times."""
     from llm_quest_amd import ddp
     from llm_quest_amd import kernels as K

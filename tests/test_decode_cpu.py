@@ -1,4 +1,4 @@
-"""KV cache host logic (SURVEY.md section 8 row f4): capacity growth policy and position bookkeeping of utils.KVCache, which are
+"""KV cache host logic: capacity growth policy and position bookkeeping of utils.KVCache, which are
 pure Python and mirror llm_quest/utils.py:409-531."""
 
 import math

@@ -132,7 +132,7 @@ def test_param_arena_views_and_grad_targets():
 
 
 def test_hf_qwen3_checkpoint_import_round_trip(tmp_path, capsys):
-    """HF parameter names -> this package's (SURVEY 8 row f2): a synthetic HF-named checkpoint built from one model loads
+    """HF parameter names -> this package's: a synthetic HF-named checkpoint built from one model loads
     into a second model bit for bit, through a dict and through a .safetensors file; bad shapes / unknown names are reported."""
     from safetensors.torch import save_file
 

@@ -284,7 +284,7 @@ def _oracle_compare(mine, l_mine, oracle_run):
 
 
 def test_full_size_qwen3_text_step_matches_the_cpu_oracle():
-    """BASELINE configs[2] at FULL size against the CPU oracle: Qwen3-0.6B, S = 1024, B = 1, ``global_loss`` on the shifted ids (engine.py:50-72).
+    """The text model at FULL size against the CPU oracle: Qwen3-0.6B, S = 1024, B = 1, ``global_loss`` on the shifted ids (engine.py:50-72).
     The tiny fixtures never reach 16 heads x 28 layers, S = 1024 or V = 151 936; a deterministic but wrong kernel at these shapes would pass the
     property tests below -- not this one.  Picks: first / last block ``w_queries``, a ``lin2``, the tied embedding / head matrix."""
     if not torch.cuda.is_available():
@@ -323,7 +323,7 @@ def test_full_size_qwen3_text_step_matches_the_cpu_oracle():
 
 
 def test_full_width_reduced_depth_qwen35_step_matches_the_cpu_oracle():
-    """BASELINE configs[4] (Qwen3.5-style VLM) at FULL WIDTH and reduced depth against the CPU oracle: emb 1024, GDN 16 x 128 heads, gated attention
+    """The Qwen3.5-style VLM at FULL WIDTH and reduced depth against the CPU oracle: emb 1024, GDN 16 x 128 heads, gated attention
     8 x 256 heads over 2 kv groups, ffn 3584, V = 248 320, 4 text layers (3 GatedDeltaNet + 1 gated attention: one period of the hybrid pattern), a
     2-layer 768-wide vision tower on 8 x 224 x 224 frames, S = 708 = 512 text tokens + 196 merged vision rows, B = 1, MRoPE-I position ids.  The
     oracle -- pinned to the reference's ``Qwen3_5VLM.forward`` by tests/golden/qwen35_vlm_tiny -- runs the same weights twice, text stack in bf16
@@ -383,8 +383,8 @@ def test_full_width_reduced_depth_qwen35_step_matches_the_cpu_oracle():
 
 
 def test_full_size_vit_base_step_matches_the_cpu_oracle():
-    """BASELINE configs[1] at FULL size against the CPU oracle: ViT-Base/16, 224 x 224, B = 2, ``drop_rate`` 0, class head + CE.  The oracle's low
-    precision run is the reference under ``torch.autocast(bf16)`` (SURVEY 9.17: what this path's dtype flow reproduces), its twin plain fp32.
+    """The ViT at FULL size against the CPU oracle: ViT-Base/16, 224 x 224, B = 2, ``drop_rate`` 0, class head + CE.  The oracle's low
+    precision run is the reference under ``torch.autocast(bf16)`` (what this path's dtype flow reproduces), its twin plain fp32.
     Picks: every third block's ``w_keys``, the patch projection, the classifier."""
     if not torch.cuda.is_available():
         pytest.skip("needs an MI355X")
@@ -420,7 +420,7 @@ def test_full_size_vit_base_step_matches_the_cpu_oracle():
 
 
 def test_baseline_size_properties_config2_vit_base():
-    """BASELINE configs[1]: ViT-Base/16 224x224 fwd+bwd at B = 64 (full size): loss ~ ln(100) at init, finite gradients, bit-identical
+    """ViT-Base/16 224x224 fwd+bwd at B = 64 (full size): loss ~ ln(100) at init, finite gradients, bit-identical
     repeat (no atomics anywhere on this path)."""
     import math
 
@@ -450,7 +450,7 @@ def test_baseline_size_properties_config2_vit_base():
 
 
 def test_baseline_size_properties_config3_qwen3_text_s1024():
-    """BASELINE configs[2]: Qwen3-0.6B text-only at S = 1024 (B = 8): loss ~ ln V at init, finite gradients, bit-identical repeat, and a
+    """Qwen3-0.6B text-only at S = 1024 (B = 8): loss ~ ln V at init, finite gradients, bit-identical repeat, and a
     change to the LAST token changes no earlier row of the final hidden states (causality at full depth and length)."""
     import math
 
@@ -483,7 +483,7 @@ def test_baseline_size_properties_config3_qwen3_text_s1024():
 
 
 def test_baseline_size_properties_config5_qwen35_vlm():
-    """BASELINE configs[4]: Qwen3.5-style VLM, 8 frames of 224x224 + 512 text tokens (S = 708), B = 2 at full model size: loss ~ ln V at
+    """Qwen3.5-style VLM, 8 frames of 224x224 + 512 text tokens (S = 708), B = 2 at full model size: loss ~ ln V at
     init, finite gradients on every parameter, bit-identical repeat of loss and gradients."""
     import math
 

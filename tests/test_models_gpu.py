@@ -1,7 +1,7 @@
 """Module-level parity on a real MI355X: the drop-in nn.Modules / engine functions vs fixtures generated from the
 reference (tests/golden) and vs the CPU oracle.
 
-Tolerances follow SURVEY.md section 8c: the scalar loss within 1e-3 relative of the CPU reference; bf16 tensors are judged
+Tolerances: the scalar loss within 1e-3 relative of the CPU reference; bf16 tensors are judged
 against the reference's OWN bf16 noise floor, measured as reference-bf16 vs its fp32 twin ("1.5x rule").
 """
 
@@ -168,14 +168,14 @@ def test_vit_tiny_forward(golden):
     img = t["in.image"].cuda()
     hid = m(img, output_hidden_states=True)
     assert hid.dtype == F32 and hid.shape == t["out.hidden"].shape
-    # bf16 MFMA operands with an fp32 residual stream vs the reference's all-fp32 ViT (autocast-level noise, SURVEY 9.17)
+    # bf16 MFMA operands with an fp32 residual stream vs the reference's all-fp32 ViT (autocast-level noise)
     assert rel_l2(hid, t["out.hidden"]) < 1e-2
     assert rel_l2(m(img), t["out.logits"]) < 2e-2
 
 
 def test_vit_tiny_training_step_matches_reference(golden):
     """BASELINE config 2 on the tiny fixture: ViT fwd + CE + bwd; every parameter gradient vs the fp32 reference.
-    bf16 MFMA operands over fp32 masters (autocast-level noise, SURVEY 9.17), hence the 3e-2 gradient tolerance."""
+    bf16 MFMA operands over fp32 masters (autocast-level noise), hence the 3e-2 gradient tolerance."""
     from llm_quest_amd.engine import _cross_entropy
     from llm_quest_amd.multimodal.vision_transformer.vit_model import ViTModel
 

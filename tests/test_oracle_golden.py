@@ -105,7 +105,7 @@ def test_gqa_module(golden):
 
 
 def test_gqa_upstream_known_answer(golden):
-    """The seeded __main__ demo of qwen3_attention.py:154-185; SURVEY.md section 4 quotes its first output row."""
+    """The seeded __main__ demo of qwen3_attention.py:154-185."""
     t = golden("per_op")
     sd = sub_dict(t, "gqa_toy.sd.")
     cfg = dict(n_heads=6, num_kv_groups=2, head_dim=2)
@@ -241,7 +241,7 @@ def test_qwen35_text_index_and_small_ops(golden):
     t = golden("qwen35_text_tiny")
     for name, sec in {"s11_11_10": [11, 11, 10], "s2_2_2": [2, 2, 2], "s3_3_2": [3, 3, 2]}.items():
         assert np.array_equal(q35t.mrope_axis_of_frequency(sec, sum(sec)), t[f"mrope.axis.{name}"].numpy()), name
-    # the pattern SURVEY.md records for [11, 11, 10]: [T, H, W] x 10, then T, H
+    # the pattern for [11, 11, 10]: [T, H, W] x 10, then T, H
     assert q35t.mrope_axis_of_frequency([11, 11, 10], 32).tolist() == [0, 1, 2] * 10 + [0, 1]
     c, s = q35t.mrope_coeffs(t["mrope.cos"], t["mrope.sin"], t["mrope.pid"], [3, 3, 2])
     q = t["mrope.q"]

@@ -1,4 +1,4 @@
-"""Input pipeline (SURVEY.md section 8 row f3), CPU side: the oracle's restatement of Pillow's resampler against committed Pillow
+"""Input pipeline, CPU side: the oracle's restatement of Pillow's resampler against committed Pillow
 vectors and against Pillow itself, the host-built coefficient tables against the oracle's, and the pad / mask contract."""
 
 import numpy as np

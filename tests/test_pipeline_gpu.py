@@ -1,4 +1,4 @@
-"""Input pipeline (SURVEY.md section 8 row f3) on HIP kernels vs the oracle (pinned to Pillow): resize + ToTensor + Normalize bit-exact,
+"""Input pipeline on HIP kernels vs the oracle (pinned to Pillow): resize + ToTensor + Normalize bit-exact,
 pad / truncate / mask exact, the prefetching batch iterator == per-item results."""
 
 import numpy as np

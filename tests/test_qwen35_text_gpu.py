@@ -1,4 +1,4 @@
-"""BASELINE config 5 text stack on HIP kernels vs the CPU oracle (oracle/qwen3_5_text.py, itself
+"""The Qwen3.5 text stack on HIP kernels vs the CPU oracle (oracle/qwen3_5_text.py, itself
 pinned to fixtures generated from the reference): kernel level first, then layers and the tiny hybrid model.
 Bit-exact: index gathers.  <= 1 bf16 ulp: elementwise ops whose rounding points are reproduced.  Stated relative-L2 tolerances
 elsewhere (bf16 operands, fp32 accumulation in a different order than ATen's)."""

@@ -1,7 +1,7 @@
-"""Drop-in boundary (SURVEY.md section 8b): every public symbol of the reference's hot-path modules exists in ``llm_quest_amd`` under
+"""Drop-in boundary: every public symbol of the reference's hot-path modules exists in ``llm_quest_amd`` under
 the same import path with the same argument list.  ``tests/golden/signatures.json`` was read from the reference's source by
 ``oracle/gen_golden.py::gen_signatures`` (names and argument lists only); here the same ast collector runs over this package.
-The only differences allowed are the trailing keyword extensions listed below (each documented in DESIGN.md section 1)."""
+The only differences allowed are the trailing keyword extensions listed below."""
 
 import json
 import os

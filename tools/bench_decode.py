@@ -1,4 +1,4 @@
-"""Decode throughput of Qwen3-0.6B through the KV cache (SURVEY.md section 8 row f4): prefill P tokens, then N one-token steps.
+"""Decode throughput of Qwen3-0.6B through the KV cache: prefill P tokens, then N one-token steps.
 Bound: HBM -- every step streams all weights once (1.19 GB bf16 incl. the tied 151 936 x 1024 head) plus the cache.
 GPU box only:  python tools/bench_decode.py [--batch 1] [--prompt 512] [--steps 64] [--graph]"""
 import argparse, os, sys, time

@@ -8,8 +8,8 @@
 //     tile, so every LDS-DMA piece and every barrier is amortised over twice the matrix work, and K / V come over the fabric once per pair;
 //   * one wave per SIMD with the whole register file: O^T of both groups (128 registers) and the Q rows (64) are OWNED accumulator registers
 //     (attn_common.h), S^T tiles and packed P live in VGPRs, every MFMA is an asm statement, LDS fragment reads run PD MFMAs ahead in a ring;
-//   * a lone wave can hide about 24 cycles of vector issue behind a 32-cycle MFMA, and costs grow faster than linearly past that (DESIGN.md
-//     section 5, tools/microbench/mfma_gap.hip).  So the softmax is cut to exp2 + row-sum add + half a bf16 pack + half a max3 per score, and
+//   * a lone wave can hide about 24 cycles of vector issue behind a 32-cycle MFMA, and costs grow faster than linearly past that 
+//     (tools/microbench/mfma_gap.hip).  So the softmax is cut to exp2 + row-sum add + half a bf16 pack + half a max3 per score, and
 //     laid out so that the exp2 are spread evenly over the MFMA gaps (two in every other gap):
 //       - the scale log2(e) / sqrt(d) is folded into the Q rows once per block (bf16(q * c): one more rounding of a bf16 operand, far inside
 //         the reference's own noise -- it rounds the scores themselves to bf16, twice);

@@ -1,5 +1,5 @@
 """Chunked (WY / UT-transform) form of the gated delta rule, forward and hand-written backward, in plain torch fp64 -- the algorithm
-a chunked kernel pair would implement (round 3 built the forward on fp32 MFMA: 409 us against the sequential kernel's 363 at B = 8 -- it left the tree in round 6;
+a chunked kernel pair would implement (a first forward on fp32 MFMA took 409 us against the sequential kernel's 363 at B = 8;
 on split-bf16 operands its products would cost a fifth), checked here against the sequential recurrence the reference runs
 (qwen3_next_attention.py:103-159) and its autograd gradients.  CPU only, no package import:  python tools/experimental/gdr_chunk_proto.py
 
