@@ -8,7 +8,7 @@ spawned before this process has touched the GPU -- and relays rank 0's JSON line
 
 A step = vision tower (frozen ViT-B/16, eval) -> ffn adapter -> early-fusion concat -> Qwen3-0.6B decoder on the fused
 709-token sequence -> tied LM head + cross entropy on the 512 text positions -> full backward (adapter + LLM), plus the
-RCCL gradient all-reduce when N > 1.  The optimizer step is NOT part of the metric (SURVEY.md section 8d); gradients are
+RCCL gradient all-reduce when N > 1.  The optimizer step is NOT part of the metric; gradients are
 dropped between steps (zero_grad(set_to_none=True)).  Synthetic seeded inputs, random-init weights, inputs resident in
 HBM before the timed region.  One JSON line on rank 0.
 """
@@ -26,7 +26,7 @@ sys.path.insert(0, ROOT)
 
 N_VISION, N_TEXT, VOCAB = 197, 512, 151_936
 UNITS_PER_SAMPLE = 1 + N_TEXT  # 1 image + 512 text tokens
-ALGO_FLOP_PER_SAMPLE = 2.566e12  # SURVEY.md section 8(d): 35.13 G (frozen ViT fwd) + 3 x (2.17 G adapter + 841.5 G LLM)
+ALGO_FLOP_PER_SAMPLE = 2.566e12  # 35.13 G (frozen ViT fwd) + 3 x (2.17 G adapter + 841.5 G LLM)
 PEAK_BF16_TFLOPS = 2500.0  # MI355X dense bf16 MFMA peak (MI355X_MICROARCH.md)
 CPU_SAMPLES = 8  # size of the bounded CPU-baseline sample (~10-15 s on the box's 16-core quota)
 
@@ -53,7 +53,7 @@ def build_models(device, seed=123):
 
 
 def synthetic_batch(batch, device, seed, ragged=False):
-    """SURVEY 8d, config 4 inputs: randn images, uniform token ids, all-ones text mask; ``ragged``: real lengths ~ U[256, 512], right-padded."""
+    """The headline's inputs: randn images, uniform token ids, all-ones text mask; ``ragged``: real lengths ~ U[256, 512], right-padded."""
     g = torch.Generator().manual_seed(seed)
     img = torch.randn(batch, 3, 224, 224, generator=g)
     ids = torch.randint(0, VOCAB, (batch, N_TEXT), generator=g)
@@ -276,7 +276,7 @@ def launch_ranks(n):
 
 
 # ------------------------------------------------------------------------------------------------ the other BASELINE configurations
-# ``--config 2 | 3 | 5`` print the same JSON schema for BASELINE.json's configs[1], configs[2] and configs[4] (inputs, units,
+# ``--config 2 | 3 | 5`` print the same JSON schema for the three other workloads (inputs, units,
 # algorithmic FLOP per sample).  They are parity-test configurations of the same kernels, not the headline: the default (``--config 4``) is
 # untouched by them.  No counter files are kept for them, so ``roofline.traffic`` is null.
 OTHER_CONFIGS = {
@@ -294,7 +294,7 @@ OTHER_CONFIGS = {
 
 
 def _other_config_step(cfg_id, batch, device, rank):
-    """Builds the model and the synthetic batch of configs 2 / 3 / 5 (seeded as SURVEY 8d says) and returns (step_fn, sync, state_for_cpu)."""
+    """Builds the model and the synthetic batch of configs 2 / 3 / 5 (seeded) and returns (step_fn, sync, state_for_cpu)."""
     from llm_quest_amd import ddp
 
     torch.manual_seed(123)
@@ -303,7 +303,7 @@ def _other_config_step(cfg_id, batch, device, rank):
         from llm_quest_amd.engine import _cross_entropy
         from llm_quest_amd.multimodal.vision_transformer.vit_model import ViTModel
 
-        cfg = dict(VIT_BASE_CONFIG, drop_rate=0.0)  # the parity setting; drop_rate 0.1 (as configured upstream) costs 12-13 % (DESIGN.md section 5)
+        cfg = dict(VIT_BASE_CONFIG, drop_rate=0.0)  # the parity setting; drop_rate 0.1 (as configured upstream) costs 12-13 %
         with torch.device(device):
             model = ViTModel(cfg).train()
         g = torch.Generator().manual_seed(123 + rank)
@@ -523,7 +523,7 @@ def main():
     ap.add_argument("--gpus", type=int, default=1)
     ap.add_argument("--steps", type=int, default=10)
     ap.add_argument("--warmup", type=int, default=3)
-    ap.add_argument("--config", type=int, choices=[2, 3, 4, 5], default=4, help="BASELINE.json configuration (1-based, as SURVEY.md numbers them): 4 = the headline VLM early-fusion step "
+    ap.add_argument("--config", type=int, choices=[2, 3, 4, 5], default=4, help="which workload: 4 = the headline VLM early-fusion step "
                     "(default; everything below describes it), 2 = ViT-B/16, 3 = Qwen3-0.6B text-only at S = 1024, 5 = Qwen3.5-style VLM -- the same JSON schema for each")
     ap.add_argument("--batch", type=int, default=None, help="per-GPU micro-batch (samples); default 160 for the headline (--config 2 / 3 / 5: 332 / 64 / 32).  Headline: 160 x 709 tokens keep 165 GiB of the 288 GB of HBM live; same-box pairs: 64 -> 34.2 / 34.1 %%, "
                     "128 -> +1.4 %%, 160 -> 35.0 / 34.9 %%, 192 -> level with 160 (202 GiB).  More rounds of tiles per launch amortise every launch's fill and tail.  (92 -- every "
@@ -657,7 +657,7 @@ def main():
         elapsed = float(t)
     loss_gpu = float(loss.detach())
 
-    # The metric is forward + backward ("optimizer step excluded (state it)").  So that nothing of a real
+    # The metric is forward + backward, the optimizer step excluded.  So that nothing of a real
     # training step is left unmeasured, the same K steps are timed again WITH the optimizer: global-norm clip 1.0 + AdamW on the
     # parameter arenas (llm_quest_amd/optim.py::ArenaAdamW), reported beside `value`, never instead of it.
     train_step = None
@@ -691,8 +691,8 @@ def main():
         train_step = {"what": "the same steps including the optimizer: global-norm clip 1.0 + AdamW (ArenaAdamW, one fused launch per parameter arena)",
                       "ms_per_step": round(el2 / args.steps * 1e3, 3), "value": round(world * args.batch * UNITS_PER_SAMPLE * args.steps / el2, 1), "unit": "img+tok/s"}
 
-    # The reference's VLM loop runs the frozen tower in fp32 (vlm_engine.py:99-104, outside autocast); the package's default tower multiplies bf16 operands (DESIGN.md
-    # section 4).  So that the driver's line also carries the step at the reference's precision, the same K steps are timed once more with
+    # The reference's VLM loop runs the frozen tower in fp32 (vlm_engine.py:99-104, outside autocast); the package's default tower multiplies bf16
+    # operands.  So that the line also carries the step at the reference's precision, the same K steps are timed once more with
     # vit.tower_precision = "fp32" (split-bf16 GEMMs + exact-fp32 attention: hidden states within 1e-4 of the oracle's), reported beside `value`.
     fp32_tower = None
     if world == 1 and tower != "fp32" and args.fp32_tower_leg == "on":
@@ -785,7 +785,7 @@ def main():
             except Exception as exc:  # the baseline is a reported number, never the measured path
                 line["cpu_baseline"] = {"value": None, "unit": "img+tok/s", "cores": os.cpu_count(), "kind": "port", "sample": f"failed: {exc!r}"}
         if world == 1 and args.other_configs == "on" and not args.batch_given and not args.ragged:
-            # BASELINE configs 2, 3 and 5 beside the headline (a few steps each, own processes: this one first gives its memory back), so that the driver's record
+            # the other workloads beside the headline (a few steps each, own processes: this one first gives its memory back), so that one record
             # carries them too; `python bench.py --config N` prints each one's full line
             vit = ad = llm = img = ids = mask = ahead = sync = loss = None  # (the closures above see the same cells)
             if args.optimizer == "on":

@@ -3,7 +3,7 @@ flags those files are built with (the ``CXXFLAGS`` / ``FLAGS_<file>`` lines of c
 unrelated source to ``SRCS`` must not invalidate the counters of kernels that did not change).
 
 Counter files under ``profiles/`` are taken in separate ``rocprofv3 --pmc`` passes and committed; each carries the fingerprint of the
-sources it was measured on, written ON THE GPU BOX AT COLLECTION TIME (``tools/collect_evidence.sh`` -> ``stamp.json`` beside the raw
+sources it was measured on, written ON THE GPU MACHINE AT COLLECTION TIME (``tools/collect_evidence.sh`` -> ``stamp.json`` beside the raw
 counters, with the sha-256 of the library that was loaded); the aggregators copy that stamp, they never recompute it.  ``bench.py`` prints a
 counter-derived figure only when the stamp equals the fingerprint of the sources it runs, so a kernel edit can never leave a stale
 ``traffic`` in the bench line; ``tests/test_zz_evidence_cpu.py`` fails while the committed stamp of ``EVIDENCE_ROUND`` is stale at HEAD."""
@@ -64,7 +64,7 @@ def collection_stamp(evidence_dir):
         return json.load(f)
 
 
-if __name__ == "__main__":  # python -m llm_quest_amd.fingerprint <git sha> <batch>  (collection time, on the GPU box)
+if __name__ == "__main__":  # python -m llm_quest_amd.fingerprint <git sha> <batch>  (collection time, on the GPU machine)
     import sys
 
     print(json.dumps({"kernel_sources_sha": kernel_sources_sha(), "all_sources_sha": all_sources_sha(), "library_sha": library_sha(), "git_sha": sys.argv[1] if len(sys.argv) > 1 else "unknown",

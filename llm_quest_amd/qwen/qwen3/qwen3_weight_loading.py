@@ -1,7 +1,7 @@
 """Hugging Face -> this package's parameter names for Qwen3 (API of
 ``llm_quest/qwen/qwen3/qwen3_weight_loading.py``; the shared helpers live in ``llm_quest_amd/utils.py`` as upstream's do in ``utils.py``).
 
-There is no network on the build / GPU boxes, so the download step is replaced by a local source: a dict of tensors or a
+Nothing is downloaded: the download step is replaced by a local source: a dict of tensors or a
 ``.safetensors`` file / directory of shards that the caller already has.  Name mapping, shape checks, weight tying and the
 loading report behave as upstream; the loaded parameters land in the model's arenas (``load_state_dict`` copies into the
 existing views, so fused QKV / gate-up GEMMs see them without any re-packing).

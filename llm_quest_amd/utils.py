@@ -315,7 +315,7 @@ class SlotStateCache:
 
 
 # ----------------------------------------------------------------------------------------------- checkpoint import (row f2)
-# API of the "WEIGHTS LOADING" helpers of llm_quest/utils.py:921-1035.  The build / GPU boxes have no network, so
+# API of the "WEIGHTS LOADING" helpers of llm_quest/utils.py:921-1035.  Nothing is downloaded:
 # ``download_hf_weights`` resolves its argument against the local filesystem (a .safetensors file, a directory of shards with
 # or without ``model.safetensors.index.json``) instead of the hub; everything downstream of it behaves as upstream.
 def read_local_checkpoint(source):

@@ -4,7 +4,7 @@ TEST INFRASTRUCTURE ONLY (see oracle/__init__.py).  Run from the repo root:
 
     PYTHONDONTWRITEBYTECODE=1 python oracle/gen_golden.py [--ref /root/reference] [--out tests/golden]
 
-It imports the reference package (never copied into this repo, never present on the GPU box), builds seeded
+It imports the reference package (never copied into this repo, never present on the GPU machine), builds seeded
 tiny models / per-op cases, and stores inputs, state_dicts, outputs and gradients as ``*.safetensors`` (tensor
 data only).  ``torch.__version__`` and the thread count are recorded in each file's metadata.
 """

@@ -1168,7 +1168,7 @@ def test_persistent_nt_kernel_equals_the_per_tile_kernel_bit_for_bit(M, N, K_, m
 
 @pytest.mark.parametrize("M,N,K_", [(709 * 5 + 3, 1024, 2048), (2600, 4096, 512), (4099, 264, 384), (513, 776, 2048), (300, 256, 320), (2049, 1288, 640), (70000, 1536, 128)])
 def test_weight_stationary_walk_equals_the_per_tile_kernel_bit_for_bit(M, N, K_, monkeypatch):
-    """Round 6: the persistent NT kernel's weight-stationary XCD walk (tile hint 7 with ablation bit 3; the library's own choice by shape, MI355_GEMM_WALK) changes only
+    """The persistent NT kernel's weight-stationary XCD walk (tile hint 7 with ablation bit 3; the library's own choice by shape, MI355_GEMM_WALK) changes only
     WHICH workgroup computes a tile and when: every epilogue gives the per-tile kernel's bits on ragged M, N that is no multiple of the tile or of a column group (empty
     tiles are walked as zero work), fewer pairs than row streams, more tiles than CUs.  Then the same through the automatic choice with the walk forced on / off."""
     from llm_quest_amd import _lib as L
@@ -1198,7 +1198,7 @@ def test_weight_stationary_walk_equals_the_per_tile_kernel_bit_for_bit(M, N, K_,
 
 @pytest.mark.parametrize("M,N,K_", [(709 * 5 + 3, 1024, 1024), (4099, 264, 384), (513, 776, 2048), (300, 256, 320), (5000, 3072, 1024)])
 def test_ping_pong_nt_kernel_is_exact_on_exact_products_and_within_fp32_noise_otherwise(M, N, K_):
-    """Round 6, tile hint 8 (gemm_nt_pp_kernel; opt-in, not the library's choice): the two wave groups run a write-out apart on one stream, so a tile's K-tiles are summed in a
+    """Tile hint 8 (gemm_nt_pp_kernel; opt-in, not the library's choice): the two wave groups run a write-out apart on one stream, so a tile's K-tiles are summed in a
     ROTATED order.  On small-integer operands every product and partial sum is exact: the same bits as tile 2 for every epilogue.  On random operands the fp32 sums differ
     in their last bits: a bf16 output may move by one unit in the last place where a sum sits on a rounding boundary (< 0.1 % of the elements), never more."""
     from llm_quest_amd import _lib as L

@@ -81,7 +81,7 @@ def _rank(rank, world, port, q):
 
 def test_two_rccl_ranks_equal_the_single_process_global_batch(golden):
     if not torch.cuda.is_available() or torch.cuda.device_count() < 2:
-        pytest.skip("needs two MI355X (the driver's 8-GPU node); one-GPU boxes cover the protocol with gloo + a one-rank RCCL group")
+        pytest.skip("needs two MI355X ; one-GPU machines cover the protocol with gloo + a one-rank RCCL group")
     import torch.multiprocessing as mp
 
     from llm_quest_amd.multimodal.vlm_engine import vlm_step_loss
@@ -120,7 +120,7 @@ def test_bench_refuses_more_ranks_than_gpus():
 
 @pytest.mark.timeout(900)
 def test_bench_two_rank_rehearsal_runs_the_whole_n_gt_1_path_on_one_gpu():
-    """``MI355_DDP_REHEARSAL=1 python bench.py --gpus 2`` as a fresh child process on a one-GPU box: the bench starts its own two ranks
+    """``MI355_DDP_REHEARSAL=1 python bench.py --gpus 2`` as a fresh child process on a one-GPU machine: the bench starts its own two ranks
     (torch.distributed.run), they share the GPU and exchange over gloo -- rank start-up, parameter broadcast, every block bucket on the
     communication stream, the tied head / embedding bucket (dense or in two parts, by bytes), barriers, max-over-ranks timing and the ONE JSON
     line all execute; only RCCL itself does not.  The line must say it is a rehearsal, and rank 0's loss must equal the one-rank run's

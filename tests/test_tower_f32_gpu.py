@@ -66,7 +66,7 @@ def test_split_operand_gemm_is_fp32_grade(K, M, N, Kd, gelu):
 
 @pytest.mark.parametrize("rows,width", [(197 * 3 + 1, 768), (130, 64), (65, 3072)])
 def test_producers_write_the_split_operand_themselves_bit_for_bit(K, rows, width):
-    """Round 6: LayerNorm and the Linear (+ GELU) epilogue leave their fp32 result as [hi | lo | hi] directly (MI355_DT_SPLIT3): the same bits as the fp32 output
+    """LayerNorm and the Linear (+ GELU) epilogue leave their fp32 result as [hi | lo | hi] directly (MI355_DT_SPLIT3): the same bits as the fp32 output
     followed by mi355_split3_bf16, without the fp32 round trip."""
     from llm_quest_amd import _lib as L
 

@@ -1,9 +1,9 @@
 """The committed counter evidence must belong to the kernels at HEAD (runs last in the CPU suite: the file name sorts behind every other test).
 
 ``bench.py`` prints ``roofline.traffic`` only when ``profiles/<round>_pmc_tcc_step.json`` carries the fingerprint of the kernel sources it runs
-(llm_quest_amd/fingerprint.py).  Round 3 lost that field in the driver's record because a commit after the last collection changed the
-fingerprint; this test turns the same situation into a red suite: after the round's last kernel-affecting edit, re-run
-``tools/collect_evidence.sh`` on the GPU box and ``tools/aggregate_evidence.sh`` here, and commit the new profiles."""
+(llm_quest_amd/fingerprint.py).  A commit behind the last collection
+changes the fingerprint, and the field is gone; this test turns that into a red suite: after the last kernel-affecting edit, re-run
+``tools/collect_evidence.sh`` on the GPU machine and ``tools/aggregate_evidence.sh`` here, and commit the new profiles."""
 
 import json
 import os
@@ -29,7 +29,7 @@ def test_committed_counter_files_were_measured_on_the_kernel_sources_at_head():
     stamp = _load("stamp.json")
     assert stamp["kernel_sources_sha"] == head, (
         f"profiles/{F.EVIDENCE_ROUND}_stamp.json was taken on kernel sources {stamp['kernel_sources_sha']}, HEAD has {head}: re-collect the evidence "
-        "(tools/collect_evidence.sh on the GPU box, tools/aggregate_evidence.sh here) as the LAST kernel-affecting act of the round")
+        "(tools/collect_evidence.sh on the GPU machine, tools/aggregate_evidence.sh here) as the LAST kernel-affecting act")
     for name in ("pmc_tcc_step.json", "pmc_tcc_gemm.json", "pmc_sq_counters.json"):
         d = _load(name)
         assert d["kernel_sources_sha"] == head, f"profiles/{F.EVIDENCE_ROUND}_{name} is stale ({d['kernel_sources_sha']} != {head})"

@@ -1,4 +1,4 @@
-"""A/B of the attention backward with and without the dS scratch (kernels._ATTN_DS_SPILL) at the headline shape.  GPU box only."""
+"""A/B of the attention backward with and without the dS scratch (kernels._ATTN_DS_SPILL) at the headline shape.  GPU only."""
 import os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

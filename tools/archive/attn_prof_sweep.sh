@@ -1,5 +1,5 @@
 #!/bin/bash
-# In-kernel stamps of the dK/dV pass under several profiling builds (GPU box only; the library it leaves behind is a profiling build).
+# In-kernel stamps of the dK/dV pass under several profiling builds (GPU only; the library it leaves behind is a profiling build).
 #   bash tools/attn_prof_sweep.sh 16 48 80 144
 set -e
 R=${GRAFT_REPO_ROOT:-$(cd "$(dirname "$0")/.." && pwd)}

@@ -1,7 +1,7 @@
 """Step time of BASELINE configs[4] (Qwen3.5-style multimodal: Qwen3-ViT 3-D patches on 8 x 224 x 224 frames + hybrid GDN / gated
 attention text stack, S = 708 = 512 text tokens + 196 merged vision rows), forward + loss + backward on ONE GPU, plus a per-kernel
 HIP-event breakdown of one GDN layer's recurrence kernels.  A parity-test configuration, not the bench line.
-GPU box only:  python tools/bench_config5.py [--batch 8] [--steps 5]
+GPU only:  python tools/bench_config5.py [--batch 8] [--steps 5]
 8 GPUs (BASELINE's DDP form):  python -m torch.distributed.run --nnodes=1 --nproc-per-node 8 --master-addr 127.0.0.1 tools/bench_config5.py"""
 import argparse, os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

@@ -1,7 +1,7 @@
 """Step times of the two other single-GPU BASELINE configurations (parity-test cases, not bench lines):
   configs[1]  ViT-Base/16 224x224 forward+backward (classification loss), bf16 MFMA operands over fp32 masters
   configs[2]  Qwen3-0.6B text-only, seq 1024, bf16 forward+backward
-GPU box only:  python tools/bench_configs.py [--vit-batch 64] [--llm-batch 8]"""
+GPU only:  python tools/bench_configs.py [--vit-batch 64] [--llm-batch 8]"""
 import argparse, os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

@@ -1,4 +1,4 @@
-# Tile-walk experiment (GPU box): memory-side traffic and duration of the gate-up forward GEMM under each super-group height.
+# Tile-walk experiment (GPU): memory-side traffic and duration of the gate-up forward GEMM under each super-group height.
 #   bash tools/collect_walk.sh   -> gpurun_out/walk/{g3,g2,g4,g6,g8,g16}_{fetch,write}
 set -e
 cd /tmp && export TMPDIR=/tmp

@@ -1,4 +1,4 @@
-"""Ablation switches of the alternating-group GEMM loop on one full-occupancy shape per form (GPU box only)."""
+"""Ablation switches of the alternating-group GEMM loop on one full-occupancy shape per form (GPU only)."""
 import sys, os
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

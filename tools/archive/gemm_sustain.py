@@ -1,6 +1,6 @@
 """Burst vs sustained throughput of the gate-up forward GEMM (45376 x 6144 x 1024, NT), random vs zero operands: is the step limited by clocks
 (ramp-up from idle, power give-back on real data)?  Measured: 5 launches 794, 50: 862, 500: 932, 3000: 941 TFLOP/s (tile 2, random data), 973 on zeros --
-short isolated sweeps UNDER-state the kernels (clock ramp), sustained random data costs 3.4 % against zeros.  GPU box only: python tools/gemm_sustain.py"""
+short isolated sweeps UNDER-state the kernels (clock ramp), sustained random data costs 3.4 % against zeros.  GPU only: python tools/gemm_sustain.py"""
 import sys, os, torch, time
 sys.path.insert(0, os.environ.get("GRAFT_REPO_ROOT", "/root/repo"))
 from llm_quest_amd import _lib as L, kernels as K

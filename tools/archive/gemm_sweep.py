@@ -1,4 +1,4 @@
-"""Measure every GEMM tile configuration on the shapes of the VLM step (HIP events, random data).  GPU box only:
+"""Measure every GEMM tile configuration on the shapes of the VLM step (HIP events, random data).  GPU only:
     python tools/gemm_sweep.py [--batch 32]"""
 import argparse, sys, os
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

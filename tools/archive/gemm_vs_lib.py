@@ -1,6 +1,6 @@
 """This package's GEMM kernel vs the vendor library (torch.matmul -> hipBLASLt / rocBLAS) on the training step's own shapes, all three forms,
 sustained (200 back-to-back launches on random data, after a warm-up burst).  A yardstick for the roofline fraction, not a dependency: the
-product path never calls the library.  GPU box only: python tools/gemm_vs_lib.py"""
+product path never calls the library.  GPU only: python tools/gemm_vs_lib.py"""
 import os
 import sys
 import time

@@ -1,4 +1,4 @@
-"""Forward attention time at the headline shape (and the ViT shape).  GPU box only."""
+"""Forward attention time at the headline shape (and the ViT shape).  GPU only."""
 import os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

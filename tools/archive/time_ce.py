@@ -1,4 +1,4 @@
-"""Cross-entropy pass at the headline shape (32 832 rows x 151 936, loss + in-place gradient).  MI355_CE_ROW_IN_REGISTERS=0 selects the two-read kernel.  GPU box only."""
+"""Cross-entropy pass at the headline shape (32 832 rows x 151 936, loss + in-place gradient).  MI355_CE_ROW_IN_REGISTERS=0 selects the two-read kernel.  GPU only."""
 import os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

@@ -1,6 +1,6 @@
 """The NT projections of the step at batch 160 on the default tile, isolated (plain, SwiGLU-forward, SwiGLU-backward, residual, delta epilogues).  Under a
 -DGEMM_EPI_ABL=1 build (tools/build_variant.sh epi1 gemm_p2 ...) the write-out is cut away: the difference is what prologue-free overlap could at most buy.
-GPU box only."""
+GPU only."""
 import sys, os, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd import _lib as L, kernels as K

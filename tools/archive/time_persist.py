@@ -1,5 +1,5 @@
 """The persistent NT kernel (tile hint 7) against the per-tile kernel (hint 2): bit-identity on ragged and step shapes for every epilogue it carries (plain, residual,
-SwiGLU forward, SwiGLU backward), then time on the step's NT shapes.  GPU box only."""
+SwiGLU forward, SwiGLU backward), then time on the step's NT shapes.  GPU only."""
 import sys, os, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd import _lib as L, kernels as K

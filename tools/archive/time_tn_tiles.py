@@ -1,4 +1,4 @@
-"""Weight-gradient (TN) GEMM shapes of the step per tile configuration, sustained.  GPU box only."""
+"""Weight-gradient (TN) GEMM shapes of the step per tile configuration, sustained.  GPU only."""
 import sys, os, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd import _lib as L, kernels as K

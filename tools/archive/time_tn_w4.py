@@ -1,5 +1,5 @@
 """Weight-gradient (TN) GEMMs of the step at batch 160 (K = 113 440 tokens): the 8-wave alternating loop (tile 3, the default) against the 4-wave 128x128-per-wave
-loop (tile 5) -- single launches, the grouped launch of a block's four weight gradients, and the LM head's.  Results must be bit-identical.  GPU box only."""
+loop (tile 5) -- single launches, the grouped launch of a block's four weight gradients, and the LM head's.  Results must be bit-identical.  GPU only."""
 import sys, os, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd import _lib as L, kernels as K

@@ -1,4 +1,4 @@
-"""Frozen ViT-B/16 forward (the tower of the headline step: B = 64, eval, no grad), per NT tile choice.  GPU box only."""
+"""Frozen ViT-B/16 forward (the tower of the headline step: B = 64, eval, no grad), per NT tile choice.  GPU only."""
 import os, sys
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

@@ -1,4 +1,4 @@
-"""The block's grouped weight-gradient launch and the LM head's weight gradient (TN, tile 5), isolated; correctness against an fp32 reference on a slice.  GPU box only."""
+"""The block's grouped weight-gradient launch and the LM head's weight gradient (TN, tile 5), isolated; correctness against an fp32 reference on a slice.  GPU only."""
 import sys, os, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd import _lib as L, kernels as K

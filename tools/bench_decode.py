@@ -1,6 +1,6 @@
 """Decode throughput of Qwen3-0.6B through the KV cache: prefill P tokens, then N one-token steps.
 Bound: HBM -- every step streams all weights once (1.19 GB bf16 incl. the tied 151 936 x 1024 head) plus the cache.
-GPU box only:  python tools/bench_decode.py [--batch 1] [--prompt 512] [--steps 64] [--graph]"""
+GPU only:  python tools/bench_decode.py [--batch 1] [--prompt 512] [--steps 64] [--graph]"""
 import argparse, os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

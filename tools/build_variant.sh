@@ -1,5 +1,5 @@
 #!/bin/bash
-# Profiling builds: one copy of libmi355vlm.so with extra -D flags on ONE source, kept under build_variants/ (git-ignored, travels to the GPU box).
+# Profiling builds: one copy of libmi355vlm.so with extra -D flags on ONE source, kept under build_variants/ (git-ignored, travels with the tree).
 #   bash tools/build_variant.sh <tag> <source stem: attention | gemm_p2 | ...> "<extra flags>"
 # Use on the box through MI355_LIB_PATH=build_variants/libmi355vlm_<tag>.so (llm_quest_amd/_lib.py).
 set -e

@@ -1,4 +1,4 @@
-# Evidence collection (GPU box, from the repo root):   ROUND=head GIT_SHA=<sha> BATCH=160 bash tools/collect_evidence.sh
+# Evidence collection (GPU machine, from the repo root):   ROUND=head GIT_SHA=<sha> BATCH=160 bash tools/collect_evidence.sh
 # Writes raw rocprofv3 output under gpurun_out/${ROUND}ev/ and a stamp (kernel-source fingerprint, sha-256 of the loaded library, git sha, batch)
 # taken HERE, at collection time; tools/aggregate_evidence.sh turns it into profiles/${ROUND}_* in the container and copies the stamp.
 set -e

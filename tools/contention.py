@@ -1,6 +1,6 @@
 """What a few busy CUs cost a GEMM launch: the per-tile kernel (hint 2) and the persistent kernel (hint 7, fixed share per workgroup) timed alone and beside an "occupier" on a second
 stream that holds ~N CUs for the whole measurement (a 128x128-tile GEMM with few tiles and a very long K: two workgroups per CU, nothing else fits beside them).  This is the
-situation of a backward whose bucket all-reduces run beside its GEMMs (RCCL: one workgroup = one CU per channel).  GPU box only."""
+situation of a backward whose bucket all-reduces run beside its GEMMs (RCCL: one workgroup = one CU per channel).  GPU only."""
 import sys, os, torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd import _lib as L, kernels as K

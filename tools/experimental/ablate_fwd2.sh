@@ -1,5 +1,5 @@
 #!/bin/bash
-# Timing-only builds of the second-generation attention forward (GPU box only; results are wrong by construction): which part of a tile costs what.
+# Timing-only builds of the second-generation attention forward (GPU only; results are wrong by construction): which part of a tile costs what.
 #   bash tools/ablate_fwd2.sh 0 1 2 3 4 8 12 15
 set -e
 R=${GRAFT_REPO_ROOT:-$(cd "$(dirname "$0")/.." && pwd)}

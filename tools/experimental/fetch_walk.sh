@@ -1,5 +1,5 @@
 #!/bin/bash
-# FETCH_SIZE of the persistent NT kernel with (hint 7 + 2048) and without (hint 7) the weight-stationary walk, per shape (GPU box, repo root).
+# FETCH_SIZE of the persistent NT kernel with (hint 7 + 2048) and without (hint 7) the weight-stationary walk, per shape (GPU machine, repo root).
 set -e
 cd /tmp && export TMPDIR=/tmp
 R=$GRAFT_REPO_ROOT; O=$R/gpurun_out/fetch_walk; rm -rf $O; mkdir -p $O

@@ -1,5 +1,5 @@
 """Ablation switches of the per-tile NT kernel (tile 2: bit 0 = no DMA after the first K-tile, bit 1 = no fragment reads, bit 2 = no barrier) on the step's QKV shape:
-what the main loop would run at without its memory side, its LDS side, its barriers.  GPU box only."""
+what the main loop would run at without its memory side, its LDS side, its barriers.  GPU only."""
 import sys, os
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch

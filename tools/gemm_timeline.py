@@ -1,5 +1,5 @@
 """Per-workgroup wall-clock timeline of one NT GEMM launch (profiling build -DGEMM_TL=1 of the tile's part, tools/build_variant.sh tl gemm_p2 "-DGEMM_TL=1",
-MI355_LIB_PATH=build_variants/libmi355vlm_tl.so): where a CU's time goes between the MFMAs of one tile and the MFMAs of the next.  GPU box only.
+MI355_LIB_PATH=build_variants/libmi355vlm_tl.so): where a CU's time goes between the MFMAs of one tile and the MFMAs of the next.  GPU only.
 Stamps (100 MHz): 0 entry, 1 first K-tile landed, 2 main loop done, 3 barrier in front of the write-out, 4 write-out issued, 5 stores retired."""
 import sys, os, ctypes
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

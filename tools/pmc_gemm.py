@@ -24,7 +24,7 @@ def avg(d, counter):
     return sum(vals) / len(vals), sum(durs) / len(durs)
 
 
-stamp = collection_stamp(sys.argv[2])  # written on the GPU box when the counters were collected
+stamp = collection_stamp(sys.argv[2])  # written on the GPU machine when the counters were collected
 out = {"kernel_sources_sha": stamp["kernel_sources_sha"], "library_sha": stamp["library_sha"], "git_sha": stamp["git_sha"],
        "note": __doc__.strip().split("\n", 2)[2], "kernels": {}}
 for spec in sys.argv[3:]:

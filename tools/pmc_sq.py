@@ -28,7 +28,7 @@ for d in dirs:
             t[1] += float(r["End_Timestamp"]) - float(r["Start_Timestamp"])
 sys.path.insert(0, __import__("os").path.dirname(__import__("os").path.dirname(__import__("os").path.abspath(__file__))))
 from llm_quest_amd.fingerprint import collection_stamp
-stamp = collection_stamp(coll)  # written on the GPU box when the counters were collected
+stamp = collection_stamp(coll)  # written on the GPU machine when the counters were collected
 sha = stamp["git_sha"]
 res = {"label": label, "git_sha": sha, "note": __doc__.split("\n\n")[0].split("\n", 1)[1] if False else "per-dispatch averages; see tools/pmc_sq.py for units", "kernels": {}}
 for k, cs in agg.items():

@@ -37,7 +37,7 @@ for name in set(fetch) | set(write):
     rows.append({"kernel": short(name), "launches_per_step": per_step, "fetch_bytes": int(fb), "write_bytes": int(wb)})
 rows.sort(key=lambda r: -(r["fetch_bytes"] + r["write_bytes"]))
 tot_f, tot_w = sum(r["fetch_bytes"] for r in rows), sum(r["write_bytes"] for r in rows)
-stamp = collection_stamp(sys.argv[5])  # written on the GPU box when the counters were collected
+stamp = collection_stamp(sys.argv[5])  # written on the GPU machine when the counters were collected
 config = sys.argv[6] if len(sys.argv) > 6 else None  # "config2" / "config3" / "config5": `bench.py --config N` at its default batch (no optimizer re-run: warm-up + timed steps only)
 out = {
     "kernel_sources_sha": stamp["kernel_sources_sha"], "all_sources_sha": stamp.get("all_sources_sha"), "library_sha": stamp["library_sha"], "git_sha": stamp["git_sha"],

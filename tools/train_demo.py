@@ -1,7 +1,7 @@
 """Full-size end-to-end check of the WHOLE train step (BASELINE configs[3] models, per-GPU batch 16): the reference's loop
 `vlm_training_loop_simple` (forward, loss, backward, global-norm clip 1.0, optimizer step) on the HIP kernels with ArenaAdamW,
 a fixed synthetic batch repeated, loss printed per epoch: it has to fall from ln(V) = 11.93 as the model memorises the batch.
-GPU box only:  python tools/train_demo.py [--steps 30] [--batch 16]"""
+GPU only:  python tools/train_demo.py [--steps 30] [--batch 16]"""
 import argparse, os, sys, time
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 import torch
