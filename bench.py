@@ -169,7 +169,7 @@ def pmc_step_traffic():
 
 
 def dominant_kernel_rate(batch, device):
-    """HIP-event timing of the step's dominant kernel class (gemm_nt_persist_kernel for the NT forms, gemm_bf16_kernel for TN) on its largest shapes, on the stream the
+    """HIP-event timing of the step's dominant kernel class (gemm_quad_kernel for the NT forms, gemm_quad_grouped_kernel for TN) on its largest shapes, on the stream the
     kernels are launched on (torch's current stream)."""
     from llm_quest_amd import _lib as L
     from llm_quest_amd import kernels as K
@@ -760,7 +760,7 @@ def main():
                 "what": "v_mfma_f32_32x32x16_bf16 on every SIMD, random bf16 operands in registers, no memory traffic, measured on this board right after the timed steps: on random data the "
                         "board's power cap holds the pipe itself below the 2 500 TFLOP/s of `peak` (DESIGN.md section 5)"}
         if world == 1:
-            line["roofline"]["dominant_kernel"] = {"name": "gemm_nt_persist_kernel / gemm_grouped_kernel (NT projections on the persistent form of tile 2; the block's weight gradients as one grouped launch on tile 5)", "hip_event_timing": dominant_kernel_rate(args.batch, device)}
+            line["roofline"]["dominant_kernel"] = {"name": "gemm_quad_kernel / gemm_quad_grouped_kernel (256x256 tiles by four waves of 128x128: NT projections, a persistent workgroup per CU; the block's weight gradients as one grouped launch)", "hip_event_timing": dominant_kernel_rate(args.batch, device)}
             pmc, why_gemm = pmc_traffic()
             step_pmc, why_step = pmc_step_traffic()
             pmc_batch = step_pmc.get("per_gpu_batch") if step_pmc else None

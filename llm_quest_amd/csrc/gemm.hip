@@ -19,6 +19,7 @@
 //   * Epilogue: accumulators -> LDS (fp32, 64x64 at a time per wave) -> row-contiguous 16-B global stores with
 //     bias/GELU/residual fused, or raw fp32 slabs when K is split (few output tiles + long K: weight gradients).
 //   * Workgroup -> tile map: XCD-aware (blocks b and b+8 share an L2) then 3-row super-groups.
+// The large NT products and weight gradients are gemm_quad.h's, the mid-size NT and NN products gemm_ring_kernel's; gemm_tile serves the other forms, fused epilogues and sizes.
 #include <type_traits>
 
 #include "common.h"
@@ -31,15 +32,6 @@ namespace {
 // same-box pairs -- the main loops are the same instructions with the operand registers exchanged, and that is enough to move the step by 1 %.
 #ifndef GEMM_SWAP
 #define GEMM_SWAP 0
-#endif
-#ifndef GEMM_C_AUX_WALK
-#define GEMM_C_AUX_WALK 2
-#endif
-#ifndef GEMM_C_AUX_OLD
-#define GEMM_C_AUX_OLD 0
-#endif
-#ifndef MI355_GEMM_WALK_DEFAULT
-#define MI355_GEMM_WALK_DEFAULT 2  // see walk_on()
 #endif
 #ifndef MI355_GEMM_PP_DEFAULT
 #define MI355_GEMM_PP_DEFAULT 0  // see pp_mask()
@@ -164,8 +156,8 @@ __device__ __forceinline__ const bf16_t* uniform_ptr(const bf16_t* ptr) {
     return (const bf16_t*)(((unsigned long long)hi << 32) | lo);
 }
 
-__device__ __forceinline__ void dma_piece(const void* base, unsigned voff, char* lds_dst) {
-    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, 0x7fffffff, 0x00020000);
+__device__ __forceinline__ void dma_piece(const void* base, unsigned voff, char* lds_dst, int num_records = 0x7fffffff) {
+    auto rsrc = __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(base), 0, num_records, 0x00020000);
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, LDS_PTR(lds_dst), 16, voff, 0, 0, 0);
 }
 
@@ -273,7 +265,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int pid, co
     unsigned voffA[T::A_PPW], voffB[T::B_PPW];
     int kneedA[T::A_PPW], kneedB[T::B_PPW];
     constexpr int BK = T::BK;
-    // SPLIT (NT on the 8-wave 256x256 tile): the requests of a SIMD's two waves (w and w + 4) are divided by OPERAND, as in gemm_nt_persist_kernel -- waves 0-3 request
+    // SPLIT (NT on the 8-wave 256x256 tile): the requests of a SIMD's two waves (w and w + 4) are divided by OPERAND -- waves 0-3 request
     // the A-panel pieces of both (their own in the "A" set below, their partner's in the "B" set), behind the barrier; waves 4-7 the B-panel pieces of both, a phase later
     constexpr bool SPLIT = T::NW == 8 && T::BK == 64 && !A_TR && !B_TR && T::A_PPW == T::B_PPW;
     const bool a_side = !SPLIT || wave < 4;
@@ -1167,421 +1159,8 @@ __global__ __launch_bounds__(T::NTHREADS, T::MIN_WAVES) void gemm_bf16_kernel(Ge
     gemm_tile<T, A_TR, B_TR, OUT_DT>(p, xcd_chunked(blockIdx.x - split * nwg, nwg), split, smem);
 }
 
-// ---------------------------------------------------------------------------------------------- persistent NT kernel (tile hint 7)
-// tools/gemm_timeline.py (per-workgroup wall-clock stamps) on the QKV projection of the step, 256x256 tile, K = 1024: of a tile's 31.0 us turn on its CU the
-// main loop is 24.8; the rest is prologue 1.9 (entry -> first K-tile landed), barrier 0.6, write-out 2.45 (LDS-bandwidth: 512 KiB of fp32 staging traffic per tile),
-// stores retiring 0.5 and 0.8 between a workgroup's end and its successor's entry.  This kernel keeps ONE workgroup per CU alive over its share of the tiles:
-//   * the K-tile stream runs across tile boundaries (the last two barriers of a tile request the next tile's first two K-tiles), so there is no prologue, no
-//     retire wait and no workgroup turnover;
-//   * the write-out stages through a 32-KiB region BESIDE the two stages (4 KiB per wave: 32 rows x 64 columns of packed bf16 at a time, swizzled, not padded), so it
-//     needs no barrier and does not collide with the stream; the B fragment is the MFMA's first operand, so a lane holds four consecutive columns of a row and
-//     packs them itself: a quarter of the LDS bytes of the fp32 staging.
-// Results are bit-identical to gemm_bf16_kernel (same MFMA sequence per output, same rounding).  NT form, bf16 output, K % 64 == 0, N % 8 == 0, no bias.
-#if GEMM_PART == 2 || !defined(GEMM_PART)
-#if GEMM_TL
-#define TLQ(q, i) do { if (threadIdx.x == 0 && (q) < 32768) { g_gemm_tl[q][i] = __builtin_amdgcn_s_memrealtime(); g_gemm_tl[q][(i) + 1] = __builtin_readcyclecounter(); } } while (0)  // + the shader clock's counter: cycles / time = the clock the tile ran at
-#else
-#define TLQ(q, i) do { } while (0)
-#endif
-template <int KIND, bool RES, bool WALK>  // KIND: MI355_EPI_NONE (RES: + bf16 residual, added in fp32 before the rounding), MI355_EPI_SWIGLU_FWD, MI355_EPI_SWIGLU_BWD (see gemm_tile's epilogue for both)
-__global__ __launch_bounds__(512, 2) void gemm_nt_persist_kernel(GemmParams p, int ntiles) {
-    using T = Cfg256;
-    constexpr int BK = 64, HM = T::FM / 2;
-    static_assert(T::A_PPW == 4 && T::B_PPW == 4 && T::FM == 8 && T::FN == 4 && T::NS == 2, "written for 8 waves of 128x64 on two 64-KiB stages");
-    __shared__ __attribute__((aligned(16))) char smem[2 * T::STAGE + 32768];
-    const int lane = threadIdx.x & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    char* const stg = smem + 2 * T::STAGE + wave * 4096;
-    const int wr0 = (wave / T::WN) * T::WTM, wc0 = (wave % T::WN) * T::WTN;
-    const int nt = (int)(p.K / BK);
-    const int G = gridDim.x;
-
-    // the walk: by default tile blockIdx.x + j G of the XCD-chunked order in 6-row groups.  WALK (ablate bit 3, MI355_GEMM_WALK): weight-stationary per XCD, as in
-    // gemm_nt_pp_kernel -- column panels four at a time, an XCD owns a contiguous run of (column group, row panel) pairs, its 32 workgroups are 4 column panels x 8 row
-    // streams, stream r takes the run's pairs r, r + 8, ...; at K = 1 024 an XCD's four weight panels (2 MB) stay in its L2 for the whole launch.  A column group's
-    // missing panels (N / 256 not a multiple of 4) are walked as empty tiles (everything beyond the matrix: zero operands, no stores).  Needs the full grid of 256.
-    constexpr bool walk = WALK;
-    // cache policy of the output stores (0 default, 2 = nt, 16 = sc1, 18 = both).  Same-box bench.py pairs with the walk by shape: base 435.7 / 436.4 ms, nt on the
-    // weight-stationary launches 434.3 / 435.1, sc1 436.1 / 435.3, sc1 nt 434.5 / 434.8: nt there (the tile is written once and next read by another kernel; the L2 keeps the
-    // weight panels instead)
-    constexpr int CAUX = WALK ? GEMM_C_AUX_WALK : GEMM_C_AUX_OLD;
-    const int wk_xcd = blockIdx.x & 7, wk_l = blockIdx.x >> 3, wk_ci = wk_l & 3;
-    const int64_t wk_pairs = (int64_t)((p.tiles_n + 3) >> 2) * p.tiles_m;
-    const int wk_lo = (int)(wk_pairs * wk_xcd / 8) + (wk_l >> 2), wk_hi = (int)(wk_pairs * (wk_xcd + 1) / 8);
-    const int wk_J = wk_hi > wk_lo ? (wk_hi - wk_lo + 7) / 8 : 0;
-    const int qend = walk ? (int)blockIdx.x + wk_J * G : ntiles;  // this workgroup's tiles: q = blockIdx.x + j G < qend
-    auto origin = [&](int q, int64_t& m0, int64_t& n0) {
-        if (walk) {
-            const int pp = wk_lo + 8 * ((q - (int)blockIdx.x) / G);
-            const int cg = pp / p.tiles_m;
-            m0 = (int64_t)(pp - cg * p.tiles_m) * T::BM;
-            n0 = (int64_t)(cg * 4 + wk_ci) * T::BN;
-            return;
-        }
-        const int pid = xcd_chunked(q, ntiles);
-        constexpr int GROUP_M = 6;
-        const int in_group = GROUP_M * p.tiles_n;
-        const int first_m = (pid / in_group) * GROUP_M;
-        const int gsz = min(p.tiles_m - first_m, GROUP_M);
-        m0 = (int64_t)(first_m + (pid % in_group) % gsz) * T::BM;
-        n0 = (int64_t)((pid % in_group) / gsz) * T::BN;
-    };
-    // ---- the request side of the stream: tile qi, K-tile ti, element number si (stage si & 1).  The LDS-DMA requests of a SIMD's two waves (w and w + 4) are divided by
-    // OPERAND, not by wave: wave w requests the A-panel pieces of both (8 per K-tile), right behind the barrier that frees the stage; wave w + 4 requests the B-panel
-    // pieces of both (weights: they come from L2) a phase later, under its partner's MFMAs.  Issued symmetrically (every wave its own 4 + 4 behind the barrier), both waves
-    // of a SIMD stand in the CU's one address unit's queue at the same time and the matrix pipe idles; with the two request bursts half a K-tile apart, one wave of every
-    // SIMD always multiplies.  (All 16 requests on wave w, none on w + 4: between the two -- the requesting wave's burst plus its own 64 MFMAs is the K-tile's critical path.)
-    // The SwiGLU-backward form keeps all 16 requests on wave w (BY_OPERAND false): with the second request point in the K-tile its register allocation spills 72 values.
-    constexpr bool BY_OPERAND = KIND != MI355_EPI_SWIGLU_BWD;
-    const bool a_side = wave < 4;
-    const int wlo = wave & 3;
-    unsigned voff[2 * T::A_PPW];  // this wave's operand: pieces of waves wlo (0-3) and wlo + 4 (4-7)
-    [[maybe_unused]] unsigned voff2[2 * T::B_PPW];  // !BY_OPERAND: wave w's B-panel pieces
-    static_assert(T::A_PPW == T::B_PPW, "one offset array serves either operand");
-    const bf16_t* baseX = p.A;
-    [[maybe_unused]] const bf16_t* baseY = p.B;
-    auto plan = [&](int q) {
-        int64_t m0, n0;
-        origin(q, m0, n0);
-        int l = lane;
-        asm volatile("" : "+v"(l));  // recomputed from the lane number once per tile: hoisted, the per-piece rows and chunks would occupy 16 registers across the main loop
-        if (a_side) {  // (wave-uniform)
-            baseX = uniform_ptr(p.A + m0 * p.lda);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                unsigned v[T::A_PPW];
-                int unused[T::A_PPW];
-                piece_offsets<false, T::BM, BK, T::A_PPW>(wlo + 4 * h, l, p.lda, p.M - m0, v, unused);
-#pragma unroll
-                for (int j = 0; j < T::A_PPW; ++j) voff[h * T::A_PPW + j] = v[j];
-                if constexpr (!BY_OPERAND) {
-                    piece_offsets<false, T::BN, BK, T::B_PPW>(wlo + 4 * h, l, p.ldb, p.N - n0, v, unused);
-#pragma unroll
-                    for (int j = 0; j < T::B_PPW; ++j) voff2[h * T::B_PPW + j] = v[j];
-                }
-            }
-            if constexpr (!BY_OPERAND) baseY = uniform_ptr(p.B + n0 * p.ldb);
-        } else if constexpr (BY_OPERAND) {
-            baseX = KIND == MI355_EPI_SWIGLU_FWD ? uniform_ptr(p.B) : uniform_ptr(p.B + n0 * p.ldb);
-#pragma unroll
-            for (int h = 0; h < 2; ++h) {
-                const int w = wlo + 4 * h;
-                unsigned v[T::B_PPW];
-                if constexpr (KIND == MI355_EPI_SWIGLU_FWD) {
-                    // every 64 output columns of the tile are [32 lin1 rows | the 32 lin_gate rows of the SAME hidden units] of the fused weight (see gemm_tile)
-                    const int64_t nh = p.N >> 1;
-#pragma unroll
-                    for (int j = 0; j < T::B_PPW; ++j) {
-                        const int r = (w * T::B_PPW + j) * 8 + l / 8;
-                        const int c = swz_rowk<BK>(l % 8, r);
-                        const int64_t hid = (n0 >> 1) + (r >> 6) * 32 + (r & 31);
-                        v[j] = hid < nh ? (unsigned)((((r >> 5) & 1) * nh + hid) * p.ldb * 2 + c * 16) : OOB;
-                    }
-                } else {
-                    int unused[T::B_PPW];
-                    piece_offsets<false, T::BN, BK, T::B_PPW>(w, l, p.ldb, p.N - n0, v, unused);
-                }
-#pragma unroll
-                for (int j = 0; j < T::B_PPW; ++j) voff[h * T::B_PPW + j] = v[j];
-            }
-        }
-    };
-    int qi = blockIdx.x, ti = 0, si = 0;
-    auto request_next = [&]() {  // this wave's operand of element si
-        if (qi < qend) {
-            char* dst = smem + (si & 1) * T::STAGE + (a_side ? 0 : T::A_BYTES) + wlo * T::A_PPW * 1024;
-            const bf16_t* px = baseX + (int64_t)ti * BK;
-#pragma unroll
-            for (int h = 0; h < 2; ++h)
-#pragma unroll
-                for (int j = 0; j < T::A_PPW; ++j) dma_piece(px, voff[h * T::A_PPW + j], dst + (h * 4 * T::A_PPW + j) * 1024);
-            if constexpr (!BY_OPERAND) {
-                const bf16_t* py = baseY + (int64_t)ti * BK;
-#pragma unroll
-                for (int h = 0; h < 2; ++h)
-#pragma unroll
-                    for (int j = 0; j < T::B_PPW; ++j) dma_piece(py, voff2[h * T::B_PPW + j], dst + T::A_BYTES + (h * 4 * T::B_PPW + j) * 1024);
-            }
-            if (++ti == nt) {
-                ti = 0;
-                qi += G;
-                if (qi < qend) plan(qi);
-            }
-        }
-        ++si;
-    };
-
-    int qc = blockIdx.x, sc = 0;  // the multiplying side: tile qc, element number sc
-    if (qc >= qend) return;
-    plan(qi);
-    f32x4 acc[T::FM][T::FN];
-    bf16x8 aE[HM], aO[HM], b0[T::FN], b1[T::FN];
-    auto loadA = [&](bf16x8 (&a)[HM], const char* sA, int kk, int mh) {
-#pragma unroll
-        for (int i = 0; i < HM; ++i) a[i] = frag_rowk<BK>(sA, wr0 + (mh * HM + i) * 16, kk, lane);
-    };
-    auto loadB = [&](bf16x8 (&b)[T::FN], const char* sB, int kk) {
-#pragma unroll
-        for (int j = 0; j < T::FN; ++j) b[j] = frag_rowk<BK>(sB, wc0 + j * 16, kk, lane);
-    };
-    // B fragment first: the lane holds C[row lane & 15][4 (lane >> 4) + e].  ZERO: the tile's first k-step starts from the constant 0 (no accumulator is cleared anywhere)
-    auto mma = [&](bool zero, const bf16x8 (&a)[HM], const bf16x8 (&b)[T::FN], int mh) {
-        if (zero) {  // wave-uniform
-#pragma unroll
-            for (int i = 0; i < HM; ++i)
-#pragma unroll
-                for (int j = 0; j < T::FN; ++j) acc[mh * HM + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], (f32x4){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
-        } else {
-#pragma unroll
-            for (int i = 0; i < HM; ++i)
-#pragma unroll
-                for (int j = 0; j < T::FN; ++j) acc[mh * HM + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[mh * HM + i][j], 0, 0, 0);
-        }
-    };
-    bool more_tiles = false;
-    auto kstep = [&](int t) {  // one element of the stream: 64 MFMAs in four phases (k-step, row half), the next element's first fragments requested under the last
-        const char* sA = smem + (sc & 1) * T::STAGE;
-        const char* sB = sA + T::A_BYTES;
-        loadA(aO, sA, 0, 1);
-        mma(t == 0, aE, b0, 0);
-        if (BY_OPERAND && !a_side && sc > 0) request_next();  // the B panels of element sc + 1 (its A panels were requested behind the last barrier; elements 0 and 1: before the loop)
-        loadB(b1, sB, 1);
-        loadA(aE, sA, 1, 0);
-        mma(t == 0, aO, b0, 1);
-        loadA(aO, sA, 1, 1);
-        mma(false, aE, b1, 0);
-        const bool last = t + 1 == nt;
-        if (!last || more_tiles) {
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this wave's reads of the element are complete ...
-            wait_vmcnt<0>();                                    // ... its share of the next element has landed (and the previous tile's stores have retired)
-            __builtin_amdgcn_s_barrier();                       // ... for every wave
-            if (a_side) request_next();                         // the A panels of element sc + 2 into the stage just left: at the end of a tile that is the NEXT tile's stream
-            if (!last) {
-                const char* nA = smem + ((sc + 1) & 1) * T::STAGE;
-                loadB(b0, nA + T::A_BYTES, 0);
-                loadA(aE, nA, 0, 0);
-            }
-        }
-        mma(false, aO, b1, 1);
-        ++sc;
-    };
-    if (BY_OPERAND || a_side) request_next();  // elements 0 and 1: both operands
-    wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-    if (BY_OPERAND || a_side) request_next();
-    loadB(b0, smem + T::A_BYTES, 0);
-    loadA(aE, smem, 0, 0);
-    for (;;) {
-        TLQ(qc, 0);
-        more_tiles = qc + G < qend;
-        for (int t = 0; t < nt; ++t) kstep(t);
-        TLQ(qc, 2);
-        // ---- write-out of tile qc: 4 sub-blocks of 32 rows x 64 columns per wave; packed bf16 through this wave's own 4 KiB.  LDS operations of a wave execute in
-        // order, so sub-block sb + 1 is staged right behind the row reads of sub-block sb, whose stores go out while it is being packed; rows and columns beyond the
-        // matrix are dropped by the buffer range check (offset OOB), so the passes have no branches.
-        int le = lane;
-        asm volatile("" : "+v"(le));  // derived per tile, not kept across the main loop
-        const int g = le >> 4, r16 = le & 15;
-        // staging addresses of this lane.  Write side: row r = ii * 16 + r16 of a 32 x 64 sub-block (128-byte rows), 16-byte chunk (2 j + g / 2) ^ (r & 7), 8-byte half
-        // (g & 1) ^ (r >> 3 & 1): the 16 rows one store instruction covers hit 32 distinct banks.  Read side: row pass * 8 + lane / 8, chunk (lane & 7) ^ (row & 7).
-        const int wr_off = r16 * 128 + ((((g & 1) ^ (r16 >> 3)) & 1) << 3), wr_x = r16 & 7;
-        const int rd_row = le >> 3, rd_ch = le & 7;
-        const int rd_off = rd_row * 128 + ((rd_ch ^ (rd_row & 7)) << 4);  // (pass * 8 + rd_row) & 7 == rd_row & 7
-        int64_t m0, n0;
-        origin(qc, m0, n0);
-        const int64_t rows_left = p.M - m0 - wr0;
-        u32x4 rd[4];
-        [[maybe_unused]] u32x2 rres[2][T::FN];   // RES: the residual of a sub-block in the accumulators' layout (8-byte loads)
-        [[maybe_unused]] u32x4 uv[4], gv[4];     // SwiGLU backward: the forward's gate-up pair of a sub-block's rows (16-byte loads)
-        [[maybe_unused]] u32x2 partner[4];       // SwiGLU forward: the other operand of the four units this lane activates
-        [[maybe_unused]] float psum[4][4];       // attention delta: this wave's half-head row sums (sub-block, pass), complete in every lane of the row's eight
-        const int hi4 = rd_ch >> 2;
-        // column base of this wave in C (and R), validity of this lane's 8 columns
-        int64_t cbase, cbase2 = 0;
-        bool col_ok;
-        if constexpr (KIND == MI355_EPI_SWIGLU_FWD) {
-            const int64_t nh = p.N >> 1, hid = (n0 >> 1) + (wc0 >> 6) * 32 + (rd_ch & 3) * 8;
-            col_ok = hid < nh;
-            cbase = (hi4 ? nh : 0) + hid;  // gate-up output: u into [:, hid], g into [:, N/2 + hid]
-            cbase2 = hid + 4 * hi4;        // activation output (R): four units per lane
-        } else {
-            cbase = n0 + wc0 + rd_ch * 8;
-            col_ok = cbase < p.N;
-        }
-        auto rsrc_c = __builtin_amdgcn_make_buffer_rsrc(reinterpret_cast<bf16_t*>(p.C) + (m0 + wr0) * p.ldc, 0, 0x7fffffff, 0x00020000);
-        auto rsrc_r = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(reinterpret_cast<const bf16_t*>(p.R)) + (m0 + wr0) * p.ldr, 0, 0x7fffffff, 0x00020000);
-        auto fetch_res = [&](int sb) {  // residual of sub-block sb, requested a sub-block before it is packed
-            if constexpr (RES) {
-#pragma unroll
-                for (int ii = 0; ii < 2; ++ii)
-#pragma unroll
-                    for (int j = 0; j < T::FN; ++j) {
-                        const int row = sb * 32 + ii * 16 + r16;
-                        const int64_t col = n0 + wc0 + j * 16 + 4 * g;
-                        rres[ii][j] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rsrc_r, (row < rows_left && col < p.N) ? (unsigned)((row * p.ldr + col) * 2) : OOB, 0, 0));
-                    }
-            }
-        };
-        auto fetch_ug = [&](int sb) {  // gate-up rows of sub-block sb, requested when it is staged, used a sub-block later (after the stores of sb - 1 have consumed theirs)
-            if constexpr (KIND == MI355_EPI_SWIGLU_BWD || KIND == MI355_EPI_ATTN_DELTA) {
-#pragma unroll
-                for (int pass = 0; pass < 4; ++pass) {
-                    const int row = sb * 32 + pass * 8 + rd_row;
-                    const bool ok = col_ok && row < rows_left;
-                    uv[pass] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_r, ok ? (unsigned)((row * p.ldr + cbase) * 2) : OOB, 0, 0));  // delta: the forward's ctx
-                    if constexpr (KIND == MI355_EPI_SWIGLU_BWD)
-                        gv[pass] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rsrc_r, ok ? (unsigned)((row * p.ldr + cbase + p.N) * 2) : OOB, 0, 0));
-                }
-            }
-        };
-        auto stores = [&](int sb) {
-#pragma unroll
-            for (int pass = 0; pass < 4; ++pass) {
-                const u32x4 o = (pass & 1) ? (u32x4){rd[pass][2], rd[pass][3], rd[pass][0], rd[pass][1]} : rd[pass];  // rows 8-15 of a 16-row tile were written with their halves exchanged
-                const int row = sb * 32 + pass * 8 + rd_row;
-                const bool ok = col_ok && row < rows_left;
-                if constexpr (KIND == MI355_EPI_SWIGLU_BWD) {
-                    // o = d(act) of hidden units cbase..+7, rounded to bf16: d(gate-up) = [d * g sig(g) | d * u sig(g) (1 + g (1 - sig(g)))] into C[:, unit], C[:, N + unit] (ldc = 2N)
-                    u32x4 o0, o1;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        float du[2], dg[2];
-#pragma unroll
-                        for (int hlf = 0; hlf < 2; ++hlf) {
-                            const float d_ = hlf ? __uint_as_float(o[e] & 0xffff0000u) : __uint_as_float(o[e] << 16);
-                            const float u_ = hlf ? __uint_as_float(uv[pass][e] & 0xffff0000u) : __uint_as_float(uv[pass][e] << 16);
-                            const float g_ = hlf ? __uint_as_float(gv[pass][e] & 0xffff0000u) : __uint_as_float(gv[pass][e] << 16);
-                            swiglu_grads(d_, u_, g_, du[hlf], dg[hlf]);
-                        }
-                        o0[e] = pack_bf2(du[0], du[1]);
-                        o1[e] = pack_bf2(dg[0], dg[1]);
-                    }
-                    __builtin_amdgcn_raw_buffer_store_b128(o0, rsrc_c, ok ? (unsigned)((row * p.ldc + cbase) * 2) : OOB, 0, CAUX);
-                    __builtin_amdgcn_raw_buffer_store_b128(o1, rsrc_c, ok ? (unsigned)((row * p.ldc + cbase + p.N) * 2) : OOB, 0, CAUX);
-                } else {
-                    __builtin_amdgcn_raw_buffer_store_b128(o, rsrc_c, ok ? (unsigned)((row * p.ldc + cbase) * 2) : OOB, 0, CAUX);
-                    if constexpr (KIND == MI355_EPI_ATTN_DELTA) {
-                        // o = d(ctx), rounded; uv = ctx: the row's dot product over this lane's 8 columns, folded over the row's eight lanes = half a head (the wave's 64 columns)
-                        float dsum = 0.f;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e)
-                            dsum += __uint_as_float(o[e] << 16) * __uint_as_float(uv[pass][e] << 16) + __uint_as_float(o[e] & 0xffff0000u) * __uint_as_float(uv[pass][e] & 0xffff0000u);
-                        dsum += __shfl_xor(dsum, 1, 64);
-                        dsum += __shfl_xor(dsum, 2, 64);
-                        dsum += __shfl_xor(dsum, 4, 64);
-                        psum[sb][pass] = dsum;
-                    }
-                    if constexpr (KIND == MI355_EPI_SWIGLU_FWD) {
-                        // this lane's 8 columns are u (chunks 0-3) or g (chunks 4-7) of 8 hidden units; it activates four of them: units 0-3 (u lanes) resp. 4-7 (g lanes),
-                        // the other operand = the partner lane's chunk, read back from the staging rows; a = u * silu(g) on the ROUNDED operands, as mi355_swiglu_fwd sees them
-                        // (operands are picked with selects, word by word: written as `hi4 ? act(other, mine) : act(mine, other)` on an indexed `o[2 * hi4 + ..]`, every lane
-                        // ran both sides of a divergent branch -- twice the exponentials -- behind a chain of compares for the index)
-                        const u32x2 pv = partner[pass];
-                        const unsigned own0 = hi4 ? o[2] : o[0], own1 = hi4 ? o[3] : o[1];
-                        const unsigned uw[2] = {hi4 ? pv[0] : own0, hi4 ? pv[1] : own1}, gw[2] = {hi4 ? own0 : pv[0], hi4 ? own1 : pv[1]};
-                        float a4[4];
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) {
-                            const float u_ = (e & 1) ? __uint_as_float(uw[e >> 1] & 0xffff0000u) : __uint_as_float(uw[e >> 1] << 16);
-                            const float g_ = (e & 1) ? __uint_as_float(gw[e >> 1] & 0xffff0000u) : __uint_as_float(gw[e >> 1] << 16);
-                            a4[e] = swiglu_act(u_, g_);
-                        }
-                        const u32x2 av = {pack_bf2(a4[0], a4[1]), pack_bf2(a4[2], a4[3])};
-                        __builtin_amdgcn_raw_buffer_store_b64(av, rsrc_r, ok ? (unsigned)((row * p.ldr + cbase2) * 2) : OOB, 0, 0);
-                    }
-                }
-            }
-        };
-        fetch_res(0);
-#pragma unroll
-        for (int sb = 0; sb < 4; ++sb) {
-#pragma unroll
-            for (int ii = 0; ii < 2; ++ii)
-#pragma unroll
-                for (int j = 0; j < T::FN; ++j) {
-                    f32x4 v = acc[sb * 2 + ii][j];
-                    if constexpr (RES) {
-                        v[0] += __uint_as_float(rres[ii][j][0] << 16);
-                        v[1] += __uint_as_float(rres[ii][j][0] & 0xffff0000u);
-                        v[2] += __uint_as_float(rres[ii][j][1] << 16);
-                        v[3] += __uint_as_float(rres[ii][j][1] & 0xffff0000u);
-                    }
-                    const u32x2 pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3])};
-                    *reinterpret_cast<u32x2*>(stg + ii * 2048 + wr_off + (((2 * j + (g >> 1)) ^ wr_x) << 4)) = pk;
-                }
-            if (sb > 0) stores(sb - 1);
-            if (sb < 3) fetch_res(sb + 1);
-            fetch_ug(sb);
-#pragma unroll
-            for (int pass = 0; pass < 4; ++pass) {
-                rd[pass] = *reinterpret_cast<const u32x4*>(stg + pass * 1024 + rd_off);
-                if constexpr (KIND == MI355_EPI_SWIGLU_FWD) {
-                    // partner chunk rd_ch ^ 4 of the same row, its half hi4 (units 4-7 of the partner's eight for g lanes, 0-3 for u lanes); odd passes hold rows whose halves are exchanged
-                    const int prow = rd_row;  // (pass * 8 + rd_row) & 7
-                    partner[pass] = *reinterpret_cast<const u32x2*>(stg + pass * 1024 + rd_row * 128 + ((((rd_ch ^ 4) ^ (prow & 7))) << 4) + (((hi4 ^ pass) & 1) << 3));
-                }
-            }
-        }
-        stores(3);
-        if constexpr (KIND == MI355_EPI_ATTN_DELTA) {
-            // a head's two halves sit in two neighbouring waves: every wave parks its 128 row sums in its own staging region (behind its last row reads: LDS operations
-            // execute in order), one barrier, then one thread per (row, head) adds the halves in a fixed order and writes the attention backward's three row constants.
-            // The regions are next written in the following tile's write-out, which every wave reaches only through that tile's K-loop barriers.
-            static_assert(T::NTHREADS == 512 && T::WN == 4 && T::WTN == 64, "delta write-out: 2 x 4 waves of 128 x 64 on a 256 x 256 tile");
-            float* part = reinterpret_cast<float*>(stg);
-#pragma unroll
-            for (int sb = 0; sb < 4; ++sb)
-#pragma unroll
-                for (int pass = 0; pass < 4; ++pass)
-                    if (rd_ch == 0) part[sb * 32 + pass * 8 + rd_row] = psum[sb][pass];
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            __builtin_amdgcn_s_barrier();
-            const int t_ = threadIdx.x, row = t_ & 255, hsel = t_ >> 8;
-            const float* p0 = reinterpret_cast<const float*>(smem + 2 * T::STAGE + ((row >> 7) * 4 + 2 * hsel) * 4096);
-            const float sum = p0[row & 127] + p0[1024 + (row & 127)];
-            const int64_t gm = m0 + row, head = (n0 >> 7) + hsel;
-            if (gm < p.M && head < p.ad_Hq) {
-                const int64_t bb = gm / p.ad_S, sq = gm - bb * p.ad_S;
-                const int64_t di = (bb * p.ad_Hq + head) * p.ad_S + sq;
-                p.ad_delta[di] = sum;
-                p.ad_ndl[di] = -sum;
-                p.ad_nl2[di] = -p.ad_lse[di] * 1.4426950408889634f;
-            }
-        }
-        TLQ(qc, 4);
-        qc += G;
-        if (qc >= qend) break;
-        const char* nA = smem + (sc & 1) * T::STAGE;
-        loadB(b0, nA + T::A_BYTES, 0);
-        loadA(aE, nA, 0, 0);
-    }
-}
-
-int launch_persist(GemmParams p, hipStream_t s) {
-    using T = Cfg256;
-    p.tiles_m = (int)((p.M + T::BM - 1) / T::BM);
-    p.tiles_n = (int)((p.N + T::BN - 1) / T::BN);
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    MI355_REQUIRE(tiles < 0x7fffffffLL / 16, "mi355_gemm_bf16: grid too large");
-    const dim3 grid((unsigned)((tiles < 256 && !(p.ablate & 8)) ? tiles : 256)), block(T::NTHREADS);  // one workgroup per CU
-#define PERSIST_LAUNCH(KIND_, RES_)                                                                                                      \
-    do {                                                                                                                                 \
-        if (p.ablate & 8) hipLaunchKernelGGL((gemm_nt_persist_kernel<KIND_, RES_, true>), grid, block, 0, s, p, (int)tiles);               \
-        else hipLaunchKernelGGL((gemm_nt_persist_kernel<KIND_, RES_, false>), grid, block, 0, s, p, (int)tiles);                           \
-    } while (0)
-    if (p.epilogue == MI355_EPI_SWIGLU_FWD) PERSIST_LAUNCH(MI355_EPI_SWIGLU_FWD, false);
-    else if (p.epilogue == MI355_EPI_SWIGLU_BWD) PERSIST_LAUNCH(MI355_EPI_SWIGLU_BWD, false);
-    else if (p.epilogue == MI355_EPI_ATTN_DELTA) PERSIST_LAUNCH(MI355_EPI_ATTN_DELTA, false);
-    else if (p.R) PERSIST_LAUNCH(MI355_EPI_NONE, true);
-    else PERSIST_LAUNCH(MI355_EPI_NONE, false);
-#undef PERSIST_LAUNCH
-    MI355_LAUNCH_CHECK("mi355_gemm_bf16(persistent)");
-    return 0;
-}
-#endif  // part 2
-
 // ---------------------------------------------------------------------------------------------- ping-pong persistent NT kernel (tile hint 8)
-// gemm_nt_persist_kernel's two waves per SIMD (w and w + 4: the upper and the lower 128 rows of the 256 x 256 tile) reach their write-out together, so the
+// The two waves per SIMD of an eight-wave tile (w and w + 4: the upper and the lower 128 rows of the 256 x 256 tile) reach their write-out together, so the
 // matrix pipe of every SIMD idles for the whole write-out: 2.45 of a tile's 27.5 us with the plain epilogue at K = 1 024, a quarter of the tile with the SwiGLU
 // forms (1.26 PF plain, 1.11 / 0.84 PF fused).  VALU / LDS / store issue and the matrix pipe are separate resources of a SIMD; what keeps them from
 // overlapping is only that both waves are in the same phase.  This kernel runs the two wave groups E K-tiles apart:
@@ -1593,12 +1172,12 @@ int launch_persist(GemmParams p, hipStream_t s) {
 //     at and wraps around: every output is the sum over all K-tiles in an order ROTATED by a multiple of E, so results equal the per-tile kernel's up to the
 //     fp32 summation order (bit-identical whenever the products are exact; tests/test_kernels_gpu.py), and are the same bits on every run.
 //   * requests: every wave asks for its own four pieces of the weight panel and, for slots in which its group multiplies, its own four pieces of the activation
-//     panel; waves 0-3 right behind the barrier that frees the stage, waves 4-7 half a slot later (the CU has one address unit: see gemm_nt_persist_kernel).
+//     panel; waves 0-3 right behind the barrier that frees the stage, waves 4-7 half a slot later (the CU has one address unit).
 // NT form, bf16 output, K % 64 == 0, K / 64 >= E, N % 8 == 0, no bias.
 //
 // STATUS: correct on every epilogue kind (tools/experimental/pp_check.py: bit-identical to tile 2 on integer operands, fp32-summation noise on random ones), and
-// SLOWER than gemm_nt_persist_kernel wherever the write-out matters, so the library does not choose it (MI355_GEMM_PP_DEFAULT 0; tile hint 8 / MI355_GEMM_PP select it).
-// Batch 160, isolated, us (hint 7 -> hint 8): QKV 771 -> 881, out-proj + residual 424 -> 453, gate-up + SwiGLU 1 310 -> 1 451, down dgrad + SwiGLU backward 905 -> 1 063,
+// SLOWER than an eight-wave persistent workgroup wherever the write-out matters -- hint 7's kernel then; gemm_quad.h's, which took its place, is faster than both -- so the library does not choose it
+// (MI355_GEMM_PP_DEFAULT 0; tile hint 8 / MI355_GEMM_PP select it).  Batch 160, isolated, us (eight-wave persistent -> hint 8): QKV 771 -> 881, out-proj + residual 424 -> 453, gate-up + SwiGLU 1 310 -> 1 451, down dgrad + SwiGLU backward 905 -> 1 063,
 // LM head forward 21.8 -> 22.6 ms; long-K shapes level (dqkv 733 -> 752, LM head dgrad 19.3 -> 18.6 ms: the walk).  In the step: +1.5 ... +7 ms per kind.  Why:
 //   * with NO write-out work at all (ablate bit 0) the same launches take 732 / 360 / 1 073 / 621 us and 19.3 ms: -5 ... -31 % -- the overlap is there to be had;
 //   * but a slot in which only one group multiplies does not get shorter than ~0.9 us (against 1.55 us for a slot with both): the stream is two stages deep, a slot's
@@ -1662,7 +1241,7 @@ __global__ __launch_bounds__(512, 2) void gemm_nt_pp_kernel(GemmParams p, int nt
     auto tile_m0 = [&](const Walk& w) { return (int64_t)w.sr * T::BM; };
     auto tile_n0 = [&](const Walk& w) { return (int64_t)(w.cg * 4 + ci) * T::BN; };
 
-    // ---- the request side, divided by OPERAND as in gemm_nt_persist_kernel: waves 0-3 ask for the activation panel (both halves: it comes from HBM, so early, right
+    // ---- the request side, divided by OPERAND: waves 0-3 ask for the activation panel (both halves: it comes from HBM, so early, right
     // behind the barrier that frees the stage), waves 4-7 for the weight panel (L2) half a slot later.  A wave therefore follows two streams of four pieces each:
     //   waves 0-3: stream 1 = rows 32 w .. + 31 of the upper group's tile (on the upper group's clock), stream 2 = the same rows of the lower half (lower group's clock: E behind);
     //   waves 4-7: streams 1 / 2 = weight-panel rows 64 (w - 4) .. + 31 / + 32 .. + 63, both on the upper group's clock (the weight stream follows the upper group's tile
@@ -1757,7 +1336,7 @@ __global__ __launch_bounds__(512, 2) void gemm_nt_pp_kernel(GemmParams p, int nt
         }
     };
 
-    // ---- the multiplying side (gemm_nt_persist_kernel's K-tile, unchanged)
+    // ---- the multiplying side (gemm_tile's K-tile)
     f32x4 acc[T::FM][T::FN];
     bf16x8 aE[HM], aO[HM], b0[T::FN], b1[T::FN];
     auto loadA = [&](bf16x8 (&a)[HM], const char* sA, int kk, int mh) {
@@ -1814,7 +1393,7 @@ __global__ __launch_bounds__(512, 2) void gemm_nt_pp_kernel(GemmParams p, int nt
         mma(false, aO, b1, 1);
     };
 
-    // ---- write-out chunk c of this group's tile cj: sub-block c (32 rows x 64 columns per wave) through the wave's own 4 KiB of packed bf16, as in gemm_nt_persist_kernel
+    // ---- write-out chunk c of this group's tile cj: sub-block c (32 rows x 64 columns per wave) through the wave's own 4 KiB of packed bf16
     [[maybe_unused]] float psum[4][4];  // attention delta: this wave's half-head row sums (sub-block, pass)
     auto epi_chunk = [&](auto sb_c, const int cj) __attribute__((always_inline)) {
         constexpr int sb = decltype(sb_c)::value;
@@ -2029,6 +1608,39 @@ struct GroupTable {
     int start[MAX_GROUP + 1];  // first tile of each problem in the concatenated list
     int count;
 };
+
+#if GEMM_PART >= 8 || !defined(GEMM_PART)
+#include "gemm_quad.h"
+
+// persistent: one workgroup per CU walks its share of the tiles, else a workgroup per tile
+template <bool TR>
+int launch_quad(GemmParams p, int out_dtype, bool persistent, hipStream_t s) {
+    p.tiles_m = (int)((p.M + 255) / 256);
+    p.tiles_n = (int)((p.N + 255) / 256);
+    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
+    MI355_REQUIRE(tiles < 0x7fffffffLL / 16, "mi355_gemm_bf16: grid too large");
+    const dim3 grid((unsigned)(persistent && tiles > 256 ? 256 : tiles)), block(256);
+#define QUAD(OUT_, KIND_) gemm_quad_kernel<TR, OUT_, KIND_>
+    void (*kernel)(GemmParams);
+    const bool b16 = out_dtype == MI355_DT_BF16;
+    if constexpr (TR) {
+        if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
+        else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
+    } else {
+        if (p.epilogue == MI355_EPI_SWIGLU_FWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_FWD);
+        else if (p.epilogue == MI355_EPI_SWIGLU_BWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_BWD);
+        else if (p.epilogue == MI355_EPI_ATTN_DELTA) kernel = QUAD(MI355_DT_BF16, MI355_EPI_ATTN_DELTA);
+        else if (p.R && p.bias) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES | QUAD_BIAS) : QUAD(MI355_DT_F32, QUAD_RES | QUAD_BIAS);
+        else if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
+        else if (p.bias) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_BIAS) : QUAD(MI355_DT_F32, QUAD_BIAS);
+        else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
+    }
+#undef QUAD
+    hipLaunchKernelGGL(kernel, grid, block, QUAD_SMEM, s, p);
+    MI355_LAUNCH_CHECK("mi355_gemm_bf16(four waves)");
+    return 0;
+}
+#endif
 
 template <class T, bool A_TR, bool B_TR, int OUT_DT>
 __global__ __launch_bounds__(T::NTHREADS, T::MIN_WAVES) void gemm_grouped_kernel(GroupTable tbl) {
@@ -2440,6 +2052,25 @@ int launch_grouped(GroupTable& tbl, int out_dtype, hipStream_t s) {
     return 0;
 }
 
+#if GEMM_PART == 9 || !defined(GEMM_PART)
+int launch_quad_grouped(GroupTable& tbl, int out_dtype, hipStream_t s) {
+    int64_t total = 0;
+    for (int i = 0; i < tbl.count; ++i) {
+        GemmParams& p = tbl.g[i];
+        p.tiles_m = (int)((p.M + 255) / 256);
+        p.tiles_n = (int)((p.N + 255) / 256);
+        tbl.start[i] = (int)total;
+        total += (int64_t)p.tiles_m * p.tiles_n;
+        MI355_REQUIRE(total < 0x7fffffffLL / 16, "mi355_gemm_bf16_grouped: grid too large");
+    }
+    for (int i = tbl.count; i <= MAX_GROUP; ++i) tbl.start[i] = (int)total;
+    if (out_dtype == MI355_DT_BF16) hipLaunchKernelGGL(gemm_quad_grouped_kernel<MI355_DT_BF16>, dim3((unsigned)total), dim3(256), QUAD_SMEM, s, tbl);
+    else hipLaunchKernelGGL(gemm_quad_grouped_kernel<MI355_DT_F32>, dim3((unsigned)total), dim3(256), QUAD_SMEM, s, tbl);
+    MI355_LAUNCH_CHECK("mi355_gemm_bf16_grouped(four waves)");
+    return 0;
+}
+#endif
+
 template <class T>
 int launch_grouped_form(int form, GroupTable& tbl, int out_dtype, hipStream_t s) {
     switch (form) {
@@ -2534,7 +2165,9 @@ __global__ __launch_bounds__(256) void colsum_kernel(int64_t M, int64_t N, const
         return launch_grouped_form<CFG>(form, *static_cast<GroupTable*>(table), out_dtype, (hipStream_t)stream);                                   \
     }
 GEMM_BRIDGE_DECL(1) GEMM_BRIDGE_DECL(2) GEMM_BRIDGE_DECL(3) GEMM_BRIDGE_DECL(4) GEMM_BRIDGE_DECL(5)
-extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_persist_part2(const void* params, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_nt_part8(const void* params, int out_dtype, int persistent, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_tn_part9(const void* params, int out_dtype, int persistent, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_grouped_part9(void* table, int out_dtype, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_pp_part6(const void* params, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_ring_part7(int form, const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream);
 #if GEMM_PART == 7 || GEMM_PART == -1
@@ -2548,8 +2181,16 @@ extern "C" int mi355_gemm_ring_part7(int form, const void* params, int out_dtype
 #if GEMM_PART == 6 || GEMM_PART == -1
 extern "C" int mi355_gemm_pp_part6(const void* params, void* stream) { return launch_pp(*static_cast<const GemmParams*>(params), (hipStream_t)stream); }
 #endif
-#if GEMM_PART == 2 || GEMM_PART == -1
-extern "C" int mi355_gemm_persist_part2(const void* params, void* stream) { return launch_persist(*static_cast<const GemmParams*>(params), (hipStream_t)stream); }
+#if GEMM_PART == 8 || GEMM_PART == -1
+extern "C" int mi355_gemm_quad_nt_part8(const void* params, int out_dtype, int persistent, void* stream) {
+    return launch_quad<false>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
+}
+#endif
+#if GEMM_PART == 9 || GEMM_PART == -1
+extern "C" int mi355_gemm_quad_tn_part9(const void* params, int out_dtype, int persistent, void* stream) {
+    return launch_quad<true>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
+}
+extern "C" int mi355_gemm_quad_grouped_part9(void* table, int out_dtype, void* stream) { return launch_quad_grouped(*static_cast<GroupTable*>(table), out_dtype, (hipStream_t)stream); }
 #endif
 #if GEMM_PART == 1 || GEMM_PART == -1
 GEMM_BRIDGE_DEF(1, Cfg128)
@@ -2596,23 +2237,21 @@ static int64_t persist_min_tiles() {
 
 // which epilogue kinds of the persistent NT kernel take the ping-pong form (tile hint 8) by themselves: a bit mask, 1 plain, 2 + residual, 4 SwiGLU forward,
 // 8 SwiGLU backward, 16 attention delta (MI355_GEMM_PP; read per call: A/B runs and tests change it inside one process)
-static bool walk_on(int64_t N, int64_t K) {
-    // MI355_GEMM_WALK: the persistent NT kernel's weight-stationary walk (gemm_nt_persist_kernel<.., WALK>) for launches the library chooses by itself: 0 never, 1 always,
-    // 2 (default) by shape: few column panels under a long K (the dgrads into d = 1024, the out / down projections), or very many column panels (the LM head).
-    // batch 160, same-box bench.py runs: never 443.3 / 443.6 / 444.7 / 445.9 ms, by shape 438.5 / 438.6 / 441.4-441.8, always 441.6 / 440.6; per shape class (16 + mask):
-    // N <= 1024 with K >= 3072 -3.7 ms, + K = 2048 -0.2, the LM head 0 to -1.2, N = 2048 0, N = 3072 / 4096 / 6144 (K = 1024) +1.0 to +1.9 ms each.  Read per call.
-    const char* e = getenv("MI355_GEMM_WALK");
-    const int mode = e && *e ? atoi(e) : MI355_GEMM_WALK_DEFAULT;
-    if (mode >= 16) {  // exploration: 16 + a mask of shape classes
-        const int m = mode - 16;
-        return ((m & 1) && N <= 1024 && K >= 3072) || ((m & 2) && N >= 64 * 256) || ((m & 4) && N <= 1024 && K == 2048) || ((m & 8) && N == 2048) || ((m & 16) && N == 3072) ||
-               ((m & 32) && N == 4096) || ((m & 64) && N == 6144);
-    }
-    return mode == 1 || (mode == 2 && ((N <= 1024 && K >= 2048) || N >= 64 * 256));
-}
 static int pp_mask() {
     const char* e = getenv("MI355_GEMM_PP");
     return e && *e ? atoi(e) : MI355_GEMM_PP_DEFAULT;
+}
+
+// what gemm_quad.h's kernels take of a problem on 256x256 tiles: four K-tiles or more, whole 16-byte groups of columns, results and residual rows that 16-byte accesses reach, 32-bit offsets within a
+// tile's rows (operands: check_operands)
+static bool quad_ok(int form, const GemmParams& p, int out_dtype) {
+    const int64_t esz = out_dtype == MI355_DT_F32 ? 4 : 2, limit = 0x7fffffffLL / (128 * esz);
+    const auto rows_ok = [&](const void* x, int64_t ld) { return (ld * esz & 15) == 0 && ((uintptr_t)x & 15) == 0 && ld < limit; };
+    if (p.K <= 192 || (p.N & 7) || p.M > 0x7fffff00 || p.N > 0x7fffff00 || !rows_ok(p.C, p.ldc) || (p.R && !rows_ok(p.R, p.ldr))) return false;
+    if (form == MI355_GEMM_TN) return !p.bias && p.epilogue == MI355_EPI_NONE;
+    if (form != MI355_GEMM_NT || (p.K & 63) || p.split3) return false;
+    if (p.epilogue == MI355_EPI_SWIGLU_FWD) return p.N * p.ldb * 2 < 0x7fffffffLL;
+    return p.epilogue == MI355_EPI_NONE || p.epilogue == MI355_EPI_SWIGLU_BWD || p.epilogue == MI355_EPI_ATTN_DELTA;
 }
 
 // Forward products and input gradients of fewer 256x256 tiles than half of the CUs: measured 92 tiles -> 128x128 wins (+2.8 % on the hybrid step), 180 tiles -> 256x256 wins.  At 128 tiles, plain
@@ -2739,23 +2378,21 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         else if (form == MI355_GEMM_NT) cfg = 2;
         else cfg = 3;
     }
-    // the persistent form of tile 2 (hint 7): same bits, no prologue / barrier / workgroup turnover per tile and a quarter of the staging traffic.  Batch 160, isolated:
-    // QKV 890-917 -> 818-825 us, gate-up + SwiGLU 1 489-1 494 -> 1 418-1 422, down dgrad + SwiGLU backward 959-986 -> 920, dqkv dgrad 788-818 -> 756-764.  Chosen by itself from two
-    // rounds of tiles upward (below that every workgroup has one tile and split-K may pay instead)
     const bool persist_ok = form == MI355_GEMM_NT && out_dtype == MI355_DT_BF16 && (epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_SWIGLU_FWD || epilogue == MI355_EPI_SWIGLU_BWD) &&
                             !bias && (K & 63) == 0 && K >= 128 && (N & 7) == 0 && (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && M >= 256 && N >= 256 &&
                             (!residual || ((ldr & 7) == 0 && ((uintptr_t)residual & 15) == 0)) && ldc * 2 * 256 < 0x7fffffffLL && ldr * 2 * 256 < 0x7fffffffLL;
-    if (cfg == 2 && tile_hint == 0 && persist_ok && ((M + 255) / 256) * ((N + 255) / 256) >= persist_min_tiles()) {
+    // four waves of 128x128 (gemm_quad.h), one workgroup per CU walking the tiles from two rounds of them upward: the same bits as tile 2, and 5, whose place they take where they can
+    const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
+    if (tile_hint == 0 && ((cfg == 2 && form == MI355_GEMM_NT) || cfg == 5) && quad_ok(form, p, out_dtype)) {
         const int kind_bit = epilogue == MI355_EPI_SWIGLU_FWD ? 4 : epilogue == MI355_EPI_SWIGLU_BWD ? 8 : residual ? 2 : 1;
-        cfg = (pp_mask() & kind_bit) ? 8 : 7;
-        if (walk_on(N, K)) p.ablate |= 8;
+        cfg = persist_ok && tiles256 >= persist_min_tiles() && (pp_mask() & kind_bit) ? 8 : 7;
     }
     // A last round of few 256x256 tiles costs as much as a full one.  Where they are few -- one to three full rounds and a remainder that 128x128 tiles (split over K as ever)
     // cover with at most one workgroup per CU -- the row panels of the full rounds go first and the remaining rows follow on the small tiles.  17 016 rows (24 samples of 709
     // tokens), N = 1024 (268 tiles), us, one launch -> two: K = 2048 109 -> 76, 3072 150 -> 102, 4096 187 -> 127, 6144 278 -> 182; N = 2048 (536 tiles) 82 -> 74; 25 216 rows,
     // N = 768 (297 tiles): K = 768 53 -> 42, 3072 147 -> 119.  Four rounds and more gain nothing (1072 tiles 131 / 132) or lose (1188 tiles 109 / 118: a remainder of 648 small tiles).
     if (tile_hint == 0 && ablate == 0 && !split3 && form != MI355_GEMM_TN && (cfg == 2 || cfg == 3 || cfg == 7)) {
-        const int64_t tn = (N + 255) / 256, tiles256 = ((M + 255) / 256) * tn, rounds = tiles256 / 256, m_main = rounds * 256 / tn * 256;
+        const int64_t tn = (N + 255) / 256, rounds = tiles256 / 256, m_main = rounds * 256 / tn * 256;
         const int64_t tail128 = ((M - m_main + 127) / 128) * ((N + 127) / 128), most[4] = {0, 256, 160, 128};
         if (rounds >= 1 && rounds <= 3 && tiles256 % 256 != 0 && m_main >= 256 && m_main < M && tail128 <= most[rounds]) {
             const int64_t esz = out_dtype == MI355_DT_F32 ? 4 : 2, rsz = epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_GELU_ERF ? esz : 2;
@@ -2769,8 +2406,8 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         cfg = 7;
     }
     if (cfg == 7) {
-        const bool ok = persist_ok;
-        if (ok) return mi355_gemm_persist_part2(&p, s);
+        const bool persistent = tile_hint == 7 || tiles256 >= persist_min_tiles();
+        if (quad_ok(form, p, out_dtype)) return form == MI355_GEMM_TN ? mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s) : mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s);
         cfg = 2;
     }
     const bool ring_epilogue = epilogue == MI355_EPI_NONE || (out_dtype == MI355_DT_BF16 && epilogue == (form == MI355_GEMM_NT ? MI355_EPI_GELU_ERF : MI355_EPI_SWIGLU_BWD));
@@ -2804,21 +2441,15 @@ extern "C" int mi355_gemm_bf16_attn_delta(int64_t M, int64_t N, int64_t K, const
     p.epilogue = MI355_EPI_ATTN_DELTA; p.tiles_m = p.tiles_n = 0; p.ksplit = 1; p.ws = nullptr; p.ablate = 0;
     p.ad_lse = lse; p.ad_delta = delta; p.ad_nl2 = neg_lse_log2e; p.ad_ndl = neg_delta; p.ad_S = S; p.ad_Hq = Hq;
     p.split3 = 0;
-    // the persistent form (same bits) from two rounds of tiles upward
-    if ((K & 63) == 0 && K >= 128 && ((M + 255) / 256) * ((N + 255) / 256) >= persist_min_tiles() && ldc * 2 * 256 < 0x7fffffffLL && ldctx * 2 * 256 < 0x7fffffffLL) {
-        if ((pp_mask() & 16) && K >= 64 * 5) return mi355_gemm_pp_part6(&p, (hipStream_t)stream);
-        if (walk_on(N, K)) p.ablate |= 8;
-        return mi355_gemm_persist_part2(&p, (hipStream_t)stream);
-    }
+    p.fold = 0;
+    const bool persistent = ((M + 255) / 256) * ((N + 255) / 256) >= persist_min_tiles();
+    if (persistent && (pp_mask() & 16) && (K & 63) == 0 && K >= 64 * 5 && ldc * 2 * 256 < 0x7fffffffLL && ldctx * 2 * 256 < 0x7fffffffLL) return mi355_gemm_pp_part6(&p, (hipStream_t)stream);
+    if (quad_ok(MI355_GEMM_NT, p, MI355_DT_BF16)) return mi355_gemm_quad_nt_part8(&p, MI355_DT_BF16, persistent, (hipStream_t)stream);
     return mi355_gemm_part2(MI355_GEMM_NT, &p, MI355_DT_BF16, nullptr, 0, (hipStream_t)stream);
 }
 
-extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint,
-                                       void* stream) {
-    MI355_REQUIRE(form >= 0 && form <= 2, "mi355_gemm_bf16_grouped: bad form %d", form);
-    MI355_REQUIRE(count >= 1 && count <= MAX_GROUP && problems, "mi355_gemm_bf16_grouped: count must be 1..%d", MAX_GROUP);
-    MI355_REQUIRE(out_dtype == MI355_DT_BF16 || out_dtype == MI355_DT_F32, "mi355_gemm_bf16_grouped: bad out_dtype");
-    MI355_REQUIRE(tile_hint == 0 || tile_hint == 1 || tile_hint == 3 || tile_hint == 4 || tile_hint == 5, "mi355_gemm_bf16_grouped: tile_hint must be 0 (auto), 1 (128x128), 3, 4 or 5 (256x256)");
+// tile_hint: as mi355_gemm_bf16_grouped's, or 7 (gemm_quad.h where it takes every problem, else 5)
+static int grouped_launches(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* stream) {
     GroupTable tbl;
     tbl.count = count;
     int64_t tiles256 = 0, longest = 0;
@@ -2831,7 +2462,7 @@ extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_pro
         p.M = q.M; p.N = q.N; p.K = q.K; p.lda = q.lda; p.ldb = q.ldb; p.ldc = q.ldc; p.ldr = q.ldr;
         p.epilogue = MI355_EPI_NONE; p.tiles_m = p.tiles_n = 0; p.ksplit = 1; p.ws = nullptr; p.ablate = 0;
         p.ad_lse = nullptr; p.ad_delta = p.ad_nl2 = p.ad_ndl = nullptr; p.ad_S = p.ad_Hq = 0;
-        p.split3 = 0;
+        p.split3 = 0, p.fold = 0;
         tiles256 += ((q.M + 255) / 256) * ((q.N + 255) / 256);
         longest = q.K > longest ? q.K : longest;
         small |= q.M < 256 || q.N < 256;
@@ -2859,16 +2490,29 @@ extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_pro
                 int n = 0;
                 for (int i = 0; i < count; ++i)
                     if ((int)(best >> i & 1) != rest) part[n++] = problems[i];
-                if (int rc = mi355_gemm_bf16_grouped(form, n, part, out_dtype, rest ? 1 : 5, stream)) return rc;
+                if (int rc = grouped_launches(form, n, part, out_dtype, rest ? 1 : 7, stream)) return rc;
             }
             return 0;
         }
     }
     hipStream_t s = (hipStream_t)stream;
-    if (cfg == 5) return mi355_gemm_grouped_part5(form, &tbl, out_dtype, s);
+    // four waves of 128x128 (gemm_quad.h): the bits of tile 5
+    bool quad = form == MI355_GEMM_TN && (cfg == 7 || (cfg == 5 && tile_hint == 0));
+    for (int i = 0; i < count; ++i) quad = quad && quad_ok(form, tbl.g[i], out_dtype);
+    if (quad) return mi355_gemm_quad_grouped_part9(&tbl, out_dtype, s);
+    if (cfg == 5 || cfg == 7) return mi355_gemm_grouped_part5(form, &tbl, out_dtype, s);
     if (cfg == 4) return mi355_gemm_grouped_part4(form, &tbl, out_dtype, s);
     if (cfg == 3) return mi355_gemm_grouped_part3(form, &tbl, out_dtype, s);
     return mi355_gemm_grouped_part1(form, &tbl, out_dtype, s);
+}
+
+extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint,
+                                       void* stream) {
+    MI355_REQUIRE(form >= 0 && form <= 2, "mi355_gemm_bf16_grouped: bad form %d", form);
+    MI355_REQUIRE(count >= 1 && count <= MAX_GROUP && problems, "mi355_gemm_bf16_grouped: count must be 1..%d", MAX_GROUP);
+    MI355_REQUIRE(out_dtype == MI355_DT_BF16 || out_dtype == MI355_DT_F32, "mi355_gemm_bf16_grouped: bad out_dtype");
+    MI355_REQUIRE(tile_hint == 0 || tile_hint == 1 || tile_hint == 3 || tile_hint == 4 || tile_hint == 5, "mi355_gemm_bf16_grouped: tile_hint must be 0 (auto), 1 (128x128), 3, 4 or 5 (256x256)");
+    return grouped_launches(form, count, problems, out_dtype, tile_hint, stream);
 }
 
 extern "C" int mi355_colsum(int64_t M, int64_t N, const void* X, int x_dtype, int64_t ldx, float* out, int accumulate,

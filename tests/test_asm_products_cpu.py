@@ -1,4 +1,4 @@
-"""Matrix products issued from asm statements (csrc/attention_generic.hip: add_cols) are invisible to the compiler's hazard recognizer: nothing keeps it from moving an accumulator while
+"""Matrix products issued from asm statements (csrc/attention_generic.hip: add_cols; csrc/gemm_quad.h) are invisible to the compiler's hazard recognizer: nothing keeps it from moving an accumulator while
 a product still writes it, except where the source stands.  So the code that was built is read: behind such a product, on every path, its tile is only accumulated to until the matrix
 pipe has written it."""
 import os
@@ -86,14 +86,16 @@ def test_the_reader_finds_an_early_access():
 
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="no hipcc")
-def test_tiles_of_asm_products_are_read_late_enough(tmp_path):
+@pytest.mark.parametrize("source,define,least", [("attention_generic.hip", [], 9),  # the three kernels at head dim 256, with and without dropout
+                                                 ("gemm.hip", ["-DGEMM_PART=8"], 11), ("gemm.hip", ["-DGEMM_PART=9"], 6)])  # four waves of 128x128 (gemm_quad.h)
+def test_tiles_of_asm_products_are_read_late_enough(tmp_path, source, define, least):
     make = open(os.path.join(CSRC, "Makefile")).read()
     flags = re.search(r"^CXXFLAGS = (.*)$", make, re.M).group(1).replace("$(ARCH)", "gfx950").replace("$(NOPK)", re.search(r"^NOPK = (.*)$", make, re.M).group(1)).split()
-    out = tmp_path / "attention_generic.s"
-    subprocess.run(["hipcc", *flags, "-S", "--cuda-device-only", os.path.join(CSRC, "attention_generic.hip"), "-o", str(out)], check=True, capture_output=True)
+    out = tmp_path / "kernels.s"
+    subprocess.run(["hipcc", *flags, *define, "-S", "--cuda-device-only", os.path.join(CSRC, source), "-o", str(out)], check=True, capture_output=True)
     kernels = re.findall(r"^(_Z\w+):[^\n]*\n(.*?)^\s*\.section\s+\.rodata", out.read_text(), re.S | re.M)
     with_asm = 0
     for name, body in kernels:
         assert not early_accesses(body.splitlines()), name
         with_asm += bool(re.search(r"#ASMSTART[^#]*v_mfma", body))
-    assert with_asm >= 9  # the three kernels at head dim 256, with and without dropout
+    assert with_asm >= least
