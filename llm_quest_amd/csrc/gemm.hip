@@ -1742,8 +1742,9 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
 // 0.75 us, in pairs 1.05 us for both -- each wave waits for its own LDS reads and its own DMA, one K-tile ahead.  Here ONE workgroup of four waves has the CU and all of its LDS: four
 // K-tiles of the BM x 128 output tile, three in flight while one is multiplied, one barrier a K-tile; the fragments of the next half K-tile are read between the products of this one
 // (two register sets), the requests issued there too.  BM = 192 (96 x 64 a wave): 5 664 x 1 024 is 240 tiles, one round of the 256 CUs, where 128 x 128 gave 360 for 2 x 256 places, and LDS and L2 carry a sixth fewer
-// bytes a flop.  What bounds it: the panels' way from L2 to LDS, 13 TB/s over the chip at 0.64 us (BM 128) and 0.76 us (BM 192) a K-tile with
-// every CU at work; alone on the chip a workgroup takes 0.44 and 0.6, its LDS reads and writes 0.4.
+// bytes a flop.  What bounds it: a CU's requests, 64 bytes a clock from L2 to LDS -- 640 (BM 192) of the 768 clocks that a K-tile's products take, 512 of 512 (BM 128) -- beside which the products of one
+// wave per SIMD wait for each other's.  Every instruction in the loop counts (stages, LDS addresses and the edges' masks are out of it); us before that -> now: 333 x 4 096, K = 1 024 12.3 -> 11.0; 996 x 1 024,
+// K = 2 048 19.0 -> 17.0; 5 664 x 1 024, K = 1 024 21.0 -> 19.4, 3 584 49.6 -> 47.4, 8 256 99.8 -> 98.6; NN 333 x 2 048, K = 1 024 13.1 -> 10.5; 996 x 1 024, K = 6 144 27.7 -> 26.9.
 // (The ring is dynamic LDS: told its size, the compiler gives the one wave per SIMD all 512 registers, half of them accumulation registers, and moves the sums back and forth -- 1.4 times
 // the time.)
 // NT and NN forms, plain epilogue (bias and residual allowed).  The bits of gemm_bf16_kernel in as many shares of K: every output is summed over K in the same order.
@@ -1757,7 +1758,7 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
 template <int BM, int OUT_DT, bool FOLD, bool B_TR, int KIND>
 __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     constexpr int BN = 128, NS = 4, FM = BM / 32, FN = 4;
-    constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, A_PPW = A_BYTES / 4096, B_PPW = 4, PPW = A_PPW + B_PPW, STG_LD = 68;
+    constexpr int A_BYTES = BM * 128, STAGE = A_BYTES + BN * 128, A_PPW = A_BYTES / 4096, B_PPW = 4, PPW = A_PPW + B_PPW, HALF = PPW / 2, STG_LD = 68;
     static_assert(A_BYTES % 4096 == 0 && (NS - 1) * PPW <= 63 && FM >= 4, "pieces divide over four waves; the vmcnt field is 6 bits; reads are dealt over four rows of products");
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int lane = threadIdx.x & 63;
@@ -1771,29 +1772,50 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     const int t0 = (int)((int64_t)nt * split / p.ksplit), n = (int)((int64_t)nt * (split + 1) / p.ksplit) - t0;
     const int kend = (int)min(p.K, (int64_t)(t0 + n) * 64);  // K < 2^30: lda >= K, and 256 rows span < 2 GiB
 
+    // Requests: nothing but a place in LDS is computed for one -- rows past the end (NN: of B's K) lie beyond num_records, columns (NN) past the end have the offset OOB, K-tiles past the share's end no
+    // records at all, and what K's remainder leaves out of a row's 64 is masked once, in front of the K-tile that has it.
     unsigned voffA[A_PPW], voffB[B_PPW];
     int kneedA[A_PPW], kneedB[B_PPW];
-    piece_offsets<false, BM, 64, A_PPW>(wave, lane, p.lda, p.M - m0, voffA, kneedA);
-    piece_offsets<B_TR, BN, 64, B_PPW>(wave, lane, p.ldb, p.N - n0, voffB, kneedB);
-    const bf16_t* baseA = uniform_ptr(p.A + m0 * p.lda);
-    const bf16_t* baseB = uniform_ptr(B_TR ? p.B + n0 : p.B + n0 * p.ldb);
-    const int64_t stepB = B_TR ? p.ldb : 1;
-    auto issue = [&](int t, int from, int to) {  // this wave's pieces [from, to) of K-tile t; past the end out of range: zeros, and the counts of the waits below hold
-        const int k0 = t < n ? (t0 + t) * 64 : 0, krem = t < n ? kend - k0 : 0;
-        char* dA = smem + (t & (NS - 1)) * STAGE + wave * A_PPW * 1024;
-        char* dB = smem + (t & (NS - 1)) * STAGE + A_BYTES + wave * B_PPW * 1024;
+    piece_offsets<false, BM, 64, A_PPW>(wave, lane, p.lda, BM, voffA, kneedA);
+    piece_offsets<B_TR, BN, 64, B_PPW>(wave, lane, p.ldb, B_TR ? p.N - n0 : BN, voffB, kneedB);
+    const int64_t stepB = B_TR ? 128 * p.ldb : 128;
+    const char* reqA = (const char*)uniform_ptr(p.A + m0 * p.lda + (int64_t)t0 * 64);
+    const char* reqB = (const char*)uniform_ptr(B_TR ? p.B + (int64_t)t0 * 64 * p.ldb + n0 : p.B + n0 * p.ldb + (int64_t)t0 * 64);
+    const int krem = kend - (t0 + n - 1) * 64;
+    const int recA = (int)(min((int64_t)BM, p.M - m0) * p.lda * 2), recB = (int)((B_TR ? 64 : min((int64_t)BN, p.N - n0)) * p.ldb * 2), recT = B_TR ? (int)(krem * p.ldb * 2 - n0 * 2) : recB;
+    int rq = 0;            // the K-tile requested next
+    auto edge = [&]() {  // the share's last K-tile
+        if (rq != n - 1 || krem == 64) return;
+        asm volatile("");  // (a branch, not selects on every K-tile)
 #pragma unroll
-        for (int j = 0; j < PPW; ++j) {
-            if (j < from || j >= to) continue;
-            if (j < A_PPW) dma_piece(baseA + k0, kneedA[j < A_PPW ? j : 0] < krem ? voffA[j < A_PPW ? j : 0] : OOB, dA + j * 1024);
-            else dma_piece(baseB + k0 * stepB, kneedB[j < A_PPW ? 0 : j - A_PPW] < krem ? voffB[j < A_PPW ? 0 : j - A_PPW] : OOB, dB + (j - A_PPW) * 1024);
+        for (int j = 0; j < A_PPW; ++j) voffA[j] = kneedA[j] < krem ? voffA[j] : OOB;
+        if constexpr (!B_TR) {
+#pragma unroll
+            for (int j = 0; j < B_PPW; ++j) voffB[j] = kneedB[j] < krem ? voffB[j] : OOB;
         }
     };
+    auto advance = [&]() {
+        ++rq;
+        reqA += 128, reqB += stepB;
+        edge();
+    };
+    auto issue = [&](int stage, int j) {  // this wave's piece j of K-tile rq
+        const bool isA = j < A_PPW;
+        char* dst = smem + stage * STAGE + (isA ? (wave * A_PPW + j) * 1024 : A_BYTES + (wave * B_PPW + j - A_PPW) * 1024);
+        if (isA) dma_piece(reqA, voffA[isA ? j : 0], dst, rq < n ? recA : 0);
+        else dma_piece(reqB, voffB[isA ? 0 : j - A_PPW], dst, rq < n ? (rq == n - 1 ? recT : recB) : 0);
+    };
     const int wr0 = (wave >> 1) * (BM / 2), wc0 = (wave & 1) * 64;
-    // the swizzle of a row goes by its last four bits: one lane offset serves every fragment of a half (frag_rowk)
-    const int off0 = (lane & 15) * 128 + (swz_rowk<64>(lane >> 4, lane & 15) << 4), off1 = (lane & 15) * 128 + (swz_rowk<64>(4 + (lane >> 4), lane & 15) << 4);
-    auto frag_a = [&](int t, int off, int i) { return *reinterpret_cast<const bf16x8*>(smem + (t & (NS - 1)) * STAGE + wr0 * 128 + off + i * 2048); };
-    auto frag_b = [&](int t, int off, int j) { return *reinterpret_cast<const bf16x8*>(smem + (t & (NS - 1)) * STAGE + A_BYTES + wc0 * 128 + off + j * 2048); };
+    // the swizzle of a row goes by its last four bits: one lane offset serves every fragment of a half (frag_rowk); a stage's is its own register, so that every read is one instruction
+    unsigned offa[NS], offb[NS];
+#pragma unroll
+    for (int st = 0; st < NS; ++st) {
+        const unsigned at = (unsigned)(uintptr_t)LDS_PTR(smem) + st * STAGE + (lane & 15) * 128 + (swz_rowk<64>(lane >> 4, lane & 15) << 4);
+        offa[st] = at + wr0 * 128, offb[st] = at + A_BYTES + wc0 * 128;
+    }
+    typedef const __attribute__((address_space(3))) bf16x8* lds_frag;
+    auto frag_a = [&](int st, int kk, int i) { return *(lds_frag)(uintptr_t)((offa[st] ^ (kk * 64)) + i * 2048); };
+    auto frag_b = [&](int st, int kk, int j) { return *(lds_frag)(uintptr_t)((offb[st] ^ (kk * 64)) + j * 2048); };
     // B_TR: [64 k][128 columns]; the XOR of a lane's row reaches into the column bits, so each of the wave's four column tiles has a lane offset of its own (frag_tr)
     unsigned offt[FN];
 #pragma unroll
@@ -1801,8 +1823,8 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
         const int g = lane >> 4, q = (lane >> 2) & 3, chunk = ((wc0 >> 3) + 2 * j + ((lane & 3) >> 1)) ^ ((q | ((g & 1) << 2)) << 1);
         offt[j] = (unsigned)(uintptr_t)LDS_PTR(smem) + A_BYTES + (8 * g + q) * 256 + (chunk << 4) + (lane & 1) * 8;
     }
-    auto issue_bt = [&](TrHalves& f, int t, auto kk, int j) {  // the first (kk 0) or second half of K-tile t; read asynchronously: tr_wait_join stands at the end of the same half
-        const unsigned addr = offt[j] + (t & (NS - 1)) * STAGE;
+    auto issue_bt = [&](TrHalves& f, int st, auto kk, int j) {  // the first (kk 0) or second half of the stage; read asynchronously: tr_wait_join stands at the end of the same half
+        const unsigned addr = offt[j] + st * STAGE;
         asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%c3\n\tds_read_b64_tr_b16 %1, %2 offset:%c4"
                      : "=&v"(f.lo), "=&v"(f.hi)
                      : "v"(addr), "i"(decltype(kk)::value * 8192), "i"(decltype(kk)::value * 8192 + 1024));
@@ -1827,25 +1849,24 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
 #pragma unroll
             for (int j = 0; j < FN; ++j) tot[i][j] = (f32x4){0.f, 0.f, 0.f, 0.f};
     }
-    // products of one half K-tile; the reads of the next half (of K-tile t) and the requests for K-tile `next` stand between their rows, in this order: left to itself the compiler puts
-    // the reads behind all products, where nothing covers them, and ten requests in a row hold the one wave of a SIMD up (the second half's requests in front of its products: 5 % more)
-    auto half = [&](const bf16x8 (&a)[FM], const bf16x8 (&b)[FN], int t, auto kk, bf16x8 (&an)[FM], bf16x8 (&bn)[FN], int next) {
-        const int off = decltype(kk)::value ? off1 : off0;
+    // Products of one half K-tile; the reads of the next half (of stage st, k-step kk) behind its first ones, one each, the requests [from, to) for K-tile rq evenly over it, in this order: left to itself
+    // the compiler puts the reads behind all products, where nothing covers them.  One wave per SIMD issues an instruction every four clocks and has nobody to fill in for what it waits for: everything
+    // else is out of the loop, which is four K-tiles long so that stages are constants.
+    auto half = [&](const bf16x8 (&a)[FM], const bf16x8 (&b)[FN], auto st_c, auto kk, bf16x8 (&an)[FM], bf16x8 (&bn)[FN], int qstage, int from, int to) __attribute__((always_inline)) {
+        constexpr int ST = decltype(st_c)::value, KK = decltype(kk)::value, P = FM * FN;
         TrHalves h[FN];
 #pragma unroll
-        for (int i = 0; i < FM; ++i) {
-            if constexpr (B_TR) {  // column fragments first, and nothing requested in front of the last row of products: it covers the wait at the end
-                if (i == 0) {
-#pragma unroll
-                    for (int j = 0; j < FN; ++j) issue_bt(h[j], t, kk, j);
-                } else if (2 * i - 2 < FM) an[2 * i - 2] = frag_a(t, off, 2 * i - 2), an[2 * i - 1] = frag_a(t, off, 2 * i - 1);
-            } else if (i < 2) bn[2 * i] = frag_b(t, off, 2 * i), bn[2 * i + 1] = frag_b(t, off, 2 * i + 1);
-            else if (2 * i - 4 < FM) an[2 * i - 4] = frag_a(t, off, 2 * i - 4), an[2 * i - 3] = frag_a(t, off, 2 * i - 3);
-            if (!B_TR && i == FM - 1 && 2 * i - 2 < FM) an[FM - 2] = frag_a(t, off, FM - 2), an[FM - 1] = frag_a(t, off, FM - 1);
-            __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-            for (int j = 0; j < FN; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);  // lane: four columns of row lane & 15
-            if (next >= 0) issue(next, i * PPW / FM, (i + 1) * PPW / FM);
+        for (int s = 0; s < P; ++s) {
+            const int i = s / FN, j = s % FN;
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[j], a[i], acc[i][j], 0, 0, 0);  // lane: four columns of row lane & 15
+            if (s < FN) {  // column fragments first: the next half starts with all of them
+                if constexpr (B_TR) issue_bt(h[s], ST, kk, s);
+                else bn[s] = frag_b(ST, KK, s);
+            } else if (s < FN + FM) {
+                an[s - FN] = frag_a(ST, KK, s - FN);
+            }
+            const int q0 = from + s * (to - from) / P, q1 = from + (s + 1) * (to - from) / P;
+            if (q1 > q0) issue(qstage, q0);
             __builtin_amdgcn_sched_barrier(0);
         }
         if constexpr (B_TR) {
@@ -1853,34 +1874,51 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
             tr_wait_join<0>(h, bn);
         }
     };
+    using std::integral_constant;
     bf16x8 a0[FM], b0[FN], a1[FM], b1[FN];
+    edge();
 #pragma unroll
-    for (int t = 0; t < NS; ++t) issue(t, 0, PPW);
-    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * PPW) : "memory");
+    for (int t = 0; t < NS; ++t) {
+#pragma unroll
+        for (int j = 0; j < (t < NS - 1 ? PPW : HALF); ++j) issue(t, j);
+        if (t < NS - 1) advance();
+    }
+    asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * PPW + HALF) : "memory");
     __builtin_amdgcn_s_barrier();
     if constexpr (B_TR) {
         TrHalves h[FN];
 #pragma unroll
-        for (int j = 0; j < FN; ++j) issue_bt(h[j], 0, std::integral_constant<int, 0>{}, j);
+        for (int j = 0; j < FN; ++j) issue_bt(h[j], 0, integral_constant<int, 0>{}, j);
         tr_wait_join<0>(h, b0);
     } else {
 #pragma unroll
-        for (int j = 0; j < FN; ++j) b0[j] = frag_b(0, off0, j);
+        for (int j = 0; j < FN; ++j) b0[j] = frag_b(0, 0, j);
     }
 #pragma unroll
-    for (int i = 0; i < FM; ++i) a0[i] = frag_a(0, off0, i);
+    for (int i = 0; i < FM; ++i) a0[i] = frag_a(0, 0, i);
     if constexpr (B_TR) __builtin_amdgcn_s_waitcnt(0xc07f);  // (as at the end of `half`, whose state the loop's top shares)
-    for (int t = 0; t < n; ++t) {
+    using InFlight = integral_constant<int, (NS - 2) * PPW>;
+    auto kstep = [&](auto st_c) __attribute__((always_inline)) {
+        constexpr int ST = decltype(st_c)::value;
         __builtin_amdgcn_sched_barrier(0);
-        half(a0, b0, t, std::integral_constant<int, 1>{}, a1, b1, -1);
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                    // this wave's reads of K-tile t are complete
-        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 2) * PPW) : "memory");  // its pieces of t + 1 have landed
-        __builtin_amdgcn_s_barrier();                                         // ... and every wave's
+        half(a0, b0, st_c, integral_constant<int, 1>{}, a1, b1, (ST + NS - 1) % NS, HALF, PPW);  // (the other pieces of the K-tile that the last half asked for)
+        advance();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                     // this wave's reads of the K-tile are complete
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(InFlight::value) : "memory");  // its pieces of the next one have landed
+        __builtin_amdgcn_s_barrier();                                          // ... and every wave's
         __builtin_amdgcn_sched_barrier(0);
-        half(a1, b1, t + 1, std::integral_constant<int, 0>{}, a0, b0, t + NS);                            // t + NS goes into the stage that t has left
-        if constexpr (FOLD) {
-            if (--left == 0) fold();
-        }
+        half(a1, b1, integral_constant<int, (ST + 1) % NS>{}, integral_constant<int, 0>{}, a0, b0, ST, 0, HALF);  // into the stage that this K-tile has left
+        if (FOLD && --left == 0) fold();
+    };
+    for (int t = 0;; t += NS) {
+        kstep(integral_constant<int, 0>{});
+        if (t + 1 >= n) break;
+        kstep(integral_constant<int, 1>{});
+        if (t + 2 >= n) break;
+        kstep(integral_constant<int, 2>{});
+        if (t + 3 >= n) break;
+        kstep(integral_constant<int, 3>{});
+        if (t + 4 >= n) break;
     }
     if constexpr (FOLD) {
         fold();
@@ -2016,8 +2054,9 @@ int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStr
     constexpr int FUSED = B_TR ? MI355_EPI_SWIGLU_BWD : MI355_EPI_GELU_ERF;
     if (p.epilogue == FUSED) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, FUSED>), grid, dim3(256), lds, s, p);
     else if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
-    else if (BM == 192 || !p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
-    else hipLaunchKernelGGL((gemm_ring_kernel<128, MI355_DT_F32, true, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);  // (192 rows: running sums do not fit the registers)
+    else if constexpr (BM == 192) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);  // (running sums do not fit the registers)
+    else if (!p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
+    else hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, true, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
     if (ksplit > 1) launch_splitk_reduce(p, out_dtype, s);
     MI355_LAUNCH_CHECK("mi355_gemm_bf16(ring)");
     return 0;
