@@ -19,6 +19,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "quad.h"
 
 #define ST(s) ((hipStream_t)(s))
 
@@ -551,6 +552,8 @@ __global__ __launch_bounds__(512, 2) void bgemm_wide_kernel(BgemmArgs p, int bat
         tile(id);
     }
 }
+
+#include "bgemm_quad.h"
 
 // ---- fp32 A times bf16 B on the matrix pipe, with the fp32 product's accuracy.  An fp32 number is the sum of three bf16 numbers exactly (its 24 significant bits cut into three
 // runs of 8 by truncation: no rounding, no overflow; what is lost lies below 2^-133), a product of two bf16 numbers is exact in fp32, and the accumulator is fp32 -- so three
@@ -1115,6 +1118,16 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
         // where the line lies, us, wide / small tiles, K = 1024: 2048 x 4096 (128 wide tiles: half the chip) 40 / 36, 4096 x 4096 46 / 70.  With groups the small kernel's grid is
         // mostly empty and its tiles are no fuller: 640 rows in 16 groups, N = 1024, K = 1792 (72 tiles at most) 32 / 38
         if (vec && K % WK == 0 && wide_tiles >= (grp_offs ? 64 : 160) && wide_tiles <= (1 << 30)) {
+            const int64_t words = c_dt == MI355_DT_F32 ? 4 : 8;  // of 16 bytes
+            // four waves wherever they can: K in pairs of K-tiles, two pairs at least; a panel's weights within a descriptor; the groups in the tables; columns and rows of C in whole 16 bytes.  Faster
+            // at every size that comes this far (bgemm_quad.h); the eight-wave kernel takes the rest
+            if (K % 128 == 0 && K >= 256 && batch <= QUAD_GROUPS && sbn * 2 * 512 < 0x7fffffffLL && (epi >= 2 ? n_out : N) % 8 == 0 && ldc % words == 0 && c_bs % words == 0 && ((uintptr_t)C & 15) == 0) {
+                const unsigned grid = (unsigned)(wide_tiles < 256 ? wide_tiles : 256), lds = QUAD_SMEM + (2 * 256 + 2 * (QUAD_GROUPS + 1)) * 4;
+                if (epi >= 2) bgemm_quad_kernel<true><<<grid, 256, lds, ST(stream)>>>(p, batch, (int)wide_tn);
+                else bgemm_quad_kernel<false><<<grid, 256, lds, ST(stream)>>>(p, batch, (int)wide_tn);
+                MI355_LAUNCH_CHECK("bgemm(four waves)");
+                return 0;
+            }
             bgemm_wide_kernel<<<(unsigned)wide_tiles, 512, 0, ST(stream)>>>(p, batch, (int)wide_tn);
             MI355_LAUNCH_CHECK("bgemm(wide)");
             return 0;

@@ -23,6 +23,7 @@
 #include <type_traits>
 
 #include "common.h"
+#include "quad.h"
 
 namespace {
 

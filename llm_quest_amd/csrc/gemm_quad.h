@@ -17,12 +17,7 @@
 //     (Beside the products of the last and the next K-tile instead of between them: level.  Stores left out: 91.8.)
 // The sum of every output runs over K in the order of gemm_tile's: the same bits.
 
-constexpr int QUAD_PANEL = 16384, QUAD_STAGE = 4 * QUAD_PANEL, QUAD_SMEM = 2 * QUAD_STAGE;
 constexpr int QUAD_RES = 16, QUAD_BIAS = 32;  // added to KIND (MI355_EPI_NONE): residual, bias
-
-// first: the sum starts at the constant 0 (no accumulator is cleared anywhere)
-__device__ __forceinline__ void quad_mma_first(f32x4& c, const bf16x8& a, const bf16x8& b) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, 0" : "=a"(c) : "v"(b), "v"(a)); }
-__device__ __forceinline__ void quad_mma(f32x4& c, const bf16x8& a, const bf16x8& b) { asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+a"(c) : "v"(b), "v"(a)); }
 
 // q, q + G, ... < ntiles: the tiles of this workgroup (CHUNK: in a numbering that deals them over the XCDs).  TR: both operands K-strided (TN), else both K-contiguous (NT).  More than three K-tiles.
 template <bool TR, int OUT_DT, int KIND_, bool CHUNK = true>
@@ -229,45 +224,8 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     };
     auto write_out = [&](auto res_c) __attribute__((always_inline)) {  // (grouped: residual or none, every problem its own)
         constexpr bool ADD_R = decltype(res_c)::value;
-        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' way through the pipe: the compiler does not know that the statements above are products (`value` below stays behind this one: both are volatile)
+        asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' way through the pipe: the compiler does not know that the statements above are products (quad_value stays behind this one: both are volatile)
         const auto rc = __builtin_amdgcn_make_buffer_rsrc(corner_of(p.C, p.ldc), 0, rows * ldc, 0x00020000);
-        auto value = [](const f32x4& c, int e) __attribute__((always_inline)) {  // moved where it is used (left to the compiler the accumulators of many blocks are moved out at once, and spilled)
-            float x;
-            asm volatile("v_accvgpr_read_b32 %0, %1" : "=v"(x) : "a"(c[e]));
-            return x;
-        };
-        auto swap = [](unsigned x, unsigned y, unsigned& lo, unsigned& hi) __attribute__((always_inline)) {
-            const auto s = __builtin_amdgcn_permlane16_swap(x, y, false, false);
-            lo = s[0], hi = s[1];
-        };
-        // rows 0-7 (half 0) or 8-15 of 16: a's in the lanes of bit 3 clear, b's in the others
-        auto rows_of = [](unsigned a, unsigned b, int half) __attribute__((always_inline)) {
-            return (unsigned)(half == 0 ? __builtin_amdgcn_update_dpp((int)a, (int)b, 0x128, 0xf, 0xc, false) : __builtin_amdgcn_update_dpp((int)b, (int)a, 0x128, 0xf, 0x3, false));
-        };
-        auto packed = [&](const f32x4 (&c)[4], u32x4 (&o)[2]) __attribute__((always_inline)) {  // a 16 x 64 block as bf16, o[half]
-            unsigned a[4], b[4];
-#pragma unroll
-            for (int e = 0; e < 2; ++e) {
-                swap(pack_bf2(value(c[0], 2 * e), value(c[0], 2 * e + 1)), pack_bf2(value(c[1], 2 * e), value(c[1], 2 * e + 1)), a[e], a[2 + e]);
-                swap(pack_bf2(value(c[2], 2 * e), value(c[2], 2 * e + 1)), pack_bf2(value(c[3], 2 * e), value(c[3], 2 * e + 1)), b[e], b[2 + e]);
-            }
-#pragma unroll
-            for (int half = 0; half < 2; ++half)
-#pragma unroll
-                for (int e = 0; e < 4; ++e) o[half][e] = rows_of(a[e], b[e], half);
-        };
-        auto spread = [&](const f32x4 (&c)[4], float (&o)[2][8]) __attribute__((always_inline)) {  // the same in fp32
-            unsigned a[8], b[8];
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                swap(__float_as_uint(value(c[0], e)), __float_as_uint(value(c[1], e)), a[e], a[4 + e]);
-                swap(__float_as_uint(value(c[2], e)), __float_as_uint(value(c[3], e)), b[e], b[4 + e]);
-            }
-#pragma unroll
-            for (int half = 0; half < 2; ++half)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) o[half][e] = __uint_as_float(rows_of(a[e], b[e], half));
-        };
         constexpr int NT_STORE = 2;  // non-temporal
         constexpr int BW = B16 ? 8 : 4;  // consecutive columns of a lane
         [[maybe_unused]] float bias[2][QW][BW];
@@ -291,8 +249,8 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                 // column half 0 is u, half 1 the same units' g: u into C[:, unit], g into C[:, N/2 + unit], u silu(g) of the rounded operands into R[:, unit]
                 const auto ra = __builtin_amdgcn_make_buffer_rsrc(corner_of(p.R, p.ldr), 0, rows * ldr, 0x00020000);
                 u32x4 u[2], g[2];
-                packed(acc[ha][0][i], u);
-                packed(acc[ha][1][i], g);
+                quad_packed(acc[ha][0][i], u);
+                quad_packed(acc[ha][1][i], g);
 #pragma unroll
                 for (int half = 0; half < 2; ++half) {
                     u32x4 act;
@@ -313,13 +271,13 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                     for (int w = 0; w < 2; ++w) {
                         float a[4], b[4];
 #pragma unroll
-                        for (int e = 0; e < 4; ++e) a[e] = value(acc[ha][hb][i][2 * w], e), b[e] = value(acc[ha][hb][i][2 * w + 1], e);
+                        for (int e = 0; e < 4; ++e) a[e] = quad_value(acc[ha][hb][i][2 * w], e), b[e] = quad_value(acc[ha][hb][i][2 * w + 1], e);
 #pragma unroll
                         for (int half = 0; half < 2; ++half) {
                             u32x4 o;
 #pragma unroll
                             for (int e = 0; e < 4; ++e) {
-                                float v = __uint_as_float(rows_of(__float_as_uint(a[e]), __float_as_uint(b[e]), half));
+                                float v = __uint_as_float(quad_rows(__float_as_uint(a[e]), __float_as_uint(b[e]), half));
                                 if constexpr (BIAS) v += bias[hb][w][e];
                                 if constexpr (ADD_R) v += __uint_as_float(rv[blk & 1][hb][half][w][e]);
                                 o[e] = __float_as_uint(v);
@@ -329,7 +287,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                     }
                 } else if constexpr (BIAS || ADD_R) {
                     float v[2][8];
-                    spread(acc[ha][hb][i], v);
+                    quad_spread(acc[ha][hb][i], v);
 #pragma unroll
                     for (int half = 0; half < 2; ++half) {
 #pragma unroll
@@ -342,7 +300,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                     }
                 } else {
                     u32x4 o[2];
-                    packed(acc[ha][hb][i], o);
+                    quad_packed(acc[ha][hb][i], o);
 #pragma unroll
                     for (int half = 0; half < 2; ++half) {
                         const unsigned at = vc[hb][0] + (unsigned)((blk * 16 + half * 8) * ldc);
@@ -371,7 +329,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                                 unsigned x, y;
                                 const auto s32 = __builtin_amdgcn_permlane32_swap(__float_as_uint(d), __float_as_uint(d), false, false);
                                 d = __uint_as_float(s32[0]) + __uint_as_float(s32[1]);
-                                swap(__float_as_uint(d), __float_as_uint(d), x, y);
+                                quad_swap(__float_as_uint(d), __float_as_uint(d), x, y);
                                 d = __uint_as_float(x) + __uint_as_float(y);
                                 d += wave_dpp<0x128>(d);
                                 dot[blk][half] = hb == 0 ? d : dot[blk][half] + d;

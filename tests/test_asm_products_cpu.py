@@ -1,6 +1,6 @@
-"""Matrix products issued from asm statements (csrc/attention_generic.hip: add_cols; csrc/gemm_quad.h) are invisible to the compiler's hazard recognizer: nothing keeps it from moving an accumulator while
-a product still writes it, except where the source stands.  So the code that was built is read: behind such a product, on every path, its tile is only accumulated to until the matrix
-pipe has written it."""
+"""Matrix products issued from asm statements (csrc/attention_generic.hip: add_cols; csrc/quad.h) are invisible to the compiler's hazard recognizer: nothing keeps it from moving an accumulator while
+a product still writes it, or an operand into place right before a product that reads it, except where the source stands.  So the code that was built is read: behind such a product, on every path, its
+tile is only accumulated to until the matrix pipe has written it; before it, no vector instruction has written what it reads for two wait states."""
 import os
 import re
 import shutil
@@ -9,6 +9,7 @@ import subprocess
 import pytest
 
 CSRC = os.path.join(os.path.dirname(os.path.dirname(os.path.abspath(__file__))), "llm_quest_amd", "csrc")
+FRESH = 2  # wait states from a vector instruction to a product that reads what it wrote
 WAIT = 19  # wait states from a 16-pass product to any other access of its tile; those here have no more passes
 BRANCH = re.compile(r"^s_(cbranch_\w+|branch)\s+(\S+)")
 
@@ -74,6 +75,39 @@ def early_accesses(body):
     return sorted(bad)
 
 
+def late_operands(body):
+    """(instruction, product) of every vector instruction that writes what an asm product reads less than FRESH wait states later, in the order of the text (a jump spends as many)."""
+    recent, bad, asm = [], [], False
+    for line in body:
+        asm = True if "#ASMSTART" in line else False if "#ASMEND" in line else asm
+        text = line.split(";")[0].strip()
+        if not text or text.startswith(".") or text.endswith(":"):
+            continue
+        op, _, rest = text.partition(" ")
+        named = re.findall(r"[va]\[\d+:\d+\]|[va]\d+|[^,\s]+", rest)
+        written = set()
+        if op.startswith("v_mfma"):
+            if asm:
+                left, read = FRESH, set().union(*(registers(x) for x in named[1:4]))
+                for spent, by, what in reversed(recent):
+                    if left <= 0:
+                        break
+                    if what & read:
+                        bad.append((by, text))
+                    left -= spent
+        elif op.startswith("v_") and named:
+            written = set().union(*(registers(x) for x in named[: 2 if "swap" in op else 1]))
+        recent = recent[-FRESH:] + [(int(rest) + 1 if op == "s_nop" else 1, text, written)]
+    return bad
+
+
+def test_the_reader_finds_a_late_operand():
+    product = [";;#ASMSTART", "v_mfma_f32_16x16x32_bf16 a[0:3], v[0:3], v[4:7], a[0:3]", ";;#ASMEND"]
+    move = "v_accvgpr_read_b32 v5, a40"
+    assert late_operands([move] + product) and late_operands([move, "s_nop 0"] + product) and late_operands([move, "v_add_u32_e32 v9, v9, v8"] + product)
+    assert not late_operands([move, "s_nop 1"] + product) and not late_operands([move] + product[1:2]) and not late_operands(["v_mov_b32_e32 v9, v0"] + product)
+
+
 def test_the_reader_finds_an_early_access():
     """On text: a read right behind a product, one behind enough waits, a tile accumulated to, a read at the top of a loop whose end issues the product."""
     product = [";;#ASMSTART", "v_mfma_f32_32x32x16_bf16 a[0:15], v[0:3], v[4:7], a[0:15]", ";;#ASMEND"]
@@ -87,7 +121,8 @@ def test_the_reader_finds_an_early_access():
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="no hipcc")
 @pytest.mark.parametrize("source,define,least", [("attention_generic.hip", [], 9),  # the three kernels at head dim 256, with and without dropout
-                                                 ("gemm.hip", ["-DGEMM_PART=8"], 11), ("gemm.hip", ["-DGEMM_PART=9"], 6)])  # four waves of 128x128 (gemm_quad.h)
+                                                 ("gemm.hip", ["-DGEMM_PART=8"], 11), ("gemm.hip", ["-DGEMM_PART=9"], 6),  # four waves of 128x128 (gemm_quad.h)
+                                                 ("bgemm.hip", [], 2)])  # (bgemm_quad.h)
 def test_tiles_of_asm_products_are_read_late_enough(tmp_path, source, define, least):
     make = open(os.path.join(CSRC, "Makefile")).read()
     flags = re.search(r"^CXXFLAGS = (.*)$", make, re.M).group(1).replace("$(ARCH)", "gfx950").replace("$(NOPK)", re.search(r"^NOPK = (.*)$", make, re.M).group(1)).split()
@@ -96,6 +131,6 @@ def test_tiles_of_asm_products_are_read_late_enough(tmp_path, source, define, le
     kernels = re.findall(r"^(_Z\w+):[^\n]*\n(.*?)^\s*\.section\s+\.rodata", out.read_text(), re.S | re.M)
     with_asm = 0
     for name, body in kernels:
-        assert not early_accesses(body.splitlines()), name
+        assert not early_accesses(body.splitlines()) and not late_operands(body.splitlines()), name
         with_asm += bool(re.search(r"#ASMSTART[^#]*v_mfma", body))
     assert with_asm >= least
