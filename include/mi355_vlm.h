@@ -87,7 +87,7 @@ int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, in
                     int64_t ldb, void* C, int64_t ldc, int out_dtype, const float* bias, const void* residual,
                     int64_t ldr, int epilogue, void* workspace, int64_t workspace_bytes, int tile_hint, void* stream);
 /* Which kernel mi355_gemm_bf16 takes by itself (tile_hint 0) for the NT form with a plain epilogue: rows | K shares << 8 of the one-round ring of K-tiles (128- or 192-row tiles), 0: another one.
- * may_split: a workspace, no bias, N % 8 == 0, ldc and ldr multiples of 4. */
+ * may_split: a workspace, no bias, N % 8 == 0, ldc and ldr multiples of 4.  (Long sums of those that 256x256 tiles in shares of K are faster at go there instead.) */
 int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes);
 /* The same for the NN form. */
 int mi355_gemm_nn_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes);
@@ -105,6 +105,8 @@ typedef struct mi355_gemm_problem {
     const void* residual; int64_t ldr;
 } mi355_gemm_problem;
 int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* stream);
+/* The same with scratch for shares of K (16-byte aligned, as mi355_gemm_bf16's; NULL: none), which few tiles of long sums are then cut into. */
+int mi355_gemm_bf16_grouped_ws(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* workspace, int64_t workspace_bytes, void* stream);
 
 /* The out-projection's dgrad of an attention block with the attention backward's row constants as its epilogue (replaces the GEMM + the delta pass
  * of mi355_attn_bwd*; reference: autograd of ctx @ out_proj.weight^T followed by the softmax backward's row sums, qwen3_attention.py:123-146):

@@ -20,6 +20,7 @@
 //     bias/GELU/residual fused, or raw fp32 slabs when K is split (few output tiles + long K: weight gradients).
 //   * Workgroup -> tile map: XCD-aware (blocks b and b+8 share an L2) then 3-row super-groups.
 // The large NT products and weight gradients are gemm_quad.h's, the mid-size NT and NN products gemm_ring_kernel's; gemm_tile serves the other forms, fused epilogues and sizes.
+#include <algorithm>
 #include <type_traits>
 
 #include "common.h"
@@ -1610,39 +1611,6 @@ struct GroupTable {
     int count;
 };
 
-#if GEMM_PART >= 8 || !defined(GEMM_PART)
-#include "gemm_quad.h"
-
-// persistent: one workgroup per CU walks its share of the tiles, else a workgroup per tile
-template <bool TR>
-int launch_quad(GemmParams p, int out_dtype, bool persistent, hipStream_t s) {
-    p.tiles_m = (int)((p.M + 255) / 256);
-    p.tiles_n = (int)((p.N + 255) / 256);
-    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n;
-    MI355_REQUIRE(tiles < 0x7fffffffLL / 16, "mi355_gemm_bf16: grid too large");
-    const dim3 grid((unsigned)(persistent && tiles > 256 ? 256 : tiles)), block(256);
-#define QUAD(OUT_, KIND_) gemm_quad_kernel<TR, OUT_, KIND_>
-    void (*kernel)(GemmParams);
-    const bool b16 = out_dtype == MI355_DT_BF16;
-    if constexpr (TR) {
-        if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
-        else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
-    } else {
-        if (p.epilogue == MI355_EPI_SWIGLU_FWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_FWD);
-        else if (p.epilogue == MI355_EPI_SWIGLU_BWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_BWD);
-        else if (p.epilogue == MI355_EPI_ATTN_DELTA) kernel = QUAD(MI355_DT_BF16, MI355_EPI_ATTN_DELTA);
-        else if (p.R && p.bias) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES | QUAD_BIAS) : QUAD(MI355_DT_F32, QUAD_RES | QUAD_BIAS);
-        else if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
-        else if (p.bias) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_BIAS) : QUAD(MI355_DT_F32, QUAD_BIAS);
-        else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
-    }
-#undef QUAD
-    hipLaunchKernelGGL(kernel, grid, block, QUAD_SMEM, s, p);
-    MI355_LAUNCH_CHECK("mi355_gemm_bf16(four waves)");
-    return 0;
-}
-#endif
-
 template <class T, bool A_TR, bool B_TR, int OUT_DT>
 __global__ __launch_bounds__(T::NTHREADS, T::MIN_WAVES) void gemm_grouped_kernel(GroupTable tbl) {
     __shared__ __attribute__((aligned(16))) char smem[T::SMEM];
@@ -1737,6 +1705,61 @@ int launch(GemmParams p, int out_dtype, void* workspace, int64_t workspace_bytes
     MI355_LAUNCH_CHECK("mi355_gemm_bf16");
     return 0;
 }
+
+#if GEMM_PART >= 8 || !defined(GEMM_PART)
+#include "gemm_quad.h"
+
+void launch_quad_fold(GroupTable& tbl, int out_dtype, hipStream_t s) {
+    int64_t groups = 0, blocks = 0;
+    for (int i = 0; i < tbl.count; ++i) groups += tbl.g[i].M * tbl.g[i].N / 4;
+    const bool wide = groups >= 4 * 256 * 1024;  // four a thread as soon as that leaves four blocks a CU
+    for (int i = 0; i < tbl.count; ++i) {
+        tbl.start[i] = (int)blocks;
+        blocks += (tbl.g[i].M * tbl.g[i].N / 4 + (wide ? 1023 : 255)) / (wide ? 1024 : 256);
+    }
+    for (int i = tbl.count; i <= MAX_GROUP; ++i) tbl.start[i] = (int)blocks;
+    const bool b16 = out_dtype == MI355_DT_BF16;
+    void (*kernel)(GroupTable) = wide ? (b16 ? quad_fold_kernel<MI355_DT_BF16, 4> : quad_fold_kernel<MI355_DT_F32, 4>) : b16 ? quad_fold_kernel<MI355_DT_BF16, 1> : quad_fold_kernel<MI355_DT_F32, 1>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)blocks), dim3(256), 0, s, tbl);
+}
+
+// persistent: one workgroup per CU walks its share of the tiles, else a workgroup per tile
+template <bool TR>
+int launch_quad(GemmParams p, int out_dtype, bool persistent, hipStream_t s) {
+    p.tiles_m = (int)((p.M + 255) / 256);
+    p.tiles_n = (int)((p.N + 255) / 256);
+    const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * p.ksplit;
+    MI355_REQUIRE(tiles < 0x7fffffffLL / 16, "mi355_gemm_bf16: grid too large");
+    const dim3 grid((unsigned)(persistent && tiles > 256 ? 256 : tiles)), block(256);
+#define QUAD(OUT_, KIND_) gemm_quad_kernel<TR, OUT_, KIND_>
+    void (*kernel)(GemmParams);
+    const bool b16 = out_dtype == MI355_DT_BF16;
+    if (p.ksplit > 1) {
+        kernel = QUAD(MI355_DT_F32, QUAD_SPLIT);
+    } else if constexpr (TR) {
+        if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
+        else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
+    } else {
+        if (p.epilogue == MI355_EPI_SWIGLU_FWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_FWD);
+        else if (p.epilogue == MI355_EPI_SWIGLU_BWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_BWD);
+        else if (p.epilogue == MI355_EPI_ATTN_DELTA) kernel = QUAD(MI355_DT_BF16, MI355_EPI_ATTN_DELTA);
+        else if (p.R && p.bias) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES | QUAD_BIAS) : QUAD(MI355_DT_F32, QUAD_RES | QUAD_BIAS);
+        else if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
+        else if (p.bias) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_BIAS) : QUAD(MI355_DT_F32, QUAD_BIAS);
+        else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
+    }
+#undef QUAD
+    hipLaunchKernelGGL(kernel, grid, block, QUAD_SMEM, s, p);
+    if (p.ksplit > 1) {
+        GroupTable one;
+        one.count = 1;
+        for (int i = 0; i < MAX_GROUP; ++i) one.g[i] = p;
+        launch_quad_fold(one, out_dtype, s);
+    }
+    MI355_LAUNCH_CHECK("mi355_gemm_bf16(four waves)");
+    return 0;
+}
+#endif
 
 // ---------------------------------------------------------------------------------------------- mid-size NT products: one workgroup per CU, a ring of four K-tiles
 // Products of too few 256x256 tiles (under half of the CUs) used to run on Cfg128, whose workgroups only reach the matrix pipe's rate in pairs: alone on a CU a K-tile of 64 took
@@ -2104,8 +2127,15 @@ int launch_quad_grouped(GroupTable& tbl, int out_dtype, hipStream_t s) {
         MI355_REQUIRE(total < 0x7fffffffLL / 16, "mi355_gemm_bf16_grouped: grid too large");
     }
     for (int i = tbl.count; i <= MAX_GROUP; ++i) tbl.start[i] = (int)total;
-    if (out_dtype == MI355_DT_BF16) hipLaunchKernelGGL(gemm_quad_grouped_kernel<MI355_DT_BF16>, dim3((unsigned)total), dim3(256), QUAD_SMEM, s, tbl);
-    else hipLaunchKernelGGL(gemm_quad_grouped_kernel<MI355_DT_F32>, dim3((unsigned)total), dim3(256), QUAD_SMEM, s, tbl);
+    const int shares = tbl.g[0].ksplit;
+    if (shares > 1) {
+        hipLaunchKernelGGL((gemm_quad_grouped_kernel<MI355_DT_F32, true>), dim3((unsigned)(total * shares)), dim3(256), QUAD_SMEM, s, tbl);
+        launch_quad_fold(tbl, out_dtype, s);
+    } else if (out_dtype == MI355_DT_BF16) {
+        hipLaunchKernelGGL((gemm_quad_grouped_kernel<MI355_DT_BF16, false>), dim3((unsigned)total), dim3(256), QUAD_SMEM, s, tbl);
+    } else {
+        hipLaunchKernelGGL((gemm_quad_grouped_kernel<MI355_DT_F32, false>), dim3((unsigned)total), dim3(256), QUAD_SMEM, s, tbl);
+    }
     MI355_LAUNCH_CHECK("mi355_gemm_bf16_grouped(four waves)");
     return 0;
 }
@@ -2310,13 +2340,13 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
-static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold) {
+static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold, double& least) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
     if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
     // fp32 results show the length of their sums: those are no longer than Cfg128's, whose shares the workgroups of 128 rows may also take one after the other (FOLD)
     const int shares = out_dtype == MI355_DT_F32 && may_split ? choose_ksplit((M + 127) / 128 * tn, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes) : 1;
     int rows = 0;
-    double least = 0;
+    least = 0;
     for (int r = 128; r <= 192; r += 64) {
         const int64_t tiles = (M + r - 1) / r * tn;
         for (int64_t ks = r == 192 ? shares : 1; ks * tiles <= 256 && ks <= 16 && (ks == 1 || (may_split && nt >= 32 && ks * M * N * 4 <= ws_bytes)); ++ks) {
@@ -2332,15 +2362,59 @@ static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype,
     return rows;
 }
 
+// Shares of K for `tiles` 256x256 tiles (of `outputs` outputs in all) of gemm_quad.h, too few of them to fill the chip: the number with the least time, which is a K-tile's (1.05 us in a short sum; in a long
+// one the board's power limit sets it, 0.35 + 1.08 times the part of the CUs that work), 12 us for the launches and the first round's write-out, 8 for another one's, and the slabs' way at 6 TB/s.
+// 1: none is 3 % and 4 us better than `now`.  Fitted and checked on: us, without shares -> here (share count)
+//   NT by 1 024: 5 664 rows, K = 248 320 2 751 -> 2 033 (8), 16 384 186 -> 162 (2), 8 256 96 / 101 (not taken); 8 192 rows, K = 16 384 274 -> 203 (2), 3 072 53 / 60; 12 288 rows (192 tiles),
+//   K = 151 936 2 715 -> 2 530 (4);
+//   TN, 25 216 tokens, fp32: 3 072 x 768 168 -> 104 (7), 2 304 x 768 134 -> 84 (9), 768 x 768 54 / 55; a ViT block's four together (108 tiles) 406 -> 287 (2); 8 192 tokens 124 -> 104, 4 096 64 / 66;
+//   TN groups, bf16, 5 664 / 16 384 tokens: 16 tiles 61 -> 33 / 168 -> 55 (8), 48 62 -> 50 / 169 -> 94 (5), 64 63 -> 57 / 170 -> 112 (4), 80 81 -> 65 / 219 -> 136 (3), 96 82 -> 73 / 232 -> 174 (2),
+//   128 91 -> 89 / 295 -> 221 (2).
+// fp32 results show the length of their sums: `least` is the number of shares that they have now.
+static int quad_shares(int64_t tiles, int64_t outputs, int64_t K, int least, int64_t ws_bytes, double now) {
+    const int64_t nt = (K + 63) / 64;
+    int best = 1;
+    double best_us = std::min(0.97 * now, now - 4);
+    for (int s = least > 2 ? least : 2; s <= 16 && s * outputs * 4 <= ws_bytes; ++s) {
+        const int64_t share = quad_share(K, s), rounds = (tiles * s + 255) / 256;
+        if (nt - (s - 1) * share < 3) continue;  // (the last one's, made even: four K-tiles at least)
+        const double filled = (double)(tiles * s) / (double)(rounds * 256), hot = std::max(1.0, 0.35 + 1.08 * filled), length = std::min(1.0, std::max(0.0, (double)(rounds * share - 40) / 80));
+        const double us = (double)(rounds * share) * (1.05 + (hot - 1.05) * length) + 4 + 8.0 * (double)rounds + (double)(s * outputs) * 8 / 6e6;
+        if (us < best_us) best_us = us, best = s;
+    }
+    return best;
+}
+
+// the same of one plain product (NT, TN) that the automatic choice is about to give to other tiles
+static int quad_shares_of(int form, int64_t M, int64_t N, int64_t K, int out_dtype, int64_t ws_bytes) {
+    const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), nt = (K + 63) / 64, t128 = ((M + 127) / 128) * ((N + 127) / 128);
+    if (form == MI355_GEMM_NN || M < 256 || N < 256 || tiles >= 256 || nt < 64) return 1;
+    const int ks = choose_ksplit(t128, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes);
+    const int64_t rounds = (t128 * ks + 255) / 256;
+    double now = 4 + (double)(rounds * ((nt + ks - 1) / ks)) * (rounds == 1 ? 0.67 : 0.49) + (ks > 1 ? 3 + (double)(ks * M * N) * 8 / 4.5e6 : 0);  // 128x128, two a CU
+    int least = ks;
+    if (form == MI355_GEMM_NT) {
+        int ksplit, fold;
+        double us;
+        if (!small_tiles(form, M, N, MI355_EPI_NONE)) now = 12 + (double)nt * (0.35 + 1.08 * (double)tiles / 256), least = 1;
+        else if (choose_ring(form, M, N, K, out_dtype, true, ws_bytes, ksplit, fold, us)) now = 0.94 * us;  // (at long sums that is 5 % too much)
+    } else if (tiles > 128 && M * N > 5 * 1024 * 1024) {
+        now = 12 + (double)nt * (0.35 + 1.08 * (double)tiles / 256), least = 1;
+    }
+    return quad_shares(tiles, M * N, K, out_dtype == MI355_DT_F32 ? least : 1, ws_bytes, now);
+}
+
 // input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
 // 128x128 / 256x256: K = 248 320, 333 rows 294 / 304, 602 585 / 446, 2 048 1 298 / 1 092; K = 20 000, 708 rows 54 / 57, 1 300 88 / 82; by 768, K = 50 256, 602 rows 83 / 81
 static bool long_split_nn(int64_t M, int64_t N, int64_t K, bool may_split, int64_t workspace_bytes) {
     return may_split && !(N & 7) && workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
 }
 
+// (what gemm_ring_kernel would take: of those, gemm_quad.h takes the ones that are faster in its shares of K)
 static int ring_query(int form, int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) {
     int ksplit = 1, fold;
-    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(form, M, N, MI355_EPI_NONE) ? choose_ring(form, M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit, fold) : 0;
+    double us;
+    const int rows = M > 0 && N > 0 && K > 0 && small_tiles(form, M, N, MI355_EPI_NONE) ? choose_ring(form, M, N, K, out_dtype, may_split != 0, workspace_bytes, ksplit, fold, us) : 0;
     return rows ? rows | ksplit << 8 : 0;
 }
 extern "C" int mi355_gemm_nt_ring(int64_t M, int64_t N, int64_t K, int out_dtype, int may_split, int64_t workspace_bytes) { return ring_query(MI355_GEMM_NT, M, N, K, out_dtype, may_split, workspace_bytes); }
@@ -2407,7 +2481,11 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         if (M < 256 || N < 256) cfg = 1;
         else if (long_split && tiles256 < 128) cfg = 3;
         else if (small_tiles(form, M, N, epilogue)) cfg = 1;
-        // weight gradients: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Batch 160:
+        // weight gradients that gemm_quad.h takes: two 128x128 tiles per CU up to half of the CUs' worth of 256x256 ones, else those.  us, the choice before (in brackets its tile) -> here: 151 936 x 1 024,
+        // 197 tokens 142 (2) -> 106, 333 181 (1) -> 138, 602 250 (3) -> 196, 1 000 354 (3) -> 275; 248 320 x 1 024, 333 tokens 294 (3) -> 212; 50 256 x 768, 602 80 (1) -> 59; 12 288 x 1 024, 200 16 (1)
+        // -> 12, 900 37 (1) -> 26; 144 tiles, 512 tokens 21.5 (1) -> 16, 1 024 34 (1) -> 25, 3 072 86 (1) -> 60.  Not at 128 tiles: 200 11.0 / 11.4, 602 17.1 / 17.5, 2 048 38.5 / 39.6; 64: 8.5 / 11.4, 17 / 23
+        else if (form == MI355_GEMM_TN && quad_ok(form, p, out_dtype)) cfg = M * N <= 5 * 1024 * 1024 || tiles256 <= 128 ? 1 : 7;
+        // those that it does not: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)
         // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,
         // which the four waves have no partner to hide (151 936 x 1 024, tile 5 / 3 / 1: 61 tokens 117 / 96 / 100, 333 196 / 174 / 200, 602 259 / 248 / 275, 1 024 367 / 374 / 398;
@@ -2426,6 +2504,11 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     if (tile_hint == 0 && ((cfg == 2 && form == MI355_GEMM_NT) || cfg == 5) && quad_ok(form, p, out_dtype)) {
         const int kind_bit = epilogue == MI355_EPI_SWIGLU_FWD ? 4 : epilogue == MI355_EPI_SWIGLU_BWD ? 8 : residual ? 2 : 1;
         cfg = persist_ok && tiles256 >= persist_min_tiles() && (pp_mask() & kind_bit) ? 8 : 7;
+    }
+    if (tile_hint == 0 && ablate == 0 && epilogue == MI355_EPI_NONE && !bias && workspace && !(ldc & 3) && (!residual || !(ldr & 3)) && (cfg == 1 || cfg == 7) && quad_ok(form, p, out_dtype)) {
+        p.ksplit = quad_shares_of(form, M, N, K, out_dtype, workspace_bytes), p.ws = (float*)workspace;
+        const bool persistent = tiles256 * p.ksplit >= persist_min_tiles();
+        if (p.ksplit > 1) return form == MI355_GEMM_TN ? mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s) : mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s);
     }
     // A last round of few 256x256 tiles costs as much as a full one.  Where they are few -- one to three full rounds and a remainder that 128x128 tiles (split over K as ever)
     // cover with at most one workgroup per CU -- the row panels of the full rounds go first and the remaining rows follow on the small tiles.  17 016 rows (24 samples of 709
@@ -2454,7 +2537,8 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     if (cfg == 1 && tile_hint == 0 && form != MI355_GEMM_TN && ring_epilogue && !split3 && ablate == 0) {
         int ksplit = 1;
         const bool may_split = epilogue == MI355_EPI_NONE && workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));
-        if (const int rows = choose_ring(form, M, N, K, out_dtype, may_split, workspace_bytes, ksplit, p.fold)) return mi355_gemm_ring_part7(form, &p, out_dtype, rows, ksplit, workspace, s);
+        double us;
+        if (const int rows = choose_ring(form, M, N, K, out_dtype, may_split, workspace_bytes, ksplit, p.fold, us)) return mi355_gemm_ring_part7(form, &p, out_dtype, rows, ksplit, workspace, s);
     }
     switch (cfg) {
         case 2: return mi355_gemm_part2(form, &p, out_dtype, workspace, workspace_bytes, s);
@@ -2488,11 +2572,11 @@ extern "C" int mi355_gemm_bf16_attn_delta(int64_t M, int64_t N, int64_t K, const
     return mi355_gemm_part2(MI355_GEMM_NT, &p, MI355_DT_BF16, nullptr, 0, (hipStream_t)stream);
 }
 
-// tile_hint: as mi355_gemm_bf16_grouped's, or 7 (gemm_quad.h where it takes every problem, else 5)
-static int grouped_launches(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* stream) {
+// tile_hint: as mi355_gemm_bf16_grouped's, 7 (gemm_quad.h where it takes every problem, else 5) or 9 (shares of K or 1)
+static int grouped_launches(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* workspace, int64_t workspace_bytes, void* stream) {
     GroupTable tbl;
     tbl.count = count;
-    int64_t tiles256 = 0, longest = 0;
+    int64_t tiles256 = 0, outputs = 0, longest = 0;
     bool small = false;
     for (int i = 0; i < count; ++i) {
         const mi355_gemm_problem& q = problems[i];
@@ -2504,17 +2588,23 @@ static int grouped_launches(int form, int count, const mi355_gemm_problem* probl
         p.ad_lse = nullptr; p.ad_delta = p.ad_nl2 = p.ad_ndl = nullptr; p.ad_S = p.ad_Hq = 0;
         p.split3 = 0, p.fold = 0;
         tiles256 += ((q.M + 255) / 256) * ((q.N + 255) / 256);
+        outputs += q.M * q.N;
         longest = q.K > longest ? q.K : longest;
         small |= q.M < 256 || q.N < 256;
     }
     for (int i = count; i < MAX_GROUP; ++i) tbl.g[i] = tbl.g[0];
-    // 256x256 tiles (one workgroup per CU) once they cover most of the chip; otherwise 128x128 (two per CU, 4x the tiles)
-    int cfg = tile_hint ? tile_hint : ((small || tiles256 < 160) ? 1 : (form == MI355_GEMM_TN ? 5 : 3));
+    bool quad = form == MI355_GEMM_TN;
+    for (int i = 0; i < count; ++i) quad = quad && quad_ok(form, tbl.g[i], out_dtype);
+    // 256x256 tiles (one workgroup per CU) once they cover most of the chip -- those of gemm_quad.h more than half of it --; otherwise 128x128 (two per CU, 4x the tiles).  us, 128x128 / gemm_quad.h: 144 tiles,
+    // 250 tokens 14.9 / 11.8, 602 23.5 / 18.1, 1 500 44 / 32; 240 tiles 18 / 13.4, 29 / 21, 57 / 39
+    int cfg = tile_hint ? tile_hint : ((small || tiles256 < (quad ? 129 : 160)) ? 1 : (form == MI355_GEMM_TN ? 5 : 3));
     // Weight gradients whose 256x256 tiles are one round and up to half of a second.  Few tokens: 128x128 tiles, two per CU.  Many: the problems that fill the round best go on it
     // and the others follow on 128x128 tiles, which all have a place at once.  us, one launch on 256x256 / one on 128x128 / two launches: 328 tiles (8 224, 7 168, 3 584 and 2 048 by
     // 1 024) 333 tokens 45 / 39 / 39, 1 024 77 / 67 / 70, 2 048 121 / 109 / 106, 5 664 291 / 282 / 254; 288 tiles 2 048 tokens 114 / 92 / 91, 5 664 271 / 233 / 211; 320 tiles
     // 333 tokens 42 / 33 / 39, 5 664 274 / 241 / 218; 384 tiles 1 500 tokens 93 / 91.  Not below one round (240 tiles, 2 048 tokens 64 / 74) nor from 672 tiles on (197 / 239).
-    if (tile_hint == 0 && cfg == 5 && tiles256 > 256 && tiles256 <= 384 && longest < 2048) cfg = 1;
+    // (The tiles of gemm_quad.h, one launch on 128x128 / one / two: 276 tiles, 250 tokens 22.7 / 24.0 / 21.7, 602 36 / 37 / 32, 1 500 73 / 68 / 60; 332 tiles 26.5 / 23.8 / 23.7, 43 / 38 / 37, 83 / 70 / 69;
+    // 368 tiles, 124 of them in the second, 27 / 24.3 / 24.9, 47 / 37.5 / 38.6, 88 / 72 / 75, 2 048 tokens 116 / 93 / 94, 3 072 166 / 135 / 134.)
+    if (tile_hint == 0 && cfg == 5 && !quad && tiles256 > 256 && tiles256 <= 384 && longest < 2048) cfg = 1;
     if (tile_hint == 0 && cfg == 5 && tiles256 > 256 && tiles256 <= 384) {
         unsigned best = 0;
         int64_t best_tiles = 0;
@@ -2524,21 +2614,31 @@ static int grouped_launches(int form, int count, const mi355_gemm_problem* probl
                 if (pick >> i & 1) t += ((problems[i].M + 255) / 256) * ((problems[i].N + 255) / 256);
             if (t <= 256 && t > best_tiles) best_tiles = t, best = pick;
         }
-        if (best && tiles256 - best_tiles <= 128) {
+        if (best && tiles256 - best_tiles <= (quad && longest < 2048 ? 96 : 128)) {
             mi355_gemm_problem part[MAX_GROUP];
             for (int rest = 0; rest < 2; ++rest) {
                 int n = 0;
                 for (int i = 0; i < count; ++i)
                     if ((int)(best >> i & 1) != rest) part[n++] = problems[i];
-                if (int rc = grouped_launches(form, n, part, out_dtype, rest ? 1 : 7, stream)) return rc;
+                if (int rc = grouped_launches(form, n, part, out_dtype, rest ? 9 : 7, workspace, workspace_bytes, stream)) return rc;
             }
             return 0;
         }
     }
     hipStream_t s = (hipStream_t)stream;
+    if (cfg == 9) cfg = 1;
+    if (form == MI355_GEMM_TN && cfg == 1 && tile_hint != 1 && workspace && !small && tiles256 <= 128 && longest >= 4096) {
+        bool fits = quad;
+        for (int i = 0; i < count; ++i) fits = fits && problems[i].K == longest && !(problems[i].ldc & 3) && (!problems[i].residual || !(problems[i].ldr & 3));
+        const int shares = fits ? quad_shares(tiles256, outputs, longest, 1, workspace_bytes, 4 + (double)((longest + 63) / 64) * (tiles256 <= 64 ? 0.66 : 0.95)) : 1;
+        if (shares > 1) {
+            float* at = (float*)workspace;
+            for (int i = 0; i < count; ++i) tbl.g[i].ksplit = shares, tbl.g[i].ws = at, at += shares * tbl.g[i].M * tbl.g[i].N;
+            return mi355_gemm_quad_grouped_part9(&tbl, out_dtype, s);
+        }
+    }
     // four waves of 128x128 (gemm_quad.h): the bits of tile 5
-    bool quad = form == MI355_GEMM_TN && (cfg == 7 || (cfg == 5 && tile_hint == 0));
-    for (int i = 0; i < count; ++i) quad = quad && quad_ok(form, tbl.g[i], out_dtype);
+    quad = quad && (cfg == 7 || (cfg == 5 && tile_hint == 0));
     if (quad) return mi355_gemm_quad_grouped_part9(&tbl, out_dtype, s);
     if (cfg == 5 || cfg == 7) return mi355_gemm_grouped_part5(form, &tbl, out_dtype, s);
     if (cfg == 4) return mi355_gemm_grouped_part4(form, &tbl, out_dtype, s);
@@ -2546,13 +2646,17 @@ static int grouped_launches(int form, int count, const mi355_gemm_problem* probl
     return mi355_gemm_grouped_part1(form, &tbl, out_dtype, s);
 }
 
-extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint,
-                                       void* stream) {
+extern "C" int mi355_gemm_bf16_grouped_ws(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* workspace, int64_t workspace_bytes, void* stream) {
     MI355_REQUIRE(form >= 0 && form <= 2, "mi355_gemm_bf16_grouped: bad form %d", form);
     MI355_REQUIRE(count >= 1 && count <= MAX_GROUP && problems, "mi355_gemm_bf16_grouped: count must be 1..%d", MAX_GROUP);
     MI355_REQUIRE(out_dtype == MI355_DT_BF16 || out_dtype == MI355_DT_F32, "mi355_gemm_bf16_grouped: bad out_dtype");
     MI355_REQUIRE(tile_hint == 0 || tile_hint == 1 || tile_hint == 3 || tile_hint == 4 || tile_hint == 5, "mi355_gemm_bf16_grouped: tile_hint must be 0 (auto), 1 (128x128), 3, 4 or 5 (256x256)");
-    return grouped_launches(form, count, problems, out_dtype, tile_hint, stream);
+    MI355_REQUIRE(workspace == nullptr || ((uintptr_t)workspace & 15) == 0, "mi355_gemm_bf16_grouped: workspace must be 16-byte aligned");
+    return grouped_launches(form, count, problems, out_dtype, tile_hint, workspace, workspace_bytes, stream);
+}
+
+extern "C" int mi355_gemm_bf16_grouped(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* stream) {
+    return mi355_gemm_bf16_grouped_ws(form, count, problems, out_dtype, tile_hint, nullptr, 0, stream);
 }
 
 extern "C" int mi355_colsum(int64_t M, int64_t N, const void* X, int x_dtype, int64_t ldx, float* out, int accumulate,

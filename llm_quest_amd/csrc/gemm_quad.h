@@ -18,21 +18,28 @@
 // The sum of every output runs over K in the order of gemm_tile's: the same bits.
 
 constexpr int QUAD_RES = 16, QUAD_BIAS = 32;  // added to KIND (MI355_EPI_NONE): residual, bias
+constexpr int QUAD_SPLIT = 64;                // alone: p.ksplit shares of K, each with its own fp32 [M, N] of p.ws (splitk_reduce_kernel adds them up)
 
-// q, q + G, ... < ntiles: the tiles of this workgroup (CHUNK: in a numbering that deals them over the XCDs).  TR: both operands K-strided (TN), else both K-contiguous (NT).  More than three K-tiles.
+// q, q + G, ... < ntiles: the tiles (SPLIT: and shares of K, those of one share after each other) of this workgroup (CHUNK: in a numbering that deals them over the XCDs).  TR: both operands K-strided (TN), else both K-contiguous (NT).  More than three K-tiles.
 template <bool TR, int OUT_DT, int KIND_, bool CHUNK = true>
 __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int G, const int ntiles, char* smem) {
     constexpr int KIND = KIND_ & 15, ADD = KIND_ & ~15;
-    constexpr bool B16 = OUT_DT == MI355_DT_BF16;
+    constexpr bool B16 = OUT_DT == MI355_DT_BF16, SPLIT = ADD == QUAD_SPLIT;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
-    const int nt_all = (int)((p.K + 63) >> 6), nt = nt_all + (nt_all & 1);
+    const int nt_all = (int)((p.K + 63) >> 6), nt_even = nt_all + (nt_all & 1), per = SPLIT ? (int)quad_share(p.K, p.ksplit) : 0;
     constexpr int ESZ = B16 ? 2 : 4;
 
-    // tile number -> its corner: XCD-chunked, row groups under every column panel (six NT, three TN: see gemm_tile)
-    auto origin = [&](int t, int& m0, int& n0) {
+    // tile number -> its corner and first K-tile: XCD-chunked, row groups under every column panel (six NT, three TN: see gemm_tile)
+    auto origin = [&](int t, int& m0, int& n0, int& k0) {
         constexpr int GROUP_M = TR ? 3 : 6;
-        const int pid = CHUNK ? xcd_chunked(t, ntiles) : t, in_group = GROUP_M * p.tiles_n, first_m = (pid / in_group) * GROUP_M, gsz = min(p.tiles_m - first_m, GROUP_M);
+        int pid = CHUNK ? xcd_chunked(t, ntiles) : t;
+        k0 = 0;
+        if constexpr (SPLIT) {
+            const int tiles = p.tiles_m * p.tiles_n, share = pid / tiles;
+            pid -= share * tiles, k0 = share * per;
+        }
+        const int in_group = GROUP_M * p.tiles_n, first_m = (pid / in_group) * GROUP_M, gsz = min(p.tiles_m - first_m, GROUP_M);
         m0 = (first_m + (pid % in_group) % gsz) * 256;
         n0 = ((pid % in_group) / gsz) * 256;
     };
@@ -62,8 +69,9 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     int kreq = 0, recA = 0, recB = 0;
     int tailA = 0, tailB = 0;
     const int tail_at = TR && (p.K & 63) ? nt_all - 1 : -1;  // the K-tile that K ends in
-    auto open = [&](int m0, int n0) {
-        kreq = 0;
+    const int64_t stepA = TR ? 128 * p.lda : 128, stepB = TR ? 128 * p.ldb : 128;
+    auto open = [&](int m0, int n0, int k0) {
+        kreq = k0;
         if constexpr (TR) {
             baseA = (const char*)uniform_ptr(p.A + m0), baseB = (const char*)uniform_ptr(p.B + n0);
             recA = (int)(128 * p.lda), recB = (int)(128 * p.ldb);
@@ -74,8 +82,8 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
             baseA = (const char*)uniform_ptr(p.A + m0 * p.lda), baseB = (const char*)uniform_ptr(p.B + bn0 * p.ldb);
             recA = (int)(min((int64_t)256, p.M - m0) * p.lda * 2), recB = (int)((KIND == MI355_EPI_SWIGLU_FWD ? p.N - bn0 : min((int64_t)256, p.N - bn0)) * p.ldb * 2);
         }
+        if constexpr (SPLIT) baseA += k0 * stepA, baseB += k0 * stepB;
     };
-    const int64_t stepA = TR ? 128 * p.lda : 128, stepB = TR ? 128 * p.ldb : 128;
     auto advance = [&]() {
         ++kreq;
         baseA += stepA, baseB += stepB;
@@ -160,10 +168,10 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
         advance();
     };
 
-    int m0, n0;
-    origin(q, m0, n0);
+    int m0, n0, k0;
+    origin(q, m0, n0, k0);
     if constexpr (!TR) plan(m0, n0);
-    open(m0, n0);
+    open(m0, n0, k0);
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
 #pragma unroll
@@ -198,7 +206,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
         mw = m + wm * 128, nw = SW_FWD ? (n >> 1) + wn * 64 : n + wn * 128;
         rows = (int)max((int64_t)0, min((int64_t)128, p.M - mw));
         const int cols = (int)min((int64_t)128, (SW_FWD ? p.N >> 1 : p.N) - nw);
-        ldc = (int)p.ldc * ESZ, ldr = (int)p.ldr * ESZ;
+        ldc = (int)(SPLIT ? p.N : p.ldc) * ESZ, ldr = (int)p.ldr * ESZ;
 #pragma unroll
         for (int hb = 0; hb < 2; ++hb)
 #pragma unroll
@@ -225,7 +233,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     auto write_out = [&](auto res_c) __attribute__((always_inline)) {  // (grouped: residual or none, every problem its own)
         constexpr bool ADD_R = decltype(res_c)::value;
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' way through the pipe: the compiler does not know that the statements above are products (quad_value stays behind this one: both are volatile)
-        const auto rc = __builtin_amdgcn_make_buffer_rsrc(corner_of(p.C, p.ldc), 0, rows * ldc, 0x00020000);
+        const auto rc = __builtin_amdgcn_make_buffer_rsrc(corner_of(SPLIT ? p.ws + (int64_t)(k0 / max(per, 1)) * p.M * p.N : p.C, SPLIT ? p.N : p.ldc), 0, rows * ldc, 0x00020000);
         constexpr int NT_STORE = 2;  // non-temporal
         constexpr int BW = B16 ? 8 : 4;  // consecutive columns of a lane
         [[maybe_unused]] float bias[2][QW][BW];
@@ -362,15 +370,16 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     ktile(I0{}, std::true_type{}, Cold{});
     ktile(I1{}, std::false_type{}, Cold{});
     for (;;) {
+        const int nt = SPLIT ? min(per, nt_even - k0) : nt_even;
         for (int t = 4; t < nt; t += 2) {
             ktile(I0{}, std::false_type{}, Cold{});
             ktile(I1{}, std::false_type{}, Cold{});
         }
         const int next = q + G;  // the last two K-tiles request the next tile's first two (none: a K-tile past the end, zeros)
-        int m1 = m0, n1 = n0;
+        int m1 = m0, n1 = n0, k1 = k0;
         if (next < ntiles) {
-            origin(next, m1, n1);
-            open(m1, n1);
+            origin(next, m1, n1, k1);
+            open(m1, n1, k1);
         } else {
             kreq = nt_all;
         }
@@ -387,7 +396,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
             write_out(integral_constant<bool, RES>{});
         }
         if (next >= ntiles) break;
-        q = next, m0 = m1, n0 = n1;
+        q = next, m0 = m1, n0 = n1, k0 = k1;
         ktile(I0{}, std::true_type{}, Behind{});
         ktile(I1{}, std::false_type{}, Cold{});
     }
@@ -397,18 +406,69 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
 template <bool TR, int OUT_DT, int KIND>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    quad_tiles<TR, OUT_DT, KIND>(p, blockIdx.x, gridDim.x, p.tiles_m * p.tiles_n, smem);
+    quad_tiles<TR, OUT_DT, KIND>(p, blockIdx.x, gridDim.x, p.tiles_m * p.tiles_n * (KIND == QUAD_SPLIT ? p.ksplit : 1), smem);
 }
 
-// several problems of the TN form in one launch, a workgroup per tile (see gemm_grouped_kernel)
-template <int OUT_DT>
+// several problems of the TN form in one launch, a workgroup per tile, or per tile and share of K (see gemm_grouped_kernel)
+template <int OUT_DT, bool SPLIT>
 __global__ __launch_bounds__(256, 1) void gemm_quad_grouped_kernel(GroupTable tbl) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    const int v = xcd_chunked(blockIdx.x, tbl.start[tbl.count]);
+    const int tiles = tbl.start[tbl.count];
+    int v = xcd_chunked(blockIdx.x, gridDim.x), share = 0;
+    if constexpr (SPLIT) share = v / tiles, v -= share * tiles;
     int g = 0;
 #pragma unroll
     for (int i = 1; i < MAX_GROUP; ++i)
         if (i < tbl.count && v >= tbl.start[i]) g = i;
     const GemmParams p = tbl.g[g];
-    quad_tiles<true, OUT_DT, QUAD_RES, false>(p, v - tbl.start[g], 1 << 30, p.tiles_m * p.tiles_n, smem);
+    quad_tiles<true, OUT_DT, SPLIT ? QUAD_SPLIT : QUAD_RES, false>(p, v - tbl.start[g] + share * p.tiles_m * p.tiles_n, 1 << 30, p.tiles_m * p.tiles_n * (SPLIT ? p.ksplit : 1), smem);
+}
+
+// C = the sum of a problem's shares, in their order (+ R).  U groups of four columns a thread, start[i] the first block of problem i.  Four shares' loads go out before the first is added.
+template <int OUT_DT, int U>
+__global__ __launch_bounds__(256) void quad_fold_kernel(GroupTable tbl) {
+    int g = 0;
+#pragma unroll
+    for (int i = 1; i < MAX_GROUP; ++i)
+        if (i < tbl.count && (int)blockIdx.x >= tbl.start[i]) g = i;
+    const GemmParams p = tbl.g[g];
+    const int64_t all = p.M * p.N, at = ((int64_t)(blockIdx.x - tbl.start[g]) * (256 * U) + threadIdx.x) * 4;
+    f32x4 acc[U];
+    int64_t from[U];  // (past the end: the last group again)
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        from[u] = min(at + u * 1024, all - 4);
+        acc[u] = *reinterpret_cast<const f32x4*>(p.ws + from[u]);
+    }
+    int share = 1;
+    for (; share + 4 <= p.ksplit; share += 4) {
+        f32x4 v[4][U];
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int u = 0; u < U; ++u) v[s][u] = *reinterpret_cast<const f32x4*>(p.ws + (share + s) * all + from[u]);
+#pragma unroll
+        for (int s = 0; s < 4; ++s)
+#pragma unroll
+            for (int u = 0; u < U; ++u) acc[u] += v[s][u];
+    }
+    for (; share < p.ksplit; ++share)
+#pragma unroll
+        for (int u = 0; u < U; ++u) acc[u] += *reinterpret_cast<const f32x4*>(p.ws + share * all + from[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+        if (at + u * 1024 >= all) continue;
+        const int64_t m = (at + u * 1024) / p.N, n = at + u * 1024 - m * p.N;
+        if constexpr (OUT_DT == MI355_DT_BF16) {
+            if (p.R) {
+                const u32x2 r = *reinterpret_cast<const u32x2*>((const bf16_t*)p.R + m * p.ldr + n);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) acc[u][e] += __uint_as_float(e & 1 ? r[e >> 1] & 0xffff0000u : r[e >> 1] << 16);
+            }
+            *reinterpret_cast<u32x2*>((bf16_t*)p.C + m * p.ldc + n) = u32x2{pack_bf2(acc[u][0], acc[u][1]), pack_bf2(acc[u][2], acc[u][3])};
+        } else {
+            if (p.R) acc[u] += *reinterpret_cast<const f32x4*>((const float*)p.R + m * p.ldr + n);
+            *reinterpret_cast<f32x4*>((float*)p.C + m * p.ldc + n) = acc[u];
+        }
+    }
 }

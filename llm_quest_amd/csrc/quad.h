@@ -3,6 +3,7 @@
 #include "common.h"
 
 constexpr int QUAD_PANEL = 16384, QUAD_STAGE = 4 * QUAD_PANEL, QUAD_SMEM = 2 * QUAD_STAGE;
+__host__ __device__ constexpr int64_t quad_share(int64_t K, int ksplit) { return ((K + 63) / 64 + 2 * ksplit - 1) / (2 * ksplit) * 2; }  // K-tiles of one of ksplit shares of K, an even number; the last one's are what is left
 
 // Sums in the accumulation registers: left to itself the compiler moves part of 256 of them back and forth.  B's fragment is the first operand: a lane holds C[row lane & 15][4 (lane >> 4) + e].
 // first: the sum starts at the constant 0 (no accumulator is cleared anywhere)

@@ -25,7 +25,7 @@
 #include "../../include/mi355_vlm.h"
 
 #define WRAP_ENTRIES(E) \
-    E(gemm_bf16) E(gemm_bf16_grouped) E(colsum) E(rmsnorm_fwd) E(rmsnorm_bwd) E(reduce_rows_f32) E(qknorm_rope_fwd) E(qknorm_rope_bwd) E(swiglu_fwd) E(swiglu_bwd) E(attn_fwd) E(attn_bwd_ws) \
+    E(gemm_bf16) E(gemm_bf16_grouped_ws) E(colsum) E(rmsnorm_fwd) E(rmsnorm_bwd) E(reduce_rows_f32) E(qknorm_rope_fwd) E(qknorm_rope_bwd) E(swiglu_fwd) E(swiglu_bwd) E(attn_fwd) E(attn_bwd_ws) \
     E(attn_bwd_qnorm) E(add_f32_to_bf16) E(layernorm_fwd) E(layernorm_bwd_bf16) E(reduce_rows_into) E(gelu_fwd) E(gelu_bwd_colsum) E(copy2d) E(zc_weight) E(headnorm_rope_fwd) E(headnorm_rope_bwd) \
     E(sigmoid_gate_fwd) E(sigmoid_gate_bwd) E(attn_generic_fwd) E(attn_generic_bwd) E(gdn_gates_fwd) E(gdn_gates_bwd) E(causal_conv_silu_fwd) E(causal_conv_silu_bwd) E(l2norm_fwd) E(l2norm_bwd) \
     E(gated_rmsnorm_fwd) E(gated_rmsnorm_bwd) E(gemv_bf16) E(gemv_bf16_f32out) E(hyper_mix) E(bgemm) E(latent_attn) E(qkv_rows_append) E(group_rmsnorm_sum) E(ragged_conv) E(gated_headnorm) E(glu_rows) \
@@ -687,7 +687,10 @@ OP(gemm_grouped, "form", "problems", "tile") {
         need(b.size(!bt) == K && out.shape({M, N}) && out.dtype() == odt && (!r || (r.rows() && r.dtype() == odt && r.shape({M, N}))));
         p[i].M = M, p[i].N = N, p[i].K = K, p[i].A = a.ptr(), p[i].lda = a.ld(), p[i].B = b.ptr(), p[i].ldb = b.ld(), p[i].C = out.ptr(), p[i].ldc = out.ld(), p[i].residual = r.ptr(), p[i].ldr = r.ld();
     }
-    LAUNCH(gemm_bf16_grouped, form, n, p, code(odt), 0);
+    const bool split = at && p[0].K >= kernels_int("GROUP_SPLIT_MIN_K");
+    T ws;
+    if (split) ws = c.workspace(c.from(PyTuple_GET_ITEM(PyList_GET_ITEM(c.v[1], 0), 0)));
+    LAUNCH(gemm_bf16_grouped_ws, form, n, p, code(odt), 0, ws, split ? kernels_int("WS_BYTES") : 0L);
     Py_RETURN_NONE;
 }
 

@@ -31,6 +31,7 @@ _TILE_NT_PLAIN = int(os.environ.get("MI355_GEMM_TILE_NT_PLAIN", "0"))  # profili
 DGRAD_NT = os.environ.get("MI355_DGRAD_NT", "1") != "0"  # 0: dgrad GEMMs in the NN form on the weight as stored (A/B measurements)
 DGRAD_NT_MIN_ROWS = 4096  # below this the transpose pass is not paid back
 _WS = {}
+GROUP_SPLIT_MIN_K = 4096  # grouped weight gradients over fewer tokens need no split-K scratch (csrc/gemm.hip: quad_shares)
 WS_BYTES = 512 << 20  # split-K scratch per device (fp32 slabs of the largest weight-gradient GEMM)
 
 
@@ -222,7 +223,9 @@ def gemm_grouped(form, problems, tile=0):
             if residual.dtype != odt or tuple(residual.shape) != (M, N):
                 raise ValueError("gemm_grouped: residual must match the output's shape and dtype")
             q.residual, q.ldr = residual.data_ptr(), residual.stride(0)
-    L.call("mi355_gemm_bf16_grouped", form, len(problems), _c.addressof(table), L.dt_code(odt), tile or _TILE_BY_FORM[form] or (_TILE_OVERRIDE if _TILE_OVERRIDE in (1, 3, 4, 5) else 0))
+    hint = tile or _TILE_BY_FORM[form] or (_TILE_OVERRIDE if _TILE_OVERRIDE in (1, 3, 4, 5) else 0)
+    split = form == L.GEMM_TN and not hint and table[0].K >= GROUP_SPLIT_MIN_K  # the library may cut few tiles' long sums into shares of K
+    L.call("mi355_gemm_bf16_grouped_ws", form, len(problems), _c.addressof(table), L.dt_code(odt), hint, L.ptr(_workspace(problems[0][0].device)) if split else None, WS_BYTES if split else 0)
 
 
 # Measured (ViT-B/16 training step, B = 256, same box): fused 65.5 ms, separate kernels 64.1 ms -- erf / tanh in the epilogue sit on the tile's critical

@@ -62,3 +62,40 @@ def test_grouped_weight_gradients(tokens, odt):
     K.gemm_grouped(L.GEMM_TN, problems)
     for a, b, out, r in problems:
         assert torch.equal(out, K.gemm(L.GEMM_TN, a, b, out_dtype=odt, residual=r, allow_split_k=False, tile=5))
+
+
+def off(got, want, terms, odt):
+    """Relative error of sums of `terms` products within what fp32 sums (and a bf16 result: eight significant bits) are off by."""
+    got, want = got.double(), want.double()
+    return float((got - want).norm() / want.norm()) < 2**-24 * terms**0.5 + (2**-8 if odt == BF16 else 0)
+
+
+# few tiles of long sums: shares of K, added up by a second kernel.  K = 64 n of every remainder of shares; rows, columns and (TN) K that end inside a tile; one tile in sixteen shares, several rounds of the CUs
+@pytest.mark.parametrize("form,M,N,K_", [("nt", 257, 264, 4096), ("nt", 5664, 1024, 12288), ("nt", 8100, 1024, 8256), ("nt", 300, 520, 16448), ("nt", 12100, 1000, 33024),
+                                         ("tn", 264, 256, 4097), ("tn", 1000, 1288, 8191), ("tn", 3072, 768, 5664), ("tn", 6144, 1024, 5665), ("tn", 2304, 776, 12287)])
+@pytest.mark.parametrize("odt", [BF16, F32])
+@pytest.mark.parametrize("residual", [False, True])
+def test_shares_of_k(form, M, N, K_, odt, residual):
+    A, B = (draw(M, M, K_), draw(N, N, K_)) if form == "nt" else (draw(M, K_, M), draw(N, K_, N))
+    C = torch.full((M + 1, N + 8), 7.0, dtype=odt, device="cuda")
+    r = draw(4, M, N, dtype=odt) if residual else None
+    K.gemm(L.GEMM_NT if form == "nt" else L.GEMM_TN, A, B, out=C[:M, :N], residual=r)
+    assert bool((C[M:] == 7).all()) and bool((C[:, N:] == 7).all())
+    rows = torch.cat([torch.arange(min(64, M)), torch.arange(max(0, M - 64), M)]).cuda()
+    want = A[rows].double() @ B.double().T if form == "nt" else A[:, rows].double().T @ B.double()
+    assert off(C[rows, :N], want + (r[rows].double() if residual else 0), K_, odt)
+
+
+# a block's weight gradients in shares: alone, and behind a first launch that the others fill (332 tiles)
+@pytest.mark.parametrize("tokens,shapes", [(4096, [(512, 512)] * 3), (5664, [(8256, 1024), (1024, 2048), (7168, 1024), (1024, 3584)]), (8191, [(2304, 768), (768, 776), (3072, 768)])])
+@pytest.mark.parametrize("odt", [BF16, F32])
+def test_shares_of_grouped_weight_gradients(tokens, shapes, odt):
+    problems = []
+    for i, (m, n) in enumerate(shapes):
+        C = torch.full((m + 1, n + 8), 7.0, dtype=odt, device="cuda")
+        problems.append((draw(i, tokens, m), draw(i + 9, tokens, n), C[:m, :n], draw(5, m, n, dtype=odt) if i == 1 else None, C))
+    K.gemm_grouped(L.GEMM_TN, [q[:4] for q in problems])
+    for a, b, c, r, whole in problems:
+        assert bool((whole[c.shape[0] :] == 7).all()) and bool((whole[:, c.shape[1] :] == 7).all())
+        want = a[:, -96:].double().T @ b.double()
+        assert off(c[-96:], want + (r[-96:].double() if r is not None else 0), tokens, odt)
