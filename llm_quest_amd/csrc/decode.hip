@@ -35,6 +35,10 @@ __device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8]) {
 // activation is the epilogue -- eight up rows and their gate rows make a group; every activation is worked out once, not once a workgroup.
 // Bound: a launch of a few MB is a chain of memory round trips (operand rows, row sums, weights, results), so the weights' trip runs under the operands': loads return in
 // order, hence operand loads first, weights behind them, and the next 16 rows' weights under this one's products.
+// EVEN: the waves' runs are whole chunks of T steps and end with K: no load has a condition (a branch, a select and an address of its own each: 28 of them in front of the first
+// product were 1 us of a launch), operand rows past the last one are that row again, and what they give is not stored.  us, six rows, weights from memory, before -> EVEN: RMSNorm + 4096 x
+// 1024 6.9 -> 5.8, RMSNorm + SwiGLU of 6144 x 1024 7.9 -> 7.5, 1024 x 3072 5.3 -> 4.9, 1024 x 2048 4.6 -> 4.2.  One row (gemv_one_kernel, T strips of 512 k): 4.9 -> 4.4, 5.2 -> 4.6,
+// 3.8 -> 3.5.  T 4 or 8: chunks of 7 steps (K = 3584) gain nothing, nor do 384 workgroups for 384 groups.
 constexpr int GEMV_STEPS = 8;  // of 32 k in flight per wave: 8 x 16 bytes a lane
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
     u32x4 o;
@@ -44,14 +48,14 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
 }
 __device__ __forceinline__ float rbf(float x) { return bf2f(f2bf(x)); }
 
-template <int NW, int PRO, bool F32, bool GLU, int ROWS>
+template <int NW, int PRO, bool F32, bool GLU, int ROWS, int T, bool EVEN>
 __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, int steps, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ nw, float eps,
                                                        const bf16_t* __restrict__ W, int64_t ldw, void* __restrict__ y, int64_t ldy, const void* __restrict__ res, int64_t ldr) {
-    constexpr int T = GEMV_STEPS;
+    static_assert(!EVEN || (PRO != 2 && NW * T % 16 == 0), "whole strips of 512 k");
     __shared__ float rs[8];
     __shared__ __attribute__((aligned(16))) float part[2][NW][8][16];
     __shared__ __attribute__((aligned(16))) bf16_t act[PRO == 2 ? NW : 1][8][PRO == 2 ? 32 * T + 8 : 8];  // PRO 2: a wave's run of the activated rows
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, r16 = lane & 15, kg = (lane >> 4) * 8;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), r16 = lane & 15, kg = (lane >> 4) * 8;
     const int nvec = K >> 3, chunks = (steps + T - 1) / T;
     const int k_lo = wave * steps * 32, k_hi = min(K, k_lo + steps * 32);
     constexpr int GN = GLU ? 8 : ROWS;  // columns of a group
@@ -68,6 +72,13 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
                 xf[t] = in ? *reinterpret_cast<const u32x4*>(x + m * ldx + k) : z4;
                 gf[t] = in ? *reinterpret_cast<const u32x4*>(x + m * ldx + K + k) : z4;
             }
+        } else if constexpr (EVEN) {
+            const bf16_t *row = x + min(r16, M - 1) * ldx + k_lo + c * T * 32 + kg, *g = nw + k_lo + c * T * 32 + kg;
+#pragma unroll
+            for (int t = 0; t < T; ++t) {
+                xf[t] = *reinterpret_cast<const u32x4*>(row + t * 32);
+                if constexpr (PRO == 1) gf[t] = *reinterpret_cast<const u32x4*>(g + t * 32);
+            }
         } else {
 #pragma unroll
             for (int t = 0; t < T; ++t) {
@@ -81,6 +92,13 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
     auto request_w = [&](u32x4 (&w)[T], int64_t g, int c) {
         const int64_t n = g * GN + (r16 & (GN - 1));
         const bf16_t* row = W + ((n < N ? n : N - 1) + (GLU && r16 >= 8 ? N : 0)) * ldw;
+        if constexpr (EVEN) {
+            if (!on) return;
+            row += k_lo + c * T * 32 + kg;
+#pragma unroll
+            for (int t = 0; t < T; ++t) w[t] = *reinterpret_cast<const u32x4*>(row + t * 32);
+            return;
+        }
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const int k = k_lo + (c * T + t) * 32 + kg;
@@ -97,7 +115,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
                 unpack8(gf[t], b);
 #pragma unroll
                 for (int e = 0; e < 8; ++e) o[e] = a[e] * r * b[e];
-                xf[t] = r16 < M ? pack8(o) : z4;
+                xf[t] = EVEN || r16 < M ? pack8(o) : z4;
             }
         } else if constexpr (PRO == 2) {
 #pragma unroll
@@ -117,17 +135,21 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
         }
     };
     int64_t g = blockIdx.x;
+    if constexpr (EVEN && ROWS == 8) {
+#pragma unroll
+        for (int t = 0; t < T; ++t) w0[t] = w1[t] = z4;
+    }
     if constexpr (PRO == 1) {  // row sums: rows wave, wave + NW
         u32x4 v0[4];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v0[i] = wave < M && lane + 64 * i < nvec ? *reinterpret_cast<const u32x4*>(x + wave * ldx + (lane + 64 * i) * 8) : z4;
+        for (int i = 0; i < 4; ++i) v0[i] = wave < M && (EVEN ? 0 : lane) + 64 * i < nvec ? *reinterpret_cast<const u32x4*>(x + wave * ldx + (lane + 64 * i) * 8) : z4;
         request_x(0);
         request_w(w0, g, 0);
         for (int m = wave; m < M; m += NW) {
             float ss = 0.f, v[8];
 #pragma unroll
             for (int i = 0; i < 4; ++i)
-                if (lane + 64 * i < nvec) {
+                if ((EVEN ? 0 : lane) + 64 * i < nvec) {
                     unpack8(m == wave ? v0[i] : *reinterpret_cast<const u32x4*>(x + m * ldx + (lane + 64 * i) * 8), v);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
@@ -240,20 +262,20 @@ __device__ __forceinline__ void fold_splits8(const SplitRow& fold, int k, float 
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = out[e] / lg;
 }
-template <int T, int PRO, bool F32, bool GLU>
+template <int T, int PRO, bool F32, bool GLU, bool EVEN>
 __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const bf16_t* __restrict__ x, const bf16_t* __restrict__ nw, float eps, const bf16_t* __restrict__ W, int64_t ldw,
                                                        void* __restrict__ y, const void* __restrict__ res, SplitRow fold) {
     extern __shared__ __attribute__((aligned(16))) bf16_t act[];  // PRO 2, 3: [K]
     constexpr int C = GLU ? 2 : 1;  // columns of a wave; T strips in registers (the smallest of 2, 4, 8 that holds the row; longer rows go through eight at a time)
-    const int lane = threadIdx.x & 63, its = (K + 511) >> 9;
+    const int lane = threadIdx.x & 63, its = EVEN ? T : (K + 511) >> 9;
     const u32x4 z4 = {0u, 0u, 0u, 0u};
     u32x4 xr[T], nr[PRO == 1 ? T : 1], w[C][T];
     auto request_x = [&](int base) {
 #pragma unroll
         for (int t = 0; t < T; ++t) {
             const int k = (base + t) * 512 + lane * 8;
-            xr[t] = k < K ? *reinterpret_cast<const u32x4*>((PRO >= 2 ? act : x) + k) : z4;
-            if constexpr (PRO == 1) nr[t] = k < K ? *reinterpret_cast<const u32x4*>(nw + k) : z4;
+            xr[t] = EVEN || k < K ? *reinterpret_cast<const u32x4*>((PRO >= 2 ? act : x) + k) : z4;
+            if constexpr (PRO == 1) nr[t] = EVEN || k < K ? *reinterpret_cast<const u32x4*>(nw + k) : z4;
         }
     };
     auto request_w = [&](int64_t n, int base) {
@@ -262,7 +284,7 @@ __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const b
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 const int k = (base + t) * 512 + lane * 8;
-                w[c][t] = k < K ? *reinterpret_cast<const u32x4*>(W + (n + c * N) * ldw + k) : z4;
+                w[c][t] = EVEN || k < K ? *reinterpret_cast<const u32x4*>(W + (n + c * N) * ldw + k) : z4;
             }
     };
     float r = 0.f;
@@ -312,7 +334,7 @@ __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const b
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
         }
-        for (int k = T * 512 + lane * 8; k < K; k += 512) {
+        for (int k = T * 512 + lane * 8; !EVEN && k < K; k += 512) {
             unpack8(*reinterpret_cast<const u32x4*>(x + k), v);
 #pragma unroll
             for (int e = 0; e < 8; ++e) ss += v[e] * v[e];
@@ -708,7 +730,7 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(const float* __restric
 // eight would take a second chunk and half of it empty (K of 2 049 to 3 072): its operands are only requested behind the first one's products.  Groups of eight weight rows, not
 // sixteen, while those leave half the CUs without one: a CU's loads, 64 bytes a clock, are what a group takes longest for.  Both together: 1024 x 2048 and 1024 x 3072, six rows, 5.7
 // us in the mean of the two (by the profiler's clock) -> 4.4 and 5.4.  How many waves share a sum depends on N and K alone, so a product with its prologue keeps the bits of the two launches.
-// us of one launch, weights from memory, before (a column per wave on the vector pipe for up to eight rows) -> the matrix pipe in groups of 16:   N x K      1 row          6 rows
+// us of one launch, weights from memory, before (a column per wave on the vector pipe for up to eight rows) -> the matrix pipe in groups of 16 (without EVEN, whose figures stand at the kernel):   N x K      1 row          6 rows
 //     RMSNorm + 4096 x 1024    4.9 -> 4.5     9.0 -> 6.2          |   1024 x 3072 (from activated rows)    4.6 -> 3.5     7.9 -> 5.8
 //     RMSNorm + 6144 x 1024    6.6 -> 5.7    11.3 -> 7.9          |   1024 x 2048                          3.8 -> 2.9     6.3 -> 4.5
 //     RMSNorm + 151936 x 1024   52 -> 52      152 -> 56           |   3072 x 4096                          8.5 -> 7.1    14.0 -> 9.0
@@ -716,8 +738,8 @@ template <int PRO, bool F32, bool GLU = false>
 static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, const void* nw, float eps, const void* W, int64_t ldw, void* y, int64_t ldy, const void* res, int64_t ldr, void* stream, SplitRow fold = {}) {
     if (M == 1) {
         const int64_t blocks = (N + 3) / 4;
-#define GEMV(T) gemv_one_kernel<T, PRO, F32, GLU><<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO >= 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res, fold)
-        if (K <= 1024) GEMV(2); else if (K <= 2048) GEMV(4); else GEMV(8);
+#define GEMV(T) (K == T * 512 ? gemv_one_kernel<T, PRO, F32, GLU, true> : gemv_one_kernel<T, PRO, F32, GLU, false>)<<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO >= 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res, fold)
+        if (K <= 1024) GEMV(2); else if (K <= 2048) GEMV(4); else if (K <= 3072) GEMV(6); else GEMV(8);
 #undef GEMV
         return;
     }
@@ -728,7 +750,12 @@ static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, con
         const bool half = !GLU && groups <= 128;
         const int64_t work = half ? (N + 7) / 8 : groups;
         const int grid = (int)(work < most ? work : most), steps = (all + waves - 1) / waves;
-#define GEMV(NW, R) gemv_kernel<NW, PRO, F32, GLU, R><<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, (void*)y, ldy, res, ldr)
+        const bool even = PRO != 2 && K == steps * waves * 32;
+        constexpr int T4 = PRO == 2 ? GEMV_STEPS : 4;
+#define GEMV(NW, R) \
+    (even && steps % GEMV_STEPS == 0       ? gemv_kernel<NW, PRO, F32, GLU, R, GEMV_STEPS, PRO != 2> \
+     : even && steps == 4                  ? gemv_kernel<NW, PRO, F32, GLU, R, T4, PRO != 2> \
+                                           : gemv_kernel<NW, PRO, F32, GLU, R, GEMV_STEPS, false>)<<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, (void*)y, ldy, res, ldr)
         if (waves == 4) GEMV(4, 16);
         else if (half && !GLU) {
             if (waves == 12) GEMV(12, GLU ? 16 : 8); else GEMV(8, GLU ? 16 : 8);
