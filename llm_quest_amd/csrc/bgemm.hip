@@ -1085,6 +1085,8 @@ __global__ __launch_bounds__(64 * SW) void bgemm_f32_rows_kernel(BgemmArgs p, in
     }
 }
 
+extern "C" __attribute__((visibility("hidden"))) void mi355_gemv_bias_part(int M, int64_t N, int K, const void* x, int64_t ldx, const void* W, int64_t ldw, void* y, int64_t ldy, const float* bias, void* stream);
+
 extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_dt, int64_t lda, int64_t a_bs, const void* B, int b_dt, int64_t sbn, int64_t sbk,
                            int64_t b_bs, void* C, int c_dt, int64_t ldc, int64_t c_bs, const int* grp_offs, const int* a_rows, int a_div, const int* c_rows,
                            const float* row_scale, int epi, int use_mfma, const float* bias, float limit, int n_out, void* stream) {
@@ -1106,6 +1108,12 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
     p.epi = epi, p.a_dt = a_dt, p.b_dt = b_dt, p.c_dt = c_dt;
     p.rows_last = grp_offs && (M <= 64 * (int64_t)batch || (int64_t)batch * N * K <= 64 << 20);
     const bool vec = sbk == 1 && K % 8 == 0 && lda % 8 == 0 && a_bs % 8 == 0 && sbn % 8 == 0 && b_bs % 8 == 0 && ((uintptr_t)A & 15) == 0 && ((uintptr_t)B & 15) == 0;
+    // one to eight rows with a bias: the weight streams of decode.hip (1024 x 1024, six rows, 24.4 -> 3.8 us; 128-column tiles leave all but eight CUs idle)
+    if (use_mfma && batch == 1 && M <= 8 && bias && c_dt == MI355_DT_BF16 && vec && epi == 0 && !grp_offs && !a_rows && !c_rows && !row_scale) {
+        mi355_gemv_bias_part(M, N, K, A, lda, B, sbn, C, ldc, bias, stream);
+        MI355_LAUNCH_CHECK("bgemm(few rows)");
+        return 0;
+    }
     if (use_mfma && grp_offs && M <= STREAM_ROWS && K >= 256 && vec) {
         const dim3 grid = tile_grid(p, (N + (epi >= 2 ? 63 : 31)) / (epi >= 2 ? 64 : 32), (M + 31) / 32, batch);
         if (epi >= 2) bgemm_stream_kernel<true, false><<<grid, 64 * SW, 0, ST(stream)>>>(p);

@@ -39,6 +39,7 @@ __device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8]) {
 // product were 1 us of a launch), operand rows past the last one are that row again, and what they give is not stored.  us, six rows, weights from memory, before -> EVEN: RMSNorm + 4096 x
 // 1024 6.9 -> 5.8, RMSNorm + SwiGLU of 6144 x 1024 7.9 -> 7.5, 1024 x 3072 5.3 -> 4.9, 1024 x 2048 4.6 -> 4.2.  One row (gemv_one_kernel, T strips of 512 k): 4.9 -> 4.4, 5.2 -> 4.6,
 // 3.8 -> 3.5.  T 4 or 8: chunks of 7 steps (K = 3584) gain nothing, nor do 384 workgroups for 384 groups.
+constexpr int OUT_BF16 = 0, OUT_F32 = 1, OUT_BF16_BIAS = 2;  // what is stored, and what `res` is: bf16 rows of a residual, or one fp32 row
 constexpr int GEMV_STEPS = 8;  // of 32 k in flight per wave: 8 x 16 bytes a lane
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
     u32x4 o;
@@ -48,7 +49,7 @@ __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
 }
 __device__ __forceinline__ float rbf(float x) { return bf2f(f2bf(x)); }
 
-template <int NW, int PRO, bool F32, bool GLU, int ROWS, int T, bool EVEN>
+template <int NW, int PRO, int OUT, bool GLU, int ROWS, int T, bool EVEN>
 __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, int steps, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ nw, float eps,
                                                        const bf16_t* __restrict__ W, int64_t ldw, void* __restrict__ y, int64_t ldy, const void* __restrict__ res, int64_t ldr) {
     static_assert(!EVEN || (PRO != 2 && NW * T % 16 == 0), "whole strips of 512 k");
@@ -180,7 +181,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
         float add = 0.f;
         if (cn == chunks) {
             cn = 0, gn += gridDim.x;
-            if (res && m < M && n < N && r16 < GN) add = F32 ? ((const float*)res)[n] : bf2f(((const bf16_t*)res)[m * ldr + n]);
+            if (res && m < M && n < N && r16 < GN) add = OUT ? ((const float*)res)[n] : bf2f(((const bf16_t*)res)[m * ldr + n]);
         }
         if (gn < groups) request_w(next, gn, cn);
 #pragma unroll
@@ -198,7 +199,7 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
 #pragma unroll
                     for (int i = 1; i < NW; ++i) gate += part[flip][i][m][8 + (r16 & 7)];
                     ((bf16_t*)y)[m * ldy + n] = f2bf(swiglu_act(rbf(s), rbf(gate)));
-                } else if constexpr (F32) ((float*)y)[m * ldy + n] = res ? s + add : s;
+                } else if constexpr (OUT == OUT_F32) ((float*)y)[m * ldy + n] = res ? s + add : s;
                 else ((bf16_t*)y)[m * ldy + n] = f2bf(res ? s + add : s);
             }
             flip ^= 1;  // (the next group's sums go beside these: its barrier is behind every read of them)
@@ -262,7 +263,7 @@ __device__ __forceinline__ void fold_splits8(const SplitRow& fold, int k, float 
 #pragma unroll
     for (int e = 0; e < 8; ++e) o[e] = out[e] / lg;
 }
-template <int T, int PRO, bool F32, bool GLU, bool EVEN>
+template <int T, int PRO, int OUT, bool GLU, bool EVEN>
 __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const bf16_t* __restrict__ x, const bf16_t* __restrict__ nw, float eps, const bf16_t* __restrict__ W, int64_t ldw,
                                                        void* __restrict__ y, const void* __restrict__ res, SplitRow fold) {
     extern __shared__ __attribute__((aligned(16))) bf16_t act[];  // PRO 2, 3: [K]
@@ -347,7 +348,7 @@ __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const b
 #pragma unroll
         for (int c = 0; c < C; ++c) acc[c] = 0.f;
         float add = 0.f;
-        if (res) add = F32 ? ((const float*)res)[n] : bf2f(((const bf16_t*)res)[n]);
+        if (res) add = OUT ? ((const float*)res)[n] : bf2f(((const bf16_t*)res)[n]);
         for (int base = 0; base < its; base += T) {
             if (!first) {
                 if (its > T) request_x(base);
@@ -372,7 +373,7 @@ __global__ __launch_bounds__(256) void gemv_one_kernel(int64_t N, int K, const b
         for (int c = 0; c < C; ++c) acc[c] = wave_sum(acc[c]);
         if (lane == 0) {
             if constexpr (GLU) ((bf16_t*)y)[n] = f2bf(swiglu_act(rbf(acc[0]), rbf(acc[C - 1])));
-            else if constexpr (F32) ((float*)y)[n] = res ? acc[0] + add : acc[0];
+            else if constexpr (OUT == OUT_F32) ((float*)y)[n] = res ? acc[0] + add : acc[0];
             else ((bf16_t*)y)[n] = f2bf(res ? acc[0] + add : acc[0]);
         }
     }
@@ -734,11 +735,11 @@ __global__ __launch_bounds__(64) void argmax_merge_kernel(const float* __restric
 //     RMSNorm + 4096 x 1024    4.9 -> 4.5     9.0 -> 6.2          |   1024 x 3072 (from activated rows)    4.6 -> 3.5     7.9 -> 5.8
 //     RMSNorm + 6144 x 1024    6.6 -> 5.7    11.3 -> 7.9          |   1024 x 2048                          3.8 -> 2.9     6.3 -> 4.5
 //     RMSNorm + 151936 x 1024   52 -> 52      152 -> 56           |   3072 x 4096                          8.5 -> 7.1    14.0 -> 9.0
-template <int PRO, bool F32, bool GLU = false>
+template <int PRO, int OUT, bool GLU = false>
 static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, const void* nw, float eps, const void* W, int64_t ldw, void* y, int64_t ldy, const void* res, int64_t ldr, void* stream, SplitRow fold = {}) {
     if (M == 1) {
         const int64_t blocks = (N + 3) / 4;
-#define GEMV(T) (K == T * 512 ? gemv_one_kernel<T, PRO, F32, GLU, true> : gemv_one_kernel<T, PRO, F32, GLU, false>)<<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO >= 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res, fold)
+#define GEMV(T) (K == T * 512 ? gemv_one_kernel<T, PRO, OUT, GLU, true> : gemv_one_kernel<T, PRO, OUT, GLU, false>)<<<(int)(blocks < 2048 ? blocks : 2048), 256, PRO >= 2 ? (size_t)K * 2 : 0, ST(stream)>>>(N, K, (const bf16_t*)x, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, y, res, fold)
         if (K <= 1024) GEMV(2); else if (K <= 2048) GEMV(4); else if (K <= 3072) GEMV(6); else GEMV(8);
 #undef GEMV
         return;
@@ -753,9 +754,9 @@ static void gemv_launch(int M, int64_t N, int K, const void* x, int64_t ldx, con
         const bool even = PRO != 2 && K == steps * waves * 32;
         constexpr int T4 = PRO == 2 ? GEMV_STEPS : 4;
 #define GEMV(NW, R) \
-    (even && steps % GEMV_STEPS == 0       ? gemv_kernel<NW, PRO, F32, GLU, R, GEMV_STEPS, PRO != 2> \
-     : even && steps == 4                  ? gemv_kernel<NW, PRO, F32, GLU, R, T4, PRO != 2> \
-                                           : gemv_kernel<NW, PRO, F32, GLU, R, GEMV_STEPS, false>)<<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, (void*)y, ldy, res, ldr)
+    (even && steps % GEMV_STEPS == 0       ? gemv_kernel<NW, PRO, OUT, GLU, R, GEMV_STEPS, PRO != 2> \
+     : even && steps == 4                  ? gemv_kernel<NW, PRO, OUT, GLU, R, T4, PRO != 2> \
+                                           : gemv_kernel<NW, PRO, OUT, GLU, R, GEMV_STEPS, false>)<<<grid, 64 * NW, 0, ST(stream)>>>(M, N, K, steps, (const bf16_t*)x, ldx, (const bf16_t*)nw, eps, (const bf16_t*)W, ldw, (void*)y, ldy, res, ldr)
         if (waves == 4) GEMV(4, 16);
         else if (half && !GLU) {
             if (waves == 12) GEMV(12, GLU ? 16 : 8); else GEMV(8, GLU ? 16 : 8);
@@ -770,7 +771,7 @@ extern "C" int mi355_gemv_bf16(int M, int64_t N, int K, const void* x, int64_t l
     MI355_REQUIRE(M >= 1 && M <= 8, "gemv_bf16: 1..8 rows (got %d); larger batches go through mi355_gemm_bf16", M);
     MI355_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= K && ldw >= K && ldy >= N, "gemv_bf16: K and the leading dimensions of x / W must be multiples of 8");
     MI355_REQUIRE(x && W && y && (!residual || ldr >= N), "gemv_bf16: null pointer or residual pitch too small");
-    gemv_launch<0, false>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);
+    gemv_launch<0, OUT_BF16>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);
     MI355_LAUNCH_CHECK("gemv_bf16");
     return 0;
 }
@@ -780,9 +781,14 @@ extern "C" int mi355_gemv_bf16_f32out(int M, int64_t N, int K, const void* x, in
     MI355_REQUIRE(M >= 1 && M <= 8, "gemv_bf16_f32out: 1..8 rows (got %d)", M);
     MI355_REQUIRE(N > 0 && K > 0 && K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && ldx >= K && ldw >= K && ldy >= N, "gemv_bf16_f32out: K and the leading dimensions of x / W must be multiples of 8");
     MI355_REQUIRE(x && W && y, "gemv_bf16_f32out: null pointer");
-    gemv_launch<0, true>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, bias, 0, stream);
+    gemv_launch<0, OUT_F32>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, bias, 0, stream);
     MI355_LAUNCH_CHECK("gemv_bf16_f32out");
     return 0;
+}
+
+// bgemm.hip's products of one to eight bf16 rows with a bias, results in bf16
+extern "C" __attribute__((visibility("hidden"))) void mi355_gemv_bias_part(int M, int64_t N, int K, const void* x, int64_t ldx, const void* W, int64_t ldw, void* y, int64_t ldy, const float* bias, void* stream) {
+    gemv_launch<0, OUT_BF16_BIAS>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, bias, 0, stream);
 }
 
 extern "C" int mi355_gemv_bf16_pro(int M, int64_t N, int K, const void* x, int64_t ldx, int prologue, const void* norm_w, float eps, const void* W, int64_t ldw,
@@ -795,8 +801,8 @@ extern "C" int mi355_gemv_bf16_pro(int M, int64_t N, int K, const void* x, int64
     // is where an earlier image of all rows ended, and is kept because it decides which launches, and so which bits, a step of that size has.
     MI355_REQUIRE((int64_t)M * K * 2 + 32 <= 65536, "gemv_bf16_pro: takes operand rows (here %d x %d bf16) up to 64 KiB less 32 bytes", M, K);
     MI355_REQUIRE(x && W && y && (!residual || ldr >= N) && (prologue != 1 || norm_w), "gemv_bf16_pro: null pointer or residual pitch too small");
-    if (prologue == 1) gemv_launch<1, false>(M, N, K, x, ldx, norm_w, eps, W, ldw, y, ldy, residual, ldr, stream);
-    else gemv_launch<2, false>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);
+    if (prologue == 1) gemv_launch<1, OUT_BF16>(M, N, K, x, ldx, norm_w, eps, W, ldw, y, ldy, residual, ldr, stream);
+    else gemv_launch<2, OUT_BF16>(M, N, K, x, ldx, nullptr, 0.f, W, ldw, y, ldy, residual, ldr, stream);
     MI355_LAUNCH_CHECK("gemv_bf16_pro");
     return 0;
 }
@@ -907,10 +913,10 @@ extern "C" int mi355_decode_block(int B, int d, int F, int Hq, int Hkv, int D, c
                                  scale, eps, splits, parts, stream, !fold)) return rc;
     if (fold) {
         MI355_REQUIRE(w_out, "decode_block: null pointer");
-        gemv_launch<3, false>(1, d, (int)nc, ctx, nc, nullptr, 0.f, w_out, nc, h1, l1, h, d, stream, SplitRow{parts, D, splits});
+        gemv_launch<3, OUT_BF16>(1, d, (int)nc, ctx, nc, nullptr, 0.f, w_out, nc, h1, l1, h, d, stream, SplitRow{parts, D, splits});
         MI355_LAUNCH_CHECK("decode_block(out)");
     } else if (int rc = mi355_gemv_bf16(B, d, (int)nc, ctx, nc, w_out, nc, h1, l1, h, d, stream)) return rc;
-    gemv_launch<1, false, true>(B, F, d, h1, l1, norm2_w, eps, w_gate_up, d, act, la, nullptr, 0, stream);
+    gemv_launch<1, OUT_BF16, true>(B, F, d, h1, l1, norm2_w, eps, w_gate_up, d, act, la, nullptr, 0, stream);
     MI355_LAUNCH_CHECK("decode_block(gate, up)");
     return mi355_gemv_bf16(B, d, F, act, la, w_down, F, out, d, h1, l1, stream);
 }

@@ -186,3 +186,18 @@ def test_gla_in_groups_of_16_and_of_8_tokens(H, dk, dv, fixed, dt):
             want, size = torch.einsum("hk,hkv->hv", qt, s), torch.einsum("hk,hkv->hv", qt.abs(), m)
             assert bool(((got[t].double().view(H, dv) - want).abs() <= EPS * (16 * (t - offs[i] + 1) + dk + 40) * size).all())
         assert bool(((st[sl].double() - s).abs() <= EPS * (16 * n[i] + 4) * m).all())
+
+
+@pytest.mark.parametrize("M,K,N", [(1, 8, 7), (1, 1024, 33), (2, 264, 130), (3, 1024, 1024), (5, 1000, 17), (8, 2048, 2056), (6, 3072, 1025), (8, 512, 16400)])
+def test_few_bf16_rows_with_a_bias(M, K, N):
+    """Whole numbers whose sums fp32 holds exactly: the results are the exact sums rounded once; rows beside the operands and beside the bias are not read into them."""
+    from llm_quest_amd import kernels_seq as S
+
+    g = torch.Generator().manual_seed(M + K + N)
+    x = torch.full((M + 1, K + 8), float("nan"), dtype=BF16, device="cuda")
+    x[:M, :K] = torch.randint(-8, 9, (M, K), generator=g).cuda()
+    w = torch.randint(-8, 9, (N, K), generator=g).to(BF16).cuda()
+    bias = torch.randint(-999, 1000, (N,), generator=g).float().cuda()
+    want = (x[:M, :K].double() @ w.double().T + bias.double()).float()
+    for dt in (BF16, F32):
+        assert torch.equal(S.linear(x[:M, :K], w, bias=bias, out_dtype=dt), want.to(dt))
