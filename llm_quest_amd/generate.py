@@ -199,12 +199,21 @@ class RaggedBatch:
         slotted = []
         import numpy as np
 
-        for seq_id, toks in entries:
-            toks = np.asarray(toks, dtype=np.int64).reshape(-1)
-            if toks.size and (int(toks.min()) < 0 or int(toks.max()) >= vocab):
-                raise ValueError(f"sequence {seq_id!r}: token id outside [0, {vocab})")
-            slot = cache.slot(seq_id) if seq_id in cache else cache.open(seq_id)
-            slotted.append((slot, toks))
+        new = []
+        try:
+            for seq_id, toks in entries:
+                toks = np.asarray(toks, dtype=np.int64).reshape(-1)
+                if toks.size and (int(toks.min()) < 0 or int(toks.max()) >= vocab):
+                    raise ValueError(f"sequence {seq_id!r}: token id outside [0, {vocab})")
+                if seq_id in cache:
+                    slot = cache.slot(seq_id)
+                else:
+                    slot = cache.open(seq_id, clear=False)
+                    new.append(slot)
+                slotted.append((slot, toks))
+        finally:
+            if new:
+                cache.clear(new)
         st = SeqStep(cache, slotted, self.device, self.model.act_dtype)
         rows = []
         for i, (_, toks) in enumerate(slotted):

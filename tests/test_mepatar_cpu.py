@@ -148,3 +148,12 @@ def test_slot_cache_named_states_and_step_descriptors(tmp_path):
     cache.close("a")
     c = cache.open("c")  # the freed slot comes back zeroed
     assert c == a and float(cache.state(0, "S")[c].abs().max()) == 0.0 and float(cache.state(2, "conv")[c].abs().max()) == 0.0 and cache.length[c] == 0
+    d = cache.open("d")  # slots that are opened together are cleared together, side by side or not, and nothing beside them
+    for slots, kept in (([b, d], c), ([d, c], b), ([c, b], d), ([d, b, c], None)):
+        cache.state(0, "S").fill_(3.0), cache.state(2, "conv").fill_(4.0)
+        cache.clear(slots)
+        for s in (b, c, d):
+            assert set(cache.state(0, "S")[s].flatten().tolist()) == {3.0 if s == kept else 0.0} and set(cache.state(2, "conv")[s].flatten().tolist()) == {4.0 if s == kept else 0.0}
+    cache.close("d")
+    cache.state(0, "S").fill_(3.0)
+    assert cache.open("e", clear=False) == d and float(cache.state(0, "S")[d].min()) == 3.0
