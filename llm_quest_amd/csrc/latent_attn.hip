@@ -676,25 +676,52 @@ __global__ __launch_bounds__(256) void latent_attn_combine_kernel(LatAttnArgs p,
     if (tok >= p.n_new[s] || head >= p.H) return;
     const int64_t blk0 = (((int64_t)s * gy + by) * tiles + tile) * p.splits;
     const int64_t stride = (int64_t)MQ * (2 + DVP);
-    float m = -__builtin_huge_valf();
-    for (int i = 0; i < p.splits; ++i) m = fmaxf(m, p.ws[(blk0 + i) * stride + row]);
+    // The first AT splits' statistics and the lane's first column of each are requested before anything is done with them: one round trip, not one for each split and use (us, six one-token sequences of
+    // 8 heads, three splits, 10.6 -> 4.3).
+    constexpr int AT = 8;
+    const float NEG = -__builtin_huge_valf();
+    const float* src = p.ws + blk0 * stride + row;
+    float ms[AT], ls[AT], w[AT];
+    auto columns = [&](int dv) {
+#pragma unroll
+        for (int j = 0; j < AT; ++j) w[j] = p.ws[(blk0 + min(j, p.splits - 1)) * stride + 2 * MQ + (int64_t)row * DVP + dv];
+    };
+#pragma unroll
+    for (int j = 0; j < AT; ++j) ms[j] = src[min(j, p.splits - 1) * stride], ls[j] = src[min(j, p.splits - 1) * stride + MQ];
+    columns(min(lane, p.DV - 1));
+    float m = NEG;
+#pragma unroll
+    for (int j = 0; j < AT; ++j) m = fmaxf(m, ms[j]);
+    for (int i = AT; i < p.splits; ++i) m = fmaxf(m, src[i * stride]);
     float l = 0.f;
     if (p.sink) {
         const float sk = p.sink[head] * 1.4426950408889634f;
         m = fmaxf(m, sk);
         l = exp2f(sk - m);
     }
-    for (int i = 0; i < p.splits; ++i) {
-        const float mi = p.ws[(blk0 + i) * stride + row];
-        if (mi != -__builtin_huge_valf()) l += p.ws[(blk0 + i) * stride + MQ + row] * exp2f(mi - m);
+#pragma unroll
+    for (int j = 0; j < AT; ++j) {  // (a split that holds no key of the row: no part of the sums)
+        const float f = j >= p.splits || ms[j] == NEG ? 0.f : exp2f(ms[j] - m);
+        if (f != 0.f) l += ls[j] * f;
+        ms[j] = f;
+    }
+    for (int i = AT; i < p.splits; ++i) {
+        const float mi = src[i * stride];
+        if (mi != NEG) l += src[i * stride + MQ] * exp2f(mi - m);
     }
     const int64_t o0 = ((int64_t)p.q_row0[s] + tok) * p.ldo + (int64_t)head * p.o_hs;
     for (int dv = lane; dv < p.DV; dv += 64) {
+        if (dv != lane) columns(dv);
         float acc = 0.f;
-        for (int i = 0; i < p.splits; ++i) {
-            const float mi = p.ws[(blk0 + i) * stride + row], w = p.ws[(blk0 + i) * stride + 2 * MQ + (int64_t)row * DVP + dv];
-            if (p.sig_bias) acc += w;  // sigmoid weights simply add up
-            else if (mi != -__builtin_huge_valf()) acc += w * exp2f(mi - m);
+#pragma unroll
+        for (int j = 0; j < AT; ++j) {
+            if (p.sig_bias) acc += j < p.splits ? w[j] : 0.f;  // sigmoid weights simply add up
+            else if (ms[j] != 0.f) acc += w[j] * ms[j];
+        }
+        for (int i = AT; i < p.splits; ++i) {
+            const float mi = src[i * stride], wi = p.ws[(blk0 + i) * stride + 2 * MQ + (int64_t)row * DVP + dv];
+            if (p.sig_bias) acc += wi;
+            else if (mi != NEG) acc += wi * exp2f(mi - m);
         }
         float v = p.sig_bias ? acc : acc / l;
         if (p.gate) v *= gate_of(p.gate[((int64_t)p.q_row0[s] + tok) * p.ldg + (int64_t)head * p.DV + dv]);

@@ -10,10 +10,14 @@
 // The next tile's keys and values are (but for the widest rows) requested before the current tile's arithmetic; only steps with a key that some row of the wave does not
 // see are masked; tiles with the most keys start first.  A tile walks the 64-key steps of key_steps (kept first tokens, then its window).  Options: a sink in the
 // denominator, or sigmoid weights instead of the softmax (SIG); key splits as in latent_attn.hip; a sigmoid gate on the output.
+// Bound: vector instructions, about 570 a step of 64 keys beside 32 products (capped scores), in a one-token step the 2 500 in front of and behind it.  us, 8 prompts of 1 024 tokens under a window of
+// 512, 16 heads over 2 of 128, 117 -> 90 with what a load and a mask no longer compute (six of 900, 8 heads, 52 -> 36; one token a sequence 16 -> 14).
 #pragma once
 #include "latent_attn.h"
 
 #define LOG2E 1.4426950408889634f
+
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 struct DiffJoinArgs {  // the join of two maps: o = a1 - lam a2, o / sqrt(mean(o^2) + eps) * c
     float lam, eps, c;
@@ -60,14 +64,13 @@ __global__ __launch_bounds__(256, NVB <= 4 && DKS * MAPS <= 16 ? 2 : 1) void lat
         const float* qrow = p.Q + (qr0 + (row_ok ? tok : 0)) * p.ldq + (int64_t)(row_ok ? head : 0) * p.q_hs + (MAPS == 2 ? map * p.D1 : 0);
 #pragma unroll
         for (int st = 0; st < DKS; ++st) {
-            float v[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const int d = 16 * st + 8 * hf + j;
-                v[j] = (row_ok && d < DK) ? qrow[d] : 0.f;
-            }
-            const u32x4 pk = {pack_bf2(v[0], v[1]), pack_bf2(v[2], v[3]), pack_bf2(v[4], v[5]), pack_bf2(v[6], v[7])};
-            qf[st] = __builtin_bit_cast(bf16x8, pk);
+            // eight features at a time (DK is a multiple of 8; the rows of Q need no more than a float's alignment), no branch: a lane without a query reads token 0's, groups past
+            // DK read the last one and become zeros
+            const int d = 16 * st + 8 * hf;
+            const f32x4u *src = (const f32x4u*)(qrow + min(d, DK - 8)), a = src[0], b = src[1];
+            const bool in = row_ok && d < DK;
+            const u32x4 pk = {pack_bf2(a[0], a[1]), pack_bf2(a[2], a[3]), pack_bf2(b[0], b[1]), pack_bf2(b[2], b[3])};
+            qf[st] = __builtin_bit_cast(bf16x8, in ? pk : u32x4{0u, 0u, 0u, 0u});
         }
     }
     const int n_keys = past + min(tok0 + tm, n_new);
@@ -80,12 +83,9 @@ __global__ __launch_bounds__(256, NVB <= 4 && DKS * MAPS <= 16 ? 2 : 1) void lat
         v_lo = min(all_steps, split * per);
         v_hi = min(all_steps, v_lo + per);
     }
-    // the last key any row of this wave sees, and the last one that all of its rows see
-    int wave_lim = lim, wave_all = row_ok ? lim : 0x7fffffff;
-#pragma unroll
-    for (int of = 32; of > 0; of >>= 1) wave_lim = max(wave_lim, __shfl_xor(wave_lim, of, 64)), wave_all = min(wave_all, __shfl_xor(wave_all, of, 64));
-    wave_lim = __builtin_amdgcn_readfirstlane(wave_lim);
-    wave_all = __builtin_amdgcn_readfirstlane(wave_all);
+    // the last key any row of this wave sees, and the last one that all of its rows see: positions grow with the row
+    const unsigned with = (unsigned)__ballot(row_ok);  // (both halves of the wave hold the same rows)
+    const int wave_lim = with ? __builtin_amdgcn_readlane(lim, 31 - __builtin_clz(with)) : -1, wave_all = with ? __builtin_amdgcn_readlane(lim, __builtin_ctz(with)) : 0x7fffffff;
 
     // the first key of a row's window or chunk (it grows with the row's position, so the wave's first and last rows bound it)
     const int row_lo = OPT == LAT_ALL ? 0 : tile_key_floor(lim, p.window, p.chunk);
@@ -106,7 +106,27 @@ __global__ __launch_bounds__(256, NVB <= 4 && DKS * MAPS <= 16 ? 2 : 1) void lat
 
     const u32x4 zero4 = {0u, 0u, 0u, 0u};
     u32x4 kreg[NKU], vreg[NVU];
+    // One part of keys, rows of 2^n words: a thread's words lie whole rows apart, one offset and one add each; keys past the end lie beyond num_records, features past the row's have the offset OOB.
+    // (A branch, a 64-bit product and a select of the part for every word were a tenth of a step, and half of a one-token step's instructions with the query's.)
+    constexpr bool POW2 = 256 % (KROW / 8) == 0;
+    const bool plain = POW2 && p.D2 == 0 && p.ldk1 < (1 << 23) && p.ldv < (1 << 23);
+    unsigned ko = 0, vo = 0;
+    if (plain) {
+        const int d0 = (tid % (KROW / 8)) * 8, m = MAPS == 2 ? d0 / DKP : 0, d = MAPS == 2 ? d0 % DKP : d0, dv = (tid % (DVP / 8)) * 8;
+        ko = d < DK ? (unsigned)((tid / (KROW / 8)) * (int)p.ldk1 + m * p.D1 + d) * 2 : 0x80000000u;
+        vo = dv < p.DV ? (unsigned)((tid / (DVP / 8)) * (int)p.ldv + dv) * 2 : 0x80000000u;
+    }
     auto fetch = [&](int j0) {
+        if (plain) {
+            const int left = min(64, n_keys - j0);
+            const auto kr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(K1 + (int64_t)j0 * p.ldk1), 0, left * (int)p.ldk1 * 2, 0x00020000);
+            const auto vr = __builtin_amdgcn_make_buffer_rsrc(const_cast<bf16_t*>(V + (int64_t)j0 * p.ldv), 0, left * (int)p.ldv * 2, 0x00020000);
+#pragma unroll
+            for (int u = 0; u < NKU; ++u) kreg[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(kr, ko + (unsigned)(u * (2048 / KROW) * (int)p.ldk1 * 2), 0, 0));
+#pragma unroll
+            for (int u = 0; u < NVU; ++u) vreg[u] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(vr, vo + (unsigned)(u * (2048 / DVP) * (int)p.ldv * 2), 0, 0));
+            return;
+        }
 #pragma unroll
         for (int u = 0; u < NKU; ++u) {
             const int c = tid + 256 * u, key = c / (KROW / 8), d0 = (c % (KROW / 8)) * 8, j = j0 + key;
@@ -188,7 +208,8 @@ __global__ __launch_bounds__(256, NVB <= 4 && DKS * MAPS <= 16 ? 2 : 1) void lat
 #pragma unroll
                     for (int r = 0; r < 16; ++r) {
                         const int o = kb * 32 + 8 * (r >> 2) + (r & 3);
-                        if (o > over || (o < under && o >= kept)) sacc[kb][r] = NEG;
+                        const bool hidden = (o > over) | ((o < under) & (o >= kept));  // (no branches)
+                        sacc[kb][r] = hidden ? NEG : sacc[kb][r];
                     }
             }
         } else if (j0 + 63 > wave_all) {  // wave-uniform: only steps that reach a row's own position hide keys

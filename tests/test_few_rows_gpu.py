@@ -201,3 +201,44 @@ def test_few_bf16_rows_with_a_bias(M, K, N):
     want = (x[:M, :K].double() @ w.double().T + bias.double()).float()
     for dt in (BF16, F32):
         assert torch.equal(S.linear(x[:M, :K], w, bias=bias, out_dtype=dt), want.to(dt))
+
+
+@pytest.mark.parametrize("D,DV,window,cap,new,past", [(64, 64, 0, 0.0, [5, 130], [0, 70]), (128, 128, 100, 0.0, [1, 200, 17], [63, 0, 300]), (128, 40, 64, 5.0, [70, 3], [1, 400]), (256, 256, 0, 0.0, [9, 65], [120, 0]),
+                                                      (72, 24, 50, 0.0, [33], [200]), (136, 136, 0, 2.0, [33], [200]), (128, 128, 0, 0.0, [1, 1], [4000, 2100]), (64, 64, 0, 0.0, [1], [600])])
+def test_keys_of_one_part_and_of_two_give_the_same_attention(D, DV, window, cap, new, past):
+    """Keys of one part come by their own loads (rows past the end are NaN here: they lie behind the descriptor's end), those of two parts by the general ones; queries at any
+    alignment.  The arithmetic is the same, so are the bits.  One new token over many keys: up to 15 splits, more than the join requests at once.  Against 64 bits: queries, weights and
+    results rounded to bf16 or held in it, 2^-9 each (a weight's error is its score's)."""
+    from llm_quest_amd import kernels_seq as S
+
+    H, half = 4, (D // 16) * 8
+    g = torch.Generator().manual_seed(D + DV + window)
+    total = [n + p for n, p in zip(new, past)]
+    rows = [t + 70 for t in total]
+    k, v = torch.full((sum(rows), D), float("nan")), torch.full((sum(rows), DV), float("nan"))
+    at = [sum(rows[:i]) for i in range(len(rows))]
+    for a, t in zip(at, total):
+        k[a : a + t], v[a : a + t] = torch.randn(t, D, generator=g), torch.randn(t, DV, generator=g)
+    k, v, q = k.to(BF16).cuda(), v.to(BF16).cuda(), torch.randn(sum(new), H * D, generator=g).cuda()
+    shifted = torch.zeros(sum(new), H * D + 3, device="cuda")
+    shifted[:, 1 : H * D + 1] = q
+    k0, q0 = i32(at), i32([sum(new[:i]) for i in range(len(new))])
+    desc = (q0, i32(new), i32(past), k0, k0, k0)
+
+    def run(q, k1, k2, D1, D2):
+        out = torch.full((sum(new), H * DV), float("nan"), device="cuda")
+        S.latent_attn(q, k1, k2, v, out, H, H, D1, D2, DV, D, D1, DV, DV, desc, max(new), D**-0.5, max_keys=max(total), kv_rep=H, window=window, softcap=cap)
+        return out
+
+    one = run(q, k, None, D, 0)
+    assert torch.equal(one, run(shifted[:, 1 : H * D + 1], k, None, D, 0))
+    assert torch.equal(one, run(q, k[:, :half].contiguous(), k[:, half:].contiguous(), half, D - half))
+    for i, (n, p) in enumerate(zip(new, past)):
+        r = slice(int(q0[i]), int(q0[i]) + n)
+        ks, vs, qs = k[at[i] : at[i] + n + p].double(), v[at[i] : at[i] + n + p].double(), q[r].double().view(n, H, D)
+        s, mag = (qs @ ks.T) * D**-0.5, (qs.abs() @ ks.abs().T * D**-0.5).amax()
+        s = cap * torch.tanh(s / cap) if cap else s
+        pos, j = p + torch.arange(n, device="cuda")[:, None], torch.arange(n + p, device="cuda")[None]
+        w = torch.softmax(s.masked_fill(((j > pos) | (j <= pos - (window or n + p + 1)))[:, None], float("-inf")), -1)
+        err = (2.0**-8 * mag + 2.0**-8) * (w @ vs.abs()) + 1e-30
+        assert bool(((one[r].double().view(n, H, DV) - w @ vs).abs() <= err).all())
