@@ -1724,21 +1724,25 @@ void launch_quad_fold(GroupTable& tbl, int out_dtype, hipStream_t s) {
 }
 
 // persistent: one workgroup per CU walks its share of the tiles, else a workgroup per tile
-template <bool TR>
+template <int FORM>
 int launch_quad(GemmParams p, int out_dtype, bool persistent, hipStream_t s) {
     p.tiles_m = (int)((p.M + 255) / 256);
     p.tiles_n = (int)((p.N + 255) / 256);
     const int64_t tiles = (int64_t)p.tiles_m * p.tiles_n * p.ksplit;
     MI355_REQUIRE(tiles < 0x7fffffffLL / 16, "mi355_gemm_bf16: grid too large");
     const dim3 grid((unsigned)(persistent && tiles > 256 ? 256 : tiles)), block(256);
-#define QUAD(OUT_, KIND_) gemm_quad_kernel<TR, OUT_, KIND_>
+#define QUAD(OUT_, KIND_) gemm_quad_kernel<FORM, OUT_, KIND_>
     void (*kernel)(GemmParams);
     const bool b16 = out_dtype == MI355_DT_BF16;
     if (p.ksplit > 1) {
         kernel = QUAD(MI355_DT_F32, QUAD_SPLIT);
-    } else if constexpr (TR) {
+    } else if constexpr (FORM == MI355_GEMM_TN) {
         if (p.R) kernel = b16 ? QUAD(MI355_DT_BF16, QUAD_RES) : QUAD(MI355_DT_F32, QUAD_RES);
         else kernel = b16 ? QUAD(MI355_DT_BF16, MI355_EPI_NONE) : QUAD(MI355_DT_F32, MI355_EPI_NONE);
+    } else if constexpr (FORM == MI355_GEMM_NN) {
+        if (p.epilogue == MI355_EPI_SWIGLU_BWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_BWD);
+        else if (p.R) kernel = QUAD(MI355_DT_BF16, QUAD_RES);
+        else kernel = QUAD(MI355_DT_BF16, MI355_EPI_NONE);
     } else {
         if (p.epilogue == MI355_EPI_SWIGLU_FWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_FWD);
         else if (p.epilogue == MI355_EPI_SWIGLU_BWD) kernel = QUAD(MI355_DT_BF16, MI355_EPI_SWIGLU_BWD);
@@ -2237,6 +2241,7 @@ __global__ __launch_bounds__(256) void colsum_kernel(int64_t M, int64_t N, const
 GEMM_BRIDGE_DECL(1) GEMM_BRIDGE_DECL(2) GEMM_BRIDGE_DECL(3) GEMM_BRIDGE_DECL(4) GEMM_BRIDGE_DECL(5)
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_nt_part8(const void* params, int out_dtype, int persistent, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_tn_part9(const void* params, int out_dtype, int persistent, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_nn_part10(const void* params, int out_dtype, int persistent, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_grouped_part9(void* table, int out_dtype, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_pp_part6(const void* params, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_ring_part7(int form, const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream);
@@ -2253,12 +2258,17 @@ extern "C" int mi355_gemm_pp_part6(const void* params, void* stream) { return la
 #endif
 #if GEMM_PART == 8 || GEMM_PART == -1
 extern "C" int mi355_gemm_quad_nt_part8(const void* params, int out_dtype, int persistent, void* stream) {
-    return launch_quad<false>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
+    return launch_quad<MI355_GEMM_NT>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
+}
+#endif
+#if GEMM_PART == 10 || GEMM_PART == -1
+extern "C" int mi355_gemm_quad_nn_part10(const void* params, int out_dtype, int persistent, void* stream) {
+    return launch_quad<MI355_GEMM_NN>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
 }
 #endif
 #if GEMM_PART == 9 || GEMM_PART == -1
 extern "C" int mi355_gemm_quad_tn_part9(const void* params, int out_dtype, int persistent, void* stream) {
-    return launch_quad<true>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
+    return launch_quad<MI355_GEMM_TN>(*static_cast<const GemmParams*>(params), out_dtype, persistent != 0, (hipStream_t)stream);
 }
 extern "C" int mi355_gemm_quad_grouped_part9(void* table, int out_dtype, void* stream) { return launch_quad_grouped(*static_cast<GroupTable*>(table), out_dtype, (hipStream_t)stream); }
 #endif
@@ -2319,7 +2329,8 @@ static bool quad_ok(int form, const GemmParams& p, int out_dtype) {
     const auto rows_ok = [&](const void* x, int64_t ld) { return (ld * esz & 15) == 0 && ((uintptr_t)x & 15) == 0 && ld < limit; };
     if (p.K <= 192 || (p.N & 7) || p.M > 0x7fffff00 || p.N > 0x7fffff00 || !rows_ok(p.C, p.ldc) || (p.R && !rows_ok(p.R, p.ldr))) return false;
     if (form == MI355_GEMM_TN) return !p.bias && p.epilogue == MI355_EPI_NONE;
-    if (form != MI355_GEMM_NT || (p.K & 63) || p.split3) return false;
+    if ((p.K & 63) || p.split3) return false;
+    if (form == MI355_GEMM_NN) return out_dtype == MI355_DT_BF16 && !p.bias && (p.epilogue == MI355_EPI_NONE || p.epilogue == MI355_EPI_SWIGLU_BWD);
     if (p.epilogue == MI355_EPI_SWIGLU_FWD) return p.N * p.ldb * 2 < 0x7fffffffLL;
     return p.epilogue == MI355_EPI_NONE || p.epilogue == MI355_EPI_SWIGLU_BWD || p.epilogue == MI355_EPI_ATTN_DELTA;
 }
@@ -2340,6 +2351,10 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
+static int launch_quad_form(int form, const GemmParams& p, int out_dtype, bool persistent, hipStream_t s) {
+    return form == MI355_GEMM_NT ? mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s) : form == MI355_GEMM_NN ? mi355_gemm_quad_nn_part10(&p, out_dtype, persistent, s) : mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s);
+}
+
 static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold, double& least) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
     if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
@@ -2371,11 +2386,11 @@ static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype,
 //   TN groups, bf16, 5 664 / 16 384 tokens: 16 tiles 61 -> 33 / 168 -> 55 (8), 48 62 -> 50 / 169 -> 94 (5), 64 63 -> 57 / 170 -> 112 (4), 80 81 -> 65 / 219 -> 136 (3), 96 82 -> 73 / 232 -> 174 (2),
 //   128 91 -> 89 / 295 -> 221 (2).
 // fp32 results show the length of their sums: `least` is the number of shares that they have now.
-static int quad_shares(int64_t tiles, int64_t outputs, int64_t K, int least, int64_t ws_bytes, double now) {
+static int quad_shares(int64_t tiles, int64_t outputs, int64_t K, int least, int64_t ws_bytes, double now, int most = 16) {
     const int64_t nt = (K + 63) / 64;
     int best = 1;
     double best_us = std::min(0.97 * now, now - 4);
-    for (int s = least > 2 ? least : 2; s <= 16 && s * outputs * 4 <= ws_bytes; ++s) {
+    for (int s = least > 2 ? least : 2; s <= most && s * outputs * 4 <= ws_bytes; ++s) {
         const int64_t share = quad_share(K, s), rounds = (tiles * s + 255) / 256;
         if (nt - (s - 1) * share < 3) continue;  // (the last one's, made even: four K-tiles at least)
         const double filled = (double)(tiles * s) / (double)(rounds * 256), hot = std::max(1.0, 0.35 + 1.08 * filled), length = std::min(1.0, std::max(0.0, (double)(rounds * share - 40) / 80));
@@ -2385,10 +2400,29 @@ static int quad_shares(int64_t tiles, int64_t outputs, int64_t K, int least, int
     return best;
 }
 
-// the same of one plain product (NT, TN) that the automatic choice is about to give to other tiles
+// input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
+// 128x128 / 256x256: K = 248 320, 333 rows 294 / 304, 602 585 / 446, 2 048 1 298 / 1 092; K = 20 000, 708 rows 54 / 57, 1 300 88 / 82; by 768, K = 50 256, 602 rows 83 / 81
+static bool long_split_nn(int64_t M, int64_t N, int64_t K, bool may_split, int64_t workspace_bytes) {
+    return may_split && !(N & 7) && workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
+}
+
+// the same of one plain product that the automatic choice is about to give to other tiles
 static int quad_shares_of(int form, int64_t M, int64_t N, int64_t K, int out_dtype, int64_t ws_bytes) {
     const int64_t tiles = ((M + 255) / 256) * ((N + 255) / 256), nt = (K + 63) / 64, t128 = ((M + 127) / 128) * ((N + 127) / 128);
-    if (form == MI355_GEMM_NN || M < 256 || N < 256 || tiles >= 256 || nt < 64) return 1;
+    if (M < 256 || N < 256 || tiles >= 256 || nt < 64) return 1;
+    if (form == MI355_GEMM_NN) {
+        // long sums only: as above with many more shares of few tiles (their K-tiles, 0.86 us a pair on 128x128 tiles and 2.45 on eight waves' 256x256, are what the transposing reads make of them)
+        if (small_tiles(form, M, N, MI355_EPI_NONE) && nt < 256) return 1;
+        int ksplit, fold;
+        double now;
+        if (!small_tiles(form, M, N, MI355_EPI_NONE)) now = 12 + (double)nt * (0.35 + 1.08 * (double)tiles / 256);
+        else if (long_split_nn(M, N, K, true, ws_bytes)) now = 10 + 2.45 * (double)nt / (double)(256 / tiles);
+        else if (!choose_ring(form, M, N, K, out_dtype, true, ws_bytes, ksplit, fold, now)) {
+            const int ks = choose_ksplit(t128, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes);
+            now = 10 + 0.86 * (double)((t128 * ks + 255) / 256) * (double)((nt + ks - 1) / ks);
+        }
+        return quad_shares(tiles, M * N, K, 1, ws_bytes, now, 32);
+    }
     const int ks = choose_ksplit(t128, 512, K, M, N, MI355_EPI_NONE, nullptr, 0, 0, ws_bytes);
     const int64_t rounds = (t128 * ks + 255) / 256;
     double now = 4 + (double)(rounds * ((nt + ks - 1) / ks)) * (rounds == 1 ? 0.67 : 0.49) + (ks > 1 ? 3 + (double)(ks * M * N) * 8 / 4.5e6 : 0);  // 128x128, two a CU
@@ -2402,12 +2436,6 @@ static int quad_shares_of(int form, int64_t M, int64_t N, int64_t K, int out_dty
         now = 12 + (double)nt * (0.35 + 1.08 * (double)tiles / 256), least = 1;
     }
     return quad_shares(tiles, M * N, K, out_dtype == MI355_DT_F32 ? least : 1, ws_bytes, now);
-}
-
-// input gradients of a vocabulary-wide layer: a long K split over the chip fills it with either tile, and the larger one needs half the bytes from LDS.  By 1 024 columns, us,
-// 128x128 / 256x256: K = 248 320, 333 rows 294 / 304, 602 585 / 446, 2 048 1 298 / 1 092; K = 20 000, 708 rows 54 / 57, 1 300 88 / 82; by 768, K = 50 256, 602 rows 83 / 81
-static bool long_split_nn(int64_t M, int64_t N, int64_t K, bool may_split, int64_t workspace_bytes) {
-    return may_split && !(N & 7) && workspace_bytes >= 64 * M * N && ((M > 512 && K >= 32768) || (M >= 1024 && K >= 16384));
 }
 
 // (what gemm_ring_kernel would take: of those, gemm_quad.h takes the ones that are faster in its shares of K)
@@ -2494,7 +2522,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         // 217 / 223, 333 281 / 276, 500 363 / 336, 700 437 / 421; 151 936 x 1 024 97 / 89, 113 / 110, 139 / 143, 175 / 178, 226 / 213, 272 / 263)
         else if (form == MI355_GEMM_TN) cfg = M * N <= 5 * 1024 * 1024 || tiles256 < 160 ? 1 : K >= 1024 ? 5 : tiles256 >= 1024 ? ((K - 1) % 64 >= 32 ? 2 : 3) : 1;
         else if (form == MI355_GEMM_NT) cfg = 2;
-        else cfg = 3;
+        else cfg = quad_ok(form, p, out_dtype) ? 7 : 3;
     }
     const bool persist_ok = form == MI355_GEMM_NT && out_dtype == MI355_DT_BF16 && (epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_SWIGLU_FWD || epilogue == MI355_EPI_SWIGLU_BWD) &&
                             !bias && (K & 63) == 0 && K >= 128 && (N & 7) == 0 && (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && M >= 256 && N >= 256 &&
@@ -2505,10 +2533,10 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         const int kind_bit = epilogue == MI355_EPI_SWIGLU_FWD ? 4 : epilogue == MI355_EPI_SWIGLU_BWD ? 8 : residual ? 2 : 1;
         cfg = persist_ok && tiles256 >= persist_min_tiles() && (pp_mask() & kind_bit) ? 8 : 7;
     }
-    if (tile_hint == 0 && ablate == 0 && epilogue == MI355_EPI_NONE && !bias && workspace && !(ldc & 3) && (!residual || !(ldr & 3)) && (cfg == 1 || cfg == 7) && quad_ok(form, p, out_dtype)) {
+    if (tile_hint == 0 && ablate == 0 && epilogue == MI355_EPI_NONE && !bias && workspace && !(ldc & 3) && (!residual || !(ldr & 3)) && (cfg == 1 || cfg == 7 || cfg == 3) && quad_ok(form, p, out_dtype)) {
         p.ksplit = quad_shares_of(form, M, N, K, out_dtype, workspace_bytes), p.ws = (float*)workspace;
         const bool persistent = tiles256 * p.ksplit >= persist_min_tiles();
-        if (p.ksplit > 1) return form == MI355_GEMM_TN ? mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s) : mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s);
+        if (p.ksplit > 1) return launch_quad_form(form, p, out_dtype, persistent, s);
     }
     // A last round of few 256x256 tiles costs as much as a full one.  Where they are few -- one to three full rounds and a remainder that 128x128 tiles (split over K as ever)
     // cover with at most one workgroup per CU -- the row panels of the full rounds go first and the remaining rows follow on the small tiles.  17 016 rows (24 samples of 709
@@ -2521,7 +2549,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
             const int64_t esz = out_dtype == MI355_DT_F32 ? 4 : 2, rsz = epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_GELU_ERF ? esz : 2;
             if (int rc = mi355_gemm_bf16(form, m_main, N, K, A, lda, B, ldb, C, ldc, out_dtype, bias, residual, ldr, epilogue, workspace, workspace_bytes, 0, stream)) return rc;
             return mi355_gemm_bf16(form, M - m_main, N, K, (const bf16_t*)A + m_main * lda, lda, B, ldb, (char*)C + m_main * ldc * esz, ldc, out_dtype, bias,
-                                   residual ? (const char*)residual + m_main * ldr * rsz : nullptr, ldr, epilogue, workspace, workspace_bytes, form == MI355_GEMM_NT ? 0 : 1, stream);
+                                   residual ? (const char*)residual + m_main * ldr * rsz : nullptr, ldr, epilogue, workspace, workspace_bytes, form == MI355_GEMM_NT || cfg == 7 ? 0 : 1, stream);
         }
     }
     if (cfg == 8) {  // ping-pong form: needs at least as many K-tiles as write-out slots
@@ -2530,7 +2558,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     }
     if (cfg == 7) {
         const bool persistent = tile_hint == 7 || tiles256 >= persist_min_tiles();
-        if (quad_ok(form, p, out_dtype)) return form == MI355_GEMM_TN ? mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s) : mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s);
+        if (quad_ok(form, p, out_dtype)) return launch_quad_form(form, p, out_dtype, persistent, s);
         cfg = 2;
     }
     const bool ring_epilogue = epilogue == MI355_EPI_NONE || (out_dtype == MI355_DT_BF16 && epilogue == (form == MI355_GEMM_NT ? MI355_EPI_GELU_ERF : MI355_EPI_SWIGLU_BWD));

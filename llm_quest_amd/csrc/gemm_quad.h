@@ -12,6 +12,8 @@
 //   * The stream of K-tiles runs on over a workgroup's tiles: while one is written out the next one's first two K-tiles are under way.
 //   * Edges: rows (NT) or K (TN) past the end lie beyond num_records of the stream's buffer descriptor, columns (TN) past the end get the offset OOB: both load zeros.  An odd number of
 //     K-tiles is made even by one of zeros.
+//   * NN: A as in the NT form, B's panels as in the TN form, fragments by transposing reads.  us, copy of the weight + NT -> NN: 16 384 x 1 024, K = 3 072 78.7 -> 73.6, 6 144 146 -> 140.5; 5 664 x 3 584,
+//     K = 1 024 60 -> 50; eight waves' tile -> here in shares of K: 602 x 1 024, K = 151 936 292 -> 182, 1 300 x 1 024, K = 20 032 90 -> 63.
 //   * Write-out from the registers: B's fragment is the product's first operand, so a lane holds four consecutive columns of a row; v_permlane16_swap makes eight of them, a rotation by eight lanes makes
 //     whole rows of 128 bytes, and no LDS is touched.  Whole lines with the non-temporal hint leave the L2 to the operands: 16 384 x 4 096, K = 1 024 107.0 -> 103.9 us (segments of 64 bytes 109.7).
 //     (Beside the products of the last and the next K-tile instead of between them: level.  Stores left out: 91.8.)
@@ -20,19 +22,21 @@
 constexpr int QUAD_RES = 16, QUAD_BIAS = 32;  // added to KIND (MI355_EPI_NONE): residual, bias
 constexpr int QUAD_SPLIT = 64;                // alone: p.ksplit shares of K, each with its own fp32 [M, N] of p.ws (splitk_reduce_kernel adds them up)
 
-// q, q + G, ... < ntiles: the tiles (SPLIT: and shares of K, those of one share after each other) of this workgroup (CHUNK: in a numbering that deals them over the XCDs).  TR: both operands K-strided (TN), else both K-contiguous (NT).  More than three K-tiles.
-template <bool TR, int OUT_DT, int KIND_, bool CHUNK = true>
+// q, q + G, ... < ntiles: the tiles (SPLIT: and shares of K, those of one share after each other) of this workgroup (CHUNK: in a numbering that deals them over the XCDs).  FORM: which operands are K-strided, none (NT), B (NN) or both (TN).  More than three K-tiles.
+template <int FORM, int OUT_DT, int KIND_, bool CHUNK = true>
 __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int G, const int ntiles, char* smem) {
     constexpr int KIND = KIND_ & 15, ADD = KIND_ & ~15;
+    constexpr bool TA = FORM == MI355_GEMM_TN, TB = FORM != MI355_GEMM_NT;
+    static_assert(!TB || KIND != MI355_EPI_SWIGLU_FWD);
     constexpr bool B16 = OUT_DT == MI355_DT_BF16, SPLIT = ADD == QUAD_SPLIT;
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave >> 1, wn = wave & 1;
     const int nt_all = (int)((p.K + 63) >> 6), nt_even = nt_all + (nt_all & 1), per = SPLIT ? (int)quad_share(p.K, p.ksplit) : 0;
     constexpr int ESZ = B16 ? 2 : 4;
 
-    // tile number -> its corner and first K-tile: XCD-chunked, row groups under every column panel (six NT, three TN: see gemm_tile)
+    // tile number -> its corner and first K-tile: XCD-chunked, row groups under every column panel (six NT and NN, three TN: see gemm_tile)
     auto origin = [&](int t, int& m0, int& n0, int& k0) {
-        constexpr int GROUP_M = TR ? 3 : 6;
+        constexpr int GROUP_M = TA ? 3 : 6;
         int pid = CHUNK ? xcd_chunked(t, ntiles) : t;
         k0 = 0;
         if constexpr (SPLIT) {
@@ -52,36 +56,29 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                if constexpr (TR) {  // [64 k][128 columns], swizzled as in piece_offsets
-                    const int k = wave * 16 + j * 4 + (lane >> 4), c = (lane & 15) ^ (tr_f(k) << 1);
-                    const int col = (c >> 3) * 128 + h * 64 + (c & 7) * 8;
-                    vA[h][j] = col < p.M - m0 ? (unsigned)((k * p.lda + col) * 2) : OOB;
-                    vB[h][j] = col < p.N - n0 ? (unsigned)((k * p.ldb + col) * 2) : OOB;
-                } else {  // [128 rows][64 k]
-                    const int r = wave * 32 + j * 8 + (lane >> 3), c = swz_rowk<64>(lane & 7, r) * 16;
-                    const int row = (r >> 6) * 128 + h * 64 + (r & 63);
-                    vA[h][j] = (unsigned)(row * p.lda * 2 + c);
-                    vB[h][j] = (unsigned)((KIND == MI355_EPI_SWIGLU_FWD ? h * (p.N >> 1) + r : row) * p.ldb * 2 + c);
-                }
+                // K-strided: [64 k][128 columns], swizzled as in piece_offsets
+                const int k = wave * 16 + j * 4 + (lane >> 4), ck = (lane & 15) ^ (tr_f(k) << 1), col = (ck >> 3) * 128 + h * 64 + (ck & 7) * 8;
+                // K-contiguous: [128 rows][64 k]
+                const int r = wave * 32 + j * 8 + (lane >> 3), c = swz_rowk<64>(lane & 7, r) * 16, row = (r >> 6) * 128 + h * 64 + (r & 63);
+                if constexpr (TA) vA[h][j] = col < p.M - m0 ? (unsigned)((k * p.lda + col) * 2) : OOB;
+                else vA[h][j] = (unsigned)(row * p.lda * 2 + c);
+                if constexpr (TB) vB[h][j] = col < p.N - n0 ? (unsigned)((k * p.ldb + col) * 2) : OOB;
+                else vB[h][j] = (unsigned)((KIND == MI355_EPI_SWIGLU_FWD ? h * (p.N >> 1) + r : row) * p.ldb * 2 + c);
             }
     };
-    const char *baseA, *baseB;  // the K-tile requested next, its number, its buffers' sizes (NT: to the end of the tile's last row; TN: of the K-tile's last row)
+    const char *baseA, *baseB;  // the K-tile requested next, its number, its buffers' sizes (K-contiguous: to the end of the tile's last row; K-strided: of the K-tile's last row)
     int kreq = 0, recA = 0, recB = 0;
     int tailA = 0, tailB = 0;
-    const int tail_at = TR && (p.K & 63) ? nt_all - 1 : -1;  // the K-tile that K ends in
-    const int64_t stepA = TR ? 128 * p.lda : 128, stepB = TR ? 128 * p.ldb : 128;
+    const int tail_at = TA && (p.K & 63) ? nt_all - 1 : -1;  // the K-tile that K ends in
+    const int64_t stepA = TA ? 128 * p.lda : 128, stepB = TB ? 128 * p.ldb : 128;
     auto open = [&](int m0, int n0, int k0) {
         kreq = k0;
-        if constexpr (TR) {
-            baseA = (const char*)uniform_ptr(p.A + m0), baseB = (const char*)uniform_ptr(p.B + n0);
-            recA = (int)(128 * p.lda), recB = (int)(128 * p.ldb);
-            tailA = (int)(((p.K & 63) * p.lda - m0) * 2), tailB = (int)(((p.K & 63) * p.ldb - n0) * 2);
-            plan(m0, n0);
-        } else {
-            const int64_t bn0 = KIND == MI355_EPI_SWIGLU_FWD ? n0 >> 1 : n0;
-            baseA = (const char*)uniform_ptr(p.A + m0 * p.lda), baseB = (const char*)uniform_ptr(p.B + bn0 * p.ldb);
-            recA = (int)(min((int64_t)256, p.M - m0) * p.lda * 2), recB = (int)((KIND == MI355_EPI_SWIGLU_FWD ? p.N - bn0 : min((int64_t)256, p.N - bn0)) * p.ldb * 2);
-        }
+        const int64_t bn0 = KIND == MI355_EPI_SWIGLU_FWD ? n0 >> 1 : n0;
+        baseA = (const char*)uniform_ptr(TA ? p.A + m0 : p.A + m0 * p.lda), baseB = (const char*)uniform_ptr(TB ? p.B + n0 : p.B + bn0 * p.ldb);
+        recA = (int)(TA ? 128 * p.lda : min((int64_t)256, p.M - m0) * p.lda * 2);
+        recB = (int)(TB ? 128 * p.ldb : (KIND == MI355_EPI_SWIGLU_FWD ? p.N - bn0 : min((int64_t)256, p.N - bn0)) * p.ldb * 2);
+        if constexpr (TA) tailA = (int)(((p.K & 63) * p.lda - m0) * 2), tailB = (int)(((p.K & 63) * p.ldb - n0) * 2);
+        if constexpr (TB) plan(m0, n0);
         if constexpr (SPLIT) baseA += k0 * stepA, baseB += k0 * stepB;
     };
     auto advance = [&]() {
@@ -89,7 +86,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
         baseA += stepA, baseB += stepB;
     };
     auto request = [&](int stage, int panel, int j) {  // panels 0, 1: A0, A1; 2, 3: B0, B1
-        const int rec = TR && kreq == tail_at ? (panel < 2 ? tailA : tailB) : panel < 2 ? recA : recB;
+        const int rec = TA && kreq == tail_at ? (panel < 2 ? tailA : tailB) : panel < 2 ? recA : recB;
         dma_piece(panel < 2 ? baseA : baseB, panel < 2 ? vA[panel & 1][j] : vB[panel & 1][j], smem + stage * QUAD_STAGE + panel * QUAD_PANEL + wave * 4096 + j * 1024, kreq < nt_all ? rec : 0);
     };
 
@@ -98,7 +95,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     const int r16 = lane & 15;
     const int off0 = r16 * 128 + (swz_rowk<64>(lane >> 4, r16) << 4);  // the swizzle of a row goes by its last four bits: one lane offset a k-step serves every fragment
     [[maybe_unused]] unsigned offA[4], offB[4];
-    if constexpr (TR) {  // the XOR of a lane's row reaches into the column bits: one lane offset per column tile (frag_tr)
+    if constexpr (TB) {  // the XOR of a lane's row reaches into the column bits: one lane offset per column tile (frag_tr)
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int g = lane >> 4, kq = (lane >> 2) & 3, fx = (kq | ((g & 1) << 2)) << 1, row = (8 * g + kq) * 256 + (lane & 1) * 8;
@@ -111,7 +108,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
         TrHalves(&h)[2][4] = halves;
         constexpr int STAGE = decltype(stage_c)::value, PANEL = decltype(panel_c)::value;
         const int kk = n >> 2, i = n & 3;
-        if constexpr (TR) {
+        if constexpr (PANEL < 2 ? TA : TB) {
             const unsigned addr = (PANEL < 2 ? offA[i] : offB[i]) + STAGE * QUAD_STAGE;
             if (kk == 0) asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%c3\n\tds_read_b64_tr_b16 %1, %2 offset:%c4" : "=&v"(h[0][i].lo), "=&v"(h[0][i].hi) : "v"(addr), "i"(PANEL * QUAD_PANEL), "i"(PANEL * QUAD_PANEL + 1024));
             else asm volatile("ds_read_b64_tr_b16 %0, %2 offset:%c3\n\tds_read_b64_tr_b16 %1, %2 offset:%c4" : "=&v"(h[1][i].lo), "=&v"(h[1][i].hi) : "v"(addr), "i"(PANEL * QUAD_PANEL + 8192), "i"(PANEL * QUAD_PANEL + 9216));
@@ -119,8 +116,8 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
             f[kk][i] = *reinterpret_cast<const bf16x8*>(smem + STAGE * QUAD_STAGE + PANEL * QUAD_PANEL + (PANEL < 2 ? wm : wn) * 8192 + i * 2048 + (off0 ^ (kk * 64)));
         }
     };
-    auto join = [&](bf16x8 (&f)[2][4]) __attribute__((always_inline)) {  // TR: waits for the reads of a phase
-        if constexpr (TR) {
+    auto join = [&](bf16x8 (&f)[2][4], auto panel_c) __attribute__((always_inline)) {  // a K-strided panel's reads: waits for those of a phase
+        if constexpr (decltype(panel_c)::value < 2 ? TA : TB) {
             TrHalves(&h)[2][4] = halves;
             asm volatile("s_waitcnt lgkmcnt(0)" : TRH(h[0][0]), TRH(h[0][1]), TRH(h[0][2]), TRH(h[0][3]), TRH(h[1][0]), TRH(h[1][1]), TRH(h[1][2]), TRH(h[1][3])::"memory");
 #pragma unroll
@@ -147,7 +144,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
             if ((s & 7) == 5) request(qstage, qpanel, s >> 3);
             __builtin_amdgcn_sched_barrier(0);
         }
-        join(next);
+        join(next, rpanel);
         if constexpr (WAIT >= 0) {
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             asm volatile("s_waitcnt vmcnt(%0)" ::"n"(WAIT) : "memory");
@@ -170,7 +167,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
 
     int m0, n0, k0;
     origin(q, m0, n0, k0);
-    if constexpr (!TR) plan(m0, n0);
+    if constexpr (!TB) plan(m0, n0);
     open(m0, n0, k0);
 #pragma unroll
     for (int st = 0; st < 2; ++st) {
@@ -182,10 +179,10 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int n = 0; n < 8; ++n) read_frag(fa[0], I0{}, I0{}, n);
-    join(fa[0]);
+    join(fa[0], I0{});
 #pragma unroll
     for (int n = 0; n < 8; ++n) read_frag(fb[0], I0{}, I2{}, n);
-    join(fb[0]);
+    join(fb[0], I2{});
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_sched_barrier(0);
@@ -403,10 +400,10 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the zeros past the end must not reach the LDS of a workgroup that follows
 }
 
-template <bool TR, int OUT_DT, int KIND>
+template <int FORM, int OUT_DT, int KIND>
 __global__ __launch_bounds__(256, 1) void gemm_quad_kernel(GemmParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    quad_tiles<TR, OUT_DT, KIND>(p, blockIdx.x, gridDim.x, p.tiles_m * p.tiles_n * (KIND == QUAD_SPLIT ? p.ksplit : 1), smem);
+    quad_tiles<FORM, OUT_DT, KIND>(p, blockIdx.x, gridDim.x, p.tiles_m * p.tiles_n * (KIND == QUAD_SPLIT ? p.ksplit : 1), smem);
 }
 
 // several problems of the TN form in one launch, a workgroup per tile, or per tile and share of K (see gemm_grouped_kernel)
@@ -421,7 +418,7 @@ __global__ __launch_bounds__(256, 1) void gemm_quad_grouped_kernel(GroupTable tb
     for (int i = 1; i < MAX_GROUP; ++i)
         if (i < tbl.count && v >= tbl.start[i]) g = i;
     const GemmParams p = tbl.g[g];
-    quad_tiles<true, OUT_DT, SPLIT ? QUAD_SPLIT : QUAD_RES, false>(p, v - tbl.start[g] + share * p.tiles_m * p.tiles_n, 1 << 30, p.tiles_m * p.tiles_n * (SPLIT ? p.ksplit : 1), smem);
+    quad_tiles<MI355_GEMM_TN, OUT_DT, SPLIT ? QUAD_SPLIT : QUAD_RES, false>(p, v - tbl.start[g] + share * p.tiles_m * p.tiles_n, 1 << 30, p.tiles_m * p.tiles_n * (SPLIT ? p.ksplit : 1), smem);
 }
 
 // C = the sum of a problem's shares, in their order (+ R).  U groups of four columns a thread, start[i] the first block of problem i.  Four shares' loads go out before the first is added.

@@ -113,7 +113,7 @@ def _persist_min_tiles():
 
 
 def _nt_tick(M, N, eligible=True, device=None):
-    """Called in front of every NT launch.  Counts only launches the library would put on the persistent kernel (csrc/gemm.hip ``persist_ok``: bf16 output, no bias,
+    """Called in front of every NT launch, and of an input gradient that stands in its place (``dgrad_on_quad``).  Counts only launches the library would put on the persistent kernel (csrc/gemm.hip ``persist_ok``: bf16 output, no bias,
     plain / SwiGLU epilogue, no tile hint -- the caller says so through ``eligible`` -- and at least the threshold's tiles), and only those of the window's own stream."""
     if not eligible or ((M + 255) // 256) * ((N + 255) // 256) < _persist_min_tiles():
         return
@@ -302,7 +302,10 @@ def gemm_dgrad_swiglu_bwd(dy, w, gu, tile=0):
     if dy.dtype != BF16 or w.dtype != BF16 or gu.dtype != BF16 or w.shape[0] != Kd or not gu.is_contiguous() or tuple(gu.shape) != (M, 2 * F):
         raise ValueError("gemm_dgrad_swiglu_bwd: dY [M, N_out], W [N_out, F], gate-up output contiguous [M, 2F], all bf16")
     out = torch.empty_like(gu)
-    if DGRAD_NT and M >= DGRAD_NT_MIN_ROWS:
+    quad = M >= DGRAD_NT_MIN_ROWS and not tile and not _TILE_SWIGLU_BWD and dgrad_on_quad(M, F, Kd, epilogue=True)
+    if quad:
+        _nt_tick(M, F, device=dy.device)
+    if DGRAD_NT and M >= DGRAD_NT_MIN_ROWS and not quad:
         wt = transpose(w)  # [F, N_out]: the same product in the K-contiguous form
         _nt_tick(M, F, eligible=not (tile or _TILE_SWIGLU_BWD or _TILE_BY_FORM[L.GEMM_NT] or _TILE_OVERRIDE) and Kd % 64 == 0 and Kd >= 128, device=dy.device)
         L.call("mi355_gemm_bf16", L.GEMM_NT, M, F, Kd, L.ptr(dy), dy.stride(0), L.ptr(wt), wt.stride(0), L.ptr(out), out.stride(0), L.DT_BF16, None,
@@ -734,14 +737,26 @@ def dgrad_on_ring(M, N, Kd, dtype=BF16):
     return r != 0 and (r != (128 | 1 << 8) or Kd < 6144)
 
 
+def dgrad_on_quad(M, N, Kd, out=None, epilogue=False):
+    """Whether dX [M, N] = dY [M, Kd] W runs in the NN form on 256 x 256 tiles of four waves (csrc/gemm_quad.h), as fast there as in the NT form and without the copy: more than half of the CUs' worth of tiles, or
+    a sum that is divided over the chip.  us, copy + NT / NN: 16 384 x 1 024, K = 3 072 78.7 / 73.6, 6 144 146 / 140.5; 5 664 x 3 584, K = 1 024 60.1 / 49.8; 25 216 x 3 072, K = 768 111.6 / 109.2;
+    12 288 x 1 024, K = 151 936 2 735 / 2 655; 5 664 x 1 024, K = 248 320 2 296 / 2 132."""
+    if (out is not None and (out.dtype != BF16 or out.data_ptr() % 16 or out.stride(0) % 8)) or any(_TILE_BY_FORM.values()) or _TILE_OVERRIDE:
+        return False
+    tiles = ((M + 255) // 256) * ((N + 255) // 256)
+    return min(M, N) >= 256 and N % 8 == 0 and Kd % 64 == 0 and Kd > 192 and (tiles > 128 or (Kd > 16384 and not epilogue))
+
+
 @L.native
 def dgrad(dy, w, out=None):
-    """dX = dY W for a Linear with weight W [N_out, N_in].  Where ``dgrad_transposes`` says so and ``dgrad_on_ring`` does not, W is transposed first (one pass over the
-    weight, 63 MB per transformer block) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads.
+    """dX = dY W for a Linear with weight W [N_out, N_in].  Where ``dgrad_transposes`` says so and neither ``dgrad_on_ring`` nor ``dgrad_on_quad`` does, W is transposed first (one pass over the
+    weight) and the product runs in the K-contiguous NT form, whose main loop needs no transposing LDS reads.
     The result is the same sum in the same order per K-tile, bit-identical to the NN form where neither is split over K."""
     M, (Kd, N) = dy.shape[0], w.shape
     if DGRAD_NT and dgrad_transposes(M, N, Kd) and (Kd & 7) == 0 and (N & 7) == 0 and not dgrad_on_ring(M, N, Kd, BF16 if out is None else out.dtype):
-        return gemm(L.GEMM_NT, dy, transpose(w), out=out)
+        if not dgrad_on_quad(M, N, Kd, out):
+            return gemm(L.GEMM_NT, dy, transpose(w), out=out)
+        _nt_tick(M, N, device=dy.device)
     return gemm(L.GEMM_NN, dy, w, out=out)
 
 

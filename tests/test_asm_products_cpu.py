@@ -121,7 +121,7 @@ def test_the_reader_finds_an_early_access():
 
 @pytest.mark.skipif(shutil.which("hipcc") is None, reason="no hipcc")
 @pytest.mark.parametrize("source,define,least", [("attention_generic.hip", [], 9),  # the three kernels at head dim 256, with and without dropout
-                                                 ("gemm.hip", ["-DGEMM_PART=8"], 11), ("gemm.hip", ["-DGEMM_PART=9"], 6),  # four waves of 128x128 (gemm_quad.h)
+                                                 ("gemm.hip", ["-DGEMM_PART=8"], 11), ("gemm.hip", ["-DGEMM_PART=9"], 6), ("gemm.hip", ["-DGEMM_PART=10"], 4),  # four waves of 128x128 (gemm_quad.h)
                                                  ("bgemm.hip", [], 2)])  # (bgemm_quad.h)
 def test_tiles_of_asm_products_are_read_late_enough(tmp_path, source, define, least):
     make = open(os.path.join(CSRC, "Makefile")).read()

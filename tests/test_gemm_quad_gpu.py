@@ -34,6 +34,38 @@ def test_nt_gives_the_bits_of_the_eight_wave_tile(M, N, K_, odt, bias, residual)
     assert torch.equal(nt(A, B, odt, b, r, 7, 8), nt(A, B, odt, b, r, 2, 8))
 
 
+# weights as they lie: rows of A end inside a tile, columns of B too (its rows are K's, whole K-tiles); odd and even counts of K-tiles; more tiles than CUs
+@pytest.mark.parametrize("M,N,K_", [(1, 256, 256), (257, 264, 320), (383, 520, 448), (512, 512, 576), (700, 8, 1024), (130, 1288, 2048), (33_000, 520, 256), (17_000, 1800, 320)])
+@pytest.mark.parametrize("kind", ["plain", "residual", "swiglu"])
+def test_nn_gives_the_bits_of_the_eight_wave_tile(M, N, K_, kind):
+    A, B, W = draw(M, M, K_ + 8)[:, :K_], draw(N, K_, N + 24)[:, :N], 2 * N if kind == "swiglu" else N
+    r = None if kind == "plain" else draw(4, M, W + 16)[:, :W]
+
+    def take(hint):
+        C = torch.full((M + 1, W + 8), 7.0, dtype=BF16, device="cuda")
+        L.call("mi355_gemm_bf16", L.GEMM_NN, M, N, K_, L.ptr(A), A.stride(0), L.ptr(B), B.stride(0), L.ptr(C), C.stride(0), L.DT_BF16, None, L.ptr(r), 0 if r is None else r.stride(0),
+               L.EPI_SWIGLU_BWD if kind == "swiglu" else 0, None, 0, hint)
+        assert bool((C[M:] == 7).all()) and bool((C[:, W:] == 7).all())
+        return C[:M, :W]
+
+    assert torch.equal(take(7), take(2))
+
+
+# the library's own choice of input gradients: a main part and a remainder on small tiles, long sums in shares of K (one tile in 32, eight, 32 and 192 tiles), plain and behind SwiGLU; against the transposed weight's product
+@pytest.mark.parametrize("M,N,K_", [(4352, 3080, 256), (17016, 1024, 320), (2836, 3072, 1024), (256, 256, 20032), (333, 1024, 50304), (1300, 1000, 33024), (12100, 1000, 16448), (498, 2048, 16384)])
+def test_input_gradients_of_weights_as_they_lie(M, N, K_):
+    dy, w = draw(M, M, K_), draw(N, K_, N) * K_**-0.5
+    wt = w.T.contiguous()
+    got, want = K.dgrad(dy, w), dy.double() @ w.double() if M * K_ < 1e8 else None
+    assert off(got, K.gemm(L.GEMM_NT, dy, wt, out_dtype=F32), K_, BF16)
+    if want is not None:
+        assert off(got, want, K_, BF16)
+    if K_ <= 1024:
+        assert K.dgrad_on_quad(M, N, K_) and torch.equal(got, K.gemm(L.GEMM_NT, dy, wt, allow_split_k=False)) or M == 17016  # (its remainder's sums are cut in either form)
+        gu = draw(7, M, 2 * N)
+        assert torch.equal(K.gemm_dgrad_swiglu_bwd(dy, w, gu), K.swiglu_bwd(gu, K.gemm(L.GEMM_NN, dy, w, allow_split_k=False), N))
+
+
 # K = tokens: the shortest, remainders of one row and of all but one in the last K-tile, odd and even counts; columns that end inside a tile; more tiles than CUs
 @pytest.mark.parametrize("M,N,K_", [(256, 256, 193), (264, 520, 257), (512, 256, 1024), (1000, 1288, 639), (2048, 8, 705), (4104, 4360, 321)])
 @pytest.mark.parametrize("odt", [BF16, F32])
