@@ -58,6 +58,7 @@ SIGNATURES = {
     "mi355_patchify": [_I, _I, _I, _I, _I, _P, _P, _I, _P],
     "mi355_layernorm_fwd": [_L, _I, _P, _P, _P, _P, _I, _P, _P, _F, _I, _P],
     "mi355_layernorm_bwd_bf16": [_L, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _P, _I, _F, _I, _P],
+    "mi355_reduce_rows_each": [_P, _L, _I, _L, _P, _I] * 4 + [_P],
     "mi355_reduce_rows_into": [_I, _I, _L, _P, _P, _P, _P, _P, _I, _P],
     "mi355_layernorm_bwd": [_L, _I, _P, _P, _P, _P, _P, _I, _P, _P, _P, _I, _F, _I, _P],
     "mi355_cast": [_L, _P, _I, _P, _I, _P],

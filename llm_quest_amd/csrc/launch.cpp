@@ -16,7 +16,7 @@
 #define MI355_ENTRIES(E) \
     E(gemm_bf16) E(gemm_bf16_grouped) E(gemm_bf16_grouped_ws) E(gemm_bf16_attn_delta) E(adamw) E(colsum) E(rmsnorm_fwd) E(rmsnorm_bwd) E(reduce_rows_f32) E(qknorm_rope_fwd) E(qknorm_rope_bwd) \
     E(swiglu_fwd) E(swiglu_bwd) E(attn_fwd) E(attn_bwd) E(attn_bwd_ws) E(attn_bwd_qnorm) E(cross_entropy) E(ce_finalize) E(embedding_fwd) E(embedding_bwd) \
-    E(embedding_bwd_sorted) E(copy2d) E(transpose_bf16) E(patchify) E(layernorm_fwd) E(layernorm_bwd_bf16) E(reduce_rows_into) E(layernorm_bwd) E(cast) \
+    E(embedding_bwd_sorted) E(copy2d) E(transpose_bf16) E(patchify) E(layernorm_fwd) E(layernorm_bwd_bf16) E(reduce_rows_into) E(reduce_rows_each) E(layernorm_bwd) E(cast) \
     E(vit_embed_assemble) E(split3_bf16) E(attn_f32_fwd) E(sumsq) E(clip_scale) E(add_f32_to_bf16) E(scale_bf16) E(gelu_fwd) E(gelu_bwd) E(gelu_bwd_colsum) E(patchify3d) \
     E(merge_patches) E(scatter_rows) E(zc_weight) E(mrope_table) E(rowmask) E(headnorm_rope_fwd) E(headnorm_rope_bwd) E(sigmoid_gate_fwd) E(sigmoid_gate_bwd) \
     E(attn_generic_fwd) E(attn_generic_bwd) E(gdn_gates_fwd) E(gdn_gates_bwd) E(causal_conv_silu_fwd) E(causal_conv_silu_bwd) E(l2norm_fwd) E(l2norm_bwd) \

@@ -26,7 +26,7 @@
 
 #define WRAP_ENTRIES(E) \
     E(gemm_bf16) E(gemm_bf16_grouped_ws) E(colsum) E(rmsnorm_fwd) E(rmsnorm_bwd) E(reduce_rows_f32) E(qknorm_rope_fwd) E(qknorm_rope_bwd) E(swiglu_fwd) E(swiglu_bwd) E(attn_fwd) E(attn_bwd_ws) \
-    E(attn_bwd_qnorm) E(add_f32_to_bf16) E(layernorm_fwd) E(layernorm_bwd_bf16) E(reduce_rows_into) E(gelu_fwd) E(gelu_bwd_colsum) E(copy2d) E(zc_weight) E(headnorm_rope_fwd) E(headnorm_rope_bwd) \
+    E(attn_bwd_qnorm) E(add_f32_to_bf16) E(layernorm_fwd) E(layernorm_bwd_bf16) E(reduce_rows_into) E(reduce_rows_each) E(gelu_fwd) E(gelu_bwd_colsum) E(copy2d) E(zc_weight) E(headnorm_rope_fwd) E(headnorm_rope_bwd) \
     E(sigmoid_gate_fwd) E(sigmoid_gate_bwd) E(attn_generic_fwd) E(attn_generic_bwd) E(gdn_gates_fwd) E(gdn_gates_bwd) E(causal_conv_silu_fwd) E(causal_conv_silu_bwd) E(l2norm_fwd) E(l2norm_bwd) \
     E(gated_rmsnorm_fwd) E(gated_rmsnorm_bwd) E(gemv_bf16) E(gemv_bf16_f32out) E(hyper_mix) E(bgemm) E(latent_attn) E(qkv_rows_append) E(group_rmsnorm_sum) E(ragged_conv) E(gated_headnorm) E(glu_rows) \
     E(add_layernorm_fwd) E(rmsnorm_rows) E(latent_kv_append) E(rope_heads) E(gla_fwd) E(router_logits) E(moe_route) E(moe_dispatch) E(moe_choose) E(unary_rows) E(embed_hash_fwd)
@@ -392,7 +392,7 @@ OP(rmsnorm_fwd, "x2d", "w", "eps", "want_rstd") {
     return tuple(y, rstd);
 }
 
-OP(rmsnorm_bwd, "x2d", "w", "rstd", "dy", "dres", "dw_out", "dw_accumulate") {
+OP(rmsnorm_bwd, "x2d", "w", "rstd", "dy", "dres", "dw_out", "dw_accumulate", "partial") {
     const T x = c.tensor(0), w = c.tensor(1), rstd = c.tensor(2), dy = c.tensor(3), dres = c.maybe(4);
     T dw = c.maybe(5);
     need(x.dim() == 2 && dy.contiguous() && dy.like(x) && dy.is(BF16) && (!dres || (dres.contiguous() && dres.like(x) && dres.is(BF16))));
@@ -402,6 +402,7 @@ OP(rmsnorm_bwd, "x2d", "w", "rstd", "dy", "dres", "dw_out", "dw_accumulate") {
     const T dx = c.empty_like(x), part = c.empty(x, {parts, width}, F32);
     need(dry || slot::reduce_rows_f32.address);
     LAUNCH(rmsnorm_bwd, rows, width, x, w, rstd, dy, dres, dx, part, parts);
+    if (c.truth(7, false)) return tuple(dx, part);
     if (!dw) dw = c.empty(x, {width}, F32);
     LAUNCH(reduce_rows_f32, parts, width, part, dw, dw_code, (int)accumulate);
     return tuple(dx, dw);
@@ -418,7 +419,7 @@ OP(qknorm_rope_fwd, "qkv", "qw", "kw", "cos", "sin", "pos", "Hq", "Hkv", "D", "e
     return tuple(q, k, rstd);
 }
 
-OP(qknorm_rope_bwd, "qkv", "qw", "kw", "cos", "sin", "pos", "rstd", "dq", "dk", "dqkv", "Hq", "Hkv", "D") {
+OP(qknorm_rope_bwd, "qkv", "qw", "kw", "cos", "sin", "pos", "rstd", "dq", "dk", "dqkv", "Hq", "Hkv", "D", "partial") {
     const T qkv = c.tensor(0), qw = c.maybe(1), kw = c.maybe(2), cos = c.maybe(3), sin = c.maybe(4), pos = c.maybe(5), rstd = c.maybe(6), dq = c.maybe(7), dk = c.tensor(8), dqkv = c.tensor(9);
     const int64_t Hq = c.integer(10), Hkv = c.integer(11), D = c.integer(12);
     need(qkv.dim() == 2);
@@ -429,6 +430,7 @@ OP(qknorm_rope_bwd, "qkv", "qw", "kw", "cos", "sin", "pos", "rstd", "dq", "dk", 
     const T part = c.empty(qkv, {parts, 2 * D}, F32);
     need(dry || slot::reduce_rows_f32.address);
     LAUNCH(qknorm_rope_bwd, tokens, Hq, Hkv, D, qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, part, parts);
+    if (c.truth(13, false)) return tuple(T{part.t.narrow(1, 0, D)}, T{part.t.narrow(1, D, D)});
     const T dw = c.empty(qkv, {2 * D}, F32);
     LAUNCH(reduce_rows_f32, parts, 2 * D, part, dw, MI355_DT_F32, 0);
     return tuple(T{dw.t.narrow(0, 0, D)}, T{dw.t.narrow(0, D, D)});
@@ -515,7 +517,7 @@ OP(attn_bwd, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", "dq", 
     Py_RETURN_NONE;
 }
 
-OP(attn_bwd_qnorm, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", "dk", "dv", "qkv", "qw", "cos", "sin", "pos", "rstd", "dqkv", "key_mask", "causal", "scale", "delta") {
+OP(attn_bwd_qnorm, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", "dk", "dv", "qkv", "qw", "cos", "sin", "pos", "rstd", "dqkv", "key_mask", "causal", "scale", "delta", "partial") {
     const int64_t B = c.integer(6), S = c.integer(7), Hq = c.integer(8), Hkv = c.integer(9), D = c.integer(10);
     need(D == 128 && c.given(14) && kernels_true("FUSE_QNORM_BWD") && kernels_true("_ATTN_DS_SPILL"));
     const T q = c.tensor(0), k = c.tensor(1), v = c.tensor(2), o = c.tensor(3), dO = c.tensor(4), lse = c.tensor(5), dk = c.tensor(11), dv = c.tensor(12), qkv = c.tensor(13), qw = c.tensor(14), cos = c.tensor(15),
@@ -546,15 +548,18 @@ OP(attn_bwd_qnorm, "q", "k", "v", "o", "do", "lse", "B", "S", "Hq", "Hkv", "D", 
     const T part = c.empty(q, {parts, D}, F32);
     LAUNCH(attn_bwd_qnorm, B, S, Hq, Hkv, D, q, q.ld(), k, k.ld(), v, v.ld(), o, o.ld(), dO, dO.ld(), lse, delta, dk, dk.ld(), dv, dv.ld(), mask, flags, scale, ws, bytes, qkv, qkv.ld(), qw, cos, sin, pos, rstd,
            rstd.size(1), dqkv, dqkv.ld(), part, cs16);
-    const T dw = c.empty(q, {D}, F32);  // one partial row per workgroup: summed in two fixed-order levels
+    const bool partial = c.truth(24, false);
+    const T dw = partial ? T{} : c.empty(q, {D}, F32);  // one partial row per workgroup: summed in two fixed-order levels
     int64_t fold = 1;
     for (int64_t f : {64, 32, 16, 8})
         if (fold == 1 && parts % f == 0 && parts / f >= 8) fold = f;
     if (fold > 1) {
         const T mid = c.empty(q, {fold * D}, F32);
         LAUNCH(reduce_rows_f32, parts / fold, fold * D, part, mid, MI355_DT_F32, 0);
+        if (partial) return wrapped(T{mid.t.view({fold, D})});
         LAUNCH(reduce_rows_f32, fold, D, mid, dw, MI355_DT_F32, 0);
     } else {
+        if (partial) return wrapped(part);
         LAUNCH(reduce_rows_f32, parts, D, part, dw, MI355_DT_F32, 0);
     }
     return wrapped(dw);
@@ -601,6 +606,25 @@ Dests destinations(Call& c, PyObject* seq, int64_t width) {
     }
     need(any);
     return d;
+}
+
+OP(reduce_rows_each, "sums") {
+    need(c.v[0] && PyList_CheckExact(c.v[0]));
+    const int n = (int)PyList_GET_SIZE(c.v[0]);
+    need(n >= 1 && n <= 4);
+    T part[4], out[4];
+    int64_t parts[4] = {}, width[4] = {}, ld[4] = {}, flags[4] = {};
+    for (int i = 0; i < n; ++i) {
+        PyObject* q = PyList_GET_ITEM(c.v[0], i);
+        need(PyTuple_CheckExact(q) && PyTuple_GET_SIZE(q) == 3 && PyBool_Check(PyTuple_GET_ITEM(q, 2)));
+        part[i] = c.from(PyTuple_GET_ITEM(q, 0)), out[i] = c.from(PyTuple_GET_ITEM(q, 1));
+        need(part[i] && out[i] && part[i].rows() && part[i].is(F32) && part[i].numel() > 0 && out[i].contiguous() && out[i].numel() == part[i].size(1));
+        parts[i] = part[i].size(0), width[i] = part[i].size(1), ld[i] = parts[i] > 1 ? part[i].ld() : width[i];
+        flags[i] = (code(out[i].dtype()) == MI355_DT_BF16 ? 1 : 0) | (PyTuple_GET_ITEM(q, 2) == Py_True ? 2 : 0);
+    }
+    LAUNCH(reduce_rows_each, part[0], ld[0], parts[0], width[0], out[0], flags[0], part[1], ld[1], parts[1], width[1], out[1], flags[1], part[2], ld[2], parts[2], width[2], out[2], flags[2], part[3],
+           ld[3], parts[3], width[3], out[3], flags[3]);
+    Py_RETURN_NONE;
 }
 
 OP(reduce_rows_into, "partial", "parts", "width", "dests") {

@@ -341,8 +341,8 @@ def rmsnorm_fwd(x2d, w, eps=1e-6, want_rstd=True):
 
 
 @L.native
-def rmsnorm_bwd(x2d, w, rstd, dy, dres=None, dw_out=None, dw_accumulate=False):
-    """Returns (dx [+ dres], dw).  dw goes to ``dw_out`` (bf16/fp32, optionally accumulated) or a new fp32 tensor."""
+def rmsnorm_bwd(x2d, w, rstd, dy, dres=None, dw_out=None, dw_accumulate=False, partial=False):
+    """Returns (dx [+ dres], dw).  dw goes to ``dw_out`` (bf16/fp32, optionally accumulated) or a new fp32 tensor; ``partial``: it is left as fp32 rows to be added up (``reduce_rows_each``)."""
     L.require_gpu(x2d, w, rstd, dy, dres)
     rows, width = x2d.shape
     if not (dy.is_contiguous() and dy.shape == x2d.shape and dy.dtype == BF16):
@@ -353,6 +353,8 @@ def rmsnorm_bwd(x2d, w, rstd, dy, dres=None, dw_out=None, dw_accumulate=False):
     parts = min(NORM_PARTS, (rows + 3) // 4)
     part = torch.empty((parts, width), dtype=F32, device=x2d.device)
     L.call("mi355_rmsnorm_bwd", rows, width, L.ptr(x2d), L.ptr(w), L.ptr(rstd), L.ptr(dy), L.ptr(dres), L.ptr(dx), L.ptr(part), parts)
+    if partial:
+        return dx, part
     dw = torch.empty(width, dtype=F32, device=x2d.device) if dw_out is None else dw_out
     L.call("mi355_reduce_rows_f32", parts, width, L.ptr(part), L.ptr(dw), L.dt_code(dw.dtype), int(dw_accumulate and dw_out is not None))
     return dx, dw
@@ -377,8 +379,8 @@ def qknorm_rope_fwd(qkv, qw, kw, cos, sin, pos, Hq, Hkv, D, eps=1e-6):
 
 
 @L.native
-def qknorm_rope_bwd(qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, Hq, Hkv, D):
-    """Writes d(qkv)[:, :(Hq+Hkv)*D] into dqkv (the V third is left to the caller); returns (dqw_f32, dkw_f32).
+def qknorm_rope_bwd(qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, Hq, Hkv, D, partial=False):
+    """Writes d(qkv)[:, :(Hq+Hkv)*D] into dqkv (the V third is left to the caller); returns (dqw_f32, dkw_f32), ``partial``: as rows to be added up (``reduce_rows_each``).
     dq=None: the key heads only (the query heads' share ran inside attn_bwd_qnorm); dqw_f32 is then zeros."""
     L.require_gpu(qkv, dk, dqkv)
     tokens = qkv.shape[0]
@@ -394,6 +396,8 @@ def qknorm_rope_bwd(qkv, qw, kw, cos, sin, pos, rstd, dq, dk, dqkv, Hq, Hkv, D):
     parts = min(QK_PARTS, (tokens * ((Hq + Hkv + hpw - 1) // hpw) + 3) // 4)
     part = torch.empty((parts, 2 * D), dtype=F32, device=qkv.device)
     L.call("mi355_qknorm_rope_bwd", tokens, Hq, Hkv, D, L.ptr(qkv), L.ptr(qw), L.ptr(kw), L.ptr(cos), L.ptr(sin), L.ptr(pos), L.ptr(rstd), L.ptr(dq), L.ptr(dk), L.ptr(dqkv), L.ptr(part), parts)
+    if partial:
+        return part[:, :D], part[:, D:]
     dw = torch.empty(2 * D, dtype=F32, device=qkv.device)
     L.call("mi355_reduce_rows_f32", parts, 2 * D, L.ptr(part), L.ptr(dw), L.DT_F32, 0)
     return dw[:D], dw[D:]
@@ -580,9 +584,9 @@ def dgrad_attn_delta(dy, w, ctx, lse, B, S, Hq, D):
 
 
 @L.native
-def attn_bwd_qnorm(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dk, dv, qkv, qw, cos, sin, pos, rstd, dqkv, key_mask=None, causal=True, scale=None, delta=None):
+def attn_bwd_qnorm(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dk, dv, qkv, qw, cos, sin, pos, rstd, dqkv, key_mask=None, causal=True, scale=None, delta=None, partial=False):
     """attn_bwd whose dQ pass ends in the backward of the QK-norm + RoPE of the query heads: writes d(qkv)[:, :Hq*D] into ``dqkv`` (dQ never exists
-    as a matrix) and returns the fp32 [D] gradient of the query norm weight -- or None when this form does not apply (head_dim != 128, no scratch
+    as a matrix) and returns the fp32 [D] gradient of the query norm weight (``partial``: as rows to be added up) -- or None when this form does not apply (head_dim != 128, no scratch
     for the one-product dQ pass, knob off): the caller then runs attn_bwd + qknorm_rope_bwd."""
     if not (FUSE_QNORM_BWD and _ATTN_DS_SPILL and D == 128) or qw is None:
         return None
@@ -624,13 +628,17 @@ def attn_bwd_qnorm(q, k, v, o, do, lse, B, S, Hq, Hkv, D, dk, dv, qkv, qw, cos, 
         L.ptr(cs16),
     )
     # one partial row per workgroup: summed in two fixed-order levels (a single launch over thousands of rows runs on two workgroups)
-    dw = torch.empty(D, dtype=F32, device=q.device)
+    dw = None if partial else torch.empty(D, dtype=F32, device=q.device)
     fold = next((f for f in (64, 32, 16, 8) if parts % f == 0 and parts // f >= 8), 1)
     if fold > 1:
         mid = torch.empty(fold * D, dtype=F32, device=q.device)
         L.call("mi355_reduce_rows_f32", parts // fold, fold * D, L.ptr(part), L.ptr(mid), L.DT_F32, 0)
+        if partial:
+            return mid.view(fold, D)
         L.call("mi355_reduce_rows_f32", fold, D, L.ptr(mid), L.ptr(dw), L.DT_F32, 0)
     else:
+        if partial:
+            return part
         L.call("mi355_reduce_rows_f32", parts, D, L.ptr(part), L.ptr(dw), L.DT_F32, 0)
     return dw
 
@@ -958,6 +966,22 @@ def layernorm_bwd(x2d, scale, mean, rsig, dy, dres=None, eps=1e-5, dscale_out=No
                 L.call("mi355_reduce_rows_f32", 1, width, L.ptr(src.contiguous()), L.ptr(dst), L.DT_F32, 0)
             outs.append(dst)
     return dx, outs[0], outs[1]
+
+
+@L.native
+def reduce_rows_each(sums):
+    """Up to four (partial fp32 [parts, n] with unit inner stride, out [n] bf16 / fp32, accumulate): out (+)= the sum over the parts, one launch.  The bits of ``mi355_reduce_rows_f32``, and of that with
+    ``add_f32_to_bf16`` behind it."""
+    if not 1 <= len(sums) <= 4:
+        raise ValueError("reduce_rows_each: one to four sums")
+    args = []
+    for part, out, accumulate in sums:
+        L.require_gpu(part, out)
+        _rowmajor(part, "partial sums")
+        if part.dtype != F32 or part.numel() == 0 or not out.is_contiguous() or out.numel() != part.shape[1]:
+            raise ValueError("reduce_rows_each: fp32 rows, each with a contiguous destination of their width")
+        args += [L.ptr(part), part.stride(0) if part.shape[0] > 1 else part.shape[1], part.shape[0], part.shape[1], L.ptr(out), (L.dt_code(out.dtype) == L.DT_BF16) | bool(accumulate) << 1]
+    L.call("mi355_reduce_rows_each", *args, *[None, 0, 0, 0, None, 0] * (4 - len(sums)))
 
 
 @L.native

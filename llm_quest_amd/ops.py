@@ -113,27 +113,30 @@ def attention_forward(att, arena, h1, rt):
     return ctx, (qkv, q, k, rstd, lse)
 
 
-def attention_backward(att, arena, h1, ctx, saved, dctx, rt, defer=None, delta=None):
-    """Returns dh1 [M,d]; writes the QKV / QK-norm weight gradients.  ``delta``: the softmax backward's row sums when the out-projection's
+def attention_backward(att, arena, h1, ctx, saved, dctx, rt, defer=None, delta=None, sums=None):
+    """Returns dh1 [M,d]; writes the QKV / QK-norm weight gradients (the latter, where ``sums`` is a list, when the caller has it added up: ``kernels.reduce_rows_each``).  ``delta``: the softmax backward's row sums when the out-projection's
     dgrad already left them (kernels.dgrad_attn_delta)."""
     Hq, Hkv, D = att.num_heads, att.num_kv_groups, att.head_dim
     qkv, q, k, rstd, lse = saved
     v = qkv[:, (Hq + Hkv) * D :]
     dqkv = torch.empty_like(qkv)
     dk = torch.empty_like(k)
+    mine = [] if sums is None else sums
     # the dQ pass ends in the QK-norm + RoPE backward of the query heads when it can (head_dim 128, scratch for the one-product form) ...
     dqw = K.attn_bwd_qnorm(q, k, v, ctx, dctx, lse, rt.B, rt.S, Hq, Hkv, D, dk, dqkv[:, (Hq + Hkv) * D :], qkv, att.q_norm.weight, rt.cos, rt.sin, rt.pos, rstd, dqkv,
-                           key_mask=rt.key_mask, causal=True, scale=att.att_scaling, delta=delta)
+                           key_mask=rt.key_mask, causal=True, scale=att.att_scaling, delta=delta, partial=True)
     if dqw is not None:
-        _, dkw = K.qknorm_rope_bwd(qkv, att.q_norm.weight, att.k_norm.weight, rt.cos, rt.sin, rt.pos, rstd, None, dk, dqkv, Hq, Hkv, D)
+        _, dkw = K.qknorm_rope_bwd(qkv, att.q_norm.weight, att.k_norm.weight, rt.cos, rt.sin, rt.pos, rstd, None, dk, dqkv, Hq, Hkv, D, partial=True)
     else:  # ... otherwise dQ is a matrix and one kernel handles every head
         dq = torch.empty_like(q)
         K.attn_bwd(q, k, v, ctx, dctx, lse, rt.B, rt.S, Hq, Hkv, D, dq, dk, dqkv[:, (Hq + Hkv) * D :], key_mask=rt.key_mask, causal=True, scale=att.att_scaling)
-        dqw, dkw = K.qknorm_rope_bwd(qkv, att.q_norm.weight, att.k_norm.weight, rt.cos, rt.sin, rt.pos, rstd, dq, dk, dqkv, Hq, Hkv, D)
+        dqw, dkw = K.qknorm_rope_bwd(qkv, att.q_norm.weight, att.k_norm.weight, rt.cos, rt.sin, rt.pos, rstd, dq, dk, dqkv, Hq, Hkv, D, partial=True)
     for p, g in ((att.q_norm.weight, dqw), (att.k_norm.weight, dkw)):
         view, acc = _vecgrad(arena, p)
         if view is not None:
-            K.add_f32_to_bf16(g.contiguous(), view if acc else None, view)
+            mine.append((g, view, acc))
+    if sums is None and mine:
+        K.reduce_rows_each(mine)
     wqkv = arena.fused(att.w_queries.weight, att.w_values.weight)
     dh1 = K.dgrad(dqkv, wqkv)
     _wgrad(arena, att.w_queries.weight, att.w_values.weight, dqkv, h1, defer)
@@ -199,7 +202,8 @@ def block_backward(blk, saved, dx3, rt, rows=None):
     dh2 = K.dgrad(dgu, wgu)
     _wgrad(arena, ffn.lin1.weight, ffn.lin_gate.weight, dgu, h2, wg)
     gview, gacc = _vecgrad(arena, blk.norm2.weight)
-    dx2, _ = K.rmsnorm_bwd(x2, blk.norm2.weight, rstd2, dh2, dres=dx3, dw_out=gview, dw_accumulate=gacc)
+    dx2, part = K.rmsnorm_bwd(x2, blk.norm2.weight, rstd2, dh2, dres=dx3, partial=True)
+    sums = [] if gview is None else [(part, gview, gacc)]  # the block's vector gradients: added up by one launch at the end
     if rows is not None:  # the FFN half ran on the kept rows: the others receive no gradient from it
         dx2 = _put_rows(dx2, rt.B, rt.S, rows)
     # ---- attention half
@@ -207,9 +211,13 @@ def block_backward(blk, saved, dx3, rt, rows=None):
     fused = K.dgrad_attn_delta(dx2, att.out_proj.weight, ctx, att_saved[4], rt.B, rt.S, att.num_heads, att.head_dim)
     dctx, delta = fused if fused is not None else (K.dgrad(dx2, att.out_proj.weight), None)
     _wgrad(arena, att.out_proj.weight, None, dx2, ctx, wg)
-    dh1 = attention_backward(att, arena, h1, ctx, att_saved, dctx, rt, wg, delta)
+    dh1 = attention_backward(att, arena, h1, ctx, att_saved, dctx, rt, wg, delta, sums)
     gview, gacc = _vecgrad(arena, blk.norm1.weight)
-    dx, _ = K.rmsnorm_bwd(x, blk.norm1.weight, rstd1, dh1, dres=dx2, dw_out=gview, dw_accumulate=gacc)
+    dx, part = K.rmsnorm_bwd(x, blk.norm1.weight, rstd1, dh1, dres=dx2, partial=True)
+    if gview is not None:
+        sums.append((part, gview, gacc))
+    if sums:
+        K.reduce_rows_each(sums)
     _flush_wgrads(wg)
     hook = getattr(blk, "_grad_ready", None)
     if hook is not None:

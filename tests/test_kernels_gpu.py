@@ -1407,3 +1407,24 @@ def test_embedding_gradient_of_runs_on_block_edges(K, lengths, accumulate):
     got = out.cpu()
     bound = max(lengths) * 2.0 ** -24 * mag + 2.0 ** -8 * want.abs()
     assert ((got[:, :520].double() - want).abs() <= bound).all() and torch.equal(got[:, 520:], table[:, 520:])
+
+
+@pytest.mark.parametrize("sums", [[(1, 1)], [(1, 8), (700, 1024)], [(16, 128), (64, 128), (33, 65)], [(512, 1024), (2, 64), (63, 63), (129, 2048)]])
+def test_several_row_sums_in_one_launch(K, sums):
+    """The bits of a launch each, and of one with ``add_f32_to_bf16`` behind it; rows in a wider matrix, widths that end inside a workgroup's columns; nothing beside a destination is written."""
+    from llm_quest_amd import _lib as L
+
+    g = torch.Generator().manual_seed(len(sums))
+    for dt, acc in ((BF16, False), (BF16, True), (torch.float32, False), (torch.float32, True)):
+        parts = [dev(torch.randn(p, n + 8 * i, generator=g))[:, :n] for i, (p, n) in enumerate(sums)]
+        wide = [dev(torch.randn(n + 2, generator=g).to(dt)) for _, n in sums]
+        outs, want = [w[1:-1] for w in wide], []
+        for p, o in zip(parts, outs):
+            alone = torch.empty(p.shape[1], device="cuda")
+            L.call("mi355_reduce_rows_f32", p.shape[0], p.shape[1], L.ptr(p.contiguous()), L.ptr(alone), L.DT_F32, 0)
+            want.append((alone + (o.float() if acc else 0)).to(dt))
+        ends = [(w[0].item(), w[-1].item()) for w in wide]
+        K.reduce_rows_each([(p, o, acc) for p, o in zip(parts, outs)])
+        assert all(torch.equal(o, w) for o, w in zip(outs, want)) and ends == [(w[0].item(), w[-1].item()) for w in wide]
+    with pytest.raises(ValueError, match="one to four"):
+        K.reduce_rows_each([])

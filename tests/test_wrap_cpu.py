@@ -236,6 +236,7 @@ def test_training_rows(both):
         assert both("rmsnorm_fwd", x, w) and both("rmsnorm_fwd", x, w, 1e-5, want_rstd=False) and not both("rmsnorm_fwd", rows(M, W, pad=8) if M > 1 else x.float(), w) and not both("rmsnorm_fwd", x, w[:-1])
         r = torch.randn(M)
         assert both("rmsnorm_bwd", x, w, r, g) and both("rmsnorm_bwd", x, w, r, g, dres=g, dw_out=torch.zeros(W), dw_accumulate=True) and both("rmsnorm_bwd", x, w, r, g, dw_out=torch.zeros(W, dtype=B))
+        assert both("rmsnorm_bwd", x, w, r, g, dres=g, partial=True)
         assert not both("rmsnorm_bwd", x, w, r, g.float()) and not both("rmsnorm_bwd", x, w, r, rows(M + 1, W)) and not both("rmsnorm_bwd", x, w, r, g, dres=rows(M, W, F))
         assert both("swiglu_fwd", rows(M, 2 * W), W) and both("swiglu_bwd", rows(M, 2 * W), g, W) and not both("swiglu_fwd", x, W) and not both("swiglu_bwd", rows(M, 2 * W), rows(M, W + 1), W)
         xf, s = rows(M, W, F), torch.randn(W)
@@ -247,6 +248,9 @@ def test_training_rows(both):
             assert both("layernorm_bwd_bf16", xf, s, r, r, dy, xf, d) and both("layernorm_bwd_bf16", xf, s, r, r, dy, None, tuple(d), eps=1e-6, mode=1)
         one = torch.zeros(W)
         assert not both("layernorm_bwd_bf16", xf, s, r, r, g, xf, [(one, True), None, (one, True)]) and not both("layernorm_bwd_bf16", xf, s, r, r, g, xf, [(w, True), None, None])
+        sums = [(rows(5, W, F), torch.zeros(W, dtype=B), True), (rows(1, W, F, 8), torch.zeros(W), False), (rows(7, 2 * W, F)[:, W:], torch.zeros(W, dtype=B), False), (rows(2, 8, F), torch.zeros(2, 4), True)]
+        assert all(both("reduce_rows_each", sums[:n]) for n in (1, 2, 3, 4)) and not both("reduce_rows_each", []) and not both("reduce_rows_each", sums + sums[:1])
+        assert not both("reduce_rows_each", [(rows(5, W, F), torch.zeros(W + 1), True)]) and not both("reduce_rows_each", [(rows(5, W), torch.zeros(W), True)])
         assert both("reduce_rows_into", rows(3, 2 * W, F), 3, W, [(one, False), (torch.zeros(W), True)]) and not both("reduce_rows_into", rows(3, W, F), 3, W, [None])
         assert both("gelu_fwd", x) and both("gelu_fwd", x, tanh=True) and not both("gelu_fwd", xf) and both("gelu_bwd_colsum", x, g, (one, True)) and not both("gelu_bwd_colsum", x, g, None)
         assert both("colsum", rows(M, W, pad=4)) and both("colsum", xf, one, True) and not both("colsum", x, torch.zeros(W + 1)) and both("add_f32_to_bf16", one, None, w) and both("add_f32_to_bf16", one, w, w)
@@ -279,10 +283,10 @@ def test_attention(both, D, monkeypatch):
     assert both("attn_bwd", q, k, v, o, do, lse, Bn, Sn, Hq, Hkv, D, dq, dk, dv, None, False)
     monkeypatch.setattr(K, "_ATTN_DS_SPILL", True)
     for a in (dq, None):
-        assert both("qknorm_rope_bwd", qkv, qw, kw, cs, cs, pos, rstd, a, dk, dqkv, Hq, Hkv, D)
+        assert both("qknorm_rope_bwd", qkv, qw, kw, cs, cs, pos, rstd, a, dk, dqkv, Hq, Hkv, D) and both("qknorm_rope_bwd", qkv, qw, kw, cs, cs, pos, rstd, a, dk, dqkv, Hq, Hkv, D, True)
     args = (q, k, v, o, do, lse, Bn, Sn, Hq, Hkv, D, dk, dv, qkv, qw, cs, cs, pos, rstd, dqkv)
     taken = D == 128
-    assert both("attn_bwd_qnorm", *args) is taken and both("attn_bwd_qnorm", *args, key_mask=mask, causal=True, scale=0.2, delta=torch.randn(Bn, Hq, Sn)) is taken
+    assert both("attn_bwd_qnorm", *args) is taken and both("attn_bwd_qnorm", *args, partial=True) is taken and both("attn_bwd_qnorm", *args, key_mask=mask, causal=True, scale=0.2, delta=torch.randn(Bn, Hq, Sn)) is taken
     assert not both("attn_bwd_qnorm", *args[:14], None, *args[15:]) and not both("attn_bwd_qnorm", *args, delta=lse[:, :1])
     monkeypatch.setattr(K, "_attn_scratch", lambda d, n: None)
     assert not both("attn_bwd_qnorm", *args) and both("attn_bwd", q, k, v, o, do, lse, Bn, Sn, Hq, Hkv, D, dq, dk, dv)
