@@ -746,7 +746,7 @@ OP(headnorm_rope_fwd, "src", "H", "D", "head_stride", "w_eff", "cos_t", "sin_t",
     return tuple(out, rstd);
 }
 
-OP(headnorm_rope_bwd, "src", "H", "D", "head_stride", "w_eff", "cos_t", "sin_t", "pos", "rstd", "dout", "dsrc", "dhead_stride") {
+OP(headnorm_rope_bwd, "src", "H", "D", "head_stride", "w_eff", "cos_t", "sin_t", "pos", "rstd", "dout", "dsrc", "dhead_stride", "partial") {
     const T src = c.tensor(0), w = c.maybe(4), cos = c.maybe(5), sin = c.maybe(6), pos = c.maybe(7), rstd = c.maybe(8), dout = c.tensor(9), dsrc = c.tensor(10);
     const int64_t H = c.integer(1), D = c.integer(2), hs = c.integer(3), dhs = c.integer(11);
     need(heads(src, H, D, hs) && heads(dsrc, H, D, dhs) && (!cos || cos.dim() == 2));
@@ -754,7 +754,7 @@ OP(headnorm_rope_bwd, "src", "H", "D", "head_stride", "w_eff", "cos_t", "sin_t",
     need(dout.is(BF16) && dout.contiguous() && dout.shape({tokens, H * D}) && (dry || slot::reduce_rows_f32.address));
     const T part = c.empty(src, {parts, D}, F32);
     LAUNCH(headnorm_rope_bwd, tokens, H, D, R, src, src.ld(), hs, w, cos, sin, pos, rstd, dout, dsrc, dsrc.ld(), dhs, part, parts);
-    return wrapped(reduce_parts(c, part));
+    return wrapped(c.truth(12, false) ? part : reduce_parts(c, part));
 }
 
 OP(sigmoid_gate_fwd, "ctx", "gate", "H", "D", "gate_head_stride") {
@@ -808,7 +808,7 @@ OP(gdn_gates_fwd, "b_lin", "a_lin", "log_A", "dt_bias") {
     return tuple(beta, alpha);
 }
 
-OP(gdn_gates_bwd, "b_lin", "a_lin", "log_A", "dt_bias", "dbeta", "dalpha", "db_lin", "da_lin") {
+OP(gdn_gates_bwd, "b_lin", "a_lin", "log_A", "dt_bias", "dbeta", "dalpha", "db_lin", "da_lin", "partial") {
     const T b = c.tensor(0), a = c.tensor(1), A = c.tensor(2), dt = c.tensor(3), dbeta = c.tensor(4), dalpha = c.tensor(5), db = c.tensor(6), da = c.tensor(7);
     need(b.dim() == 2 && cols(db) && cols(da));
     const int64_t tokens = b.size(0), H = b.size(1), parts = std::max<int64_t>(1, std::min<int64_t>(256, (tokens * H + 255) / 256));
@@ -817,6 +817,7 @@ OP(gdn_gates_bwd, "b_lin", "a_lin", "log_A", "dt_bias", "dbeta", "dalpha", "db_l
     need(dry || slot::reduce_rows_f32.address);
     const T part = c.empty(b, {parts, 2 * H}, F32);
     LAUNCH(gdn_gates_bwd, tokens, H, b, a, b.ld(), A, dt, dbeta, dalpha, db, da, db.ld(), part, parts);
+    if (c.truth(8, false)) return tuple(T{part.t.narrow(1, 0, H)}, T{part.t.narrow(1, H, H)});
     const T both = reduce_parts(c, part);
     return tuple(T{both.t.narrow(0, 0, H)}, T{both.t.narrow(0, H, H)});
 }
@@ -830,7 +831,7 @@ OP(causal_conv_silu_fwd, "x", "w", "B", "S") {
     return wrapped(y);
 }
 
-OP(causal_conv_silu_bwd, "x", "w", "dy", "dx", "B", "S") {
+OP(causal_conv_silu_bwd, "x", "w", "dy", "dx", "B", "S", "partial") {
     const T x = c.tensor(0), w = c.tensor(1), dy = c.tensor(2), dx = c.tensor(3);
     const int64_t B = c.integer(4), S = c.integer(5), chunk = c.constant("CONV_TOKEN_CHUNK");
     need(chunk > 0 && cols(x) && cols(dx) && w.dim() >= 1 && dy.is(BF16) && dy.contiguous() && dy.shape({B * S, x.size(1)}) && dx.shape({B * S, x.size(1)}) && (dry || slot::reduce_rows_f32.address));
@@ -839,7 +840,7 @@ OP(causal_conv_silu_bwd, "x", "w", "dy", "dx", "B", "S") {
     const T ws = mine == x.t.storage().data() || mine == dy.t.storage().data() ? c.empty(x, {B * S, C}, BF16) : T{};
     const T part = c.empty(x, {B * ((S + chunk - 1) / chunk), C * ks}, F32);
     LAUNCH(causal_conv_silu_bwd, B, S, C, ks, x, x.ld(), w, dy, ws, dx, dx.ld(), part, chunk);
-    return wrapped(reduce_parts(c, part));
+    return wrapped(c.truth(6, false) ? part : reduce_parts(c, part));
 }
 
 OP(l2norm_fwd, "x", "H", "D") {
@@ -868,14 +869,14 @@ OP(gated_rmsnorm_fwd, "o", "w_f32", "gate", "H", "D", "eps") {
     return tuple(out, rstd);
 }
 
-OP(gated_rmsnorm_bwd, "o", "w_f32", "gate", "rstd", "dout", "dgate", "H", "D") {
+OP(gated_rmsnorm_bwd, "o", "w_f32", "gate", "rstd", "dout", "dgate", "H", "D", "partial") {
     const T o = c.tensor(0), w = c.tensor(1), gate = c.tensor(2), rstd = c.tensor(3), dout = c.tensor(4), dgate = c.tensor(5);
     const int64_t H = c.integer(6), D = c.integer(7);
     need(cols(dgate) && o.dim() == 2 && gate.dim() >= 1 && dout.is(BF16) && dout.contiguous() && dout.like(o) && dgate.like(o) && (dry || slot::reduce_rows_f32.address));
     const int64_t parts = std::max<int64_t>(1, std::min<int64_t>(c.constant("NORM_PARTS"), (o.size(0) * H + 3) / 4));
     const T d_o = c.empty_like(o), part = c.empty(o, {parts, D}, F32);
     LAUNCH(gated_rmsnorm_bwd, o.size(0), H, D, o, w, gate, gate.ld(), rstd, dout, d_o, dgate, dgate.ld(), part, parts);
-    return tuple(d_o, reduce_parts(c, part));
+    return tuple(d_o, c.truth(8, false) ? part : reduce_parts(c, part));
 }
 
 // ---------------------------------------------------------------------------------------------- ops_decode.py, kernels_seq.py

@@ -95,8 +95,8 @@ def headnorm_rope_fwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, eps=1e-6
 
 
 @L.native
-def headnorm_rope_bwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, rstd, dout, dsrc, dhead_stride):
-    """Writes d(src) into the strided view ``dsrc``; returns d(w_eff) fp32 [D]."""
+def headnorm_rope_bwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, rstd, dout, dsrc, dhead_stride, partial=False):
+    """Writes d(src) into the strided view ``dsrc``; returns d(w_eff) fp32 [D], ``partial``: as rows to be added up (``kernels.reduce_rows_each``)."""
     L.require_gpu(src, dout, dsrc)
     _check_heads(src, H, D, head_stride, "headnorm_rope_bwd")
     _check_heads(dsrc, H, D, dhead_stride, "headnorm_rope_bwd(dsrc)")
@@ -108,7 +108,7 @@ def headnorm_rope_bwd(src, H, D, head_stride, w_eff, cos_t, sin_t, pos, rstd, do
     part = torch.empty((parts, D), dtype=F32, device=src.device)
     L.call("mi355_headnorm_rope_bwd", tokens, H, D, R, L.ptr(src), src.stride(0), head_stride, L.ptr(w_eff), L.ptr(cos_t), L.ptr(sin_t), L.ptr(pos), L.ptr(rstd),
            L.ptr(dout), L.ptr(dsrc), dsrc.stride(0), dhead_stride, L.ptr(part), parts)
-    return _reduce_parts(part)
+    return part if partial else _reduce_parts(part)
 
 
 @L.native
@@ -177,8 +177,8 @@ def gdn_gates_fwd(b_lin, a_lin, log_A, dt_bias):
 
 
 @L.native
-def gdn_gates_bwd(b_lin, a_lin, log_A, dt_bias, dbeta, dalpha, db_lin, da_lin):
-    """Writes d(b_lin), d(a_lin) into the given column views; returns (dlog_A fp32 [Hv], ddt_bias fp32 [Hv])."""
+def gdn_gates_bwd(b_lin, a_lin, log_A, dt_bias, dbeta, dalpha, db_lin, da_lin, partial=False):
+    """Writes d(b_lin), d(a_lin) into the given column views; returns (dlog_A fp32 [Hv], ddt_bias fp32 [Hv]), ``partial``: as rows to be added up."""
     L.require_gpu(b_lin, a_lin, dbeta, dalpha, db_lin, da_lin)
     tokens, Hv = b_lin.shape
     _cols(db_lin, "gdn_gates_bwd(db_lin)")
@@ -192,6 +192,8 @@ def gdn_gates_bwd(b_lin, a_lin, log_A, dt_bias, dbeta, dalpha, db_lin, da_lin):
     part = torch.empty((parts, 2 * Hv), dtype=F32, device=b_lin.device)
     L.call("mi355_gdn_gates_bwd", tokens, Hv, L.ptr(b_lin), L.ptr(a_lin), b_lin.stride(0), L.ptr(log_A), L.ptr(dt_bias), L.ptr(dbeta), L.ptr(dalpha),
            L.ptr(db_lin), L.ptr(da_lin), db_lin.stride(0), L.ptr(part), parts)
+    if partial:
+        return part[:, :Hv], part[:, Hv:]
     both = _reduce_parts(part)
     return both[:Hv], both[Hv:]
 
@@ -225,8 +227,8 @@ CONV_TOKEN_CHUNK = 32
 
 
 @L.native
-def causal_conv_silu_bwd(x, w, dy, dx, B, S):
-    """Writes d(x) into the column view ``dx``; returns d(weight) fp32 flat [C*k]."""
+def causal_conv_silu_bwd(x, w, dy, dx, B, S, partial=False):
+    """Writes d(x) into the column view ``dx``; returns d(weight) fp32 flat [C*k], ``partial``: as rows to be added up."""
     L.require_gpu(x, w, dy, dx)
     _cols(x, "causal_conv_silu_bwd")
     _cols(dx, "causal_conv_silu_bwd(dx)")
@@ -238,7 +240,7 @@ def causal_conv_silu_bwd(x, w, dy, dx, B, S):
     chunks = B * ((S + CONV_TOKEN_CHUNK - 1) // CONV_TOKEN_CHUNK)
     part = torch.empty((chunks, C * ks), dtype=F32, device=x.device)
     L.call("mi355_causal_conv_silu_bwd", B, S, C, ks, L.ptr(x), x.stride(0), L.ptr(w), L.ptr(dy), L.ptr(ws), L.ptr(dx), dx.stride(0), L.ptr(part), CONV_TOKEN_CHUNK)
-    return _reduce_parts(part)
+    return part if partial else _reduce_parts(part)
 
 
 @L.native
@@ -364,8 +366,8 @@ def gated_rmsnorm_fwd(o, w_f32, gate, H, D, eps=1e-6):
 
 
 @L.native
-def gated_rmsnorm_bwd(o, w_f32, gate, rstd, dout, dgate, H, D):
-    """Writes d(gate) into the column view ``dgate``; returns (d_o bf16, dw fp32 [D])."""
+def gated_rmsnorm_bwd(o, w_f32, gate, rstd, dout, dgate, H, D, partial=False):
+    """Writes d(gate) into the column view ``dgate``; returns (d_o bf16, dw fp32 [D], ``partial``: as rows to be added up)."""
     L.require_gpu(o, gate, rstd, dout, dgate)
     _cols(dgate, "gated_rmsnorm_bwd(dgate)")
     if not (dout.dtype == BF16 and dout.is_contiguous() and dout.shape == o.shape) or tuple(dgate.shape) != tuple(o.shape):
@@ -374,4 +376,4 @@ def gated_rmsnorm_bwd(o, w_f32, gate, rstd, dout, dgate, H, D):
     parts = max(1, min(NORM_PARTS, (o.shape[0] * H + 3) // 4))
     part = torch.empty((parts, D), dtype=F32, device=o.device)
     L.call("mi355_gated_rmsnorm_bwd", o.shape[0], H, D, L.ptr(o), L.ptr(w_f32), L.ptr(gate), gate.stride(0), L.ptr(rstd), L.ptr(dout), L.ptr(d_o), L.ptr(dgate), dgate.stride(0), L.ptr(part), parts)
-    return d_o, _reduce_parts(part)
+    return d_o, part if partial else _reduce_parts(part)

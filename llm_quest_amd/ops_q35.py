@@ -38,22 +38,26 @@ def arena_for_bf16(module):
     return ar
 
 
-def _bf16_vec_grad(arena, p, g_f32):
-    """p.grad (bf16, in the arena) (+)= g (fp32)."""
+def _vec_sum(sums, arena, p, part):
+    """p.grad (bf16, in the arena) (+)= the sum of the rows of ``part``, once ``_flush_sums`` has run."""
     view, acc = _vecgrad(arena, p)
     if view is not None:
-        K.add_f32_to_bf16(g_f32.contiguous(), view if acc else None, view)
+        sums.append((part, view, acc))
 
 
-def _f32_param_grad(p, g_f32):
-    """Stand-alone fp32 parameter: p.grad (+)= g."""
+def _f32_sum(sums, p, part):
+    """The same for a stand-alone fp32 parameter."""
     if not p.requires_grad:
         return
-    g = g_f32.reshape(p.shape)
-    if p.grad is None:
-        p.grad = g.clone()
-    else:
-        Q._reduce_parts(g.reshape(1, -1).contiguous(), out=p.grad.view(-1), accumulate=True)
+    acc = p.grad is not None
+    if not acc:
+        p.grad = torch.empty(p.shape, dtype=F32, device=p.device)
+    sums.append((part, p.grad.view(-1), acc))
+
+
+def _flush_sums(sums):
+    for i in range(0, len(sums), 4):
+        K.reduce_rows_each(sums[i : i + 4])
 
 
 class Runtime:
@@ -123,7 +127,9 @@ def gated_attention_forward(att, arena, h1, rt):
     return gated, (proj, wq, wk, q, k, rstd_q, rstd_k, ctx, lse, drop)
 
 
-def gated_attention_backward(att, arena, h1, saved, dgated, rt, defer=None):
+def gated_attention_backward(att, arena, h1, saved, dgated, rt, defer=None, sums=None):
+    """``sums``: a list that the vector gradients join, for the caller to add up (``_flush_sums``)."""
+    mine = [] if sums is None else sums
     H, G, D, QG, KV = _att_dims(att)
     proj, wq, wk, q, k, rstd_q, rstd_k, ctx, lse, drop = saved
     dproj = torch.empty_like(proj)
@@ -135,10 +141,12 @@ def gated_attention_backward(att, arena, h1, saved, dgated, rt, defer=None):
         K.attn_dropout_bwd(q, k, proj[:, QG + KV :], ctx, dctx, lse, rt.B, rt.S, H, G, D, dq, dk, dproj[:, QG + KV :], *drop, causal=True)
     else:
         Q.attn_generic_bwd(q, k, proj[:, QG + KV :], ctx, dctx, lse, rt.B, rt.S, H, G, D, dq, dk, dproj[:, QG + KV :], key_mask=rt.key_mask)
-    dwq = Q.headnorm_rope_bwd(proj[:, :QG], H, D, 2 * D, wq, rt.cos_t, rt.sin_t, rt.pos, rstd_q, dq, dproj[:, :QG], 2 * D)
-    dwk = Q.headnorm_rope_bwd(proj[:, QG : QG + KV], G, D, D, wk, rt.cos_t, rt.sin_t, rt.pos, rstd_k, dk, dproj[:, QG : QG + KV], D)
-    _bf16_vec_grad(arena, att.q_norm.scale, dwq)
-    _bf16_vec_grad(arena, att.k_norm.scale, dwk)
+    dwq = Q.headnorm_rope_bwd(proj[:, :QG], H, D, 2 * D, wq, rt.cos_t, rt.sin_t, rt.pos, rstd_q, dq, dproj[:, :QG], 2 * D, partial=True)
+    dwk = Q.headnorm_rope_bwd(proj[:, QG : QG + KV], G, D, D, wk, rt.cos_t, rt.sin_t, rt.pos, rstd_k, dk, dproj[:, QG : QG + KV], D, partial=True)
+    _vec_sum(mine, arena, att.q_norm.scale, dwq)
+    _vec_sum(mine, arena, att.k_norm.scale, dwk)
+    if sums is None:
+        _flush_sums(mine)
     w = arena.fused(att.w_queries_gate.weight, att.w_values.weight)
     dh1 = K.dgrad(dproj, w)
     _wgrad(arena, att.w_queries_gate.weight, att.w_values.weight, dproj, h1, defer)
@@ -167,22 +175,26 @@ def gdn_forward(att, arena, h1, rt, keep=True):
     return gated, (h1, proj, y, qn, kn, beta, alpha, o, ck, rstd_p)
 
 
-def gdn_backward(att, arena, saved, dgated, rt, defer=None):
+def gdn_backward(att, arena, saved, dgated, rt, defer=None, sums=None):
+    """``sums``: as ``gated_attention_backward``'s."""
+    mine = [] if sums is None else sums
     Hqk, Hv, Dk, Dv, QK, VG, C = _gdn_dims(att)
     h1, proj, y, qn, kn, beta, alpha, o, ck, rstd_p = saved
     dproj = torch.empty_like(proj)
-    d_o, dpw = Q.gated_rmsnorm_bwd(o, att.post_norm.weight, proj[:, C : C + VG], rstd_p, dgated, dproj[:, C : C + VG], Hv, Dv)
-    _f32_param_grad(att.post_norm.weight, dpw)
+    d_o, dpw = Q.gated_rmsnorm_bwd(o, att.post_norm.weight, proj[:, C : C + VG], rstd_p, dgated, dproj[:, C : C + VG], Hv, Dv, partial=True)
+    _f32_sum(mine, att.post_norm.weight, dpw)
     dy = torch.empty_like(y)
     dqn, dkn, dbeta, dalpha = Q.gated_delta_rule_bwd(qn, kn, y[:, 2 * QK :], beta, alpha, ck, d_o, dy[:, 2 * QK :], rt.B, rt.S, Hqk, Hv, Dk, Dv)
     Q.l2norm_bwd(y[:, :QK], dqn, dy[:, :QK], Hqk, Dk)
     Q.l2norm_bwd(y[:, QK : 2 * QK], dkn, dy[:, QK : 2 * QK], Hqk, Dk)
-    dcw = Q.causal_conv_silu_bwd(proj[:, :C], att.conv1d.weight, dy, dproj[:, :C], rt.B, rt.S)
-    _bf16_vec_grad(arena, att.conv1d.weight, dcw)
+    dcw = Q.causal_conv_silu_bwd(proj[:, :C], att.conv1d.weight, dy, dproj[:, :C], rt.B, rt.S, partial=True)
+    _vec_sum(mine, arena, att.conv1d.weight, dcw)
     dlog_A, ddtb = Q.gdn_gates_bwd(proj[:, C + VG : C + VG + Hv], proj[:, C + VG + Hv :], att.log_A, att.dt_bias, dbeta, dalpha,
-                                   dproj[:, C + VG : C + VG + Hv], dproj[:, C + VG + Hv :])
-    _f32_param_grad(att.log_A, dlog_A)
-    _bf16_vec_grad(arena, att.dt_bias, ddtb)
+                                   dproj[:, C + VG : C + VG + Hv], dproj[:, C + VG + Hv :], partial=True)
+    _f32_sum(mine, att.log_A, dlog_A)
+    _vec_sum(mine, arena, att.dt_bias, ddtb)
+    if sums is None:
+        _flush_sums(mine)
     w = arena.fused(att.w_qkv.weight, att.w_alpha.weight)
     dh1 = K.dgrad(dproj, w)
     _wgrad(arena, att.w_qkv.weight, att.w_alpha.weight, dproj, h1, defer)
@@ -229,17 +241,19 @@ def block_backward(blk, saved, dx3, rt):
     _wgrad(arena, ffn.lin2.weight, None, dx3, a, wg)
     dh2 = K.dgrad(dgu, arena.fused(ffn.lin1.weight, ffn.lin_gate.weight))
     _wgrad(arena, ffn.lin1.weight, ffn.lin_gate.weight, dgu, h2, wg)
-    gview, gacc = _vecgrad(arena, blk.norm2.scale)
-    dx2, _ = K.rmsnorm_bwd(x2, w2, rstd2, dh2, dres=dx3, dw_out=gview, dw_accumulate=gacc)
+    sums = []  # the block's vector gradients: added up at its end, four to a launch
+    dx2, part = K.rmsnorm_bwd(x2, w2, rstd2, dh2, dres=dx3, partial=True)
+    _vec_sum(sums, arena, blk.norm2.scale, part)
     # ---- token-mixer half
     dmix = K.dgrad(dx2, att.out_proj.weight)
     _wgrad(arena, att.out_proj.weight, None, dx2, mix, wg)
     if blk.is_linear:
-        dh1 = gdn_backward(att, arena, att_saved, dmix, rt, wg)
+        dh1 = gdn_backward(att, arena, att_saved, dmix, rt, wg, sums)
     else:
-        dh1 = gated_attention_backward(att, arena, h1, att_saved, dmix, rt, wg)
-    gview, gacc = _vecgrad(arena, blk.norm1.scale)
-    dx, _ = K.rmsnorm_bwd(x, w1, rstd1, dh1, dres=dx2, dw_out=gview, dw_accumulate=gacc)
+        dh1 = gated_attention_backward(att, arena, h1, att_saved, dmix, rt, wg, sums)
+    dx, part = K.rmsnorm_bwd(x, w1, rstd1, dh1, dres=dx2, partial=True)
+    _vec_sum(sums, arena, blk.norm1.scale, part)
+    _flush_sums(sums)
     _flush_wgrads(wg)
     hook = getattr(blk, "_grad_ready", None)
     if hook is not None:

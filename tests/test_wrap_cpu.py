@@ -298,16 +298,18 @@ def test_hybrid_rows(both):
     wide, cs, pos, w = rows(T, 2 * H * D + 5), torch.randn(T, 8), ints(T), torch.randn(D).to(B)
     assert both("headnorm_rope_fwd", wide, H, D, 2 * D, w, cs, cs, pos) and both("headnorm_rope_fwd", wide, H, D, D, w, None, None, None) and not both("headnorm_rope_fwd", wide, H, D, 3 * D, w, cs, cs, pos)
     rstd, dout = torch.randn(T, H), rows(T, H * D)
-    assert both("headnorm_rope_bwd", wide, H, D, 2 * D, w, cs, cs, pos, rstd, dout, rows(T, H * D), D) and not both("headnorm_rope_bwd", wide, H, D, 2 * D, w, cs, cs, pos, rstd, dout.float(), rows(T, H * D), D)
+    assert both("headnorm_rope_bwd", wide, H, D, 2 * D, w, cs, cs, pos, rstd, dout, rows(T, H * D), D) and both("headnorm_rope_bwd", wide, H, D, 2 * D, w, cs, cs, pos, rstd, dout, rows(T, H * D), D, True) and not both("headnorm_rope_bwd", wide, H, D, 2 * D, w, cs, cs, pos, rstd, dout.float(), rows(T, H * D), D)
     ctx = rows(T, H * D)
     assert both("sigmoid_gate_fwd", ctx, wide, H, D, 2 * D) and both("sigmoid_gate_bwd", ctx, wide, H, D, 2 * D, dout, rows(T, 2 * H * D), 2 * D) and not both("sigmoid_gate_fwd", ctx, wide.float(), H, D, D)
     both_ = rows(T, 2 * H)
     b, a, A, dt = both_[:, :H], both_[:, H:], torch.randn(H), torch.randn(H).to(B)
     g = torch.randn(T, H)
     assert both("gdn_gates_fwd", b, a, A, dt) and not both("gdn_gates_fwd", b, rows(T, H), A, dt) and both("gdn_gates_bwd", b, a, A, dt, g, g, both_[:, :H], both_[:, H:])
+    assert both("gdn_gates_bwd", b, a, A, dt, g, g, both_[:, :H], both_[:, H:], partial=True)
     assert not both("gdn_gates_bwd", b, a, A, dt, g, g.to(B), both_[:, :H], both_[:, H:])
     x, cw = wide[:, : H * D], torch.randn(H * D, 1, 4).to(B)
     assert both("causal_conv_silu_fwd", x, cw, 2, 3) and not both("causal_conv_silu_fwd", x, cw, 2, 4) and not both("causal_conv_silu_fwd", x, cw.float(), 2, 3)
+    assert both("causal_conv_silu_bwd", x, cw, dout, rows(T, H * D), 2, 3, True) and both("gated_rmsnorm_bwd", ctx, wf, x, rstd, dout, rows(T, H * D), H, D, True)
     assert both("causal_conv_silu_bwd", x, cw, dout, rows(T, H * D), 2, 3) and both("causal_conv_silu_bwd", x, cw, dout, x, 2, 3) and both("causal_conv_silu_bwd", x, cw, dout, dout, 2, 3)
     assert both("l2norm_fwd", x, H, D) and both("l2norm_bwd", x, dout, x, H, D) and not both("l2norm_fwd", x, H, D + 1) and not both("l2norm_bwd", x, dout.float(), x, H, D)
     wf = torch.randn(D)
