@@ -1775,12 +1775,14 @@ int launch_quad(GemmParams p, int out_dtype, bool persistent, hipStream_t s) {
 // K = 2 048 19.0 -> 17.0; 5 664 x 1 024, K = 1 024 21.0 -> 19.4, 3 584 49.6 -> 47.4, 8 256 99.8 -> 98.6; NN 333 x 2 048, K = 1 024 13.1 -> 10.5; 996 x 1 024, K = 6 144 27.7 -> 26.9.
 // (The ring is dynamic LDS: told its size, the compiler gives the one wave per SIMD all 512 registers, half of them accumulation registers, and moves the sums back and forth -- 1.4 times
 // the time.)
-// NT and NN forms, plain epilogue (bias and residual allowed).  The bits of gemm_bf16_kernel in as many shares of K: every output is summed over K in the same order.
+// NT and NN forms, plain epilogue (bias and residual allowed) or a fused one (KIND).  The bits of gemm_bf16_kernel in as many shares of K: every output is summed over K in the same order.
 // B_TR (NN): the column fragments come by transposing reads issued from asm, the whole half's in front of its first row of products, and each half ends with a wait for them.  gemm_bf16_kernel's NN
 // form waits for its one K-tile in flight; us with weights from memory, gemm_bf16_kernel -> here: 333 x 1 024, K = 1 024 20.3 -> 13.3, 3 584 21.5 -> 17.6; 996 x 1 024, K = 4 096 27.6 -> 22.4,
 // 6 144 46.5 -> 26.7; 996 x 4 096, K = 1 024 25.2 -> 16.0; 2 000 x 2 048, K = 2 048 52.0 -> 23.6.  With every CU at work a K-tile of 128 rows takes 0.07 us longer than in the NT form.
 // KIND: a fused epilogue in the write-out, the same bits: SwiGLU's backward behind the NN form (its [u | g] rows requested as a residual's are) and GELU behind the NT form; us, gemm_bf16_kernel -> here:
 // 333 x 3 072, K = 1 024, SwiGLU backward 24.8 -> 16.5, 996 rows 28.9 -> 18.6, 1 416 rows 32.1 -> 23.4; K = 768, GELU, 333 rows 23.3 -> 18.7, 1 200 24.0 -> 19.9.
+// SwiGLU's forward behind the NT form, in one round of the CUs as the others; us, gemm_bf16_kernel -> here, weights from memory: 333 rows, 1 024 -> 2 x 3 584 21.7 -> 13.9, 602, 2 x 3 072 21.7 -> 14.7,
+// 1 056, 2 x 3 584 39.4 -> 28.0, 200, 2 048 -> 2 x 8 192 34.3 -> 21.3.
 // FOLD: the sum over K is cut every p.fold K-tiles and the cuts are added in order -- as near to 64 bits as that many shares of K, without their slabs (2 000 x 1 024, K = 4 096, fp32: 2.7e-7
 // uncut, 1.7e-7 in four).
 template <int BM, int OUT_DT, bool FOLD, bool B_TR, int KIND>
@@ -1806,11 +1808,21 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     int kneedA[A_PPW], kneedB[B_PPW];
     piece_offsets<false, BM, 64, A_PPW>(wave, lane, p.lda, BM, voffA, kneedA);
     piece_offsets<B_TR, BN, 64, B_PPW>(wave, lane, p.ldb, B_TR ? p.N - n0 : BN, voffB, kneedB);
+    // SwiGLU forward: 64 units a tile; of a column wave's 64 rows of B the first 32 are lin1's, the others the lin_gate rows of the same units, so that a lane holds both operands of an activation
+    constexpr bool SW_FWD = KIND == MI355_EPI_SWIGLU_FWD;
+    static_assert(!SW_FWD || !B_TR);
+    if constexpr (SW_FWD) {
+#pragma unroll
+        for (int j = 0; j < B_PPW; ++j) {
+            const int r = (wave * B_PPW + j) * 8 + (lane >> 3), unit = (r >> 6) * 32 + (r & 31);
+            voffB[j] += (unsigned)(((r & 32 ? (int)(p.N >> 1) : 0) + unit - r) * (int)p.ldb * 2);
+        }
+    }
     const int64_t stepB = B_TR ? 128 * p.ldb : 128;
     const char* reqA = (const char*)uniform_ptr(p.A + m0 * p.lda + (int64_t)t0 * 64);
-    const char* reqB = (const char*)uniform_ptr(B_TR ? p.B + (int64_t)t0 * 64 * p.ldb + n0 : p.B + n0 * p.ldb + (int64_t)t0 * 64);
+    const char* reqB = (const char*)uniform_ptr(SW_FWD ? p.B + (n0 >> 1) * p.ldb + (int64_t)t0 * 64 : B_TR ? p.B + (int64_t)t0 * 64 * p.ldb + n0 : p.B + n0 * p.ldb + (int64_t)t0 * 64);
     const int krem = kend - (t0 + n - 1) * 64;
-    const int recA = (int)(min((int64_t)BM, p.M - m0) * p.lda * 2), recB = (int)((B_TR ? 64 : min((int64_t)BN, p.N - n0)) * p.ldb * 2), recT = B_TR ? (int)(krem * p.ldb * 2 - n0 * 2) : recB;
+    const int recA = (int)(min((int64_t)BM, p.M - m0) * p.lda * 2), recB = (int)((SW_FWD ? p.N - (n0 >> 1) : B_TR ? 64 : min((int64_t)BN, p.N - n0)) * p.ldb * 2), recT = B_TR ? (int)(krem * p.ldb * 2 - n0 * 2) : recB;
     int rq = 0;            // the K-tile requested next
     auto edge = [&]() {  // the share's last K-tile
         if (rq != n - 1 || krem == 64) return;
@@ -1957,6 +1969,32 @@ __global__ __launch_bounds__(256, 2) void gemm_ring_kernel(GemmParams p) {
     }
     // ---- 16 rows of the wave's 64 columns at a time through LDS, to leave as whole row segments
     float* stg = reinterpret_cast<float*>(smem) + wave * 16 * STG_LD;
+    if constexpr (SW_FWD) {  // u into C[:, unit], g into C[:, N / 2 + unit], u silu(g) of the rounded operands into R[:, unit]; F % 32 == 0, rows in whole 16 bytes (the entry point's condition)
+        const int64_t F = p.N >> 1, unit = (n0 >> 1) + (wc0 >> 1) + (lane & 3) * 8;
+        asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __syncthreads();
+#pragma unroll
+        for (int i = 0; i < FM; ++i) {
+            const int64_t gm = m0 + wr0 + i * 16 + (lane >> 2);
+#pragma unroll
+            for (int j = 0; j < FN; ++j) *reinterpret_cast<f32x4*>(stg + (lane & 15) * STG_LD + j * 16 + (lane >> 4) * 4) = acc[i][j];
+            __builtin_amdgcn_wave_barrier();
+            u32x4 w[3];
+            const float* row = stg + (lane >> 2) * STG_LD + (lane & 3) * 8;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                w[0][e] = pack_bf2(row[2 * e], row[2 * e + 1]), w[1][e] = pack_bf2(row[32 + 2 * e], row[33 + 2 * e]);
+                w[2][e] = pack_bf2(swiglu_act(__uint_as_float(w[0][e] << 16), __uint_as_float(w[1][e] << 16)), swiglu_act(__uint_as_float(w[0][e] & 0xffff0000u), __uint_as_float(w[1][e] & 0xffff0000u)));
+            }
+            __builtin_amdgcn_wave_barrier();
+            if (gm >= p.M || unit >= F) continue;
+            bf16_t* c = reinterpret_cast<bf16_t*>(p.C) + gm * p.ldc + unit;
+            *reinterpret_cast<u32x4*>(c) = w[0];
+            *reinterpret_cast<u32x4*>(c + F) = w[1];
+            *reinterpret_cast<u32x4*>(reinterpret_cast<bf16_t*>(const_cast<void*>((const void*)p.R)) + gm * p.ldr + unit) = w[2];
+        }
+        return;
+    }
     constexpr bool B16 = OUT_DT == MI355_DT_BF16;
     constexpr int VEC = B16 ? 7 : 3;  // elements - 1 of 16 bytes
     const bool slabs = !B16 && p.ksplit > 1;
@@ -2081,6 +2119,7 @@ int launch_ring(GemmParams p, int out_dtype, int ksplit, void* workspace, hipStr
     constexpr int lds = 4 * (BM + 128) * 128;  // gemm_ring_kernel's NS stages
     constexpr int FUSED = B_TR ? MI355_EPI_SWIGLU_BWD : MI355_EPI_GELU_ERF;
     if (p.epilogue == FUSED) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, FUSED>), grid, dim3(256), lds, s, p);
+    else if (!B_TR && p.epilogue == MI355_EPI_SWIGLU_FWD) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, B_TR ? MI355_EPI_NONE : MI355_EPI_SWIGLU_FWD>), grid, dim3(256), lds, s, p);
     else if (ksplit == 1 && out_dtype == MI355_DT_BF16) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_BF16, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
     else if constexpr (BM == 192) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);  // (running sums do not fit the registers)
     else if (!p.fold) hipLaunchKernelGGL((gemm_ring_kernel<BM, MI355_DT_F32, false, B_TR, MI355_EPI_NONE>), grid, dim3(256), lds, s, p);
@@ -2561,7 +2600,8 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         if (quad_ok(form, p, out_dtype)) return launch_quad_form(form, p, out_dtype, persistent, s);
         cfg = 2;
     }
-    const bool ring_epilogue = epilogue == MI355_EPI_NONE || (out_dtype == MI355_DT_BF16 && epilogue == (form == MI355_GEMM_NT ? MI355_EPI_GELU_ERF : MI355_EPI_SWIGLU_BWD));
+    const bool ring_epilogue = epilogue == MI355_EPI_NONE || (out_dtype == MI355_DT_BF16 && epilogue == (form == MI355_GEMM_NT ? MI355_EPI_GELU_ERF : MI355_EPI_SWIGLU_BWD)) ||
+                               (epilogue == MI355_EPI_SWIGLU_FWD && N * ldb * 2 < 0x7fffffffLL);
     if (cfg == 1 && tile_hint == 0 && form != MI355_GEMM_TN && ring_epilogue && !split3 && ablate == 0) {
         int ksplit = 1;
         const bool may_split = epilogue == MI355_EPI_NONE && workspace && !bias && !(N & 7) && !(ldc & 3) && (!residual || !(ldr & 3));

@@ -209,6 +209,25 @@ def test_fused_epilogues_are_the_128_x_128_kernels(M, N, K, rows):
         assert torch.equal(take(L.GEMM_NT, Wt, N, residual, L.EPI_GELU, 0, bias), take(L.GEMM_NT, Wt, N, residual, L.EPI_GELU, 1, bias))
 
 
+@pytest.mark.parametrize("M,F_,K", [(1, 32, 256), (127, 64, 320), (130, 96, 1000), (333, 3584, 1024), (257, 416, 328), (5100, 480, 328), (1056, 3584, 512)])
+def test_swiglu_forward_is_the_128_x_128_kernels(M, F_, K):
+    """Gate-up rows and activations have the bits of hint 1 and of the product and ``swiglu_fwd`` by themselves; rows, units (32 of a tile's 64) and K end inside a tile; nothing beside either is written."""
+    from llm_quest_amd import kernels as KK
+
+    g = torch.Generator(device="cuda").manual_seed(M + F_)
+    A, W = torch.randn(M, K, generator=g, device="cuda").to(BF16), (torch.randn(2 * F_, K + 8, generator=g, device="cuda") * 0.1).to(BF16)[:, :K]
+
+    def take(hint):
+        C, act = torch.full((M + 1, 2 * F_ + 8), 7.0, dtype=BF16, device="cuda"), torch.full((M + 1, F_ + 8), 7.0, dtype=BF16, device="cuda")
+        L.call("mi355_gemm_bf16", L.GEMM_NT, M, 2 * F_, K, A.data_ptr(), K, W.data_ptr(), W.stride(0), C.data_ptr(), C.stride(0), L.DT_BF16, None, act.data_ptr(), act.stride(0), L.EPI_SWIGLU_FWD, None, 0, hint)
+        assert all(bool((x[M:] == 7).all()) and bool((x[:, n:] == 7).all()) for x, n in ((C, 2 * F_), (act, F_)))
+        return C[:M, : 2 * F_], act[:M, :F_]
+
+    (gu, act), (want_gu, want_act) = take(0), take(1)
+    assert torch.equal(gu, want_gu) and torch.equal(act, want_act)
+    assert torch.equal(act, KK.swiglu_fwd(gu.contiguous(), F_))
+
+
 @pytest.mark.parametrize("tokens", [32, 33, 64, 96, 97, 500, 1000])
 def test_wide_weight_gradients_of_few_tokens(tokens):
     """Gradients of a thousand 256 x 256 tiles: the two tiles that a short sum may take give the same bits, which are the fp32 sum rounded once."""
