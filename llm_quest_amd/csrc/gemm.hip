@@ -1133,7 +1133,7 @@ __device__ __forceinline__ void gemm_tile(const GemmParams& p, const int pid, co
     // a third copy of the passes for the SwiGLU-forward form (231.9 vs 233.6 ms/step); not on the 4-wave tile, where a third copy of its four
     // sub-blocks stops the unroller and the accumulators land in scratch
     constexpr bool SWIGLU_FWD_COPY = !A_TR && !B_TR && OUT_DT == MI355_DT_BF16 && T::NW == 8;
-    constexpr bool SWIGLU_BWD_COPY = !A_TR && OUT_DT == MI355_DT_BF16 && T::NW == 8;  // the down-projection's dgrad (NT on W^T in the step, NN otherwise)
+    constexpr bool SWIGLU_BWD_COPY = !A_TR && OUT_DT == MI355_DT_BF16 && T::NW == 8;  // the down-projection's dgrad (of sizes that neither gemm_quad.h nor gemm_ring_kernel takes)
     constexpr bool DELTA_COPY = !A_TR && !B_TR && OUT_DT == MI355_DT_BF16 && T::NW == 8 && T::BK == 64;  // the out-projection's dgrad (NT on W^T), tile 2 only
     if (p.epilogue == MI355_EPI_NONE) {
         run_epilogue(std::integral_constant<int, MI355_EPI_NONE>{});
