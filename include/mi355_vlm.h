@@ -278,7 +278,8 @@ int mi355_layernorm_bwd(int64_t rows, int width, const float* x, const float* sc
  * [parts][3 * width] = dscale | dshift | column sums.  width 768 or 1024, operands 16-byte aligned. */
 int mi355_layernorm_bwd_bf16(int64_t rows, int width, const float* x, const float* scale, const float* mean, const float* rsig, const void* dy, int dy_dtype,
                              const float* dres, float* dx, void* dx_bf16, float* partial, int parts, float eps, int mode, void* stream);
-/* Up to four sums as mi355_reduce_rows_f32's in one launch: out_i[n_i] (+)= sum over the parts_i rows, of pitch ld_i, of p_i (NULL: no such sum).  flags_i: 1 = out_i bf16 (else fp32), 2 = added to. */
+/* Up to four sums as mi355_reduce_rows_f32's in one launch: out_i[n_i] (+)= sum over the parts_i rows, of pitch ld_i, of p_i (NULL: no such sum).  flags_i: 1 = out_i bf16 (else fp32), 2 = added to.  Destinations
+ * do not overlap (refused): the sums of a launch have no order. */
 int mi355_reduce_rows_each(const float* p0, int64_t ld0, int parts0, int64_t n0, void* out0, int flags0, const float* p1, int64_t ld1, int parts1, int64_t n1, void* out1, int flags1,
                            const float* p2, int64_t ld2, int parts2, int64_t n2, void* out2, int flags2, const float* p3, int64_t ld3, int parts3, int64_t n3, void* out3, int flags3, void* stream);
 /* mi355_reduce_rows_f32 over partial [parts][segments * n], every segment into a destination of its own (NULL: dropped; bit i of accumulate: added to). */

@@ -747,6 +747,11 @@ extern "C" int mi355_reduce_rows_each(const float* p0, int64_t ld0, int parts0, 
     for (int i = 0; i < REDUCE_EACH; ++i) {
         if (!given.partial[i]) continue;
         MI355_REQUIRE(given.parts[i] > 0 && given.n[i] > 0 && given.ld[i] >= given.n[i] && given.out[i] && (given.flags[i] & ~3) == 0 && given.n[i] <= 1 << 24, "mi355_reduce_rows_each: bad arguments of sum %d", i);
+        const uintptr_t from = (uintptr_t)given.out[i], to = from + given.n[i] * (given.flags[i] & 1 ? 2 : 4);
+        for (int j = 0; j < count; ++j) {  // the workgroups of one launch store in no order
+            const uintptr_t other = (uintptr_t)e.out[j], end = other + e.n[j] * (e.flags[j] & 1 ? 2 : 4);
+            MI355_REQUIRE(from >= end || other >= to, "mi355_reduce_rows_each: the destination of sum %d overlaps another one's", i);
+        }
         e.partial[count] = given.partial[i], e.out[count] = given.out[i], e.n[count] = given.n[i], e.ld[count] = given.ld[i], e.parts[count] = given.parts[i], e.flags[count] = given.flags[i];
         e.start[count++] = (int)blocks;
         blocks += (given.n[i] + 63) / 64;

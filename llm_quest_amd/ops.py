@@ -68,6 +68,23 @@ def _vecgrad(arena, p):
     return arena.grad_target(p)
 
 
+def _flush_sums(sums):
+    """The vector gradients of a block, [(partial rows, destination, accumulate)], up to four to a launch (``kernels.reduce_rows_each``).  The sums of a launch have no order, so one that adds to what
+    another of them stores -- a parameter that the block holds twice, say a key norm tied to the query norm -- waits for the next launch."""
+    batch, spans = [], []
+    for q in sums:
+        a = q[1].data_ptr()
+        b = a + q[1].numel() * q[1].element_size()
+        if len(batch) == 4 or any(a < hi and lo < b for lo, hi in spans):
+            K.reduce_rows_each(batch)
+            batch, spans = [], []
+        batch.append(q)
+        spans.append((a, b))
+    if batch:
+        K.reduce_rows_each(batch)
+    sums.clear()
+
+
 class Runtime:
     """Per-forward constants shared by all blocks: positions, key mask, RoPE tables, shape."""
 
@@ -114,7 +131,7 @@ def attention_forward(att, arena, h1, rt):
 
 
 def attention_backward(att, arena, h1, ctx, saved, dctx, rt, defer=None, delta=None, sums=None):
-    """Returns dh1 [M,d]; writes the QKV / QK-norm weight gradients (the latter, where ``sums`` is a list, when the caller has it added up: ``kernels.reduce_rows_each``).  ``delta``: the softmax backward's row sums when the out-projection's
+    """Returns dh1 [M,d]; writes the QKV / QK-norm weight gradients (the latter, where ``sums`` is a list, when the caller has it added up: ``_flush_sums``).  ``delta``: the softmax backward's row sums when the out-projection's
     dgrad already left them (kernels.dgrad_attn_delta)."""
     Hq, Hkv, D = att.num_heads, att.num_kv_groups, att.head_dim
     qkv, q, k, rstd, lse = saved
@@ -135,8 +152,8 @@ def attention_backward(att, arena, h1, ctx, saved, dctx, rt, defer=None, delta=N
         view, acc = _vecgrad(arena, p)
         if view is not None:
             mine.append((g, view, acc))
-    if sums is None and mine:
-        K.reduce_rows_each(mine)
+    if sums is None:
+        _flush_sums(mine)
     wqkv = arena.fused(att.w_queries.weight, att.w_values.weight)
     dh1 = K.dgrad(dqkv, wqkv)
     _wgrad(arena, att.w_queries.weight, att.w_values.weight, dqkv, h1, defer)
@@ -203,7 +220,7 @@ def block_backward(blk, saved, dx3, rt, rows=None):
     _wgrad(arena, ffn.lin1.weight, ffn.lin_gate.weight, dgu, h2, wg)
     gview, gacc = _vecgrad(arena, blk.norm2.weight)
     dx2, part = K.rmsnorm_bwd(x2, blk.norm2.weight, rstd2, dh2, dres=dx3, partial=True)
-    sums = [] if gview is None else [(part, gview, gacc)]  # the block's vector gradients: added up by one launch at the end
+    sums = [] if gview is None else [(part, gview, gacc)]  # the block's vector gradients: added up at the end, four to a launch
     if rows is not None:  # the FFN half ran on the kept rows: the others receive no gradient from it
         dx2 = _put_rows(dx2, rt.B, rt.S, rows)
     # ---- attention half
@@ -216,8 +233,7 @@ def block_backward(blk, saved, dx3, rt, rows=None):
     dx, part = K.rmsnorm_bwd(x, blk.norm1.weight, rstd1, dh1, dres=dx2, partial=True)
     if gview is not None:
         sums.append((part, gview, gacc))
-    if sums:
-        K.reduce_rows_each(sums)
+    _flush_sums(sums)
     _flush_wgrads(wg)
     hook = getattr(blk, "_grad_ready", None)
     if hook is not None:

@@ -21,7 +21,7 @@ from . import _lib as L
 from . import kernels as K
 from . import kernels_q35 as Q
 from .arena import ParamArena
-from .ops import FUSE_SWIGLU_BWD, FUSE_SWIGLU_FWD, _flush_wgrads, _vecgrad, _wgrad
+from .ops import FUSE_SWIGLU_BWD, FUSE_SWIGLU_FWD, _flush_sums, _flush_wgrads, _vecgrad, _wgrad
 
 BF16, F32 = torch.bfloat16, torch.float32
 
@@ -53,11 +53,6 @@ def _f32_sum(sums, p, part):
     if not acc:
         p.grad = torch.empty(p.shape, dtype=F32, device=p.device)
     sums.append((part, p.grad.view(-1), acc))
-
-
-def _flush_sums(sums):
-    for i in range(0, len(sums), 4):
-        K.reduce_rows_each(sums[i : i + 4])
 
 
 class Runtime:
