@@ -68,20 +68,35 @@ def _vecgrad(arena, p):
     return arena.grad_target(p)
 
 
+def _vec_sum(sums, arena, p, part):
+    """p.grad (+)= the sum of the rows of ``part``, once ``_flush_sums`` has run; ``arena`` None: a stand-alone fp32 parameter."""
+    if p.requires_grad:
+        sums.append((part, arena, p))
+
+
 def _flush_sums(sums):
-    """The vector gradients of a block, [(partial rows, destination, accumulate)], up to four to a launch (``kernels.reduce_rows_each``).  The sums of a launch have no order, so one that adds to what
-    another of them stores -- a parameter that the block holds twice, say a key norm tied to the query norm -- waits for the next launch."""
-    batch, spans = [], []
-    for q in sums:
-        a = q[1].data_ptr()
-        b = a + q[1].numel() * q[1].element_size()
-        if len(batch) == 4 or any(a < hi and lo < b for lo, hi in spans):
-            K.reduce_rows_each(batch)
-            batch, spans = [], []
-        batch.append(q)
-        spans.append((a, b))
-    if batch:
-        K.reduce_rows_each(batch)
+    """The vector gradients of a block, up to four to a launch (``kernels.reduce_rows_each``).  The sums of a launch have no order, so one that adds to what another of them stores -- a parameter that
+    the block holds twice, say a key norm tied to the query norm -- waits for the next launch.  A gradient is attached where it is written: a backward that ends before (an allocation that fails)
+    leaves ``.grad`` as it was."""
+    made = {id(p): torch.empty(p.shape, dtype=F32, device=p.device) for _, arena, p in sums if arena is None and p.grad is None}
+    launches, keys = [], ()
+    for part, arena, p in sums:
+        own = None if arena is not None else made[id(p)] if p.grad is None else p.grad
+        key = id(p) if own is None else own.untyped_storage().data_ptr()  # (an arena's gradients do not overlap)
+        if len(keys) in (0, 4) or key in keys:
+            launches.append([])
+            keys = set()
+        launches[-1].append((part, arena, p, own))
+        keys.add(key)
+    for group in launches:
+        ready = []
+        for part, arena, p, own in group:
+            view, acc = arena.grad_target(p) if own is None else (own.view(-1), p.grad is not None)
+            ready.append((part, view, acc))
+        K.reduce_rows_each(ready)
+        for _, _, p, own in group:
+            if own is not None and p.grad is None:
+                p.grad = own
     sums.clear()
 
 
@@ -148,10 +163,8 @@ def attention_backward(att, arena, h1, ctx, saved, dctx, rt, defer=None, delta=N
         dq = torch.empty_like(q)
         K.attn_bwd(q, k, v, ctx, dctx, lse, rt.B, rt.S, Hq, Hkv, D, dq, dk, dqkv[:, (Hq + Hkv) * D :], key_mask=rt.key_mask, causal=True, scale=att.att_scaling)
         dqw, dkw = K.qknorm_rope_bwd(qkv, att.q_norm.weight, att.k_norm.weight, rt.cos, rt.sin, rt.pos, rstd, dq, dk, dqkv, Hq, Hkv, D, partial=True)
-    for p, g in ((att.q_norm.weight, dqw), (att.k_norm.weight, dkw)):
-        view, acc = _vecgrad(arena, p)
-        if view is not None:
-            mine.append((g, view, acc))
+    _vec_sum(mine, arena, att.q_norm.weight, dqw)
+    _vec_sum(mine, arena, att.k_norm.weight, dkw)
     if sums is None:
         _flush_sums(mine)
     wqkv = arena.fused(att.w_queries.weight, att.w_values.weight)
@@ -218,9 +231,9 @@ def block_backward(blk, saved, dx3, rt, rows=None):
     wgu = arena.fused(ffn.lin1.weight, ffn.lin_gate.weight)
     dh2 = K.dgrad(dgu, wgu)
     _wgrad(arena, ffn.lin1.weight, ffn.lin_gate.weight, dgu, h2, wg)
-    gview, gacc = _vecgrad(arena, blk.norm2.weight)
+    sums = []  # the block's vector gradients: added up at its end, four to a launch
     dx2, part = K.rmsnorm_bwd(x2, blk.norm2.weight, rstd2, dh2, dres=dx3, partial=True)
-    sums = [] if gview is None else [(part, gview, gacc)]  # the block's vector gradients: added up at the end, four to a launch
+    _vec_sum(sums, arena, blk.norm2.weight, part)
     if rows is not None:  # the FFN half ran on the kept rows: the others receive no gradient from it
         dx2 = _put_rows(dx2, rt.B, rt.S, rows)
     # ---- attention half
@@ -229,10 +242,8 @@ def block_backward(blk, saved, dx3, rt, rows=None):
     dctx, delta = fused if fused is not None else (K.dgrad(dx2, att.out_proj.weight), None)
     _wgrad(arena, att.out_proj.weight, None, dx2, ctx, wg)
     dh1 = attention_backward(att, arena, h1, ctx, att_saved, dctx, rt, wg, delta, sums)
-    gview, gacc = _vecgrad(arena, blk.norm1.weight)
     dx, part = K.rmsnorm_bwd(x, blk.norm1.weight, rstd1, dh1, dres=dx2, partial=True)
-    if gview is not None:
-        sums.append((part, gview, gacc))
+    _vec_sum(sums, arena, blk.norm1.weight, part)
     _flush_sums(sums)
     _flush_wgrads(wg)
     hook = getattr(blk, "_grad_ready", None)

@@ -21,7 +21,7 @@ from . import _lib as L
 from . import kernels as K
 from . import kernels_q35 as Q
 from .arena import ParamArena
-from .ops import FUSE_SWIGLU_BWD, FUSE_SWIGLU_FWD, _flush_sums, _flush_wgrads, _vecgrad, _wgrad
+from .ops import FUSE_SWIGLU_BWD, FUSE_SWIGLU_FWD, _flush_sums, _flush_wgrads, _vec_sum, _wgrad
 
 BF16, F32 = torch.bfloat16, torch.float32
 
@@ -36,23 +36,6 @@ def arena_for_bf16(module):
                 object.__setattr__(m, "_arena", ar)
     ar.ensure()
     return ar
-
-
-def _vec_sum(sums, arena, p, part):
-    """p.grad (bf16, in the arena) (+)= the sum of the rows of ``part``, once ``_flush_sums`` has run."""
-    view, acc = _vecgrad(arena, p)
-    if view is not None:
-        sums.append((part, view, acc))
-
-
-def _f32_sum(sums, p, part):
-    """The same for a stand-alone fp32 parameter."""
-    if not p.requires_grad:
-        return
-    acc = p.grad is not None
-    if not acc:
-        p.grad = torch.empty(p.shape, dtype=F32, device=p.device)
-    sums.append((part, p.grad.view(-1), acc))
 
 
 class Runtime:
@@ -177,7 +160,7 @@ def gdn_backward(att, arena, saved, dgated, rt, defer=None, sums=None):
     h1, proj, y, qn, kn, beta, alpha, o, ck, rstd_p = saved
     dproj = torch.empty_like(proj)
     d_o, dpw = Q.gated_rmsnorm_bwd(o, att.post_norm.weight, proj[:, C : C + VG], rstd_p, dgated, dproj[:, C : C + VG], Hv, Dv, partial=True)
-    _f32_sum(mine, att.post_norm.weight, dpw)
+    _vec_sum(mine, None, att.post_norm.weight, dpw)
     dy = torch.empty_like(y)
     dqn, dkn, dbeta, dalpha = Q.gated_delta_rule_bwd(qn, kn, y[:, 2 * QK :], beta, alpha, ck, d_o, dy[:, 2 * QK :], rt.B, rt.S, Hqk, Hv, Dk, Dv)
     Q.l2norm_bwd(y[:, :QK], dqn, dy[:, :QK], Hqk, Dk)
@@ -186,7 +169,7 @@ def gdn_backward(att, arena, saved, dgated, rt, defer=None, sums=None):
     _vec_sum(mine, arena, att.conv1d.weight, dcw)
     dlog_A, ddtb = Q.gdn_gates_bwd(proj[:, C + VG : C + VG + Hv], proj[:, C + VG + Hv :], att.log_A, att.dt_bias, dbeta, dalpha,
                                    dproj[:, C + VG : C + VG + Hv], dproj[:, C + VG + Hv :], partial=True)
-    _f32_sum(mine, att.log_A, dlog_A)
+    _vec_sum(mine, None, att.log_A, dlog_A)
     _vec_sum(mine, arena, att.dt_bias, ddtb)
     if sums is None:
         _flush_sums(mine)

@@ -19,7 +19,7 @@ class Kernels:
     """Stands in for kernels.py and kernels_q35.py: rows to be added up are whole numbers, so a sum has one value; everything else is a matrix of no interest."""
 
     def __init__(self):
-        self.g, self.given, self.launches = torch.Generator().manual_seed(3), [], 0
+        self.g, self.given, self.launches, self.fails = torch.Generator().manual_seed(3), [], 0, None
 
     def __getattr__(self, name):
         def call(*a, **kw):
@@ -28,6 +28,8 @@ class Kernels:
         return call
 
     def rows(self, n):
+        if len(self.given) == self.fails:
+            raise MemoryError
         self.given.append(torch.randint(-4, 5, (3, n), generator=self.g).float())
         return self.given[-1]
 
@@ -121,6 +123,25 @@ def test_every_vector_gradient_is_the_sum_of_its_contributions(kernels, make, or
         assert p.grad.dtype == p.dtype and torch.equal(p.grad.float(), total)
     if not tied:
         assert kernels.launches == 2 * ((len(order) + 3) // 4)
+
+
+@pytest.mark.parametrize("make,order", [(qwen3, QWEN3), (lambda: hybrid(3), GATED), (lambda: hybrid(0), DELTA)])
+def test_a_backward_that_ends_early_leaves_no_unwritten_gradient(kernels, make, order):
+    """An allocation fails in front of one of the sums: the gradients are what they were, none at first and then the first pass's, and the pass that follows adds to those."""
+    blk, backward = make()
+    params, want = [blk.get_parameter(n) for n in order], None
+    for _ in range(2):
+        for fails in range(len(order)):
+            kernels.given.clear()
+            kernels.fails = fails
+            with pytest.raises(MemoryError):
+                backward()
+            assert all(p.grad is None for p in params) if want is None else all(torch.equal(p.grad.float(), t) for p, t in zip(params, want))
+        kernels.given.clear()
+        kernels.fails = None
+        backward()
+        want = [part.sum(0).view(p.shape) + (0 if want is None else want[i]) for i, (p, part) in enumerate(zip(params, kernels.given))]
+        assert all(torch.equal(p.grad.float(), t) for p, t in zip(params, want))
 
 
 def test_overlapping_destinations_are_refused():
