@@ -53,13 +53,21 @@ def _wgrad(arena, first, last, dy, x, defer=None):
 
 
 def _flush_wgrads(defer):
-    """The weight gradients of one block, each too small to fill the chip, as one grouped TN launch per output dtype."""
-    by_dtype = {}
-    for q in defer:
-        by_dtype.setdefault(q[2].dtype, []).append(q)
-    for qs in by_dtype.values():
-        K.gemm_grouped(L.GEMM_TN, qs)
-    defer.clear()
+    """The weight gradients of one block, each too small to fill the chip, as one grouped TN launch per output dtype (and another where a matrix comes again, one that the block holds twice: the
+    products of a launch have no order)."""
+    while defer:
+        by_dtype, again, spans = {}, [], []
+        for q in defer:
+            lo = q[2].data_ptr()
+            hi = lo + q[2].numel() * q[2].element_size()
+            if any(a < hi and lo < b for a, b in spans):
+                again.append(q)
+            else:
+                by_dtype.setdefault(q[2].dtype, []).append(q)
+            spans.append((lo, hi))
+        for qs in by_dtype.values():
+            K.gemm_grouped(L.GEMM_TN, qs)
+        defer[:] = again
 
 
 def _vecgrad(arena, p):

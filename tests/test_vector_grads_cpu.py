@@ -144,6 +144,39 @@ def test_a_backward_that_ends_early_leaves_no_unwritten_gradient(kernels, make, 
         assert all(torch.equal(p.grad.float(), t) for p, t in zip(params, want))
 
 
+@pytest.mark.parametrize("tied", [{}, {"ffn.lin2": "att.out_proj"}, {"att.out_proj": "att.w_keys"}, {"ffn.lin2": "att.w_queries", "att.out_proj": "att.w_values"}])
+def test_a_weight_that_a_block_holds_twice_is_in_one_grouped_launch_once(kernels, tied, monkeypatch):
+    """The products of a grouped launch have no order either."""
+    blk = TransformerBlock(dict(emb_dim=D, hidden_dim=D, n_heads=2, num_kv_groups=2, head_dim=HEAD, dtype=BF16), 0)
+    for a, b in tied.items():
+        (owner, name), (other, theirs) = a.rpartition(".")[::2], b.rpartition(".")[::2]
+        setattr(blk.get_submodule(owner), name, getattr(blk.get_submodule(other), theirs))
+    arena, g, want, wg = ops.arena_for(blk), torch.Generator().manual_seed(5), {}, []
+    att, ffn = blk.att, blk.ffn
+    launched = []
+
+    def gemm_grouped(form, problems):
+        spans = sorted((out.data_ptr(), out.data_ptr() + out.numel() * out.element_size()) for _, _, out, _ in problems)
+        assert all(a[1] <= b[0] for a, b in zip(spans, spans[1:])), "two products of one launch have the same destination"
+        launched.append(len(problems))
+        for dy, x, out, r in reversed(problems):
+            out.copy_(dy.float().T @ x.float() + (0 if r is None else r.float()))
+
+    monkeypatch.setattr(kernels, "gemm_grouped", gemm_grouped, raising=False)
+    for _ in range(2):
+        for first, last, rows in ((ffn.lin2, None, D), (ffn.lin1, ffn.lin_gate, 2 * D), (att.out_proj, None, D), (att.w_queries, att.w_values, 6 * HEAD)):
+            dy, x = (torch.randint(-2, 3, (4, n), generator=g).to(BF16) for n in (rows, D))
+            ops._wgrad(arena, first.weight, None if last is None else last.weight, dy, x, wg)
+            total = dy.float().T @ x.float()
+            parts = [first] if last is None else [ffn.lin1, ffn.lin_gate] if first is ffn.lin1 else [att.w_queries, att.w_keys, att.w_values]
+            for m, t in zip(parts, total.split([m.weight.shape[0] for m in parts])):
+                want[m.weight] = want.get(m.weight, 0) + t
+        ops._flush_wgrads(wg)
+        assert not wg
+    assert all(torch.equal(p.grad.float(), t) for p, t in want.items())
+    assert tied or launched == [4, 4]
+
+
 def test_overlapping_destinations_are_refused():
     """By the entry point itself, before anything is launched."""
     part, out = torch.zeros(2, 8), torch.zeros(24)
