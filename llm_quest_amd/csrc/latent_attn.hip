@@ -700,10 +700,10 @@ __global__ __launch_bounds__(256) void latent_attn_combine_kernel(LatAttnArgs p,
         l = exp2f(sk - m);
     }
 #pragma unroll
-    for (int j = 0; j < AT; ++j) {  // (a split that holds no key of the row: no part of the sums)
-        const float f = j >= p.splits || ms[j] == NEG ? 0.f : exp2f(ms[j] - m);
-        if (f != 0.f) l += ls[j] * f;
-        ms[j] = f;
+    for (int j = 0; j < AT; ++j) {  // (a split that holds no key of the row: no part of the sums.  One whose weight is too small for a number still is: what is not finite in it stays so)
+        const bool holds = j < p.splits && ms[j] != NEG;
+        ms[j] = holds ? exp2f(ms[j] - m) : -1.f;
+        if (holds) l += ls[j] * ms[j];
     }
     for (int i = AT; i < p.splits; ++i) {
         const float mi = src[i * stride];
@@ -716,7 +716,7 @@ __global__ __launch_bounds__(256) void latent_attn_combine_kernel(LatAttnArgs p,
 #pragma unroll
         for (int j = 0; j < AT; ++j) {
             if (p.sig_bias) acc += j < p.splits ? w[j] : 0.f;  // sigmoid weights simply add up
-            else if (ms[j] != 0.f) acc += w[j] * ms[j];
+            else if (!(ms[j] < 0.f)) acc += w[j] * ms[j];
         }
         for (int i = AT; i < p.splits; ++i) {
             const float mi = src[i * stride], wi = p.ws[(blk0 + i) * stride + 2 * MQ + (int64_t)row * DVP + dv];

@@ -242,3 +242,25 @@ def test_keys_of_one_part_and_of_two_give_the_same_attention(D, DV, window, cap,
         w = torch.softmax(s.masked_fill(((j > pos) | (j <= pos - (window or n + p + 1)))[:, None], float("-inf")), -1)
         err = (2.0**-8 * mag + 2.0**-8) * (w @ vs.abs()) + 1e-30
         assert bool(((one[r].double().view(n, H, DV) - w @ vs).abs() <= err).all())
+
+
+@pytest.mark.parametrize("past", [700, 4000])
+def test_what_is_not_finite_in_a_split_without_weight(past):
+    """Keys whose weight is too small for a number still multiply their values: what is not finite there shows, whether a tile's keys are one split (no ``max_keys``) or several that are joined."""
+    from llm_quest_amd import kernels_seq as S
+
+    H, D, n = 4, 64, past + 1
+    k, v, q = torch.full((n, D), -4.0), torch.randn(n, D, generator=torch.Generator().manual_seed(past)), torch.full((1, H * D), 4.0, device="cuda")
+    k[:64] = 4.0  # all of the weight: the other scores are 369 powers of two below
+    v[past - 40, 5], v[past - 40, 7], v[past - 41, 9] = float("nan"), float("inf"), float("-inf")
+    k, v, zero = k.to(BF16).cuda(), v.to(BF16).cuda(), i32([0])
+    out = []
+    for keys in (0, n):
+        o = torch.empty(1, H * D, device="cuda")
+        S.latent_attn(q, k, None, v, o, H, H, D, 0, D, D, D, D, D, (zero, i32([1]), i32([past]), zero, zero, zero), 1, D**-0.5, max_keys=keys, kv_rep=H)
+        out.append(o.view(H, D))
+    assert S.attn_key_splits(1, 1, 1, H, n) > 1
+    for o in out:
+        assert bool(o[:, [5, 7, 9]].isnan().all()) and int(o.isnan().sum()) == 3 * H
+    fine = [i for i in range(D) if i not in (5, 7, 9)]
+    assert torch.allclose(out[0][:, fine], out[1][:, fine], rtol=2**-7, atol=1e-6)
