@@ -53,6 +53,7 @@ template <int NW, int PRO, int OUT, bool GLU, int ROWS, int T, bool EVEN>
 __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, int steps, const bf16_t* __restrict__ x, int64_t ldx, const bf16_t* __restrict__ nw, float eps,
                                                        const bf16_t* __restrict__ W, int64_t ldw, void* __restrict__ y, int64_t ldy, const void* __restrict__ res, int64_t ldr) {
     static_assert(!EVEN || (PRO != 2 && NW * T % 16 == 0), "whole strips of 512 k");
+    constexpr bool REPEAT = PRO == 1 && ROWS == 8;  // lanes past the last operand row: that row again, else one branch around the loads
     __shared__ float rs[8];
     __shared__ __attribute__((aligned(16))) float part[2][NW][8][16];
     __shared__ __attribute__((aligned(16))) bf16_t act[PRO == 2 ? NW : 1][8][PRO == 2 ? 32 * T + 8 : 8];  // PRO 2: a wave's run of the activated rows
@@ -74,7 +75,9 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
                 gf[t] = in ? *reinterpret_cast<const u32x4*>(x + m * ldx + K + k) : z4;
             }
         } else if constexpr (EVEN) {
-            const bf16_t *row = x + min(r16, M - 1) * ldx + k_lo + c * T * 32 + kg, *g = nw + k_lo + c * T * 32 + kg;
+            const int m = REPEAT ? min(r16, M - 1) : r16;
+            if (m >= M) return;
+            const bf16_t *row = x + m * ldx + k_lo + c * T * 32 + kg, *g = nw + k_lo + c * T * 32 + kg;
 #pragma unroll
             for (int t = 0; t < T; ++t) {
                 xf[t] = *reinterpret_cast<const u32x4*>(row + t * 32);
@@ -136,9 +139,13 @@ __global__ __launch_bounds__(64 * NW) void gemv_kernel(int M, int64_t N, int K, 
         }
     };
     int64_t g = blockIdx.x;
-    if constexpr (EVEN && ROWS == 8) {
+    if constexpr (EVEN) {  // what no load writes
 #pragma unroll
-        for (int t = 0; t < T; ++t) w0[t] = w1[t] = z4;
+        for (int t = 0; t < T; ++t) {
+            if constexpr (!REPEAT) xf[t] = z4;
+            if constexpr (!REPEAT && PRO == 1) gf[t] = z4;
+            if constexpr (ROWS == 8) w0[t] = w1[t] = z4;
+        }
     }
     if constexpr (PRO == 1) {  // row sums: rows wave, wave + NW
         u32x4 v0[4];
