@@ -36,9 +36,11 @@ __device__ __forceinline__ void unpack8(const u32x4 v, float (&f)[8]) {
 // Bound: a launch of a few MB is a chain of memory round trips (operand rows, row sums, weights, results), so the weights' trip runs under the operands': loads return in
 // order, hence operand loads first, weights behind them, and the next 16 rows' weights under this one's products.
 // EVEN: the waves' runs are whole chunks of T steps and end with K: no load has a condition (a branch, a select and an address of its own each: 28 of them in front of the first
-// product were 1 us of a launch), operand rows past the last one are that row again, and what they give is not stored.  us, six rows, weights from memory, before -> EVEN: RMSNorm + 4096 x
+// product were 1 us of a launch), what rows past the last one give is not stored.  us, six rows, weights from memory, before -> EVEN: RMSNorm + 4096 x
 // 1024 6.9 -> 5.8, RMSNorm + SwiGLU of 6144 x 1024 7.9 -> 7.5, 1024 x 3072 5.3 -> 4.9, 1024 x 2048 4.6 -> 4.2.  One row (gemv_one_kernel, T strips of 512 k): 4.9 -> 4.4, 5.2 -> 4.6,
 // 3.8 -> 3.5.  T 4 or 8: chunks of 7 steps (K = 3584) gain nothing, nor do 384 workgroups for 384 groups.
+// Lanes past the last operand row stay out of its loads (one branch; the row again, REPEAT, is as many requests as sixteen rows: eight rows, 4096 x 2048 7.0 us against 6.5, 3072 x 3072 8.3 / 7.3).  REPEAT where
+// the row sums come first and the weights of a group are eight rows: three rows, RMSNorm + 1024 x 2048 5.1 / 5.8.
 constexpr int OUT_BF16 = 0, OUT_F32 = 1, OUT_BF16_BIAS = 2;  // what is stored, and what `res` is: bf16 rows of a residual, or one fp32 row
 constexpr int GEMV_STEPS = 8;  // of 32 k in flight per wave: 8 x 16 bytes a lane
 __device__ __forceinline__ u32x4 pack8(const float (&f)[8]) {
