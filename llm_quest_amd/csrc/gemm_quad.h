@@ -16,6 +16,8 @@
 //     K = 1 024 60 -> 50; eight waves' tile -> here in shares of K: 602 x 1 024, K = 151 936 292 -> 182, 1 300 x 1 024, K = 20 032 90 -> 63.
 //   * Write-out from the registers: B's fragment is the product's first operand, so a lane holds four consecutive columns of a row; v_permlane16_swap makes eight of them, a rotation by eight lanes makes
 //     whole rows of 128 bytes, and no LDS is touched.  Whole lines with the non-temporal hint leave the L2 to the operands: 16 384 x 4 096, K = 1 024 107.0 -> 103.9 us (segments of 64 bytes 109.7).
+//     Rows that start inside a line (a pitch or a corner that is no multiple of 128 bytes) go without it: two waves' parts of a line meet in the L2.  us, with it -> without: 12 288 x 5 000, K = 1 024 132 -> 103,
+//     17 016 x 2 056 in fp32, K = 512 89 -> 56, 8 224 x 3 080 in fp32 from 640 tokens 60 -> 49.
 //     (Beside the products of the last and the next K-tile instead of between them: level.  Stores left out: 91.8.)
 // The sum of every output runs over K in the order of gemm_tile's: the same bits.
 
@@ -227,11 +229,17 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                         rv[blk & 1][hb][half][w] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rr, vr[hb][SW_BWD ? 0 : w] + (unsigned)((blk * 16 + half * 8) * ldr + (SW_BWD ? w * (int)p.N * 2 : 0)), 0, 0));
         }
     };
+    auto corner_c = [&]() { return corner_of(SPLIT ? p.ws + (int64_t)(k0 / max(per, 1)) * p.M * p.N : p.C, SPLIT ? p.N : p.ldc); };
     auto write_out = [&](auto res_c) __attribute__((always_inline)) {  // (grouped: residual or none, every problem its own)
         constexpr bool ADD_R = decltype(res_c)::value;
         asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");  // the last products' way through the pipe: the compiler does not know that the statements above are products (quad_value stays behind this one: both are volatile)
-        const auto rc = __builtin_amdgcn_make_buffer_rsrc(corner_of(SPLIT ? p.ws + (int64_t)(k0 / max(per, 1)) * p.M * p.N : p.C, SPLIT ? p.N : p.ldc), 0, rows * ldc, 0x00020000);
-        constexpr int NT_STORE = 2;  // non-temporal
+        const auto rc = __builtin_amdgcn_make_buffer_rsrc(corner_c(), 0, rows * ldc, 0x00020000);
+        // non-temporal: whole lines only (SwiGLU: of both halves of C's columns)
+        const bool whole = (((unsigned)(uintptr_t)corner_c() | (unsigned)ldc | (SW_FWD || SW_BWD ? (unsigned)p.N * (SW_FWD ? 1 : 2) : 0u)) & 127) == 0;
+        auto put = [&](const u32x4& o, unsigned at) __attribute__((always_inline)) {
+            if (whole) __builtin_amdgcn_raw_buffer_store_b128(o, rc, at, 0, 2);
+            else __builtin_amdgcn_raw_buffer_store_b128(o, rc, at, 0, 0);
+        };
         constexpr int BW = B16 ? 8 : 4;  // consecutive columns of a lane
         [[maybe_unused]] float bias[2][QW][BW];
         if constexpr (BIAS) {
@@ -263,8 +271,8 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                     for (int e = 0; e < 4; ++e)
                         act[e] = pack_bf2(swiglu_act(__uint_as_float(u[half][e] << 16), __uint_as_float(g[half][e] << 16)), swiglu_act(__uint_as_float(u[half][e] & 0xffff0000u), __uint_as_float(g[half][e] & 0xffff0000u)));
                     const unsigned at = vc[0][0] + (unsigned)((blk * 16 + half * 8) * ldc);
-                    __builtin_amdgcn_raw_buffer_store_b128(u[half], rc, at, 0, NT_STORE);
-                    __builtin_amdgcn_raw_buffer_store_b128(g[half], rc, at + (unsigned)p.N, 0, NT_STORE);
+                    put(u[half], at);
+                    put(g[half], at + (unsigned)p.N);
                     __builtin_amdgcn_raw_buffer_store_b128(act, ra, vr[0][0] + (unsigned)((blk * 16 + half * 8) * ldr), 0, 0);
                 }
                 continue;
@@ -287,7 +295,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                                 if constexpr (ADD_R) v += __uint_as_float(rv[blk & 1][hb][half][w][e]);
                                 o[e] = __float_as_uint(v);
                             }
-                            __builtin_amdgcn_raw_buffer_store_b128(o, rc, vc[hb][w] + (unsigned)((blk * 16 + half * 8) * ldc), 0, NT_STORE);
+                            put(o, vc[hb][w] + (unsigned)((blk * 16 + half * 8) * ldc));
                         }
                     }
                 } else if constexpr (BIAS || ADD_R) {
@@ -301,7 +309,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                             if constexpr (ADD_R) v[half][e] += __uint_as_float(e & 1 ? rv[blk & 1][hb][half][0][e >> 1] & 0xffff0000u : rv[blk & 1][hb][half][0][e >> 1] << 16);
                         }
                         const u32x4 o = {pack_bf2(v[half][0], v[half][1]), pack_bf2(v[half][2], v[half][3]), pack_bf2(v[half][4], v[half][5]), pack_bf2(v[half][6], v[half][7])};
-                        __builtin_amdgcn_raw_buffer_store_b128(o, rc, vc[hb][0] + (unsigned)((blk * 16 + half * 8) * ldc), 0, NT_STORE);
+                        put(o, vc[hb][0] + (unsigned)((blk * 16 + half * 8) * ldc));
                     }
                 } else {
                     u32x4 o[2];
@@ -320,10 +328,10 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
                                 swiglu_grads(__uint_as_float(o[half][e] & 0xffff0000u), __uint_as_float(u[e] & 0xffff0000u), __uint_as_float(g[e] & 0xffff0000u), du[1], dg[1]);
                                 o0[e] = pack_bf2(du[0], du[1]), o1[e] = pack_bf2(dg[0], dg[1]);
                             }
-                            __builtin_amdgcn_raw_buffer_store_b128(o0, rc, at, 0, NT_STORE);
-                            __builtin_amdgcn_raw_buffer_store_b128(o1, rc, at + (unsigned)(p.N * 2), 0, NT_STORE);
+                            put(o0, at);
+                            put(o1, at + (unsigned)(p.N * 2));
                         } else {
-                            __builtin_amdgcn_raw_buffer_store_b128(o[half], rc, at, 0, NT_STORE);
+                            put(o[half], at);
                             if constexpr (DELTA) {
                                 // o = d(ctx), rounded: its product with ctx over the half head's 64 columns, folded over the row's eight lanes from their lowest column bit up
                                 const u32x4 cv = rv[blk & 1][hb][half][0];

@@ -133,4 +133,7 @@ def test_tiles_of_asm_products_are_read_late_enough(tmp_path, source, define, le
     for name, body in kernels:
         assert not early_accesses(body.splitlines()) and not late_operands(body.splitlines()), name
         with_asm += bool(re.search(r"#ASMSTART[^#]*v_mfma", body))
+        if "gemm_quad" in name:  # results in whole lines past the L2, parts of lines into it
+            stores = [line for line in body.splitlines() if "buffer_store_dwordx4" in line]
+            assert len([line for line in stores if " nt" in line]) == len([line for line in stores if " nt" not in line]) - (16 if "ELi3E" in name else 0), name  # (SwiGLU forward: the activations too)
     assert with_asm >= least

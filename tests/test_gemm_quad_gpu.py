@@ -131,3 +131,28 @@ def test_shares_of_grouped_weight_gradients(tokens, shapes, odt):
         assert bool((whole[c.shape[0] :] == 7).all()) and bool((whole[:, c.shape[1] :] == 7).all())
         want = a[:, -96:].double().T @ b.double()
         assert off(c[-96:], want + (r[-96:].double() if r is not None else 0), tokens, odt)
+
+
+# rows of results in whole lines of 128 bytes (stored past the L2) and in parts of them: pitches that are a multiple of it and one that is not, a corner beside a line's start; columns that end inside a line
+@pytest.mark.parametrize("form,M,N,K_", [("nt", 383, 520, 448), ("nt", 17_000, 1792, 320), ("nn", 383, 520, 448), ("swiglu", 383, 544, 448), ("swiglu", 383, 520, 448), ("swiglu", 4000, 1088, 256), ("gateup", 600, 576, 320),
+                                         ("gateup", 600, 512, 320), ("tn", 520, 1288, 639)])
+@pytest.mark.parametrize("odt", [BF16, F32])
+def test_results_in_whole_lines_and_in_parts_of_them(form, M, N, K_, odt):
+    if form not in ("nt", "tn") and odt == F32:
+        pytest.skip("bf16 results only")
+    A, B = (draw(M, K_, M), draw(N, K_, N)) if form == "tn" else (draw(M, M, K_), draw(N, K_, N) if form in ("nn", "swiglu") else draw(N, N, K_))
+    gu, act = draw(4, M, 2 * N), torch.empty(M, N // 2, dtype=BF16, device="cuda")
+    W = 2 * N if form == "swiglu" else N
+
+    def take(hint, ld, first):
+        C = torch.full((M + 1, ld), 7.0, dtype=odt, device="cuda")
+        at = C[:M, first : first + W]
+        L.call("mi355_gemm_bf16", {"nt": L.GEMM_NT, "gateup": L.GEMM_NT, "tn": L.GEMM_TN}.get(form, L.GEMM_NN), M, N, K_, L.ptr(A), A.stride(0), L.ptr(B), B.stride(0), L.ptr(at), ld, L.dt_code(odt), None,
+               *{"swiglu": (L.ptr(gu), 2 * N, L.EPI_SWIGLU_BWD), "gateup": (L.ptr(act), N // 2, L.EPI_SWIGLU_FWD)}.get(form, (None, 0, 0)), None, 0, hint)
+        assert bool((C[M:] == 7).all()) and bool((C[:, :first] == 7).all()) and bool((C[:, first + W :] == 7).all())
+        return at
+
+    want = take(5 if form == "tn" else 2, W, 0)
+    whole = (W + 127) // 64 * 64  # of elements: whole lines in either type
+    for ld, first in ((whole, 0), (whole + 64, 64), (whole, 8), (W + 8, 0), (W + 24, 16)):
+        assert torch.equal(take(7, ld, first), want), (ld, first)
