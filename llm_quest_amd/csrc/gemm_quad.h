@@ -257,7 +257,7 @@ __device__ __forceinline__ void quad_tiles(const GemmParams& p, int q, const int
         for (int blk = 0; blk < 8; ++blk) {
             const int ha = blk >> 2, i = blk & 3;
             __builtin_amdgcn_sched_barrier(0);
-            if (blk < 7) fetch(blk + 1, true);
+            if (blk < 7) fetch(blk + 1, ADD_R || !RES);
             if constexpr (SW_FWD) {
                 // column half 0 is u, half 1 the same units' g: u into C[:, unit], g into C[:, N/2 + unit], u silu(g) of the rounded operands into R[:, unit]
                 const auto ra = __builtin_amdgcn_make_buffer_rsrc(corner_of(p.R, p.ldr), 0, rows * ldr, 0x00020000);
