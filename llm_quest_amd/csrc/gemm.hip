@@ -1161,6 +1161,10 @@ __global__ __launch_bounds__(T::NTHREADS, T::MIN_WAVES) void gemm_bf16_kernel(Ge
     gemm_tile<T, A_TR, B_TR, OUT_DT>(p, xcd_chunked(blockIdx.x - split * nwg, nwg), split, smem);
 }
 
+#if GEMM_PART == 2 || !defined(GEMM_PART)
+#include "gemm_persist.h"
+#endif
+
 // ---------------------------------------------------------------------------------------------- ping-pong persistent NT kernel (tile hint 8)
 // The two waves per SIMD of an eight-wave tile (w and w + 4: the upper and the lower 128 rows of the 256 x 256 tile) reach their write-out together, so the
 // matrix pipe of every SIMD idles for the whole write-out: 2.45 of a tile's 27.5 us with the plain epilogue at K = 1 024, a quarter of the tile with the SwiGLU
@@ -2282,6 +2286,7 @@ extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_nt_part8(co
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_tn_part9(const void* params, int out_dtype, int persistent, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_nn_part10(const void* params, int out_dtype, int persistent, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_quad_grouped_part9(void* table, int out_dtype, void* stream);
+extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_persist_part2(const void* params, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_pp_part6(const void* params, void* stream);
 extern "C" __attribute__((visibility("hidden"))) int mi355_gemm_ring_part7(int form, const void* params, int out_dtype, int rows, int ksplit, void* ws, void* stream);
 #if GEMM_PART == 7 || GEMM_PART == -1
@@ -2294,6 +2299,9 @@ extern "C" int mi355_gemm_ring_part7(int form, const void* params, int out_dtype
 #endif
 #if GEMM_PART == 6 || GEMM_PART == -1
 extern "C" int mi355_gemm_pp_part6(const void* params, void* stream) { return launch_pp(*static_cast<const GemmParams*>(params), (hipStream_t)stream); }
+#endif
+#if GEMM_PART == 2 || GEMM_PART == -1
+extern "C" int mi355_gemm_persist_part2(const void* params, void* stream) { return launch_persist(*static_cast<const GemmParams*>(params), (hipStream_t)stream); }
 #endif
 #if GEMM_PART == 8 || GEMM_PART == -1
 extern "C" int mi355_gemm_quad_nt_part8(const void* params, int out_dtype, int persistent, void* stream) {
@@ -2372,6 +2380,18 @@ static bool quad_ok(int form, const GemmParams& p, int out_dtype) {
     if (form == MI355_GEMM_NN) return out_dtype == MI355_DT_BF16 && !p.bias && (p.epilogue == MI355_EPI_NONE || p.epilogue == MI355_EPI_SWIGLU_BWD);
     if (p.epilogue == MI355_EPI_SWIGLU_FWD) return p.N * p.ldb * 2 < 0x7fffffffLL;
     return p.epilogue == MI355_EPI_NONE || p.epilogue == MI355_EPI_SWIGLU_BWD || p.epilogue == MI355_EPI_ATTN_DELTA;
+}
+
+// Sums over K for which an NT product of two rounds of tiles and more runs on gemm_persist.h's eight waves: 192 and less (four K-tiles are what the four waves start from), and what a write-out without
+// anything beside it and an odd K-tile cost them.  Four waves / eight: plain, K = 320 1.10 - 1.22, 448 1.05 - 1.17, 576 1.02 - 1.12, 704 0.99 - 1.08, 832 0.96 - 1.06, 960 0.94 - 0.99; 256 1.02 - 1.11, 384 0.99 - 1.09, 512
+// 0.96 - 1.07, 768 0.91 - 0.99.  SwiGLU forward, 256 0.91 - 1.06, 320 0.93 - 1.15, 448 1.01 - 1.10, 512 0.89 - 1.02, 576 0.92 - 1.07, 704 0.88 - 1.05, 832 0.87 - 1.04; attention delta 320 1.05 - 1.08, 448 1.02 - 1.04, 576
+// 0.99 - 1.02; with a residual 0.71 - 1.03, SwiGLU backward 0.73 - 1.05.
+static bool short_nt(int epilogue, bool residual, int64_t K) {
+    const bool odd = K & 64;
+    if (K <= 192) return true;
+    if (epilogue == MI355_EPI_SWIGLU_FWD) return K <= (odd ? 704 : 256);
+    if (epilogue == MI355_EPI_ATTN_DELTA) return K <= (odd ? 448 : 256);
+    return epilogue == MI355_EPI_NONE && !residual && K <= (odd ? 832 : 512);
 }
 
 // Forward products and input gradients of fewer 256x256 tiles than half of the CUs: measured 92 tiles -> 128x128 wins (+2.8 % on the hybrid step), 180 tiles -> 256x256 wins.  At 128 tiles, plain
@@ -2568,7 +2588,8 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
                             (!residual || ((ldr & 7) == 0 && ((uintptr_t)residual & 15) == 0)) && ldc * 2 * 256 < 0x7fffffffLL && ldr * 2 * 256 < 0x7fffffffLL;
     // four waves of 128x128 (gemm_quad.h), one workgroup per CU walking the tiles from two rounds of them upward: the same bits as tile 2, and 5, whose place they take where they can
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
-    if (tile_hint == 0 && ((cfg == 2 && form == MI355_GEMM_NT) || cfg == 5) && quad_ok(form, p, out_dtype)) {
+    const bool short_sum = persist_ok && tiles256 >= persist_min_tiles() && short_nt(epilogue, residual != nullptr, K);
+    if (tile_hint == 0 && ((cfg == 2 && form == MI355_GEMM_NT) || cfg == 5) && (short_sum || quad_ok(form, p, out_dtype))) {
         const int kind_bit = epilogue == MI355_EPI_SWIGLU_FWD ? 4 : epilogue == MI355_EPI_SWIGLU_BWD ? 8 : residual ? 2 : 1;
         cfg = persist_ok && tiles256 >= persist_min_tiles() && (pp_mask() & kind_bit) ? 8 : 7;
     }
@@ -2597,7 +2618,8 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     }
     if (cfg == 7) {
         const bool persistent = tile_hint == 7 || tiles256 >= persist_min_tiles();
-        if (quad_ok(form, p, out_dtype)) return launch_quad_form(form, p, out_dtype, persistent, s);
+        if (quad_ok(form, p, out_dtype) && !(tile_hint == 0 && short_sum)) return launch_quad_form(form, p, out_dtype, persistent, s);
+        if (persist_ok) return mi355_gemm_persist_part2(&p, s);
         cfg = 2;
     }
     const bool ring_epilogue = epilogue == MI355_EPI_NONE || (out_dtype == MI355_DT_BF16 && epilogue == (form == MI355_GEMM_NT ? MI355_EPI_GELU_ERF : MI355_EPI_SWIGLU_BWD)) ||
@@ -2636,6 +2658,7 @@ extern "C" int mi355_gemm_bf16_attn_delta(int64_t M, int64_t N, int64_t K, const
     p.fold = 0;
     const bool persistent = ((M + 255) / 256) * ((N + 255) / 256) >= persist_min_tiles();
     if (persistent && (pp_mask() & 16) && (K & 63) == 0 && K >= 64 * 5 && ldc * 2 * 256 < 0x7fffffffLL && ldctx * 2 * 256 < 0x7fffffffLL) return mi355_gemm_pp_part6(&p, (hipStream_t)stream);
+    if (persistent && (K & 63) == 0 && K >= 128 && short_nt(MI355_EPI_ATTN_DELTA, true, K) && ldc * 2 * 256 < 0x7fffffffLL && ldctx * 2 * 256 < 0x7fffffffLL) return mi355_gemm_persist_part2(&p, (hipStream_t)stream);
     if (quad_ok(MI355_GEMM_NT, p, MI355_DT_BF16)) return mi355_gemm_quad_nt_part8(&p, MI355_DT_BF16, persistent, (hipStream_t)stream);
     return mi355_gemm_part2(MI355_GEMM_NT, &p, MI355_DT_BF16, nullptr, 0, (hipStream_t)stream);
 }

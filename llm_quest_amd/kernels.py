@@ -748,10 +748,13 @@ def dgrad_on_ring(M, N, Kd, dtype=BF16):
 def dgrad_on_quad(M, N, Kd, out=None, epilogue=False):
     """Whether dX [M, N] = dY [M, Kd] W runs in the NN form on 256 x 256 tiles of four waves (csrc/gemm_quad.h), as fast there as in the NT form and without the copy: more than half of the CUs' worth of tiles, or
     a sum that is divided over the chip.  us, copy + NT / NN: 16 384 x 1 024, K = 3 072 78.7 / 73.6, 6 144 146 / 140.5; 5 664 x 3 584, K = 1 024 60.1 / 49.8; 25 216 x 3 072, K = 768 111.6 / 109.2;
-    12 288 x 1 024, K = 151 936 2 735 / 2 655; 5 664 x 1 024, K = 248 320 2 296 / 2 132."""
+    12 288 x 1 024, K = 151 936 2 735 / 2 655; 5 664 x 1 024, K = 248 320 2 296 / 2 132.  Short sums over two rounds of tiles and more are faster on the copy and eight waves (csrc/gemm_persist.h): 33 000 x 3 072, K = 256 70 / 74,
+    320 79 / 96, 576 127 / 132, 512 113 / 114, 704 level."""
     if (out is not None and (out.dtype != BF16 or out.data_ptr() % 16 or out.stride(0) % 8)) or any(_TILE_BY_FORM.values()) or _TILE_OVERRIDE:
         return False
     tiles = ((M + 255) // 256) * ((N + 255) // 256)
+    if not epilogue and tiles >= PERSIST_MIN_TILES and (Kd <= 256 or (Kd % 128 and Kd <= 576)):
+        return False
     return min(M, N) >= 256 and N % 8 == 0 and Kd % 64 == 0 and Kd > 192 and (tiles > 128 or (Kd > 16384 and not epilogue))
 
 

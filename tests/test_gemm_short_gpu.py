@@ -1,0 +1,59 @@
+"""NT products of short sums over many tiles (csrc/gemm_persist.h): the bits of the eight-wave tile (hint 2), which has its own tests against 64 bits, and which sums take it."""
+
+import pytest
+import torch
+
+from llm_quest_amd import _lib as L
+from llm_quest_amd import kernels as K
+
+pytestmark = pytest.mark.gpu
+BF16, F32 = torch.bfloat16, torch.float32
+
+
+def draw(seed, *shape, dtype=BF16):
+    return torch.randn(*shape, generator=torch.Generator(device="cuda").manual_seed(seed), device="cuda").to(dtype)
+
+
+def kernels_of(fn):
+    fn()
+    torch.cuda.synchronize()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+        fn()
+        torch.cuda.synchronize()
+    return {e.key for e in p.key_averages()}
+
+
+# two K-tiles and more, odd and even numbers of them; rows and columns that end inside a tile, more tiles than CUs (a workgroup walks two or three), more than 128 column panels (their own walk; panels that are no multiple of four)
+@pytest.mark.parametrize("M,N,K_", [(300, 264, 128), (513, 776, 192), (2049, 1288, 256), (33_001, 776, 320), (12_000, 2056, 192), (16_640, 2048, 512), (300, 33_288, 128), (700, 33_800, 320)])
+def test_bits_of_the_eight_wave_tile(M, N, K_, monkeypatch):
+    monkeypatch.setenv("MI355_GEMM_PERSIST_MIN_TILES", "1")
+    x, w, res = draw(M, M, K_ + 8)[:, :K_], draw(N, N, K_), draw(3, M, N)
+    wide = torch.full((M + 1, N + 8), 7.0, dtype=BF16, device="cuda")
+    K.gemm(L.GEMM_NT, x, w, out=wide[:M, :N], allow_split_k=False)
+    assert bool((wide[M:] == 7).all()) and bool((wide[:, N:] == 7).all())
+    assert torch.equal(wide[:M, :N], K.gemm(L.GEMM_NT, x, w, tile=2, allow_split_k=False))
+    assert torch.equal(K.gemm(L.GEMM_NT, x, w, residual=res, allow_split_k=False), K.gemm(L.GEMM_NT, x, w, residual=res, tile=2, allow_split_k=False))
+    F = N // 64 * 32
+    for a, b in zip(K.gemm_gateup_swiglu(x, w[: 2 * F]), K.gemm_gateup_swiglu(x, w[: 2 * F], tile=2)):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("K_,plain,gateup,residual", [(128, True, True, True), (192, True, True, True), (256, True, True, False), (320, True, True, False), (512, True, False, False), (576, True, True, False),
+                                                      (640, False, False, False), (704, True, True, False), (768, False, False, False), (832, True, False, False), (896, False, False, False), (960, False, False, False)])
+def test_which_sums_take_it(K_, plain, gateup, residual):
+    M, N = 16_384, 2048  # 512 tiles; under them, and where the caller keeps persistent kernels off, none does
+    x, w, res = draw(1, M, K_), draw(2, N, K_), draw(3, M, N)
+    took = lambda fn: any("gemm_nt_persist_kernel" in n for n in kernels_of(fn))
+    assert took(lambda: K.gemm(L.GEMM_NT, x, w)) is plain
+    assert took(lambda: K.gemm_gateup_swiglu(x, w)) is gateup
+    assert took(lambda: K.gemm(L.GEMM_NT, x, w, residual=res)) is residual
+    assert not took(lambda: K.gemm(L.GEMM_NT, x[: M - 256], w))
+    if K_ in (128, 320, 640):
+        wn = draw(2, K_, N)
+        assert took(lambda: K.dgrad(x, wn)) is plain and K.dgrad_on_quad(M, N, K_) is not plain
+        K.persistent_gemm(False)
+        try:
+            assert not took(lambda: K.gemm(L.GEMM_NT, x, w))
+        finally:
+            K.persistent_gemm(True)
+
