@@ -2568,10 +2568,11 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
         if (M < 256 || N < 256) cfg = 1;
         else if (long_split && tiles256 < 128) cfg = 3;
         else if (small_tiles(form, M, N, epilogue)) cfg = 1;
-        // weight gradients that gemm_quad.h takes: two 128x128 tiles per CU up to half of the CUs' worth of 256x256 ones, else those.  us, the choice before (in brackets its tile) -> here: 151 936 x 1 024,
+        // weight gradients that gemm_quad.h takes: two 128x128 tiles per CU where those are one round, and where few tokens' 256x256 ones need a second round for a few of them (fp32, 264 tiles 200 tokens 28.6 / 31.2, 1 000
+        // 57.3 / 58.7, 2 000 116 / 95; 288 tiles 200 28.9 / 31.1, 640 44.6 / 43.5); else the larger ones.  us, the choice before (in brackets its tile) -> here: 151 936 x 1 024,
         // 197 tokens 142 (2) -> 106, 333 181 (1) -> 138, 602 250 (3) -> 196, 1 000 354 (3) -> 275; 248 320 x 1 024, 333 tokens 294 (3) -> 212; 50 256 x 768, 602 80 (1) -> 59; 12 288 x 1 024, 200 16 (1)
         // -> 12, 900 37 (1) -> 26; 144 tiles, 512 tokens 21.5 (1) -> 16, 1 024 34 (1) -> 25, 3 072 86 (1) -> 60.  Not at 128 tiles: 200 11.0 / 11.4, 602 17.1 / 17.5, 2 048 38.5 / 39.6; 64: 8.5 / 11.4, 17 / 23
-        else if (form == MI355_GEMM_TN && quad_ok(form, p, out_dtype)) cfg = M * N <= 5 * 1024 * 1024 || tiles256 <= 128 ? 1 : 7;
+        else if (form == MI355_GEMM_TN && quad_ok(form, p, out_dtype)) cfg = M * N <= 5 * 1024 * 1024 || ((M + 127) / 128) * ((N + 127) / 128) <= 512 || (tiles256 > 256 && K < (tiles256 <= 272 ? 1024 : tiles256 <= 288 ? 512 : 0)) ? 1 : 7;
         // those that it does not: the 4-wave loop (128x128 per wave: a third fewer transposing reads per MFMA than the 8-wave tiles, every read issued from asm).  Batch 160:
         // the block's grouped launch 3 327 -> 3 028 us, the LM head's 25.9 -> 22.7 ms in isolation; in the step 469.0 / 468.9 -> 456.9 / 458.0 ms (same box, bit-identical)
         // Under 160 tiles two small ones per CU fill the chip better (6 144 x 1 024, us, tile 5 / 1: 61 tokens 14 / 9, 602 26 / 17, 2 048 57 / 38, 5 664 137 / 91); few tokens are write-out,
@@ -2667,7 +2668,7 @@ extern "C" int mi355_gemm_bf16_attn_delta(int64_t M, int64_t N, int64_t K, const
 static int grouped_launches(int form, int count, const mi355_gemm_problem* problems, int out_dtype, int tile_hint, void* workspace, int64_t workspace_bytes, void* stream) {
     GroupTable tbl;
     tbl.count = count;
-    int64_t tiles256 = 0, outputs = 0, longest = 0;
+    int64_t tiles256 = 0, tiles128 = 0, outputs = 0, longest = 0;
     bool small = false;
     for (int i = 0; i < count; ++i) {
         const mi355_gemm_problem& q = problems[i];
@@ -2679,6 +2680,7 @@ static int grouped_launches(int form, int count, const mi355_gemm_problem* probl
         p.ad_lse = nullptr; p.ad_delta = p.ad_nl2 = p.ad_ndl = nullptr; p.ad_S = p.ad_Hq = 0;
         p.split3 = 0, p.fold = 0;
         tiles256 += ((q.M + 255) / 256) * ((q.N + 255) / 256);
+        tiles128 += ((q.M + 127) / 128) * ((q.N + 127) / 128);
         outputs += q.M * q.N;
         longest = q.K > longest ? q.K : longest;
         small |= q.M < 256 || q.N < 256;
@@ -2686,9 +2688,10 @@ static int grouped_launches(int form, int count, const mi355_gemm_problem* probl
     for (int i = count; i < MAX_GROUP; ++i) tbl.g[i] = tbl.g[0];
     bool quad = form == MI355_GEMM_TN;
     for (int i = 0; i < count; ++i) quad = quad && quad_ok(form, tbl.g[i], out_dtype);
-    // 256x256 tiles (one workgroup per CU) once they cover most of the chip -- those of gemm_quad.h more than half of it --; otherwise 128x128 (two per CU, 4x the tiles).  us, 128x128 / gemm_quad.h: 144 tiles,
+    // 256x256 tiles (one workgroup per CU) once they cover most of the chip -- those of gemm_quad.h as soon as the others are more than one round --; otherwise 128x128 (two per CU, 4x the tiles).  us, 128x128 /
+    // gemm_quad.h: 504 small tiles (129 large ones), 440 tokens 14.8 / 16.7, 2 850 51.8 / 55.0; 144 large ones,
     // 250 tokens 14.9 / 11.8, 602 23.5 / 18.1, 1 500 44 / 32; 240 tiles 18 / 13.4, 29 / 21, 57 / 39
-    int cfg = tile_hint ? tile_hint : ((small || tiles256 < (quad ? 129 : 160)) ? 1 : (form == MI355_GEMM_TN ? 5 : 3));
+    int cfg = tile_hint ? tile_hint : ((small || (quad ? tiles128 <= 512 : tiles256 < 160)) ? 1 : (form == MI355_GEMM_TN ? 5 : 3));
     // Weight gradients whose 256x256 tiles are one round and up to half of a second.  Few tokens: 128x128 tiles, two per CU.  Many: the problems that fill the round best go on it
     // and the others follow on 128x128 tiles, which all have a place at once.  us, one launch on 256x256 / one on 128x128 / two launches: 328 tiles (8 224, 7 168, 3 584 and 2 048 by
     // 1 024) 333 tokens 45 / 39 / 39, 1 024 77 / 67 / 70, 2 048 121 / 109 / 106, 5 664 291 / 282 / 254; 288 tiles 2 048 tokens 114 / 92 / 91, 5 664 271 / 233 / 211; 320 tiles

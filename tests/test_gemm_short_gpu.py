@@ -57,3 +57,14 @@ def test_which_sums_take_it(K_, plain, gateup, residual):
         finally:
             K.persistent_gemm(True)
 
+
+def test_weight_gradients_just_beyond_one_round_of_tiles():
+    """Few tokens: 128 x 128 tiles (in brackets those of 256 x 256) where they are one round of two a CU, and where the larger ones need a second round for a few."""
+    def small(T, shapes, odt=BF16):
+        pr = [(draw(1, T, m), draw(2, T, n), torch.empty(m, n, dtype=odt, device="cuda"), None) for m, n in shapes]
+        fn = (lambda: K.gemm(L.GEMM_TN, pr[0][0], pr[0][1], out_dtype=odt)) if len(shapes) == 1 else (lambda: K.gemm_grouped(L.GEMM_TN, pr))
+        return not any("gemm_quad" in n for n in kernels_of(fn))
+
+    assert small(300, [(2304, 768), (768, 2048), (4112, 768), (768, 2056)])  # 504 (129)
+    assert not small(300, [(2304, 768), (768, 2304), (4112, 768), (768, 2056)])  # 516 (132)
+    assert small(640, [(8224, 2048)]) and small(640, [(8704, 2048)]) and not small(1024, [(8704, 2048)]) and small(300, [(9216, 2048)]) and not small(640, [(9216, 2048)]) and not small(300, [(9472, 2048)])  # (264, 272, 288, 296)
