@@ -307,7 +307,7 @@ struct Registered {
     PyObject* op##_body(Call& c)
 
 // ---------------------------------------------------------------------------------------------- kernels.py
-// product with the checks of kernels.gemm; no tile hint, no split3 output.  A launch that the persistent kernel may take goes to Python, which counts those.
+// product with the checks of kernels.gemm; no tile hint, no split3 output.  A launch that a window of kernels.py counts goes to Python (see _nt_tick).
 T product(Call& c, int form, const T& a, const T& b, T out, at::ScalarType out_dtype, const T& bias, const T& residual, int epilogue, bool may_split) {
     need(a.rows() && b.rows() && a.is(BF16) && b.is(BF16));
     const bool at = form == MI355_GEMM_TN, bt = form != MI355_GEMM_NT;
@@ -364,7 +364,7 @@ OP(gemm_dgrad_swiglu_bwd, "dy", "w", "gu", "tile") {
     need(c.integer(3, 0) == 0 && dy.rows() && w.rows());
     const int64_t M = dy.size(0), K = dy.size(1), F = w.size(1);
     need(dy.is(BF16) && w.is(BF16) && gu.is(BF16) && w.size(0) == K && gu.contiguous() && gu.shape({M, 2 * F}) && kernels_int("_TILE_OVERRIDE") == 0);
-    need(M < kernels_int("DGRAD_NT_MIN_ROWS") && kernels_true("DGRAD_NT"));  // (from there on the NT form, on a transposed weight)
+    need(M < kernels_int("DGRAD_NT_MIN_ROWS") && kernels_true("DGRAD_NT"));  // (from there on kernels.dgrad_on_quad decides about the form)
     PyObject* key = PyLong_FromLong(MI355_GEMM_NN);
     PyObject* tile = PyDict_GetItem(kernels_item("_TILE_BY_FORM"), key);
     Py_DECREF(key);

@@ -5,6 +5,7 @@ pointer reaches the GPU, allocates outputs with torch (device memory plumbing on
 torch's current stream.
 """
 
+import contextlib
 import os
 
 import torch
@@ -49,10 +50,10 @@ _PERSIST_USER = os.environ.get("MI355_GEMM_PERSIST_MIN_TILES")  # the user's own
 
 
 def persistent_gemm(enabled):
-    """The library takes the persistent NT kernel (one workgroup per CU for a launch's whole length, csrc/gemm.hip) by itself from 512 tiles upward.  That kernel
-    assumes its 256 workgroups all START together: a CU that a collective's channel occupies takes no GEMM workgroup (each needs the CU's whole register file and
-    LDS), and the workgroups that find no CU only start when the first ones have walked their whole share -- the launch then lasts up to twice as long, where the
-    per-tile kernel merely loses the occupied CUs' share.  ``ddp.GradSync`` therefore switches the automatic choice off from the first collective of a backward until
+    """The library takes persistent kernels (one workgroup per CU for a launch's whole length, csrc/gemm.hip) for products of 512 tiles and more by itself.  They
+    assume that their 256 workgroups all START together: a CU that a collective's channel occupies takes no GEMM workgroup (each needs the CU's whole register file and
+    LDS), and the workgroups that find no CU only start when the first ones have walked their whole share -- the launch then lasts up to twice as long, where a workgroup
+    per tile merely loses the occupied CUs' share.  ``ddp.GradSync`` therefore switches the automatic choice off from the first collective of a backward until
     the streams have joined (``persistent_gemm(False)`` ... ``persistent_gemm(True)``); an explicit ``tile=7`` still selects it."""
     if not enabled:
         os.environ["MI355_GEMM_PERSIST_MIN_TILES"] = "1000000000"
@@ -62,11 +63,27 @@ def persistent_gemm(enabled):
         os.environ["MI355_GEMM_PERSIST_MIN_TILES"] = _PERSIST_USER
 
 
+@contextlib.contextmanager
+def beside_another_stream():
+    """Products enqueued inside run beside another stream's (``multimodal.vlm_engine.VisionAhead``): a workgroup per tile.  What was in force before is back behind it; a window that is open stays open."""
+    before, window = os.environ.get("MI355_GEMM_PERSIST_MIN_TILES"), _window_is_open()
+    persistent_gemm(False)
+    try:
+        yield
+    finally:
+        if window and not _window_is_open():
+            persistent_gemm(True)
+        elif before is None:
+            os.environ.pop("MI355_GEMM_PERSIST_MIN_TILES", None)
+        else:
+            os.environ["MI355_GEMM_PERSIST_MIN_TILES"] = before
+
+
 PERSIST_MIN_TILES = 512  # csrc/gemm.hip: persist_min_tiles()
 
 
 class _GemmWindow:
-    """A bounded stretch of the compute stream in which NT launches stay off the persistent kernel (``ddp.GradSync`` opens one behind every bucket group it hands to the
+    """A bounded stretch of the compute stream in which products stay off persistent kernels (``ddp.GradSync`` opens one behind every bucket group it hands to the
     communication stream): ``left`` launches to go, then ``on_close`` -- the compute stream waits for the group's collectives -- and the library's own choice is back.
     ``stream``: the compute stream the window belongs to (captured when it opens); launches on other streams (a vision tower running ahead, an evaluation stream) neither
     count against it nor close it."""
@@ -79,12 +96,16 @@ class _GemmWindow:
 _WINDOW = _GemmWindow()
 
 
+def _window_is_open():
+    return _WINDOW.left > 0 or _WINDOW.on_close is not None
+
+
 def open_gemm_window(launches, on_close=None, stream=None):
     """The next ``launches`` persistent-sized NT GEMM launches of ``stream`` (default: the current one) run on the per-tile kernel (a collective's channels hold CUs
     meanwhile; the persistent kernel's 256 workgroups must all start together, see ``persistent_gemm``); in front of the launch after them ``on_close()`` runs and the
     persistent kernel is allowed again.  A window opened while one is open extends it; both hand-offs run at its end."""
     w = _WINDOW
-    if w.left == 0 and w.on_close is None:
+    if not _window_is_open():
         persistent_gemm(False)
         w.stats["windows"] += 1
         w.stream = stream
@@ -99,7 +120,7 @@ def open_gemm_window(launches, on_close=None, stream=None):
 def close_gemm_window():
     """End the window now (``GradSync.finish_step``; also the first launch behind a window's last one)."""
     w = _WINDOW
-    if w.left == 0 and w.on_close is None:
+    if not _window_is_open():
         return
     w.closed_early = w.left > 0  # ended by finish_step before its launches ran out (the hand-off callbacks may ask)
     cb, w.left, w.on_close, w.stream = w.on_close, 0, None, None
@@ -113,8 +134,9 @@ def _persist_min_tiles():
 
 
 def _nt_tick(M, N, eligible=True, device=None):
-    """Called in front of every NT launch, and of an input gradient that stands in its place (``dgrad_on_quad``).  Counts only launches the library would put on the persistent kernel (csrc/gemm.hip ``persist_ok``: bf16 output, no bias,
-    plain / SwiGLU epilogue, no tile hint -- the caller says so through ``eligible`` -- and at least the threshold's tiles), and only those of the window's own stream."""
+    """Called in front of every NT launch, and of an input gradient that stands in its place (``dgrad_on_quad``): a window's length is counted in those of bf16 results without bias, plain or
+    with a SwiGLU epilogue, that the library would put on a persistent kernel (csrc/gemm.hip ``persist_ok``, at least the threshold's tiles; no tile hint) -- the caller says so through
+    ``eligible`` -- and in those of the window's own stream.  What else is persistent by size (a bias, fp32 results, weight gradients) is kept off while the window is open, and not counted."""
     if not eligible or ((M + 255) // 256) * ((N + 255) // 256) < _persist_min_tiles():
         return
     w = _WINDOW

@@ -123,7 +123,9 @@ class VisionAhead:
             self.stream = torch.cuda.Stream(device=dev)
         ready = torch.cuda.Event()
         ready.record(torch.cuda.current_stream(dev))  # whatever produced `images` on the main stream
-        with torch.cuda.stream(self.stream), torch.no_grad():
+        from llm_quest_amd import kernels as K
+
+        with torch.cuda.stream(self.stream), torch.no_grad(), K.beside_another_stream():
             self.stream.wait_event(ready)
             hidden = _vision_states(self.vit, images, self.hf)
             done = torch.cuda.Event()

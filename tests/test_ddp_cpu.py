@@ -393,6 +393,44 @@ def test_persistent_gemm_switch_restores_the_users_threshold(monkeypatch):
     assert os.environ[var] == "64"
 
 
+def test_a_tower_beside_the_step_stays_off_persistent_kernels(monkeypatch):
+    """VisionAhead enqueues the next batch's tower beside this batch's step: its products run a workgroup per tile, and what was in force before is in force again -- the library's threshold, the user's,
+    a switch that is off, a window that is open (and none that has closed meanwhile)."""
+    import contextlib
+    import os
+    from types import SimpleNamespace as NS
+
+    from llm_quest_amd import kernels as K
+    from llm_quest_amd.multimodal import vlm_engine as V
+
+    var, seen = "MI355_GEMM_PERSIST_MIN_TILES", []
+    stream = NS(wait_event=lambda e: None)
+    monkeypatch.setattr(torch, "cuda", NS(Stream=lambda device: stream, Event=lambda: NS(record=lambda s: None), current_stream=lambda d: stream, stream=lambda s: contextlib.nullcontext()))
+    monkeypatch.setattr(K, "_WINDOW", K._GemmWindow())
+    meanwhile = []
+    monkeypatch.setattr(V, "_vision_states", lambda *a: seen.append(os.environ.get(var)) or [f() for f in meanwhile])
+    ahead = V.VisionAhead(NS(parameters=lambda: []))
+    images = NS(device="cuda:0", record_stream=lambda s: None)
+    monkeypatch.delenv(var, raising=False)
+    for user in (None, "64"):
+        monkeypatch.setattr(K, "_PERSIST_USER", user)
+        K.persistent_gemm(True)
+        ahead.submit(images)
+        assert os.environ.get(var) == user
+        K.persistent_gemm(False)
+        ahead.submit(images)
+        assert os.environ[var] == "1000000000"
+        K.persistent_gemm(True)
+        K.open_gemm_window(2, None)
+        ahead.submit(images)
+        assert os.environ[var] == "1000000000" and K._WINDOW.left == 2
+        meanwhile.append(K.close_gemm_window)
+        ahead.submit(images)
+        assert os.environ.get(var) == user
+        meanwhile.clear()
+    assert seen == ["1000000000"] * 8
+
+
 def test_gemm_window_bounds_the_per_tile_stretch_behind_a_bucket_group(monkeypatch):
     """kernels.open_gemm_window(k, on_close): the next k persistent-sized NT launches stay off the persistent kernel, the launch after them first runs the
     hand-off (the compute stream's wait for the group's collectives) and re-enables it; small launches do not count; a window opened inside a window extends
