@@ -1127,9 +1127,13 @@ extern "C" int mi355_bgemm(int batch, int M, int N, int K, const void* A, int a_
         // mostly empty and its tiles are no fuller: 640 rows in 16 groups, N = 1024, K = 1792 (72 tiles at most) 32 / 38
         if (vec && K % WK == 0 && wide_tiles >= (grp_offs ? 64 : 160) && wide_tiles <= (1 << 30)) {
             const int64_t words = c_dt == MI355_DT_F32 ? 4 : 8;  // of 16 bytes
-            // four waves wherever they can: K in pairs of K-tiles, two pairs at least; a panel's weights within a descriptor; the groups in the tables; columns and rows of C in whole 16 bytes.  Faster
-            // at every size that comes this far (bgemm_quad.h); the eight-wave kernel takes the rest
-            if (K % 128 == 0 && K >= 256 && batch <= QUAD_GROUPS && sbn * 2 * 512 < 0x7fffffffLL && (epi >= 2 ? n_out : N) % 8 == 0 && ldc % words == 0 && c_bs % words == 0 && ((uintptr_t)C & 15) == 0) {
+            // four waves where they can -- K in pairs of K-tiles, two pairs at least; a panel's weights within a descriptor; the groups in the tables; columns and rows of C in whole 16 bytes -- and are faster: all
+            // products of one matrix; groups from the K on where a tile's products outweigh its look-ups and a write-out with nothing beside it.  Four waves / eight, mean over 4 - 64 groups and 300 - 16 000 rows
+            // (single ones up to 0.1 beside it): plain and squared 256 1.05 - 1.13, 512 1.00 - 1.05, 640 0.95 - 1.03, 768 0.94 - 1.01, 1 024 0.93 - 1.00, 2 048 0.86 - 0.91; SiLU 256 0.96 - 1.02, 512 0.91 - 0.97, 1 024
+            // 0.90 - 0.94; the longer activations 256 1.07 - 1.10, 640 1.00 - 1.07, 768 0.99 - 1.03, 1 024 0.97 - 0.99 (single ones 1.15), 1 280
+            // 0.94 - 0.97, 2 048 0.89 - 0.97.  One matrix: 256 0.54 - 0.79, 1 024 0.65 - 0.85
+            const int least = !grp_offs ? 256 : epi == 4 ? 512 : epi >= 2 ? 1280 : 768;
+            if (K % 128 == 0 && K >= least && batch <= QUAD_GROUPS && sbn * 2 * 512 < 0x7fffffffLL && (epi >= 2 ? n_out : N) % 8 == 0 && ldc % words == 0 && c_bs % words == 0 && ((uintptr_t)C & 15) == 0) {
                 const unsigned grid = (unsigned)(wide_tiles < 256 ? wide_tiles : 256), lds = QUAD_SMEM + (2 * 256 + 2 * (QUAD_GROUPS + 1)) * 4;
                 if (epi >= 2) bgemm_quad_kernel<true><<<grid, 256, lds, ST(stream)>>>(p, batch, (int)wide_tn);
                 else bgemm_quad_kernel<false><<<grid, 256, lds, ST(stream)>>>(p, batch, (int)wide_tn);

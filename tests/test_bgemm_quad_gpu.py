@@ -13,6 +13,9 @@ EDGES = [1, 0, 15, 17, 31, 33, 63, 65, 0, 127, 129, 191, 193, 223, 225, 255, 256
 # the shortest sum (four K-tiles), longer ones; columns that end inside a tile and inside its first half; more tiles than CUs (a workgroup walks several of different heights)
 CASES = [(EDGES, 1032, 256, 0, F32), (EDGES, 2568, 384, 0, BF16), (EDGES, 2560, 512, 1, F32), (EDGES, 1856, 256, 4, BF16), (EDGES, 2048, 640, 2, F32), (EDGES, 1216, 256, 3, BF16),
          ([1100, 0, 3, 700], 5000, 256, 0, BF16), ([2] * 250, 264, 256, 4, BF16), ([], 2056, 256, 1, BF16), ([], 4096, 384, 4, F32)]
+# ... the same at the shortest sums that groups take the four waves for (bgemm.hip; under them the eight-wave kernel's): 768, SiLU 512, the other gated ones 1 280
+CASES += [(EDGES, 1032, 768, 0, F32), (EDGES, 2568, 896, 0, BF16), (EDGES, 2560, 768, 1, F32), (EDGES, 1856, 512, 4, BF16), (EDGES, 2048, 1280, 2, F32), (EDGES, 1216, 1408, 3, BF16), ([1100, 0, 3, 700], 5000, 768, 0, BF16),
+          ([2] * 250, 264, 512, 4, BF16)]
 
 
 @pytest.mark.parametrize("lens,N,K,epi,odt", CASES)
@@ -57,3 +60,18 @@ def test_groups_of_rows(lens, N, K, epi, odt):
         got = out[dst, :width].double()
         rows = (got - y).norm(dim=1) / (y.norm(dim=1) + 1e-30)  # row by row: one that came from another place is off by about its size
         assert float(rows.max()) < tol, (b, len(src))
+
+
+@pytest.mark.parametrize("K,epi,quad", [(640, 0, False), (768, 0, True), (640, 1, False), (768, 1, True), (384, 4, False), (512, 4, True), (1152, 2, False), (1280, 2, True), (1152, 3, False), (1280, 3, True), (832, 0, False)])
+def test_which_sums_of_groups_take_four_waves(K, epi, quad):
+    a, w, out = torch.zeros(900, K, dtype=BF16, device="cuda"), torch.zeros(8, 2048, K, dtype=BF16, device="cuda"), torch.empty(900, 1024 if epi >= 2 else 2048, dtype=BF16, device="cuda")
+    offs = torch.tensor([0, 100, 100, 300, 440, 460, 700, 899, 900], dtype=torch.int32, device="cuda")
+
+    def run():
+        S.bgemm(a, w, out, 900, 2048, K, grp_offs=offs, batch=8, lda=K, sbn=K, b_bs=2048 * K, epi=epi, limit=1.0, n_out=1024 if epi >= 2 else 0)
+        torch.cuda.synchronize()
+
+    run()
+    with torch.profiler.profile(activities=[torch.profiler.ProfilerActivity.CUDA]) as p:
+        run()
+    assert any("bgemm_quad_kernel" in e.key for e in p.key_averages()) is quad
