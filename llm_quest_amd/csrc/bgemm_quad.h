@@ -48,11 +48,11 @@ __global__ __launch_bounds__(256, 1) void bgemm_quad_kernel(BgemmArgs p, int bat
         b = __builtin_amdgcn_readfirstlane(b);
         const int before = __builtin_amdgcn_readfirstlane(tiles[b]), mine = __builtin_amdgcn_readfirstlane(tiles[b + 1]) - before, local = at - before * tn, tm = local % mine;
         const int row0 = p.grp_offs ? __builtin_amdgcn_readfirstlane(offs[b]) : 0, rows = __builtin_amdgcn_readfirstlane(offs[b + 1]) - __builtin_amdgcn_readfirstlane(offs[b]);
-        const int share = (rows + mine - 1) / mine, m0 = tm * share;
+        const int share = (rows + mine - 1) / mine, m0 = tm * share;  // (share <= 256 and 256 (mine - 1) < rows: no tile is without rows)
         Tile t;
         t.b = b, t.n0 = local / mine * 256;
-        t.first = row0 + min(m0, rows - 1);
-        t.cnt = max(min(share, rows - m0), 0);  // (rounding up can leave the last of some hundred tiles without any)
+        t.first = row0 + m0;
+        t.cnt = min(share, rows - m0);
         t.per = ((t.cnt + 1) / 2 + 15) & ~15;
         return t;
     };
@@ -82,14 +82,14 @@ __global__ __launch_bounds__(256, 1) void bgemm_quad_kernel(BgemmArgs p, int bat
         for (int h = 0; h < 2; ++h)
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const int r = pr + j * 8, own = h * 64 + (r & 63), row = t.first + min((own < t.per ? (r >> 6) * t.per + own : t.cnt), max(t.cnt, 1) - 1);
+                const int r = pr + j * 8, own = h * 64 + (r & 63), row = t.first + min((own < t.per ? (r >> 6) * t.per + own : t.cnt), t.cnt - 1);
                 next_row[h][j] = a_list[p.a_rows ? row : 0];
                 if (!p.a_rows) next_row[h][j] = row;
             }
         const unsigned long long at = (unsigned long long)((const bf16_t*)p.B + (int64_t)t.b * p.b_bs + (int64_t)t.n0 * p.sbn);
         nextB = (const char*)(((unsigned long long)__builtin_amdgcn_readfirstlane((unsigned)(at >> 32)) << 32) | (unsigned)__builtin_amdgcn_readfirstlane((unsigned)at));
         next_recB = (int)(min(256, p.N - t.n0) * p.sbn * 2);
-        const int row = t.first + min(tid, max(t.cnt, 1) - 1);
+        const int row = t.first + min(tid, t.cnt - 1);
         next_to = c_list[p.c_rows ? row : 0];
         if (!p.c_rows) next_to = row;
     };
