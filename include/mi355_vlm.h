@@ -77,11 +77,12 @@ int mi355_abi_version(void);
  *   tile_hint    0 = choose by shape; 1 = 128x128 tile (4 waves), 2 = 256x256 tile (8 waves), 3 = 256x256, alternating wave groups,
  *                4 = 3 with one barrier per phase, 5 = 256x256 as four waves of 128x128 (one per SIMD, accumulators in AGPRs),
  *                7 = 256x256 as four waves of 128x128 on a ring of panels, ONE workgroup per CU walking its share of the tiles (the K-tile stream runs across tile
- *                    boundaries; the bits of 2 and 5): NT form with K % 64 == 0, plain (bias, residual, bf16 or fp32 output), SwiGLU-forward and SwiGLU-backward epilogues,
- *                    and TN form, plain without bias; K > 192, N % 8 == 0, 16-byte aligned rows; other calls fall back to 2.  0 takes the kernel by itself, as one
- *                    workgroup per CU from 512 tiles upward, below that a workgroup per tile (environment variable MI355_GEMM_PERSIST_MIN_TILES, read per call, moves that
- *                    threshold: the 256 workgroups assume they all start together, so a caller that runs collectives or another stream's kernels beside its GEMMs
- *                    raises it for that time -- llm_quest_amd/ddp.py does)
+ *                    boundaries; the bits of 2 and 5): NT form with K % 64 == 0, plain (bias, residual, bf16 or fp32 output), SwiGLU-forward and SwiGLU-backward epilogues;
+ *                    NN form with K % 64 == 0, bf16 output, plain (residual) and SwiGLU-backward; TN form, plain without bias; K > 192, N % 8 == 0, 16-byte aligned rows.
+ *                    NT calls of 128 <= K <= 192 (bf16, no bias) run on eight waves per CU instead, other calls fall back to 2.  0 takes the kernels by itself, as one
+ *                    workgroup per CU from 512 tiles upward (short sums of the NT form on the eight waves), below that a workgroup per tile (environment variable
+ *                    MI355_GEMM_PERSIST_MIN_TILES, read per call, moves that threshold: the 256 workgroups assume they all start together, so a caller that runs
+ *                    collectives or another stream's kernels beside its GEMMs raises it for that time -- llm_quest_amd/ddp.py does)
  * Requirements: K-contiguous dims multiple of 8 elements (16-byte rows).            */
 int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const void* A, int64_t lda, const void* B,
                     int64_t ldb, void* C, int64_t ldc, int out_dtype, const float* bias, const void* residual,

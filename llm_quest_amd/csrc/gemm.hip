@@ -2402,6 +2402,10 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
     return M < 256 || N < 256 || (form != MI355_GEMM_TN && tiles256 < 128 + (epilogue == MI355_EPI_NONE));
 }
 
+static int launch_quad_form(int form, const GemmParams& p, int out_dtype, bool persistent, hipStream_t s) {
+    return form == MI355_GEMM_NT ? mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s) : form == MI355_GEMM_NN ? mi355_gemm_quad_nn_part10(&p, out_dtype, persistent, s) : mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s);
+}
+
 // Tile rows (128 or 192; 0: none fits) and K shares of gemm_ring_kernel for a product of too few 256x256 tiles.  Only in ONE round of the 256 CUs: with more tiles Cfg128's two
 // workgroups per CU are the better filling (996 x 6144, K = 1024: 21 us, this kernel in two rounds 25).  The least of: the launch (3.5 us, 4.5 with 192 rows), its K-tiles (0.44 us each
 // where up to a quarter of the CUs work, 0.62 from half of them on; 192 rows 0.6 / 0.76), and for K shares -- from 32 K-tiles on, as in choose_ksplit -- the reduction's launch and bytes.
@@ -2410,10 +2414,6 @@ static bool small_tiles(int form, int64_t M, int64_t N, int epilogue) {
 // us, Cfg128 (split as choose_ksplit has it) -> here: 5 664 x 1024, K = 2048 / 3584 / 7168 / 8256: 37.5 / 57.5 / 109 / 123 -> 32.5 / 48.7 / 88 / 100; 4 096 x 1024, K = 1024 / 3584:
 // 17.1 / 64.5 -> 14.9 / 39.5; 2 048 x 1024, K = 3584: 42.4 -> 30.2; 996 rows, 1024 x 3072 / 4096 x 1024 / 2048 x 1024: 23.6 / 17.8 / 15.6 -> 20.3 / 14.5 / 12.6; 333 rows, 4096 x 1024 /
 // 1024 x 3584: 15.2 / 17.9 -> 12.1 / 16.1.
-static int launch_quad_form(int form, const GemmParams& p, int out_dtype, bool persistent, hipStream_t s) {
-    return form == MI355_GEMM_NT ? mi355_gemm_quad_nt_part8(&p, out_dtype, persistent, s) : form == MI355_GEMM_NN ? mi355_gemm_quad_nn_part10(&p, out_dtype, persistent, s) : mi355_gemm_quad_tn_part9(&p, out_dtype, persistent, s);
-}
-
 static int choose_ring(int form, int64_t M, int64_t N, int64_t K, int out_dtype, bool may_split, int64_t ws_bytes, int& ksplit, int& fold, double& least) {
     const int64_t nt = (K + 63) / 64, tn = (N + 127) / 128;
     if (nt < 4) return 0;  // less than the ring: the launch is all of the time, and 128 KiB of LDS hold the next one up (K = 168, 17 x 144: 5.7 / 6.3 us)
@@ -2543,7 +2543,7 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
                       "mi355_gemm_bf16(SwiGLU backward epilogue): bf16 output [M, 2N] (ldc >= 2N), residual = the forward gate-up output [M, 2N], N %% 8 == 0, no bias");
     const int ablate = tile_hint >> 8;
     tile_hint &= 0xff;
-    MI355_REQUIRE((tile_hint >= 0 && tile_hint <= 5) || tile_hint == 7 || tile_hint == 8, "mi355_gemm_bf16: tile_hint must be 0 (auto), 1 (128x128), 2 (256x256), 3 (256x256, alternating wave groups), 4 (3 with one barrier per phase), 5 (256x256, four waves of 128x128), 7 (2 as a persistent workgroup per CU) or 8 (7 with the two wave groups a write-out apart)");
+    MI355_REQUIRE((tile_hint >= 0 && tile_hint <= 5) || tile_hint == 7 || tile_hint == 8, "mi355_gemm_bf16: tile_hint must be 0 (auto), 1 (128x128), 2 (256x256), 3 (256x256, alternating wave groups), 4 (3 with one barrier per phase), 5 (256x256, four waves of 128x128), 7 (256x256, four waves of 128x128 on a ring of panels, a persistent workgroup per CU) or 8 (eight waves, persistent, the two wave groups a write-out apart)");
     GemmParams p;
     p.A = (const bf16_t*)A; p.B = (const bf16_t*)B; p.C = C; p.bias = bias; p.R = residual;
     p.M = M; p.N = N; p.K = K; p.lda = lda; p.ldb = ldb; p.ldc = ldc; p.ldr = ldr;
@@ -2587,10 +2587,10 @@ extern "C" int mi355_gemm_bf16(int form, int64_t M, int64_t N, int64_t K, const 
     const bool persist_ok = form == MI355_GEMM_NT && out_dtype == MI355_DT_BF16 && (epilogue == MI355_EPI_NONE || epilogue == MI355_EPI_SWIGLU_FWD || epilogue == MI355_EPI_SWIGLU_BWD) &&
                             !bias && (K & 63) == 0 && K >= 128 && (N & 7) == 0 && (ldc & 7) == 0 && ((uintptr_t)C & 15) == 0 && M >= 256 && N >= 256 &&
                             (!residual || ((ldr & 7) == 0 && ((uintptr_t)residual & 15) == 0)) && ldc * 2 * 256 < 0x7fffffffLL && ldr * 2 * 256 < 0x7fffffffLL;
-    // four waves of 128x128 (gemm_quad.h), one workgroup per CU walking the tiles from two rounds of them upward: the same bits as tile 2, and 5, whose place they take where they can
+    // four waves of 128x128 (gemm_quad.h), one workgroup per CU walking the tiles from two rounds of them upward: the same bits as tile 2, whose place they take where they can
     const int64_t tiles256 = ((M + 255) / 256) * ((N + 255) / 256);
     const bool short_sum = persist_ok && tiles256 >= persist_min_tiles() && short_nt(epilogue, residual != nullptr, K);
-    if (tile_hint == 0 && ((cfg == 2 && form == MI355_GEMM_NT) || cfg == 5) && (short_sum || quad_ok(form, p, out_dtype))) {
+    if (tile_hint == 0 && cfg == 2 && form == MI355_GEMM_NT && (short_sum || quad_ok(form, p, out_dtype))) {
         const int kind_bit = epilogue == MI355_EPI_SWIGLU_FWD ? 4 : epilogue == MI355_EPI_SWIGLU_BWD ? 8 : residual ? 2 : 1;
         cfg = persist_ok && tiles256 >= persist_min_tiles() && (pp_mask() & kind_bit) ? 8 : 7;
     }
