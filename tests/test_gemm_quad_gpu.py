@@ -61,7 +61,13 @@ def test_input_gradients_of_weights_as_they_lie(M, N, K_):
     if want is not None:
         assert off(got, want, K_, BF16)
     if K_ <= 1024:
-        assert K.dgrad_on_quad(M, N, K_) and torch.equal(got, K.gemm(L.GEMM_NT, dy, wt, allow_split_k=False)) or M == 17016  # (its remainder's sums are cut in either form)
+        assert K.dgrad_on_quad(M, N, K_)
+        # (17 016 rows are cut: whole rounds of 256 tiles, and a remainder on small tiles whose sums are cut in either form)
+        main = M if M != 17016 else 256 // ((N + 255) // 256) * 256
+        assert torch.equal(got[:main], K.gemm(L.GEMM_NT, dy[:main], wt, allow_split_k=False))
+        if main < M:  # row by row: a few wrong ones at the seam are off by their size
+            want = dy[main:].double() @ w.double()
+            assert float(((got[main:].double() - want).norm(dim=1) / want.norm(dim=1)).max()) < 2**-24 * K_**0.5 + 2**-8
         gu = draw(7, M, 2 * N)
         assert torch.equal(K.gemm_dgrad_swiglu_bwd(dy, w, gu), K.swiglu_bwd(gu, K.gemm(L.GEMM_NN, dy, w, allow_split_k=False), N))
 

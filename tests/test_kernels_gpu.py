@@ -1166,34 +1166,34 @@ def test_persistent_nt_kernel_equals_the_per_tile_kernel_bit_for_bit(M, N, K_, m
     assert torch.equal(gu0, gu2) and torch.equal(a0, a2)
 
 
-@pytest.mark.parametrize("M,N,K_", [(709 * 5 + 3, 1024, 2048), (2600, 4096, 512), (4099, 264, 384), (513, 776, 2048), (300, 256, 320), (2049, 1288, 640), (70000, 1536, 128)])
+@pytest.mark.parametrize("M,N,K_", [(709 * 5 + 3, 1024, 2048), (2600, 4096, 512), (4099, 264, 384), (513, 776, 2048), (300, 256, 320), (2049, 1288, 640), (70000, 1536, 128), (1100, 33_032, 128), (520, 34_056, 512)])
 def test_weight_stationary_walk_equals_the_per_tile_kernel_bit_for_bit(M, N, K_, monkeypatch):
-    """The persistent NT kernel's weight-stationary XCD walk (tile hint 7 with ablation bit 3; the library's own choice by shape, MI355_GEMM_WALK) changes only
-    WHICH workgroup computes a tile and when: every epilogue gives the per-tile kernel's bits on ragged M, N that is no multiple of the tile or of a column group (empty
-    tiles are walked as zero work), fewer pairs than row streams, more tiles than CUs.  Then the same through the automatic choice with the walk forced on / off."""
+    """Persistent workgroups walk tiles in an order of their own -- short sums over more than 128 column panels weight-stationary per XCD --, which changes only WHICH workgroup computes a tile and when:
+    every epilogue gives the per-tile kernel's bits on ragged M, N that is no multiple of the tile or of a column group (empty tiles are walked as zero work), fewer pairs than row streams, more
+    tiles than CUs.  By hint 7, and through the automatic choice from one tile on, which takes short sums to the eight-wave kernel and N > 32 768 of them to its walk."""
     from llm_quest_amd import _lib as L
     from llm_quest_amd import kernels as K
 
-    W = 7 + (8 << 8)
     g = torch.Generator().manual_seed(M + 3 * N + 7 * K_)
     rnd = lambda *s: dev((0.3 * torch.randn(*s, generator=g)).to(BF16))
     x, w, res = rnd(M, K_), rnd(N, K_), rnd(M, N)
     ref = K.gemm(L.GEMM_NT, x, w, tile=2, allow_split_k=False)
-    got = torch.full_like(ref, 7.0)  # every element must be written
-    K.gemm(L.GEMM_NT, x, w, out=got, tile=W)
-    assert torch.equal(got, ref)
-    assert torch.equal(K.gemm(L.GEMM_NT, x, w, residual=res, tile=W), K.gemm(L.GEMM_NT, x, w, residual=res, tile=2, allow_split_k=False))
+    ref_res = K.gemm(L.GEMM_NT, x, w, residual=res, tile=2, allow_split_k=False)
     F = (N // 64) * 32
     wgu = rnd(2 * F, K_)
     gu2, a2 = K.gemm_gateup_swiglu(x, wgu, tile=2)
-    guw, aw = K.gemm_gateup_swiglu(x, wgu, tile=W)
-    assert torch.equal(guw, gu2) and torch.equal(aw, a2)
-    dy, w2, gu = rnd(M, K_), rnd(K_, N), rnd(M, 2 * N)
-    assert torch.equal(K.gemm_dgrad_swiglu_bwd(dy, w2, gu, tile=W), K.gemm_dgrad_swiglu_bwd(dy, w2, gu, tile=2))
-    monkeypatch.setenv("MI355_GEMM_PERSIST_MIN_TILES", "1")
-    for mode in ("1", "0", "2"):
-        monkeypatch.setenv("MI355_GEMM_WALK", mode)
-        assert torch.equal(K.gemm(L.GEMM_NT, x, w, allow_split_k=False), ref), mode
+    for tile in (7, 0):
+        if tile == 0:
+            monkeypatch.setenv("MI355_GEMM_PERSIST_MIN_TILES", "1")
+        got = torch.full_like(ref, 7.0)  # every element must be written
+        K.gemm(L.GEMM_NT, x, w, out=got, tile=tile, allow_split_k=False)
+        assert torch.equal(got, ref)
+        assert torch.equal(K.gemm(L.GEMM_NT, x, w, residual=res, tile=tile, allow_split_k=False), ref_res)
+        guw, aw = K.gemm_gateup_swiglu(x, wgu, tile=tile)
+        assert torch.equal(guw, gu2) and torch.equal(aw, a2)
+        if N < 32_768:
+            dy, w2, gu = rnd(M, K_), rnd(K_, N), rnd(M, 2 * N)
+            assert torch.equal(K.gemm_dgrad_swiglu_bwd(dy, w2, gu, tile=tile), K.gemm_dgrad_swiglu_bwd(dy, w2, gu, tile=2))
 
 
 @pytest.mark.parametrize("M,N,K_", [(709 * 5 + 3, 1024, 1024), (4099, 264, 384), (513, 776, 2048), (300, 256, 320), (5000, 3072, 1024)])
