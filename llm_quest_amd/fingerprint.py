@@ -15,7 +15,7 @@ import re
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 EVIDENCE_ROUND = "head"  # profiles/<EVIDENCE_ROUND>_* are the counter files bench.py reads
-FILES = ("attention.hip", "attn_common.h", "elementwise.hip", "gemm.hip", "norm_rope.hip", "common.h")
+FILES = ("attention.hip", "attn_common.h", "elementwise.hip", "gemm.hip", "gemm_persist.h", "gemm_quad.h", "lane_sums.h", "norm_rope.hip", "quad.h", "common.h")
 _FLAG_LINES = re.compile(r"^(CXXFLAGS|ARCH|FLAGS_(?:attention|elementwise|gemm|norm_rope))\s*\??=")
 
 

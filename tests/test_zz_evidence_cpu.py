@@ -24,6 +24,17 @@ def test_the_fingerprint_ignores_everything_but_the_steps_sources_and_flags(tmp_
     assert len(F.kernel_sources_sha()) == 16 and F.kernel_sources_sha() == F.kernel_sources_sha()
 
 
+def test_the_fingerprint_covers_every_header_of_the_steps_sources():
+    """A kernel that moved into a header of its own would otherwise change under counters that still count as its."""
+    import re
+
+    csrc = os.path.join(ROOT, "llm_quest_amd", "csrc")
+    for name in F.FILES:
+        with open(os.path.join(csrc, name)) as f:
+            for header in re.findall(r'^#include "([^"]+)"', f.read(), re.M):
+                assert header in F.FILES or not os.path.exists(os.path.join(csrc, header)) or header.startswith(".."), (name, header)
+
+
 def test_committed_counter_files_were_measured_on_the_kernel_sources_at_head():
     head = F.kernel_sources_sha()
     stamp = _load("stamp.json")
