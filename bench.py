@@ -184,8 +184,8 @@ def dominant_kernel_rate(batch, device):
     out = {}
     for name, fn, flops in (
         ("NT gate-up fwd", lambda: K.gemm(L.GEMM_NT, x, w), 2.0 * M * 6144 * 1024),
-        ("gate-up dgrad (the step's form)", lambda: K.dgrad(dy, w), 2.0 * M * 6144 * 1024),
-        ("NN gate-up dgrad (form not used by the step)", lambda: K.gemm(L.GEMM_NN, dy, w), 2.0 * M * 6144 * 1024),
+        ("NN gate-up dgrad (the step's form: the weight as it lies)", lambda: K.dgrad(dy, w), 2.0 * M * 6144 * 1024),
+        ("NT gate-up dgrad on a transposed copy of the weight (not used by the step)", lambda: K.gemm(L.GEMM_NT, dy, K.transpose(w)), 2.0 * M * 6144 * 1024),
         ("TN block weight gradients, grouped (the step's launch: QKV, out_proj, gate-up, down = 240 tiles)", lambda: K.gemm_grouped(L.GEMM_TN, group), 2.0 * M * sum(o * i for o, i in shapes)),
     ):
         for _ in range(3):

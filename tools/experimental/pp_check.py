@@ -96,41 +96,6 @@ def check():
     return bad
 
 
-def check_walk():
-    """hint 7 with the weight-stationary walk == hint 2, bit for bit (same K order), every epilogue, ragged shapes"""
-    bad = 0
-    W = 7 + 2048
-    for M, N, Kd in [(709 * 5 + 3, 1024, 1024), (2600, 4096, 512), (4099, 264, 384), (513, 776, 2048), (300, 256, 320), (2049, 1288, 640), (5000, 3072, 1024), (70000, 1536, 128)]:
-        g = torch.Generator().manual_seed(M + N + Kd)
-        x, w, res = rnd(M, Kd, g=g), rnd(N, Kd, g=g), rnd(M, N, g=g)
-        ok = torch.equal(K.gemm(L.GEMM_NT, x, w, tile=W), K.gemm(L.GEMM_NT, x, w, tile=2, allow_split_k=False))
-        ok &= torch.equal(K.gemm(L.GEMM_NT, x, w, residual=res, tile=W), K.gemm(L.GEMM_NT, x, w, residual=res, tile=2, allow_split_k=False))
-        F = (N // 64) * 32
-        wgu = rnd(2 * F, Kd, g=g)
-        a, b = K.gemm_gateup_swiglu(x, wgu, tile=W), K.gemm_gateup_swiglu(x, wgu, tile=2)
-        ok &= torch.equal(a[0], b[0]) and torch.equal(a[1], b[1])
-        dy, w2, gu = rnd(M, Kd, g=g), rnd(Kd, N, g=g), rnd(M, 2 * N, g=g)
-        ok &= torch.equal(K.gemm_dgrad_swiglu_bwd(dy, w2, gu, tile=W), K.gemm_dgrad_swiglu_bwd(dy, w2, gu, tile=2))
-        print("ok " if ok else "BAD", "walk", M, N, Kd, flush=True)
-        bad += not ok
-    os.environ["MI355_GEMM_PERSIST_MIN_TILES"] = "1"
-    for B, S, Hq, D, d in ((6, 709, 16, 128, 1024), (14, 300, 4, 128, 512)):
-        g = torch.Generator().manual_seed(B * S)
-        dy, w, ctx = rnd(B * S, d, g=g), rnd(d, Hq * D, g=g), rnd(B * S, Hq * D, g=g)
-        lse = torch.randn(B, Hq, S, generator=g).to(dev)
-        os.environ["MI355_GEMM_WALK"] = "0"
-        r0 = K.dgrad_attn_delta(dy, w, ctx, lse, B, S, Hq, D)
-        os.environ["MI355_GEMM_WALK"] = "1"
-        r1 = K.dgrad_attn_delta(dy, w, ctx, lse, B, S, Hq, D)
-        ok = torch.equal(r0[0], r1[0]) and torch.equal(r0[1], r1[1])
-        print("ok " if ok else "BAD", "walk delta", B, S, flush=True)
-        bad += not ok
-    os.environ.pop("MI355_GEMM_WALK", None)
-    os.environ.pop("MI355_GEMM_PERSIST_MIN_TILES", None)
-    print("WALK CHECK", "FAILED" if bad else "PASSED", flush=True)
-    return bad
-
-
 def timeit(fn, reps):
     ev = [torch.cuda.Event(enable_timing=True) for _ in range(reps + 1)]
     ev[0].record()
@@ -189,7 +154,7 @@ def bench():
 if __name__ == "__main__":
     rc = 0
     if mode in ("check", "both"):
-        rc = check_walk() + check()
+        rc = check()
     if mode in ("time", "both") and not rc:
         bench()
     sys.exit(1 if rc else 0)

@@ -7,7 +7,7 @@ sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))
 from llm_quest_amd.fingerprint import collection_stamp
 
 
-GEMM_KERNELS = ("gemm_bf16_kernel", "gemm_quad_kernel", "gemm_quad_grouped_kernel", "gemm_grouped_kernel")
+GEMM_KERNELS = ("gemm_bf16_kernel", "gemm_nt_persist_kernel", "gemm_quad_kernel", "gemm_quad_grouped_kernel", "gemm_grouped_kernel")
 
 
 def avg(d, counter):
