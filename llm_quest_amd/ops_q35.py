@@ -21,7 +21,7 @@ from . import _lib as L
 from . import kernels as K
 from . import kernels_q35 as Q
 from .arena import ParamArena
-from .ops import FUSE_SWIGLU_BWD, FUSE_SWIGLU_FWD, _flush_sums, _flush_wgrads, _vec_sum, _wgrad
+from .ops import FUSE_SWIGLU_BWD, FUSE_SWIGLU_FWD, _flush_sums, _flush_wgrads, _vec_sum, _vecgrad, _wgrad
 
 BF16, F32 = torch.bfloat16, torch.float32
 
