@@ -140,12 +140,11 @@ def test_shares_of_grouped_weight_gradients(tokens, shapes, odt):
 
 
 # rows of results in whole lines of 128 bytes (stored past the L2) and in parts of them: pitches that are a multiple of it and one that is not, a corner beside a line's start; columns that end inside a line
-@pytest.mark.parametrize("form,M,N,K_", [("nt", 383, 520, 448), ("nt", 17_000, 1792, 320), ("nn", 383, 520, 448), ("swiglu", 383, 544, 448), ("swiglu", 383, 520, 448), ("swiglu", 4000, 1088, 256), ("gateup", 600, 576, 320),
-                                         ("gateup", 600, 512, 320), ("tn", 520, 1288, 639)])
-@pytest.mark.parametrize("odt", [BF16, F32])
+WHOLE = [("nt", 383, 520, 448), ("nt", 17_000, 1792, 320), ("tn", 520, 1288, 639), ("nn", 383, 520, 448), ("swiglu", 383, 544, 448), ("swiglu", 383, 520, 448), ("swiglu", 4000, 1088, 256), ("gateup", 600, 576, 320), ("gateup", 600, 512, 320)]
+
+
+@pytest.mark.parametrize("form,M,N,K_,odt", [(*c, odt) for c in WHOLE for odt in (BF16, F32)[: 2 if c[0] in ("nt", "tn") else 1]])
 def test_results_in_whole_lines_and_in_parts_of_them(form, M, N, K_, odt):
-    if form not in ("nt", "tn") and odt == F32:
-        pytest.skip("bf16 results only")
     A, B = (draw(M, K_, M), draw(N, K_, N)) if form == "tn" else (draw(M, M, K_), draw(N, K_, N) if form in ("nn", "swiglu") else draw(N, N, K_))
     gu, act = draw(4, M, 2 * N), torch.empty(M, N // 2, dtype=BF16, device="cuda")
     W = 2 * N if form == "swiglu" else N
