@@ -79,32 +79,32 @@ def _vecgrad(arena, p):
 def _vec_sum(sums, arena, p, part):
     """p.grad (+)= the sum of the rows of ``part``, once ``_flush_sums`` has run; ``arena`` None: a stand-alone fp32 parameter."""
     if p.requires_grad:
-        sums.append((part, arena, p))
+        sums.append((part, arena, p, torch.empty(p.shape, dtype=F32, device=p.device) if arena is None and p.grad is None else None))
 
 
 def _flush_sums(sums):
     """The vector gradients of a block, up to four to a launch (``kernels.reduce_rows_each``).  The sums of a launch have no order, so one that adds to what another of them stores -- a parameter that
     the block holds twice, say a key norm tied to the query norm -- waits for the next launch.  A gradient is attached where it is written: a backward that ends before (an allocation that fails)
     leaves ``.grad`` as it was."""
-    made = {id(p): torch.empty(p.shape, dtype=F32, device=p.device) for _, arena, p in sums if arena is None and p.grad is None}
-    launches, keys = [], ()
-    for part, arena, p in sums:
-        own = None if arena is not None else made[id(p)] if p.grad is None else p.grad
-        key = id(p) if own is None else own.untyped_storage().data_ptr()  # (an arena's gradients do not overlap)
-        if len(keys) in (0, 4) or key in keys:
-            launches.append([])
-            keys = set()
-        launches[-1].append((part, arena, p, own))
-        keys.add(key)
-    for group in launches:
-        ready = []
-        for part, arena, p, own in group:
-            view, acc = arena.grad_target(p) if own is None else (own.view(-1), p.grad is not None)
+    i = 0
+    while i < len(sums):
+        ready, fresh, seen = [], [], []
+        for part, arena, p, made in sums[i : i + 4]:
+            if any(q is p for q in seen):
+                break
+            seen.append(p)
+            if arena is not None:
+                view, acc = arena.grad_target(p)
+            else:
+                view, acc = p.grad, True
+                if view is None:
+                    view, acc = made, False
+                    fresh.append((p, made))
             ready.append((part, view, acc))
         K.reduce_rows_each(ready)
-        for _, _, p, own in group:
-            if own is not None and p.grad is None:
-                p.grad = own
+        for p, made in fresh:
+            p.grad = made
+        i += len(ready)
     sums.clear()
 
 
