@@ -19,7 +19,7 @@
 //   * Epilogue: accumulators -> LDS (fp32, 64x64 at a time per wave) -> row-contiguous 16-B global stores with
 //     bias/GELU/residual fused, or raw fp32 slabs when K is split (few output tiles + long K: weight gradients).
 //   * Workgroup -> tile map: XCD-aware (blocks b and b+8 share an L2) then 3-row super-groups.
-// The large NT products and weight gradients are gemm_quad.h's, the mid-size NT and NN products gemm_ring_kernel's; gemm_tile serves the other forms, fused epilogues and sizes.
+// The large products of every form are gemm_quad.h's, those of short sums among the NT ones gemm_persist.h's, the mid-size NT and NN products gemm_ring_kernel's; gemm_tile serves the other epilogues, sizes and pitches.
 #include <algorithm>
 #include <type_traits>
 

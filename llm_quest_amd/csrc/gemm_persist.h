@@ -8,7 +8,7 @@
 //   * the write-out stages through a 32-KiB region BESIDE the two stages (4 KiB per wave: 32 rows x 64 columns of packed bf16 at a time, swizzled, not padded), so it
 //     needs no barrier and does not collide with the stream; the B fragment is the MFMA's first operand, so a lane holds four consecutive columns of a row and
 //     packs them itself: a quarter of the LDS bytes of gemm_tile's fp32 staging.
-//   * more than 128 column panels (vocabulary-wide heads): WALK.  us, without -> with: 2 048 x 151 936, K = 256 229 -> 187, 512 359 -> 309, 1 024 x 248 320, K = 512 311 -> 255; 4 096 x 32 000 125 / 130.
+//   * more than 128 column panels (vocabulary-wide heads): WALK.  us, without -> with: 2 048 x 151 936, K = 256 229 -> 185, 512 359 -> 306, 1 024 x 248 320, K = 512 311 -> 249; 4 096 x 32 000, 512 125 / 130.
 // The bits of gemm_bf16_kernel (same MFMA sequence per output, same rounding).  bf16 output, K % 64 == 0, K >= 128, N % 8 == 0, no bias.
 template <int KIND, bool RES, bool WALK>  // KIND: MI355_EPI_NONE (RES: + bf16 residual, added in fp32 before the rounding), MI355_EPI_SWIGLU_FWD, MI355_EPI_SWIGLU_BWD (see gemm_tile's epilogue for both)
 __global__ __launch_bounds__(512, 2) void gemm_nt_persist_kernel(GemmParams p, int ntiles) {
