@@ -130,6 +130,35 @@ def test_gradient_accumulation_and_zero_grad(golden):
         assert rel_l2(p.grad, g1[n]) < 1e-2, n
 
 
+def test_gradients_of_norms_that_a_block_holds_twice(golden):
+    """A key norm tied to the query norm, one norm for both halves: the gradient is the sum of both uses', rounded to bf16 after each, and the same bits in every pass (the two sums are never in one
+    launch, whose workgroups store in no order)."""
+    t = golden("qwen3_tiny")
+    ids, tgt = t["in.ids"].cuda(), t["in.targets"].cuda()
+    grads, tied = [], (("att.k_norm", "att.q_norm"), ("norm2", "norm1"))
+    for tie in (False, True):
+        m = make_qwen(t)
+        with torch.no_grad():
+            for blk in m.trf_blocks:
+                for a, b in tied:
+                    blk.get_parameter(a + ".weight").copy_(blk.get_parameter(b + ".weight"))
+        if tie:
+            for blk in m.trf_blocks:
+                blk.att.k_norm.weight, blk.norm2.weight = blk.att.q_norm.weight, blk.norm1.weight
+        passes = []
+        for _ in range(3):
+            m.zero_grad(set_to_none=True)
+            h = m.forward_hidden(ids)
+            m.lm_loss(h.reshape(-1, h.shape[-1]), tgt.reshape(-1)).backward()
+            passes.append([{n: blk.get_parameter(n + ".weight").grad.float().clone() for n in ("att.q_norm", "att.k_norm", "norm1", "norm2")} for blk in m.trf_blocks])
+        assert all(torch.equal(p[i][n], passes[0][i][n]) for p in passes for i in range(len(p)) for n in p[i])
+        grads.append(passes[0])
+    for one, both in zip(*grads):
+        for a, b in tied:
+            want, size = one[a] + one[b], one[a].abs() + one[b].abs()
+            assert torch.equal(both[a], both[b]) and bool(((both[a] - want).abs() <= 2.0**-7 * size + 1e-30).all())  # (three roundings of at most 2^-8 of either's size)
+
+
 def test_standalone_submodules(golden):
     """GroupedQueryAttention / FFN / RMSNorm called on their own (reference call convention) vs golden per-op fixtures."""
     from llm_quest_amd.common.buffers import GlobalBuffers
