@@ -58,6 +58,25 @@ def test_which_sums_take_it(K_, plain, gateup, residual):
             K.persistent_gemm(True)
 
 
+@pytest.mark.parametrize("B,S,Hq", [(6, 709, 4), (9, 500, 3)])
+@pytest.mark.parametrize("K_", [128, 192, 256, 320, 384, 448])
+def test_attention_constants_behind_short_sums(B, S, Hq, K_, monkeypatch):
+    """d(ctx) in the bits of the plain product, its row sums with ctx per head (128 products of 16-bit numbers in fp32, in any order), their negatives and the scaled lse in the backward's scratch; an odd
+    number of heads, rows that end inside a tile.  384 is four waves' (csrc/gemm.hip: short_nt)."""
+    monkeypatch.setenv("MI355_GEMM_PERSIST_MIN_TILES", "1")
+    dy, w, ctx, lse = draw(1, B * S, K_), draw(2, K_, Hq * 128), draw(3, B * S, Hq * 128), draw(4, B, Hq, S, dtype=F32)
+    fn = lambda: K.dgrad_attn_delta(dy, w, ctx, lse, B, S, Hq, 128)
+    dctx, delta = fn()
+    assert any("gemm_nt_persist_kernel" in n for n in kernels_of(fn)) is (K_ != 384)
+    assert torch.equal(dctx, K.gemm(L.GEMM_NT, dy, w.T.contiguous(), tile=2, allow_split_k=False))
+    prod = (dctx.double() * ctx.double()).view(B, S, Hq, 128).permute(0, 2, 1, 3)
+    assert bool(((delta.double() - prod.sum(-1)).abs() <= 128 * 2.0**-24 * prod.abs().sum(-1)).all())
+    lib, n = L.load(), 4 * B * Hq * S
+    ws = K._attn_scratch(dy.device, lib.mi355_attn_bwd_workspace_bytes(B, S, Hq, 128))
+    nl2, ndl = (ws[o : o + n].view(F32).view(B, Hq, S) for o in (lib.mi355_attn_bwd_workspace_rowconst_offset(B, S, Hq, 128, i) for i in (0, 1)))
+    assert torch.equal(ndl, -delta) and torch.equal(nl2, -lse * torch.tensor(1.4426950408889634, dtype=F32, device="cuda"))
+
+
 def test_weight_gradients_just_beyond_one_round_of_tiles():
     """Few tokens: 128 x 128 tiles (in brackets those of 256 x 256) where they are one round of two a CU, and where the larger ones need a second round for a few."""
     def small(T, shapes, odt=BF16):
