@@ -88,18 +88,23 @@ def _flush_sums(sums):
     leaves ``.grad`` as it was."""
     i = 0
     while i < len(sums):
-        ready, fresh, seen = [], [], []
+        ready, fresh, seen, spans = [], [], [], []
         for part, arena, p, made in sums[i : i + 4]:
             if any(q is p for q in seen):
                 break
-            seen.append(p)
             if arena is not None:
                 view, acc = arena.grad_target(p)
+            elif p.grad is None:
+                view, acc = made, False
+                fresh.append((p, made))
             else:
                 view, acc = p.grad, True
-                if view is None:
-                    view, acc = made, False
-                    fresh.append((p, made))
+                lo = view.data_ptr()
+                hi = lo + 4 * view.numel()
+                if any(a < hi and lo < b for a, b in spans):  # two parameters that were given one tensor's memory for their gradients
+                    break
+                spans.append((lo, hi))
+            seen.append(p)
             ready.append((part, view, acc))
         K.reduce_rows_each(ready)
         for p, made in fresh:

@@ -144,6 +144,18 @@ def test_a_backward_that_ends_early_leaves_no_unwritten_gradient(kernels, make, 
         assert all(torch.equal(p.grad.float(), t) for p, t in zip(params, want))
 
 
+def test_fp32_gradients_in_one_tensors_memory(kernels):
+    """A program may have given stand-alone parameters gradients that share memory: both sums arrive, as one launch behind the other."""
+    blk, backward = hybrid(0)
+    a, b = blk.att.post_norm.weight, blk.att.log_A
+    memory = torch.zeros(HEAD)
+    a.grad, b.grad = memory, memory[1:3]
+    backward()
+    want = kernels.given[1].sum(0)
+    want[1:3] += kernels.given[3].sum(0)
+    assert torch.equal(memory, want)
+
+
 @pytest.mark.parametrize("tied", [{}, {"ffn.lin2": "att.out_proj"}, {"att.out_proj": "att.w_keys"}, {"ffn.lin2": "att.w_queries", "att.out_proj": "att.w_values"}])
 def test_a_weight_that_a_block_holds_twice_is_in_one_grouped_launch_once(kernels, tied, monkeypatch):
     """The products of a grouped launch have no order either."""
